@@ -10,7 +10,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 41
+ABI_VERSION = 42
 _lib = None
 _lock = threading.Lock()
 
@@ -126,6 +126,9 @@ _SIGNATURES = {
     "blm_attn_prefill_mfma": [_c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int,
                               _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
                               _c_int, _c_int, _c_void_p, _c_int, _c_float, _c_int, _c_void_p],
+    "blm_gemm_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "blm_gemv_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "blm_gemv_f32_geometry": [_c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p],
     "blm_gemm_tiled": [_c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                        _c_int, _c_int, _c_void_p],
     "blm_gemv_skinny": [_c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int,
@@ -517,6 +520,63 @@ def gemm_tiled(a, w, out):
     return out
 
 
+# rows x columns of a block's tile of gemm_f32 -> code of the C ABI
+F32_TILES = {(128, 128): 0, (128, 64): 1, (64, 128): 2, (64, 64): 3}
+
+
+def f32_rows(a, w):
+    """Whether the 32-bit matrix-core products take these operands: float32 with rows in units of 16 bytes."""
+    return (a.dtype == w.dtype == torch.float32 and a.shape[1] % 4 == 0 and a.stride(1) == 1 and a.stride(0) % 4 == 0
+            and a.stride(0) >= a.shape[1] and w.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def gemm_f32(a, w, out, gated=False, tile=(128, 128)):
+    """The float32 product for many rows: out[M, N] = a[M, K] @ w[N, K]^T, or out [groups, M, N] partial products over that
+    many groups of K (the reader sums them).  gated=True: w is [gate rows; up rows] ([2 N, K]) and out = silu(a gate^T) * (a up^T)."""
+    _gpu(a, w, out)
+    groups = out.shape[0] if out.dim() == 3 else 1
+    M, N = out.shape[-2:]
+    if not f32_rows(a, w) or out.dtype != torch.float32 or out.stride(-1) != 1:
+        raise KernelError("gemm_f32: operands must be float32 with rows in units of 16 bytes")
+    if a.shape[0] != M or w.shape != (N * (2 if gated else 1), a.shape[1]):
+        raise KernelError(f"gemm_f32: shapes a={tuple(a.shape)} w={tuple(w.shape)} out={tuple(out.shape)} do not fit")
+    if out.dim() == 3:
+        _contig("out", out)
+    if tile not in F32_TILES:
+        raise KernelError(f"gemm_f32: tile {tile} is not one of {sorted(F32_TILES)}")
+    _call("blm_gemm_f32", a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, a.shape[1], a.stride(0), out.stride(-2), 1 if gated else 0,
+          groups, F32_TILES[tile], _stream())
+    return out
+
+
+def gemv_f32_geometry(M, N, K, groups=1):
+    """(blocks over all groups, wavefronts per block) that gemv_f32 launches for M rows of a [N, K] matrix in that many groups
+    of K, or None if it does not take them."""
+    blocks, waves = ctypes.c_int(0), ctypes.c_int(0)
+    ok = library().blm_gemv_f32_geometry(int(M), int(N), int(K), int(groups), ctypes.byref(blocks), ctypes.byref(waves))
+    return (blocks.value, waves.value) if ok else None
+
+
+def gemv_f32(a, packed, out, K, gated=False):
+    """The float32 product for up to 16 rows, streaming packed = pack_weight(w, gated) of w [N, K] once.  out: float32 [M, N],
+    or [groups, M, N] partial products over that many groups of K; gated=True: [M, I] = silu(a gate^T) * (a up^T) for a
+    matrix of 2 I rows."""
+    _gpu(a, packed, out)
+    groups = out.shape[0] if out.dim() == 3 else 1
+    M, N = out.shape[-2], out.shape[-1] * (2 if gated else 1)
+    if a.shape != (M, K) or a.dtype != torch.float32 or out.dtype != torch.float32 or packed.dtype != torch.float32:
+        raise KernelError(f"gemv_f32: float32 operands wanted, shapes a={tuple(a.shape)} out={tuple(out.shape)} K={K}")
+    if packed.numel() != ((N + 15) // 16) * ((K + 15) // 16) * 256 or not packed.is_contiguous():
+        raise KernelError(f"gemv_f32: the packed weights have {packed.numel()} elements, not those of a [{N}, {K}] matrix")
+    if a.stride(1) != 1 or out.stride(-1) != 1:
+        raise KernelError("gemv_f32: a and out need unit stride along their rows")
+    if out.dim() == 3:
+        _contig("out", out)
+    _call("blm_gemv_f32", a.data_ptr(), packed.data_ptr(), out.data_ptr(), M, N, K, a.stride(0), out.stride(-2), 1 if gated else 0,
+          groups, _stream())
+    return out
+
+
 def gemv_skinny(a, w, out):
     """The same product for M <= 8 rows; streams w once."""
     M, N, K = _check_mm(a, w, out)
@@ -544,26 +604,27 @@ def gemv_mfma_geometry(M, N, K, groups=1):
 
 
 def pack_weight(w, gated=False):
-    """Copy of a bfloat16 weight matrix [N, K] in the order the matrix-core skinny product streams
-    it: packed[tile, step, lane, e] = w[tile*16 + lane%16, step*32 + (lane//16)*8 + e], with N
-    padded to a multiple of 16 and K to a multiple of 32 by zeros.  Returns a flat tensor.
+    """Copy of a bfloat16 or float32 weight matrix [N, K] in the order the matrix-core skinny product streams
+    it: packed[tile, step, lane, e] = w[tile*16 + lane%16, step*S + (lane//16)*E + e], with E elements of 16 bytes (eight or
+    four), S = 4 E, N padded to a multiple of 16 and K to a multiple of S by zeros.  Returns a flat tensor.
     gated=True: w is [gate rows; up rows]; its rows are first re-ordered into blocks of 8 gate rows
     followed by the 8 matching up rows, so that each tile holds 8 gated pairs (gemv_mfma gated=True)."""
-    if w.dtype != torch.bfloat16 or w.dim() != 2:
-        raise KernelError("pack_weight: needs a bfloat16 matrix")
+    if w.dtype not in (torch.bfloat16, torch.float32) or w.dim() != 2:
+        raise KernelError("pack_weight: needs a bfloat16 or float32 matrix")
     N, K = w.shape
+    E = 16 // w.element_size()
     if gated:
         if N % 16:
             raise KernelError("pack_weight: a gated matrix needs a multiple of 8 features")
         half = N // 2
         w = torch.stack([w[:half].view(half // 8, 8, K), w[half:].view(half // 8, 8, K)], dim=1).reshape(N, K)
-    Np, Kp = (N + 15) // 16 * 16, (K + 31) // 32 * 32
+    Np, Kp = (N + 15) // 16 * 16, -(-K // (4 * E)) * 4 * E
     if (Np, Kp) != (N, K):
         padded = torch.zeros(Np, Kp, dtype=w.dtype, device=w.device)
         padded[:N, :K] = w
         w = padded
     # [tile, row, step, kg, e] -> [tile, step, kg, row, e]
-    return w.view(Np // 16, 16, Kp // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous().view(-1)
+    return w.view(Np // 16, 16, Kp // (4 * E), 4, E).permute(0, 2, 3, 1, 4).contiguous().view(-1)
 
 
 def gemv_mfma(a, packed, out, K, gated=False, activation="silu"):

@@ -1,9 +1,11 @@
 """What parts need from the machine: device, activation dtype, and the matrix product.
 
 Matrix products ``x[M,K] @ w[N,K]^T``:
-* float32 weights: the hand-written float kernels always (plain fused multiply-adds, no
+* float32 weights: the hand-written float kernels always (float operands, products and sums, no
   reduced-precision matrix mode), whatever the activation dtype.  This is the whole float32 path
-  and also what keeps a tensor that a checkpoint stores in 32 bits exact in a bfloat16 run.
+  and also what keeps a tensor that a checkpoint stores in 32 bits exact in a bfloat16 run.  With float32
+  activations whose rows lie in units of 16 bytes: up to 16 rows ops.gemv_f32 on a packed copy, more rows
+  ops.gemm_f32 (f32_plan chooses its tile and groups of K); everything else ops.gemm_tiled.
 * bfloat16 weights, up to 64 rows (decode): the hand-written skinny kernel on the matrix cores that
   streams the weight once (where the width fits its registers: see ops.gemv_mfma_group_limit).  From
   17 rows on, the products that come as partial planes (output and down projection) and, from 33 rows
@@ -81,6 +83,34 @@ def rows_plan(N, K, compute_units):
     return groups, columns
 
 
+# Tiles of ops.gemm_f32: microseconds for a step of 32 along K of a block that has its compute unit to itself (the loads'
+# latency shows), and per step and block where blocks share a unit (the matrix instructions' rate).  Measured with 17 to
+# 2,048 rows at [3072, 2048], [2048, 2048], [16384, 2048], [2048, 8192], [5000, 1416].
+F32_STEP_US = {(128, 128): (2.33, 2.0), (128, 64): (1.25, 1.0), (64, 128): (1.2, 1.0), (64, 64): (0.7, 0.5)}
+F32_SKINNY_MAX_ROWS = 16
+F32_SKINNY_GROUP_K = 2048
+
+
+def f32_plan(M, N, K, compute_units, planes=False, gated=False):
+    """(tile, groups of K, microseconds) of ops.gemm_f32 that a sum of its parts' costs finds fastest: every unit works through
+    its share of the blocks, and every plane of partial products is written once and read once by the norm that adds it.
+    Against the best tile and groups of the sweep the choice is within 6 % from 250 rows on and within 20 % below."""
+    best = None
+    for (bm, bn), (alone, shared) in F32_STEP_US.items():
+        if gated and bn != 128:
+            continue
+        tiles = -(-M // bm) * -(-N // (bn // 2 if gated else bn))
+        for groups in (1, 2, 4, 8) if planes and not gated else (1,):
+            if groups > 1 and K // groups < 128:
+                continue
+            steps = -(-K // groups // 32)
+            per_unit = -(-tiles * groups // compute_units)
+            us = 3.0 + steps * max(alone, per_unit * shared) + (M * N * groups * 8 / 4e6 if groups > 1 else 0.0)
+            if best is None or us < best[2] * 0.999:
+                best = ((bm, bn), groups, us)
+    return best
+
+
 class FusedProjectionPlan:
     """Launch geometry of a projection that a part fuses with work of its own (Runtime.qkv_plan).
     kernel: "rows" (ops.gemm_rows_qkv_rope's geometry: `rows` rows staged per block, `columns` columns
@@ -139,6 +169,7 @@ class Runtime:
             raise RuntimeError("no GPU is visible to this process; burn-lm_amd has no CPU path")
         self.ops = ops
         self._k_groups = {}     # (N, K, M) -> groups of K, as chosen once (see k_groups)
+        self._f32_plans = {}    # the same for the float32 products
         ops.library()  # fail now, loudly, if the kernel library cannot be had
         ops.arrival_counters(self.device)   # allocated here, before any graph capture can be open
         ops.gemm_mfma_init(self.device)     # likewise: a function attribute is set once per device
@@ -175,6 +206,10 @@ class Runtime:
         # product has no planes)
         packable = w.dtype == torch.bfloat16 and K % 8 == 0 and K >= 8 and (
             ops.gemv_mfma_supported(1, N, K) and N % 16 == 0 if gated else True)
+        if w.dtype == torch.float32:
+            # the gated product has no planes, so a longer K or an odd number of pairs goes as a plain product and a pass
+            packable = self.dtype == torch.float32 and K % 4 == 0
+            gated = gated and N % 16 == 0 and K <= F32_SKINNY_GROUP_K
         return LinearWeight(w, packable, gated)
 
     def k_groups(self, N, K, M=1):
@@ -212,6 +247,40 @@ class Runtime:
             return best
         # no grouping within the bounds: the coarsest one the kernel takes
         return next((g for g in (1, 2, 4, 8, 16, 32, 64) if ops.gemv_mfma_geometry(M, N, K, g) is not None), 64)
+
+    def f32_skinny_groups(self, M, N, K, planes):
+        """Into how many groups ops.gemv_f32 cuts K: the fewest that it takes and, where the planes may stay apart, whose
+        blocks fill at least GROUP_MIN_FILL of a round on the compute units (us at 8 rows, in 1 / 2 / 4 groups: [2048, 2048]
+        8.7 / 6.6 / 5.7 with 128 / 256 / 256 blocks; [2048, 8192] in 4 / 8 groups 16.0 / 15.6)."""
+        key = (M, N, K, planes)
+        known = self._f32_plans.get(key)
+        if known is None:
+            taken = [(g, ops.gemv_f32_geometry(M, N, K, g)) for g in (1, 2, 4, 8, 16, 32, 64)]
+            taken = [(g, geometry[0]) for g, geometry in taken if geometry is not None]
+            full = [g for g, blocks in taken if blocks >= GROUP_MIN_FILL * self.compute_units and K // g >= 256]
+            known = self._f32_plans[key] = (full[0] if planes and full else taken[0][0]) if taken else 0
+        return known
+
+    def _f32_linear(self, x, w, holder, out, planes):
+        """The float32 product of operands that ops.f32_rows takes, or None where the older kernels do it."""
+        M, K = x.shape
+        N = w.shape[0]
+        if M <= F32_SKINNY_MAX_ROWS and holder is not None and holder.packable and not holder.gated:
+            groups = self.f32_skinny_groups(M, N, K, planes)
+            if groups == 1:
+                return ops.gemv_f32(x, holder.packed, out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device), K)
+            if groups:
+                parts = ops.gemv_f32(x, holder.packed, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), K)
+                if planes:
+                    return parts
+                if out is None or out.is_contiguous():
+                    return ops.sum_planes(parts, out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device))
+        if M <= SKINNY_MAX_ROWS:
+            return None
+        tile, groups, _ = f32_plan(M, N, K, self.compute_units, planes)
+        if groups > 1:
+            return ops.gemm_f32(x, w, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), tile=tile)
+        return ops.gemm_f32(x, w, out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device), tile=tile)
 
     def rows_plan(self, N, K):
         """(groups of K, columns per block) for a product of 17 to 64 rows that may come as partial planes."""
@@ -315,6 +384,10 @@ class Runtime:
         out_dtype = out_dtype or self.dtype
         planes = partials and out is None       # the result may come as float32 partial planes
         if w.dtype == torch.float32 or x.dtype == torch.float32:
+            if out_dtype == torch.float32 and ops.f32_rows(x, w):
+                done = self._f32_linear(x, w, holder, out, planes)
+                if done is not None:
+                    return done
             if out is None:
                 out = torch.empty(M, N, dtype=out_dtype, device=x.device)
             if M <= SKINNY_MAX_ROWS and x.dtype == w.dtype == out_dtype == torch.float32 and K % 8 == 0 \
@@ -417,6 +490,15 @@ class Runtime:
         plain = w.w if isinstance(w, LinearWeight) else w
         if activation not in ("silu", "gelu_tanh"):
             raise ValueError(f"gated_linear: activation {activation!r} unknown (silu, gelu_tanh)")
+        if plain.dtype == torch.float32 and self.dtype == torch.float32 and activation == "silu" and ops.f32_rows(x, plain):
+            if M <= F32_SKINNY_MAX_ROWS:
+                if isinstance(w, LinearWeight) and w.packable and w.gated:
+                    return ops.gemv_f32(x, w.packed, torch.empty(M, inner, dtype=torch.float32, device=x.device), K, gated=True)
+            else:
+                tile, _, fused = f32_plan(M, inner, K, self.compute_units, gated=True)
+                # few rows: the plain product's smaller tiles and the pass behind it (12 bytes an element)
+                if fused <= f32_plan(M, 2 * inner, K, self.compute_units)[2] + 3.0 + M * inner * 12 / 5e6:
+                    return ops.gemm_f32(x, plain, torch.empty(M, inner, dtype=torch.float32, device=x.device), gated=True, tile=tile)
         silu = activation == "silu"      # the row-ring kernel gates with silu only; the others take the activation
         fusable = (x.dtype == plain.dtype == self.dtype == torch.bfloat16 and K % 8 == 0 and x.stride(1) == 1
                    and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and plain.is_contiguous())
@@ -472,7 +554,7 @@ class Runtime:
             tile = ((256, 256) if m256 * -(-inner // 128) >= self.compute_units else
                     (256, 128) if m256 * -(-inner // 64) >= self.compute_units else (128, 128))
             return ops.gemm_mfma(x, plain, torch.empty(M, inner, dtype=self.dtype, device=x.device), gated=True, tile=tile, activation=activation)
-        gu = self.linear(x, plain)
+        gu = self.linear(x, w if isinstance(w, LinearWeight) and not w.gated else plain)
         act = torch.empty(M, inner, dtype=gu.dtype, device=x.device)
         (ops.swiglu if silu else ops.gelu_glu)(gu, act)
         return act

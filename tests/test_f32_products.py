@@ -1,0 +1,109 @@
+"""The float32 products on the matrix cores alone: every tile, the edges of tiles, remainders of K, groups of K, the gating,
+rows that are longer than what is multiplied; and the runtime's choice among them over the forms that it accepts.
+
+The bound on an element's error is that of a sum of K products in any order with one rounding per product and addition:
+(K + 2) 2^-24 times the sum of the products' sizes (and a few roundings more for the gating)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -24
+
+
+def operands(M, N, K, pad=0, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    whole = torch.full((M, K + pad), float("nan"))
+    whole[:, :K] = torch.randn(M, K, generator=g)
+    return whole.cuda()[:, :K], torch.randn(N, K, generator=g).cuda()
+
+
+def check(got, x, w, gated=False):
+    x64, w64 = x.double(), w.double()
+    want, room = x64 @ w64.t(), (x.shape[1] + 2) * EPS * (x64.abs() @ w64.abs().t())
+    if gated:
+        g, u = want.chunk(2, -1)
+        dg, du = room.chunk(2, -1)
+        want = torch.nn.functional.silu(g) * u
+        room = 1.1 * dg * u.abs() + du * g.abs() + dg * du + 8 * EPS * want.abs()     # |silu'| < 1.1, |silu(g)| <= |g|
+    assert bool(((got.double() - want).abs() <= room + 1e-30).all()), float(((got.double() - want).abs() / (room + 1e-30)).max())
+
+
+@pytest.mark.parametrize("tile", [(128, 128), (128, 64), (64, 128), (64, 64)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (17, 33, 28), (63, 64, 32), (64, 65, 36), (65, 130, 160), (129, 127, 260), (257, 515, 96)])
+def test_many_rows(tile, M, N, K):
+    from burn_lm_amd.csrc import ops
+    x, w = operands(M, N, K, pad=4 * (M % 3))
+    check(ops.gemm_f32(x, w, torch.full((M, N), float("nan"), device="cuda"), tile=tile), x, w)
+    for groups in (2, 3, 8):
+        check(ops.gemm_f32(x, w, torch.full((groups, M, N), float("nan"), device="cuda"), tile=tile).sum(0), x, w)
+
+
+@pytest.mark.parametrize("tile", [(128, 128), (64, 128)])
+@pytest.mark.parametrize("M,I,K", [(17, 8, 28), (64, 64, 32), (65, 65, 36), (129, 200, 260)])
+def test_many_rows_gated(tile, M, I, K):
+    from burn_lm_amd.csrc import ops
+    x, w = operands(M, 2 * I, K, pad=4)
+    check(ops.gemm_f32(x, w, torch.full((M, I), float("nan"), device="cuda"), gated=True, tile=tile), x, w, gated=True)
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 15, 16])
+@pytest.mark.parametrize("N,K", [(1, 4), (16, 16), (17, 20), (100, 512), (33, 516), (48, 2048), (2048, 2044)])
+def test_few_rows(M, N, K):
+    from burn_lm_amd.csrc import ops
+    x, w = operands(M, N, K, pad=4 * (M % 2))
+    packed = ops.pack_weight(w)
+    for groups in (1, 2, 3):
+        out = torch.full((groups, M, N), float("nan"), device="cuda")
+        check((ops.gemv_f32(x, packed, out, K)).sum(0), x, w)
+    wide = torch.full((M, N + 3), float("nan"), device="cuda")
+    check(ops.gemv_f32(x, packed, wide[:, :N], K), x, w)
+    assert bool(wide[:, N:].isnan().all())
+
+
+@pytest.mark.parametrize("M,I,K", [(1, 8, 4), (3, 24, 100), (8, 72, 516), (16, 256, 2048)])
+def test_few_rows_gated(M, I, K):
+    from burn_lm_amd.csrc import ops
+    x, w = operands(M, 2 * I, K)
+    check(ops.gemv_f32(x, ops.pack_weight(w, gated=True), torch.full((M, I), float("nan"), device="cuda"), K, gated=True), x, w, gated=True)
+
+
+def test_refused():
+    from burn_lm_amd.csrc import ops
+    x, w = operands(17, 32, 2052)
+    out = torch.empty(17, 32, device="cuda")
+    with pytest.raises(ops.KernelError):
+        ops.gemv_f32(x, ops.pack_weight(w), out, 2052)                        # 17 rows
+    with pytest.raises(ops.KernelError):
+        ops.gemv_f32(x[:8], ops.pack_weight(w), out[:8], 2052)                # more than a group's stretch
+    with pytest.raises(ops.KernelError):
+        ops.gemm_f32(x[:, 1:], w[:, 1:].contiguous(), out)                    # rows at odd addresses
+    assert not ops.f32_rows(x[:, 1:], w) and not ops.f32_rows(x.t(), w) and not ops.f32_rows(x.bfloat16(), w)
+
+
+@pytest.mark.parametrize("K", [64, 70, 2048, 2052, 4100])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 70])
+def test_runtime_takes_every_form(M, K):
+    """The choice of kernel against 64 bits: weights that were bound, plain ones, results that come as planes or go into a given
+    tensor, rows with a stride, sizes that are no multiples of four (the older kernels), gated and not."""
+    from burn_lm_amd.engine.runtime import Runtime
+    rt = Runtime(torch.float32, "cuda:0")
+    x, w = operands(M, 48, K, pad=0 if K % 4 else 8)
+    for weight in (rt.weight(w), w):
+        check(rt.linear(x, weight), x, w)
+        got = rt.linear(x, weight, partials=True)
+        check(got.sum(0) if got.dim() == 3 else got, x, w)
+        given = torch.full((M, 50), float("nan"), device="cuda")
+        check(rt.linear(x, weight, out=given[:, :48]), x, w)
+        assert bool(given[:, 48:].isnan().all())
+    check(rt.gated_linear(x, rt.weight(w, gated=True)), x, w, gated=True)
+    check(rt.gated_linear(x, w), x, w, gated=True)
+
+
+def test_plan_keeps_its_bounds():
+    from burn_lm_amd.engine.runtime import f32_plan
+    for M in (9, 64, 65, 1000):
+        for N in (1, 64, 5000):
+            for K in (4, 130, 8192):
+                tile, groups, us = f32_plan(M, N, K, 256, planes=True)
+                assert groups == 1 or K // groups >= 128
+                assert f32_plan(M, N, K, 256)[1] == 1 and f32_plan(M, N, K, 256, gated=True)[0][1] == 128 and us > 0
