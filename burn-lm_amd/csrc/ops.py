@@ -118,6 +118,11 @@ _SIGNATURES = {
     "blm_attn_paged": [_c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int,
                        _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int,
                        _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p],
+    "blm_attn_f32_supported": [_c_int, _c_int],
+    "blm_attn_prefill_f32": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int,
+                             _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_void_p],
+    "blm_attn_decode_f32": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int,
+                            _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p],
     "blm_attn_decode": [_c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int,
                         _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int,
                         _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_float, _c_int, _c_void_p],
@@ -409,6 +414,57 @@ def attn_paged(q, q_row_stride, out, positions, token_seq, block_table, kcache, 
           token_seq.data_ptr(), block_table.data_ptr(), block_table.shape[1], kcache.data_ptr(), vcache.data_ptr(),
           page_size, T, nh, nkv, hd, float(scale), int(window), n_splits, _ptr(part_o), _ptr(part_ml),
           _ptr(arrivals if n_splits > 1 else None), _stream())
+    return out
+
+
+def attn_f32_supported(q, q_row_stride, kcache, vcache, hd, page_size):
+    """Whether the float32 matrix-core attention takes this case (else attn_paged does)."""
+    return (q.dtype == kcache.dtype == vcache.dtype == torch.float32 and q_row_stride % 4 == 0
+            and not any(t.data_ptr() % 16 for t in (q, kcache, vcache)) and bool(library().blm_attn_f32_supported(int(hd), int(page_size))))
+
+
+def _attn_f32_check(name, q, q_row_stride, out, kcache, vcache, page_size, nh, nkv, hd):
+    _contig("out", out); _contig("kcache", kcache); _contig("vcache", vcache)
+    if out.shape[1] != nh * hd or out.dtype != torch.float32 or not attn_f32_supported(q, q_row_stride, kcache, vcache, hd, page_size):
+        raise KernelError(f"{name}: out must be float32 [T, heads*head_dim], q and the cache float32 in units of 16 bytes")
+    if q.stride(-1) != 1 or q_row_stride < nh * hd:
+        raise KernelError(f"{name}: q rows must be contiguous and at least heads*head_dim long")
+    _check_planes(name, kcache, vcache, nkv, page_size, hd)
+
+
+def attn_prefill_f32(q, q_row_stride, out, positions, cu_seqlens, block_table, kcache, vcache, page_size, n_seqs, max_new, nh, nkv,
+                     hd, scale, window=0):
+    """Causal float32 attention of packed sequences over their cached keys; arguments as attn_prefill_mfma."""
+    _gpu(q, out, positions, cu_seqlens, block_table, kcache, vcache)
+    _attn_f32_check("attn_prefill_f32", q, q_row_stride, out, kcache, vcache, page_size, nh, nkv, hd)
+    _i32("positions", positions, out.shape[0]); _i32("cu_seqlens", cu_seqlens, n_seqs + 1); _i32("block_table", block_table)
+    if block_table.shape[0] < n_seqs:
+        raise KernelError("attn_prefill_f32: the page table has fewer rows than there are sequences")
+    _call("blm_attn_prefill_f32", q.data_ptr(), q_row_stride, out.data_ptr(), positions.data_ptr(), cu_seqlens.data_ptr(),
+          block_table.data_ptr(), block_table.shape[1], kcache.data_ptr(), vcache.data_ptr(), int(n_seqs), int(max_new), nh, nkv, hd,
+          float(scale), int(window), _stream())
+    return out
+
+
+def attn_decode_f32(q, q_row_stride, out, positions, token_seq, block_table, kcache, vcache, page_size, nh, nkv, hd, scale, window=0,
+                    n_splits=1):
+    """Float32 attention of one token per row over its sequence's cached keys; arguments as attn_paged."""
+    _gpu(q, out, positions, token_seq, block_table, kcache, vcache)
+    _attn_f32_check("attn_decode_f32", q, q_row_stride, out, kcache, vcache, page_size, nh, nkv, hd)
+    T = out.shape[0]
+    _i32("positions", positions, T); _i32("token_seq", token_seq, T); _i32("block_table", block_table)
+    n_splits = max(1, int(n_splits))
+    part_o = part_ml = arrivals = None
+    if n_splits > 1:
+        arrivals = arrival_counters(out.device)
+        if T * nh > arrivals.numel():
+            n_splits = 1      # more (token, head) pairs than counters: enough parallel work without cutting
+        else:
+            part_o = torch.empty(T * nh * n_splits * hd, dtype=torch.float32, device=out.device)
+            part_ml = torch.empty(T * nh * n_splits * 2, dtype=torch.float32, device=out.device)
+    _call("blm_attn_decode_f32", q.data_ptr(), q_row_stride, out.data_ptr(), positions.data_ptr(), token_seq.data_ptr(),
+          block_table.data_ptr(), block_table.shape[1], kcache.data_ptr(), vcache.data_ptr(), T, nh, nkv, hd, float(scale), int(window),
+          n_splits, _ptr(part_o), _ptr(part_ml), _ptr(arrivals if n_splits > 1 else None), _stream())
     return out
 
 

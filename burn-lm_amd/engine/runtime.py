@@ -87,13 +87,14 @@ def rows_plan(N, K, compute_units):
 # latency shows), and per step and block where blocks share a unit (the matrix instructions' rate).  Measured with 17 to
 # 2,048 rows at [3072, 2048], [2048, 2048], [16384, 2048], [2048, 8192], [5000, 1416].
 F32_STEP_US = {(128, 128): (2.33, 2.0), (128, 64): (1.25, 1.0), (64, 128): (1.2, 1.0), (64, 64): (0.7, 0.5)}
+F32_SHARE_US = 0.1
 F32_SKINNY_MAX_ROWS = 16
 F32_SKINNY_GROUP_K = 2048
 
 
 def f32_plan(M, N, K, compute_units, planes=False, gated=False):
     """(tile, groups of K, microseconds) of ops.gemm_f32 that a sum of its parts' costs finds fastest: every unit works through
-    its share of the blocks, and every plane of partial products is written once and read once by the norm that adds it.
+    its share of the blocks, and every plane of partial products is read once by the norm that adds it.
     Against the best tile and groups of the sweep the choice is within 6 % from 250 rows on and within 20 % below."""
     best = None
     for (bm, bn), (alone, shared) in F32_STEP_US.items():
@@ -105,7 +106,7 @@ def f32_plan(M, N, K, compute_units, planes=False, gated=False):
                 continue
             steps = -(-K // groups // 32)
             per_unit = -(-tiles * groups // compute_units)
-            us = 3.0 + steps * max(alone, per_unit * shared) + (M * N * groups * 8 / 4e6 if groups > 1 else 0.0)
+            us = 3.0 + steps * max(alone, per_unit * shared + F32_SHARE_US) + (M * N * groups * 4 / 5e6 if groups > 1 else 0.0)
             if best is None or us < best[2] * 0.999:
                 best = ((bm, bn), groups, us)
     return best

@@ -61,6 +61,18 @@ def decode_splits(pages: int, blocks: int, head_dim: int, compute_units: int = 2
     return max(1, n)
 
 
+def decode_splits_f32(pages: int, blocks: int, head_dim: int, compute_units: int = 256) -> int:
+    """The same for float32 (ops.attn_decode_f32): a block's eight wavefronts take a page each, and a page takes one about
+    5 us (8 for wide heads), most of it the fetch's latency and the products of sixteen columns of which a group fills few;
+    the merge takes 2.  So pieces of three pages (two for wide heads), as long as every block has a compute unit to
+    itself; never more than 16 (us per call in pieces of the rule / whole, 32 heads of 64 in 8 groups: 8 pages at batch 1 11.1 / 12.2,
+    at batch 8 12.3 / 13.3; 12 pages at batch 8 13.1 / 17.5, at batch 16 18.1 / 22.9; 50 pages at batch 16 in two 48.4, in four
+    57.4; 24 heads of 128: 8 pages at batch 8 17.3 / 25.1)."""
+    if pages <= 4 and head_dim <= 64:
+        return 1
+    return max(1, min(pages // (3 if head_dim <= 64 else 2), compute_units // max(1, blocks), 16))
+
+
 class Attention(Mixer):
     """params: width, heads, kv_heads, head_dim, scale, window (0 = all keys), position (the
     position-encoding object, given by the model builder).  names: q, k, v, o."""
@@ -138,6 +150,16 @@ class Attention(Mixer):
             rt.ops.attn_prefill_mfma(qkv, qkv.shape[1], out, step.positions, step.cu_seqlens, table, view.k, view.v,
                                      view.page_size, step.n_seqs, step.max_new, nh, nkv, hd, self.scale, self.window,
                                      queries=queries)
+        elif rt.ops.attn_f32_supported(qkv, qkv.shape[1], view.k, view.v, hd, view.page_size) and qkv.shape[0] <= 65535:
+            if step.max_new == 1:
+                span = step.max_len_after if not self.window else min(step.max_len_after, self.window + view.page_size)
+                blocks = qkv.shape[0] * nkv * ((nh // nkv + 15) // 16)
+                n_splits = decode_splits_f32((span + view.page_size - 1) // view.page_size, blocks, hd, rt.compute_units)
+                rt.ops.attn_decode_f32(qkv, qkv.shape[1], out, step.positions, step.token_seq, table, view.k, view.v, view.page_size,
+                                       nh, nkv, hd, self.scale, self.window, n_splits)
+            else:
+                rt.ops.attn_prefill_f32(qkv, qkv.shape[1], out, step.positions, step.cu_seqlens, table, view.k, view.v,
+                                        view.page_size, step.n_seqs, step.max_new, nh, nkv, hd, self.scale, self.window)
         else:
             # the generic kernel has one wavefront per (token, head); with few tokens over long key
             # ranges the ranges are cut so that the whole chip has work
