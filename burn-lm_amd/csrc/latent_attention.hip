@@ -22,7 +22,8 @@ typedef __attribute__((ext_vector_type(4))) float lat_f32x4;
 // ---------------------------------------------------------------------------------------
 // down [T][ld_down]: R latent lanes then Dr key lanes.  q [T][ld_q], head h at h * (dn + Dr).  cos_sin [positions][half_t]
 // (cos, sin), of which the first rot/2 pairs turn lanes (i, i + rot/2) of the Dr part, or (adjacent) lanes (2i, 2i + 1).
-// qabs [T][H][R + Dr] (float or the cache's type) gets the rotated query parts at lane R.  vcache (may be null):
+// qabs [T][H][q_lanes] (float or the cache's type) gets the rotated query parts at lane q_at (absorbed queries: R + Dr and R;
+// rotated parts alone: Dr and 0).  vcache (may be null):
 // pages [R][page] that receive the latent transposed, for the matrix-core attention.
 // ---------------------------------------------------------------------------------------
 template <typename TA, typename TQ>
@@ -31,7 +32,7 @@ __global__ void latent_write_kernel(const TA* __restrict__ down, int ld_down, co
                                     int half_t, int rot, TQ* __restrict__ qabs, TA* __restrict__ kcache, TA* __restrict__ vcache,
                                     const int* __restrict__ positions, const int* __restrict__ token_seq,
                                     const int* __restrict__ block_table, int table_width, int page_size, int R, int Dr,
-                                    int write_kv, int adjacent) {
+                                    int write_kv, int adjacent, int q_lanes, int q_at) {
   __shared__ float red[17];
   const int t = blockIdx.x;
   const int b = token_seq[t];
@@ -51,7 +52,7 @@ __global__ void latent_write_kernel(const TA* __restrict__ down, int ld_down, co
       const float other = to_float(src[adjacent ? d ^ 1 : (d < half ? d + half : d - half)]);
       v = first ? v * c.x - other * c.y : v * c.x + other * c.y;
     }
-    qabs[((size_t)t * H + h) * (R + Dr) + R + d] = from_float<TQ>(v);
+    qabs[((size_t)t * H + h) * q_lanes + q_at + d] = from_float<TQ>(v);
   }
   const int page = block_table[(size_t)b * table_width + pos / page_size];
   if (!write_kv || page < 0) return;
@@ -85,14 +86,17 @@ __global__ void latent_write_kernel(const TA* __restrict__ down, int ld_down, co
 extern "C" int blm_latent_write(const void* down, int ld_down, const void* q, int ld_q, int dtype, int T, int H, int dn,
                                 const float* norm_w, float eps, const void* cos_sin, int half_t, int rot, void* qabs,
                                 int qabs_dtype, void* kcache, void* vcache, const int* positions, const int* token_seq, const int* block_table,
-                                int table_width, int page_size, int R, int Dr, int write_kv, int adjacent, hipStream_t stream) {
+                                int table_width, int page_size, int R, int Dr, int write_kv, int adjacent, int absorbed,
+                                hipStream_t stream) {
+  const int q_lanes = absorbed ? R + Dr : Dr, q_at = absorbed ? R : 0;
   BLM_REQUIRE(T > 0 && H > 0 && dn >= 0 && R > 0 && Dr >= 0, "latent_write: bad sizes");
   BLM_REQUIRE(rot % 2 == 0 && rot >= 0 && rot <= Dr && rot / 2 <= half_t, "latent_write: %d turning lanes do not fit %d", rot, Dr);
   BLM_REQUIRE(page_size > 0 && table_width > 0 && ld_down >= R + Dr && ld_q >= H * (dn + Dr), "latent_write: bad geometry");
 #define BLM_LW(TA, TQ)                                                                                                  \
   hipLaunchKernelGGL((latent_write_kernel<TA, TQ>), dim3(T), dim3(256), 0, stream, (const TA*)down, ld_down, (const TA*)q, \
                      ld_q, H, dn, norm_w, eps, (const float2*)cos_sin, half_t, rot, (TQ*)qabs, (TA*)kcache, (TA*)vcache,  \
-                     positions, token_seq, block_table, table_width, page_size, R, Dr, write_kv, adjacent)
+                     positions, token_seq, block_table, table_width, page_size, R, Dr, write_kv, adjacent, \
+                     q_lanes, q_at)
   if (dtype == BLM_F32 && qabs_dtype == BLM_F32) BLM_LW(float, float);
   else if (dtype == BLM_BF16 && qabs_dtype == BLM_F32) BLM_LW(bf16, float);
   else if (dtype == BLM_BF16 && qabs_dtype == BLM_BF16) BLM_LW(bf16, bf16);

@@ -94,7 +94,10 @@ _SIGNATURES = {
     "blm_xielu": [_c_void_p, _c_void_p, _c_int, ctypes.c_longlong, _c_float, _c_float, _c_void_p],
     "blm_latent_write": [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_float, _c_void_p,
                          _c_int, _c_int, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int,
-                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "blm_latent_prompt_supported": [_c_int, _c_int, _c_int, _c_int, _c_int],
+    "blm_latent_prompt_init": [],
+    "blm_latent_prompt": [_c_void_p, _c_int] + [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 5 + [_c_int] * 8 + [_c_float, _c_int, _c_void_p, _c_void_p],
     "blm_latent_attn_mfma": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int,
                              _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_void_p, _c_void_p, _c_int,
                              _c_void_p, _c_void_p],
@@ -1053,12 +1056,14 @@ def latent_write(down, q, norm_w, eps, cos_sin, rot, qabs, kcache, step, block_t
     (norm_w, eps), the first `rot` of the Dr key lanes are turned by the token's position (pairs half of rot
     apart, or adjacent lanes 2i and 2i + 1; cos_sin float32 [positions, n, 2]), and the row [latent | key lanes] goes into the token's place of the
     key pages [pages, 1, page, R + Dr].  The queries' Dr lanes are turned alike into qabs[:, :, R:] (float32
-    [T, H, R + Dr], or the cache's dtype).  vcache: pages [pages, 1, R, page] that get the latent transposed."""
+    [T, H, R + Dr], or the cache's dtype; or qabs [T, H, Dr]: the turned lanes alone).  vcache: pages [pages, 1, R, page] that get
+    the latent transposed."""
     _gpu(down, q, norm_w, cos_sin, qabs, kcache, block_table, vcache)
     T = q.shape[0]
     _contig("cos_sin", cos_sin); _contig("kcache", kcache); _contig("qabs", qabs)
     _f32("norm_w", norm_w, R)
-    if qabs.numel() != T * H * (R + Dr) or qabs.dtype not in (torch.float32, kcache.dtype):
+    absorbed = qabs.shape[-1] == R + Dr
+    if qabs.numel() != T * H * qabs.shape[-1] or qabs.shape[-1] not in (R + Dr, Dr) or qabs.dtype not in (torch.float32, kcache.dtype):
         raise KernelError("latent_write: qabs is [T, H, R + Dr] in float32 or the cache's dtype")
     if vcache is not None:
         _contig("vcache", vcache)
@@ -1080,7 +1085,7 @@ def latent_write(down, q, norm_w, eps, cos_sin, rot, qabs, kcache, step, block_t
     _call("blm_latent_write", down.data_ptr(), ld_down, q.data_ptr(), q.stride(0), _code(q), T, H, dn, norm_w.data_ptr(),
           float(eps), cos_sin.data_ptr(), cos_sin.shape[1], rot, qabs.data_ptr(), _code(qabs), kcache.data_ptr(),
           _ptr(vcache), step.positions.data_ptr(), step.token_seq.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size,
-          R, Dr, 1 if write_kv else 0, 1 if adjacent else 0, _stream())
+          R, Dr, 1 if write_kv else 0, 1 if adjacent else 0, 1 if absorbed else 0, _stream())
 
 
 def rmsnorm_rows(x, w, eps, out):
@@ -1161,6 +1166,53 @@ def latent_attn(qabs, olat, kcache, step, block_table, page_size, H, R, Dr, scal
           step.token_seq.data_ptr(), block_table.data_ptr(), block_table.shape[1], kcache.data_ptr(), page_size, T, H, R,
           Dr, float(scale), n_splits, _ptr(part_o), _ptr(part_ml), _ptr(arrivals), int(window), _ptr(sinks), _stream())
     return olat
+
+
+def latent_prompt_supported(dtype, R, Dn, Dr, Dv, page_size=64):
+    """Whether prompts may run with expanded keys and values (latent_prompt)."""
+    return dtype == torch.bfloat16 and bool(library().blm_latent_prompt_supported(int(R), int(Dn), int(Dr), int(Dv), int(page_size)))
+
+
+_latent_prompt_ready = set()
+
+
+def latent_prompt_init(device=None):
+    """Once per device, outside any stream capture, before the first latent_prompt (its pages take more shared memory than a
+    kernel gets without asking)."""
+    index = torch.device(device or "cuda").index
+    index = torch.cuda.current_device() if index is None else index
+    if index not in _latent_prompt_ready:
+        with torch.cuda.device(index):
+            _call("blm_latent_prompt_init")
+        _latent_prompt_ready.add(index)
+
+
+def latent_prompt(q, q_turned, out, kcache, w_uk, w_uv, step, block_table, pages_per_seq, H, R, Dn, Dr, Dv, scale, window=0, sinks=None):
+    """Attention of a step's tokens over the latents in the cache, with keys and values expanded per head into workspaces of this
+    call.  q [T, H * (Dn + Dr)] (the Dn lanes are read), q_turned [T, H, Dr] the turned lanes (latent_write), key pages
+    [pages, 1, 64, R + Dr], w_uk [H * Dn, R], w_uv [H * Dv, R], out [T, H * Dv], all bfloat16; pages_per_seq: pages that
+    cover every sequence's length."""
+    _gpu(q, q_turned, out, kcache, w_uk, w_uv, block_table, sinks)
+    latent_prompt_init(q.device)
+    T = q.shape[0]
+    for name, t, shape in (("q_turned", q_turned, (T, H, Dr)), ("out", out, (T, H * Dv)), ("w_uk", w_uk, (H * Dn, R)), ("w_uv", w_uv, (H * Dv, R))):
+        _contig(name, t)
+        if tuple(t.shape) != shape:
+            raise KernelError(f"latent_prompt: {name} is {tuple(t.shape)}, not {shape}")
+    _contig("kcache", kcache); _i32("block_table", block_table)
+    if any(t.dtype != torch.bfloat16 for t in (q, q_turned, out, kcache, w_uk, w_uv)) or q.stride(1) != 1 or q.shape[1] != H * (Dn + Dr):
+        raise KernelError("latent_prompt: bfloat16 operands, q [T, H * (Dn + Dr)] with contiguous rows")
+    if tuple(kcache.shape[1:]) != (1, 64, R + Dr) or T != step.n_tokens or step.cu_seqlens.numel() < step.n_seqs + 1 \
+            or block_table.shape[0] < step.n_seqs or pages_per_seq * 64 < step.max_len_after:
+        raise KernelError("latent_prompt: the pages or the step's index arrays do not fit")
+    if sinks is not None:
+        _f32("sinks", sinks, H)
+    keys, values = (torch.empty(step.n_seqs * pages_per_seq * H * 64 * d, dtype=torch.bfloat16, device=q.device) for d in (Dn, Dv))
+    _call("blm_latent_prompt", q.data_ptr(), q.stride(0), q_turned.data_ptr(), out.data_ptr(), step.positions.data_ptr(),
+          step.cu_seqlens.data_ptr(), step.lens_after.data_ptr(), block_table.data_ptr(), block_table.shape[1], kcache.data_ptr(),
+          w_uk.data_ptr(), w_uv.data_ptr(), keys.data_ptr(), values.data_ptr(), int(pages_per_seq), step.n_seqs, step.max_new, H, R,
+          Dn, Dr, Dv, float(scale), int(window), _ptr(sinks), _stream())
+    return out
 
 
 def latent_attn_mfma_supported(dtype, R, Dr, page_size=64):

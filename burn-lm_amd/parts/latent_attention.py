@@ -5,7 +5,8 @@
 A head's plain key is ``W_uk c`` and its value ``W_uv c``; score = (q_plain . k_plain + q_rot . k_rot) * scale,
 causal softmax, output projection over the concatenated heads.  Only ``[c | k_rot]`` is cached: the scores are
 computed as ``(W_uk^T q_plain) . c`` and the values applied as ``W_uv (sum_j p_j c_j)``, which is the same
-function, so the cache holds one row of kv_rank + rot_dim lanes per token for all heads and no value pages.
+function, so the cache holds one row of kv_rank + rot_dim lanes per token for all heads and no value pages.  Longer
+prompts in bfloat16 expand the keys and values of the rows they see instead (see ``expands``).
 Rotation: lane i of the first ``rot_dims`` turned lanes pairs with lane i + rot_dims/2 (``pairing="half"``, the
 default), or lane 2i with lane 2i + 1 (``pairing="adjacent"``).
 
@@ -25,6 +26,13 @@ import torch
 from .base import KVNeed, Mixer, TensorSpec
 
 DECODE_BLOCKS_PER_UNIT = 2     # blocks of four (token, head) wavefronts the split decode aims for per compute unit
+# Prompts expand keys and values from this many new tokens per sequence on (us of the whole mixer at width 2048, R = 512, 16
+# heads of 128 + 64 / 128, absorbed / expanded: 32 tokens 92 / 70, behind 1,000 others 357 / 73; 64: 79 / 68; 512: 238 / 89; 2,048:
+# 735 / 151 with a window of 1,024, 971 / 155 without; four sequences of 128: 132 / 85), while the rows that the page tables can
+# name are at most so many, or so many times the step's tokens (the workspaces hold a key and a value per head for each: 8 KB a
+# row at 16 heads of 128 lanes).
+EXPAND_MIN_NEW = 32
+EXPAND_MAX_ROWS = (16384, 4)
 MFMA_MAX_PIECES = 64           # most pieces the matrix-core decode cuts a sequence's half pages into
 
 
@@ -106,10 +114,24 @@ class LatentAttention(Mixer):
         H, dn, dv, R = self.H, self.dn, self.dv, self.R
         self.w_uk_t = tensors[n["uk"]].view(H, dn, R).transpose(1, 2).contiguous()   # [H, R, dn]: q_plain -> latent lanes
         self.w_uv = tensors[n["uv"]].view(H, dv, R).contiguous()
+        self.w_uk = tensors[n["uk"]].contiguous()            # [H * dn, R]: latents -> plain keys
         self.w_o = rt.weight(tensors[n["o"]])
         rt.ops.latent_attn_init(rt.device)
         self.use_mfma = (os.environ.get("BURN_LM_AMD_LATENT_MFMA") != "0" and self.scale > 0 and self.w_uk_t.dtype == torch.bfloat16
                          and rt.ops.latent_attn_mfma_supported(rt.dtype, R, self.dr))
+
+        self.can_expand = (self.use_mfma and self.w_uk.dtype == self.w_uv.dtype == torch.bfloat16
+                           and rt.ops.latent_prompt_supported(rt.dtype, R, dn, self.dr, dv))
+        if self.can_expand:
+            rt.ops.latent_prompt_init(rt.device)
+
+    def expands(self, step, q, view):
+        """Whether the step's keys and values are expanded per head instead of absorbing the projections into queries and
+        results: 2 R (dn + dv) operations per row and head once, against 2 (2 R + dr - dn - dr - dv) fewer per query and row."""
+        rows = step.n_seqs * -(-step.max_len_after // 64) * 64
+        return (self.can_expand and step.max_new > 1 and view.v.numel() > 0 and view.page_size == 64
+                and step.n_tokens >= EXPAND_MIN_NEW * step.n_seqs and rows <= max(EXPAND_MAX_ROWS[0], EXPAND_MAX_ROWS[1] * step.n_tokens)
+                and step.n_seqs <= 65535 and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0)
 
     def _matrices(self):
         return [self.w_in.w, self.w_o.w, self.w_uk_t, self.w_uv] + ([self.w_uq.w] if self.q_rank else [])
@@ -126,34 +148,50 @@ class LatentAttention(Mixer):
         return 2 * self.H * (2 * self.R + self.dr) * pairs
 
     def forward(self, x, step, view):
-        qabs, gate = self._project(x, step, view)
-        return self.output(self.attend(qabs, step, view), gate)
+        qd, q, gate = self._inputs(x)
+        if self.expands(step, q, view):
+            rt, H = self.rt, self.H
+            turned = torch.empty(x.shape[0], H, self.dr, dtype=rt.dtype, device=x.device)
+            self._write(qd, q, turned, step, view, view.v)
+            o = torch.empty(x.shape[0], H * self.dv, dtype=rt.dtype, device=x.device)
+            rt.ops.latent_prompt(q, turned, o, view.k, self.w_uk, self.w_uv.view(H * self.dv, self.R), step, view.block_table(step),
+                                 -(-step.max_len_after // 64), H, self.R, self.dn, self.dr, self.dv, self.scale, window=self.window,
+                                 sinks=self.sinks)
+            return self._finish(o, gate)
+        return self.output(self.attend(self._absorb(qd, q, step, view), step, view), gate)
 
     def project(self, x, step, view):
         """The absorbed queries [tokens, heads, kv_rank + rot_dim] of the step's tokens; their latents and turned key
         parts are in the cache afterwards."""
-        return self._project(x, step, view)[0]
+        qd, q, _ = self._inputs(x)
+        return self._absorb(qd, q, step, view)
 
-    def _project(self, x, step, view):
-        """project's queries, and the output gate's columns of the stacked projection (None without a gate)."""
-        rt, ops = self.rt, self.rt.ops
-        H, dn, dr, R = self.H, self.dn, self.dr, self.R
-        T = x.shape[0]
+    def _inputs(self, x):
+        """The stacked projection's rows, the queries before any turning, and the output gate's columns (None without a gate)."""
+        rt = self.rt
+        qd = rt.linear(x, self.w_in)                         # [T, H (dn + dr) or q_rank | R + dr]
+        q = qd[:, :self.n_q]
+        if self.q_rank:
+            cq = rt.ops.rmsnorm_rows(q, self.q_norm_w, self.eps, torch.empty(x.shape[0], self.q_rank, dtype=qd.dtype, device=x.device))
+            q = rt.linear(cq, self.w_uq)
+        return qd, q, (qd[:, self.gate_at:self.gate_at + self.H * self.dv] if self.gated else None)
+
+    def _write(self, qd, q, turned, step, view, vcache):
+        """The turned query lanes into turned ([tokens, heads, kv_rank + rot_dim] or [.., rot_dim]), the step's rows into the cache."""
         if self.borrows == bool(view.store):
             raise ValueError("a layer with a down-projection keeps its own rows, a borrowing layer reads another's")
-        qd = rt.linear(x, self.w_in)                         # [T, H (dn + dr) or q_rank | R + dr]
-        q, down = qd[:, :self.n_q], (None if self.borrows else qd[:, self.down_at:self.down_at + self.down_n])
-        if self.q_rank:
-            cq = rt.ops.rmsnorm_rows(q, self.q_norm_w, self.eps, torch.empty(T, self.q_rank, dtype=qd.dtype, device=x.device))
-            q = rt.linear(cq, self.w_uq)
+        down = None if self.borrows else qd[:, self.down_at:self.down_at + self.down_n]
+        self.rt.ops.latent_write(down, q, self.norm_w, self.eps, self.position.table, self.rot, turned, view.k, step,
+                                 view.block_table(step), view.page_size, self.H, self.dn, self.R, self.dr, write_kv=view.store,
+                                 vcache=vcache if view.store else None, adjacent=self.adjacent)
+
+    def _absorb(self, qd, q, step, view):
+        rt, H, dn, dr, R, T = self.rt, self.H, self.dn, self.dr, self.R, q.shape[0]
         mfma = self.use_mfma and view.v.numel() > 0 and view.page_size == 64
-        qabs = torch.empty(T, H, R + dr, dtype=rt.dtype if mfma else torch.float32, device=x.device)
-        ops.latent_write(down, q, self.norm_w, self.eps,
-                         self.position.table, self.rot, qabs, view.k, step, view.block_table(step), view.page_size, H, dn,
-                         R, dr, write_kv=view.store, vcache=view.v if mfma and view.store else None,
-                         adjacent=self.adjacent)
-        ops.head_project(q, dn + dr, self.w_uk_t, qabs.view(T, H * (R + dr)), R + dr)
-        return qabs, (qd[:, self.gate_at:self.gate_at + H * self.dv] if self.gated else None)
+        qabs = torch.empty(T, H, R + dr, dtype=rt.dtype if mfma else torch.float32, device=q.device)
+        self._write(qd, q, qabs, step, view, view.v if mfma else None)
+        rt.ops.head_project(q, dn + dr, self.w_uk_t, qabs.view(T, H * (R + dr)), R + dr)
+        return qabs
 
     def attend(self, qabs, step, view):
         """Every (token, head)'s weighted sum of the latents it sees -> float32 [tokens, heads, kv_rank]."""
@@ -186,6 +224,9 @@ class LatentAttention(Mixer):
         T = olat.shape[0]
         o = torch.empty(T, self.H * self.dv, dtype=rt.dtype, device=olat.device)
         rt.ops.head_project(olat.view(T, self.H * self.R), self.R, self.w_uv, o, self.dv)
+        return self._finish(o, gate)
+
+    def _finish(self, o, gate):
         if gate is not None:
-            rt.ops.sigmoid_gate(o, gate)
-        return rt.linear(o, self.w_o, partials=True)
+            self.rt.ops.sigmoid_gate(o, gate)
+        return self.rt.linear(o, self.w_o, partials=True)
