@@ -10,7 +10,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 42
+ABI_VERSION = 43
 _lib = None
 _lock = threading.Lock()
 
@@ -51,6 +51,7 @@ _SIGNATURES = {
                      _c_void_p, _c_int, _c_void_p],
     "blm_head_gate": [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_map_difference": [_c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_void_p],
+    "blm_moe_grouped": [_c_void_p, _c_int] + [_c_void_p] * 3 + [_c_int] + [_c_void_p] * 4 + [_c_int] * 5 + [_c_void_p],
     "blm_moe_table": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_int, _c_int, _c_void_p],
     "blm_sigmoid_gate": [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_gelu_glu": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
@@ -1544,6 +1545,32 @@ def moe_gate(gate_up, weights, out, n_experts, expert_inner):
     _call("blm_moe_gate", gate_up.data_ptr(), weights.data_ptr(), out.data_ptr(), _code(out), T, I, n_experts,
           expert_inner, _stream())
     return out
+
+
+MOE_GROUPED_STEP, MOE_GROUPED_EXPERTS, MOE_GROUPED_TOP = 64, 256, 64
+
+
+def moe_grouped(x, w_gate_up, w_down, weights, n_experts, top):
+    """float32 planes [top, T, D] whose sum is ``sum_e weights[t, e] * W_down_e (silu(W_gate_e x) * (W_up_e x))``: every token
+    by its own experts only (those with a weight that is not zero, at most `top` of a token).  bfloat16 x [T, D], w_gate_up
+    [2 E f, D] (the experts' gates, then their ups), w_down [D, E f]; weights float32 [T, E + 1] (the last column is not read)."""
+    _gpu(x, w_gate_up, w_down, weights)
+    T, D = x.shape
+    f = w_down.shape[1] // n_experts
+    for name, t in (("x", x), ("w_gate_up", w_gate_up), ("w_down", w_down)):
+        _contig(name, t)
+        if t.dtype != torch.bfloat16:
+            raise KernelError(f"moe_grouped: {name} must be bfloat16")
+    _f32("weights", weights, T * (n_experts + 1))
+    if tuple(w_gate_up.shape) != (2 * n_experts * f, D) or tuple(w_down.shape) != (D, n_experts * f):
+        raise KernelError("moe_grouped: w_gate_up [2 E f, D], w_down [D, E f]")
+    planes = torch.empty(top, T, D, dtype=torch.float32, device=x.device)
+    lists = torch.empty(n_experts * T + n_experts, dtype=torch.int32, device=x.device)
+    act = torch.empty(T * top, f, dtype=x.dtype, device=x.device)
+    _call("blm_moe_grouped", x.data_ptr(), D, w_gate_up.data_ptr(), w_down.data_ptr(), weights.data_ptr(), n_experts + 1,
+          planes.data_ptr(), lists.data_ptr(), lists.data_ptr() + 4 * n_experts * T, act.data_ptr(), T, D, n_experts, f, top,
+          _stream())
+    return planes
 
 
 def moe_route_grouped(logits, correction, n_experts, n_identity, groups, keep, top, weights, score="softmax", renormalize=True):

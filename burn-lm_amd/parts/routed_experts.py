@@ -2,24 +2,38 @@
 with the largest router logits ``W_router x + b``, weighted by the softmax over the chosen logits only; a shared
 expert of the same form may run for every token, times ``sigmoid(W_sg x)`` (one number per token).
 
-The router's logits, the choice and the weights are float32.  All experts run as ONE stacked product: their gate
-and up projections are the rows of one matrix, their down projections the columns of another, and every expert's
+The router's logits, the choice and the weights are float32.  In steps of few rows all experts run as ONE stacked product:
+their gate and up projections are the rows of one matrix, their down projections the columns of another, and every expert's
 gated activations are multiplied by the token's weight for that expert (zero for experts it did not choose)
 before the one down projection, which so adds the chosen experts' outputs up.  That computes every expert for
-every token: the same weights are read as in a batch that uses every expert, nothing depends on which tokens
-share a step, and no step shape depends on the routing, so steps replay from recorded graphs."""
+every token, and reads the same weights as a batch that uses every expert.
+
+In steps of many rows of experts without clamps and without a shared one, every token goes through its own experts only
+(``ops.moe_grouped``; see ``_grouped`` for where): lists of every expert's tokens are made on the device, and the launches'
+sizes come from the number of rows alone.  Either way a token's result does not depend on which tokens share its step
+(beyond the number of rows), and no step shape depends on the routing, so steps replay from recorded graphs."""
 from __future__ import annotations
 
 import torch
 
 from .base import FeedForward, TensorSpec, Term
 
+# From how many rows on, and at how many times fewer products (tiles' padding counted, half a tile for each expert), every
+# token runs through its own experts only.  Measured, us for the whole feed-forward behind the router, all experts / own ones
+# (experts, chosen, inner, width): 16, 4, 512, 2048 at 256 rows 59.6 / 54.6, 512 rows 67.7 / 55.5, 2,048 rows 178 / 112, 8,192
+# rows 612 / 336; 128, 8, 128, 1024 at 256 rows 50.7 / 68.6, 512 rows 75.6 / 73.0, 2,048 rows 226 / 99; 16, 2, 256, 2048 at 512
+# rows 46.4 / 46.7, 2,048 rows 95 / 58.  With less than half the products saved nothing is won: 4, 2, 1024, 1024 (1.9 times
+# fewer) at 4,096 rows 112.6 / 107.5, and a plane more for the next norm; 4, 3, 512, 1024 (1.3 times) 65.4 / 79.6.
+GROUPED_MIN_ROWS = 512
+GROUPED_MIN_GAIN = 2
+GROUPED_TILE = 256
 
 class RoutedExperts(FeedForward):
     """params: width, experts, top, expert_inner, shared_inner (0: no shared expert).
     names: router, router_bias, e<i>.gate / e<i>.up / e<i>.down for every expert, and with a shared expert
     shared.gate, shared.up, shared.down, shared.sg."""
     graph_safe = True
+    clamped = False
 
     def tensor_specs(self):
         p, n = self.params, self.names
@@ -64,7 +78,11 @@ class RoutedExperts(FeedForward):
         return sum(w.w.numel() * w.w.element_size() for w in (self.w_gate_up, self.w_down, self.w_router))
 
     def step_flops(self, rows):
-        return 2 * rows * sum(w.w.numel() for w in (self.w_gate_up, self.w_down, self.w_router))
+        return self._expert_flops(rows) + 2 * rows * self.w_router.w.numel()
+
+    def _expert_flops(self, rows):
+        flops = 2 * rows * (self.w_gate_up.w.numel() + self.w_down.w.numel())
+        return flops * self.top // self.E if self._grouped(rows) else flops
 
     def route(self, x):
         """float32 [tokens, experts + 1]: every expert's weight for every token (zero if not chosen), and the shared
@@ -74,16 +92,31 @@ class RoutedExperts(FeedForward):
         weights = torch.empty(x.shape[0], self.E + 1, dtype=torch.float32, device=x.device)
         return rt.ops.moe_route(logits, self.router_bias, self.E, self.top, self.E if self.s else -1, weights)
 
-    def forward(self, x, step):
-        rt = self.rt
-        weights = self.route(x)
+    def _mix(self, x, weights):
+        """The experts' results for [tokens, width] by the weights of `route`, without clamps."""
+        rt, ops = self.rt, self.rt.ops
+        if self._grouped(x.shape[0]):
+            return ops.moe_grouped(x, self.w_gate_up.w, self.w_down.w, weights, self.E, self.top)
         gu = rt.linear(x, self.w_gate_up)
         act = torch.empty(x.shape[0], self.inner, dtype=gu.dtype, device=x.device)
-        return rt.linear(rt.ops.moe_gate(gu, weights, act, self.E, self.f), self.w_down, partials=True)
+        return rt.linear(ops.moe_gate(gu, weights, act, self.E, self.f), self.w_down, partials=True)
+
+    def _grouped(self, T):
+        """Whether in a step of T rows every token goes through its own experts only (rather than all through all)."""
+        ops, gu, down = self.rt.ops, self.w_gate_up.w, self.w_down.w
+        D = gu.shape[1]
+        return (self.rt.dtype == gu.dtype == down.dtype == torch.bfloat16 and self.s == 0 and not self.clamped and T >= GROUPED_MIN_ROWS
+                and self.f % ops.MOE_GROUPED_STEP == 0 and D % ops.MOE_GROUPED_STEP == 0
+                and self.E <= ops.MOE_GROUPED_EXPERTS and self.top <= ops.MOE_GROUPED_TOP and self.top <= self.E
+                and max(gu.numel(), T * D, T * self.top) < 2 ** 30
+                and T * self.E >= GROUPED_MIN_GAIN * (T * self.top + GROUPED_TILE // 2 * self.E))
+
+    def forward(self, x, step):
+        return self._mix(x, self.route(x))
 
 
 class GroupedRoutedExperts(RoutedExperts):
-    """The same stacked experts behind another router: the scores are the softmax of ``W_router x`` over all experts;
+    """The same experts behind another router: the scores are the softmax of ``W_router x`` over all experts;
     the choice goes by ``score + correction`` (a stored vector), only among the experts of the ``keep`` best of
     ``groups`` equal groups of neighbouring experts (a group ranks by its largest corrected score); the ``top`` chosen
     experts' weights are their scores (without the correction) over the sum of the chosen scores.  The last
@@ -169,13 +202,13 @@ class GroupedRoutedExperts(RoutedExperts):
     def forward_terms(self, x, step):
         rt = self.rt
         weights = self.route(x)
-        gu = rt.linear(x, self.w_gate_up)
-        act = torch.empty(x.shape[0], self.inner, dtype=gu.dtype, device=x.device)
         if self.clamped:
+            gu = rt.linear(x, self.w_gate_up)
+            act = torch.empty(x.shape[0], self.inner, dtype=gu.dtype, device=x.device)
             rt.ops.moe_gate_clamped(gu, weights, act, self.E, self.f, self.limit, self.alpha, self.shared_limit)
+            terms = [Term(rt.linear(act, self.w_down, partials=True))]
         else:
-            rt.ops.moe_gate(gu, weights, act, self.E, self.f)
-        terms = [Term(rt.linear(act, self.w_down, partials=True))]
+            terms = [Term(self._mix(x, weights))]
         if self.I:
             terms.append(Term(x, 1.0, weights[:, self.E]))
         return terms
@@ -190,7 +223,7 @@ class GroupedRoutedExperts(RoutedExperts):
 
 
 class TableExperts(RoutedExperts):
-    """The same stacked experts without a router: a stored table ``[vocab, top]`` names every token id's experts (the
+    """The same experts without a router: a stored table ``[vocab, top]`` names every token id's experts (the
     entries of a row differ), each with the weight ``1 / top``.  The step's token ids are read on the device, also those
     that a decode step's host has not seen yet.
 
@@ -226,12 +259,10 @@ class TableExperts(RoutedExperts):
         return sum(w.w.numel() * w.w.element_size() for w in (self.w_gate_up, self.w_down)) + 4 * self.top * rows
 
     def step_flops(self, rows):
-        return 2 * rows * sum(w.w.numel() for w in (self.w_gate_up, self.w_down))
+        return self._expert_flops(rows)
 
     def forward(self, x, step):
         rt = self.rt
         weights = torch.empty(x.shape[0], self.E + 1, dtype=torch.float32, device=x.device)
         rt.ops.moe_table(self.table, step.token_ids, weights, self.E, step.token_source)
-        gu = rt.linear(x, self.w_gate_up)
-        act = torch.empty(x.shape[0], self.inner, dtype=gu.dtype, device=x.device)
-        return rt.linear(rt.ops.moe_gate(gu, weights, act, self.E, self.f), self.w_down, partials=True)
+        return self._mix(x, weights)

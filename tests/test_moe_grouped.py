@@ -1,0 +1,109 @@
+"""Experts of many rows: every token through its own experts only, against 64 bits and against all through all.
+
+The bound: a token's gated activations are rounded to bfloat16 once (2^-9 of their size each) and all sums are float32, so a
+result is off by at most 2^-9 times the sum of its products' sizes, and as much again for the float32 sums of up to 2,048."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -8
+
+
+def choices(T, E, top, g, kind):
+    w = torch.zeros(T, E + 1)
+    if kind == "one":                                    # every token the same experts: the others have no rows
+        idx = torch.arange(top).expand(T, top)
+    else:
+        idx = torch.rand(T, E, generator=g).argsort(1)[:, :top]
+    w.scatter_(1, idx, torch.rand(T, top, generator=g) + 0.1)
+    if kind == "missing":                                # tokens with fewer experts, or none
+        w[:, :E][torch.rand(T, E, generator=g) < 0.4] = 0
+        w[T // 2] = 0
+    w[:, E] = 7.0
+    return w
+
+
+@pytest.mark.parametrize("kind", ["all", "one", "missing"])
+@pytest.mark.parametrize("T,E,top,f,D", [(1, 2, 1, 64, 64), (130, 3, 2, 64, 192), (257, 16, 4, 192, 128), (1100, 5, 5, 128, 320),
+                                         (300, 128, 8, 64, 64)])
+def test_kernels(T, E, top, f, D, kind):
+    from burn_lm_amd.csrc import ops
+    g = torch.Generator().manual_seed(T + E)
+    x, gu, down = (torch.randn(*s, generator=g).mul_(s[1] ** -0.5 if s[0] != T else 1).bfloat16()
+                   for s in ((T, D), (2 * E * f, D), (D, E * f)))
+    w = choices(T, E, top, g, kind)
+    y = ops.moe_grouped(x.cuda(), gu.cuda(), down.cuda(), w.cuda(), E, top)
+    assert y.shape == (top, T, D)
+    both = x.double() @ gu.double().t()
+    act = torch.nn.functional.silu(both[:, :E * f]) * both[:, E * f:] * w[:, :E].double().repeat_interleave(f, 1)
+    want, bound = act @ down.double().t(), EPS * (act.abs() @ down.double().abs().t()) + 1e-6
+    assert ((y.double().sum(0).cpu() - want).abs() <= bound).all()
+    # a token's result does not depend on the others, nor on their number
+    rows = torch.randperm(T, generator=g)[: T // 2 + 1]
+    again = ops.moe_grouped(x[rows].cuda(), gu.cuda(), down.cuda(), w[rows].contiguous().cuda(), E, top)
+    assert torch.equal(again, y[:, rows.cuda()])
+
+
+def test_weights_that_are_no_numbers():
+    from burn_lm_amd.csrc import ops
+    T, E, top, f, D = 150, 4, 2, 64, 64
+    g = torch.Generator().manual_seed(0)
+    x, gu, down = (torch.randn(*s, generator=g).bfloat16().cuda() for s in ((T, D), (2 * E * f, D), (D, E * f)))
+    w = choices(T, E, top, g, "all")
+    plain = ops.moe_grouped(x, gu, down, w.cuda(), E, top)
+    w[5] = float("nan")
+    y = ops.moe_grouped(x, gu, down, w.cuda(), E, top)
+    others = torch.arange(T) != 5
+    assert y[:, 5].isnan().all() and torch.equal(y[:, others.cuda()], plain[:, others.cuda()])
+
+
+def test_refusals():
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.csrc.ops import KernelError
+    x, gu, down, w = (torch.zeros(*s, dtype=torch.bfloat16, device="cuda") for s in ((4, 64), (256, 64), (64, 128), (4, 3)))
+    for bad in (dict(x=x.float()), dict(gu=gu[:128]), dict(down=down[:32]), dict(weights=w), dict(top=3), dict(x=x[:, :32].contiguous())):
+        a = dict(x=x, gu=gu, down=down, weights=w.float(), top=2) | bad
+        with pytest.raises(KernelError):
+            ops.moe_grouped(a["x"], a["gu"], a["down"], a["weights"], 2, a["top"])
+
+
+@pytest.mark.parametrize("kind", ["router", "groups", "table"])
+def test_parts_take_either_way(kind, monkeypatch):
+    """A step of many rows through the parts, against the same step with every expert for every token: that form rounds gates,
+    ups and activations to bfloat16 (three times 2^-9), this one the activations once."""
+    import burn_lm_amd.parts.routed_experts as RE
+    from burn_lm_amd.engine.runtime import Runtime
+    rt, g = Runtime(), torch.Generator().manual_seed(3)
+    T, D, E, top, f = 700, 128, 8, 2, 64
+    names = {n: n for n in ["router", "router_bias", "correction", "table"] + [f"e{e}.{r}" for e in range(E) for r in ("gate", "up", "down")]}
+    n_router = E + 2 if kind == "groups" else E
+    t = {f"e{e}.{r}": (torch.randn(*((D, f) if r == "down" else (f, D)), generator=g) * D ** -0.5).bfloat16().cuda()
+         for e in range(E) for r in ("gate", "up", "down")}
+    t["router"] = torch.randn(n_router, D, generator=g).bfloat16().cuda()
+    t["router_bias"], t["correction"] = torch.randn(E, generator=g).cuda(), torch.randn(n_router, generator=g).cuda()
+    t["table"] = torch.rand(50, E, generator=g).argsort(1)[:, :top].int().cuda()
+    params = dict(width=D, experts=E, top=top, expert_inner=f, vocab=50, identity=2)
+    part = dict(router=RE.RoutedExperts, groups=RE.GroupedRoutedExperts, table=RE.TableExperts)[kind](params, names)
+    part.bind(t, rt)
+
+    class Step:
+        token_ids = torch.randint(-1, 50, (T,), generator=g).int().cuda()     # -1: a row of no token
+        token_source = None
+    x = torch.randn(T, D, generator=g).bfloat16().cuda()
+    add = lambda terms: sum((y.y.double().sum(0) if y.y.dim() == 3 else y.y.double()) * (1 if y.row is None else y.row.double()[:, None]) for y in terms)
+    assert part._grouped(T)
+    terms = part.forward_terms(x, Step)
+    assert terms[0].y.shape == (top, T, D)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = part.forward_terms(x, Step)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded[0].y, terms[0].y)
+    monkeypatch.setattr(RE, "GROUPED_MIN_ROWS", T + 1)
+    assert not part._grouped(T)
+    want, got = add(part.forward_terms(x, Step)), add(terms)
+    assert (got - want).norm() <= 3 * 2 ** -9 * want.norm()
+    if kind == "table":
+        assert got[Step.token_ids < 0].abs().max() == 0
