@@ -10,6 +10,8 @@
 // Measured (us, 2,048 tokens, 16 experts of 512 at width 2048, 4 chosen; before: the stacked products and the gating pass):
 // gate/up with gating 122 -> 61, down 77 -> 41, lists 6.5.  Tried: 128 x 128 tiles, two blocks a unit (stages of 32: 70 and 43),
 // the compiler's own order of reads, loads and products (72 and 44), four wavefronts of 128 x 64 (83 and 54).
+#include <type_traits>
+
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 mg_bf16x8;
@@ -163,16 +165,16 @@ __global__ void __launch_bounds__(64 * MG_WAVES, 2)
   };
   // Half a stage: its eight products; in between the next half's eight pieces from the shared memory and half the loads of
   // another stage.
-  auto work = [&](const Pieces& now, Pieces& next, int next_buf, int next_half, bool loads, int k0, int to, int first_load) {
+  auto work = [&](const Pieces& now, Pieces& next, int next_buf, int next_half, bool loads, int k0, int to, int first_load, bool live) {
 #pragma unroll
     for (int g = 0; g < 8; ++g) {
       if (g < 4) {
-        read(next_buf, next_half, next, g >> 1, g & 1, false);
-        read(next_buf, next_half, next, g >> 1, g & 1, true);
+        if (live) read(next_buf, next_half, next, g >> 1, g & 1, false);
+        if (live) read(next_buf, next_half, next, g >> 1, g & 1, true);
       } else if (loads && g - 4 < LOADS / 2) {
         fetch(k0, to, first_load + g - 4);
       }
-      multiply(now, g >> 2, (g >> 1) & 1, g & 1);
+      if (live) multiply(now, g >> 2, (g >> 1) & 1, g & 1);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -186,34 +188,44 @@ __global__ void __launch_bounds__(64 * MG_WAVES, 2)
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LOADS + HALF) : "memory");
   else
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      read(0, 0, left, x, i, false);
-      read(0, 0, left, x, i, true);
-    }
   // A stage's buffer is free once all have its second half in registers (the wait and barrier in the middle): the first loads
   // of the stage three behind it go out in the second half, the others in the next stage's first.  The order is held fast:
   // left to itself the compiler reads first and multiplies then, and issues a stage's loads at a stretch, and the matrix cores
   // idle meanwhile.
-  int s = 0, buf = 0, last = 2;               // buffers of stage s and of stage s + 2
-  for (; s + 3 < stages; ++s) {
-    work(left, right, buf, 1, true, (s + 2) * MG_BK, last, HALF);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LOADS) : "memory");
-    last = buf;
-    buf = buf == 2 ? 0 : buf + 1;
-    work(right, left, buf, 0, true, (s + 3) * MG_BK, last, 0);
-  }
-  if (stages >= 3)
+  // Wavefronts whose rows are all behind the end only load: a part of a tile leaves the others the LDS (us, 512 tokens of the
+  // case above: 30.0 -> 26.9 and 17.0 -> 15.7; 1,000 tokens by 8 of 128 experts of 128 at width 1024: 23.0 -> 19.4 and 34.8 ->
+  // 32.7).  Putting the full tiles in front of the parts was slower: an expert's weights are then read twice.
+  auto run = [&](auto live_type) {
+    constexpr bool live = decltype(live_type)::value;
 #pragma unroll
-    for (int i = HALF; i < LOADS; ++i) fetch((stages - 1) * MG_BK, last, i);
-  for (; s < stages; ++s) {
-    work(left, right, buf, 1, false, 0, 0, 0);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    buf = buf == 2 ? 0 : buf + 1;
-    work(right, left, buf, 0, false, 0, 0, 0);      // (behind the last stage: an older one's pieces, not used)
-  }
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (live) read(0, 0, left, x, i, false);
+        if (live) read(0, 0, left, x, i, true);
+      }
+    int s = 0, buf = 0, last = 2;               // buffers of stage s and of stage s + 2
+    for (; s + 3 < stages; ++s) {
+      work(left, right, buf, 1, true, (s + 2) * MG_BK, last, HALF, live);
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LOADS) : "memory");
+      last = buf;
+      buf = buf == 2 ? 0 : buf + 1;
+      work(right, left, buf, 0, true, (s + 3) * MG_BK, last, 0, live);
+    }
+    if (stages >= 3)
+#pragma unroll
+      for (int i = HALF; i < LOADS; ++i) fetch((stages - 1) * MG_BK, last, i);
+    for (; s < stages; ++s) {
+      work(left, right, buf, 1, false, 0, 0, 0, live);
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      buf = buf == 2 ? 0 : buf + 1;
+      work(right, left, buf, 0, false, 0, 0, 0, live);      // (behind the last stage: an older one's pieces, not used)
+    }
+  };
+  if (wm < rows)
+    run(std::integral_constant<bool, true>{});
+  else
+    run(std::integral_constant<bool, false>{});
   // acc[i][j][v]: row wm + 32 i + 8 (v / 4) + 4 hb + v % 4, column wn + 32 j + c
 #pragma unroll
   for (int i = 0; i < 2; ++i)
