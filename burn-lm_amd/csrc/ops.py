@@ -10,7 +10,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 43
+ABI_VERSION = 44
 _lib = None
 _lock = threading.Lock()
 
@@ -167,7 +167,7 @@ _SIGNATURES = {
     "blm_probe_mfma": [_c_int, _c_int, _c_int, _c_void_p, _c_void_p],
     "blm_static_scratch_init": [],
     "blm_argmax_static": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
-    "blm_sample": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_float, _c_float, _c_void_p, _c_void_p,
+    "blm_sample": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_float, _c_float, _c_void_p, _c_void_p, _c_int,
                    _c_void_p],
 }
 
@@ -255,6 +255,7 @@ def _ptr(t):
 
 
 ARRIVAL_COUNTERS = 1 << 16
+ARRIVAL_LINE = 32
 _arrivals = {}
 
 
@@ -271,6 +272,12 @@ def arrival_counters(device):
             raise KernelError("arrival_counters: the first call for a device must come before any graph capture")
         buf = _arrivals[key] = torch.zeros(ARRIVAL_COUNTERS, dtype=torch.int32, device=torch.device("cuda", key))
     return buf
+
+
+def arrival_step(n):
+    """How many counters apart n shared results' counters lie: a line each of the cache where the atomics are done (they queue
+    up there for the line, not for the counter) while the buffer holds as many."""
+    return ARRIVAL_LINE if n * ARRIVAL_LINE <= ARRIVAL_COUNTERS else 1
 
 
 def _check_planes(who, kcache, vcache, nkv, page_size, hd):
@@ -932,7 +939,8 @@ def sample(logits, uniforms, temperature, top_p=1.0, out=None):
     lib = library()
     scratch = torch.empty((int(lib.blm_sample_scratch_bytes(R, V)) + 7) // 8, dtype=torch.int64, device=logits.device)
     _call("blm_sample", logits.data_ptr(), uniforms.data_ptr(), out.data_ptr(), R, V, logits.stride(0),
-          float(temperature), float(top_p), scratch.data_ptr(), counters.data_ptr(), _stream())
+          float(temperature), float(top_p), scratch.data_ptr(), counters.data_ptr(), arrival_step(R),
+          _stream())
     return out
 
 

@@ -193,7 +193,7 @@ __device__ __forceinline__ unsigned long long shfl_down_u64(unsigned long long v
 template <bool VEC>
 __global__ void __launch_bounds__(SMP_THREADS)
     sample_max_kernel(const float* __restrict__ logits, int V, int ld, int slice_len, float* part_max,
-                      SampleRow* rows, unsigned long long* hist, int n_rows, int* counters, int with_hist) {
+                      SampleRow* rows, unsigned long long* hist, int n_rows, int* counters, int counter_step, int with_hist) {
   __shared__ float red[17];
   __shared__ int flag;
   const int row = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x;
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(SMP_THREADS)
   }
   mx = block_max(mx, red);
   if (tid == 0) smp_store(part_max + row * SMP_SLICES + slice, mx);
-  if (!smp_arrive_last(counters + row, &flag, gridDim.x)) return;
+  if (!smp_arrive_last(counters + (size_t)row * counter_step, &flag, gridDim.x)) return;
   float m = tid < (int)gridDim.x ? smp_load(part_max + row * SMP_SLICES + tid) : -INFINITY;
   m = block_max(m, red);
   if (tid == 0) {
@@ -231,7 +231,7 @@ __global__ void __launch_bounds__(SMP_THREADS)
 template <bool VEC, int LEVEL>
 __global__ void __launch_bounds__(SMP_THREADS)
     sample_level_kernel(const float* __restrict__ logits, int V, int ld, int slice_len, float k2, float top_p,
-                        SampleRow* rows, unsigned long long* hist, int n_rows, int* counters) {
+                        SampleRow* rows, unsigned long long* hist, int n_rows, int* counters, int counter_step) {
   __shared__ unsigned long long bins[SMP_BINS];
   __shared__ unsigned long long wave_tot[SMP_WAVES];
   __shared__ unsigned long long chosen_above;
@@ -267,7 +267,7 @@ __global__ void __launch_bounds__(SMP_THREADS)
   unsigned long long* row_hist = hist + ((size_t)LEVEL * n_rows + row) * SMP_BINS;
   for (int b = tid; b < SMP_BINS; b += SMP_THREADS)
     if (bins[b]) __hip_atomic_fetch_add(row_hist + b, bins[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (!smp_arrive_last(counters + row, &flag, gridDim.x)) return;
+  if (!smp_arrive_last(counters + (size_t)row * counter_step, &flag, gridDim.x)) return;
 
   // thread t looks after bins 8 t .. 8 t + 7
   constexpr int PER = SMP_BINS / SMP_THREADS;
@@ -341,7 +341,7 @@ template <bool VEC>
 __global__ void __launch_bounds__(SMP_THREADS)
     sample_pick_kernel(const float* __restrict__ logits, const float* __restrict__ uniforms, int* __restrict__ out, int V,
                        int ld, int slice_len, float k2, int use_tau, const SampleRow* rows, float* chunk_mass,
-                       int* counters) {
+                       int* counters, int counter_step) {
   __shared__ float red[17];
   __shared__ float wave_sums[SMP_WAVES];
   __shared__ float round_sums[SMP_ROUND][SMP_WAVES];
@@ -377,7 +377,7 @@ __global__ void __launch_bounds__(SMP_THREADS)
       smp_store(row_mass + slice * chunks + c0 + tid, t);
     }
   }
-  if (!smp_arrive_last(counters + row, &flag, gridDim.x)) return;
+  if (!smp_arrive_last(counters + (size_t)row * counter_step, &flag, gridDim.x)) return;
 
   // chunks in index order: slice by slice; first their total, then the chunk in which u * total falls
   const int n = gridDim.x * chunks;
@@ -478,12 +478,14 @@ extern "C" long long blm_sample_scratch_bytes(int R, int V) {
 }
 
 // scratch: blm_sample_scratch_bytes(R, V) bytes, 8-byte aligned: three histograms per row, the rows'
-// states, the slices' maxima, the chunks' masses.  counters: R zeroed ints, left zeroed.
+// states, the slices' maxima, the chunks' masses.  counters: R zeroed ints, counter_step apart, left
+// zeroed.
 extern "C" int blm_sample(const float* logits, const float* uniforms, int* out, int R, int V, int ld,
-                          float temperature, float top_p, void* scratch, int* counters, hipStream_t stream) {
+                          float temperature, float top_p, void* scratch, int* counters, int counter_step, hipStream_t stream) {
   BLM_REQUIRE(R > 0 && R <= 65535 && V > 0 && ld >= V, "sample: bad sizes R=%d V=%d ld=%d", R, V, ld);
   BLM_REQUIRE(temperature > 0.f, "sample: temperature must be > 0 (got %g); use argmax for 0", (double)temperature);
   BLM_REQUIRE(top_p > 0.f, "sample: top_p must be > 0 (got %g)", (double)top_p);
+  BLM_REQUIRE(counter_step >= 1, "sample: counters %d apart", counter_step);
   BLM_REQUIRE(scratch != nullptr && ((uintptr_t)scratch % 8) == 0 && counters != nullptr, "sample: scratch and counters needed");
   const int slice_len = sample_slice_len(R, V);
   unsigned long long* hist = reinterpret_cast<unsigned long long*>(scratch);
@@ -497,17 +499,17 @@ extern "C" int blm_sample(const float* logits, const float* uniforms, int* out, 
 #define SMP_LAUNCH(VEC)                                                                                              \
   do {                                                                                                               \
     hipLaunchKernelGGL(sample_max_kernel<VEC>, grid, block, 0, stream, logits, V, ld, slice_len, part_max, rows,     \
-                       hist, R, counters, cut);                                                                      \
+                       hist, R, counters, counter_step, cut);                                                                      \
     if (cut) {                                                                                                       \
       hipLaunchKernelGGL((sample_level_kernel<VEC, 0>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
-                         rows, hist, R, counters);                                                                   \
+                         rows, hist, R, counters, counter_step);                                                     \
       hipLaunchKernelGGL((sample_level_kernel<VEC, 1>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
-                         rows, hist, R, counters);                                                                   \
+                         rows, hist, R, counters, counter_step);                                                     \
       hipLaunchKernelGGL((sample_level_kernel<VEC, 2>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
-                         rows, hist, R, counters);                                                                   \
+                         rows, hist, R, counters, counter_step);                                                     \
     }                                                                                                                \
     hipLaunchKernelGGL(sample_pick_kernel<VEC>, grid, block, 0, stream, logits, uniforms, out, V, ld, slice_len, k2, \
-                       cut, rows, chunk_mass, counters);                                                             \
+                       cut, rows, chunk_mass, counters, counter_step);                                                             \
   } while (0)
   if (vec) SMP_LAUNCH(true);
   else SMP_LAUNCH(false);
