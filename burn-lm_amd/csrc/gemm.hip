@@ -1,11 +1,12 @@
 // Matrix products C[M,N] = A[M,K] * W[N,K]^T (W in checkpoint layout, K contiguous).
 //   gemm_tiled   : any sizes, any mix of float / bf16 operands, float accumulation with plain
-//                  fused multiply-adds.  It is the true 32-bit product of the float path and the
-//                  always-right fallback.  From 32 rows and 32 columns on the multiply-adds are
+//                  fused multiply-adds.  It is the always-right fallback, of the float path too
+//                  (whose products gemm_f32.hip takes where rows and addresses are whole 16-byte
+//                  units).  From 32 rows and 32 columns on the multiply-adds are
 //                  those of the matrix cores' float instruction (v_mfma_f32_32x32x2_f32: float
 //                  operands, float products, float sums, nothing narrowed), which does the same
 //                  arithmetic about five times as fast.
-//   gemv_skinny  : M <= 8 rows (decode).  Streams each weight row once with 16-byte loads;
+//   gemv_skinny  : M <= 8 rows that no packed kernel takes.  Streams each weight row once with 16-byte loads;
 //                  every wavefront owns output columns and reduces over K across its lanes.
 #include "common.h"
 
