@@ -136,7 +136,7 @@ extern "C" int blm_argmax_static(const float* logits, int* out, int R, int V, in
 }
 
 #define SMP_BINS 2048
-#define SMP_SLICES 32      // most blocks per row (fewer when there are many rows)
+#define SMP_SLICES 32      // most blocks per row (fewer when there are many rows or few logits)
 #define SMP_THREADS 256
 #define SMP_CHUNK (SMP_THREADS * 4)   // elements per chunk: four neighbours per thread
 #define SMP_WAVES (SMP_THREADS / BLM_WAVE)
@@ -461,21 +461,26 @@ __global__ void __launch_bounds__(SMP_THREADS)
   }
 }
 
-// Blocks per row.  Measured with the nucleus cut at a vocabulary of 128K (one block of 1024 threads per
-// row took 77 us whatever the number of rows): 32 blocks 42 us for one row, 16 blocks 45 us; 8 rows
-// 51 us with 16 and 55 us with 32; 64 rows 91 us with 16 and 101 us with 4.  Every pass costs
-// about 9 us of launch, coherent round trips and the last block's tail, whatever the slice's length.
-// Those are with the rows' arrival counters side by side: 1,024 blocks then queue up at two cache lines in every pass.  With a
-// line for each, 64 rows of 128K take 75.5 us (90.5 before in the same run), 64 of 1,003 49.4 (66.8), 8 of 128K 46.9 (50.0).
-static int sample_slices(int R) { return R <= 2 ? 32 : 16; }
+// Blocks per row: a slice's own time falls with their number, the device-wide atomics of all rows' blocks (histograms, arrivals)
+// grow with it and with the rows, so the best number goes with sqrt(V / R): the power of two next to sqrt(V / (16 R)).  Us, with
+// the nucleus cut, for 4 / 8 / 16 / 32 blocks (before: 32 for one or two rows, else 16): 128,256 logits: 1 row 77.1 / 59.4 /
+// 49.7 / 48.0, 8 rows 79.8 / 59.8 / 52.7 / 49.4, 32 rows 82.9 / 63.7 / 59.1 / 66.4, 64 rows 99.9 / 79.6 / 79.6 / 98.8, 128 rows
+// 118.2 / 110.3 / 127.1 / 148.5, 512 rows 292 / 330 / 402 / 590; 32,000 logits: 8 rows 47.1 / 43.9 / 44.0 / 46.1, 64 rows 50.5 /
+// 53.3 / 62.1 / 80.4, 512 rows 131 / 168 / 244 / 429.  (64 blocks win nowhere.)  All with a cache line for each row's arrival
+// counter: side by side, 1,024 blocks queue up at two lines in every pass (64 rows of 128K in 16 blocks 90.5 us).
+static int sample_slices(int R, int V) {
+  int n = 4;
+  while (n < SMP_SLICES && 32LL * n * n * R <= V) n *= 2;
+  return n;
+}
 static int sample_slice_len(int R, int V) {
-  const int n = sample_slices(R);
+  const int n = sample_slices(R, V);
   return ((V + n - 1) / n + SMP_CHUNK - 1) / SMP_CHUNK * SMP_CHUNK;
 }
 
 // Bytes of scratch that blm_sample needs for R rows of V logits (see there for the layout).
 extern "C" long long blm_sample_scratch_bytes(int R, int V) {
-  const long long chunks = (long long)sample_slices(R) * (sample_slice_len(R, V) / SMP_CHUNK);
+  const long long chunks = (long long)sample_slices(R, V) * (sample_slice_len(R, V) / SMP_CHUNK);
   return (long long)R * (3 * SMP_BINS * 8 + sizeof(SampleRow) + SMP_SLICES * 4 + chunks * 4);
 }
 
@@ -497,7 +502,7 @@ extern "C" int blm_sample(const float* logits, const float* uniforms, int* out, 
   const float k2 = 1.4426950408889634f / temperature;
   const bool vec = ld % 4 == 0 && ((uintptr_t)logits % 16) == 0;
   const int cut = top_p < 1.0f ? 1 : 0;
-  dim3 grid(sample_slices(R), R), block(SMP_THREADS);
+  dim3 grid(sample_slices(R, V), R), block(SMP_THREADS);
 #define SMP_LAUNCH(VEC)                                                                                              \
   do {                                                                                                               \
     hipLaunchKernelGGL(sample_max_kernel<VEC>, grid, block, 0, stream, logits, V, ld, slice_len, part_max, rows,     \

@@ -954,3 +954,15 @@ def _check_qkv_rope(run, pairing, M, K, nh, nkv, hd):
     out2 = torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda")
     run(dev(x), dev(W), out2, dev(positions), dev(token_seq), dev(perm), dev(cs), kd2, dev(v), page, False)
     assert torch.equal(out2.cpu(), out.cpu()) and bool((kd2.cpu() == 99).all())
+
+
+@pytest.mark.parametrize("V", [1, 5, 1023, 4097, 70001])
+def test_sample_does_not_depend_on_how_rows_are_cut(ops, V):
+    """Different numbers of rows cut the rows into different numbers of slices: every row's draw stays the same."""
+    g = torch.Generator().manual_seed(V)
+    x, u = dev(torch.randn(600, V, generator=g) * 2), dev(torch.rand(600, generator=g))
+    whole = ops.sample(x, u, 0.8, 0.9)
+    for n in (1, 2, 7, 16, 40, 130):
+        assert torch.equal(ops.sample(x[:n], u[:n].clone(), 0.8, 0.9), whole[:n])
+    full = ops.sample(x, u, 0.8, 1.0)
+    assert torch.equal(ops.sample(x[:3], u[:3].clone(), 0.8, 1.0), full[:3])
