@@ -21,6 +21,12 @@ __device__ __forceinline__ lp_f32x16 lp_mfma(lp_u32x4 a, lp_u32x4 b, lp_f32x16 c
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(lp_bf16x8, a), __builtin_bit_cast(lp_bf16x8, b), c, 0, 0, 0);
 }
 
+// acc + both numbers of a pair of bf16, one instruction
+__device__ __forceinline__ float lp_add_pair(uint32_t pair, float acc) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, 0x3f803f80u), acc, false);
+}
+
 __device__ __forceinline__ constexpr int lp_key_of(int row) { return (row & ~12) | ((row & 4) << 1) | ((row & 8) >> 1); }
 template <int LANES>     // lanes of a shared-memory row: 32, 64 or 128
 __device__ __forceinline__ int lp_twist(int row) { return LANES == 128 ? row & 15 : LANES == 64 ? (row >> 1) & 7 : (row >> 2) & 3; }
@@ -231,6 +237,7 @@ __global__ void __launch_bounds__(LP_WAVES* BLM_WAVE, 2)
       blm_swap32(top, a, b);
       const float m_new = blm_max(m, blm_max(a, b) * scale2);
       const float base = m_new == -INFINITY ? 0.f : m_new, keep = __builtin_amdgcn_exp2f(m - base);
+      // the denominator takes the rounded probabilities that the values meet: their roundings then cancel where the values agree
       float sum = 0.f;
       lp_u32x4 p[4];        // probabilities of the lane's eight keys of each sixteen
 #pragma unroll
@@ -238,8 +245,9 @@ __global__ void __launch_bounds__(LP_WAVES* BLM_WAVE, 2)
 #pragma unroll
         for (int v = 0; v < 16; v += 2) {
           const float x = __builtin_amdgcn_exp2f(fmaf(s[t][v], scale2, -base)), y = __builtin_amdgcn_exp2f(fmaf(s[t][v + 1], scale2, -base));
-          sum += x + y;
-          p[t * 2 + v / 8][v % 8 / 2] = f32x2_to_bf16x2_bits(x, y);
+          const uint32_t pair = f32x2_to_bf16x2_bits(x, y);
+          sum = lp_add_pair(pair, sum);
+          p[t * 2 + v / 8][v % 8 / 2] = pair;
         }
       l = l * keep + sum;
       m = m_new;

@@ -69,6 +69,33 @@ def test_kernels(D, DR, R, H, window, sink):
             assert bool(((got[t] - want).abs() <= bound).all()), (b, t, float(((got[t] - want).abs() / bound).max()))
 
 
+@pytest.mark.parametrize("D,DR", [(64, 32), (64, 64), (128, 32), (128, 64)])
+def test_probabilities_add_up_to_one(D, DR):
+    """Every value is one, so every result is: the weights that meet the values and the denominator are the same numbers.  All
+    keys but the first have a probability of just under half a rounding step above a half of the first's; a denominator of
+    unrounded ones would come out 2^-8 too large."""
+    from burn_lm_amd.csrc import ops
+    R, T = 64, 200
+    wk, wv = torch.zeros(D, R), torch.zeros(D, R)
+    wk[0, 1] = wv[:, 0] = 1
+    kc = torch.zeros(4, 1, PAGE, R + DR)
+    kc.view(-1, R + DR)[:T, 0] = 1            # every row's value: ones
+    kc.view(-1, R + DR)[0, 1] = 1             # the first row's key
+    q = torch.zeros(T, D + DR)
+    q[:, 0] = 1
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    b16 = lambda x: x.bfloat16().cuda()
+
+    class step:
+        n_tokens, n_seqs, max_new, max_len_after = T, 1, T, T
+        cu_seqlens, lens_after, positions = i32([0, T]), i32([T]), i32(list(range(T)))
+    out = torch.zeros(T, D, dtype=torch.bfloat16, device="cuda")
+    scale = -math.log(0.5 + 0.97 * EPS)
+    ops.latent_prompt(b16(q), torch.zeros(T, 1, DR, dtype=torch.bfloat16, device="cuda"), out, b16(kc), b16(wk), b16(wv), step, i32([[0, 1, 2, 3]]), 4, 1,
+                      R, D, DR, D, scale)
+    assert bool((out == 1).all()), float(out.min())
+
+
 def small_netanex(window):
     """One layer of differential, latent and gated attention each, sizes that the expanded form takes."""
     moe = dict(kind="moe", expert=dict(ff=32), router=dict(experts=4, top=2))
