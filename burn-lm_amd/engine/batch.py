@@ -3,7 +3,7 @@ kernels need to know about where each token belongs."""
 from __future__ import annotations
 
 from dataclasses import dataclass, field
-from typing import Dict, List, Sequence
+from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
@@ -28,6 +28,10 @@ class Step:
     host_slots: List[int] = field(default_factory=list)
     host_new: List[int] = field(default_factory=list)
     host_image: object = None    # the pinned host buffer the index arrays were copied from
+    # (tokens, sequences, longest sequence) of the recorded shape that the step is, or would be, replayed as; None if it never
+    # is.  A part whose choice between two forms goes by sizes goes by these where they are known, so that the step takes the
+    # same form before its shape is recorded and afterwards.
+    bucket: Optional[Tuple[int, int, int]] = None
     # (rows int32 [tokens], cell int64 [1]) or None.  Where rows[t] >= 0, token t is not token_ids[t] but
     # element rows[t] of the int32 array on the device whose address stands in the cell: a token that a
     # sampler left on the GPU and the host has not read.  Only given to an embedding that has forward_from.

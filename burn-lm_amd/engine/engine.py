@@ -78,7 +78,10 @@ class Engine:
         key = self.graphs.key_for(packed) if self.graphs is not None else None
         logits = self.graphs.run(key, packed) if key is not None else None
         if logits is None:
-            logits = self.model.forward(self.build_step(packed), self.cache)
+            step = self.build_step(packed)
+            if key is not None:
+                step.bucket = self.graphs.sizes(key)
+            logits = self.model.forward(step, self.cache)
             if key is not None:
                 self.graphs.after_eager(key)
         self.cache.advance_step(packed)

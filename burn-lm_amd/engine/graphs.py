@@ -16,7 +16,9 @@ buffers and its share of the graphs' memory pool).
 
 Places of the bucket that nothing fills are padding: padding tokens belong to no sequence (index
 -1), so they write no cache; padding sequences bring no token; their rows are dropped.  The kernels
-compute every row on its own, so padding changes no result.  Only models whose parts all declare
+compute every row on its own, so padding changes no result beyond the order of a product's sums (the number of
+rows chooses its tiles); parts that choose between two forms of a result by the step's sizes go by the bucket's
+sizes before the recording too (``Step.bucket``).  Only models whose parts all declare
 ``graph_safe`` are replayed this way, and no memset node is recorded (buffers are cleared, where
 needed, by kernels).
 """
@@ -73,6 +75,11 @@ def width_bucket(pages: int, max_width: int) -> int:
 _LIB = _core.library
 
 
+def shape_sizes(cache, B: int, T: int, W: int):
+    """(tokens, sequences, longest sequence) that a step of this shape is recorded with."""
+    return T or B, B, min(W * cache.page_size, cache.max_context)
+
+
 class _Captured:
     """One recorded shape: B sequences, T tokens (T = 0: a decode step, one token per sequence),
     page tables W wide."""
@@ -108,11 +115,11 @@ class _Captured:
         cu, after, rows = take(B + 1), take(B), take(B)
         tables = {gi: take(B * W).view(B, W) for gi in range(G)}
         self.src_rows = take(B)
-        span = min(W * cache.page_size, cache.max_context)
+        span = shape_sizes(cache, B, T, W)[2]
         self.step = Step(n_tokens=NT, n_seqs=B, n_wanted=B, token_ids=token_ids, positions=positions,
                          token_seq=token_seq, seq_slots=seq_slots, cu_seqlens=cu, lens_after=after, want_rows=rows,
                          block_tables=tables, max_new=1 if self.decode else T, max_position=span - 1,
-                         max_len_after=span, is_decode=self.decode, host_slots=[], host_new=[])
+                         max_len_after=span, is_decode=self.decode, host_slots=[], host_new=[], bucket=(NT, B, span))
         if self.folded:
             self.step.token_source = (self.src_rows, self.dev[self.cell_at: self.cell_at + 2].view(torch.int64))
         self.fill(None, cache)     # all padding: valid contents while capturing
@@ -204,6 +211,9 @@ class StepGraphs:
                             _BATCH_BUCKETS, len(TOKEN_BUCKETS), _TOKEN_BUCKETS, PROMPT_MAX_SEQS, cache.page_size,
                             cache.table_width, key)
         return None if key[0] < 0 else (key[0], key[1], key[2])
+
+    def sizes(self, key):
+        return shape_sizes(self._engine().cache, *key)
 
     def run(self, key, entries):
         """Replays the step if its shape has been captured; returns None if it must run eagerly

@@ -33,6 +33,11 @@ DECODE_BLOCKS_PER_UNIT = 2     # blocks of four (token, head) wavefronts the spl
 # row at 16 heads of 128 lanes).
 EXPAND_MIN_NEW = 32
 EXPAND_MAX_ROWS = (16384, 4)
+# For a shape that is recorded the bucket's sizes count, against half as many tokens and twice as many rows: sequences and
+# pages are rounded up there, each by less than two times and to powers of two, so every step within the plain bounds stays
+# within these (us of a whole step of two such mixers, absorbed / expanded: 16 sequences of 16 new tokens behind 1,000 others 2,466
+# / 1,251, 4 of 2 behind 1,000 1,271 / 756, 5 of 20 behind 3,500 1,666 / 1,040, one of 64 behind 20,000 2,516 / 1,896).
+EXPAND_BUCKET_SLACK = 2
 MFMA_MAX_PIECES = 64           # most pieces the matrix-core decode cuts a sequence's half pages into
 
 
@@ -128,10 +133,13 @@ class LatentAttention(Mixer):
     def expands(self, step, q, view):
         """Whether the step's keys and values are expanded per head instead of absorbing the projections into queries and
         results: 2 R (dn + dv) operations per row and head once, against 2 (2 R + dr - dn - dr - dv) fewer per query and row."""
-        rows = step.n_seqs * -(-step.max_len_after // 64) * 64
+        bucket = getattr(step, "bucket", None)
+        tokens, seqs, longest = bucket or (step.n_tokens, step.n_seqs, step.max_len_after)
+        slack = EXPAND_BUCKET_SLACK if bucket else 1
+        rows = seqs * -(-longest // 64) * 64
         return (self.can_expand and step.max_new > 1 and view.v.numel() > 0 and view.page_size == 64
-                and step.n_tokens >= EXPAND_MIN_NEW * step.n_seqs and rows <= max(EXPAND_MAX_ROWS[0], EXPAND_MAX_ROWS[1] * step.n_tokens)
-                and step.n_seqs <= 65535 and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0)
+                and tokens * slack >= EXPAND_MIN_NEW * seqs and rows <= max(slack * EXPAND_MAX_ROWS[0], EXPAND_MAX_ROWS[1] * tokens)
+                and seqs <= 65535 and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0)
 
     def _matrices(self):
         return [self.w_in.w, self.w_o.w, self.w_uk_t, self.w_uv] + ([self.w_uq.w] if self.q_rank else [])

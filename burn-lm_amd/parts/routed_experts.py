@@ -92,17 +92,18 @@ class RoutedExperts(FeedForward):
         weights = torch.empty(x.shape[0], self.E + 1, dtype=torch.float32, device=x.device)
         return rt.ops.moe_route(logits, self.router_bias, self.E, self.top, self.E if self.s else -1, weights)
 
-    def _mix(self, x, weights):
+    def _mix(self, x, weights, step):
         """The experts' results for [tokens, width] by the weights of `route`, without clamps."""
         rt, ops = self.rt, self.rt.ops
-        if self._grouped(x.shape[0]):
+        bucket = getattr(step, "bucket", None)
+        if self._grouped(bucket[0] if bucket else x.shape[0]):
             return ops.moe_grouped(x, self.w_gate_up.w, self.w_down.w, weights, self.E, self.top)
         gu = rt.linear(x, self.w_gate_up)
         act = torch.empty(x.shape[0], self.inner, dtype=gu.dtype, device=x.device)
         return rt.linear(ops.moe_gate(gu, weights, act, self.E, self.f), self.w_down, partials=True)
 
     def _grouped(self, T):
-        """Whether in a step of T rows every token goes through its own experts only (rather than all through all)."""
+        """Whether in a step of T rows (of a recorded shape: the bucket's) every token goes through its own experts only (rather than all through all)."""
         ops, gu, down = self.rt.ops, self.w_gate_up.w, self.w_down.w
         D = gu.shape[1]
         return (self.rt.dtype == gu.dtype == down.dtype == torch.bfloat16 and self.s == 0 and not self.clamped and T >= GROUPED_MIN_ROWS
@@ -112,7 +113,7 @@ class RoutedExperts(FeedForward):
                 and T * self.E >= GROUPED_MIN_GAIN * (T * self.top + GROUPED_TILE // 2 * self.E))
 
     def forward(self, x, step):
-        return self._mix(x, self.route(x))
+        return self._mix(x, self.route(x), step)
 
 
 class GroupedRoutedExperts(RoutedExperts):
@@ -208,7 +209,7 @@ class GroupedRoutedExperts(RoutedExperts):
             rt.ops.moe_gate_clamped(gu, weights, act, self.E, self.f, self.limit, self.alpha, self.shared_limit)
             terms = [Term(rt.linear(act, self.w_down, partials=True))]
         else:
-            terms = [Term(self._mix(x, weights))]
+            terms = [Term(self._mix(x, weights, step))]
         if self.I:
             terms.append(Term(x, 1.0, weights[:, self.E]))
         return terms
@@ -265,4 +266,4 @@ class TableExperts(RoutedExperts):
         rt = self.rt
         weights = torch.empty(x.shape[0], self.E + 1, dtype=torch.float32, device=x.device)
         rt.ops.moe_table(self.table, step.token_ids, weights, self.E, step.token_source)
-        return self._mix(x, weights)
+        return self._mix(x, weights, step)

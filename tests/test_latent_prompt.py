@@ -140,6 +140,39 @@ def test_the_part_takes_either_form(window, monkeypatch):
         assert float((a - b).abs().max() / a.abs().max()) < 2e-2
 
 
+@pytest.mark.parametrize("past,new,experts", [((2100,) * 5, (40,) * 5, 4), ((60,) * 9, (33, 32, 32, 32, 32, 32, 32, 32, 33), 4),
+                                              ((0,), (450,), 16), ((0, 0), (20, 21), 4)])
+def test_first_run_and_recording_take_the_same_form(past, new, experts, monkeypatch):
+    """A shape runs eagerly at its own size until it is recorded at its bucket's: more sequences, tokens and pages.  Whether keys
+    and values are expanded, and whether tokens run through their own experts only, does not change with that."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.loading import random_engine
+    calls = []
+    for name in ("latent_prompt", "moe_grouped"):
+        monkeypatch.setattr(ops, name, lambda *a, real=getattr(ops, name), name=name, **k: calls.append(name) or real(*a, **k))
+    config = small_netanex(0)
+    for layer in config["layers"]:
+        layer["mlp"] = dict(kind="moe", expert=dict(ff=64), router=dict(experts=experts, top=2))
+    eng = random_engine(config, seed=3, max_tokens=16 * 4096, max_seqs=16, max_context=4096)
+    g = torch.Generator().manual_seed(1)
+    toks = lambda n: torch.randint(0, 97, (n,), generator=g).tolist()
+    texts = [(toks(p), toks(n)) for p, n in zip(past, new)]
+    runs, logits = [], []
+    for _ in range(3):           # eagerly; eagerly, and at the bucket's size before and in the recording; replayed
+        slots = [eng.open() for _ in texts]
+        for s, (held, _) in zip(slots, texts):
+            if held:
+                eng.step([(s, held, list(range(len(held))))])        # (all rows wanted: never recorded)
+        calls.clear()
+        logits.append(eng.step([(s, t, [len(t) - 1]) for s, (_, t) in zip(slots, texts)]).double())
+        runs.append({name: calls.count(name) for name in ("latent_prompt", "moe_grouped")})
+        for s in slots:
+            eng.close(s)
+    assert eng.graphs.replays == 1 and sum(runs[2].values()) == 0
+    assert runs[1] == {name: 3 * n for name, n in runs[0].items()}, runs
+    assert float((logits[2] - logits[0]).abs().max() / logits[0].abs().max()) < 2e-2
+
+
 def test_rule():
     """Few new tokens, and page tables that could name far more rows than the step has tokens, stay with the absorbed form."""
     from types import SimpleNamespace as NS
