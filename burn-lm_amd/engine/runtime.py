@@ -129,14 +129,38 @@ class FusedProjectionPlan:
         return isinstance(other, FusedProjectionPlan) and (self.kernel, self.columns, self.rows) == (other.kernel, other.columns, other.rows)
 
 
+class PackingRoom:
+    """The memory that a runtime's float32 matrices may take a second time: an eighth of the device's (36 of 288 GB: every
+    matrix of a model of 8 billion weights), and only while as much stays free.  The float32 kernels for few rows that read
+    the checkpoint's layout serve the rest, as they serve matrices that have no packed form."""
+    SHARE = 8
+
+    def __init__(self, device):
+        self.device, self.taken = device, 0
+
+    def grant(self, size):
+        free, total = torch.cuda.mem_get_info(self.device)
+        free += torch.cuda.memory_reserved(self.device) - torch.cuda.memory_allocated(self.device)     # what torch holds unused
+        if self.taken + size > total // self.SHARE or free - size < total // self.SHARE:
+            return False
+        self.taken += size
+        return True
+
+    def give_back(self, size):
+        self.taken -= size
+
+
 class LinearWeight:
     """A bound weight matrix [N, K] and, where the skinny product takes it, its copy packed for that
     product.  The copy is made when a product first asks for it (``packed``): an engine that only ever
     runs prompts and large batches never holds a matrix twice.  ``packable`` says whether there is one to
-    be had; ``drop_packed()`` gives its memory back (it is made again on demand)."""
+    be had; ``drop_packed()`` gives its memory back (it is made again on demand).
+    room (float32 matrices): what grants the copy its memory.  Without it, or if the allocation fails all the
+    same, ``packed`` is None and the matrix stays unpackable, so that every later step, recorded or not, takes the
+    same kernels."""
 
-    def __init__(self, w, packable=False, gated=False, packed=None):
-        self.w, self.gated = w, gated
+    def __init__(self, w, packable=False, gated=False, packed=None, room=None):
+        self.w, self.gated, self.room = w, gated, room
         self.packable = bool(packable) or packed is not None
         self._packed = packed
         self.shape, self.dtype = w.shape, w.dtype
@@ -147,14 +171,28 @@ class LinearWeight:
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError("a weight's packed copy would have to be made while a graph is being recorded; a step "
                                    "of this shape has to run once outside a recording first")
-            self._packed = ops.pack_weight(self.w, gated=self.gated)
+            if self.room is None:
+                self._packed = ops.pack_weight(self.w, gated=self.gated)
+            else:
+                self._pack_within_room()
         return self._packed
+
+    def _pack_within_room(self):
+        size = self.w.numel() * self.w.element_size()
+        if self.room.grant(size):
+            try:
+                self._packed = ops.pack_weight(self.w, gated=self.gated)
+            except torch.cuda.OutOfMemoryError:
+                self.room.give_back(size)
+        self.packable = self._packed is not None
 
     @property
     def is_packed(self):
         return self._packed is not None
 
     def drop_packed(self):
+        if self._packed is not None and self.room is not None:
+            self.room.give_back(self.w.numel() * self.w.element_size())
         self._packed = None
 
 
@@ -171,6 +209,7 @@ class Runtime:
         self.ops = ops
         self._k_groups = {}     # (N, K, M) -> groups of K, as chosen once (see k_groups)
         self._f32_plans = {}    # the same for the float32 products
+        self.packing_room = PackingRoom(self.device)
         ops.library()  # fail now, loudly, if the kernel library cannot be had
         ops.arrival_counters(self.device)   # allocated here, before any graph capture can be open
         ops.gemm_mfma_init(self.device)     # likewise: a function attribute is set once per device
@@ -196,9 +235,10 @@ class Runtime:
         return torch.empty(*shape, dtype=dtype or self.dtype, device=self.device)
 
     def weight(self, w, gated=False):
-        """Prepares a bound matrix for linear(): bfloat16 matrices may get a packed copy that the
-        skinny product streams (made at the first product of up to 16 rows, or of up to 64 where no other
-        kernel takes them; it doubles the matrix's memory; the plain copy serves everything else).
+        """Prepares a bound matrix for linear(): bfloat16 matrices, and in a float32 run float32 ones, may get a
+        packed copy that the skinny product streams (made at the first product of up to 16 rows, or of up to 64
+        bfloat16 ones where no other kernel takes them; it doubles the matrix's memory, in float32 within
+        PackingRoom's bounds; the plain copy serves everything else).
         gated=True: w is [gate rows; up rows] of a gated feed-forward and will be used through
         gated_linear(); its packed copy pairs each gate row with its up row."""
         w = w.contiguous()
@@ -211,6 +251,7 @@ class Runtime:
             # the gated product has no planes, so a longer K or an odd number of pairs goes as a plain product and a pass
             packable = self.dtype == torch.float32 and K % 4 == 0
             gated = gated and N % 16 == 0 and K <= F32_SKINNY_GROUP_K
+            return LinearWeight(w, packable, gated, room=self.packing_room)
         return LinearWeight(w, packable, gated)
 
     def k_groups(self, N, K, M=1):
@@ -266,12 +307,13 @@ class Runtime:
         """The float32 product of operands that ops.f32_rows takes, or None where the older kernels do it."""
         M, K = x.shape
         N = w.shape[0]
-        if M <= F32_SKINNY_MAX_ROWS and holder is not None and holder.packable and not holder.gated:
+        packed = holder.packed if M <= F32_SKINNY_MAX_ROWS and holder is not None and not holder.gated else None
+        if packed is not None:
             groups = self.f32_skinny_groups(M, N, K, planes)
             if groups == 1:
-                return ops.gemv_f32(x, holder.packed, out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device), K)
+                return ops.gemv_f32(x, packed, out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device), K)
             if groups:
-                parts = ops.gemv_f32(x, holder.packed, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), K)
+                parts = ops.gemv_f32(x, packed, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), K)
                 if planes:
                     return parts
                 if out is None or out.is_contiguous():
@@ -493,8 +535,9 @@ class Runtime:
             raise ValueError(f"gated_linear: activation {activation!r} unknown (silu, gelu_tanh)")
         if plain.dtype == torch.float32 and self.dtype == torch.float32 and activation == "silu" and ops.f32_rows(x, plain):
             if M <= F32_SKINNY_MAX_ROWS:
-                if isinstance(w, LinearWeight) and w.packable and w.gated:
-                    return ops.gemv_f32(x, w.packed, torch.empty(M, inner, dtype=torch.float32, device=x.device), K, gated=True)
+                packed = w.packed if isinstance(w, LinearWeight) and w.gated else None
+                if packed is not None:
+                    return ops.gemv_f32(x, packed, torch.empty(M, inner, dtype=torch.float32, device=x.device), K, gated=True)
             else:
                 tile, _, fused = f32_plan(M, inner, K, self.compute_units, gated=True)
                 # few rows: the plain product's smaller tiles and the pass behind it (12 bytes an element)

@@ -99,6 +99,34 @@ def test_runtime_takes_every_form(M, K):
     check(rt.gated_linear(x, w), x, w, gated=True)
 
 
+@pytest.mark.parametrize("why", ["little is free", "the model is large", "the allocation fails"])
+def test_no_room_for_packed_copies(why, monkeypatch):
+    """Where the matrices do not fit the device's memory a second time, products of few rows read them as they are: nothing is
+    refused, and the matrix keeps that form."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.runtime import Runtime
+    rt = Runtime(torch.float32, "cuda:0")
+    size = 4 * 2048 * 2048
+    if why == "the allocation fails":
+        def fails(w, gated=False):
+            raise torch.cuda.OutOfMemoryError("out of memory")
+        monkeypatch.setattr(ops, "pack_weight", fails)
+    else:
+        free, total = (0, 64 * size) if why == "little is free" else (60 * size, 64 * size)
+        held = torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (free - held, total))
+    made = [rt.weight(operands(1, 2048, 2048, seed=i)[1], gated=i == 1) for i in range(10)]
+    for M in (1, 8, 9, 16):
+        x = operands(M, 1, 2048)[0]
+        for i, w in enumerate(made):
+            check((rt.gated_linear if w.gated else rt.linear)(x, w), x, w.w, gated=w.gated)
+    packed = [w.is_packed for w in made]
+    assert packed == ([True] * 8 + [False] * 2 if why == "the model is large" else [False] * 10)
+    if why == "the model is large":      # memory that is given back serves another
+        made[0].drop_packed()
+        assert rt.weight(made[9].w).packed is not None
+
+
 def test_plan_keeps_its_bounds():
     from burn_lm_amd.engine.runtime import f32_plan
     for M in (9, 64, 65, 1000):
