@@ -209,8 +209,10 @@ extern "C" int blm_gemm_f32(const void* A, const void* W, void* C, int M, int N,
 // ---------------------------------------------------------------------------------------------------------------------
 #define GV_MAX_WAVES 8
 
-// KSTEPS: steps of 16 of K per wavefront.  gated: a tile's columns are 8 gate rows and their 8 up rows, C = silu(gate) * up.
-template <int KSTEPS>
+// KSTEPS: steps of 16 of K per wavefront.  WHOLE: every wavefront of every group has all of them, none partial, and nothing is
+// tested on the way (the tests for steps that a wavefront does not have cost 0.25 us: [1000, 520] at 8 rows 4.86 -> 5.11;
+// with them a decode step of 8 at the 1B shape took 1,547 us, so 1,533).  gated: a tile's columns are 8 gate rows and their 8 up rows, C = silu(gate) * up.
+template <int KSTEPS, bool WHOLE>
 __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
     gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wp, float* __restrict__ C, int M, int N, int K,
                     int lda, int ldc, int n_tiles, int k_steps, int gated, int steps_per_group, int tiles_per_block) {
@@ -225,7 +227,7 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
   const float* ap = A + (size_t)min(row, M - 1) * lda;   // rows past the last read it again and are zeroed
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   // activations first, then the first tile's weights behind them, all asked for before any is looked at; weights behind the end
-  // of the group are some other step's, and meet activations of zero (a step past the matrix is its last)
+  // of the group are some other step's (a step past the matrix is its last), and they and their activations count as zeros
   f32x4 a[KSTEPS];
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) a[s] = *reinterpret_cast<const f32x4*>(ap + min(kbase + s * 16, K - 4));
@@ -235,7 +237,7 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
     const float* wt = Wp + ((size_t)tile * k_steps * 64 + lane) * 4;
 #pragma unroll
     for (int s = 0; s < PART; ++s)
-      w[s] = __builtin_bit_cast(f32x4, load16_stream(wt + (size_t)min(step0 + part * PART + s, k_steps - 1) * 256));
+      w[s] = __builtin_bit_cast(f32x4, load16_stream(wt + (size_t)(WHOLE ? step0 + part * PART + s : min(step0 + part * PART + s, k_steps - 1)) * 256));
   };
   f32x4 w[2][PART];
   weights(tile_begin, 0, w[0]);
@@ -253,6 +255,10 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
       f32x4 acc[8];
 #pragma unroll
       for (int x = 0; x < 8; ++x) acc[x] = zero;
+      if (!WHOLE && step0 + KSTEPS > group_end)        // zero activations alone would not do: an infinite weight would make them no numbers
+#pragma unroll
+        for (int s = 0; s < PART; ++s)
+          if (step0 + p * PART + s >= group_end) w[p & 1][s] = zero;
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int s = 0; s < PART; ++s)
@@ -341,11 +347,14 @@ extern "C" int blm_gemv_f32(const void* A, const void* Wp, void* C, int M, int N
   gemv_f32_geometry(N, K, groups, &ksteps, &waves, &blocks);
   const int per_block = (n_tiles + blocks - 1) / blocks;
   dim3 grid((unsigned)blocks, (unsigned)groups), block(waves * BLM_WAVE);
-#define BLM_GVF(KS)                                                                                                     \
-  hipLaunchKernelGGL((gemv_f32_kernel<KS>), grid, block, 0, stream, (const float*)A, (const float*)Wp, (float*)C, M, N, K, \
+#define BLM_GVF(KS, WHOLE)                                                                                              \
+  hipLaunchKernelGGL((gemv_f32_kernel<KS, WHOLE>), grid, block, 0, stream, (const float*)A, (const float*)Wp, (float*)C, M, N, K, \
                      lda, ldc, n_tiles, k_steps, gated, steps, per_block)
-  if (ksteps == 4) BLM_GVF(4);
-  else BLM_GVF(16);
+  const bool whole = K % 16 == 0 && k_steps == groups * steps && steps == waves * ksteps;
+  if (ksteps == 4 && whole) BLM_GVF(4, true);
+  else if (ksteps == 4) BLM_GVF(4, false);
+  else if (whole) BLM_GVF(16, true);
+  else BLM_GVF(16, false);
 #undef BLM_GVF
   BLM_LAUNCH_CHECK("gemv_f32");
   return 0;

@@ -67,6 +67,21 @@ def test_few_rows_gated(M, I, K):
     check(ops.gemv_f32(x, ops.pack_weight(w, gated=True), torch.full((M, I), float("nan"), device="cuda"), K, gated=True), x, w, gated=True)
 
 
+@pytest.mark.parametrize("K,at,groups", [(520, 516, 1), (64, 63, 1), (2048, 43 * 16, 3), (2048, 0, 3), (516, 512, 2)])
+@pytest.mark.parametrize("M", [1, 8, 16])
+def test_an_infinite_weight_stays_infinite(M, K, at, groups):
+    """Wavefronts whose stretch of K is shorter than the others' have steps without weights: these add zeros, whatever the
+    matrix holds elsewhere."""
+    from burn_lm_amd.csrc import ops
+    x, w = operands(M, 33, K)
+    x = x.abs() + 0.5
+    w[3, at], w[20, at] = float("inf"), float("-inf")
+    got = ops.gemv_f32(x, ops.pack_weight(w), torch.empty(groups, M, 33, device="cuda"), K).sum(0)
+    assert bool((got[:, 3] == float("inf")).all()) and bool((got[:, 20] == float("-inf")).all())
+    others = [n for n in range(33) if n not in (3, 20)]
+    check(got[:, others], x, w[others])
+
+
 def test_refused():
     from burn_lm_amd.csrc import ops
     x, w = operands(17, 32, 2052)
