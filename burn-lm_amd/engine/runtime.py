@@ -29,6 +29,7 @@ Matrix products ``x[M,K] @ w[N,K]^T``:
 """
 from __future__ import annotations
 
+import functools
 import os
 
 import torch
@@ -92,6 +93,7 @@ F32_SKINNY_MAX_ROWS = 16
 F32_SKINNY_GROUP_K = 2048
 
 
+@functools.lru_cache(maxsize=4096)      # a length asks for some ten; made anew at every product, each took 2 to 12 us of the host
 def f32_plan(M, N, K, compute_units, planes=False, gated=False):
     """(tile, groups of K, microseconds) of ops.gemm_f32 that a sum of its parts' costs finds fastest: every unit works through
     its share of the blocks, and every plane of partial products is read once by the norm that adds it.
@@ -208,7 +210,7 @@ class Runtime:
             raise RuntimeError("no GPU is visible to this process; burn-lm_amd has no CPU path")
         self.ops = ops
         self._k_groups = {}     # (N, K, M) -> groups of K, as chosen once (see k_groups)
-        self._f32_plans = {}    # the same for the float32 products
+        self._f32_groups = {}   # the same for the float32 products of up to 16 rows (see f32_skinny_groups; more rows: f32_plan)
         self.packing_room = PackingRoom(self.device)
         ops.library()  # fail now, loudly, if the kernel library cannot be had
         ops.arrival_counters(self.device)   # allocated here, before any graph capture can be open
@@ -295,12 +297,12 @@ class Runtime:
         blocks fill at least GROUP_MIN_FILL of a round on the compute units (us at 8 rows, in 1 / 2 / 4 groups: [2048, 2048]
         8.7 / 6.6 / 5.7 with 128 / 256 / 256 blocks; [2048, 8192] in 4 / 8 groups 16.0 / 15.6)."""
         key = (M, N, K, planes)
-        known = self._f32_plans.get(key)
+        known = self._f32_groups.get(key)
         if known is None:
             taken = [(g, ops.gemv_f32_geometry(M, N, K, g)) for g in (1, 2, 4, 8, 16, 32, 64)]
             taken = [(g, geometry[0]) for g, geometry in taken if geometry is not None]
             full = [g for g, blocks in taken if blocks >= GROUP_MIN_FILL * self.compute_units and K // g >= 256]
-            known = self._f32_plans[key] = (full[0] if planes and full else taken[0][0]) if taken else 0
+            known = self._f32_groups[key] = (full[0] if planes and full else taken[0][0]) if taken else 0
         return known
 
     def _f32_linear(self, x, w, holder, out, planes):

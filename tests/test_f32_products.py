@@ -150,3 +150,11 @@ def test_plan_keeps_its_bounds():
                 tile, groups, us = f32_plan(M, N, K, 256, planes=True)
                 assert groups == 1 or K // groups >= 128
                 assert f32_plan(M, N, K, 256)[1] == 1 and f32_plan(M, N, K, 256, gated=True)[0][1] == 128 and us > 0
+
+
+def test_plan_is_made_once():
+    """The same sizes again take the plan that was made for them, within a bounded number of plans."""
+    from burn_lm_amd.engine.runtime import f32_plan
+    assert f32_plan(777, 2048, 8192, 256, planes=True) is f32_plan(777, 2048, 8192, 256, planes=True)
+    assert f32_plan(777, 2048, 8192, 256) is not f32_plan(777, 2048, 8192, 256, planes=True)
+    assert f32_plan.cache_info().maxsize is not None
