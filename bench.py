@@ -444,7 +444,11 @@ def mixer_rates(engine, batch, context, prefill_tokens):
         if kind == "Attention":
             mid, mix = m.project(x, step, v), m.attend
         elif kind == "LatentAttention":
-            mid, mix = m.project(x, step, v), m.attend
+            mid, mix = m.project_expanded(x, step, v), m.attend_expanded
+            if mid is None:
+                mid, mix = m.project(x, step, v), m.attend
+            elif flops is not None:        # (a prompt of its own: nothing in front of it)
+                flops = m.expanded_flops(0, x.shape[0])
         elif kind == "HGRN2":
             mid, mix = m.project(x), m.scan
         elif kind == "ChannelDelta":

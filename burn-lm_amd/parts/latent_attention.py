@@ -151,22 +151,34 @@ class LatentAttention(Mixer):
         return 2 * rows * sum(w.numel() for w in self._matrices())
 
     def mixing_flops(self, past, new):
-        """Scores over kv_rank + rot_dim lanes and weighted latents over kv_rank lanes, per (query, visible row, head)."""
-        pairs = sum(min(past + t + 1, self.window) for t in range(new)) if self.window else new * past + new * (new + 1) // 2
-        return 2 * self.H * (2 * self.R + self.dr) * pairs
+        """The smaller of the two forms' operations.  (The expansion of the new rows takes what step_flops counts for their products
+        with W_uk and W_uv.)"""
+        absorbed = 2 * self.H * (2 * self.R + self.dr) * self._pairs(past, new)
+        return min(absorbed, self.expanded_flops(past, new) - self._expansion(new)) if self.can_expand else absorbed
+
+    def expanded_flops(self, past, new):
+        """Of attend_expanded: the expansion of every row that a new token sees, scores over dim + rot_dim lanes and weighted values
+        over vdim lanes per (query, visible row, head)."""
+        rows = new + (min(past, self.window - 1) if self.window else past)
+        return self._expansion(rows) + 2 * self.H * (self.dn + self.dr + self.dv) * self._pairs(past, new)
+
+    def _expansion(self, rows):
+        return 2 * self.R * self.H * (self.dn + self.dv) * rows
+
+    def _pairs(self, past, new):
+        return sum(min(past + t + 1, self.window) for t in range(new)) if self.window else new * past + new * (new + 1) // 2
 
     def forward(self, x, step, view):
         qd, q, gate = self._inputs(x)
         if self.expands(step, q, view):
-            rt, H = self.rt, self.H
-            turned = torch.empty(x.shape[0], H, self.dr, dtype=rt.dtype, device=x.device)
-            self._write(qd, q, turned, step, view, view.v)
-            o = torch.empty(x.shape[0], H * self.dv, dtype=rt.dtype, device=x.device)
-            rt.ops.latent_prompt(q, turned, o, view.k, self.w_uk, self.w_uv.view(H * self.dv, self.R), step, view.block_table(step),
-                                 -(-step.max_len_after // 64), H, self.R, self.dn, self.dr, self.dv, self.scale, window=self.window,
-                                 sinks=self.sinks)
-            return self._finish(o, gate)
+            return self._finish(self.attend_expanded(self._turn(qd, q, step, view), step, view), gate)
         return self.output(self.attend(self._absorb(qd, q, step, view), step, view), gate)
+
+    def project_expanded(self, x, step, view):
+        """The plain queries and their turned lanes, for attend_expanded, with the step's rows in the cache afterwards; None, with nothing
+        written, where the step runs in the absorbed form."""
+        qd, q, _ = self._inputs(x)
+        return self._turn(qd, q, step, view) if self.expands(step, q, view) else None
 
     def project(self, x, step, view):
         """The absorbed queries [tokens, heads, kv_rank + rot_dim] of the step's tokens; their latents and turned key
@@ -200,6 +212,20 @@ class LatentAttention(Mixer):
         self._write(qd, q, qabs, step, view, view.v if mfma else None)
         rt.ops.head_project(q, dn + dr, self.w_uk_t, qabs.view(T, H * (R + dr)), R + dr)
         return qabs
+
+    def _turn(self, qd, q, step, view):
+        turned = torch.empty(q.shape[0], self.H, self.dr, dtype=self.rt.dtype, device=q.device)
+        self._write(qd, q, turned, step, view, view.v)
+        return q, turned
+
+    def attend_expanded(self, queries, step, view):
+        """Every (token, head)'s weighted sum of the values it sees -> [tokens, heads * vdim], keys and values expanded per head."""
+        q, turned = queries
+        rt, H = self.rt, self.H
+        o = torch.empty(q.shape[0], H * self.dv, dtype=rt.dtype, device=q.device)
+        return rt.ops.latent_prompt(q, turned, o, view.k, self.w_uk, self.w_uv.view(H * self.dv, self.R), step, view.block_table(step),
+                                    -(-step.max_len_after // 64), H, self.R, self.dn, self.dr, self.dv, self.scale, window=self.window,
+                                    sinks=self.sinks)
 
     def attend(self, qabs, step, view):
         """Every (token, head)'s weighted sum of the latents it sees -> float32 [tokens, heads, kv_rank]."""

@@ -187,3 +187,22 @@ def test_rule():
     assert not rule(1, 1, 1, 1000) and not rule(31, 1, 31, 31) and not rule(63, 2, 40, 100)
     assert rule(4096, 1, 4096, 16384) and not rule(64, 1, 64, 32768) and rule(16384, 1, 16384, 65536) and not rule(8, 8, 1, 64)
     assert not m.expands(NS(n_seqs=1, max_len_after=64, max_new=64, n_tokens=64), q[:, 1:], view)
+
+
+@pytest.mark.parametrize("window", [0, 100])
+def test_operations_of_a_prompt(window):
+    """What a step costs at the least counts the form that it runs in: written out pair by pair for a long prompt, a portion behind
+    others and a single token."""
+    from burn_lm_amd.parts.latent_attention import LatentAttention
+    m = LatentAttention.__new__(LatentAttention)
+    m.H, m.R, m.dn, m.dr, m.dv, m.window, m.can_expand = 16, 512, 128, 64, 128, window, True
+    for past, new in ((0, 2048), (300, 700), (2000, 1), (0, 1)):
+        see = [range(max(0, t - window + 1) if window else 0, t + 1) for t in range(past, past + new)]
+        pairs, rows = sum(map(len, see)), past + new - see[0][0]
+        absorbed, own = 2 * 16 * (512 + 64 + 512) * pairs, 2 * 16 * (128 + 64 + 128) * pairs
+        expansion = 2 * 512 * 16 * (128 + 128)
+        assert m.expanded_flops(past, new) == own + expansion * rows
+        assert m.mixing_flops(past, new) == (absorbed if new == 1 and past else min(absorbed, own + expansion * (rows - new)))
+        assert (m.mixing_flops(past, new) < absorbed) == (new > 1 or past == 0)
+    m.can_expand = False
+    assert m.mixing_flops(0, 2048) == 2 * 16 * 1088 * sum(min(t + 1, window or 2048) for t in range(2048))
