@@ -119,14 +119,15 @@ class LatentAttention(Mixer):
         H, dn, dv, R = self.H, self.dn, self.dv, self.R
         self.w_uk_t = tensors[n["uk"]].view(H, dn, R).transpose(1, 2).contiguous()   # [H, R, dn]: q_plain -> latent lanes
         self.w_uv = tensors[n["uv"]].view(H, dv, R).contiguous()
-        self.w_uk = tensors[n["uk"]].contiguous()            # [H * dn, R]: latents -> plain keys
         self.w_o = rt.weight(tensors[n["o"]])
         rt.ops.latent_attn_init(rt.device)
         self.use_mfma = (os.environ.get("BURN_LM_AMD_LATENT_MFMA") != "0" and self.scale > 0 and self.w_uk_t.dtype == torch.bfloat16
                          and rt.ops.latent_attn_mfma_supported(rt.dtype, R, self.dr))
 
-        self.can_expand = (self.use_mfma and self.w_uk.dtype == self.w_uv.dtype == torch.bfloat16
+        self.can_expand = (self.use_mfma and self.w_uv.dtype == torch.bfloat16
                            and rt.ops.latent_prompt_supported(rt.dtype, R, dn, self.dr, dv))
+        # [H * dn, R]: latents -> plain keys, a second layout of w_uk_t that only the expanded form reads
+        self.w_uk = tensors[n["uk"]].contiguous() if self.can_expand else None
         if self.can_expand:
             rt.ops.latent_prompt_init(rt.device)
 

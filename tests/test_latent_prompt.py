@@ -189,6 +189,20 @@ def test_rule():
     assert not m.expands(NS(n_seqs=1, max_len_after=64, max_new=64, n_tokens=64), q[:, 1:], view)
 
 
+@pytest.mark.parametrize("dtype,dim,kept", [("bfloat16", 64, True), ("float32", 64, False), ("bfloat16", 48, False)])
+def test_second_layout_of_the_key_weights(dtype, dim, kept):
+    """Only a part that can expand its latents keeps W_uk in both layouts."""
+    from burn_lm_amd.engine.loading import random_engine
+    config = small_netanex(0)
+    for layer in config["layers"]:
+        layer["mixer"].update(dim=dim, scale=(dim + 32) ** -0.5)
+    eng = random_engine(config, seed=3, dtype=dtype, max_tokens=256, max_seqs=1, max_context=256)
+    parts = [b.mixer for b in eng.model.blocks]
+    assert all(m.can_expand == kept and (m.w_uk is not None) == kept for m in parts)
+    slot = eng.open()
+    assert bool(eng.step([(slot, list(range(90)), [89])]).isfinite().all())
+
+
 @pytest.mark.parametrize("window", [0, 100])
 def test_operations_of_a_prompt(window):
     """What a step costs at the least counts the form that it runs in: written out pair by pair for a long prompt, a portion behind
