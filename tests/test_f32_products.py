@@ -60,6 +60,20 @@ def test_few_rows(M, N, K):
     assert bool(wide[:, N:].isnan().all())
 
 
+@pytest.mark.parametrize("M", [1, 8, 16])
+@pytest.mark.parametrize("N,K,groups", [(4112, 2048, 1), (8200, 2048, 1), (8200, 2048, 3), (8209, 512, 1), (16400, 260, 2), (4099, 1000, 2)])
+def test_few_rows_of_many_columns(M, N, K, groups):
+    """Blocks that walk several column tiles, the last one fewer: weights asked for ahead across tiles, the same shared memory for
+    every tile's sums."""
+    from burn_lm_amd.csrc import ops
+    blocks, _ = ops.gemv_f32_geometry(M, N, K, groups)
+    tiles = -(-N // 16)
+    assert blocks // groups < tiles           # so some block has more than one
+    x, w = operands(M, N, K, seed=N)
+    out = torch.full((groups, M, N), float("nan"), device="cuda")
+    check(ops.gemv_f32(x, ops.pack_weight(w), out, K).sum(0), x, w)
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 8, 4), (3, 24, 100), (8, 72, 516), (16, 256, 2048)])
 def test_few_rows_gated(M, I, K):
     from burn_lm_amd.csrc import ops
@@ -80,6 +94,14 @@ def test_an_infinite_weight_stays_infinite(M, K, at, groups):
     assert bool((got[:, 3] == float("inf")).all()) and bool((got[:, 20] == float("-inf")).all())
     others = [n for n in range(33) if n not in (3, 20)]
     check(got[:, others], x, w[others])
+
+
+@pytest.mark.parametrize("M,I,K", [(1, 4104, 2048), (8, 4136, 512), (16, 4104, 2048)])
+def test_few_rows_of_many_pairs(M, I, K):
+    from burn_lm_amd.csrc import ops
+    assert ops.gemv_f32_geometry(M, 2 * I, K)[0] < I // 8
+    x, w = operands(M, 2 * I, K, seed=I)
+    check(ops.gemv_f32(x, ops.pack_weight(w, gated=True), torch.full((M, I), float("nan"), device="cuda"), K, gated=True), x, w, gated=True)
 
 
 def test_refused():

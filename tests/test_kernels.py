@@ -966,3 +966,17 @@ def test_sample_does_not_depend_on_how_rows_are_cut(ops, V):
         assert torch.equal(ops.sample(x[:n], u[:n].clone(), 0.8, 0.9), whole[:n])
     full = ops.sample(x, u, 0.8, 1.0)
     assert torch.equal(ops.sample(x[:3], u[:3].clone(), 0.8, 1.0), full[:3])
+
+
+@pytest.mark.parametrize("V", [9, 3000])
+def test_sample_of_more_rows_than_counters_apart(ops, V):
+    """Above 2,048 rows the rows' arrival counters lie side by side; every row's draw stays what it is among few rows, and the
+    counters are left as they were."""
+    g = torch.Generator().manual_seed(V)
+    x, u = dev(torch.randn(2100, V, generator=g) * 2), dev(torch.rand(2100, generator=g))
+    assert ops.arrival_step(2100) == 1 and ops.arrival_step(2048) > 1
+    for p in (0.9, 1.0):
+        whole = ops.sample(x, u, 0.8, p)
+        assert torch.equal(ops.sample(x[:2048], u[:2048].clone(), 0.8, p), whole[:2048])
+        assert torch.equal(ops.sample(x[2090:], u[2090:].clone(), 0.8, p), whole[2090:])
+    assert not bool(ops.arrival_counters(x.device).any())
