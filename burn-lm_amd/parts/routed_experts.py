@@ -96,7 +96,7 @@ class RoutedExperts(FeedForward):
         """The experts' results for [tokens, width] by the weights of `route`, without clamps."""
         rt, ops = self.rt, self.rt.ops
         bucket = getattr(step, "bucket", None)
-        if self._grouped(bucket[0] if bucket else x.shape[0]):
+        if self._grouped(bucket[0] if bucket else x.shape[0]) and x.is_contiguous() and x.data_ptr() % 16 == 0:
             return ops.moe_grouped(x, self.w_gate_up.w, self.w_down.w, weights, self.E, self.top)
         gu = rt.linear(x, self.w_gate_up)
         act = torch.empty(x.shape[0], self.inner, dtype=gu.dtype, device=x.device)

@@ -107,3 +107,26 @@ def test_parts_take_either_way(kind, monkeypatch):
     assert (got - want).norm() <= 3 * 2 ** -9 * want.norm()
     if kind == "table":
         assert got[Step.token_ids < 0].abs().max() == 0
+
+
+@pytest.mark.parametrize("form", ["columns of wider rows", "odd address"])
+def test_rows_that_the_grouped_form_does_not_take(form):
+    """Rows with a stride or at an address of their own go through all experts: the part takes what it always took."""
+    import burn_lm_amd.parts.routed_experts as RE
+    from burn_lm_amd.engine.runtime import Runtime
+    rt, g = Runtime(), torch.Generator().manual_seed(3)
+    T, D, E, top, f = 700, 128, 8, 2, 64
+    t = {f"e{e}.{r}": (torch.randn(*((D, f) if r == "down" else (f, D)), generator=g) * D ** -0.5).bfloat16().cuda()
+         for e in range(E) for r in ("gate", "up", "down")}
+    t["router"], t["router_bias"] = torch.randn(E, D, generator=g).bfloat16().cuda(), torch.zeros(E).cuda()
+    part = RE.RoutedExperts(dict(width=D, experts=E, top=top, expert_inner=f), {n: n for n in t})
+    part.bind(t, rt)
+    x = torch.randn(T, D, generator=g).bfloat16().cuda()
+    if form == "odd address":
+        given = torch.empty(T * D + 8, dtype=x.dtype, device="cuda")[1:1 + T * D].view(T, D)
+    else:
+        given = torch.empty(T, D + 8, dtype=x.dtype, device="cuda")[:, :D]
+    given.copy_(x)
+    assert part._grouped(T)
+    want, got = ((lambda y: y.double().sum(0) if y.dim() == 3 else y.double())(part.forward(v, None)) for v in (x, given))
+    assert (got - want).norm() <= 3 * 2 ** -9 * want.norm()
