@@ -130,6 +130,8 @@ class LatentAttention(Mixer):
         self.w_uk = tensors[n["uk"]].contiguous() if self.can_expand else None
         if self.can_expand:
             rt.ops.latent_prompt_init(rt.device)
+            # (a view into a larger tensor may start anywhere; the kernels read 16 bytes at a time)
+            self.w_uk, self.w_uv = (w.clone() if w.data_ptr() % 16 else w for w in (self.w_uk, self.w_uv))
 
     def expands(self, step, q, view):
         """Whether the step's keys and values are expanded per head instead of absorbing the projections into queries and

@@ -203,6 +203,26 @@ def test_second_layout_of_the_key_weights(dtype, dim, kept):
     assert bool(eng.step([(slot, list(range(90)), [89])]).isfinite().all())
 
 
+def test_weights_at_any_address():
+    """Weights per head that are views into larger tensors, at addresses that are no multiples of 16 bytes, give the same result."""
+    from burn_lm_amd.engine.loading import random_engine
+    eng = random_engine(small_netanex(0), seed=3, max_tokens=256, max_seqs=1, max_context=256)
+    m, g = eng.model.blocks[0].mixer, torch.Generator().manual_seed(5)
+    tensors = {name: (torch.randn(*spec.shape, generator=g) * 0.1).bfloat16().cuda() for name, spec in m.tensor_specs().items()}
+    odd = lambda t: torch.cat((t.new_zeros(1), t.reshape(-1)))[1:].view(t.shape)
+    slot = eng.open()
+    eng.cache.reserve([(slot, 90)])
+    step = eng.build_step([(slot, list(range(90)), [89])])
+    x = torch.randn(90, 128, generator=g).bfloat16().cuda()
+    results = []
+    for form in (lambda t: t, odd):
+        part = type(m)(m.params, m.names)
+        part.bind({name: form(t) if name in (m.names["uk"], m.names["uv"]) else t for name, t in tensors.items()}, eng.rt)
+        assert part.can_expand
+        results.append(part.forward(x, step, eng.cache.views[0]).float())
+    assert torch.equal(*results)
+
+
 @pytest.mark.parametrize("window", [0, 100])
 def test_operations_of_a_prompt(window):
     """What a step costs at the least counts the form that it runs in: written out pair by pair for a long prompt, a portion behind
