@@ -27,6 +27,9 @@ from .base import FeedForward, TensorSpec, Term
 GROUPED_MIN_ROWS = 512
 GROUPED_MIN_GAIN = 2
 GROUPED_TILE = 256
+# The grouped form's planes and activations take top * (4 width + 2 inner) bytes a row, the stacked form's gates, ups and activations
+# 6 * experts * inner: beyond this many bytes only where they are no more, so that no step needs more memory than the stacked form did.
+GROUPED_FREE_BYTES = 1 << 30
 
 class RoutedExperts(FeedForward):
     """params: width, experts, top, expert_inner, shared_inner (0: no shared expert).
@@ -110,6 +113,7 @@ class RoutedExperts(FeedForward):
                 and self.f % ops.MOE_GROUPED_STEP == 0 and D % ops.MOE_GROUPED_STEP == 0
                 and self.E <= ops.MOE_GROUPED_EXPERTS and self.top <= ops.MOE_GROUPED_TOP and self.top <= self.E
                 and max(gu.numel(), T * D, T * self.top) < 2 ** 30
+                and T * self.top * (4 * D + 2 * self.f) <= max(GROUPED_FREE_BYTES, 6 * T * self.E * self.f)
                 and T * self.E >= GROUPED_MIN_GAIN * (T * self.top + GROUPED_TILE // 2 * self.E))
 
     def forward(self, x, step):

@@ -130,3 +130,22 @@ def test_rows_that_the_grouped_form_does_not_take(form):
     assert part._grouped(T)
     want, got = ((lambda y: y.double().sum(0) if y.dim() == 3 else y.double())(part.forward(v, None)) for v in (x, given))
     assert (got - want).norm() <= 3 * 2 ** -9 * want.norm()
+
+
+def test_no_more_memory_than_the_stacked_form():
+    """Many rows of a wide model with narrow experts: planes for every choice would take several times what all experts' activations
+    take."""
+    from types import SimpleNamespace as NS
+
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.parts.routed_experts import RoutedExperts
+
+    def grouped(rows, width, inner, experts, top):
+        part = RoutedExperts.__new__(RoutedExperts)
+        part.rt, part.E, part.top, part.f, part.s = NS(ops=ops, dtype=torch.bfloat16), experts, top, inner, 0
+        matrix = lambda *shape: NS(w=torch.empty(shape, dtype=torch.bfloat16, device="meta"))
+        part.w_gate_up, part.w_down = matrix(2 * experts * inner, width), matrix(width, experts * inner)
+        return part._grouped(rows)
+    assert grouped(2048, 4096, 64, 64, 8)                                    # 0.3 GB
+    assert not grouped(131072, 4096, 64, 64, 8)                              # 17 GB against 3
+    assert grouped(65536, 2048, 512, 16, 4) and grouped(65536, 1024, 128, 128, 8)     # less than the stacked form
