@@ -38,6 +38,7 @@ EXPAND_MAX_ROWS = (16384, 4)
 # within these (us of a whole step of two such mixers, absorbed / expanded: 16 sequences of 16 new tokens behind 1,000 others 2,466
 # / 1,251, 4 of 2 behind 1,000 1,271 / 756, 5 of 20 behind 3,500 1,666 / 1,040, one of 64 behind 20,000 2,516 / 1,896).
 EXPAND_BUCKET_SLACK = 2
+EXPAND_MAX_BLOCKS = 65535      # sequences, and pages of one: the launch has a block row for each
 MFMA_MAX_PIECES = 64           # most pieces the matrix-core decode cuts a sequence's half pages into
 
 
@@ -142,7 +143,7 @@ class LatentAttention(Mixer):
         rows = seqs * -(-longest // 64) * 64
         return (self.can_expand and step.max_new > 1 and view.v.numel() > 0 and view.page_size == 64
                 and tokens * slack >= EXPAND_MIN_NEW * seqs and rows <= max(slack * EXPAND_MAX_ROWS[0], EXPAND_MAX_ROWS[1] * tokens)
-                and seqs <= 65535 and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0)
+                and seqs <= EXPAND_MAX_BLOCKS and -(-longest // 64) <= EXPAND_MAX_BLOCKS and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0)
 
     def _matrices(self):
         return [self.w_in.w, self.w_o.w, self.w_uk_t, self.w_uv] + ([self.w_uq.w] if self.q_rank else [])

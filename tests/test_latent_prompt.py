@@ -240,3 +240,15 @@ def test_operations_of_a_prompt(window):
         assert (m.mixing_flops(past, new) < absorbed) == (new > 1 or past == 0)
     m.can_expand = False
     assert m.mixing_flops(0, 2048) == 2 * 16 * 1088 * sum(min(t + 1, window or 2048) for t in range(2048))
+
+
+def test_rule_stays_within_the_launch():
+    """A sequence of more pages than a launch has rows of blocks stays with the absorbed form, however many tokens it brings."""
+    from types import SimpleNamespace as NS
+
+    from burn_lm_amd.parts.latent_attention import LatentAttention
+    m = LatentAttention.__new__(LatentAttention)
+    m.can_expand = True
+    view, q = NS(v=torch.empty(1), page_size=64), torch.empty(64, 64, dtype=torch.bfloat16)
+    rule = lambda n, after: m.expands(NS(n_seqs=1, max_len_after=after, max_new=n, n_tokens=n), q, view)
+    assert rule(1 << 21, 65535 * 64) and not rule(1 << 21, 65535 * 64 + 1)
