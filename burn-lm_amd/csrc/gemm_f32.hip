@@ -1,7 +1,8 @@
 // The true 32-bit product C[M,N] = A[M,K] * W[N,K]^T on the matrix cores' float instructions (float operands, float
 // products, float sums, nothing narrowed), with W as the checkpoint stores it (K contiguous).
-//   gemm_f32 : many rows.  A block of four wavefronts owns a tile of 128x128, 128x64 or 64x64; K in steps of 32.
-//   gemv_f32 : up to 16 rows (decode).  Streams every weight row once, whole lines at a time.
+//   gemm_f32 : many rows.  A block of four wavefronts owns a tile of 128x128, 128x64, 64x128 or 64x64 (gated:
+//              128x128 or 64x128); K in steps of 32.
+//   gemv_f32 : up to 16 rows (decode).  Streams a packed copy of the weights once, whole lines at a time.
 // Both want K, lda and the rows' addresses in units of 16 bytes; other operands take gemm_tiled.
 #include "common.h"
 
@@ -18,7 +19,7 @@ __device__ __forceinline__ float silu_times(float g, float u) { return g / (1.0f
 // permuted (piece j of row r at j ^ (r / 2 % 8)) so that the 16 rows that a quarter of a wavefront reads meet every bank.
 // An instruction takes 64 cycles of a SIMD, a step of a 64x64 wavefront tile 64 of them, so loads through registers and one
 // barrier per step hide behind the products; what bounds the kernel is the instructions' rate (157 TFLOP/s) and how evenly
-// the tiles fill the compute units, which is why there are three tiles and K may be cut into groups (partial planes).
+// the tiles fill the compute units, which is why there are four tiles and K may be cut into groups (partial planes).
 // Sums in two levels: the products of GC_CHUNK elements of K, then the chunks, so that the rounding error does not grow with
 // K additions in a row.
 // Direct loads from global into shared memory: staged through registers the same tiles took 12 % longer (the conversions of

@@ -7,8 +7,9 @@
 // What bounds it: 256 x 128 tiles by eight wavefronts share the compute unit's LDS between the direct loads (48 KB a stage), the
 // wavefronts' reads (128 KB) and 1,024 cycles of matrix instructions; a stage takes 0.75 us, and with 16 experts of 512 rows each
 // the tiles' last rows and the last round of blocks are a quarter of the time.
-// Measured (us, 2,048 tokens, 16 experts of 512 at width 2048, 4 chosen; before: the stacked products and the gating pass):
-// gate/up with gating 122 -> 61, down 77 -> 41, lists 6.5.  Tried: 128 x 128 tiles, two blocks a unit (stages of 32: 70 and 43),
+// Measured (us a call by events over repeated calls, 2,048 tokens, 16 experts of 512 at width 2048, 4 chosen; before: the stacked
+// products and the gating pass): gate/up with gating 122 -> 61, down 77 -> 41, lists 6.5 (within a whole prompt, under the profiler,
+// 66, 47 and 6.3).  Tried: 128 x 128 tiles, two blocks a unit (stages of 32: 70 and 43),
 // the compiler's own order of reads, loads and products (72 and 44), four wavefronts of 128 x 64 (83 and 54).
 #include <type_traits>
 

@@ -4,8 +4,9 @@ Matrix products ``x[M,K] @ w[N,K]^T``:
 * float32 weights: the hand-written float kernels always (float operands, products and sums, no
   reduced-precision matrix mode), whatever the activation dtype.  This is the whole float32 path
   and also what keeps a tensor that a checkpoint stores in 32 bits exact in a bfloat16 run.  With float32
-  activations whose rows lie in units of 16 bytes: up to 16 rows ops.gemv_f32 on a packed copy, more rows
-  ops.gemm_f32 (f32_plan chooses its tile and groups of K); everything else ops.gemm_tiled.
+  activations whose rows lie in units of 16 bytes: up to 16 rows ops.gemv_f32 on a packed copy, more rows (from 9
+  on where there is no such copy) ops.gemm_f32 (f32_plan chooses its tile and groups of K); everything else
+  ops.gemv_skinny up to 8 rows and ops.gemm_tiled.
 * bfloat16 weights, up to 64 rows (decode): the hand-written skinny kernel on the matrix cores that
   streams the weight once (where the width fits its registers: see ops.gemv_mfma_group_limit).  From
   17 rows on, the products that come as partial planes (output and down projection) and, from 33 rows

@@ -67,7 +67,9 @@ def decode_splits_f32(pages: int, blocks: int, head_dim: int, compute_units: int
     the merge takes 2.  So pieces of three pages (two for wide heads), as long as every block has a compute unit to
     itself; never more than 16 (us per call in pieces of the rule / whole, 32 heads of 64 in 8 groups: 8 pages at batch 1 11.1 / 12.2,
     at batch 8 12.3 / 13.3; 12 pages at batch 8 13.1 / 17.5, at batch 16 18.1 / 22.9; 50 pages at batch 16 in two 48.4, in four
-    57.4; 24 heads of 128: 8 pages at batch 8 17.3 / 25.1)."""
+    57.4; 24 heads of 128: 8 pages at batch 8 17.3 / 25.1).  Few key-value heads behind very many keys would take more
+    pieces (one head of 64 at batch 1, 16 / 32 / 64 pieces: 16,000 keys 27 / 25 / 32, 65,000 keys 73 / 49 / 44, 130,000 keys
+    135 / 82 / 61; the generic kernel 77, 202 and 248)."""
     if pages <= 4 and head_dim <= 64:
         return 1
     return max(1, min(pages // (3 if head_dim <= 64 else 2), compute_units // max(1, blocks), 16))
