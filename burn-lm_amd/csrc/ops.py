@@ -154,6 +154,8 @@ _SIGNATURES = {
     "blm_sink_attn_mfma_init": [],
     "blm_gemm_mfma": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                       _c_int, _c_int, _c_int, _c_void_p],
+    "blm_gemm_duo": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
+                     _c_void_p],
     "blm_gemv_mfma_group_limit": [_c_int],
     "blm_gemv_qkv_rope_supported": [_c_int, _c_int, _c_int, _c_int],
     "blm_gemv_qkv_rope": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p,
@@ -768,15 +770,18 @@ def static_scratch_init(device=None):
         _static_ready.add(index)
 
 
-def gemm_mfma(a, w, out, gated=False, tile=(128, 128), activation="silu"):
+def gemm_mfma(a, w, out, gated=False, tile=(128, 128), activation="silu", whole=None):
     """bfloat16 product for many rows on the matrix cores: out = a[M, K] @ w[N, K]^T, with w as the
     checkpoint stores it.  out: bfloat16 or float32 [M, N], or float32 [groups, M, N] partial
     products over that many groups of K (the reader sums them).  gated=True: w is [gate rows; up
     rows] ([2I, K]) and out is [M, I] = act(a gate^T) * (a up^T), act = silu or (activation="gelu_tanh") the tanh form
     of GELU.  tile: rows x columns of out (of
     gate and up columns together when gated) per block, one of GEMM_TILES; a third number is the depth of
-    the ring of K stages (deep rings for products of few tiles, which wait for memory, not for the matrix cores)."""
+    the ring of K stages (deep rings for products of few tiles, which wait for memory, not for the matrix cores).
+    Tiles of 256x256 are gemm_duo's where it takes the operands (`whole`: see there)."""
     _gpu(a, w, out)
+    if tile == (256, 256) and w.dim() == 2 and gemm_duo_takes(a, w, out, gated):
+        return gemm_duo(a, w, out, gated=gated, activation=activation, whole=whole)
     gemm_mfma_init(a.device)
     groups = 1
     if out.dim() == 3:
@@ -796,6 +801,49 @@ def gemm_mfma(a, w, out, gated=False, tile=(128, 128), activation="silu"):
     _call("blm_gemm_mfma", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out), M, N, K, a.stride(0), w.stride(0),
           out.stride(-2), (2 if activation == "gelu_tanh" else 1) if gated else 0, groups, GEMM_TILES[tile], _stream())
     return out
+
+
+def gemm_duo_takes(a, w, out, gated=False):
+    """Whether gemm_duo takes these operands."""
+    K, N = a.shape[1], out.shape[-1]
+    groups = out.shape[0] if out.dim() == 3 else 1
+    each = -(-(-(-K // groups)) // 128) * 128
+    return (a.dtype == w.dtype == torch.bfloat16 and (out.dtype == torch.bfloat16 or not gated) and K % 128 == 0 and K - (groups - 1) * each >= 256
+            and N % 8 == 0 and a.stride(1) == w.stride(1) == out.stride(-1) == 1
+            and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and out.stride(-2) % 8 == 0
+            and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 0
+            and (2 if gated else 1) * N * w.stride(0) * 2 < 1 << 32 and 256 * a.stride(0) * 2 < 1 << 32)
+
+
+def gemm_duo(a, w, out, gated=False, activation="silu", whole=None):
+    """bfloat16 product of long prompts: out[M, N] = a[M, K] @ w[N, K]^T in tiles of 256x256, of which `whole` (all unless told
+    otherwise) are one block's and the others two blocks' with half the rows each.  K in multiples of 128, N of 8.  out: bfloat16, or
+    float32 [M, N], or float32 [groups, M, N] partial products over that many groups of K.  gated=True: w is [gate rows; up rows]
+    ([2N, K]) and out (bfloat16) is act(a gate^T) * (a up^T), act as in gemm_mfma."""
+    _gpu(a, w, out)
+    groups = 1
+    if out.dim() == 3:
+        groups = out.shape[0]
+        if out.dtype != torch.float32 or not out.is_contiguous():
+            raise KernelError("gemm_duo: partial outputs must be contiguous float32 [groups, M, N]")
+    M, N = out.shape[-2:]
+    K = a.shape[1]
+    if a.shape[0] != M or w.dim() != 2 or w.shape != (N * (2 if gated else 1), K):
+        raise KernelError(f"gemm_duo: shapes a={tuple(a.shape)} w={tuple(w.shape)} out={tuple(out.shape)} do not fit")
+    if a.stride(1) != 1 or w.stride(1) != 1 or out.stride(-1) != 1:
+        raise KernelError("gemm_duo: a, w and out need unit stride along their rows")
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+        raise KernelError("gemm_duo: operands must be bfloat16")
+    _call("blm_gemm_duo", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out), M, N, K, a.stride(0), w.stride(0), out.stride(-2),
+          (2 if activation == "gelu_tanh" else 1) if gated else 0, groups, gemm_duo_tiles(M, N, gated)[0] if whole is None else whole, _stream())
+    return out
+
+
+def gemm_duo_tiles(M, N, gated=False):
+    """(tiles of 256x256, halves below them): a last row of tiles of at most 128 rows is halves only."""
+    columns = -(-N // (128 if gated else 256))
+    tail = 0 < M % 256 <= 128
+    return (M // 256 if tail else -(-M // 256)) * columns, columns if tail else 0
 
 
 _rows_ready = set()

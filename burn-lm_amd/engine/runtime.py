@@ -115,6 +115,30 @@ def f32_plan(M, N, K, compute_units, planes=False, gated=False):
     return best
 
 
+# ops.gemm_duo: what half a tile takes of a whole one's time (K = 2048 / 8192, all blocks at once: 22 of 38 us, 73 of 128), and how
+# full the rounds of tiles must be for it to be the faster one: for a gated product (against the library's and the gating pass), for
+# a plain one whose last round is of whole tiles and for one round of halves (see gated_linear and duo_product).
+DUO_HALF = 0.57
+DUO_GATED_FILL = 0.62
+DUO_WHOLE_FILL = 0.93
+DUO_HALVES_FILL = 0.74
+DUO_WHOLE_K = 3072
+DUO_PLANES_K = 4096
+
+
+@functools.lru_cache(maxsize=4096)
+def duo_plan(M, N, compute_units, gated=False):
+    """(whole tiles, rounds, fill) of ops.gemm_duo: the tiles that do not fill a round run as halves where that is shorter; rounds in
+    the time of a whole tile; fill: the share of the rounds' time that works on rows and columns that exist."""
+    tiles, tail = ops.gemm_duo_tiles(M, N, gated)
+    full, rest = divmod(tiles, compute_units)
+    left = compute_units - rest if rest else 0            # units that a last, partial round of whole tiles leaves to the tail
+    whole = full + (1 if rest else 0) + DUO_HALF * -(-max(0, tail - left) // compute_units)
+    halves = full + DUO_HALF * -(-(2 * rest + tail) // compute_units)
+    rounds = min(whole, halves)
+    return tiles if whole <= halves else tiles - rest, rounds, M * N / (32768.0 if gated else 65536.0) / compute_units / rounds
+
+
 class FusedProjectionPlan:
     """Launch geometry of a projection that a part fuses with work of its own (Runtime.qkv_plan).
     kernel: "rows" (ops.gemm_rows_qkv_rope's geometry: `rows` rows staged per block, `columns` columns
@@ -454,6 +478,16 @@ class Runtime:
             groups, tile = self.mid_planes_plan(M, N, K)
             if groups:
                 return ops.gemm_mfma(x, w, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), tile=tile)
+        if planes and M > MID_PLANES_MAX_ROWS and plain_bf16 and self.fused_gate_up_measured and K >= DUO_PLANES_K:
+            # the down projection of long prompts: halves of tiles over two groups of K where these nearly fill one round (2,048
+            # rows, width 2048, K = 8192, within a prompt: 68 us and 2.6 more in the norm that adds the planes, the library's 79.6;
+            # with half the units idle or a second round behind: 1,000 rows 47 / 46 and 2,166 rows 98 / 73)
+            tiles, tail = ops.gemm_duo_tiles(M, N)
+            if DUO_HALVES_FILL * self.compute_units <= 2 * (2 * tiles + tail) <= self.compute_units:
+                out = torch.empty(2, M, N, dtype=torch.float32, device=x.device)
+                if ops.gemm_duo_takes(x, w, out):
+                    return ops.gemm_duo(x, w, out, whole=0)
+                out = None
         if (planes and self.rows_ring and 16 < M <= MFMA_SKINNY_MAX_ROWS and plain_bf16
                 and (M > 32 or K <= 4096 or -(-N // 32) * 8 <= 3 * self.compute_units)):
             # 17 to 64 rows as partial planes (measured against the packed skinny kernel at the 1B, 3B and 8B
@@ -511,9 +545,32 @@ class Runtime:
         if M <= SKINNY_MAX_ROWS and aligned:
             return ops.gemv_skinny(x, w, out)
         if out_dtype == torch.bfloat16:
+            if plain_bf16 and self.fused_gate_up_measured and self.duo_product(M, N, K) and ops.gemm_duo_takes(x, w, out):
+                return ops.gemm_duo(x, w, out, whole=duo_plan(M, N, self.compute_units)[0])
             return torch.matmul(x, w.t(), out=out)
         # float32 logits from bfloat16 operands with many rows: own kernel (float accumulation)
         return ops.gemm_tiled(x, w, out)
+
+    def duo_product(self, M, N, K):
+        """Whether a plain bfloat16 product of many rows goes to ops.gemm_duo and not to the library (us, duo / library):
+        * one round of halves, at least DUO_HALVES_FILL of the units busy: [3072, 2048] 2,048 and 2,560 rows 26.9 / 26.8 and
+          29.3 / 31.0; [2048, 8192] 3,300 and 4,096 rows 87 / 99 and 99 / 107; [5120, 3072] 1,300 and 1,536 rows 38 / 41 and
+          39 / 42 (less full: [2048, 8192] 2,560 rows 83 / 75);
+        * whole rounds and a last one of halves: [5120, 3072] 3,300, 4,096, 6,500 and 7,700 rows 99 / 110, 103 / 112, 149 / 200 and
+          174 / 277; [3072, 3072] 6,500 and 7,700 rows 103 / 101 and 109 / 117; [3072, 8192] 247 / 251 and 267 / 288; [2048, 8192]
+          9,681 rows 249 / 262;
+        * whole rounds, the last nearly full, K up to DUO_WHOLE_K: [5120, 3072] 9,681 rows 207 / 323, 9,200 rows 199 / 196;
+          [6144, 2048] 7,700 and 8,192 rows 142 / 139 and 143 / 141 (beyond that K 3-7 % behind: [6144, 4096] 8,192 rows 278 / 260;
+          and with a last round less full as much: [3072, 3072] 9,681 rows 138 / 131)."""
+        if M <= MFMA_SKINNY_MAX_ROWS:
+            return False
+        whole, rounds, fill = duo_plan(M, N, self.compute_units)
+        if rounds <= DUO_HALF:
+            return fill >= DUO_HALVES_FILL
+        tiles = ops.gemm_duo_tiles(M, N)[0]
+        if whole < tiles and tiles >= self.compute_units:
+            return True
+        return fill >= DUO_WHOLE_FILL and K <= DUO_WHOLE_K
 
     def _gated_by_library(self, M, K, inner):
         """17 to 64 rows of a gated product that are better left to the library's product and the gating kernel:
@@ -575,6 +632,16 @@ class Runtime:
                 if self.compute_units // 4 <= blocks <= self.compute_units:
                     return ops.gemm_mfma(x, plain, torch.empty(M, inner, dtype=self.dtype, device=x.device),
                                          gated=True, tile=tile, activation=activation)
+            # Longer prompts: tiles of 256x256, the ones that do not fill a round as halves (ops.gemm_duo), where the rounds are
+            # full enough (us against the library's product and the gating pass, inner size 8192: width 2048, 512 / 1,000 / 1,300 /
+            # 2,048 / 2,166 / 9,681 rows 31 / 43, 51 / 67, 76 / 97, 100 / 120, 118 / 146, 449 / 625; width 3072, 700 / 2,048 / 9,681
+            # rows 69 / 73, 152 / 176, 665 / 863; width 4096, inner size 14336, 400 / 1,300 / 4,096 rows 87 / 94, 262 / 277,
+            # 654 / 701; too little is full: that shape with 260 rows 86 / 71).
+            if M > 256:
+                whole, _, fill = duo_plan(M, inner, self.compute_units, True)
+                out = torch.empty(M, inner, dtype=self.dtype, device=x.device)
+                if fill >= DUO_GATED_FILL and ops.gemm_duo_takes(x, plain, out, gated=True):
+                    return ops.gemm_mfma(x, plain, out, gated=True, tile=(256, 256), activation=activation, whole=whole)
             # 256x128 tiles that make one round on at least three quarters of the compute units, with rows
             # that fill their tiles to 85 % and more: measured against the library's product and the gating
             # kernel 11-16 % faster with a full round (512 rows of an inner size of 8192 at widths 2048 and
@@ -586,7 +653,7 @@ class Runtime:
             if M > 256 and M * 20 >= m256 * 256 * 17 and self.compute_units * 3 // 4 <= blocks <= self.compute_units:
                 return ops.gemm_mfma(x, plain, torch.empty(M, inner, dtype=self.dtype, device=x.device),
                                      gated=True, tile=(256, 128), activation=activation)
-            # Long prompts: with whole rounds of 256x256 tiles (as many blocks as compute units, or a
+            # Long prompts of a width that is no multiple of 128: with whole rounds of 256x256 tiles (as many blocks as compute units, or a
             # multiple) and a narrow model the fused kernel is ahead of the library over the whole
             # prefill (width 2048: 2-4 % at 1,024 and 2,048 rows, 0.5-0.8 % at 3,072 and 4,096; behind by
             # 2-6 % with a partial last round, and at width 3072 behind from 1,536 rows on).  Beyond

@@ -1,0 +1,105 @@
+"""The 256x256 product of long prompts (ops.gemm_duo): whole tiles and halves, edges in rows and columns, groups of K, gating; and the
+plan that chooses between whole tiles and halves."""
+import pytest
+import torch
+
+
+def test_plan_covers_every_tile():
+    """Whole tiles and halves together are all tiles; a plan is never longer than whole tiles alone; its fill is a share."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.runtime import DUO_HALF, duo_plan
+    for gated in (False, True):
+        for M in (1, 128, 129, 256, 257, 511, 512, 1000, 2048, 2166, 4097, 9681):
+            for N in (8, 256, 264, 2048, 3072, 8192, 14336):
+                tiles, tail = ops.gemm_duo_tiles(M, N, gated)
+                columns = -(-N // (128 if gated else 256))
+                assert tiles * 2 + tail >= -(-M // 128) * columns and tail in (0, columns)
+                whole, rounds, fill = duo_plan(M, N, 256, gated)
+                assert whole in (tiles, tiles - tiles % 256) and 0 < fill <= 1 / (2 * DUO_HALF) + 1e-9 or rounds > DUO_HALF and fill <= 1
+                assert rounds <= -(-(tiles + tail) // 256) + 1e-9
+
+
+def operands(M, N, K, gated, seed):
+    g = torch.Generator().manual_seed(seed)
+    a = torch.randn(M, K + 16, generator=g).bfloat16().cuda()[:, 8:K + 8]          # rows of a wider buffer
+    w = (torch.randn(N * (2 if gated else 1), K, generator=g) * K ** -0.5).bfloat16()
+    w[N // 2, K - 8:] = 3.0                                                        # a wrong order of operands cannot hide
+    return a, w.cuda()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 8, 256), (128, 256, 256), (129, 264, 384), (256, 512, 256), (300, 248, 1152), (513, 1000, 384), (2100, 520, 512)])
+@pytest.mark.parametrize("activation", [None, "silu", "gelu_tanh"])
+def test_whole_tiles_and_halves(M, N, K, activation):
+    """Every mix of whole tiles and halves gives the float64 product rounded to bfloat16 (half a step of 2^-8 of the value, and
+    float32 sums: 1e-5), and the same bits."""
+    from burn_lm_amd.csrc import ops
+    gated = activation is not None
+    a, w = operands(M, N, K, gated, M + N)
+    want = a.double() @ w.double().T
+    if gated:
+        gate, up = want.chunk(2, 1)
+        want = (torch.nn.functional.silu(gate) if activation == "silu" else torch.nn.functional.gelu(gate, approximate="tanh")) * up
+    tiles, _ = ops.gemm_duo_tiles(M, N, gated)
+    first = None
+    for whole in sorted({0, tiles // 2, tiles}):
+        big = torch.full((M, N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.gemm_duo(a, w, big[:, :N], gated=gated, activation=activation or "silu", whole=whole)
+        assert bool((big[:, N:] == 7.0).all())
+        got = big[:, :N]
+        # the gating's own float32 functions are within 2^-21 of a value of a few units
+        assert float(((got.double() - want).abs() / (want.abs() + want.abs().mean())).max()) <= 2.0 ** -8
+        first = got if first is None else first
+        assert torch.equal(got, first)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,groups", [(300, 264, 256, 1), (257, 136, 1152, 2), (640, 256, 2048, 4)])
+def test_partial_planes(M, N, K, groups):
+    """Float32 planes over groups of K, the last one shorter, as whole tiles and as halves: their sum is the product to float32's sums."""
+    from burn_lm_amd.csrc import ops
+    a, w = operands(M, N, K, False, K)
+    want = a.double() @ w.double().T
+    for whole in (0, None):
+        out = torch.full((groups, M, N), 7.0, device="cuda")
+        ops.gemm_duo(a, w, out, whole=whole)
+        assert float((out.double().sum(0) - want).abs().max() / want.abs().max()) <= 2e-6
+
+
+@pytest.mark.gpu
+def test_refuses_what_it_cannot_do():
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.csrc.ops import KernelError
+    a, w, out = (torch.zeros(n, k, dtype=torch.bfloat16, device="cuda") for n, k in ((300, 256), (264, 256), (300, 264)))
+    assert ops.gemm_duo_takes(a, w, out) and not ops.gemm_duo_takes(a[:, :192], w[:, :192], out)
+    assert not ops.gemm_duo_takes(a.flatten()[4:-252].view(-1, 256), w, out[:299])                  # off a multiple of 16 bytes
+    assert not ops.gemm_duo_takes(a, w, torch.zeros(2, 300, 264, device="cuda"))                     # a group needs 256 of K
+    for bad in (dict(whole=99), dict(whole=-1)):
+        with pytest.raises(KernelError, match="whole tiles"):
+            ops.gemm_duo(a, w, out, **bad)
+    with pytest.raises(KernelError, match="not supported"):
+        ops.gemm_duo(a[:, :192], w[:, :192], out)
+    with pytest.raises(KernelError, match="do not fit"):
+        ops.gemm_duo(a, w[:256], out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(3300, 2048, 512), (2048, 2048, 4096), (1000, 8192, 256)])
+def test_products_of_long_prompts_take_it(monkeypatch, M, N, K):
+    """The runtime's products reach it where its plan says so, and give what the plain product gives."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.runtime import Runtime
+    rt = Runtime(torch.bfloat16, "cuda:0")
+    a, w = operands(M, N, K, False, 5)
+    calls, real = [], ops.gemm_duo
+    monkeypatch.setattr(ops, "gemm_duo", lambda *x, **k: (calls.append(1), real(*x, **k))[1])
+    want = a.double() @ w.double().T
+    for planes in (False, True):
+        got = rt.linear(a, rt.weight(w), partials=planes)
+        got = got.double().sum(0) if got.dim() == 3 else got.double()
+        assert float(((got - want).abs() / (want.abs() + want.abs().mean())).max()) <= 2.0 ** -8
+    inner = N // 2
+    gate, up = want.chunk(2, 1)
+    want = torch.nn.functional.silu(gate) * up
+    got = rt.gated_linear(a, rt.weight(w, gated=True))
+    assert calls and float(((got.double() - want).abs() / (want.abs() + want.abs().mean())).max()) <= 2.0 ** -7 and got.shape == (M, inner)
