@@ -4,16 +4,16 @@
 //   moe_gemm 0 : gate and up of an expert's tokens, gathered; silu(gate) * up * weight as bfloat16 rows, expert by expert
 //   moe_gemm 1 : the down projection of these rows into float32 planes, one for each place: [top][T][D], which the reader of the
 //                feed-forward's result adds up (a token's places that are not taken are zeroed by moe_lists)
-// What bounds it: 256 x 128 tiles by eight wavefronts share the compute unit's LDS between the direct loads (48 KB a stage), the
-// wavefronts' reads (128 KB) and 1,024 cycles of matrix instructions; a stage takes 0.75 us, and with 16 experts of 512 rows each
-// the tiles' last rows and the last round of blocks are a quarter of the time.
-// Measured (us a call by events over repeated calls, 2,048 tokens, 16 experts of 512 at width 2048, 4 chosen; before: the stacked
-// products and the gating pass): gate/up with gating 122 -> 61, down 77 -> 41, lists 6.5 (within a whole prompt, under the profiler,
-// 66, 47 and 6.3).  Tried: 128 x 128 tiles, two blocks a unit (stages of 32: 70 and 43),
-// the compiler's own order of reads, loads and products (72 and 44), four wavefronts of 128 x 64 (83 and 54).
-#include <type_traits>
-
-#include "common.h"
+// Many rows run on the 256x256 tiles of gemm_duo.h (moe_duo_kernel), few rows and other widths on 256 x 128 tiles (moe_gemm_kernel;
+// the rule stands at the launch).  What bounds them: with 512 rows an expert, more or less, the last tile of an expert is a half that is
+// nearly empty, and 128 whole tiles and 36 halves are one round on 256 units; the down projection writes 67 MB of planes.
+// The 256 x 128 tiles by eight wavefronts share the compute unit's LDS between the direct loads (48 KB a stage), the wavefronts' reads
+// (128 KB) and 1,024 cycles of matrix instructions; a stage takes 0.75 us, and the last round of blocks is a quarter of the time.
+// Measured within a whole prompt, under the profiler (us, 2,048 tokens, 16 experts of 512 at width 2048, 4 chosen; the stacked products
+// and the gating pass / 256 x 128 / 256 x 256): gate/up with gating 122 / 65 / 49, down 77 / 46.5 / 38.4; lists 6.3.
+// Tried for 256 x 128: 128 x 128 tiles, two blocks a unit (stages of 32: 70 and 43), the compiler's own order of reads, loads and
+// products (72 and 44), four wavefronts of 128 x 64 (83 and 54).
+#include "gemm_duo.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 mg_bf16x8;
 typedef __attribute__((ext_vector_type(16))) float mg_f32x16;
@@ -23,6 +23,10 @@ typedef __attribute__((ext_vector_type(4))) unsigned int mg_u32x4;
 #define MG_BK 64
 #define MG_WAVES 8
 #define MG_MAX_EXPERTS 256
+
+// The same in both tiles, whose products are the same bits: a token's result does not depend on how many there are.  The hardware's
+// exponential and reciprocal, an ulp each, in front of the rounding to bfloat16 (expf and a division: 2,048 tokens 92 us, so 88).
+__device__ __forceinline__ float mg_gated(float g, float up, float weight) { return gd_silu(g) * up * weight; }
 
 // weights [T][ld]: an expert's weight for a token, zero where it is not chosen.  lists [E][T]: plane rows place * T + token of
 // the tokens that chose expert e; counts [E].  Blocks behind the first E zero the plane rows of places that no expert takes.
@@ -235,7 +239,7 @@ __global__ void __launch_bounds__(64 * MG_WAVES, 2)
       const int m = wm + i * 32 + 8 * (v >> 2) + 4 * hb + (v & 3);
       if (MODE == 0) {
         const int n = n0 + wn / 2 + c;
-        const float g = acc[i][0][v], y = g / (1.0f + expf(-g)) * acc[i][1][v] * row_weight[m];
+        const float y = mg_gated(acc[i][0][v], acc[i][1][v], row_weight[m]);
         if (m < rows && n < N) act[(size_t)(first + m0 + m) * N + n] = from_float<bf16>(y);
       } else {
 #pragma unroll
@@ -247,12 +251,148 @@ __global__ void __launch_bounds__(64 * MG_WAVES, 2)
     }
 }
 
+// The same products in the tiles of gemm_duo.h, 256 rows and 256 columns (MODE 0: 128 gates and their ups).  An expert's rows are
+// whole tiles and, where at most 128 are left, a half; or halves all of them where those come in fewer rounds on the `units`.
+template <int MODE>
+struct MgTile {
+  const char *a, *b;
+  const int* list;                            // MODE 0: the tokens of the tile's rows
+  int rows, n0, N, lda, ldw;
+  uint32_t up;
+  __device__ __forceinline__ uint32_t row(int m) const {
+    m = min(m, rows - 1);
+    return (uint32_t)(MODE == 0 ? list[m] : m) * (uint32_t)lda * 2u;
+  }
+  __device__ __forceinline__ uint32_t column(int r, int h) const {
+    const int n = min(n0 + (MODE == 0 ? r : r / 32 * 64 + h * 32 + r % 32), N - 1);
+    return (uint32_t)n * (uint32_t)ldw * 2u + (MODE == 0 && h ? up : 0u);
+  }
+};
+
+template <int MODE, int TILES>
+__device__ __forceinline__ void mg_store(const gd_f32x4 (&acc)[TILES][4], bf16* act, float* planes, const int* list, const float* row_weight,
+                                         int m0, int rows, int n0, int N, int lane) {
+  const int l16 = lane & 15, quad = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < TILES; ++i) {
+    const int m = m0 + i * 16 + l16;
+    if (MODE == 0) {
+      float v[2][4];
+      const float w = row_weight[m];
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[x][e] = mg_gated(acc[i][x][e], acc[i][2 + x][e], w);
+      const uint4 eight = gd_eight(v);
+      const int n = n0 + (quad & 1) * 16 + (quad >> 1) * 8;
+      if (m < rows && n < N) *reinterpret_cast<uint4*>(act + (size_t)m * N + n) = eight;
+    } else {
+      const int to = list[m];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int n = n0 + j * 16 + quad * 4;
+        if (m < rows && n < N) *reinterpret_cast<float4*>(planes + (size_t)to * N + n) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+      }
+    }
+  }
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(512, 2)
+    moe_duo_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw, const float* __restrict__ weights, int ld_weights,
+                   const int* __restrict__ lists, const int* __restrict__ counts, bf16* __restrict__ act, float* __restrict__ planes,
+                   int T, int E, int N, int K, int inner, int n_tiles, int units) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[9 * GD_REGION];
+  __shared__ int list[GD_TILE];
+  __shared__ float row_weight[GD_TILE];
+  __shared__ int sums[4][8], found[4];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / BLM_WAVE), lane = tid & (BLM_WAVE - 1);
+  // a thread for each expert: its whole tiles, its half behind them, its halves if it has nothing else, its rows; and by a scan
+  // those of the experts before it
+  const int mine = tid < E ? counts[tid] : 0, over = mine % GD_TILE;
+  const int own[4] = {mine / GD_TILE + (over > GD_TILE / 2), over > 0 && over <= GD_TILE / 2, (mine + GD_TILE / 2 - 1) / (GD_TILE / 2), mine};
+  int upto[4], all[4];
+#pragma unroll
+  for (int x = 0; x < 4; ++x) upto[x] = own[x];
+#pragma unroll
+  for (int d = 1; d < BLM_WAVE; d *= 2) {
+    int before[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) before[x] = __shfl_up(upto[x], d);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) upto[x] += lane >= d ? before[x] : 0;
+  }
+  if (lane == BLM_WAVE - 1)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) sums[x][wave] = upto[x];
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    all[x] = 0;
+    for (int w = 0; w < 8; ++w) {
+      if (w < wave) upto[x] += sums[x][w];
+      all[x] += sums[x][w];
+    }
+  }
+  // rounds in hundredths of a whole tile's time, a half 57 of them (see gemm_duo.hip)
+  const int wholes = all[0] * n_tiles, rest = wholes % units, beside = rest ? units - rest : 0;
+  const int mixed = wholes / units * 100 + (rest ? 100 : 0) + (max(0, all[1] * n_tiles - beside) + units - 1) / units * 57;
+  const bool halved = (all[2] * n_tiles + units - 1) / units * 57 < mixed;
+  const int share1 = halved ? 0 : (wholes + 7) / 8, count2 = all[halved ? 2 : 1] * n_tiles, share2 = (count2 + 7) / 8;
+  int b = blockIdx.x;
+  const bool half = b >= share1 * 8;
+  if (half) b -= share1 * 8;
+  const int share = half ? share2 : share1, id = (b & 7) * share + (b >> 3);       // a die has a stretch of the tiles
+  if ((b >> 3) >= share || id >= (half ? count2 : wholes)) return;
+  const int nt = id % n_tiles, tile = id / n_tiles;
+  const int kind = half ? (halved ? 2 : 1) : 0;
+  const int last = kind == 0 ? upto[0] : kind == 1 ? upto[1] : upto[2], has = kind == 0 ? own[0] : kind == 1 ? own[1] : own[2];
+  if (tile < last && tile >= last - has) {
+    const int nth = tile - (last - has);
+    found[0] = tid;
+    found[1] = kind == 0 ? nth * GD_TILE : kind == 1 ? mine / GD_TILE * GD_TILE : nth * (GD_TILE / 2);
+    found[2] = upto[3] - mine;
+    found[3] = mine;
+  }
+  __syncthreads();
+  const int e = __builtin_amdgcn_readfirstlane(found[0]), m0 = __builtin_amdgcn_readfirstlane(found[1]);
+  const int first = __builtin_amdgcn_readfirstlane(found[2]) + m0;
+  const int rows = min(half ? GD_TILE / 2 : GD_TILE, __builtin_amdgcn_readfirstlane(found[3]) - m0);
+  const int n0 = nt * (MODE == 0 ? GD_TILE / 2 : GD_TILE), wm = wave >> 2, wn = wave & 3;
+  if (tid < GD_TILE) {
+    const int to = lists[(size_t)e * T + m0 + min(tid, rows - 1)];
+    list[tid] = MODE == 0 ? to % T : to;
+    if (MODE == 0) row_weight[tid] = weights[(size_t)(to % T) * ld_weights + e];
+  }
+  __syncthreads();
+  MgTile<MODE> t;
+  t.a = reinterpret_cast<const char*>(MODE == 0 ? A : A + (size_t)first * lda);
+  t.b = reinterpret_cast<const char*>(MODE == 0 ? W + (size_t)e * N * ldw : W + (size_t)e * K);
+  t.list = list;
+  t.rows = rows;
+  t.n0 = n0;
+  t.N = N;
+  t.lda = lda;
+  t.ldw = ldw;
+  t.up = (uint32_t)inner * (uint32_t)ldw * 2u;
+  const int n = n0 + wn * (MODE == 0 ? 32 : 64);
+  if (!half) {
+    gd_f32x4 acc[8][4];
+    gd_whole(acc, t, K / GD_BK, lds, wave, lane);
+    mg_store<MODE, 8>(acc, act + (size_t)first * N, planes, list, row_weight, wm * 128, rows, n, N, lane);
+  } else {
+    gd_f32x4 acc[4][4];
+    gd_half(acc, t, K / GD_BK, lds, wave, lane);
+    mg_store<MODE, 4>(acc, act + (size_t)first * N, planes, list, row_weight, wm * 64, rows, n, N, lane);
+  }
+}
+
 // x [T][ldx], w_gate_up [2 E f][D] (the experts' gates, then their ups), w_down [D][E f], weights [T][ld_weights] float;
 // planes [top][T][D] float; lists [E * T], counts [E] ints and act [T * top][f] are workspaces of the call.  No token has more
 // than top weights that are not zero.
 extern "C" int blm_moe_grouped(const void* x, int ldx, const void* w_gate_up, const void* w_down, const float* weights, int ld_weights,
                                float* planes, int* lists, int* counts, void* act, int T, int D, int E, int f, int top,
-                               hipStream_t stream) {
+                               int units, hipStream_t stream) {
   BLM_REQUIRE(T > 0 && E > 0 && E <= MG_MAX_EXPERTS && top > 0 && top <= 64 && top <= E && D % MG_BK == 0 && f % MG_BK == 0 && D > 0 && f > 0,
               "moe_grouped: sizes T=%d D=%d experts=%d of %d, top=%d not supported", T, D, E, f, top);
   BLM_REQUIRE(ldx >= D && ldx % 8 == 0 && ld_weights >= E && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w_gate_up % 16) == 0 &&
@@ -262,13 +402,34 @@ extern "C" int blm_moe_grouped(const void* x, int ldx, const void* w_gate_up, co
   hipLaunchKernelGGL(moe_lists_kernel, dim3((unsigned)(E + (T + 63) / 64)), dim3(1024), 0, stream, weights, ld_weights, T, E, top, lists, counts, planes, D);
   BLM_LAUNCH_CHECK("moe_lists");
   const long long row_tiles = ((long long)T * top + MG_BM - 1) / MG_BM + E;       // every expert's last tile may be part empty
-  const int gu_tiles = (f + MG_BN / 2 - 1) / (MG_BN / 2), down_tiles = (D + MG_BN - 1) / MG_BN;
-  BLM_REQUIRE(row_tiles * (gu_tiles > down_tiles ? gu_tiles : down_tiles) < 2147483647LL - 8, "moe_grouped: too many tiles");
-  hipLaunchKernelGGL((moe_gemm_kernel<0>), dim3((unsigned)((row_tiles * gu_tiles + 7) / 8 * 8)), dim3(64 * MG_WAVES), 0, stream, (const bf16*)x, ldx,
-                     (const bf16*)w_gate_up, D, weights, ld_weights, lists, counts, (bf16*)act, planes, T, E, f, D, E * f, gu_tiles);
-  BLM_LAUNCH_CHECK("moe_gemm gate/up");
-  hipLaunchKernelGGL((moe_gemm_kernel<1>), dim3((unsigned)((row_tiles * down_tiles + 7) / 8 * 8)), dim3(64 * MG_WAVES), 0, stream, (const bf16*)act, f,
-                     (const bf16*)w_down, E * f, weights, ld_weights, lists, counts, (bf16*)act, planes, T, E, D, f, E * f, down_tiles);
-  BLM_LAUNCH_CHECK("moe_gemm down");
+  const long long halves = ((long long)T * top + GD_TILE / 2 - 1) / (GD_TILE / 2) + E;
+  BLM_REQUIRE(units > 0 && halves * ((D + 63) / 64 > (f + 63) / 64 ? (D + 63) / 64 : (f + 63) / 64) < 2147483647LL / 64, "moe_grouped: too many tiles");
+  // Tiles of 256x256 where K is one of theirs (multiples of 128), a pair of gate and up rows lies within 4 GiB and there is enough of
+  // them: gate/up from halves (an expert's last one half full) on two fifths of the units on, down from as many halves as units.
+  // Gate/up and down together, 16 experts of 512 at width 2048, 4 chosen, both by the smaller tiles / both by these / as the rule
+  // has it, us: 400 tokens 52 / 58 / 52, 512: 55 / 60 / 55, 600: 58 / 58 / 57, 800: 63 / 59 / 59, 1,000: 76 / 69 / 69, 1,500: 72 / 72 / 72,
+  // 2,048: 113 / 90 / 90, 8,000: 330 / 261 / 261.
+  const long long about = ((long long)T * top + (GD_TILE / 4) * E) / (GD_TILE / 2);
+  const int duo_gates = (f + GD_TILE / 2 - 1) / (GD_TILE / 2), duo_columns = (D + GD_TILE - 1) / GD_TILE;
+  if (D % 128 == 0 && D >= 256 && ((long long)E * f + f) * D * 2 < (1LL << 32) && about * duo_gates * 5 >= units * 2LL) {
+    const int tiles = duo_gates;
+    hipLaunchKernelGGL((moe_duo_kernel<0>), dim3((unsigned)(halves * tiles + 16)), dim3(512), 0, stream, (const bf16*)x, ldx, (const bf16*)w_gate_up, D, weights,
+                       ld_weights, lists, counts, (bf16*)act, planes, T, E, f, D, E * f, tiles, units);
+  } else {
+    const int tiles = (f + MG_BN / 2 - 1) / (MG_BN / 2);
+    hipLaunchKernelGGL((moe_gemm_kernel<0>), dim3((unsigned)((row_tiles * tiles + 7) / 8 * 8)), dim3(64 * MG_WAVES), 0, stream, (const bf16*)x, ldx,
+                       (const bf16*)w_gate_up, D, weights, ld_weights, lists, counts, (bf16*)act, planes, T, E, f, D, E * f, tiles);
+  }
+  BLM_LAUNCH_CHECK("moe_grouped gate/up");
+  if (f % 128 == 0 && f >= 256 && about * duo_columns >= units) {
+    const int tiles = duo_columns;
+    hipLaunchKernelGGL((moe_duo_kernel<1>), dim3((unsigned)(halves * tiles + 16)), dim3(512), 0, stream, (const bf16*)act, f, (const bf16*)w_down, E * f, weights,
+                       ld_weights, lists, counts, (bf16*)act, planes, T, E, D, f, E * f, tiles, units);
+  } else {
+    const int tiles = (D + MG_BN - 1) / MG_BN;
+    hipLaunchKernelGGL((moe_gemm_kernel<1>), dim3((unsigned)((row_tiles * tiles + 7) / 8 * 8)), dim3(64 * MG_WAVES), 0, stream, (const bf16*)act, f,
+                       (const bf16*)w_down, E * f, weights, ld_weights, lists, counts, (bf16*)act, planes, T, E, D, f, E * f, tiles);
+  }
+  BLM_LAUNCH_CHECK("moe_grouped down");
   return 0;
 }

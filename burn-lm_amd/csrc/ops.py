@@ -4,6 +4,7 @@ current HIP stream.  There is no fallback: without the library, or off the GPU, 
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 
 import torch
@@ -51,7 +52,7 @@ _SIGNATURES = {
                      _c_void_p, _c_int, _c_void_p],
     "blm_head_gate": [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_map_difference": [_c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_void_p],
-    "blm_moe_grouped": [_c_void_p, _c_int] + [_c_void_p] * 3 + [_c_int] + [_c_void_p] * 4 + [_c_int] * 5 + [_c_void_p],
+    "blm_moe_grouped": [_c_void_p, _c_int] + [_c_void_p] * 3 + [_c_int] + [_c_void_p] * 4 + [_c_int] * 6 + [_c_void_p],
     "blm_moe_table": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_int, _c_int, _c_void_p],
     "blm_sigmoid_gate": [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_gelu_glu": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
@@ -1606,6 +1607,11 @@ def moe_gate(gate_up, weights, out, n_experts, expert_inner):
 MOE_GROUPED_STEP, MOE_GROUPED_EXPERTS, MOE_GROUPED_TOP = 64, 256, 64
 
 
+@functools.lru_cache(maxsize=None)
+def compute_units(index):
+    return torch.cuda.get_device_properties(index).multi_processor_count
+
+
 def moe_grouped(x, w_gate_up, w_down, weights, n_experts, top):
     """float32 planes [top, T, D] whose sum is ``sum_e weights[t, e] * W_down_e (silu(W_gate_e x) * (W_up_e x))``: every token
     by its own experts only (those with a weight that is not zero, at most `top` of a token).  bfloat16 x [T, D], w_gate_up
@@ -1625,7 +1631,7 @@ def moe_grouped(x, w_gate_up, w_down, weights, n_experts, top):
     act = torch.empty(T * top, f, dtype=x.dtype, device=x.device)
     _call("blm_moe_grouped", x.data_ptr(), D, w_gate_up.data_ptr(), w_down.data_ptr(), weights.data_ptr(), n_experts + 1,
           planes.data_ptr(), lists.data_ptr(), lists.data_ptr() + 4 * n_experts * T, act.data_ptr(), T, D, n_experts, f, top,
-          _stream())
+          compute_units(x.device.index), _stream())
     return planes
 
 

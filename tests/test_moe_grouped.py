@@ -149,3 +149,14 @@ def test_no_more_memory_than_the_stacked_form():
     assert grouped(2048, 4096, 64, 64, 8)                                    # 0.3 GB
     assert not grouped(131072, 4096, 64, 64, 8)                              # 17 GB against 3
     assert grouped(65536, 2048, 512, 16, 4) and grouped(65536, 1024, 128, 128, 8)     # less than the stacked form
+
+
+@pytest.mark.parametrize("kind", ["all", "one", "missing"])
+@pytest.mark.parametrize("units", [8, 40, 256])
+@pytest.mark.parametrize("T,E,top,f,D", [(257, 3, 2, 256, 256), (700, 5, 2, 384, 640), (1030, 2, 1, 256, 264 * 128 // 88), (300, 64, 4, 256, 256)])
+def test_tiles_of_256(monkeypatch, T, E, top, f, D, units, kind):
+    """The tiles of 256x256: experts with whole tiles, a half behind them, or halves only (the fewer units, the more rounds there are to
+    choose by), with no rows at all, and columns that end within a tile.  The bound as above."""
+    from burn_lm_amd.csrc import ops
+    monkeypatch.setattr(ops, "compute_units", lambda index: units)
+    test_kernels(T, E, top, f, D, kind)
