@@ -12,7 +12,7 @@
 //
 // Kernels: the write of a step's tokens into the cache (RMS norm of the latent, rotation of the shared
 // key part and of the queries' rotated parts), a small batched product per head, and the attention.
-#include "common.h"
+#include "rows8.h"
 
 #include <type_traits>
 
@@ -83,6 +83,105 @@ __global__ void latent_write_kernel(const TA* __restrict__ down, int ld_down, co
   }
 }
 
+// The same for prompts (bfloat16, units of eight lanes): blocks for R8_TOKENS tokens' cache rows, of which each writes a quarter of the
+// latents and forms the norms for itself, and puts them into the transposed pages through shared memory; behind them a block a token
+// for the queries.  2,048 tokens of 16 heads'
+// 64 turning lanes, latents of 512: 16.9 us token by token, two bytes a store, so 11.3 (64 blocks with all of a row's
+// lanes each: 16.7; a wavefront's rows one after another: 28).
+__device__ __forceinline__ void lw_turn(const bf16* src, int d, int rot, int adjacent, const float* cs, float (&x)[8]) {
+  r8_load(src + d, x);
+  if (d >= rot) return;
+  float c[4], s[4];
+  if (adjacent) {
+    r8_angles(cs + d, c, s);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float u = x[2 * e], v = x[2 * e + 1];
+      x[2 * e] = u * c[e] - v * s[e];
+      x[2 * e + 1] = v * c[e] + u * s[e];
+    }
+    return;
+  }
+  const int half = rot / 2;
+  const bool first = d < half;
+  float y[8];
+  r8_load(src + (first ? d + half : d - half), y);
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    r8_angles(cs + 2 * (first ? d : d - half) + 8 * g, c, s);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[4 * g + e] = first ? x[4 * g + e] * c[e] - y[4 * g + e] * s[e] : x[4 * g + e] * c[e] + y[4 * g + e] * s[e];
+  }
+}
+
+template <typename TQ>
+__global__ void __launch_bounds__(256)
+    latent_write_prompt_kernel(const bf16* __restrict__ down, int ld_down, const bf16* __restrict__ q, int ld_q, int T, int H, int dn,
+                               const float* __restrict__ norm_w, float eps, const float* __restrict__ cos_sin, int half_t, int rot,
+                               TQ* __restrict__ qabs, bf16* __restrict__ kcache, bf16* __restrict__ vcache, const int* __restrict__ positions,
+                               const int* __restrict__ token_seq, const int* __restrict__ block_table, int table_width, int page_size, int R,
+                               int Dr, int adjacent, int q_lanes, int q_at, int tiles, int parts) {
+  extern __shared__ bf16 lw_values[];            // [R8_TOKENS][R / parts + 2]
+  if ((int)blockIdx.x >= tiles * parts) {
+    const int t = blockIdx.x - tiles * parts;
+    if (token_seq[t] < 0) return;
+    const float* cs = cos_sin + (size_t)positions[t] * half_t * 2;
+    const int units = Dr / 8;
+    for (int u = threadIdx.x; u < H * units; u += blockDim.x) {
+      const int h = u / units, d = (u - h * units) * 8;
+      float x[8];
+      lw_turn(q + (size_t)t * ld_q + (size_t)h * (dn + Dr) + dn, d, rot, adjacent, cs, x);
+      r8_store(qabs + ((size_t)t * H + h) * q_lanes + q_at + d, x);
+    }
+    return;
+  }
+  const int t0 = (int)blockIdx.x / parts * R8_TOKENS, part = blockIdx.x % parts, wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
+  constexpr int ROWS = R8_TOKENS / 4;            // of a wavefront; all of them are asked for at once, and the look-ups beside them
+  const int from = R / parts * part, to = R / parts * (part + 1), stride = R / parts + 2, d = lane * 8;
+  uint4 raw[ROWS];
+#pragma unroll
+  for (int x = 0; x < ROWS; ++x) {
+    raw[x] = make_uint4(0u, 0u, 0u, 0u);
+    if (d < R) raw[x] = *reinterpret_cast<const uint4*>(down + (size_t)min(t0 + wave * ROWS + x, T - 1) * ld_down + d);
+  }
+  float w[8] = {};
+  if (d < R) r8_load(norm_w + d, w);
+  const int mine = min(t0 + wave * ROWS + (lane & (ROWS - 1)), T - 1), my_seq = token_seq[mine], my_pos = positions[mine];
+  const int my_page = my_seq < 0 ? -1 : block_table[(size_t)my_seq * table_width + my_pos / page_size];
+#pragma unroll
+  for (int x = 0; x < ROWS; ++x) {
+    const int j = wave * ROWS + x, page = __builtin_amdgcn_readlane(my_page, x), pos = __builtin_amdgcn_readlane(my_pos, x);
+    float v[8], ss = 0.f;
+    r8_unpack(raw[x], v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss = fmaf(v[e], v[e], ss);
+    const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)R + eps);
+    if (page < 0 || t0 + j >= T) continue;
+    bf16* dst = kcache + ((size_t)page * page_size + pos % page_size) * (R + Dr);
+    if (d >= from && d < to) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = v[e] * inv * w[e];
+      const uint4 y = r8_pack(v);
+      *reinterpret_cast<uint4*>(dst + d) = y;
+      uint32_t* at = reinterpret_cast<uint32_t*>(lw_values + j * stride + d - from);
+      at[0] = y.x; at[1] = y.y; at[2] = y.z; at[3] = y.w;
+    }
+  }
+  // the key parts, a unit a thread
+  for (int u = threadIdx.x; part == 0 && u < R8_TOKENS * (Dr / 8); u += blockDim.x) {
+    const int j = u / (Dr / 8), at = (u - j * (Dr / 8)) * 8, t = t0 + j;
+    if (t >= T || token_seq[t] < 0) continue;
+    const int pos = positions[t], page = block_table[(size_t)token_seq[t] * table_width + pos / page_size];
+    if (page < 0) continue;
+    float y[8];
+    lw_turn(down + (size_t)t * ld_down + R, at, rot, adjacent, cos_sin + (size_t)pos * half_t * 2, y);
+    r8_store(kcache + ((size_t)page * page_size + pos % page_size) * (R + Dr) + R + at, y);
+  }
+  if (!vcache) return;
+  __syncthreads();
+  r8_turn_rows(lw_values, stride, from, to, R, t0, T, positions, token_seq, block_table, table_width, page_size, vcache, 1, 0);
+}
+
 extern "C" int blm_latent_write(const void* down, int ld_down, const void* q, int ld_q, int dtype, int T, int H, int dn,
                                 const float* norm_w, float eps, const void* cos_sin, int half_t, int rot, void* qabs,
                                 int qabs_dtype, void* kcache, void* vcache, const int* positions, const int* token_seq, const int* block_table,
@@ -92,6 +191,20 @@ extern "C" int blm_latent_write(const void* down, int ld_down, const void* q, in
   BLM_REQUIRE(T > 0 && H > 0 && dn >= 0 && R > 0 && Dr >= 0, "latent_write: bad sizes");
   BLM_REQUIRE(rot % 2 == 0 && rot >= 0 && rot <= Dr && rot / 2 <= half_t, "latent_write: %d turning lanes do not fit %d", rot, Dr);
   BLM_REQUIRE(page_size > 0 && table_width > 0 && ld_down >= R + Dr && ld_q >= H * (dn + Dr), "latent_write: bad geometry");
+  if (T > 64 && dtype == BLM_BF16 && R % 8 == 0 && R <= 512 && Dr % 8 == 0 && dn % 8 == 0 && rot % 8 == 0 && (adjacent || rot % 16 == 0) &&
+      half_t % 2 == 0 && ld_down % 8 == 0 && ld_q % 8 == 0 && ((uintptr_t)down % 16) == 0 && ((uintptr_t)q % 16) == 0 && ((uintptr_t)norm_w % 16) == 0 &&
+      ((uintptr_t)cos_sin % 16) == 0 && ((uintptr_t)qabs % 16) == 0 && ((uintptr_t)kcache % 16) == 0 && (qabs_dtype == BLM_BF16 || qabs_dtype == BLM_F32)) {
+    const int tiles = write_kv ? (T + R8_TOKENS - 1) / R8_TOKENS : 0, parts = R % 32 == 0 ? 4 : 1;
+#define BLM_LWP(TQ)                                                                                                                     \
+  hipLaunchKernelGGL((latent_write_prompt_kernel<TQ>), dim3((unsigned)(T + tiles * parts)), dim3(256), R8_VALUE_LDS(R / parts), stream, (const bf16*)down, \
+                     ld_down, (const bf16*)q, ld_q, T, H, dn, norm_w, eps, (const float*)cos_sin, half_t, rot, (TQ*)qabs, (bf16*)kcache, \
+                     (bf16*)vcache, positions, token_seq, block_table, table_width, page_size, R, Dr, adjacent, q_lanes, q_at, tiles, parts)
+    if (qabs_dtype == BLM_F32) BLM_LWP(float);
+    else BLM_LWP(bf16);
+#undef BLM_LWP
+    BLM_LAUNCH_CHECK("latent_write_prompt");
+    return 0;
+  }
 #define BLM_LW(TA, TQ)                                                                                                  \
   hipLaunchKernelGGL((latent_write_kernel<TA, TQ>), dim3(T), dim3(256), 0, stream, (const TA*)down, ld_down, (const TA*)q, \
                      ld_q, H, dn, norm_w, eps, (const float2*)cos_sin, half_t, rot, (TQ*)qabs, (TA*)kcache, (TA*)vcache,  \

@@ -13,7 +13,7 @@
 // Also here: what comes between the q/k/v projection and the attention: bias, rotation of the first lanes of
 // every query and key head by the token's position (lane i paired with lane i + rot/2), and the write of the
 // rotated keys and the values into the token's place of the pages.
-#include "common.h"
+#include "rows8.h"
 
 #define SA_MAX_DV_REGS 4      // value lanes per head up to 64 * this
 #define SA_MAX_DK 512
@@ -228,6 +228,190 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
+// The three above for prompts (bfloat16; every part of a row in units of eight lanes): the values' blocks (r8_values), which take the
+// longest, and a block a token with eight lanes a thread.  A pass over 2,048 rows of 3,072 and their pages is 25 MB, 5 us at
+// the rate of a copy; token by token with two bytes a lane and store it took 36 (norms of heads), 23 (of rows) and 26 (rotation, 2,166
+// rows), so 12.8, 13.1 and 10.5.
+struct QpPages {
+  const int *positions, *token_seq, *block_table;
+  int table_width, page_size;
+  bf16 *k, *v;
+};
+// kind 0: heads normed; 1: the queries' and keys' parts of the row normed; 2: the first rot lanes of a head turned.
+template <int KIND>
+__global__ void __launch_bounds__(512)
+    qkv_prompt_kernel(bf16* __restrict__ qkv, int ld, const float* __restrict__ bias, QpPages pg, int T, int H, int G, int dk, int dv,
+                      int values_at, int write_kv, const float* __restrict__ q_scale, float norm_eps, QnExtra ex,
+                      const float* __restrict__ cos_sin, int rot, int adjacent, int tiles) {
+  extern __shared__ bf16 qp_values[];
+  __shared__ float red[2][17];
+  const int Gp = G / ex.maps;
+  if ((int)blockIdx.x < tiles) {
+    const int tile = blockIdx.x, head = tile % Gp;
+    r8_values(qkv, ld, values_at + head * dv, bias, dv, tile / Gp * R8_TOKENS, T, pg.positions, pg.token_seq, pg.block_table, pg.table_width,
+              pg.page_size, pg.v, Gp, head, qp_values);
+    return;
+  }
+  const int t = blockIdx.x - tiles;
+  bf16* row = qkv + (size_t)t * ld;
+  // norms: QP_UNITS units a thread, in registers between the sums and the stores; asked for ahead of the look-ups
+  const int n_q = H * dk / 8, n_units = n_q + G * dk / 8, lanes = dk / 8;
+  constexpr int QP_UNITS = 4;
+  uint4 raw[QP_UNITS];
+  if (KIND != 2) {
+#pragma unroll
+    for (int k = 0; k < QP_UNITS; ++k) {
+      const int u = threadIdx.x + k * blockDim.x;
+      raw[k] = make_uint4(0u, 0u, 0u, 0u);
+      if (u < n_units) raw[k] = *reinterpret_cast<const uint4*>(row + u * 8);
+    }
+  }
+  const int b = pg.token_seq[t], pos = pg.positions[t];
+  if (b < 0) return;
+  const size_t page = write_kv ? pg.block_table[(size_t)b * pg.table_width + pos / pg.page_size] : 0;
+  const int in_page = write_kv ? pos % pg.page_size : 0;
+  const float growth = KIND != 2 ? qn_growth(ex, pos) : 1.0f;
+  if (KIND == 2) {
+    const int half = rot / 2, turning = adjacent ? rot / 8 : half / 8, per_head = turning + (dk - rot) / 8;
+    const float* cs = cos_sin + (size_t)pos * rot;
+    for (int u = threadIdx.x; u < (H + (write_kv ? G : 0)) * per_head; u += blockDim.x) {
+      const int head = u / per_head, i = u - head * per_head, col = head * dk;
+      const float f = q_scale && head < H ? q_scale[head] : 1.0f;
+      bf16* to = head < H ? row + col : pg.k + ((page * G + (head - H)) * pg.page_size + in_page) * dk;
+      const int d = i < turning ? i * 8 : rot + (i - turning) * 8;
+      float x[8], c[4], s[4];
+      r8_load(row + col + d, x);
+      if (bias) {
+        float a[8];
+        r8_load(bias + col + d, a);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] += a[e];
+      }
+      if (i < turning && !adjacent) {
+        float y[8], a[8];
+        r8_load(row + col + d + half, y);
+        if (bias) {
+          r8_load(bias + col + d + half, a);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] += a[e];
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          r8_angles(cs + 2 * d + 8 * g, c, s);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float xe = x[4 * g + e], ye = y[4 * g + e];
+            x[4 * g + e] = (xe * c[e] - ye * s[e]) * f;
+            y[4 * g + e] = (ye * c[e] + xe * s[e]) * f;
+          }
+        }
+        r8_store(to + d + half, y);
+      } else if (i < turning) {
+        r8_angles(cs + d, c, s);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float xe = x[2 * e], ye = x[2 * e + 1];
+          x[2 * e] = (xe * c[e] - ye * s[e]) * f;
+          x[2 * e + 1] = (ye * c[e] + xe * s[e]) * f;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] *= f;
+      }
+      r8_store(to + d, x);
+    }
+    return;
+  }
+  float x[QP_UNITS][8], ss_q = 0.f, ss_k = 0.f, f[QP_UNITS];
+#pragma unroll
+  for (int k = 0; k < QP_UNITS; ++k) {
+    const int u = threadIdx.x + k * blockDim.x;
+    float ss = 0.f;
+    r8_unpack(raw[k], x[k]);
+    if (u < n_units) {
+      if (bias) {
+        float a[8];
+        r8_load(bias + u * 8, a);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[k][e] += a[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = fmaf(x[k][e], x[k][e], ss);
+    }
+    if (KIND == 0) f[k] = 1.0f / sqrtf(r8_group_sum(ss, lanes) / (float)dk + norm_eps);
+    else if (u < n_q) ss_q += ss;
+    else ss_k += ss;
+  }
+  float f_q = 0.f, f_k = 0.f;
+  if (KIND == 1) {
+    f_q = 1.0f / sqrtf(block_sum<true>(ss_q, red[0]) / (float)(H * dk) + norm_eps);
+    f_k = 1.0f / sqrtf(block_sum<true>(ss_k, red[1]) / (float)(G * dk) + norm_eps);
+  }
+#pragma unroll
+  for (int k = 0; k < QP_UNITS; ++k) {
+    const int u = threadIdx.x + k * blockDim.x;
+    if (u >= n_units) continue;
+    const bool key = u >= n_q;
+    const int head = u / lanes, d = (u - head * lanes) * 8;
+    const float* w = key ? ex.kw : ex.qw;
+    const int w_at = KIND == 0 ? d : (key ? u - n_q : u) * 8;
+    float factor = KIND == 0 ? f[k] : key ? f_k : f_q;
+    if (!key) factor = factor * (KIND == 0 && q_scale ? q_scale[head] : 1.0f) * growth;
+    if (w) {
+      float a[8];
+      r8_load(w + w_at, a);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[k][e] = KIND == 0 ? x[k][e] * a[e] * factor : x[k][e] * factor * a[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[k][e] *= factor;
+    }
+    if (key) {
+      const int c = head - H;
+      r8_store(pg.k + ((page * Gp + c / ex.maps) * pg.page_size + in_page) * (dk * ex.maps) + (c % ex.maps) * dk + d, x[k]);
+    } else if (ex.maps == 2) {
+      bf16* o = (bf16*)ex.q_out + (size_t)t * ex.ld_q + (size_t)head * 2 * dk + d;
+      const int mine = (head & 1) * dk;
+      r8_store(o + mine, x[k]);
+      *reinterpret_cast<uint4*>(o + dk - mine) = make_uint4(0u, 0u, 0u, 0u);
+    } else {
+      r8_store(row + u * 8, x[k]);
+    }
+  }
+}
+
+// Whether qkv_prompt_kernel takes the call; few tokens stay with the kernels above (8 tokens: 5.4 and 5.2 us, a launch).
+static bool qp_takes(const void* qkv, int dtype, int ld, const float* bias, const void* kcache, int T, int H, int G, int dk, int dv, int kind,
+                     int rot, int adjacent, const void* cos_sin, const QnExtra& ex) {
+  const int n = (H + G) * dk;
+  bool ok = T > 64 && dtype == BLM_BF16 && ld % 8 == 0 && dk % 8 == 0 && dv % 8 == 0 && dv <= 512 && ((uintptr_t)qkv % 16) == 0 &&
+            ((uintptr_t)bias % 16) == 0 && ((uintptr_t)kcache % 16) == 0 && ((uintptr_t)ex.qw % 16) == 0 && ((uintptr_t)ex.kw % 16) == 0 &&
+            ((uintptr_t)ex.q_out % 16) == 0 && (ex.maps == 1 || ex.ld_q % 8 == 0);
+  if (kind == 0) ok = ok && dk <= 512 && (dk & (dk - 1)) == 0;
+  if (kind < 2) ok = ok && n <= 4 * 512 * 8;
+  if (kind == 2) ok = ok && rot % 8 == 0 && (adjacent || rot % 16 == 0) && ((uintptr_t)cos_sin % 16) == 0;
+  return ok;
+}
+static int qp_launch(int kind, void* qkv, int ld, const float* bias, const int* positions, const int* token_seq, const int* block_table,
+                     int table_width, void* kcache, void* vcache, int page_size, int T, int H, int G, int dk, int dv, int values_at, int write_kv,
+                     const float* q_scale, float norm_eps, const QnExtra& ex, const float* cos_sin, int rot, int adjacent, hipStream_t stream) {
+  const QpPages pg{positions, token_seq, block_table, table_width, page_size, (bf16*)kcache, (bf16*)vcache};
+  const long long tiles = write_kv ? (long long)((T + R8_TOKENS - 1) / R8_TOKENS) * (G / ex.maps) : 0;
+  BLM_REQUIRE(T + tiles < 2147483647LL, "qkv_prompt: too many tokens");
+  const int units = (H + (write_kv ? G : 0)) * dk / 8;
+  const int threads = kind == 2 ? 256 : units <= 64 ? 64 : units <= 512 ? (units + 63) / 64 * 64 : 512;
+  const dim3 grid((unsigned)(T + tiles)), block(threads);
+#define QP_LAUNCH(KIND)                                                                                                              \
+  hipLaunchKernelGGL((qkv_prompt_kernel<KIND>), grid, block, R8_VALUE_LDS(dv), stream, (bf16*)qkv, ld, bias, pg, T, H, G, dk, dv, values_at, \
+                     write_kv, q_scale, norm_eps, ex, cos_sin, rot, adjacent, (int)tiles)
+  if (kind == 0) QP_LAUNCH(0);
+  else if (kind == 1) QP_LAUNCH(1);
+  else QP_LAUNCH(2);
+#undef QP_LAUNCH
+  BLM_LAUNCH_CHECK("qkv_prompt");
+  return 0;
+}
+
 // Bias, norm (over a head's lanes, or whole_rows: over all of a token's queries, and of its keys), growth of the queries
 // and the write of keys and values into the pages.  H, G: heads of dk lanes in the row (maps = 2: twice the pages' heads).
 extern "C" int blm_qkv_norm(void* qkv, int dtype, int ld, const float* bias, const int* positions, const int* token_seq,
@@ -244,6 +428,9 @@ extern "C" int blm_qkv_norm(void* qkv, int dtype, int ld, const float* bias, con
               dk, dv, BLM_WAVE * QU_LANES);
   BLM_REQUIRE(every >= 0, "qkv_norm: queries that grow every %d tokens", every);
   const QnExtra ex{qw, kw, coef, every, maps, ld_q, q_out};
+  if (qp_takes(qkv, dtype, ld, bias, kcache, T, H, G, dk, dv, whole_rows ? 1 : 0, 0, 0, nullptr, ex))
+    return qp_launch(whole_rows ? 1 : 0, qkv, ld, bias, positions, token_seq, block_table, table_width, kcache, vcache, page_size, T, H, G, dk, dv,
+                     (H + G) * dk, 1, nullptr, norm_eps, ex, nullptr, 0, 0, stream);
 #define QN_ROWS(TA)                                                                                                       \
   hipLaunchKernelGGL(qkv_row_norm_kernel<TA>, dim3(T, 3), dim3(T <= 64 ? 1024 : 256), 0, stream, (TA*)qkv, ld, bias, positions, token_seq, \
                      block_table, table_width, (TA*)kcache, (TA*)vcache, page_size, H, G, dk, dv, norm_eps, ex)
@@ -276,6 +463,11 @@ extern "C" int blm_qkv_prepare(void* qkv, int dtype, int ld, const float* bias, 
   BLM_REQUIRE(ld >= H * dk + (write_kv ? G * (dk + (values_are_keys ? 0 : dv)) : 0), "qkv_prepare: rows of %d are too short", ld);
   BLM_REQUIRE(!write_kv || (kcache && vcache && block_table && page_size > 0 && table_width > 0), "qkv_prepare: the pages are missing");
   BLM_REQUIRE(rot == 0 || cos_sin, "qkv_prepare: the table of angles is missing");
+  const QnExtra none{nullptr, nullptr, 0.f, 0, 1, 0, nullptr};
+  const int kind = unit_norm ? 0 : 2;
+  if ((!unit_norm || (rot == 0 && write_kv)) && qp_takes(qkv, dtype, ld, bias, kcache, T, H, G, dk, dv, kind, rot, adjacent, cos_sin, none))
+    return qp_launch(kind, qkv, ld, bias, positions, token_seq, block_table, table_width, kcache, vcache, page_size, T, H, G, dk, dv,
+                     values_are_keys ? H * dk : (H + G) * dk, write_kv, q_scale, norm_eps, none, cos_sin, rot, adjacent, stream);
   const size_t factors = unit_norm ? (size_t)(H + G) * sizeof(float) : 0;
   BLM_REQUIRE(factors <= 60 * 1024, "qkv_prepare: %d heads are too many", H + G);
   if (unit_norm && rot == 0 && dk <= BLM_WAVE * QU_LANES && dv <= BLM_WAVE * QU_LANES && (dtype == BLM_F32 || dtype == BLM_BF16)) {
