@@ -23,6 +23,15 @@ __device__ __forceinline__ float gd_gelu(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(a * -2.8853900817779268f));
 }
 
+// mode 3: the columns are query heads, then key heads and value heads of hd lanes each; queries and keys turn in adjacent pairs
+// behind the product, keys and values go to their pages.
+struct GdRope {
+  const int *positions, *token_seq, *block_table;
+  const float* cos_sin;                      // [positions][hd / 2][2]
+  bf16 *kcache, *vcache;
+  int table_width, page_size, nh, nkv, hd, store;
+};
+
 template <int MODE>
 struct GdTile {
   const char *a, *b;
@@ -31,8 +40,9 @@ struct GdTile {
   int lda, ldw;
   __device__ __forceinline__ uint32_t row(int m) const { return (uint32_t)(min(m, rows - 1) * lda) * 2u; }
   __device__ __forceinline__ uint32_t column(int r, int h) const {
-    const int n = min(MODE != 0 ? r : r / 32 * 64 + h * 32 + r % 32, columns - 1);
-    return (uint32_t)n * (uint32_t)ldw * 2u + (MODE != 0 && h ? up : 0u);
+    const bool gated = MODE == 1 || MODE == 2;
+    const int n = min(gated ? r : r / 32 * 64 + h * 32 + r % 32, columns - 1);
+    return (uint32_t)n * (uint32_t)ldw * 2u + (gated && h ? up : 0u);
   }
 };
 
@@ -66,13 +76,66 @@ __device__ __forceinline__ void gd_store(const gd_f32x4 (&acc)[TILES][4], TC* C,
   }
 }
 
+// Rows of 16 lanes are tokens: their positions and pages lie in shared memory (page < 0: not stored).  A tile of 16 columns is of one
+// head (head sizes are multiples of 16).  Queries and keys leave as eight neighbours a lane like every other result; a value's store is
+// a run of 16 tokens, two bytes each.
+template <int TILES>
+__device__ __forceinline__ void gd_store_rope(const gd_f32x4 (&acc)[TILES][4], bf16* C, int ldc, const int* pos_of, const int* page_of, int first,
+                                              int m0, int M, int n0, int N, const GdRope& rope, int l16, int quad) {
+  const int hd = rope.hd, n_turning = (rope.nh + rope.nkv) * hd, ps = rope.page_size;
+  // the next rows' angles are asked for ahead of these rows' stores (one after another they took 12 us a tile)
+  int lane_of[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) lane_of[j] = (n0 + j * 16) % hd + quad * 4;
+  float4 angles[2][4];
+  auto ask = [&](int i) {
+    const float* row = rope.cos_sin + (size_t)pos_of[first + i * 16 + l16] * hd;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) angles[i & 1][j] = *reinterpret_cast<const float4*>(row + lane_of[j]);
+  };
+  ask(0);
+#pragma unroll
+  for (int i = 0; i < TILES; ++i) {
+    const int r = first + i * 16 + l16, m = m0 + r;
+    const int pos = pos_of[r], page = page_of[r], slot = pos % ps;
+    if (i + 1 < TILES) ask(i + 1);
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {
+      float v[2][4];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int tile = n0 + (j + x) * 16, head = tile / hd, d = lane_of[j + x];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[x][e] = acc[i][j + x][e];
+        if (tile < n_turning) {
+          const float4 cs = angles[i & 1][j + x];
+          v[x][0] = acc[i][j + x][0] * cs.x - acc[i][j + x][1] * cs.y;
+          v[x][1] = acc[i][j + x][0] * cs.y + acc[i][j + x][1] * cs.x;
+          v[x][2] = acc[i][j + x][2] * cs.z - acc[i][j + x][3] * cs.w;
+          v[x][3] = acc[i][j + x][2] * cs.w + acc[i][j + x][3] * cs.z;
+        } else if (tile < N && m < M && page >= 0) {
+          bf16* to = rope.vcache + (((size_t)page * rope.nkv + (head - rope.nh - rope.nkv)) * hd + d) * ps + slot;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) to[(size_t)e * ps] = from_float<bf16>(v[x][e]);
+        }
+      }
+      const uint4 eight = gd_eight(v);
+      const int n = n0 + (j + (quad & 1)) * 16 + (quad >> 1) * 8, head = n / hd;
+      if (m >= M || n >= n_turning) continue;
+      if (head < rope.nh) *reinterpret_cast<uint4*>(C + (size_t)m * ldc + n) = eight;
+      else if (page >= 0) *reinterpret_cast<uint4*>(rope.kcache + (((size_t)page * rope.nkv + (head - rope.nh)) * ps + slot) * hd + (n - head * hd)) = eight;
+    }
+  }
+}
+
 // Tiles in the order in which they are walked: [0, whole) as whole ones, the rest of the m_tiles x n_tiles as two halves each, and
 // behind them, where `tail`, a row of halves below the last row of tiles.
 template <int MODE, typename TC>
 __global__ void __launch_bounds__(512, 2)
     gemm_duo_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, TC* __restrict__ C, int M, int N, int K, int lda, int ldw,
-                    int ldc, int m_tiles, int n_tiles, int whole, int k_per_group) {
-  constexpr int OUT = MODE != 0 ? GD_TILE / 2 : GD_TILE;   // output columns of a tile
+                    int ldc, int m_tiles, int n_tiles, int whole, int k_per_group, GdRope rope) {
+  constexpr bool GATED = MODE == 1 || MODE == 2;
+  constexpr int OUT = GATED ? GD_TILE / 2 : GD_TILE;       // output columns of a tile
   __shared__ __attribute__((aligned(1024))) unsigned char lds[9 * GD_REGION];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / BLM_WAVE), lane = tid & (BLM_WAVE - 1);
   const int l16 = lane & 15, quad = lane >> 4, wm = wave >> 2, wn = wave & 3;      // wavefronts w and w + 4 share a SIMD
@@ -104,8 +167,24 @@ __global__ void __launch_bounds__(512, 2)
   C += (size_t)blockIdx.y * M * ldc;
   const GdTile<MODE> t = {reinterpret_cast<const char*>(A + (size_t)m0 * lda + k0), reinterpret_cast<const char*>(W + (size_t)n0 * ldw + k0),
                           M - m0, N - n0, (uint32_t)N * (uint32_t)ldw * 2u, lda, ldw};
-  const int n = n0 + wn * (MODE != 0 ? 32 : 64);
-  if (!half) {
+  const int n = n0 + wn * (GATED ? 32 : 64);
+  if constexpr (MODE == 3) {
+    __shared__ int pos_of[GD_TILE], page_of[GD_TILE];
+    if (tid < GD_TILE) {
+      const int m = min(m0 + tid, M - 1), seq = rope.token_seq[m], pos = rope.positions[m];
+      pos_of[tid] = pos;
+      page_of[tid] = seq < 0 || !rope.store ? -1 : rope.block_table[(size_t)seq * rope.table_width + pos / rope.page_size];
+    }
+    if (!half) {                             // the product's first barriers lie between these writes and the reads behind it
+      gd_f32x4 acc[8][4];
+      gd_whole(acc, t, stages, lds, wave, lane);
+      gd_store_rope(acc, C, ldc, pos_of, page_of, wm * 128, m0, M, n, N, rope, l16, quad);
+    } else {
+      gd_f32x4 acc[4][4];
+      gd_half(acc, t, stages, lds, wave, lane);
+      gd_store_rope(acc, C, ldc, pos_of, page_of, wm * 64, m0, M, n, N, rope, l16, quad);
+    }
+  } else if (!half) {
     gd_f32x4 acc[8][4];
     gd_whole(acc, t, stages, lds, wave, lane);
     gd_store<MODE, 8, TC>(acc, C, ldc, m0 + wm * 128, M, n, N, l16, quad);
@@ -119,10 +198,10 @@ __global__ void __launch_bounds__(512, 2)
 // mode 0: C[M, N] = A W^T, W [N, K].  mode 1: W [2N, K] = [gate rows; up rows], C[M, N] = silu(gate) * up; mode 2: the tanh form of
 // GELU in place of silu.  k_groups > 1: C is float [k_groups, M, ldc], a partial product over each group's stretch of K (a multiple
 // of 128).  whole: how many of the tiles are run as whole ones, the others as halves.
-extern "C" int blm_gemm_duo(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, int mode,
-                            int k_groups, int whole, hipStream_t stream) {
+static int gd_run(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, int mode,
+                  int k_groups, int whole, const GdRope* rope, hipStream_t stream) {
   BLM_REQUIRE(M >= 1 && N >= 8 && N % 8 == 0 && K >= 256 && K % 128 == 0, "gemm_duo: sizes M=%d N=%d K=%d not supported", M, N, K);
-  BLM_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && ldc % 8 == 0 && lda >= K && ldw >= K && ldc >= N, "gemm_duo: bad strides lda=%d ldw=%d ldc=%d",
+  BLM_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && ldc % 8 == 0 && lda >= K && ldw >= K && ldc >= (rope ? rope->nh * rope->hd : N), "gemm_duo: bad strides lda=%d ldw=%d ldc=%d",
               lda, ldw, ldc);
   BLM_REQUIRE(((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)C % 16) == 0, "gemm_duo: operands must be 16-byte aligned");
   BLM_REQUIRE(mode >= 0 && mode <= 2 && (c_dtype == BLM_BF16 || (c_dtype == BLM_F32 && mode == 0)), "gemm_duo: mode %d, dtype %d", mode, c_dtype);
@@ -140,12 +219,29 @@ extern "C" int blm_gemm_duo(const void* A, const void* W, void* C, int c_dtype, 
   const dim3 grid((unsigned)(whole + halves), (unsigned)k_groups), block(512);
 #define GD_LAUNCH(MODE, TC)                                                                                                        \
   hipLaunchKernelGGL((gemm_duo_kernel<MODE, TC>), grid, block, 0, stream, (const bf16*)A, (const bf16*)W, (TC*)C, M, N, K, lda, ldw, \
-                     ldc, m_tiles, n_tiles, whole, k_per_group)
-  if (mode == 1) GD_LAUNCH(1, bf16);
+                     ldc, m_tiles, n_tiles, whole, k_per_group, rope ? *rope : GdRope{})
+  if (rope) GD_LAUNCH(3, bf16);
+  else if (mode == 1) GD_LAUNCH(1, bf16);
   else if (mode == 2) GD_LAUNCH(2, bf16);
   else if (c_dtype == BLM_F32) GD_LAUNCH(0, float);
   else GD_LAUNCH(0, bf16);
 #undef GD_LAUNCH
   BLM_LAUNCH_CHECK("gemm_duo");
   return 0;
+}
+
+extern "C" int blm_gemm_duo(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, int mode,
+                            int k_groups, int whole, hipStream_t stream) {
+  return gd_run(A, W, C, c_dtype, M, N, K, lda, ldw, ldc, mode, k_groups, whole, nullptr, stream);
+}
+
+// The q/k/v projection with the rotation of queries and keys (on the float results) and the write of keys and values into their
+// pages.  qkv_out [M][ldq]: the queries.  Instead of a pass of its own over queries, keys and values (2,048 rows of 3,072: 8.9 us).
+extern "C" int blm_gemm_duo_qkv_rope(const void* A, const void* W, void* qkv_out, const int* positions, const int* token_seq,
+                                     const int* block_table, int table_width, const float* cos_sin, void* kcache, void* vcache, int page_size,
+                                     int M, int K, int lda, int ldw, int ldq, int nh, int nkv, int hd, int store, int whole, hipStream_t stream) {
+  BLM_REQUIRE(nh > 0 && nkv > 0 && hd > 0 && hd % 16 == 0 && page_size > 0 && table_width > 0, "gemm_duo_qkv_rope: head size %d not supported (a multiple of 16)", hd);
+  BLM_REQUIRE(((uintptr_t)kcache % 16) == 0 && ((uintptr_t)cos_sin % 16) == 0, "gemm_duo_qkv_rope: pages and angles must be 16-byte aligned");
+  const GdRope rope{positions, token_seq, block_table, cos_sin, (bf16*)kcache, (bf16*)vcache, table_width, page_size, nh, nkv, hd, store};
+  return gd_run(A, W, qkv_out, BLM_BF16, M, (nh + 2 * nkv) * hd, K, lda, ldw, ldq, 0, 1, whole, &rope, stream);
 }

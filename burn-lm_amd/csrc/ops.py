@@ -157,6 +157,7 @@ _SIGNATURES = {
                       _c_int, _c_int, _c_int, _c_void_p],
     "blm_gemm_duo": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                      _c_void_p],
+    "blm_gemm_duo_qkv_rope": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 11 + [_c_void_p],
     "blm_gemv_mfma_group_limit": [_c_int],
     "blm_gemv_qkv_rope_supported": [_c_int, _c_int, _c_int, _c_int],
     "blm_gemv_qkv_rope": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p,
@@ -838,6 +839,31 @@ def gemm_duo(a, w, out, gated=False, activation="silu", whole=None):
     _call("blm_gemm_duo", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out), M, N, K, a.stride(0), w.stride(0), out.stride(-2),
           (2 if activation == "gelu_tanh" else 1) if gated else 0, groups, gemm_duo_tiles(M, N, gated)[0] if whole is None else whole, _stream())
     return out
+
+
+def gemm_duo_qkv_rope(x, w, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache, page_size, nh, nkv, hd, write_kv=True,
+                      whole=None):
+    """x [M, K] @ W_qkv^T (w [(nh + 2 nkv) * hd, K], rotary partners in adjacent rows) in gemm_duo's tiles, rotary encoding of q and k
+    on the float results, q into qkv_out[:, :nh*hd], k and v into their cache pages, in one kernel.  hd a multiple of 16."""
+    _gpu(x, w, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache)
+    M, K = x.shape
+    N = (nh + 2 * nkv) * hd
+    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or qkv_out.dtype != torch.bfloat16 or kcache.dtype != torch.bfloat16:
+        raise KernelError("gemm_duo_qkv_rope: operands and the cache must be bfloat16")
+    if w.dim() != 2 or w.shape != (N, K) or w.stride(1) != 1 or x.stride(1) != 1:
+        raise KernelError(f"gemm_duo_qkv_rope: the weights must be [{N}, {K}], rows with unit stride, got {tuple(w.shape)}")
+    if qkv_out.shape[0] != M or qkv_out.stride(1) != 1 or qkv_out.shape[1] < nh * hd:
+        raise KernelError("gemm_duo_qkv_rope: qkv_out must be [M, >= heads*head_dim] with unit stride along rows")
+    _i32("positions", positions, M); _i32("token_seq", token_seq, M); _i32("block_table", block_table)
+    if cos_sin.dtype != torch.float32 or cos_sin.shape[1:] != (hd // 2, 2) or not cos_sin.is_contiguous():
+        raise KernelError("gemm_duo_qkv_rope: cos_sin must be contiguous float32 [positions, head_dim/2, 2]")
+    _contig("kcache", kcache); _contig("vcache", vcache)
+    _check_planes("gemm_duo_qkv_rope", kcache, vcache, nkv, page_size, hd)
+    _call("blm_gemm_duo_qkv_rope", x.data_ptr(), w.data_ptr(), qkv_out.data_ptr(), positions.data_ptr(), token_seq.data_ptr(),
+          block_table.data_ptr(), block_table.shape[1], cos_sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), page_size, M, K,
+          x.stride(0), w.stride(0), qkv_out.stride(0), nh, nkv, hd, 1 if write_kv else 0,
+          gemm_duo_tiles(M, N)[0] if whole is None else whole, _stream())
+    return qkv_out
 
 
 def gemm_duo_tiles(M, N, gated=False):

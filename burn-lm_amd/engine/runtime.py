@@ -120,8 +120,10 @@ def f32_plan(M, N, K, compute_units, planes=False, gated=False):
 # a plain one whose last round is of whole tiles and for one round of halves (see gated_linear and duo_product).
 DUO_HALF = 0.57
 DUO_GATED_FILL = 0.62
+DUO_GATED_LONE_FILL = 0.9
 DUO_WHOLE_FILL = 0.93
 DUO_HALVES_FILL = 0.74
+DUO_QKV_FILL = 0.6
 DUO_WHOLE_K = 3072
 DUO_PLANES_K = 4096
 
@@ -546,10 +548,21 @@ class Runtime:
             return ops.gemv_skinny(x, w, out)
         if out_dtype == torch.bfloat16:
             if plain_bf16 and self.fused_gate_up_measured and self.duo_product(M, N, K) and ops.gemm_duo_takes(x, w, out):
-                return ops.gemm_duo(x, w, out, whole=duo_plan(M, N, self.compute_units)[0])
+                return ops.gemm_duo(x, w, out, whole=self.duo_tiles(M, N))
             return torch.matmul(x, w.t(), out=out)
         # float32 logits from bfloat16 operands with many rows: own kernel (float accumulation)
         return ops.gemm_tiled(x, w, out)
+
+    def duo_tiles(self, M, N):
+        """How many of a product's tiles ops.gemm_duo runs as whole ones."""
+        return duo_plan(M, N, self.compute_units)[0]
+
+    def duo_qkv(self, M, N, K):
+        """Whether a q/k/v projection of more than 256 rows goes to ops.gemm_duo_qkv_rope, which turns queries and keys and fills the
+        pages behind the product instead of a kernel that reads its results and writes them back.  Within prompts, us a layer, this /
+        the library's product (long ones: gemm_duo's) and that kernel: 2,048 rows of 3,072, K = 2,048 39.8 / 42.1; 9,681 of 5,120,
+        K = 3,072 252.6 / 279.5; less full rounds are behind (600 rows of the latter 40 / 33, 1,000 and 1,300 of the former 31 / 27, 31 / 29)."""
+        return self.fused_gate_up_measured and M > 256 and K <= RING_QKV_K and duo_plan(M, N, self.compute_units)[2] >= DUO_QKV_FILL
 
     def duo_product(self, M, N, K):
         """Whether a plain bfloat16 product of many rows goes to ops.gemm_duo and not to the library (us, duo / library):
@@ -636,11 +649,13 @@ class Runtime:
             # full enough (us against the library's product and the gating pass, inner size 8192: width 2048, 512 / 1,000 / 1,300 /
             # 2,048 / 2,166 / 9,681 rows 31 / 43, 51 / 67, 76 / 97, 100 / 120, 118 / 146, 449 / 625; width 3072, 700 / 2,048 / 9,681
             # rows 69 / 73, 152 / 176, 665 / 863; width 4096, inner size 14336, 400 / 1,300 / 4,096 rows 87 / 94, 262 / 277,
-            # 654 / 701; too little is full: that shape with 260 rows 86 / 71).
+            # 654 / 701; too little is full: that shape with 260 rows 86 / 71).  A lone round of halves at a K beyond RING_GROUP_K has to
+            # be nearly full (width 3072 within prompts of 384 and 512 rows: 52 / 50 and equal; width 2048: 34 / 37).
             if M > 256:
-                whole, _, fill = duo_plan(M, inner, self.compute_units, True)
-                out = torch.empty(M, inner, dtype=self.dtype, device=x.device)
-                if fill >= DUO_GATED_FILL and ops.gemm_duo_takes(x, plain, out, gated=True):
+                whole, rounds, fill = duo_plan(M, inner, self.compute_units, True)
+                enough = DUO_GATED_LONE_FILL if rounds <= DUO_HALF and K > RING_GROUP_K else DUO_GATED_FILL
+                out = torch.empty(M, inner, dtype=self.dtype, device=x.device) if fill >= enough else None
+                if out is not None and ops.gemm_duo_takes(x, plain, out, gated=True):
                     return ops.gemm_mfma(x, plain, out, gated=True, tile=(256, 256), activation=activation, whole=whole)
             # 256x128 tiles that make one round on at least three quarters of the compute units, with rows
             # that fill their tiles to 85 % and more: measured against the library's product and the gating

@@ -149,11 +149,19 @@ class RotaryEncoding(PositionEncoding):
         elif (plan is not None and M <= 64 and bf16 and packable and not getattr(w_qkv, "gated", False)
                 and rt.ops.gemv_qkv_rope_supported(M, K, head_dim, self.pairing)):
             fused = "packed"     # also where the row-ring kernel was the plan and this encoding has none for it
+        elif (plan is None and bf16 and self.pairing == PAIRING["interleaved"] and raw is not None and raw.dtype == torch.bfloat16
+                and head_dim % 16 == 0 and hasattr(rt, "duo_qkv") and rt.duo_qkv(M, n_qkv, K)):
+            fused = "tiles"
         if fused is None:
             return super().project_encode_store(x, w_qkv, step, view, heads, kv_heads, head_dim)
         if step.max_position >= self.n_positions:
             raise ValueError(f"position {step.max_position} is past the rotary table of {self.n_positions}")
         qkv = torch.empty(M, n_qkv, dtype=torch.bfloat16, device=x.device)
+        if fused == "tiles":
+            if not rt.ops.gemm_duo_takes(x, raw, qkv):
+                return super().project_encode_store(x, w_qkv, step, view, heads, kv_heads, head_dim)
+            return rt.ops.gemm_duo_qkv_rope(x, raw, qkv, step.positions, step.token_seq, view.block_table(step), self.table, view.k, view.v,
+                                            view.page_size, heads, kv_heads, head_dim, write_kv=view.store, whole=rt.duo_tiles(M, n_qkv))
         if fused == "rows":
             return rt.ops.gemm_rows_qkv_rope(x, raw, qkv, step.positions, step.token_seq, view.block_table(step), self.table,
                                              view.k, view.v, view.page_size, heads, kv_heads, head_dim, write_kv=view.store,

@@ -103,3 +103,18 @@ def test_products_of_long_prompts_take_it(monkeypatch, M, N, K):
     want = torch.nn.functional.silu(gate) * up
     got = rt.gated_linear(a, rt.weight(w, gated=True))
     assert calls and float(((got.double() - want).abs() / (want.abs() + want.abs().mean())).max()) <= 2.0 ** -7 and got.shape == (M, inner)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("whole", [0, None])
+@pytest.mark.parametrize("M,K,nh,nkv,hd", [(1, 256, 2, 1, 64), (129, 384, 3, 1, 48), (257, 256, 5, 2, 128), (300, 512, 32, 8, 64), (520, 256, 1, 1, 16)])
+def test_projection_with_rotation_and_pages(M, K, nh, nkv, hd, whole):
+    """Heads across and inside tiles and wavefronts, a padding row, rows of many sequences at unlike places of their pages; with and
+    without pages to write: as the projections of fewer rows are checked."""
+    from test_kernels import _check_qkv_rope
+    from burn_lm_amd.csrc import ops
+
+    def run(x, W, out, positions, token_seq, perm, cs, kd, vd, page, write_kv):
+        ops.gemm_duo_qkv_rope(x, W, out, positions, token_seq, perm, cs, kd, vd, page, nh, nkv, hd, write_kv=write_kv, whole=whole)
+
+    _check_qkv_rope(run, "interleaved", M, K, nh, nkv, hd)
