@@ -213,11 +213,29 @@ extern "C" int blm_gemm_f32(const void* A, const void* W, void* C, int M, int N,
 // KSTEPS: steps of 16 of K per wavefront.  WHOLE: every wavefront of every group has all of them, none partial, and nothing is
 // tested on the way (the tests for steps that a wavefront does not have cost 0.25 us: [1000, 520] at 8 rows 4.86 -> 5.11;
 // with them a decode step of 8 at the 1B shape took 1,547 us, so 1,533).  gated: a tile's columns are 8 gate rows and their 8 up rows, C = silu(gate) * up.
-template <int KSTEPS, bool WHOLE>
+// ROPE: the columns are query heads, then key heads and value heads; queries and keys turn in adjacent pairs (two neighbouring
+// lanes hold a pair's sums), keys and values go to their pages.  In place of a kernel of its own behind the product, 5 us of launch
+// and look-ups (8 rows, [3072, 2048]: 8.9 + 5.3 us under the profiler, so 9.9); the rows' sequences and positions are asked for ahead of
+// everything, their pages behind the weights.
+struct GvRope {
+  const int *positions, *token_seq, *block_table;
+  const float2* cos_sin;
+  float *kcache, *vcache;
+  int table_width, page_size, nh, nkv, hd, store;
+};
+
+template <int KSTEPS, bool WHOLE, bool ROPE>
 __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
     gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wp, float* __restrict__ C, int M, int N, int K,
-                    int lda, int ldc, int n_tiles, int k_steps, int gated, int steps_per_group, int tiles_per_block) {
+                    int lda, int ldc, int n_tiles, int k_steps, int gated, int steps_per_group, int tiles_per_block, GvRope rope) {
   __shared__ float red[GV_MAX_WAVES * 256];
+  __shared__ int pos_of[16], page_of[16];
+  int my_pos = 0, my_seq = -1;
+  if (ROPE && threadIdx.x < 16) {
+    const int m = min((int)threadIdx.x, M - 1);
+    my_pos = rope.positions[m];
+    my_seq = rope.token_seq[m];
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / BLM_WAVE), lane = threadIdx.x & (BLM_WAVE - 1);
   const int n_waves = blockDim.x / BLM_WAVE;
   const int row = lane & 15, kg = lane >> 4;
@@ -244,6 +262,10 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
   weights(tile_begin, 0, w[0]);
   weights(tile_begin, 1, w[1]);
   __builtin_amdgcn_sched_barrier(0);
+  if (ROPE && threadIdx.x < 16) {            // the barrier of the first tile's sum lies between these writes and their readers
+    pos_of[threadIdx.x] = my_pos;
+    page_of[threadIdx.x] = my_seq < 0 || !rope.store ? -1 : rope.block_table[(size_t)my_seq * rope.table_width + my_pos / rope.page_size];
+  }
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) a[s] = row < M && kbase + s * 16 < K && step0 + s < group_end ? a[s] : zero;
   for (int tile = tile_begin; tile < tile_end; ++tile) {
@@ -290,7 +312,20 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
         for (int x = 0; x + 1 < n_waves; x += 2) s += red[x * 256 + idx] + red[x * 256 + 256 + idx];
         if (n_waves & 1) s += red[(n_waves - 1) * 256 + idx];
         const int n = tile * 16 + col;
-        if (m < M && n < N) C[(size_t)m * ldc + n] = s;
+        if (ROPE) {
+          const float other = blm_dpp<BLM_DPP_XOR1>(s);
+          if (m >= M || n >= N) continue;
+          const int head = n / rope.hd, d = n - head * rope.hd, pos = pos_of[m], page = page_of[m], slot = pos % rope.page_size;
+          if (head < rope.nh + rope.nkv) {
+            const float2 cs = rope.cos_sin[(size_t)pos * (rope.hd / 2) + d / 2];
+            s = d & 1 ? other * cs.y + s * cs.x : s * cs.x - other * cs.y;
+          }
+          if (head < rope.nh) C[(size_t)m * ldc + n] = s;
+          else if (page >= 0 && head < rope.nh + rope.nkv) rope.kcache[(((size_t)page * rope.nkv + (head - rope.nh)) * rope.page_size + slot) * rope.hd + d] = s;
+          else if (page >= 0) rope.vcache[(((size_t)page * rope.nkv + (head - rope.nh - rope.nkv)) * rope.hd + d) * rope.page_size + slot] = s;
+        } else if (m < M && n < N) {
+          C[(size_t)m * ldc + n] = s;
+        }
       } else if (col < 8) {
         for (int x = 0; x + 1 < n_waves; x += 2) {
           s += red[x * 256 + idx] + red[x * 256 + 256 + idx];
@@ -335,9 +370,9 @@ extern "C" int blm_gemv_f32_geometry(int M, int N, int K, int groups, int* block
 // Wp: the packed copy of W[N, K], ceil(N / 16) * ceil(K / 16) * 256 floats.  gated: W's rows come in blocks of 8 gate rows and
 // their 8 up rows, and C is [M, N / 2].  groups > 1: K in that many groups, a plane of M * N for each (ldc = N), which the
 // reader adds up.
-extern "C" int blm_gemv_f32(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int ldc, int gated, int groups,
-                            hipStream_t stream) {
-  BLM_REQUIRE(M >= 1 && M <= 16 && N > 0 && K > 0 && lda >= K && ldc >= (gated ? N / 2 : N), "gemv_f32: bad sizes M=%d N=%d K=%d lda=%d ldc=%d", M, N, K, lda, ldc);
+static int gv_run(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int ldc, int gated, int groups, const GvRope* rope,
+                  hipStream_t stream) {
+  BLM_REQUIRE(M >= 1 && M <= 16 && N > 0 && K > 0 && lda >= K && ldc >= (rope ? rope->nh * rope->hd : gated ? N / 2 : N), "gemv_f32: bad sizes M=%d N=%d K=%d lda=%d ldc=%d", M, N, K, lda, ldc);
   BLM_REQUIRE(K % 4 == 0 && lda % 4 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)Wp % 16) == 0,
               "gemv_f32: rows must start at multiples of 16 bytes and hold a multiple of four elements (K=%d lda=%d)", K, lda);
   BLM_REQUIRE(groups >= 1 && groups <= 64 && (groups == 1 || (!gated && ldc == N)), "gemv_f32: bad number of groups %d", groups);
@@ -349,8 +384,14 @@ extern "C" int blm_gemv_f32(const void* A, const void* Wp, void* C, int M, int N
   const int per_block = (n_tiles + blocks - 1) / blocks;
   dim3 grid((unsigned)blocks, (unsigned)groups), block(waves * BLM_WAVE);
 #define BLM_GVF(KS, WHOLE)                                                                                              \
-  hipLaunchKernelGGL((gemv_f32_kernel<KS, WHOLE>), grid, block, 0, stream, (const float*)A, (const float*)Wp, (float*)C, M, N, K, \
-                     lda, ldc, n_tiles, k_steps, gated, steps, per_block)
+  do {                                                                                                                  \
+    if (rope)                                                                                                           \
+      hipLaunchKernelGGL((gemv_f32_kernel<KS, WHOLE, true>), grid, block, 0, stream, (const float*)A, (const float*)Wp, (float*)C, M, N, K, \
+                         lda, ldc, n_tiles, k_steps, gated, steps, per_block, *rope);                                   \
+    else                                                                                                                \
+      hipLaunchKernelGGL((gemv_f32_kernel<KS, WHOLE, false>), grid, block, 0, stream, (const float*)A, (const float*)Wp, (float*)C, M, N, K, \
+                         lda, ldc, n_tiles, k_steps, gated, steps, per_block, GvRope{});                                \
+  } while (0)
   const bool whole = K % 16 == 0 && k_steps == groups * steps && steps == waves * ksteps;
   if (ksteps == 4 && whole) BLM_GVF(4, true);
   else if (ksteps == 4) BLM_GVF(4, false);
@@ -359,4 +400,20 @@ extern "C" int blm_gemv_f32(const void* A, const void* Wp, void* C, int M, int N
 #undef BLM_GVF
   BLM_LAUNCH_CHECK("gemv_f32");
   return 0;
+}
+
+extern "C" int blm_gemv_f32(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int ldc, int gated, int groups,
+                            hipStream_t stream) {
+  return gv_run(A, Wp, C, M, N, K, lda, ldc, gated, groups, nullptr, stream);
+}
+
+// The q/k/v projection of up to 16 rows with the rotation (rotary partners are neighbouring columns) and the write of keys and
+// values into their pages.  qkv_out [M][ldq]: the queries.
+extern "C" int blm_gemv_f32_qkv_rope(const void* A, const void* Wp, void* qkv_out, const int* positions, const int* token_seq,
+                                     const int* block_table, int table_width, const void* cos_sin, void* kcache, void* vcache, int page_size,
+                                     int M, int K, int lda, int ldq, int nh, int nkv, int hd, int store, hipStream_t stream) {
+  BLM_REQUIRE(nh > 0 && nkv > 0 && hd > 0 && hd % 2 == 0 && page_size > 0 && table_width > 0, "gemv_f32_qkv_rope: bad geometry (head size %d)", hd);
+  BLM_REQUIRE(((uintptr_t)cos_sin % 8) == 0, "gemv_f32_qkv_rope: the table of angles must be 8-byte aligned");
+  const GvRope rope{positions, token_seq, block_table, (const float2*)cos_sin, (float*)kcache, (float*)vcache, table_width, page_size, nh, nkv, hd, store};
+  return gv_run(A, Wp, qkv_out, M, (nh + 2 * nkv) * hd, K, lda, ldq, 0, 1, &rope, stream);
 }

@@ -138,6 +138,7 @@ _SIGNATURES = {
                               _c_int, _c_int, _c_void_p, _c_int, _c_float, _c_int, _c_void_p],
     "blm_gemm_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_gemv_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "blm_gemv_f32_qkv_rope": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 9 + [_c_void_p],
     "blm_gemv_f32_geometry": [_c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p],
     "blm_gemm_tiled": [_c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                        _c_int, _c_int, _c_void_p],
@@ -646,6 +647,30 @@ def gemv_f32(a, packed, out, K, gated=False):
     _call("blm_gemv_f32", a.data_ptr(), packed.data_ptr(), out.data_ptr(), M, N, K, a.stride(0), out.stride(-2), 1 if gated else 0,
           groups, _stream())
     return out
+
+
+def gemv_f32_qkv_rope(x, packed, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache, page_size, nh, nkv, hd, write_kv=True):
+    """Up to 16 float32 rows: x [M, K] @ W_qkv^T from packed = pack_weight(w) of w [(nh + 2 nkv) * hd, K] with rotary partners in
+    adjacent rows (K in one group), rotary encoding of q and k, q into qkv_out[:, :nh*hd], k and v into their cache pages, in one
+    kernel."""
+    _gpu(x, packed, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache)
+    M, K = x.shape
+    N = (nh + 2 * nkv) * hd
+    if any(t.dtype != torch.float32 for t in (x, packed, qkv_out, kcache, vcache, cos_sin)):
+        raise KernelError("gemv_f32_qkv_rope: float32 operands, pages and angles wanted")
+    if packed.numel() != ((N + 15) // 16) * ((K + 15) // 16) * 256 or not packed.is_contiguous():
+        raise KernelError(f"gemv_f32_qkv_rope: the packed weights have {packed.numel()} elements, not those of a [{N}, {K}] matrix")
+    if qkv_out.shape[0] != M or qkv_out.stride(1) != 1 or qkv_out.shape[1] < nh * hd or x.stride(1) != 1:
+        raise KernelError("gemv_f32_qkv_rope: qkv_out must be [M, >= heads*head_dim] with unit stride along rows")
+    _i32("positions", positions, M); _i32("token_seq", token_seq, M); _i32("block_table", block_table)
+    if cos_sin.shape[1:] != (hd // 2, 2) or not cos_sin.is_contiguous():
+        raise KernelError("gemv_f32_qkv_rope: cos_sin must be contiguous [positions, head_dim/2, 2]")
+    _contig("kcache", kcache); _contig("vcache", vcache)
+    _check_planes("gemv_f32_qkv_rope", kcache, vcache, nkv, page_size, hd)
+    _call("blm_gemv_f32_qkv_rope", x.data_ptr(), packed.data_ptr(), qkv_out.data_ptr(), positions.data_ptr(), token_seq.data_ptr(),
+          block_table.data_ptr(), block_table.shape[1], cos_sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), page_size, M, K,
+          x.stride(0), qkv_out.stride(0), nh, nkv, hd, 1 if write_kv else 0, _stream())
+    return qkv_out
 
 
 def gemv_skinny(a, w, out):

@@ -553,6 +553,13 @@ class Runtime:
         # float32 logits from bfloat16 operands with many rows: own kernel (float accumulation)
         return ops.gemm_tiled(x, w, out)
 
+    def f32_qkv_packed(self, x, w, M, N, K):
+        """The packed copy of a float32 q/k/v projection that ops.gemv_f32_qkv_rope reads, or None where another kernel does it."""
+        if not (isinstance(w, LinearWeight) and M <= F32_SKINNY_MAX_ROWS and w.dtype == x.dtype == torch.float32 and not w.gated
+                and ops.f32_rows(x, w.w) and self.f32_skinny_groups(M, N, K, False) == 1):
+            return None
+        return w.packed
+
     def duo_tiles(self, M, N):
         """How many of a product's tiles ops.gemm_duo runs as whole ones."""
         return duo_plan(M, N, self.compute_units)[0]

@@ -152,10 +152,18 @@ class RotaryEncoding(PositionEncoding):
         elif (plan is None and bf16 and self.pairing == PAIRING["interleaved"] and raw is not None and raw.dtype == torch.bfloat16
                 and head_dim % 16 == 0 and hasattr(rt, "duo_qkv") and rt.duo_qkv(M, n_qkv, K)):
             fused = "tiles"
+        elif (M <= 16 and self.pairing == PAIRING["interleaved"] and x.dtype == view.k.dtype == torch.float32 and head_dim % 2 == 0
+                and hasattr(rt, "f32_qkv_packed")):
+            packed = rt.f32_qkv_packed(x, w_qkv, M, n_qkv, K)
+            fused = "float32" if packed is not None else None
         if fused is None:
             return super().project_encode_store(x, w_qkv, step, view, heads, kv_heads, head_dim)
         if step.max_position >= self.n_positions:
             raise ValueError(f"position {step.max_position} is past the rotary table of {self.n_positions}")
+        if fused == "float32":
+            return rt.ops.gemv_f32_qkv_rope(x, packed, torch.empty(M, n_qkv, dtype=torch.float32, device=x.device), step.positions,
+                                            step.token_seq, view.block_table(step), self.table, view.k, view.v, view.page_size, heads,
+                                            kv_heads, head_dim, write_kv=view.store)
         qkv = torch.empty(M, n_qkv, dtype=torch.bfloat16, device=x.device)
         if fused == "tiles":
             if not rt.ops.gemm_duo_takes(x, raw, qkv):

@@ -180,3 +180,37 @@ def test_plan_is_made_once():
     assert f32_plan(777, 2048, 8192, 256, planes=True) is f32_plan(777, 2048, 8192, 256, planes=True)
     assert f32_plan(777, 2048, 8192, 256) is not f32_plan(777, 2048, 8192, 256, planes=True)
     assert f32_plan.cache_info().maxsize is not None
+
+
+@pytest.mark.parametrize("M,K,nh,nkv,hd", [(1, 64, 2, 1, 16), (3, 36, 3, 1, 6), (8, 2048, 32, 8, 64), (16, 520, 5, 5, 34), (7, 272, 1, 1, 128)])
+def test_projection_with_rotation_and_pages(M, K, nh, nkv, hd):
+    """Up to 16 rows: the fused kernel's queries and pages are those of the product followed by the rotation kernel (a rotation is two
+    products and a sum: an ulp of the larger one apart at most); a padding row writes no page, heads may end inside a tile of columns."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.runtime import Runtime
+    rt = Runtime(torch.float32, "cuda:0")
+    g = torch.Generator().manual_seed(M + K)
+    N, page = (nh + 2 * nkv) * hd, 64
+    x, w = torch.randn(M, K, generator=g).cuda(), rt.weight((torch.randn(N, K, generator=g) * K ** -0.5).cuda())
+    pos = torch.tensor([(37 * i + 5) % 250 for i in range(M)], dtype=torch.int32).cuda()
+    seq = torch.arange(M, dtype=torch.int32)
+    if M > 2:
+        seq[1] = -1
+    seq, table = seq.cuda(), torch.randperm(4 * M, generator=g).view(M, 4).int().cuda()
+    cs = torch.randn(256, hd // 2, 2, generator=g).cuda()
+    got = []
+    for fused in (True, False):
+        k, v = (torch.full((4 * M, nkv, *s), 9.0, device="cuda") for s in ((page, hd), (hd, page)))
+        for store in (False, True):
+            if fused:
+                packed = rt.f32_qkv_packed(x, w, M, N, K)
+                out = ops.gemv_f32_qkv_rope(x, packed, torch.full((M, N), 7.0, device="cuda"), pos, seq, table, cs, k, v, page, nh, nkv, hd, write_kv=store)
+                assert bool((out[:, nh * hd:] == 7).all())
+            else:
+                out = rt.linear(x, w)
+                ops.rope_kv_write(out, pos, seq, table, cs, k, v, page, nh, nkv, hd, 0, write_kv=store)
+            assert store or bool((k == 9).all() and (v == 9).all())
+        got.append((out[:, :nh * hd][seq >= 0], k, v))
+    for a, b in zip(*got):
+        assert torch.allclose(a, b, rtol=2.0 ** -21, atol=2.0 ** -20)
+    assert torch.equal(got[0][2], got[1][2])
