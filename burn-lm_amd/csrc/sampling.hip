@@ -190,8 +190,8 @@ __device__ __forceinline__ unsigned long long shfl_down_u64(unsigned long long v
 }
 
 // pass 1: the row's maximum; the last block also clears the row's histograms for the passes to come
-template <bool VEC>
-__global__ void __launch_bounds__(SMP_THREADS)
+template <bool VEC, int THREADS>
+__global__ void __launch_bounds__(THREADS)
     sample_max_kernel(const float* __restrict__ logits, int V, int ld, int slice_len, float* part_max,
                       SampleRow* rows, unsigned long long* hist, int n_rows, int* counters, int counter_step, int with_hist) {
   __shared__ float red[17];
@@ -200,10 +200,10 @@ __global__ void __launch_bounds__(SMP_THREADS)
   const float* x = logits + (size_t)row * ld;
   const int begin = slice * slice_len, end = min(V, begin + slice_len);
   float mx = -INFINITY;
-  for (int c0 = begin; c0 < end; c0 += 4 * SMP_CHUNK) {
+  for (int c0 = begin; c0 < end; c0 += 16 * THREADS) {
     float xs[4][4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) smp_load4<VEC>(x, c0 + u * SMP_CHUNK + tid * 4, end, xs[u]);
+    for (int u = 0; u < 4; ++u) smp_load4<VEC>(x, c0 + (u * THREADS + tid) * 4, end, xs[u]);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -222,18 +222,19 @@ __global__ void __launch_bounds__(SMP_THREADS)
   }
   if (with_hist)
     for (int level = 0; level < 3; ++level)
-      for (int b = tid; b < SMP_BINS; b += SMP_THREADS) hist[((size_t)level * n_rows + row) * SMP_BINS + b] = 0ull;
+      for (int b = tid; b < SMP_BINS; b += THREADS) hist[((size_t)level * n_rows + row) * SMP_BINS + b] = 0ull;
 }
 
 // passes 2 to 4: level 0 takes bits 29..19 of the weights' bit patterns, level 1 bits 18..8, level 2
 // bits 7..0 (e <= 1, so bits 31 and 30 are clear); the last block finds the lowest bin above which
 // less than the target mass lies
-template <bool VEC, int LEVEL>
-__global__ void __launch_bounds__(SMP_THREADS)
+template <bool VEC, int LEVEL, int THREADS>
+__global__ void __launch_bounds__(THREADS)
     sample_level_kernel(const float* __restrict__ logits, int V, int ld, int slice_len, float k2, float top_p,
                         SampleRow* rows, unsigned long long* hist, int n_rows, int* counters, int counter_step) {
   __shared__ unsigned long long bins[SMP_BINS];
-  __shared__ unsigned long long wave_tot[SMP_WAVES];
+  constexpr int WAVES = THREADS / BLM_WAVE;
+  __shared__ unsigned long long wave_tot[WAVES];
   __shared__ unsigned long long chosen_above;
   __shared__ int flag, found;
   const int row = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x, lane = tid & (BLM_WAVE - 1), w = tid / BLM_WAVE;
@@ -244,12 +245,12 @@ __global__ void __launch_bounds__(SMP_THREADS)
   constexpr int shift = LEVEL == 0 ? 19 : (LEVEL == 1 ? 8 : 0);
   constexpr uint32_t mask = LEVEL == 2 ? 0xffu : 0x7ffu;
   constexpr int above_bits = LEVEL == 0 ? 0 : (LEVEL == 1 ? 19 : 8);   // the digits above this level start here
-  for (int b = tid; b < SMP_BINS; b += SMP_THREADS) bins[b] = 0ull;
+  for (int b = tid; b < SMP_BINS; b += THREADS) bins[b] = 0ull;
   __syncthreads();
-  for (int c0 = begin; c0 < end; c0 += 4 * SMP_CHUNK) {
+  for (int c0 = begin; c0 < end; c0 += 16 * THREADS) {
     float xs[4][4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) smp_load4<VEC>(x, c0 + u * SMP_CHUNK + tid * 4, end, xs[u]);
+    for (int u = 0; u < 4; ++u) smp_load4<VEC>(x, c0 + (u * THREADS + tid) * 4, end, xs[u]);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -265,12 +266,12 @@ __global__ void __launch_bounds__(SMP_THREADS)
   }
   __syncthreads();
   unsigned long long* row_hist = hist + ((size_t)LEVEL * n_rows + row) * SMP_BINS;
-  for (int b = tid; b < SMP_BINS; b += SMP_THREADS)
+  for (int b = tid; b < SMP_BINS; b += THREADS)
     if (bins[b]) __hip_atomic_fetch_add(row_hist + b, bins[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (!smp_arrive_last(counters + (size_t)row * counter_step, &flag, gridDim.x)) return;
 
-  // thread t looks after bins 8 t .. 8 t + 7
-  constexpr int PER = SMP_BINS / SMP_THREADS;
+  // a thread looks after eight bins in a row, or two
+  constexpr int PER = SMP_BINS / THREADS;
   unsigned long long m[PER], tot = 0ull;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
@@ -286,12 +287,12 @@ __global__ void __launch_bounds__(SMP_THREADS)
   if (tid == 0) found = 0x7fffffff;
   if (lane == 0) wave_tot[w] = suf;
   __syncthreads();
-  for (int k = w + 1; k < SMP_WAVES; ++k) suf += wave_tot[k];
+  for (int k = w + 1; k < WAVES; ++k) suf += wave_tot[k];
   unsigned long long carry = rows[row].carry, target = rows[row].target;
   if (LEVEL == 0) {
     // the whole mass: what every bin holds
     unsigned long long total = wave_tot[0];
-    for (int k = 1; k < SMP_WAVES; ++k) total += wave_tot[k];
+    for (int k = 1; k < WAVES; ++k) total += wave_tot[k];
     target = (unsigned long long)((double)top_p * (double)total);
     if (target < 1ull) target = 1ull;
   }
@@ -314,7 +315,7 @@ __global__ void __launch_bounds__(SMP_THREADS)
   }
 }
 
-// inclusive prefix over the block's threads in thread order, and the block's total
+// inclusive prefix over the block's first SMP_THREADS threads in thread order, and their total
 __device__ __forceinline__ float smp_block_scan(float v, float* wave_sums, float& total) {
   const int lane = threadIdx.x & (BLM_WAVE - 1), w = threadIdx.x / BLM_WAVE;
   float incl = v;
@@ -324,7 +325,7 @@ __device__ __forceinline__ float smp_block_scan(float v, float* wave_sums, float
     if (lane >= d) incl += o;
   }
   __syncthreads();   // wave_sums may still be read from an earlier call
-  if (lane == BLM_WAVE - 1) wave_sums[w] = incl;
+  if (lane == BLM_WAVE - 1) wave_sums[w] = incl;      // (of all wavefronts; those behind the first four are not read)
   __syncthreads();
   float before = 0.f;
   total = 0.f;
@@ -337,14 +338,15 @@ __device__ __forceinline__ float smp_block_scan(float v, float* wave_sums, float
 
 // last pass: the kept mass of every chunk; the last block finds the chunk that holds the pick and
 // the token in it.  use_tau 0: no cut, every token with a weight is kept.
-template <bool VEC>
-__global__ void __launch_bounds__(SMP_THREADS)
+template <bool VEC, int THREADS>
+__global__ void __launch_bounds__(THREADS)
     sample_pick_kernel(const float* __restrict__ logits, const float* __restrict__ uniforms, int* __restrict__ out, int V,
                        int ld, int slice_len, float k2, int use_tau, const SampleRow* rows, float* chunk_mass,
                        int* counters, int counter_step) {
   __shared__ float red[17];
-  __shared__ float wave_sums[SMP_WAVES];
-  __shared__ float round_sums[SMP_ROUND][SMP_WAVES];
+  constexpr int GROUPS = THREADS / SMP_THREADS, EACH = GROUPS == 1 ? SMP_ROUND : SMP_ROUND / 2, ROUND = EACH * GROUPS;
+  __shared__ float wave_sums[THREADS / BLM_WAVE];
+  __shared__ float round_sums[ROUND][SMP_WAVES];
   __shared__ int flag, hit, last_with_mass;
   const int row = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x;
   const float* x = logits + (size_t)row * ld;
@@ -358,20 +360,24 @@ __global__ void __launch_bounds__(SMP_THREADS)
   };
   float* row_mass = chunk_mass + (size_t)row * gridDim.x * chunks;
   const float u = uniforms[row];   // asked for early: it may lie in host memory
-  // the chunks of the slice, SMP_ROUND at a time: all loads first, one barrier per round
-  for (int c0 = 0; c0 < chunks; c0 += SMP_ROUND) {
-    float xs[SMP_ROUND][4];
+  // the chunks of the slice, ROUND at a time, a chunk to SMP_THREADS of the threads: all loads first, one barrier per round
+  const int group = tid / SMP_THREADS, part = tid % SMP_THREADS;
+  for (int c0 = 0; c0 < chunks; c0 += ROUND) {
+    float xs[EACH][4];
 #pragma unroll
-    for (int r = 0; r < SMP_ROUND; ++r) smp_load4<VEC>(x, begin + (c0 + r) * SMP_CHUNK + tid * 4, c0 + r < chunks ? end : 0, xs[r]);
+    for (int r = 0; r < EACH; ++r) {
+      const int c = c0 + r * GROUPS + group;
+      smp_load4<VEC>(x, begin + c * SMP_CHUNK + part * 4, c < chunks ? end : 0, xs[r]);
+    }
     __syncthreads();   // round_sums may still be read from the round before
 #pragma unroll
-    for (int r = 0; r < SMP_ROUND; ++r) {
+    for (int r = 0; r < EACH; ++r) {
       const float s4 = ((kept(xs[r][0]) + kept(xs[r][1])) + kept(xs[r][2])) + kept(xs[r][3]);
       const float ws = wave_sum(s4);
-      if ((tid & (BLM_WAVE - 1)) == 0) round_sums[r][tid / BLM_WAVE] = ws;
+      if ((tid & (BLM_WAVE - 1)) == 0) round_sums[r * GROUPS + group][part / BLM_WAVE] = ws;
     }
     __syncthreads();
-    if (tid < SMP_ROUND && c0 + tid < chunks) {
+    if (tid < ROUND && c0 + tid < chunks) {
       float t = 0.f;
       for (int k = 0; k < SMP_WAVES; ++k) t += round_sums[tid][k];
       smp_store(row_mass + slice * chunks + c0 + tid, t);
@@ -379,6 +385,8 @@ __global__ void __launch_bounds__(SMP_THREADS)
   }
   if (!smp_arrive_last(counters + (size_t)row * counter_step, &flag, gridDim.x)) return;
 
+  // the first SMP_THREADS threads have the chunks from here on, and at last the chosen chunk's elements; the others none
+  const bool in = tid < SMP_THREADS;
   // chunks in index order: slice by slice; first their total, then the chunk in which u * total falls
   const int n = gridDim.x * chunks;
   if (tid == 0) { hit = 0x7fffffff; last_with_mass = -1; }
@@ -399,13 +407,13 @@ __global__ void __launch_bounds__(SMP_THREADS)
     float total = 0.f;
     for (int base = 0; base < n; base += SMP_THREADS) {
       float t;
-      smp_block_scan(base + tid < n ? smp_load(row_mass + base + tid) : 0.f, wave_sums, t);
+      smp_block_scan(in && base + tid < n ? smp_load(row_mass + base + tid) : 0.f, wave_sums, t);
       total += t;
     }
     want = u * total;
     float run = 0.f;   // mass in front of this round of chunks
     for (int base = 0; base < n; base += SMP_THREADS) {
-      const float mass = base + tid < n ? smp_load(row_mass + base + tid) : 0.f;
+      const float mass = in && base + tid < n ? smp_load(row_mass + base + tid) : 0.f;
       float t;
       const float incl = run + smp_block_scan(mass, wave_sums, t);
       if (mass > 0.f) {
@@ -432,7 +440,7 @@ __global__ void __launch_bounds__(SMP_THREADS)
   const int cs = chunk / chunks, cc = chunk % chunks;
   const int i0 = cs * slice_len + cc * SMP_CHUNK + tid * 4;
   float xs[4], es[4];
-  smp_load4<VEC>(x, i0, min(V, cs * slice_len + slice_len), xs);
+  smp_load4<VEC>(x, i0, in ? min(V, cs * slice_len + slice_len) : 0, xs);
 #pragma unroll
   for (int k = 0; k < 4; ++k) es[k] = kept(xs[k]);
   const float s4 = ((es[0] + es[1]) + es[2]) + es[3];
@@ -468,19 +476,34 @@ __global__ void __launch_bounds__(SMP_THREADS)
 // 118.2 / 110.3 / 127.1 / 148.5, 512 rows 292 / 330 / 402 / 590; 32,000 logits: 8 rows 47.1 / 43.9 / 44.0 / 46.1, 64 rows 50.5 /
 // 53.3 / 62.1 / 80.4, 512 rows 131 / 168 / 244 / 429.  (64 blocks win nowhere.)  All with a cache line for each row's arrival
 // counter: side by side, 1,024 blocks queue up at two lines in every pass (64 rows of 128K in 16 blocks 90.5 us).
-static int sample_slices(int R, int V) {
+// 16 to 64 rows of a large vocabulary: blocks of 1,024 threads, one to a compute unit, which ask for 16,384 tokens at once; 256
+// threads take 2 us for every 4,096, a trip to memory.  (The pick's sums stay those of 256 threads a chunk.)  Us, 256 threads as
+// above / 1,024 threads in 8 blocks a row up to 32 rows, in 4 beyond: 128,256 logits: 8 rows 35.5 / 37.5, 16 rows 38.6 / 38.3, 24 rows
+// 42.8 / 39.7, 32 rows 44.6 / 40.3, 48 rows 52.3 / 48.4, 64 rows 62.4 / 52.4, 128 rows 90 / 88, 256 rows 136 / 151; 50,021 logits: 32
+// rows 41.7 / 43.9, 48 rows 48.5 / 48.0, 64 rows 51.2 / 49.5, 96 rows 62 / 69.  Without the cut's three passes 33 rows 20.6 / 21.8,
+// 48 rows 22.7 / 23.2, 64 rows 28.9 / 24.5 (128,256) and 22.2 / 22.4 (50,021): there only many rows of the largest.
+static int sample_wide_slices(int R, int V, int cut) {      // 0: 256 threads
+  const int n = R <= 32 ? 8 : 4;
+  return R >= (cut ? 16 : 56) && R <= 64 && V >= n * (cut ? 12288 : 24576) ? n : 0;
+}
+static int sample_slices(int R, int V, int cut) {
+  if (const int wide = sample_wide_slices(R, V, cut)) return wide;
   int n = 4;
   while (n < SMP_SLICES && 32LL * n * n * R <= V) n *= 2;
   return n;
 }
-static int sample_slice_len(int R, int V) {
-  const int n = sample_slices(R, V);
+static int sample_slice_len(int R, int V, int cut) {
+  const int n = sample_slices(R, V, cut);
   return ((V + n - 1) / n + SMP_CHUNK - 1) / SMP_CHUNK * SMP_CHUNK;
 }
 
 // Bytes of scratch that blm_sample needs for R rows of V logits (see there for the layout).
 extern "C" long long blm_sample_scratch_bytes(int R, int V) {
-  const long long chunks = (long long)sample_slices(R, V) * (sample_slice_len(R, V) / SMP_CHUNK);
+  long long chunks = 0;
+  for (int cut = 0; cut < 2; ++cut) {
+    const long long n = (long long)sample_slices(R, V, cut) * (sample_slice_len(R, V, cut) / SMP_CHUNK);
+    chunks = n > chunks ? n : chunks;
+  }
   return (long long)R * (3 * SMP_BINS * 8 + sizeof(SampleRow) + SMP_SLICES * 4 + chunks * 4);
 }
 
@@ -494,32 +517,35 @@ extern "C" int blm_sample(const float* logits, const float* uniforms, int* out, 
   BLM_REQUIRE(top_p > 0.f, "sample: top_p must be > 0 (got %g)", (double)top_p);
   BLM_REQUIRE(counter_step >= 1, "sample: counters %d apart", counter_step);
   BLM_REQUIRE(scratch != nullptr && ((uintptr_t)scratch % 8) == 0 && counters != nullptr, "sample: scratch and counters needed");
-  const int slice_len = sample_slice_len(R, V);
+  const int cut = top_p < 1.0f ? 1 : 0;
+  const int slice_len = sample_slice_len(R, V, cut);
   unsigned long long* hist = reinterpret_cast<unsigned long long*>(scratch);
   SampleRow* rows = reinterpret_cast<SampleRow*>(hist + (size_t)3 * R * SMP_BINS);
   float* part_max = reinterpret_cast<float*>(rows + R);
   float* chunk_mass = part_max + (size_t)R * SMP_SLICES;
   const float k2 = 1.4426950408889634f / temperature;
   const bool vec = ld % 4 == 0 && ((uintptr_t)logits % 16) == 0;
-  const int cut = top_p < 1.0f ? 1 : 0;
-  dim3 grid(sample_slices(R, V), R), block(SMP_THREADS);
-#define SMP_LAUNCH(VEC)                                                                                              \
+  const bool wide = sample_wide_slices(R, V, cut) != 0;
+  dim3 grid(sample_slices(R, V, cut), R), block(wide ? 1024 : SMP_THREADS);
+#define SMP_LAUNCH(VEC, THREADS)                                                                                     \
   do {                                                                                                               \
-    hipLaunchKernelGGL(sample_max_kernel<VEC>, grid, block, 0, stream, logits, V, ld, slice_len, part_max, rows,     \
+    hipLaunchKernelGGL((sample_max_kernel<VEC, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, part_max, rows, \
                        hist, R, counters, counter_step, cut);                                                        \
     if (cut) {                                                                                                       \
-      hipLaunchKernelGGL((sample_level_kernel<VEC, 0>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
+      hipLaunchKernelGGL((sample_level_kernel<VEC, 0, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
                          rows, hist, R, counters, counter_step);                                                     \
-      hipLaunchKernelGGL((sample_level_kernel<VEC, 1>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
+      hipLaunchKernelGGL((sample_level_kernel<VEC, 1, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
                          rows, hist, R, counters, counter_step);                                                     \
-      hipLaunchKernelGGL((sample_level_kernel<VEC, 2>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
+      hipLaunchKernelGGL((sample_level_kernel<VEC, 2, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
                          rows, hist, R, counters, counter_step);                                                     \
     }                                                                                                                \
-    hipLaunchKernelGGL(sample_pick_kernel<VEC>, grid, block, 0, stream, logits, uniforms, out, V, ld, slice_len, k2, \
+    hipLaunchKernelGGL((sample_pick_kernel<VEC, THREADS>), grid, block, 0, stream, logits, uniforms, out, V, ld, slice_len, k2, \
                        cut, rows, chunk_mass, counters, counter_step);                                               \
   } while (0)
-  if (vec) SMP_LAUNCH(true);
-  else SMP_LAUNCH(false);
+  if (vec && wide) SMP_LAUNCH(true, 1024);
+  else if (vec) SMP_LAUNCH(true, SMP_THREADS);
+  else if (wide) SMP_LAUNCH(false, 1024);
+  else SMP_LAUNCH(false, SMP_THREADS);
 #undef SMP_LAUNCH
   BLM_LAUNCH_CHECK("sample");
   return 0;

@@ -980,3 +980,17 @@ def test_sample_of_more_rows_than_counters_apart(ops, V):
         assert torch.equal(ops.sample(x[:2048], u[:2048].clone(), 0.8, p), whole[:2048])
         assert torch.equal(ops.sample(x[2090:], u[2090:].clone(), 0.8, p), whole[2090:])
     assert not bool(ops.arrival_counters(x.device).any())
+
+
+@pytest.mark.parametrize("R,V", [(16, 98304), (33, 49152), (64, 50021), (32, 100003), (64, 128256)])
+def test_sample_of_many_rows_by_wide_blocks(ops, R, V):
+    """16 to 64 rows of a large vocabulary run in blocks of 1,024 threads: the same draws as row by row, with and without the nucleus."""
+    g = torch.Generator().manual_seed(V + R)
+    x, u = dev(torch.randn(R, V, generator=g) * 2), dev(torch.rand(R, generator=g))
+    x[R // 2] = -1e4                                     # flat
+    x[R // 3, V - 1] = 80.0                              # one token has it all, the last
+    u[0], u[1] = 0.0, 1.0 - 2.0 ** -24
+    for top_p in (0.9, 1.0, 1e-6):
+        whole = ops.sample(x, u, 0.8, top_p)
+        rows = torch.cat([ops.sample(x[i:i + 1].contiguous(), u[i:i + 1].contiguous(), 0.8, top_p) for i in range(R)])
+        assert torch.equal(whole, rows) and int(whole[R // 3]) == V - 1
