@@ -58,7 +58,7 @@ _SIGNATURES = {
     "blm_gelu_glu": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
     "blm_softcap": [_c_void_p, ctypes.c_longlong, _c_float, _c_void_p],
     "blm_rmsnorm_rows": [_c_void_p, _c_int, _c_int, _c_void_p, _c_float, _c_void_p, _c_int, _c_int, _c_void_p],
-    "blm_add_gated_rmsnorm": [_c_void_p, _c_void_p, _c_int, _c_int, ctypes.c_longlong, _c_void_p, _c_void_p, _c_float,
+    "blm_add_gated_rmsnorm": [_c_void_p, _c_void_p, _c_int, _c_int, ctypes.c_longlong, _c_void_p, _c_int, _c_void_p, _c_float,
                               _c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_float, _c_int, _c_void_p],
     "blm_scaled_add": [_c_void_p, _c_int, _c_int, _c_int] + [_c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_int] * 4
                       + [_c_void_p],
@@ -332,7 +332,7 @@ def add_rmsnorm(h, delta, gamma, eps, out, rows=None, write_h=True, gate=None, g
     """v = h[r] (+ delta[r]); h[r] = v if write_h; out[i] = v / sqrt(mean(v^2) + eps) * gamma,
     with r = rows[i] if rows is given, else i.  h is the float32 residual stream.  delta: [T, D] in
     out's dtype, or float32 [planes, T, D] whose planes are summed (partial matrix products).
-    gate ([T, D] in out's dtype; with gate_bias float32 [D] or None): the summed delta joins as
+    gate ([T, D] in out's dtype, rows of any stride; with gate_bias float32 [D] or None): the summed delta joins as
     mult * delta * sigmoid(gate + gate_bias)."""
     _gpu(h, delta, gamma, out, rows, gate, gate_bias)
     D = h.shape[1]
@@ -357,12 +357,11 @@ def add_rmsnorm(h, delta, gamma, eps, out, rows=None, write_h=True, gate=None, g
     elif n_out != h.shape[0]:
         raise KernelError("add_rmsnorm: out needs one row per row of h when rows is not given")
     if gate is not None:
-        _contig("gate", gate)
-        if delta is None or gate.shape != h.shape or gate.dtype != out.dtype:
-            raise KernelError("add_rmsnorm: a gate comes with a delta, is [T, D] and of out's dtype")
+        if delta is None or gate.shape != h.shape or gate.dtype != out.dtype or gate.stride(1) != 1:
+            raise KernelError("add_rmsnorm: a gate comes with a delta, is [T, D] with contiguous rows and of out's dtype")
         if gate_bias is not None:
             _f32("gate_bias", gate_bias, D)
-        _call("blm_add_gated_rmsnorm", h.data_ptr(), _ptr(delta), dcode, planes, stride, gate.data_ptr(), _ptr(gate_bias),
+        _call("blm_add_gated_rmsnorm", h.data_ptr(), _ptr(delta), dcode, planes, stride, gate.data_ptr(), max(D, gate.stride(0)), _ptr(gate_bias),
               float(mult), gamma.data_ptr(), _code(gamma), out.data_ptr(), _code(out), _ptr(rows), n_out, D, float(eps),
               1 if write_h else 0, _stream())
         return out

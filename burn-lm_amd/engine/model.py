@@ -68,6 +68,8 @@ class Model:
         self.rt = rt
         for p in self.all_parts():
             p.bind(tensors, rt)
+        for b in self.blocks:
+            b.bound()
 
     def cache_needs(self) -> List:
         return [self.blocks[pl.layer].cache_need() for pl in self.plan.order]

@@ -38,26 +38,41 @@ class ResidualGate(Part):
     def step_flops(self, rows):
         return 2 * rows * sum(w.w.numel() for w in self.weights.values())
 
-    def gated(self, role, x, y):
-        """The sublayer's result y (of the rows x it read) with its gate, for the next norm's add."""
-        return Gated(y, self.rt.linear(x, self.weights[role]), self.biases[role], self.mult)
+    def gated(self, role, x, y, z=None):
+        """The sublayer's result y (of the rows x it read) with its gate (z: its product where it is formed already), for the next
+        norm's add."""
+        return Gated(y, self.rt.linear(x, self.weights[role]) if z is None else z, self.biases[role], self.mult)
 
 
-class GatedPreNormBlock(Block):
+class _GatedMixer(Block):
+    """The mixer's half: where the mixer can, its gate's projection is part of its own first product."""
+
+    def bound(self):
+        if self.mixer.take_beside(self.gate.weights["mixer"]):
+            del self.gate.weights["mixer"]
+
+    def mixed(self, x, step, view):
+        if self.mixer.beside_at is None:
+            return self.gate.gated("mixer", x, self.mixer.forward(x, step, view))
+        y, z = self.mixer.forward_beside(x, step, view)
+        return self.gate.gated("mixer", x, y, z)
+
+
+class GatedPreNormBlock(_GatedMixer):
     roles = {"mixer_norm": "norm", "mixer": "mixer", "ffn_norm": "norm", "feed_forward": "feed_forward",
              "gate": "connection"}
 
     def forward(self, h, delta, step, view):
         x = self.mixer_norm.add_norm(h, delta)
-        a = self.gate.gated("mixer", x, self.mixer.forward(x, step, view))
+        a = self.mixed(x, step, view)
         x = self.ffn_norm.add_norm(h, a)
         return self.gate.gated("feed_forward", x, self.feed_forward.forward(x, step))
 
 
-class GatedPreNormMixerBlock(Block):
+class GatedPreNormMixerBlock(_GatedMixer):
     """The same without a feed-forward."""
     roles = {"mixer_norm": "norm", "mixer": "mixer", "gate": "connection"}
 
     def forward(self, h, delta, step, view):
         x = self.mixer_norm.add_norm(h, delta)
-        return self.gate.gated("mixer", x, self.mixer.forward(x, step, view))
+        return self.mixed(x, step, view)

@@ -110,7 +110,7 @@ class LatentAttention(Mixer):
         self.down_at = starts[1] if not self.borrows else 0
         self.down_n = 0 if self.borrows else self.R + self.dr
         self.gate_at = starts[-1] if self.gated else 0
-        self.w_in = rt.weight(torch.cat(stacked, dim=0))
+        self.w_in, self.beside_at = rt.weight(torch.cat(stacked, dim=0)), None
         # (a reading layer writes no rows and has no weight for their norm; the kernel's check wants one of its size)
         self.norm_w = torch.ones(self.R, dtype=torch.float32, device=rt.device) if self.borrows \
             else tensors[n["dkv_norm"]].float().contiguous()
@@ -173,10 +173,17 @@ class LatentAttention(Mixer):
         return sum(min(past + t + 1, self.window) for t in range(new)) if self.window else new * past + new * (new + 1) // 2
 
     def forward(self, x, step, view):
+        return self._forward(x, step, view)[0]
+
+    def forward_beside(self, x, step, view):
+        y, qd = self._forward(x, step, view)
+        return y, qd[:, self.beside_at:]
+
+    def _forward(self, x, step, view):
         qd, q, gate = self._inputs(x)
         if self.expands(step, q, view):
-            return self._finish(self.attend_expanded(self._turn(qd, q, step, view), step, view), gate)
-        return self.output(self.attend(self._absorb(qd, q, step, view), step, view), gate)
+            return self._finish(self.attend_expanded(self._turn(qd, q, step, view), step, view), gate), qd
+        return self.output(self.attend(self._absorb(qd, q, step, view), step, view), gate), qd
 
     def project_expanded(self, x, step, view):
         """The plain queries and their turned lanes, for attend_expanded, with the step's rows in the cache afterwards; None, with nothing

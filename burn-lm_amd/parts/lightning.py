@@ -45,7 +45,7 @@ class LightningAttention(Mixer):
         rows = sum(w.shape[0] for w in ws)
         if rows % 8:
             ws.append(torch.zeros(8 - rows % 8, ws[0].shape[1], dtype=ws[0].dtype, device=ws[0].device))
-        self.w_in = rt.weight(torch.cat(ws, dim=0))
+        self.w_in, self.beside_at = rt.weight(torch.cat(ws, dim=0)), None
         self.w_o = rt.weight(tensors[n["o"]])
         self.norm_w = tensors[n["norm"]].float().contiguous()
         self.in_chunks = rt.ops.lightning_chunks_supported(self.dk, self.dv)
@@ -64,6 +64,10 @@ class LightningAttention(Mixer):
 
     def forward(self, x, step, view):
         return self.output(self.scan(self.project(x), step, view))
+
+    def forward_beside(self, x, step, view):
+        proj = self.project(x)
+        return self.output(self.scan(proj, step, view)), proj[:, self.beside_at:]
 
     def project(self, x):
         """The stacked projection [q | k | v | g]."""

@@ -143,7 +143,7 @@ class SinkAttention(Mixer):
         rows = sum(w.shape[0] for w in ws)
         if rows % 8:
             ws.append(torch.zeros(8 - rows % 8, ws[0].shape[1], dtype=ws[0].dtype, device=ws[0].device))
-        self.w_in = rt.weight(torch.cat(ws, dim=0))
+        self.w_in, self.beside_at = rt.weight(torch.cat(ws, dim=0)), None
         self.bias_in = torch.cat([tensors[n[r + "_bias"]].float() for r in roles]).contiguous() if bias else None
         self.w_o = rt.weight(tensors[n["o"]])
         self.output_bias = tensors[n["o_bias"]].float().contiguous() if p.get("output_bias", bias) else None
@@ -185,6 +185,16 @@ class SinkAttention(Mixer):
         """The whole mixer, its output bias added."""
         out = self.rt.linear(self.attend(self.project(x, step, view), step, view), self.w_o)
         return out.add_(self.output_bias.to(out.dtype)) if self.output_bias is not None else out
+
+    def forward_beside(self, x, step, view):
+        """(forward's result, the other product's columns): for layers whose projected rows stay as they are (no norm of queries and
+        keys, which may hand on rows of their own)."""
+        qkv = self.project(x, step, view)
+        out = self.rt.linear(self.attend(qkv, step, view), self.w_o)
+        return (out.add_(self.output_bias.to(out.dtype)) if self.output_bias is not None else out), qkv[:, self.beside_at:]
+
+    def take_beside(self, weight):
+        return not self.qk_norm and super().take_beside(weight)
 
     def forward_unbiased(self, x, step, view):
         """(result without the output projection's bias, possibly as partial planes; that bias in float32): for a
