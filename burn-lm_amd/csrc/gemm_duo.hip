@@ -38,9 +38,9 @@ struct GdTile {
   int rows, columns;                         // that exist, from the tile's first on: those beyond are the last one again
   uint32_t up;                               // bytes from a gate row to its up row
   int lda, ldw;
+  bool gated;
   __device__ __forceinline__ uint32_t row(int m) const { return (uint32_t)(min(m, rows - 1) * lda) * 2u; }
   __device__ __forceinline__ uint32_t column(int r, int h) const {
-    const bool gated = MODE == 1 || MODE == 2;
     const int n = min(gated ? r : r / 32 * 64 + h * 32 + r % 32, columns - 1);
     return (uint32_t)n * (uint32_t)ldw * 2u + (gated && h ? up : 0u);
   }
@@ -128,12 +128,18 @@ __device__ __forceinline__ void gd_store_rope(const gd_f32x4 (&acc)[TILES][4], b
   }
 }
 
+// Gated modes: columns of tiles from `gate_tiles` on are a plain product of the rows behind the up rows, C2 [M, N2] (n_tiles counts both).
+struct GdBeside {
+  bf16* C;
+  int N, ldc, gate_tiles;
+};
+
 // Tiles in the order in which they are walked: [0, whole) as whole ones, the rest of the m_tiles x n_tiles as two halves each, and
 // behind them, where `tail`, a row of halves below the last row of tiles.
 template <int MODE, typename TC>
 __global__ void __launch_bounds__(512, 2)
     gemm_duo_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, TC* __restrict__ C, int M, int N, int K, int lda, int ldw,
-                    int ldc, int m_tiles, int n_tiles, int whole, int k_per_group, GdRope rope) {
+                    int ldc, int m_tiles, int n_tiles, int whole, int k_per_group, GdRope rope, GdBeside beside) {
   constexpr bool GATED = MODE == 1 || MODE == 2;
   constexpr int OUT = GATED ? GD_TILE / 2 : GD_TILE;       // output columns of a tile
   __shared__ __attribute__((aligned(1024))) unsigned char lds[9 * GD_REGION];
@@ -162,12 +168,14 @@ __global__ void __launch_bounds__(512, 2)
       tn = (t - group * in_group) / height;
     }
   }
-  const int m0 = tm * GD_TILE + below, n0 = tn * OUT, k0 = blockIdx.y * k_per_group, stages = min(k_per_group, K - k0) / GD_BK;
+  const bool plain = GATED && tn >= beside.gate_tiles;
+  if (plain) tn -= beside.gate_tiles;
+  const int m0 = tm * GD_TILE + below, n0 = tn * (plain ? GD_TILE : OUT), k0 = blockIdx.y * k_per_group, stages = min(k_per_group, K - k0) / GD_BK;
   if (m0 >= M) return;                       // a second half that has no rows
   C += (size_t)blockIdx.y * M * ldc;
-  const GdTile<MODE> t = {reinterpret_cast<const char*>(A + (size_t)m0 * lda + k0), reinterpret_cast<const char*>(W + (size_t)n0 * ldw + k0),
-                          M - m0, N - n0, (uint32_t)N * (uint32_t)ldw * 2u, lda, ldw};
-  const int n = n0 + wn * (GATED ? 32 : 64);
+  const GdTile<MODE> t = {reinterpret_cast<const char*>(A + (size_t)m0 * lda + k0), reinterpret_cast<const char*>(W + (size_t)(n0 + (plain ? 2 * N : 0)) * ldw + k0),
+                          M - m0, (plain ? beside.N : N) - n0, (uint32_t)N * (uint32_t)ldw * 2u, lda, ldw, GATED && !plain};
+  const int n = n0 + wn * (GATED && !plain ? 32 : 64);
   if constexpr (MODE == 3) {
     __shared__ int pos_of[GD_TILE], page_of[GD_TILE];
     if (tid < GD_TILE) {
@@ -187,11 +195,13 @@ __global__ void __launch_bounds__(512, 2)
   } else if (!half) {
     gd_f32x4 acc[8][4];
     gd_whole(acc, t, stages, lds, wave, lane);
-    gd_store<MODE, 8, TC>(acc, C, ldc, m0 + wm * 128, M, n, N, l16, quad);
+    if (GATED && plain) gd_store<0, 8, bf16>(acc, beside.C, beside.ldc, m0 + wm * 128, M, n, beside.N, l16, quad);
+    else gd_store<MODE, 8, TC>(acc, C, ldc, m0 + wm * 128, M, n, N, l16, quad);
   } else {
     gd_f32x4 acc[4][4];
     gd_half(acc, t, stages, lds, wave, lane);
-    gd_store<MODE, 4, TC>(acc, C, ldc, m0 + wm * 64, M, n, N, l16, quad);
+    if (GATED && plain) gd_store<0, 4, bf16>(acc, beside.C, beside.ldc, m0 + wm * 64, M, n, beside.N, l16, quad);
+    else gd_store<MODE, 4, TC>(acc, C, ldc, m0 + wm * 64, M, n, N, l16, quad);
   }
 }
 
@@ -199,7 +209,7 @@ __global__ void __launch_bounds__(512, 2)
 // GELU in place of silu.  k_groups > 1: C is float [k_groups, M, ldc], a partial product over each group's stretch of K (a multiple
 // of 128).  whole: how many of the tiles are run as whole ones, the others as halves.
 static int gd_run(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, int mode,
-                  int k_groups, int whole, const GdRope* rope, hipStream_t stream) {
+                  int k_groups, int whole, const GdRope* rope, GdBeside beside, hipStream_t stream) {
   BLM_REQUIRE(M >= 1 && N >= 8 && N % 8 == 0 && K >= 256 && K % 128 == 0, "gemm_duo: sizes M=%d N=%d K=%d not supported", M, N, K);
   BLM_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && ldc % 8 == 0 && lda >= K && ldw >= K && ldc >= (rope ? rope->nh * rope->hd : N), "gemm_duo: bad strides lda=%d ldw=%d ldc=%d",
               lda, ldw, ldc);
@@ -208,9 +218,11 @@ static int gd_run(const void* A, const void* W, void* C, int c_dtype, int M, int
   const int k_per_group = k_groups >= 1 ? ((K + k_groups - 1) / k_groups + 127) / 128 * 128 : 0;
   BLM_REQUIRE(k_groups >= 1 && k_groups <= 64 && (k_groups == 1 || c_dtype == BLM_F32) && K - (k_groups - 1) * k_per_group >= 256,
               "gemm_duo: %d groups of K=%d need 256 each and a float output", k_groups, K);
-  BLM_REQUIRE((size_t)256 * lda * 2 < ((size_t)1 << 32) && (size_t)(mode != 0 ? 2 : 1) * N * ldw * 2 < ((size_t)1 << 32),
+  BLM_REQUIRE((size_t)256 * lda * 2 < ((size_t)1 << 32) && ((size_t)(mode != 0 ? 2 : 1) * N + beside.N) * ldw * 2 < ((size_t)1 << 32),
               "gemm_duo: matrices of 4 GiB and more are not supported (lda=%d, N=%d, ldw=%d)", lda, N, ldw);
-  const int columns = mode != 0 ? GD_TILE / 2 : GD_TILE, n_tiles = (N + columns - 1) / columns;
+  const int columns = mode != 0 ? GD_TILE / 2 : GD_TILE;
+  beside.gate_tiles = (N + columns - 1) / columns;
+  const int n_tiles = beside.gate_tiles + (beside.N + GD_TILE - 1) / GD_TILE;
   const bool tail = M % GD_TILE != 0 && M % GD_TILE <= GD_TILE / 2;
   const int m_tiles = tail ? M / GD_TILE : (M + GD_TILE - 1) / GD_TILE;
   BLM_REQUIRE((long long)(m_tiles + 1) * n_tiles < (1LL << 29), "gemm_duo: too many tiles");
@@ -219,7 +231,7 @@ static int gd_run(const void* A, const void* W, void* C, int c_dtype, int M, int
   const dim3 grid((unsigned)(whole + halves), (unsigned)k_groups), block(512);
 #define GD_LAUNCH(MODE, TC)                                                                                                        \
   hipLaunchKernelGGL((gemm_duo_kernel<MODE, TC>), grid, block, 0, stream, (const bf16*)A, (const bf16*)W, (TC*)C, M, N, K, lda, ldw, \
-                     ldc, m_tiles, n_tiles, whole, k_per_group, rope ? *rope : GdRope{})
+                     ldc, m_tiles, n_tiles, whole, k_per_group, rope ? *rope : GdRope{}, beside)
   if (rope) GD_LAUNCH(3, bf16);
   else if (mode == 1) GD_LAUNCH(1, bf16);
   else if (mode == 2) GD_LAUNCH(2, bf16);
@@ -232,7 +244,17 @@ static int gd_run(const void* A, const void* W, void* C, int c_dtype, int M, int
 
 extern "C" int blm_gemm_duo(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, int mode,
                             int k_groups, int whole, hipStream_t stream) {
-  return gd_run(A, W, C, c_dtype, M, N, K, lda, ldw, ldc, mode, k_groups, whole, nullptr, stream);
+  return gd_run(A, W, C, c_dtype, M, N, K, lda, ldw, ldc, mode, k_groups, whole, nullptr, GdBeside{}, stream);
+}
+
+// A gated product (mode 1 or 2) with a plain one of the same rows beside it: W [2N + N2, K], C2[M, N2] the product with the last N2
+// rows.  Its tiles fill what the gated ones leave of the last round (2,166 rows, 8,192 gated and 2,048 beside, K = 2,048: 118 us
+// and 31 apart).
+extern "C" int blm_gemm_duo_beside(const void* A, const void* W, void* C, void* C2, int M, int N, int N2, int K, int lda, int ldw, int ldc, int ldc2,
+                                   int mode, int whole, hipStream_t stream) {
+  BLM_REQUIRE((mode == 1 || mode == 2) && N2 > 0 && N2 % 8 == 0 && ldc2 >= N2 && ldc2 % 8 == 0 && ((uintptr_t)C2 % 16) == 0,
+              "gemm_duo_beside: mode %d, %d columns in rows of %d not supported", mode, N2, ldc2);
+  return gd_run(A, W, C, BLM_BF16, M, N, K, lda, ldw, ldc, mode, 1, whole, nullptr, GdBeside{(bf16*)C2, N2, ldc2, 0}, stream);
 }
 
 // The q/k/v projection with the rotation of queries and keys (on the float results) and the write of keys and values into their
@@ -243,5 +265,5 @@ extern "C" int blm_gemm_duo_qkv_rope(const void* A, const void* W, void* qkv_out
   BLM_REQUIRE(nh > 0 && nkv > 0 && hd > 0 && hd % 16 == 0 && page_size > 0 && table_width > 0, "gemm_duo_qkv_rope: head size %d not supported (a multiple of 16)", hd);
   BLM_REQUIRE(((uintptr_t)kcache % 16) == 0 && ((uintptr_t)cos_sin % 16) == 0, "gemm_duo_qkv_rope: pages and angles must be 16-byte aligned");
   const GdRope rope{positions, token_seq, block_table, cos_sin, (bf16*)kcache, (bf16*)vcache, table_width, page_size, nh, nkv, hd, store};
-  return gd_run(A, W, qkv_out, BLM_BF16, M, (nh + 2 * nkv) * hd, K, lda, ldw, ldq, 0, 1, whole, &rope, stream);
+  return gd_run(A, W, qkv_out, BLM_BF16, M, (nh + 2 * nkv) * hd, K, lda, ldw, ldq, 0, 1, whole, &rope, GdBeside{}, stream);
 }

@@ -158,6 +158,7 @@ _SIGNATURES = {
                       _c_int, _c_int, _c_int, _c_void_p],
     "blm_gemm_duo": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                      _c_void_p],
+    "blm_gemm_duo_beside": [_c_void_p] * 4 + [_c_int] * 10 + [_c_void_p],
     "blm_gemm_duo_qkv_rope": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 11 + [_c_void_p],
     "blm_gemv_mfma_group_limit": [_c_int],
     "blm_gemv_qkv_rope_supported": [_c_int, _c_int, _c_int, _c_int],
@@ -890,9 +891,24 @@ def gemm_duo_qkv_rope(x, w, qkv_out, positions, token_seq, block_table, cos_sin,
     return qkv_out
 
 
-def gemm_duo_tiles(M, N, gated=False):
-    """(tiles of 256x256, halves below them): a last row of tiles of at most 128 rows is halves only."""
-    columns = -(-N // (128 if gated else 256))
+def gemm_duo_beside(a, w, out, beside, activation="silu", whole=None):
+    """gemm_duo(gated=True) with w [2N + N2, K], and beside [M, N2] = a @ (w's last N2 rows)^T in the same launch (gemm_duo_takes both)."""
+    _gpu(a, w, out, beside)
+    (M, N), N2, K = out.shape, beside.shape[1], a.shape[1]
+    if a.shape[0] != M or beside.shape[0] != M or w.shape != (2 * N + N2, K):
+        raise KernelError(f"gemm_duo_beside: shapes a={tuple(a.shape)} w={tuple(w.shape)} out={tuple(out.shape)} beside={tuple(beside.shape)} do not fit")
+    if any(t.stride(1) != 1 or t.dtype != torch.bfloat16 for t in (a, w, out, beside)):
+        raise KernelError("gemm_duo_beside: bfloat16 operands with unit stride along their rows wanted")
+    _call("blm_gemm_duo_beside", a.data_ptr(), w.data_ptr(), out.data_ptr(), beside.data_ptr(), M, N, N2, K, a.stride(0), w.stride(0),
+          out.stride(0), beside.stride(0), 2 if activation == "gelu_tanh" else 1,
+          gemm_duo_tiles(M, N, True, N2)[0] if whole is None else whole, _stream())
+    return out, beside
+
+
+def gemm_duo_tiles(M, N, gated=False, beside=0):
+    """(tiles of 256x256, halves below them): a last row of tiles of at most 128 rows is halves only.  beside: columns of a plain
+    product beside a gated one."""
+    columns = -(-N // (128 if gated else 256)) + -(-beside // 256)
     tail = 0 < M % 256 <= 128
     return (M // 256 if tail else -(-M // 256)) * columns, columns if tail else 0
 

@@ -129,16 +129,16 @@ DUO_PLANES_K = 4096
 
 
 @functools.lru_cache(maxsize=4096)
-def duo_plan(M, N, compute_units, gated=False):
+def duo_plan(M, N, compute_units, gated=False, beside=0):
     """(whole tiles, rounds, fill) of ops.gemm_duo: the tiles that do not fill a round run as halves where that is shorter; rounds in
     the time of a whole tile; fill: the share of the rounds' time that works on rows and columns that exist."""
-    tiles, tail = ops.gemm_duo_tiles(M, N, gated)
+    tiles, tail = ops.gemm_duo_tiles(M, N, gated, beside)
     full, rest = divmod(tiles, compute_units)
     left = compute_units - rest if rest else 0            # units that a last, partial round of whole tiles leaves to the tail
     whole = full + (1 if rest else 0) + DUO_HALF * -(-max(0, tail - left) // compute_units)
     halves = full + DUO_HALF * -(-(2 * rest + tail) // compute_units)
     rounds = min(whole, halves)
-    return tiles if whole <= halves else tiles - rest, rounds, M * N / (32768.0 if gated else 65536.0) / compute_units / rounds
+    return tiles if whole <= halves else tiles - rest, rounds, M * (N / (32768.0 if gated else 65536.0) + beside / 65536.0) / compute_units / rounds
 
 
 class FusedProjectionPlan:
@@ -602,6 +602,20 @@ class Runtime:
         if M > 32:
             return K > 4096 or -(-inner // 32) > 2 * self.compute_units
         return K > 4096 and -(-inner // 32) > self.compute_units
+
+    def gated_linear_beside(self, x, w, beside, stacked, activation):
+        """(gated_linear(x, w, activation), linear(x, beside)) of two matrices that lie one behind the other in `stacked`: in one launch
+        where the gated product alone would be ops.gemm_duo's and the columns beside it take no more rounds of tiles than the
+        plain product would by itself (it fills what is left of the last one)."""
+        M, K = x.shape
+        inner, n = w.shape[0] // 2, beside.shape[0]
+        if M > 256 and self.fused_gate_up_measured and stacked.dtype == self.dtype == torch.bfloat16:
+            alone, both = (duo_plan(M, inner, self.compute_units, True, b) for b in (0, n))
+            if alone[2] >= DUO_GATED_FILL and both[2] >= DUO_GATED_FILL and both[1] - alone[1] <= DUO_HALF:
+                out, z = (torch.empty(M, m, dtype=self.dtype, device=x.device) for m in (inner, n))
+                if ops.gemm_duo_takes(x, stacked, out, gated=True) and ops.gemm_duo_takes(x, stacked, z):
+                    return ops.gemm_duo_beside(x, stacked, out, z, activation=activation, whole=both[0])
+        return self.gated_linear(x, w, activation=activation), self.linear(x, beside)
 
     def gated_linear(self, x, w, activation="silu"):
         """act(x gate^T) * (x up^T) for w = [gate rows; up rows] ([2I, K]) -> [M, I]; act is silu or

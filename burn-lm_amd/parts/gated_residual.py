@@ -48,17 +48,19 @@ class _GatedMixer(Block):
     """The mixer's half: where the mixer can, its gate's projection is part of its own first product."""
 
     def bound(self):
-        if self.mixer.take_beside(self.gate.weights["mixer"]):
+        if hasattr(self.mixer, "take_beside") and self.mixer.take_beside(self.gate.weights["mixer"]):
             del self.gate.weights["mixer"]
 
     def mixed(self, x, step, view):
-        if self.mixer.beside_at is None:
+        if "mixer" in self.gate.weights:
             return self.gate.gated("mixer", x, self.mixer.forward(x, step, view))
         y, z = self.mixer.forward_beside(x, step, view)
         return self.gate.gated("mixer", x, y, z)
 
 
 class GatedPreNormBlock(_GatedMixer):
+    """Where the feed-forward can, its gate's projection runs beside its own first product as well."""
+
     roles = {"mixer_norm": "norm", "mixer": "mixer", "ffn_norm": "norm", "feed_forward": "feed_forward",
              "gate": "connection"}
 
@@ -66,7 +68,15 @@ class GatedPreNormBlock(_GatedMixer):
         x = self.mixer_norm.add_norm(h, delta)
         a = self.mixed(x, step, view)
         x = self.ffn_norm.add_norm(h, a)
-        return self.gate.gated("feed_forward", x, self.feed_forward.forward(x, step))
+        if "feed_forward" in self.gate.weights:
+            return self.gate.gated("feed_forward", x, self.feed_forward.forward(x, step))
+        y, z = self.feed_forward.forward_beside(x, step)
+        return self.gate.gated("feed_forward", x, y, z)
+
+    def bound(self):
+        super().bound()
+        if hasattr(self.feed_forward, "take_beside") and self.feed_forward.take_beside(self.gate.weights["feed_forward"]):
+            del self.gate.weights["feed_forward"]
 
 
 class GatedPreNormMixerBlock(_GatedMixer):

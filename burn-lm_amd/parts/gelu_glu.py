@@ -23,16 +23,34 @@ class GeluGLU(FeedForward):
         g, u = tensors[self.names["gate"]], tensors[self.names["up"]]
         if g.dtype != u.dtype:
             g, u = g.float(), u.float()
-        self.w_gate_up = rt.weight(torch.cat([g, u], dim=0), gated=True)
+        self.w_gate_up, self.w_beside = rt.weight(torch.cat([g, u], dim=0), gated=True), None
         self.w_down = rt.weight(tensors[self.names["down"]])
         self.inner = self.params["inner"]
 
+    def take_beside(self, weight):
+        """Whether another product of the same rows ([tokens, n] of its own) now runs beside gate and up: forward_beside."""
+        own = self.w_gate_up
+        if own.dtype != weight.dtype or own.shape[1] != weight.shape[1] or weight.gated:
+            return False
+        self.stacked = torch.cat([own.w, weight.w], dim=0)        # each of the two is a stretch of it
+        self.w_gate_up = self.rt.weight(self.stacked[:own.shape[0]], gated=True)
+        self.w_beside = self.rt.weight(self.stacked[own.shape[0]:])
+        return True
+
+    def _weights(self):
+        return [w for w in (self.w_gate_up, self.w_down, self.w_beside) if w is not None]
+
     def step_bytes(self, rows):
-        return sum(w.w.numel() * w.w.element_size() for w in (self.w_gate_up, self.w_down))
+        return sum(w.w.numel() * w.w.element_size() for w in self._weights())
 
     def step_flops(self, rows):
-        return 2 * rows * (self.w_gate_up.w.numel() + self.w_down.w.numel())
+        return 2 * rows * sum(w.w.numel() for w in self._weights())
 
     def forward(self, x, step):
         rt = self.rt
         return rt.linear(rt.gated_linear(x, self.w_gate_up, activation="gelu_tanh"), self.w_down, partials=True)
+
+    def forward_beside(self, x, step):
+        """(forward's result, the other product's)."""
+        act, z = self.rt.gated_linear_beside(x, self.w_gate_up, self.w_beside, self.stacked, "gelu_tanh")
+        return self.rt.linear(act, self.w_down, partials=True), z

@@ -118,3 +118,18 @@ def test_projection_with_rotation_and_pages(M, K, nh, nkv, hd, whole):
         ops.gemm_duo_qkv_rope(x, W, out, positions, token_seq, perm, cs, kd, vd, page, nh, nkv, hd, write_kv=write_kv, whole=whole)
 
     _check_qkv_rope(run, "interleaved", M, K, nh, nkv, hd)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("M,N,N2,K", [(129, 136, 8, 256), (300, 256, 264, 384), (520, 264, 512, 256)])
+def test_plain_columns_beside_gated_ones(M, N, N2, K, activation):
+    """A gated product with a plain one of the same rows in its launch gives the bits of the two apart, whole tiles or halves."""
+    from burn_lm_amd.csrc import ops
+    a, w = operands(M, 2 * N + N2, K, False, M)
+    new = lambda n: torch.full((M, n), 7.0, dtype=torch.bfloat16, device="cuda")
+    gated, plain = ops.gemm_duo(a, w[:2 * N], new(N), gated=True, activation=activation), ops.gemm_duo(a, w[2 * N:], new(N2))
+    tiles, _ = ops.gemm_duo_tiles(M, N, True, N2)
+    for whole in sorted({0, tiles // 2, tiles}):
+        out, z = ops.gemm_duo_beside(a, w, new(N), new(N2), activation=activation, whole=whole)
+        assert torch.equal(out, gated) and torch.equal(z, plain)
