@@ -333,7 +333,7 @@ def add_rmsnorm(h, delta, gamma, eps, out, rows=None, write_h=True, gate=None, g
     """v = h[r] (+ delta[r]); h[r] = v if write_h; out[i] = v / sqrt(mean(v^2) + eps) * gamma,
     with r = rows[i] if rows is given, else i.  h is the float32 residual stream.  delta: [T, D] in
     out's dtype, or float32 [planes, T, D] whose planes are summed (partial matrix products).
-    gate ([T, D] in out's dtype, rows of any stride; with gate_bias float32 [D] or None): the summed delta joins as
+    gate ([T, D] in out's dtype, rows of any stride from D on; with gate_bias float32 [D] or None): the summed delta joins as
     mult * delta * sigmoid(gate + gate_bias)."""
     _gpu(h, delta, gamma, out, rows, gate, gate_bias)
     D = h.shape[1]
@@ -358,7 +358,8 @@ def add_rmsnorm(h, delta, gamma, eps, out, rows=None, write_h=True, gate=None, g
     elif n_out != h.shape[0]:
         raise KernelError("add_rmsnorm: out needs one row per row of h when rows is not given")
     if gate is not None:
-        if delta is None or gate.shape != h.shape or gate.dtype != out.dtype or gate.stride(1) != 1:
+        if delta is None or gate.shape != h.shape or gate.dtype != out.dtype or (D > 1 and gate.stride(1) != 1) \
+                or (gate.shape[0] > 1 and gate.stride(0) < D):
             raise KernelError("add_rmsnorm: a gate comes with a delta, is [T, D] with contiguous rows and of out's dtype")
         if gate_bias is not None:
             _f32("gate_bias", gate_bias, D)

@@ -609,7 +609,7 @@ class Runtime:
         plain product would by itself (it fills what is left of the last one)."""
         M, K = x.shape
         inner, n = w.shape[0] // 2, beside.shape[0]
-        if M > 256 and self.fused_gate_up_measured and stacked.dtype == self.dtype == torch.bfloat16:
+        if M > 256 and self.fused_gate_up_measured and stacked.dtype == self.dtype == torch.bfloat16 and stacked.numel() < 1 << 31:
             alone, both = (duo_plan(M, inner, self.compute_units, True, b) for b in (0, n))
             if alone[2] >= DUO_GATED_FILL and both[2] >= DUO_GATED_FILL and both[1] - alone[1] <= DUO_HALF:
                 out, z = (torch.empty(M, m, dtype=self.dtype, device=x.device) for m in (inner, n))

@@ -729,3 +729,17 @@ def test_greedy_generation_through_the_server(tmp_path):
     results, _ = server.generate(prompts, stop_ids=[])
     assert [r.tokens for r in results] == want
     server.unload()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,D,ld,at", [(5, 20, 24, 0), (7, 18, 41, 3), (40, 64, 200, 136), (3, 2048, 2056, 8)])
+def test_gates_that_are_columns_of_wider_rows(T, D, ld, at):
+    """The bits of the same gates in rows of their own; rows that overlap or repeat are refused."""
+    from burn_lm_amd.csrc import ops
+    g = torch.Generator().manual_seed(D)
+    h, y, gamma, z = (torch.randn(*s, generator=g).cuda() for s in ((T, D), (T, D), (D,), (T, ld)))
+    run = lambda gate: ops.add_rmsnorm(h.clone(), y, gamma, 1e-5, torch.empty_like(h), gate=gate)
+    assert torch.equal(run(z[:, at:at + D]), run(z[:, at:at + D].contiguous()))
+    for bad in (z[:1, :D].expand(T, D), z.flatten().as_strided((T, D), (D - 1, 1)), z[:, :1].expand(T, D)):
+        with pytest.raises(ops.KernelError):
+            run(bad)
