@@ -9,6 +9,8 @@
 // instructions.
 //   attn_prefill_f32 : a wavefront has sixteen queries of one head, the four of a block share the pages through shared memory
 //   attn_decode_f32  : the sixteen columns are the heads of one group at one token; wavefronts take pages in turn
+#include <type_traits>
+
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -20,13 +22,17 @@ __device__ __forceinline__ f32x4 af_load(const float* p) { return *reinterpret_c
 __device__ __forceinline__ f32x4 af_mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ bool af_visible(int key, int pos, int window) { return key <= pos && (window <= 0 || pos - key < window); }
 
+template <int V>
+using AfInt = std::integral_constant<int, V>;
+
 // Running softmax of one page: s[t][v] holds the scaled scores of this lane's query (l % 16) with keys 16 t + 4 (l / 16) + v,
 // -infinity where the query does not see the key; they become probabilities against the new maximum.  l is this lane's part
 // of the sum.  Returns the factor for what was summed before.
+template <int TILES = 4>
 __device__ __forceinline__ float af_softmax(f32x4* s, float& m, float& l) {
   float top = s[0][0];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < TILES; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) top = fmaxf(top, s[t][v]);
   const float m_new = fmaxf(m, rows_max(top));
@@ -34,7 +40,7 @@ __device__ __forceinline__ float af_softmax(f32x4* s, float& m, float& l) {
   const float keep = expf(m - base);
   float sum = 0.f;
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < TILES; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       s[t][v] = expf(s[t][v] - base);
@@ -220,8 +226,11 @@ __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
 // the block's piece of the key range in turn, fragments straight from the pages (a page is read by one wavefront only, whole
 // lines by neighbouring instructions).  The wavefronts' results meet in shared memory; with several pieces per token the blocks
 // leave theirs in device-coherent memory, count themselves in, and the last one adds them up (as attn_paged does).
+// A page takes a wavefront 128 products, 1.7 us at the matrix cores' rate, behind the fetch of 32 KB; where a round of whole pages would
+// leave wavefronts idle it goes in halves or quarters, one to a wavefront.
 // Measured (us a layer, 32 heads of 64 in 8 groups, 8 sequences of 400 to 640 keys; before: a wavefront per head, the heads of
-// a group each reading the group's keys and values): 43.8 -> 13.3 in three pieces.
+// a group each reading the group's keys and values): 43.8 -> 13.3 in three pieces of whole pages; in a graph of its own 11.4, with
+// halves 10.5; 8 sequences of 8 pages in four pieces 10.6 -> 9.3 in halves, 8.7 in quarters; 24 heads of 128 15.9 -> 12.4.
 // ---------------------------------------------------------------------------------------------------------------------
 template <int HD>
 __global__ void __launch_bounds__(AF_DECODE_WAVES* BLM_WAVE)
@@ -258,52 +267,68 @@ __global__ void __launch_bounds__(AF_DECODE_WAVES* BLM_WAVE)
   f32x4 o[DS];
 #pragma unroll
   for (int d = 0; d < DS; ++d) o[d] = zero;
-  for (int page = page_begin + wave; page < page_end; page += AF_DECODE_WAVES) {
+  // 16 * TILES keys of a page from tile t0 on
+  auto keys = [&](int page, int t0, auto tiles_type) {
+    constexpr int TILES = decltype(tiles_type)::value;
     const size_t base = ((size_t)pages[page] * nkv + kvh) * AF_PAGE * hd;
-    f32x4 kf[DS][4], vf[DS][4];
+    f32x4 kf[DS][TILES], vf[DS][TILES];
 #pragma unroll
     for (int i = 0; i < DS; ++i)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) kf[i][t] = i * 16 + g * 4 < hd ? af_load(kcache + base + (size_t)(t * 16 + c) * hd + i * 16 + g * 4) : zero;
+      for (int t = 0; t < TILES; ++t) kf[i][t] = i * 16 + g * 4 < hd ? af_load(kcache + base + (size_t)((t0 + t) * 16 + c) * hd + i * 16 + g * 4) : zero;
     // wide heads: the values' registers are the keys' once these are multiplied
     if (HD > 64) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int d = 0; HD <= 64 && d < DS; ++d)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) vf[d][t] = af_load(vcache + base + (size_t)min(d * 16 + c, hd - 1) * AF_PAGE + t * 16 + g * 4);
-    f32x4 s[4] = {zero, zero, zero, zero};
+      for (int t = 0; t < TILES; ++t) vf[d][t] = af_load(vcache + base + (size_t)min(d * 16 + c, hd - 1) * AF_PAGE + (t0 + t) * 16 + g * 4);
+    f32x4 s[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) s[t] = zero;
 #pragma unroll
     for (int i = 0; i < DS; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) s[t] = af_mfma(kf[i][t][e], qf[i][e], s[t]);
+        for (int t = 0; t < TILES; ++t) s[t] = af_mfma(kf[i][t][e], qf[i][e], s[t]);
     if (HD > 64) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int d = 0; d < DS; ++d)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) vf[d][t] = af_load(vcache + base + (size_t)min(d * 16 + c, hd - 1) * AF_PAGE + t * 16 + g * 4);
+        for (int t = 0; t < TILES; ++t) vf[d][t] = af_load(vcache + base + (size_t)min(d * 16 + c, hd - 1) * AF_PAGE + (t0 + t) * 16 + g * 4);
       __builtin_amdgcn_sched_barrier(0);
     }
-    const int key0 = page * AF_PAGE + g * 4;
-    bool see[4][4];
+    const int key0 = page * AF_PAGE + t0 * 16 + g * 4;
+    bool see[TILES][4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < TILES; ++t)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         see[t][v] = af_visible(key0 + t * 16 + v, pos, window);
         s[t][v] = see[t][v] ? s[t][v] * scale : -INFINITY;
       }
-    const float keep = af_softmax(s, m, l);
+    const float keep = af_softmax<TILES>(s, m, l);
 #pragma unroll
     for (int d = 0; d < DS; ++d) o[d] *= keep;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < TILES; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int d = 0; d < DS; ++d) o[d] = af_mfma(see[t][e] ? vf[d][t][e] : 0.f, s[t][e], o[d]);   // an unseen value may be anything
+  };
+  // whole pages, a round of the wavefronts at a time; a last round that would leave half of them idle goes in halves of pages, one
+  // that would leave three quarters idle in quarters
+  const int left = (page_end - page_begin) % AF_DECODE_WAVES;
+  const int whole_end = 2 * left <= AF_DECODE_WAVES ? page_end - max(0, left) : page_end;
+  for (int page = page_begin + wave; page < whole_end; page += AF_DECODE_WAVES) keys(page, 0, AfInt<4>{});
+  if (4 * left > AF_DECODE_WAVES) {
+    const int half = 2 * whole_end + wave;
+    if (half < 2 * page_end) keys(half / 2, half % 2 * 2, AfInt<2>{});
+  } else {
+    const int quarter = 4 * whole_end + wave;
+    if (quarter < 4 * page_end) keys(quarter / 4, quarter % 4, AfInt<1>{});
   }
   l = rows_sum(l);
 #pragma unroll

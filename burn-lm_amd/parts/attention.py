@@ -62,17 +62,18 @@ def decode_splits(pages: int, blocks: int, head_dim: int, compute_units: int = 2
 
 
 def decode_splits_f32(pages: int, blocks: int, head_dim: int, compute_units: int = 256) -> int:
-    """The same for float32 (ops.attn_decode_f32): a block's eight wavefronts take a page each, and a page takes one about
-    5 us (8 for wide heads), most of it the fetch's latency and the products of sixteen columns of which a group fills few;
-    the merge takes 2.  So pieces of three pages (two for wide heads), as long as every block has a compute unit to
-    itself; never more than 16 (us per call in pieces of the rule / whole, 32 heads of 64 in 8 groups: 8 pages at batch 1 11.1 / 12.2,
-    at batch 8 12.3 / 13.3; 12 pages at batch 8 13.1 / 17.5, at batch 16 18.1 / 22.9; 50 pages at batch 16 in two 48.4, in four
-    57.4; 24 heads of 128: 8 pages at batch 8 17.3 / 25.1).  Few key-value heads behind very many keys would take more
+    """The same for float32 (ops.attn_decode_f32): a block's eight wavefronts take a quarter, a half or a whole page each, and a
+    whole one takes a wavefront about 5 us (8 for wide heads), most of it the fetch's latency and the products of sixteen columns of
+    which a group fills few; the merge takes 1 to 2.  So pieces of two pages, which go in quarters, as long as every block has a
+    compute unit to itself; never more than 16 (us a call, whole / in 2 / 3 / 4 pieces, 32 heads of 64 in 8 groups: 4 pages at batch 8
+    7.9 / 7.8 / - / 7.9; 8 pages at batch 1 11.8 / 10.0 / - / 8.4, at batch 8 11.9 / 10.2 / 10.0 / 8.7; 12 pages at batch 8 16.3 /
+    13.4 / 10.9 / 10.9, at batch 16 17.6 / 15.3 / 19.9; 50 pages at batch 16 55 / 38 / - / 46; 24 heads of 128: 8 pages at batch 8
+    23.8 / 16.0 / - / 12.4).  Few key-value heads behind very many keys would take more
     pieces (one head of 64 at batch 1, 16 / 32 / 64 pieces: 16,000 keys 27 / 25 / 32, 65,000 keys 73 / 49 / 44, 130,000 keys
     135 / 82 / 61; the generic kernel 77, 202 and 248)."""
     if pages <= 4 and head_dim <= 64:
         return 1
-    return max(1, min(pages // (3 if head_dim <= 64 else 2), compute_units // max(1, blocks), 16))
+    return max(1, min(pages // 2, compute_units // max(1, blocks), 16))
 
 
 class Attention(Mixer):

@@ -89,6 +89,23 @@ def test_single_tokens(nh, nkv, hd, window, splits):
             check(got[b], qkv[b, : nh * hd].reshape(nh, hd), keys[b], values[b], n - 1, hd ** -0.5, window, nh // nkv)
 
 
+@pytest.mark.parametrize("window", [0, 100])
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 64), (3, 1, 128), (4, 4, 20)])
+@pytest.mark.parametrize("pages", [1, 2, 3, 4, 5, 8, 9, 10, 11, 12, 13])
+def test_last_rounds_in_halves_and_quarters(nh, nkv, hd, pages, window):
+    """Rounds of the eight wavefronts with whole pages, and a last one in halves or quarters of pages, the last key in each of them."""
+    from burn_lm_amd.csrc import ops
+    lens = [pages * PAGE - less for less in (63, 48, 33, 32, 17, 1, 0)]
+    table, keys, values, kc, vc = case(lens, nkv, hd, pages)
+    q = torch.randn(len(lens), nh * hd, generator=torch.Generator().manual_seed(6))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    out = torch.full((len(lens), nh * hd), 7.0, device="cuda")
+    ops.attn_decode_f32(q.cuda(), nh * hd, out, i32([n - 1 for n in lens]), i32(range(len(lens))), table.cuda(), kc.cuda(), vc.cuda(), PAGE, nh, nkv, hd,
+                        hd ** -0.5, window, 1)
+    for b, n in enumerate(lens):
+        check(out[b].cpu().reshape(nh, hd), q[b].reshape(nh, hd), keys[b], values[b], n - 1, hd ** -0.5, window, nh // nkv)
+
+
 @pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
 def test_values_that_are_no_numbers_stay_with_those_that_see_them(bad):
     """A token whose value (or key) is infinite or no number: earlier queries and queries whose window has passed it agree with
