@@ -16,9 +16,6 @@ typedef __attribute__((ext_vector_type(4))) unsigned int gd_u32x4;
 #define GD_BK 64
 #define GD_GROUP 8        // row tiles that are walked together: the 32 tiles of a die at a time are 8 of rows by 4 of columns
 
-__device__ __forceinline__ float gd_silu(float x) {
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
-}
 #define GD_FENCE() __builtin_amdgcn_sched_barrier(0)
 #define GD_BARRIER()                             \
   do {                                           \

@@ -17,6 +17,9 @@
 // with K = 3,072 and 9,681 rows 824 us, now 665 (1.46 PFLOP/s).  Walking 4 or 16 row tiles together instead of 8: equal; 16: 6 % behind.
 #include "gemm_duo.h"
 
+__device__ __forceinline__ float gd_silu(float x) {
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
+}
 // the tanh form of GELU, z/2 (1 + tanh(a)) with a = sqrt(2/pi) (z + 0.044715 z^3): (1 + tanh(a)) / 2 = sigmoid(2a)
 __device__ __forceinline__ float gd_gelu(float x) {
   const float a = 0.7978845608028654f * (x + 0.044715f * x * x * x);

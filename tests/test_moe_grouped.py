@@ -160,3 +160,23 @@ def test_tiles_of_256(monkeypatch, T, E, top, f, D, units, kind):
     from burn_lm_amd.csrc import ops
     monkeypatch.setattr(ops, "compute_units", lambda index: units)
     test_kernels(T, E, top, f, D, kind)
+
+
+@pytest.mark.parametrize("T", [8000, 400])
+def test_gating_is_float32(T):
+    """Two million gates of -64 to -16 that float32 holds exactly (a b + c d of bfloat16, steps of 2^-18), ups and weights of one, an
+    identity behind them: in the tiles of many rows and in those of few, an activation is the bfloat16 next to a float32 silu, whose
+    exponential, sum and division are off by at most 2^-22 of it together (2^-23, 2^-24 and 2^-24); twice that either way."""
+    from burn_lm_amd.csrc import ops
+    g = torch.Generator().manual_seed(1)
+    D, wrong = 256, 0
+    steps = lambda n, at, step: at + torch.randint(0, 128, (n,), generator=g) * step
+    for _ in range(8000 // T):
+        x, gu = torch.zeros(T, D), torch.zeros(2 * D, D)
+        x[:, 0], x[:, 1], x[:, 2] = steps(T, -32, 2.0 ** -3), steps(T, 2.0 ** -4, 2.0 ** -11), 1.0
+        gu[:D, 0], gu[:D, 1], gu[D:, 2] = steps(D, 1, 2.0 ** -7), steps(D, 1, 2.0 ** -7), 1.0
+        y = ops.moe_grouped(x.bfloat16().cuda(), gu.bfloat16().cuda(), torch.eye(D).bfloat16().cuda(), torch.ones(T, 2).cuda(), 1, 1)[0].cpu()
+        want = torch.nn.functional.silu(x.double() @ gu[:D].double().T)
+        a, b = ((want * (1 + e * 2.0 ** -21)).bfloat16().float() for e in (-1, 1))
+        wrong += int(((y < torch.minimum(a, b)) | (y > torch.maximum(a, b))).sum())
+    assert wrong == 0
