@@ -187,10 +187,12 @@ class Mixer(Part):
 
     def take_beside(self, weight):
         """Whether w_in now holds the other weight's rows behind its own.  One product of more columns in place of two: a launch
-        less, and fuller rounds of tiles (2,166 rows, width 2048: 5,120 + 2,048 columns 47 + 31 us, as one 61)."""
+        less, and fuller rounds of tiles (2,166 rows, width 2048: 5,120 + 2,048 columns 47 + 31 us, as one 61).  Rows of both in
+        multiples of eight: the joint rows' stride is what the kernels behind the product read their own columns with, 16 bytes at a
+        time."""
         own = getattr(self, "w_in", None)
         if own is None or not hasattr(type(self), "forward_beside") or own.dtype != weight.dtype or own.shape[1] != weight.shape[1] \
-                or own.shape[0] % 8 or own.gated or weight.gated:
+                or own.shape[0] % 8 or weight.shape[0] % 8 or own.gated or weight.gated:
             return False
         self.beside_at = own.shape[0]
         self.w_in = self.rt.weight(torch.cat([own.w, weight.w], dim=0))

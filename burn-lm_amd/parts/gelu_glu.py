@@ -30,7 +30,7 @@ class GeluGLU(FeedForward):
     def take_beside(self, weight):
         """Whether another product of the same rows ([tokens, n] of its own) now runs beside gate and up: forward_beside."""
         own = self.w_gate_up
-        if own.dtype != weight.dtype or own.shape[1] != weight.shape[1] or weight.gated:
+        if own.dtype != weight.dtype or own.shape[1] != weight.shape[1] or weight.gated or weight.shape[0] % 8:
             return False
         self.stacked = torch.cat([own.w, weight.w], dim=0)        # each of the two is a stretch of it
         self.w_gate_up = self.rt.weight(self.stacked[:own.shape[0]], gated=True)
