@@ -169,6 +169,17 @@ class Norm(Part):
         return None
 
 
+def forward_goes_beside(part):
+    """Whether a part's forward_beside is its class's own word on what forward does: a subclass that brings another forward, and
+    nothing beside it, is called by that."""
+    for c in type(part).__mro__:
+        if "forward_beside" in vars(c):
+            return True
+        if "forward" in vars(c):
+            return False
+    return False
+
+
 class Mixer(Part):
     def cache_need(self):
         return None
@@ -186,17 +197,17 @@ class Mixer(Part):
     beside_at = None      # the column at which the other product's results start
 
     def take_beside(self, weight):
-        """Whether w_in now holds the other weight's rows behind its own.  One product of more columns in place of two: a launch
+        """The other weight as a view of w_in, which now holds its rows behind its own, or None.  One product of more columns in place of two: a launch
         less, and fuller rounds of tiles (2,166 rows, width 2048: 5,120 + 2,048 columns 47 + 31 us, as one 61).  Rows of both in
         multiples of eight: the joint rows' stride is what the kernels behind the product read their own columns with, 16 bytes at a
         time."""
         own = getattr(self, "w_in", None)
-        if own is None or not hasattr(type(self), "forward_beside") or own.dtype != weight.dtype or own.shape[1] != weight.shape[1] \
+        if own is None or not forward_goes_beside(self) or own.dtype != weight.dtype or own.shape[1] != weight.shape[1] \
                 or own.shape[0] % 8 or weight.shape[0] % 8 or own.gated or weight.gated:
-            return False
+            return None
         self.beside_at = own.shape[0]
         self.w_in = self.rt.weight(torch.cat([own.w, weight.w], dim=0))
-        return True
+        return self.rt.weight(self.w_in.w[self.beside_at:])
 
     def forward_terms(self, x, step, view):
         """The result as a list of Term whose sum it is; a mixer made of several may hand them on one by one."""

@@ -31,12 +31,24 @@ class ResidualGate(Part):
         self.mult = float(self.params.get("mult", 1.0))
         self.weights = {r: rt.weight(tensors[self.names[r]]) for r in self._roles()}
         self.biases = {r: tensors[self.names[r + "_bias"]].float().contiguous() for r in self._roles()}
+        self.beside = set()       # the sublayers whose own weights hold their gate's: weights has a view of them
+
+    def run_beside(self, role, sublayer):
+        """The sublayer's first product takes the gate's where it can."""
+        if role in self.weights and type(self).gated is ResidualGate.gated and hasattr(sublayer, "take_beside"):
+            taken = sublayer.take_beside(self.weights[role])
+            if taken is not None:
+                self.weights[role] = taken
+                self.beside.add(role)
+
+    def _own(self):
+        return [w.w for r, w in self.weights.items() if r not in self.beside]
 
     def step_bytes(self, rows):
-        return sum(w.w.numel() * w.w.element_size() for w in self.weights.values()) + sum(4 * b.numel() for b in self.biases.values())
+        return sum(w.numel() * w.element_size() for w in self._own()) + sum(4 * b.numel() for b in self.biases.values())
 
     def step_flops(self, rows):
-        return 2 * rows * sum(w.w.numel() for w in self.weights.values())
+        return 2 * rows * sum(w.numel() for w in self._own())
 
     def gated(self, role, x, y, z=None):
         """The sublayer's result y (of the rows x it read) with its gate (z: its product where it is formed already), for the next
@@ -44,45 +56,37 @@ class ResidualGate(Part):
         return Gated(y, self.rt.linear(x, self.weights[role]) if z is None else z, self.biases[role], self.mult)
 
 
-class _GatedMixer(Block):
-    """The mixer's half: where the mixer can, its gate's projection is part of its own first product."""
+class _Gated(Block):
+    """Where a sublayer can, its gate's projection is part of its own first product, or runs beside it."""
 
     def bound(self):
-        if hasattr(self.mixer, "take_beside") and self.mixer.take_beside(self.gate.weights["mixer"]):
-            del self.gate.weights["mixer"]
+        for role in ("mixer", "feed_forward"):
+            if role in self.roles and hasattr(self.gate, "run_beside"):
+                self.gate.run_beside(role, self._parts[role])
 
-    def mixed(self, x, step, view):
-        if "mixer" in self.gate.weights:
-            return self.gate.gated("mixer", x, self.mixer.forward(x, step, view))
-        y, z = self.mixer.forward_beside(x, step, view)
-        return self.gate.gated("mixer", x, y, z)
+    def run(self, role, x, *step):
+        part = self._parts[role]
+        if role in getattr(self.gate, "beside", ()):
+            y, z = part.forward_beside(x, *step)
+            return self.gate.gated(role, x, y, z)
+        return self.gate.gated(role, x, part.forward(x, *step))
 
 
-class GatedPreNormBlock(_GatedMixer):
-    """Where the feed-forward can, its gate's projection runs beside its own first product as well."""
-
+class GatedPreNormBlock(_Gated):
     roles = {"mixer_norm": "norm", "mixer": "mixer", "ffn_norm": "norm", "feed_forward": "feed_forward",
              "gate": "connection"}
 
     def forward(self, h, delta, step, view):
         x = self.mixer_norm.add_norm(h, delta)
-        a = self.mixed(x, step, view)
+        a = self.run("mixer", x, step, view)
         x = self.ffn_norm.add_norm(h, a)
-        if "feed_forward" in self.gate.weights:
-            return self.gate.gated("feed_forward", x, self.feed_forward.forward(x, step))
-        y, z = self.feed_forward.forward_beside(x, step)
-        return self.gate.gated("feed_forward", x, y, z)
-
-    def bound(self):
-        super().bound()
-        if hasattr(self.feed_forward, "take_beside") and self.feed_forward.take_beside(self.gate.weights["feed_forward"]):
-            del self.gate.weights["feed_forward"]
+        return self.run("feed_forward", x, step)
 
 
-class GatedPreNormMixerBlock(_GatedMixer):
+class GatedPreNormMixerBlock(_Gated):
     """The same without a feed-forward."""
     roles = {"mixer_norm": "norm", "mixer": "mixer", "gate": "connection"}
 
     def forward(self, h, delta, step, view):
         x = self.mixer_norm.add_norm(h, delta)
-        return self.mixed(x, step, view)
+        return self.run("mixer", x, step, view)

@@ -6,7 +6,7 @@ from __future__ import annotations
 
 import torch
 
-from .base import FeedForward, TensorSpec
+from .base import FeedForward, TensorSpec, forward_goes_beside
 
 
 class GeluGLU(FeedForward):
@@ -28,14 +28,14 @@ class GeluGLU(FeedForward):
         self.inner = self.params["inner"]
 
     def take_beside(self, weight):
-        """Whether another product of the same rows ([tokens, n] of its own) now runs beside gate and up: forward_beside."""
+        """The other weight as a view of what now holds its rows behind gate's and up's (forward_beside), or None."""
         own = self.w_gate_up
-        if own.dtype != weight.dtype or own.shape[1] != weight.shape[1] or weight.gated or weight.shape[0] % 8:
-            return False
+        if not forward_goes_beside(self) or own.dtype != weight.dtype or own.shape[1] != weight.shape[1] or weight.gated or weight.shape[0] % 8:
+            return None
         self.stacked = torch.cat([own.w, weight.w], dim=0)        # each of the two is a stretch of it
         self.w_gate_up = self.rt.weight(self.stacked[:own.shape[0]], gated=True)
         self.w_beside = self.rt.weight(self.stacked[own.shape[0]:])
-        return True
+        return self.w_beside
 
     def _weights(self):
         return [w for w in (self.w_gate_up, self.w_down, self.w_beside) if w is not None]

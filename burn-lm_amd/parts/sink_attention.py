@@ -194,7 +194,7 @@ class SinkAttention(Mixer):
         return (out.add_(self.output_bias.to(out.dtype)) if self.output_bias is not None else out), qkv[:, self.beside_at:]
 
     def take_beside(self, weight):
-        return not self.qk_norm and super().take_beside(weight)
+        return None if self.qk_norm else super().take_beside(weight)
 
     def forward_unbiased(self, x, step, view):
         """(result without the output projection's bias, possibly as partial planes; that bias in float32): for a
