@@ -603,18 +603,29 @@ class Runtime:
             return K > 4096 or -(-inner // 32) > 2 * self.compute_units
         return K > 4096 and -(-inner // 32) > self.compute_units
 
+    def duo_beside(self, M, inner, n):
+        """How many tiles ops.gemm_duo_beside runs as whole ones for a gated product with n plain columns beside it, or None where the
+        two run apart.  The gated tiles have to be worth it by themselves, as in gated_linear (a lone round of halves at a wide K as
+        well: the two apart are a launch and a pass more), and the columns beside them have to fit into what is left of the last
+        round, or into whole tiles where that was of halves (us, together / apart, in a graph; inner size 8192 and a width of columns
+        beside it: width 2048, 384 / 700 / 1,300 / 2,166 rows 33 / 40, 47 / 57, 91 / 102, 132 / 151; width 3072, 384 / 700 / 1,300 /
+        2,166 rows 55 / 69, 71 / 94, 135 / 156, 205 / 231, with 512 columns 384 / 700 / 1,300 rows 53 / 57, 67 / 79, 118 / 131).
+        Halves more behind full rounds are behind: width 2048, 900 / 1,000 / 2,048 rows 69 / 68, 71 / 68, 132 / 128; width 3072
+        112 / 102, 117 / 111, 195 / 191, with 512 columns 1,000 and 2,048 rows 101 / 90 and 176 / 164."""
+        alone, both = (duo_plan(M, inner, self.compute_units, True, b) for b in (0, n))
+        fits = M > 256 and min(alone[2], both[2]) >= DUO_GATED_FILL and both[1] - alone[1] < DUO_HALF - 0.01
+        return both[0] if fits else None
+
     def gated_linear_beside(self, x, w, beside, stacked, activation):
-        """(gated_linear(x, w, activation), linear(x, beside)) of two matrices that lie one behind the other in `stacked`: in one launch
-        where the gated product alone would be ops.gemm_duo's and the columns beside it take no more rounds of tiles than the
-        plain product would by itself (it fills what is left of the last one)."""
-        M, K = x.shape
-        inner, n = w.shape[0] // 2, beside.shape[0]
-        if M > 256 and self.fused_gate_up_measured and stacked.dtype == self.dtype == torch.bfloat16 and stacked.numel() < 1 << 31:
-            alone, both = (duo_plan(M, inner, self.compute_units, True, b) for b in (0, n))
-            if alone[2] >= DUO_GATED_FILL and both[2] >= DUO_GATED_FILL and both[1] - alone[1] <= DUO_HALF:
+        """(gated_linear(x, w, activation), linear(x, beside)) of two matrices that lie one behind the other in `stacked`: in one
+        launch where duo_beside says so."""
+        M, inner, n = x.shape[0], w.shape[0] // 2, beside.shape[0]
+        if self.fused_gate_up_measured and stacked.dtype == self.dtype == torch.bfloat16 and stacked.numel() < 1 << 31:
+            whole = self.duo_beside(M, inner, n)
+            if whole is not None:
                 out, z = (torch.empty(M, m, dtype=self.dtype, device=x.device) for m in (inner, n))
                 if ops.gemm_duo_takes(x, stacked, out, gated=True) and ops.gemm_duo_takes(x, stacked, z):
-                    return ops.gemm_duo_beside(x, stacked, out, z, activation=activation, whole=both[0])
+                    return ops.gemm_duo_beside(x, stacked, out, z, activation=activation, whole=whole)
         return self.gated_linear(x, w, activation=activation), self.linear(x, beside)
 
     def gated_linear(self, x, w, activation="silu"):

@@ -81,3 +81,53 @@ def test_parts_from_outside_keep_their_own_forward():
                 a = b.forward(x, None, None) if block is Block else b.run("mixer", x, None, None)
                 assert torch.equal(a.y, factor * x) and torch.allclose(a.z, x if want is None else x @ want.T, atol=1e-5)
                 assert torch.equal(b.run("feed_forward", x, None).y, 3 * x)
+
+
+def test_columns_beside_gated_ones_fit_into_their_rounds():
+    """256 units: what is left of the last round takes them, or whole tiles in place of its halves; not another round of halves."""
+    from burn_lm_amd.engine.runtime import DUO_GATED_FILL, DUO_HALF, Runtime, duo_plan
+    rt = Runtime.__new__(Runtime)
+    rt.compute_units = 256
+    for M, inner, n, taken in ((384, 8192, 2048, True), (700, 8192, 2048, True), (900, 8192, 2048, False), (1000, 8192, 2048, False), (1300, 8192, 2048, True),
+                               (2048, 8192, 2048, False), (2166, 8192, 2048, True), (384, 8192, 3072, True), (1000, 8192, 512, False), (2048, 8192, 512, False),
+                               (256, 65536, 2048, False)):
+        assert (rt.duo_beside(M, inner, n) is not None) == taken, (M, inner, n)
+    for M in range(257, 6000, 61):
+        for inner, n in ((8192, 2048), (4096, 1024), (14336, 4096), (1000, 8)):
+            whole = rt.duo_beside(M, inner, n)
+            if whole is not None:
+                alone, both = (duo_plan(M, inner, 256, True, b) for b in (0, n))
+                assert whole == both[0] and alone[2] >= DUO_GATED_FILL and alone[1] <= both[1] < alone[1] + DUO_HALF
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,together", [(384, True), (300, False), (512, False), (40, False)])
+def test_feed_forward_with_its_gate_beside(monkeypatch, M, together):
+    """On 8 units: gate, up and the residual's gate in one launch where the rule says so, else apart; either way the products of the
+    stacked weights, rows in their order, rounded to bfloat16 (half a step of 2^-8; gate and up of the library are rounded once more in
+    front of the activation, whose slope is at most 1.13)."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.runtime import Runtime
+    from burn_lm_amd.parts.gelu_glu import GeluGLU
+    rt = Runtime(torch.bfloat16, "cuda:0")
+    rt.compute_units = 8
+    K, inner, n = 256, 512, 256
+    g = torch.Generator().manual_seed(M)
+    matrix = lambda *shape: (torch.randn(*shape, generator=g) * shape[1] ** -0.5).bfloat16().cuda()
+    x, named = torch.randn(M, K, generator=g).bfloat16().cuda(), dict(gate=matrix(inner, K), up=matrix(inner, K), down=matrix(K, inner))
+    guest = matrix(n, K)
+    ffn = GeluGLU(dict(width=K, inner=inner), {r: r for r in named})
+    ffn.bind(named, rt)
+    view = ffn.take_beside(rt.weight(guest))
+    assert torch.equal(view.w, guest) and view.w.data_ptr() == ffn.stacked[2 * inner:].data_ptr()
+    calls, real = [], ops.gemm_duo_beside
+    monkeypatch.setattr(ops, "gemm_duo_beside", lambda *a, **k: (calls.append(k["whole"]), real(*a, **k))[1])
+    gate, up = x.double() @ named["gate"].double().T, x.double() @ named["up"].double().T
+    act, z = rt.gated_linear_beside(x, ffn.w_gate_up, ffn.w_beside, ffn.stacked, "gelu_tanh")
+    assert calls == ([rt.duo_beside(M, inner, n)] if together else [])
+    close = lambda got, want, steps: float(((got.double() - want).abs() / (want.abs() + want.abs().mean())).max()) <= steps * 2.0 ** -8
+    assert close(z, x.double() @ guest.double().T, 1)
+    assert close(act, torch.nn.functional.gelu(gate, approximate="tanh") * up, 1 if together else 4)
+    total = lambda y: y.double().sum(0) if y.dim() == 3 else y.double()
+    (y, again), plain = ffn.forward_beside(x, None), ffn.forward(x, None)
+    assert torch.equal(again, z) and float((total(y) - total(plain)).norm() / total(plain).norm()) <= 2.0 ** -7
