@@ -186,12 +186,12 @@ extern "C" int blm_latent_write(const void* down, int ld_down, const void* q, in
                                 const float* norm_w, float eps, const void* cos_sin, int half_t, int rot, void* qabs,
                                 int qabs_dtype, void* kcache, void* vcache, const int* positions, const int* token_seq, const int* block_table,
                                 int table_width, int page_size, int R, int Dr, int write_kv, int adjacent, int absorbed,
-                                hipStream_t stream) {
+                                int wide, hipStream_t stream) {
   const int q_lanes = absorbed ? R + Dr : Dr, q_at = absorbed ? R : 0;
   BLM_REQUIRE(T > 0 && H > 0 && dn >= 0 && R > 0 && Dr >= 0, "latent_write: bad sizes");
   BLM_REQUIRE(rot % 2 == 0 && rot >= 0 && rot <= Dr && rot / 2 <= half_t, "latent_write: %d turning lanes do not fit %d", rot, Dr);
   BLM_REQUIRE(page_size > 0 && table_width > 0 && ld_down >= R + Dr && ld_q >= H * (dn + Dr), "latent_write: bad geometry");
-  if (T > 64 && dtype == BLM_BF16 && R % 8 == 0 && R <= 512 && Dr % 8 == 0 && dn % 8 == 0 && rot % 8 == 0 && (adjacent || rot % 16 == 0) &&
+  if (wide && dtype == BLM_BF16 && R % 8 == 0 && R <= 512 && Dr % 8 == 0 && dn % 8 == 0 && rot % 8 == 0 && (adjacent || rot % 16 == 0) &&
       half_t % 2 == 0 && ld_down % 8 == 0 && ld_q % 8 == 0 && ((uintptr_t)down % 16) == 0 && ((uintptr_t)q % 16) == 0 && ((uintptr_t)norm_w % 16) == 0 &&
       ((uintptr_t)cos_sin % 16) == 0 && ((uintptr_t)qabs % 16) == 0 && ((uintptr_t)kcache % 16) == 0 && (qabs_dtype == BLM_BF16 || qabs_dtype == BLM_F32)) {
     const int tiles = write_kv ? (T + R8_TOKENS - 1) / R8_TOKENS : 0, parts = R % 32 == 0 ? 4 : 1;

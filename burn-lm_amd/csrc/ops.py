@@ -11,7 +11,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 44
+ABI_VERSION = 45
 _lib = None
 _lock = threading.Lock()
 
@@ -46,10 +46,10 @@ _SIGNATURES = {
                              _c_int, _c_int, _c_int, _c_void_p],
     "blm_qkv_prepare": [_c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int,
                         _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
-                        _c_void_p, _c_int, _c_float, _c_void_p],
+                        _c_void_p, _c_int, _c_float, _c_int, _c_void_p],
     "blm_qkv_norm": [_c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int,
                      _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_float, _c_float, _c_int, _c_int,
-                     _c_void_p, _c_int, _c_void_p],
+                     _c_void_p, _c_int, _c_int, _c_void_p],
     "blm_head_gate": [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_map_difference": [_c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_void_p],
     "blm_moe_grouped": [_c_void_p, _c_int] + [_c_void_p] * 3 + [_c_int] + [_c_void_p] * 4 + [_c_int] * 6 + [_c_void_p],
@@ -96,7 +96,7 @@ _SIGNATURES = {
     "blm_xielu": [_c_void_p, _c_void_p, _c_int, ctypes.c_longlong, _c_float, _c_float, _c_void_p],
     "blm_latent_write": [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_float, _c_void_p,
                          _c_int, _c_int, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int,
-                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_latent_prompt_supported": [_c_int, _c_int, _c_int, _c_int, _c_int],
     "blm_latent_prompt_init": [],
     "blm_latent_prompt": [_c_void_p, _c_int] + [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 5 + [_c_int] * 8 + [_c_float, _c_int, _c_void_p, _c_void_p],
@@ -1175,6 +1175,26 @@ def xielu(z, out, a_pos, a_neg):
 
 # ------------------------------------------------------------------------------------------
 # attention over a shared latent
+# From how many tokens on the kernels between a prompt's projections and its attention go eight lanes a thread and turn values in
+# tiles of 32 tokens through shared memory (csrc/rows8.h), where the tokens come in runs of eight and more of a sequence, and where
+# they do not: a tile of tokens of many sequences writes values two bytes at a time as before, behind a detour.  Us, token by token /
+# these, at 72, 128, 256, 384, 512 and 1,024 tokens in a graph; 16 heads of 128 with 4 key-value heads:
+#   heads    runs of 16 3.8/3.8 4.2/3.9 5.6/4.3 7.1/4.5 8.5/5.0 14.2/6.7; of 1 3.8/5.6 4.3/6.0 5.9/6.8 7.6/7.7 9.5/8.3 16.1/12.3;
+#            two maps of 64, of 1 4.2/5.9 5.2/6.1 7.5/7.2 9.6/7.9 11.9/8.4 21.6/12.7
+#   rows     runs of 16 5.4/4.0 6.0/4.2 6.7/4.6 7.5/4.9 7.6/5.4 12.1/7.2; of 1 5.3/5.6 6.0/6.0 7.5/6.8 8.5/7.8 9.7/8.2 14.0/12.6
+#   turns    runs of 16 7.3/3.7 7.6/3.8 8.3/4.0 9.5/4.1 9.8/4.3 15.7/5.5; of 1 7.4/5.5 7.8/5.9 8.4/6.8 11.4/7.4 13.4/8.5 17.4/11.4
+#   latents  of 512, runs of 16 5.5/7.2 5.8/7.2 6.4/7.5 7.5/7.5 8.0/7.4 11.3/7.9; of 1 5.5/9.0 5.9/9.4 6.7/9.9 8.2/10.5 9.6/11.1
+#            13.6/13.7 (a few blocks form each norm four times); the queries alone count as turns
+WIDE_ROWS_FROM = {"heads": (65, 384), "rows": (65, 128), "turns": (65, 65), "latents": (384, 1024)}
+WIDE_ROWS_RUN = 8
+
+
+def wide_rows(kind, T, step):
+    """Whether a step's T tokens go that way (a recorded shape's: by the bucket's sizes, so that every step of it goes alike)."""
+    tokens, seqs = (getattr(step, "bucket", None) or (T, getattr(step, "n_seqs", 1)))[:2]
+    return tokens >= WIDE_ROWS_FROM[kind][0 if tokens >= WIDE_ROWS_RUN * seqs else 1]
+
+
 def latent_write(down, q, norm_w, eps, cos_sin, rot, qabs, kcache, step, block_table, page_size, H, dn, R, Dr,
                  write_kv=True, vcache=None, adjacent=False):
     """down [T, >= R + Dr]: latent lanes then the shared key lanes; q [T, H * (dn + Dr)].  The latent is RMS-normed
@@ -1210,7 +1230,8 @@ def latent_write(down, q, norm_w, eps, cos_sin, rot, qabs, kcache, step, block_t
     _call("blm_latent_write", down.data_ptr(), ld_down, q.data_ptr(), q.stride(0), _code(q), T, H, dn, norm_w.data_ptr(),
           float(eps), cos_sin.data_ptr(), cos_sin.shape[1], rot, qabs.data_ptr(), _code(qabs), kcache.data_ptr(),
           _ptr(vcache), step.positions.data_ptr(), step.token_seq.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size,
-          R, Dr, 1 if write_kv else 0, 1 if adjacent else 0, 1 if absorbed else 0, _stream())
+          R, Dr, 1 if write_kv else 0, 1 if adjacent else 0, 1 if absorbed else 0,
+          1 if wide_rows("latents" if write_kv else "turns", T, step) else 0, _stream())
 
 
 def rmsnorm_rows(x, w, eps, out):
@@ -1600,7 +1621,7 @@ def qkv_norm(qkv, bias, q_weight, k_weight, eps, step, block_table, kcache, vcac
     _call("blm_qkv_norm", qkv.data_ptr(), _code(qkv), qkv.stride(0), _ptr(bias), step.positions.data_ptr(), step.token_seq.data_ptr(),
           block_table.data_ptr(), block_table.shape[1], kcache.data_ptr(), vcache.data_ptr(), page_size, T, H, G, dk, dv,
           1 if whole_rows else 0, _ptr(q_weight), _ptr(k_weight), float(eps), float(coef), int(every), maps, _ptr(q_out),
-          q_out.stride(0) if q_out is not None else 0, _stream())
+          q_out.stride(0) if q_out is not None else 0, 1 if wide_rows("rows" if whole_rows else "heads", T, step) else 0, _stream())
     return qkv if q_out is None else q_out
 
 
@@ -2072,7 +2093,8 @@ def qkv_prepare(qkv, bias, cos_sin, rot, step, block_table, kcache, vcache, page
           step.positions.data_ptr(), step.token_seq.data_ptr(), _ptr(block_table) if write_kv else 0,
           block_table.shape[1] if write_kv else 0, _ptr(kcache) if write_kv else 0, _ptr(vcache) if write_kv else 0,
           page_size, T, H, G, dk, dv, 1 if write_kv else 0, 1 if adjacent else 0, 1 if values_are_keys else 0, _ptr(q_scale),
-          0 if unit_norm_eps is None else 1, float(unit_norm_eps or 0.0), _stream())
+          0 if unit_norm_eps is None else 1, float(unit_norm_eps or 0.0),
+          1 if wide_rows("turns" if unit_norm_eps is None else "heads", T, step) else 0, _stream())
     return qkv
 
 

@@ -380,11 +380,11 @@ __global__ void __launch_bounds__(512)
   }
 }
 
-// Whether qkv_prompt_kernel takes the call; few tokens stay with the kernels above (8 tokens: 5.4 and 5.2 us, a launch).
-static bool qp_takes(const void* qkv, int dtype, int ld, const float* bias, const void* kcache, int T, int H, int G, int dk, int dv, int kind,
+// Whether qkv_prompt_kernel takes the operands (the caller says whether there are tokens enough for it: `wide`).
+static bool qp_takes(int wide, const void* qkv, int dtype, int ld, const float* bias, const void* kcache, int H, int G, int dk, int dv, int kind,
                      int rot, int adjacent, const void* cos_sin, const QnExtra& ex) {
   const int n = (H + G) * dk;
-  bool ok = T > 64 && dtype == BLM_BF16 && ld % 8 == 0 && dk % 8 == 0 && dv % 8 == 0 && dv <= 512 && ((uintptr_t)qkv % 16) == 0 &&
+  bool ok = wide && dtype == BLM_BF16 && ld % 8 == 0 && dk % 8 == 0 && dv % 8 == 0 && dv <= 512 && ((uintptr_t)qkv % 16) == 0 &&
             ((uintptr_t)bias % 16) == 0 && ((uintptr_t)kcache % 16) == 0 && ((uintptr_t)ex.qw % 16) == 0 && ((uintptr_t)ex.kw % 16) == 0 &&
             ((uintptr_t)ex.q_out % 16) == 0 && (ex.maps == 1 || ex.ld_q % 8 == 0);
   if (kind == 0) ok = ok && dk <= 512 && (dk & (dk - 1)) == 0;
@@ -417,7 +417,7 @@ static int qp_launch(int kind, void* qkv, int ld, const float* bias, const int* 
 extern "C" int blm_qkv_norm(void* qkv, int dtype, int ld, const float* bias, const int* positions, const int* token_seq,
                             const int* block_table, int table_width, void* kcache, void* vcache, int page_size, int T, int H,
                             int G, int dk, int dv, int whole_rows, const float* qw, const float* kw, float norm_eps, float coef,
-                            int every, int maps, void* q_out, int ld_q, hipStream_t stream) {
+                            int every, int maps, void* q_out, int ld_q, int wide, hipStream_t stream) {
   BLM_REQUIRE(T > 0 && H > 0 && G > 0 && dk > 0 && dv > 0, "qkv_norm: bad sizes T=%d H=%d G=%d dk=%d dv=%d", T, H, G, dk, dv);
   BLM_REQUIRE(maps == 1 || (maps == 2 && !whole_rows && H % 2 == 0 && G % 2 == 0 && q_out && ld_q >= 2 * H * dk),
               "qkv_norm: %d maps (1, or 2 with norms per head and a place for the queries)", maps);
@@ -428,7 +428,7 @@ extern "C" int blm_qkv_norm(void* qkv, int dtype, int ld, const float* bias, con
               dk, dv, BLM_WAVE * QU_LANES);
   BLM_REQUIRE(every >= 0, "qkv_norm: queries that grow every %d tokens", every);
   const QnExtra ex{qw, kw, coef, every, maps, ld_q, q_out};
-  if (qp_takes(qkv, dtype, ld, bias, kcache, T, H, G, dk, dv, whole_rows ? 1 : 0, 0, 0, nullptr, ex))
+  if (qp_takes(wide, qkv, dtype, ld, bias, kcache, H, G, dk, dv, whole_rows ? 1 : 0, 0, 0, nullptr, ex))
     return qp_launch(whole_rows ? 1 : 0, qkv, ld, bias, positions, token_seq, block_table, table_width, kcache, vcache, page_size, T, H, G, dk, dv,
                      (H + G) * dk, 1, nullptr, norm_eps, ex, nullptr, 0, 0, stream);
 #define QN_ROWS(TA)                                                                                                       \
@@ -456,7 +456,7 @@ extern "C" int blm_qkv_prepare(void* qkv, int dtype, int ld, const float* bias, 
                                const int* positions, const int* token_seq, const int* block_table, int table_width,
                                void* kcache, void* vcache, int page_size, int T, int H, int G, int dk, int dv, int write_kv,
                                int adjacent, int values_are_keys, const float* q_scale, int unit_norm, float norm_eps,
-                               hipStream_t stream) {
+                               int wide, hipStream_t stream) {
   BLM_REQUIRE(T > 0 && H > 0 && G > 0 && dk > 0 && dv > 0, "qkv_prepare: bad sizes T=%d H=%d G=%d dk=%d dv=%d", T, H, G, dk, dv);
   BLM_REQUIRE(rot >= 0 && rot % 2 == 0 && rot <= dk, "qkv_prepare: %d turning lanes of %d (even, at most the head size)", rot, dk);
   BLM_REQUIRE(!values_are_keys || dv == dk, "qkv_prepare: values that are the keys have the keys' head size, not %d", dv);
@@ -465,7 +465,7 @@ extern "C" int blm_qkv_prepare(void* qkv, int dtype, int ld, const float* bias, 
   BLM_REQUIRE(rot == 0 || cos_sin, "qkv_prepare: the table of angles is missing");
   const QnExtra none{nullptr, nullptr, 0.f, 0, 1, 0, nullptr};
   const int kind = unit_norm ? 0 : 2;
-  if ((!unit_norm || (rot == 0 && write_kv)) && qp_takes(qkv, dtype, ld, bias, kcache, T, H, G, dk, dv, kind, rot, adjacent, cos_sin, none))
+  if ((!unit_norm || (rot == 0 && write_kv)) && qp_takes(wide, qkv, dtype, ld, bias, kcache, H, G, dk, dv, kind, rot, adjacent, cos_sin, none))
     return qp_launch(kind, qkv, ld, bias, positions, token_seq, block_table, table_width, kcache, vcache, page_size, T, H, G, dk, dv,
                      values_are_keys ? H * dk : (H + G) * dk, write_kv, q_scale, norm_eps, none, cos_sin, rot, adjacent, stream);
   const size_t factors = unit_norm ? (size_t)(H + G) * sizeof(float) : 0;

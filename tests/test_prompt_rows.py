@@ -1,13 +1,32 @@
-"""What lies between a prompt's projections and its attention, eight lanes at a time (more than 64 rows), against the same rows in calls
-of few, which go element by element: norms of heads and of rows, rotation in either pairing, latents, and the pages.  Sums of squares
+"""What lies between a prompt's projections and its attention, eight lanes at a time, against the same rows in calls of few, which go
+element by element (the rule that chooses is told which it is, here): norms of heads and of rows, rotation in either pairing, latents, and the pages.  Sums of squares
 are added in another order there, so a normed value may be rounded to the neighbouring bfloat16 (2^-8 of it); all else is the same."""
 from types import SimpleNamespace
 
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
 PS = 64
+
+
+@pytest.fixture(autouse=True)
+def by_length(request, monkeypatch):
+    """Calls of more than 60 rows take the wide kernels where they can, others never."""
+    if "gpu" in request.keywords:
+        from burn_lm_amd.csrc import ops
+        monkeypatch.setattr(ops, "wide_rows", lambda kind, T, step: T > 60)
+
+
+def test_tokens_of_many_sequences_keep_the_kernels_that_are_faster_for_them():
+    """Steps of a token or a few of every sequence go token by token up to where the wide kernels were measured to be ahead; runs of
+    eight and more sooner; a shape that is recorded goes by its bucket."""
+    from burn_lm_amd.csrc import ops
+    step = lambda seqs, bucket=None: SimpleNamespace(n_seqs=seqs, bucket=bucket)
+    for kind, runs, few in (("heads", 65, 384), ("rows", 65, 128), ("turns", 65, 65), ("latents", 384, 1024)):
+        assert ops.wide_rows(kind, runs, step(runs // 8)) and not ops.wide_rows(kind, runs - 1, step(1))
+        for each in (1, 7):
+            assert ops.wide_rows(kind, few, step(-(-few // each))) and not ops.wide_rows(kind, few - 1, step(-(-few // each)))
+        assert ops.wide_rows(kind, 3, step(1, (2048, 4, 4096))) and not ops.wide_rows(kind, 4000, step(1, (64, 64, 4096)))
 
 
 def steps(T, few):
@@ -34,6 +53,7 @@ def table_of(rot, positions):
     return torch.stack((angle.cos(), angle.sin()), -1).float().cuda()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["heads", "rows", "maps"])
 @pytest.mark.parametrize("T,H,G,dk,dv,bias", [(65, 4, 2, 64, 128, True), (130, 6, 2, 8, 24, False), (300, 2, 2, 512, 512, True), (97, 40, 4, 128, 64, True)])
 def test_norms(mode, T, H, G, dk, dv, bias):
@@ -61,6 +81,7 @@ def test_norms(mode, T, H, G, dk, dv, bias):
     assert torch.equal(out[0][2], out[1][2]) and torch.equal(out[0][0][:, H * dk:], rows[:, H * dk:])
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("adjacent", [False, True])
 @pytest.mark.parametrize("T,H,G,dk,dv,rot,store,same", [(65, 4, 2, 128, 64, 64, True, False), (200, 3, 1, 40, 8, 16, True, False),
                                                         (90, 2, 2, 64, 64, 64, True, True), (130, 5, 2, 24, 16, 0, True, False),
@@ -87,10 +108,16 @@ def test_rotation(adjacent, T, H, G, dk, dv, rot, store, same):
     assert torch.equal(out[0][2], out[1][2]) and bool(out[0][2].any()) == store
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("adjacent", [False, True])
-@pytest.mark.parametrize("T,H,dn,dr,R,rot,absorbed,pages", [(65, 4, 128, 64, 512, 64, False, True), (130, 3, 8, 16, 40, 16, True, True),
-                                                            (90, 16, 64, 32, 520, 16, True, False), (70, 2, 128, 64, 960, 64, False, True)])
-def test_latents(adjacent, T, H, dn, dr, R, rot, absorbed, pages):
+@pytest.mark.parametrize("T,H,dn,dr,R,rot,absorbed,pages,store",
+                         [(65, 4, 128, 64, 512, 64, False, True, True), (130, 3, 8, 16, 40, 16, True, True, True),
+                          (90, 16, 64, 32, 480, 16, True, False, True),           # no transposed pages, a quarter of the lanes a block
+                          (97, 2, 16, 32, 504, 32, False, False, True),           # the same, units that end inside a wavefront
+                          (70, 5, 128, 64, 504, 64, True, True, True),
+                          (130, 4, 24, 64, 512, 32, False, True, False),          # another layer's rows: the queries alone
+                          (70, 2, 128, 64, 960, 64, False, True, True)])          # latents beyond the wide kernel: token by token both times
+def test_latents(adjacent, T, H, dn, dr, R, rot, absorbed, pages, store):
     from burn_lm_amd.csrc import ops
     g = torch.Generator().manual_seed(T)
     whole, parts, tables = steps(T, 60)
@@ -104,9 +131,10 @@ def test_latents(adjacent, T, H, dn, dr, R, rot, absorbed, pages):
             vc = torch.zeros(tables.numel(), 1, R, PS, dtype=torch.bfloat16, device="cuda")
             turned = torch.zeros(T, H, R + dr if absorbed else dr, dtype=dtype, device="cuda")
             for a, e, step in pieces:
-                ops.latent_write(down[a:e], q[a:e], w, 1e-5, cs, rot, turned[a:e], kc, step, tables, PS, H, dn, R, dr,
-                                 vcache=vc if pages else None, adjacent=adjacent)
+                ops.latent_write(down[a:e] if store else None, q[a:e], w, 1e-5, cs, rot, turned[a:e], kc, step, tables, PS, H, dn, R, dr,
+                                 write_kv=store, vcache=vc if pages else None, adjacent=adjacent)
             out.append((kc, vc, turned))
         for x, y in zip(*out):
             close(x, y) if dtype == torch.bfloat16 or x.dtype == torch.bfloat16 else torch.testing.assert_close(x, y, rtol=2e-6, atol=2e-6)
-        assert bool(out[0][1].any()) == pages and torch.equal(out[0][0][..., :R].transpose(2, 3)[out[0][1] != 0], out[0][1][out[0][1] != 0])
+        assert bool(out[0][0].any()) == store and bool(out[0][1].any()) == (pages and store) and bool(out[0][2].any())
+        assert torch.equal(out[0][0][..., :R].transpose(2, 3)[out[0][1] != 0], out[0][1][out[0][1] != 0])
