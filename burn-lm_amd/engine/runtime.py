@@ -117,14 +117,13 @@ def f32_plan(M, N, K, compute_units, planes=False, gated=False):
 
 # ops.gemm_duo: what half a tile takes of a whole one's time (K = 2048 / 8192, all blocks at once: 22 of 38 us, 73 of 128), and how
 # full the rounds of tiles must be for it to be the faster one: for a gated product (against the library's and the gating pass), for
-# a plain one whose last round is of whole tiles and for one round of halves (see gated_linear and duo_product).
+# one round of halves of a plain one (see gated_linear and duo_product).
 DUO_HALF = 0.57
 DUO_GATED_FILL = 0.62
 DUO_GATED_LONE_FILL = 0.9
-DUO_WHOLE_FILL = 0.93
 DUO_HALVES_FILL = 0.74
 DUO_QKV_FILL = 0.6
-DUO_WHOLE_K = 3072
+DUO_HALVES_K = 8192
 DUO_PLANES_K = 4096
 
 
@@ -572,25 +571,24 @@ class Runtime:
         return self.fused_gate_up_measured and M > 256 and K <= RING_QKV_K and duo_plan(M, N, self.compute_units)[2] >= DUO_QKV_FILL
 
     def duo_product(self, M, N, K):
-        """Whether a plain bfloat16 product of many rows goes to ops.gemm_duo and not to the library (us, duo / library):
-        * one round of halves, at least DUO_HALVES_FILL of the units busy: [3072, 2048] 2,048 and 2,560 rows 26.9 / 26.8 and
-          29.3 / 31.0; [2048, 8192] 3,300 and 4,096 rows 87 / 99 and 99 / 107; [5120, 3072] 1,300 and 1,536 rows 38 / 41 and
-          39 / 42 (less full: [2048, 8192] 2,560 rows 83 / 75);
-        * whole rounds and a last one of halves: [5120, 3072] 3,300, 4,096, 6,500 and 7,700 rows 99 / 110, 103 / 112, 149 / 200 and
-          174 / 277; [3072, 3072] 6,500 and 7,700 rows 103 / 101 and 109 / 117; [3072, 8192] 247 / 251 and 267 / 288; [2048, 8192]
-          9,681 rows 249 / 262;
-        * whole rounds, the last nearly full, K up to DUO_WHOLE_K: [5120, 3072] 9,681 rows 207 / 323, 9,200 rows 199 / 196;
-          [6144, 2048] 7,700 and 8,192 rows 142 / 139 and 143 / 141 (beyond that K 3-7 % behind: [6144, 4096] 8,192 rows 278 / 260;
-          and with a last round less full as much: [3072, 3072] 9,681 rows 138 / 131)."""
+        """Whether a plain bfloat16 product of many rows goes to ops.gemm_duo and not to the library (us, duo / library, in turn):
+        * one round of halves, at least DUO_HALVES_FILL of the units busy, K up to DUO_HALVES_K: [2048, 2048] 3,589 and 4,062 rows 31.1 /
+          33.6 and 30.6 / 32.9; [5120, 2048] 1,482 and 1,535 rows 28.8 / 31.2 and 27.9 / 30.1; [3072, 3072] 2,387 and 2,661 rows 39.0 /
+          42.8 and 39.9 / 42.4; [5120, 3072] 1,400 and 1,488 rows 50.0 / 51.5 and 47.2 / 46.6; [2048, 8192] 3,476 and 4,049 rows 99.9 /
+          106.4 and 103.6 / 106.6 (longer K goes either way: [4096, 14336] 1,738 / 1,856 / 1,917 rows 199 / 217, 201 / 196, 208 / 194);
+        * whole rounds and a last one of halves, where the library's times jump with the rows: [2048, 2048] 9,078 and 9,510 rows 70 / 66
+          and 70 / 79; [5120, 2048] 3,750 / 7,100 / 8,017 rows 70 / 80, 115 / 114, 121 / 149; [3072, 3072] 5,931 and 8,189 rows 98 / 104
+          and 106 / 115; [6144, 4096] 2,735 / 4,077 / 5,888 rows 128 / 207, 141 / 153, 216 / 211; [3072, 8192] 5,595 and 7,919 rows
+          239 / 232 and 262 / 277; [4096, 14336] 4,983 and 5,448 rows 463 / 426 and 454 / 841; 0.90 of its time over 84 sizes.
+        Whole rounds alone, full as they may be, are the library's: [2048, 2048] 8,100 rows 50.8 / 47.5, [3072, 2048] 5,217 rows 48.9 /
+        47.1, [6144, 2048] 5,345 and 7,999 rows 97.6 / 93.2 and 147.7 / 138.7, [3072, 3072] 5,326 rows 69.6 / 66.5."""
         if M <= MFMA_SKINNY_MAX_ROWS:
             return False
         whole, rounds, fill = duo_plan(M, N, self.compute_units)
         if rounds <= DUO_HALF:
-            return fill >= DUO_HALVES_FILL
+            return fill >= DUO_HALVES_FILL and K <= DUO_HALVES_K
         tiles = ops.gemm_duo_tiles(M, N)[0]
-        if whole < tiles and tiles >= self.compute_units:
-            return True
-        return fill >= DUO_WHOLE_FILL and K <= DUO_WHOLE_K
+        return whole < tiles and tiles >= self.compute_units
 
     def _gated_by_library(self, M, K, inner):
         """17 to 64 rows of a gated product that are better left to the library's product and the gating kernel:

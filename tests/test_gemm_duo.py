@@ -19,6 +19,23 @@ def test_plan_covers_every_tile():
                 assert rounds <= -(-(tiles + tail) // 256) + 1e-9
 
 
+def runtime():
+    """A runtime's rules, for 256 units, on the CPU."""
+    from burn_lm_amd.engine.runtime import Runtime
+    rt = Runtime.__new__(Runtime)
+    rt.compute_units, rt.fused_gate_up_measured = 256, True
+    return rt
+
+
+def test_plain_products_that_the_library_is_faster_with_stay_there():
+    rt = runtime()
+    for M, N, K, ours in ((2048, 2048, 2048, False), (3589, 2048, 2048, True), (1482, 5120, 2048, True), (2387, 3072, 3072, True), (4049, 2048, 8192, True),
+                          (1856, 4096, 14336, False), (9510, 2048, 2048, True), (2735, 6144, 4096, True), (7919, 3072, 8192, True),      # one round of halves; mixed
+                          (7632, 2048, 2048, False), (8183, 2048, 2048, False), (5217, 3072, 2048, False), (7999, 6144, 2048, False),    # whole rounds
+                          (5326, 3072, 3072, False), (5135, 3072, 3072, False), (60, 65536, 2048, False)):
+        assert rt.duo_product(M, N, K) == ours, (M, N, K)
+
+
 def operands(M, N, K, gated, seed):
     g = torch.Generator().manual_seed(seed)
     a = torch.randn(M, K + 16, generator=g).bfloat16().cuda()[:, 8:K + 8]          # rows of a wider buffer
