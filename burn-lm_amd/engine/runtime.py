@@ -117,14 +117,15 @@ def f32_plan(M, N, K, compute_units, planes=False, gated=False):
 
 # ops.gemm_duo: what half a tile takes of a whole one's time (K = 2048 / 8192, all blocks at once: 22 of 38 us, 73 of 128), and how
 # full the rounds of tiles must be for it to be the faster one: for a gated product (against the library's and the gating pass), for
-# one round of halves of a plain one (see gated_linear and duo_product).
+# one round of halves of a plain one or of its planes (see gated_linear, duo_product and duo_planes).
 DUO_HALF = 0.57
 DUO_GATED_FILL = 0.62
 DUO_GATED_LONE_FILL = 0.9
 DUO_HALVES_FILL = 0.74
 DUO_QKV_FILL = 0.6
 DUO_HALVES_K = 8192
-DUO_PLANES_K = 4096
+DUO_PLANES_FILL = 0.78
+DUO_PLANES_K = 6144
 
 
 @functools.lru_cache(maxsize=4096)
@@ -479,16 +480,10 @@ class Runtime:
             groups, tile = self.mid_planes_plan(M, N, K)
             if groups:
                 return ops.gemm_mfma(x, w, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), tile=tile)
-        if planes and M > MID_PLANES_MAX_ROWS and plain_bf16 and self.fused_gate_up_measured and K >= DUO_PLANES_K:
-            # the down projection of long prompts: halves of tiles over two groups of K where these nearly fill one round (2,048
-            # rows, width 2048, K = 8192, within a prompt: 68 us and 2.6 more in the norm that adds the planes, the library's 79.6;
-            # with half the units idle or a second round behind: 1,000 rows 47 / 46 and 2,166 rows 98 / 73)
-            tiles, tail = ops.gemm_duo_tiles(M, N)
-            if DUO_HALVES_FILL * self.compute_units <= 2 * (2 * tiles + tail) <= self.compute_units:
-                out = torch.empty(2, M, N, dtype=torch.float32, device=x.device)
-                if ops.gemm_duo_takes(x, w, out):
-                    return ops.gemm_duo(x, w, out, whole=0)
-                out = None
+        if planes and plain_bf16 and self.duo_planes(M, N, K):
+            planes_out = torch.empty(2, M, N, dtype=torch.float32, device=x.device)
+            if ops.gemm_duo_takes(x, w, planes_out):
+                return ops.gemm_duo(x, w, planes_out, whole=0)
         if (planes and self.rows_ring and 16 < M <= MFMA_SKINNY_MAX_ROWS and plain_bf16
                 and (M > 32 or K <= 4096 or -(-N // 32) * 8 <= 3 * self.compute_units)):
             # 17 to 64 rows as partial planes (measured against the packed skinny kernel at the 1B, 3B and 8B
@@ -569,6 +564,21 @@ class Runtime:
         the library's product (long ones: gemm_duo's) and that kernel: 2,048 rows of 3,072, K = 2,048 39.8 / 42.1; 9,681 of 5,120,
         K = 3,072 252.6 / 279.5; less full rounds are behind (600 rows of the latter 40 / 33, 1,000 and 1,300 of the former 31 / 27, 31 / 29)."""
         return self.fused_gate_up_measured and M > 256 and K <= RING_QKV_K and duo_plan(M, N, self.compute_units)[2] >= DUO_QKV_FILL
+
+    def duo_planes(self, M, N, K):
+        """Whether a product of long prompts that may come as planes (the down projection) runs as halves of ops.gemm_duo's tiles over two
+        groups of K: where these are at least DUO_PLANES_FILL of one round, and not more.  With the norm that adds the planes, us, this /
+        the library, in turn: width 2048, K = 8192, 1,639 / 1,686 / 1,870 / 1,951 / 2,048 rows 69.5 / 72.5, 64.8 / 73.6, 71.1 / 75.5,
+        70.7 / 76.5, 76.3 / 75.8 (the library's 128x128 tiles are one full round there; within prompts of the 1B shape 69.3 / 68.4);
+        K = 6144 1,638 / 1,750 / 2,048 rows 49.7 / 54.4, 58.7 / 61.3, 64.7 / 63.7; width 3072, K = 8192, 1,045 and 1,280 rows 64.1 / 74.5
+        and 71.5 / 77.1; width 4096, K = 14336, 788 and 1,024 rows 111 / 126 and 124 / 136.  With 192 blocks behind: width 2048, K = 8192,
+        1,443 and 1,532 rows 64.6 / 59.6 and 68.5 / 60.7; width 4096, K = 14336, 768 rows 117 / 111; and a shorter K gains nothing:
+        width 2048, K = 4096, 1,716 and 2,048 rows 39.5 / 39.7 and 42.8 / 41.5, K = 2048 (in a graph) 1,600 and 2,048 rows 29.6 / 27.4 and
+        36.3 / 29.9."""
+        if not self.fused_gate_up_measured or M <= MID_PLANES_MAX_ROWS or K < DUO_PLANES_K:
+            return False
+        tiles, tail = ops.gemm_duo_tiles(M, N)
+        return DUO_PLANES_FILL * self.compute_units <= 2 * (2 * tiles + tail) <= self.compute_units
 
     def duo_product(self, M, N, K):
         """Whether a plain bfloat16 product of many rows goes to ops.gemm_duo and not to the library (us, duo / library, in turn):

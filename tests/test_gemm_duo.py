@@ -36,6 +36,14 @@ def test_plain_products_that_the_library_is_faster_with_stay_there():
         assert rt.duo_product(M, N, K) == ours, (M, N, K)
 
 
+def test_planes_that_the_library_is_faster_without():
+    rt = runtime()
+    for M, N, K, ours in ((2048, 2048, 8192, True), (1639, 2048, 8192, True), (1045, 3072, 8192, True), (1024, 4096, 14336, True), (1638, 2048, 6144, True),
+                          (1532, 2048, 8192, False), (768, 4096, 14336, False), (2166, 2048, 8192, False), (2048, 2048, 4096, False), (2048, 2048, 2048, False),
+                          (512, 8192, 8192, False)):
+        assert rt.duo_planes(M, N, K) == ours, (M, N, K)
+
+
 def operands(M, N, K, gated, seed):
     g = torch.Generator().manual_seed(seed)
     a = torch.randn(M, K + 16, generator=g).bfloat16().cuda()[:, 8:K + 8]          # rows of a wider buffer
@@ -101,25 +109,31 @@ def test_refuses_what_it_cannot_do():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(3300, 2048, 512), (2048, 2048, 4096), (1000, 8192, 256)])
-def test_products_of_long_prompts_take_it(monkeypatch, M, N, K):
-    """The runtime's products reach it where its plan says so, and give what the plain product gives."""
+@pytest.mark.parametrize("M,N,K,plain,planes,gated", [(3600, 2048, 512, 0, None, 0), (3300, 2048, 512, None, None, 0), (2048, 2048, 6144, None, 0, None),
+                                                      (1000, 8192, 256, 0, None, 0), (4300, 4096, 256, 256, None, 256)])
+def test_products_of_long_prompts_take_it(monkeypatch, M, N, K, plain, planes, gated):
+    """Each of the runtime's products reaches it where its plan says so, with as many whole tiles, and where not gives the same; all are
+    what the plain product is."""
     from burn_lm_amd.csrc import ops
     from burn_lm_amd.engine.runtime import Runtime
     rt = Runtime(torch.bfloat16, "cuda:0")
     a, w = operands(M, N, K, False, 5)
     calls, real = [], ops.gemm_duo
-    monkeypatch.setattr(ops, "gemm_duo", lambda *x, **k: (calls.append(1), real(*x, **k))[1])
+    monkeypatch.setattr(ops, "gemm_duo", lambda *x, **k: (calls.append(k["whole"]), real(*x, **k))[1])
     want = a.double() @ w.double().T
-    for planes in (False, True):
-        got = rt.linear(a, rt.weight(w), partials=planes)
+    for partials, whole in ((False, plain), (True, planes if planes is not None else plain)):
+        del calls[:]
+        got = rt.linear(a, rt.weight(w), partials=partials)
+        assert calls == ([] if whole is None else [whole]) and (got.dim() == 3) == (partials and planes is not None)
         got = got.double().sum(0) if got.dim() == 3 else got.double()
         assert float(((got - want).abs() / (want.abs() + want.abs().mean())).max()) <= 2.0 ** -8
     inner = N // 2
     gate, up = want.chunk(2, 1)
     want = torch.nn.functional.silu(gate) * up
+    del calls[:]
     got = rt.gated_linear(a, rt.weight(w, gated=True))
-    assert calls and float(((got.double() - want).abs() / (want.abs() + want.abs().mean())).max()) <= 2.0 ** -7 and got.shape == (M, inner)
+    assert calls == ([] if gated is None else [gated])
+    assert float(((got.double() - want).abs() / (want.abs() + want.abs().mean())).max()) <= 2.0 ** -7 and got.shape == (M, inner)
 
 
 @pytest.mark.gpu
