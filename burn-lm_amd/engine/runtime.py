@@ -122,7 +122,7 @@ DUO_HALF = 0.57
 DUO_GATED_FILL = 0.62
 DUO_GATED_LONE_FILL = 0.9
 DUO_HALVES_FILL = 0.74
-DUO_QKV_FILL = 0.6
+DUO_QKV_FILL = 0.62
 DUO_HALVES_K = 8192
 DUO_PLANES_FILL = 0.78
 DUO_PLANES_K = 6144
@@ -560,9 +560,13 @@ class Runtime:
 
     def duo_qkv(self, M, N, K):
         """Whether a q/k/v projection of more than 256 rows goes to ops.gemm_duo_qkv_rope, which turns queries and keys and fills the
-        pages behind the product instead of a kernel that reads its results and writes them back.  Within prompts, us a layer, this /
-        the library's product (long ones: gemm_duo's) and that kernel: 2,048 rows of 3,072, K = 2,048 39.8 / 42.1; 9,681 of 5,120,
-        K = 3,072 252.6 / 279.5; less full rounds are behind (600 rows of the latter 40 / 33, 1,000 and 1,300 of the former 31 / 27, 31 / 29)."""
+        pages behind the product instead of a kernel that reads its results and writes them back.  Us, this / the product of before and
+        that kernel, in graphs: [3072, 2048] 2,048 / 2,500 / 4,000 rows 32.4 / 38.0, 36.0 / 42.4, 52.1 / 58.1; [5120, 3072] 1,218 /
+        2,048 / 3,300 rows 47.9 / 58.4, 71.9 / 73.4, 118 / 129; [6144, 4096] 1,036 / 2,048 / 4,000 rows 57.4 / 65.7, 90.1 / 98.1, 165 /
+        184.  Within prompts: 2,048 rows of the 1B shape 36.8 / 29.2 + 8.0 and a launch, 9,681 rows of the 3B shape 225 / 325 +
+        50.  Less full rounds are equal or behind:
+        [3072, 2048] 3,300 rows (fill 0.60) 54.1 / 50.8, 3,356 (0.615) 53.6 / 51.3, 1,000 (0.32) 28.4 / 27.2; [5120, 3072] 1,150 rows
+        (0.62) 50.8 / 49.2, 600 rows (0.32) 46 / 39."""
         return self.fused_gate_up_measured and M > 256 and K <= RING_QKV_K and duo_plan(M, N, self.compute_units)[2] >= DUO_QKV_FILL
 
     def duo_planes(self, M, N, K):

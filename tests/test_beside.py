@@ -131,3 +131,43 @@ def test_feed_forward_with_its_gate_beside(monkeypatch, M, together):
     total = lambda y: y.double().sum(0) if y.dim() == 3 else y.double()
     (y, again), plain = ffn.forward_beside(x, None), ffn.forward(x, None)
     assert torch.equal(again, z) and float((total(y) - total(plain)).norm() / total(plain).norm()) <= 2.0 ** -7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,together", [(512, True), (449, True), (300, False)])
+@pytest.mark.parametrize("store", [True, False])
+def test_projection_of_a_long_prompt_with_its_rotation(monkeypatch, M, together, store):
+    """On 8 units: an encoding's projection goes through the tiles that turn and store where the rule says so; queries and pages are
+    those of the product, the rotation and the write apart, which round to bfloat16 in front of the rotation as well as behind it."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.runtime import Runtime
+    from burn_lm_amd.parts.base import PositionEncoding
+    from burn_lm_amd.parts.rope import RotaryEncoding
+    rt = Runtime(torch.bfloat16, "cuda:0")
+    rt.compute_units = 8
+    nh, nkv, hd, K = 6, 1, 64, 256
+    g = torch.Generator().manual_seed(M)
+    encoding = RotaryEncoding(dict(head_dim=hd, theta=10000.0, scaling=None, pairing="interleaved"), {})
+    encoding.bind({}, rt)
+    encoding.prepare(1024, rt)
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    w = rt.weight((torch.randn((nh + 2 * nkv) * hd, K, generator=g) * K ** -0.5).bfloat16().cuda())
+    seq = (torch.arange(M) >= M // 3).int()                                 # two sequences, one that starts inside a page
+    positions = torch.where(seq == 0, torch.arange(M) + 37, torch.arange(M) - M // 3).int().cuda()
+    tables = torch.randperm(20, generator=g).int().view(2, 10).cuda()
+    step = SimpleNamespace(positions=positions, token_seq=seq.cuda(), max_position=int(positions.max()), n_tokens=M, n_seqs=2)
+    calls, real, out = [], ops.gemm_duo_qkv_rope, []
+    monkeypatch.setattr(ops, "gemm_duo_qkv_rope", lambda *a, **k: (calls.append(k["whole"]), real(*a, **k))[1])
+    for apart in (False, True):
+        k, v = torch.zeros(20, nkv, 64, hd, dtype=torch.bfloat16, device="cuda"), torch.zeros(20, nkv, hd, 64, dtype=torch.bfloat16, device="cuda")
+        view = SimpleNamespace(k=k, v=v, page_size=64, store=store, block_table=lambda step: tables)
+        run = PositionEncoding.project_encode_store if apart else RotaryEncoding.project_encode_store
+        out.append((run(encoding, x, w, step, view, nh, nkv, hd)[:, :nh * hd], k, v))
+        assert calls == ([rt.duo_tiles(M, 512)] if together else [])
+    # apart, a pair (u, v) is rounded in front of its rotation: 2^-8 (|u c| + |v s|), at most 2^-8 of the pair's length, which turning
+    # keeps; both round their results, 2^-8 each; 2 % for the roundings' own sizes and the sums' order
+    for i, (a, b) in enumerate(zip(*out)):
+        a, b = a.double(), b.double()
+        length = b.unflatten(-1, (-1, 2)).norm(dim=-1).repeat_interleave(2, -1) if i < 2 else 0.0
+        assert bool(((a - b).abs() <= 1.02 * 2.0 ** -8 * (length + 2 * b.abs())).all())
+    assert bool(out[0][1].any()) == store and bool(out[0][2].any()) == store

@@ -44,6 +44,14 @@ def test_planes_that_the_library_is_faster_without():
         assert rt.duo_planes(M, N, K) == ours, (M, N, K)
 
 
+def test_projections_of_less_full_rounds_keep_their_product_and_pass():
+    rt = runtime()
+    for M, N, K, ours in ((2048, 3072, 2048, True), (4000, 3072, 2048, True), (2048, 5120, 3072, True), (1036, 6144, 4096, True), (9681, 5120, 3072, True),
+                          (3300, 3072, 2048, False), (3356, 3072, 2048, False), (1150, 5120, 3072, False), (600, 5120, 3072, False), (256, 65536, 2048, False),
+                          (2048, 10240, 8192, False)):
+        assert rt.duo_qkv(M, N, K) == ours, (M, N, K)
+
+
 def operands(M, N, K, gated, seed):
     g = torch.Generator().manual_seed(seed)
     a = torch.randn(M, K + 16, generator=g).bfloat16().cuda()[:, 8:K + 8]          # rows of a wider buffer
