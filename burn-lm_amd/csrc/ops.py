@@ -806,9 +806,11 @@ def gemm_mfma(a, w, out, gated=False, tile=(128, 128), activation="silu", whole=
     of GELU.  tile: rows x columns of out (of
     gate and up columns together when gated) per block, one of GEMM_TILES; a third number is the depth of
     the ring of K stages (deep rings for products of few tiles, which wait for memory, not for the matrix cores).
-    Tiles of 256x256 are gemm_duo's where it takes the operands (`whole`: see there)."""
+    whole (with tiles of 256x256): that many of them whole and the others as halves, by gemm_duo."""
     _gpu(a, w, out)
-    if tile == (256, 256) and w.dim() == 2 and gemm_duo_takes(a, w, out, gated):
+    if whole is not None:
+        if tile != (256, 256):
+            raise KernelError(f"gemm_mfma: whole tiles and halves are of 256x256, not {tile}")
         return gemm_duo(a, w, out, gated=gated, activation=activation, whole=whole)
     gemm_mfma_init(a.device)
     groups = 1

@@ -17,16 +17,14 @@ Matrix products ``x[M,K] @ w[N,K]^T``:
   width): ops.gemm_rows again, a block for every 64 rows (see mid_rows_ring).
 * bfloat16 weights, 65 rows and more, narrow output and long K (the down projection of short
   prompts): partial planes from the hand-written matrix-core kernel (see mid_k_groups).
-* bfloat16 weights, many rows (prefill): the library product (hipBLASLt through torch), as the
-  reference's engine leaves its matrix products to its tensor library
-  (crates/burn-lm-llama/src/nn/attention/mha.rs:124-126).  The gate/up product of a gated
-  feed-forward runs instead on the hand-written matrix-core kernel that applies the gating in its
-  epilogue (ops.gemm_mfma) where that is faster: for short prompts whose tiles all run at once
-  and for long prompts of narrow models whose tiles come in whole rounds (see gated_linear).  With
-  BURN_LM_AMD_FUSED_GATE_UP=1 it is used for every prompt of 192 rows and more: it never writes the
-  [rows, 2 I] intermediate nor reads it back, but its lower rate eats that gain at wider shapes
-  (measured over whole prefills: -6 to +4 % at the 1B shape, -6 to +2 % at 3B, 2-7 % slower at
-  8B), so beyond the measured cases it is off unless asked for; =0 leaves every product to the library.
+* bfloat16 weights, many rows (prefill): tiles of 256x256 and their halves (ops.gemm_duo) where their rounds are full enough, and
+  with them what stands around a product: the gating of a gated feed-forward, the rotation and the page writes behind q/k/v, a
+  gate's product beside gate and up (duo_product, duo_planes, duo_qkv, duo_beside and gated_linear hold the rules and both
+  sides' times).  The gate/up product of short prompts whose tiles all run at once is ops.gemm_mfma's (gated_linear).
+  Everything else is the library's product (hipBLASLt through torch), as the reference's engine leaves its matrix
+  products to its tensor library (crates/burn-lm-llama/src/nn/attention/mha.rs:124-126).  With
+  BURN_LM_AMD_FUSED_GATE_UP=1 gate and up run on ops.gemm_mfma for every prompt of 192 rows and more that no rule above takes;
+  =0 leaves every product to the library.
 """
 from __future__ import annotations
 
@@ -712,12 +710,10 @@ class Runtime:
             if M > 256 and M * 20 >= m256 * 256 * 17 and self.compute_units * 3 // 4 <= blocks <= self.compute_units:
                 return ops.gemm_mfma(x, plain, torch.empty(M, inner, dtype=self.dtype, device=x.device),
                                      gated=True, tile=(256, 128), activation=activation)
-            # Long prompts of a width that is no multiple of 128: with whole rounds of 256x256 tiles (as many blocks as compute units, or a
-            # multiple) and a narrow model the fused kernel is ahead of the library over the whole
-            # prefill (width 2048: 2-4 % at 1,024 and 2,048 rows, 0.5-0.8 % at 3,072 and 4,096; behind by
-            # 2-6 % with a partial last round, and at width 3072 behind from 1,536 rows on).  Beyond
-            # 4,096 rows the library's large tiles are ahead (whole prefill of 8,192 tokens 19.4 ms
-            # against 20.7, of 16,384 tokens 47.9 against 49.0).
+            # Long prompts of a width that gemm_duo does not take (no multiple of 128): gemm_mfma's tiles of 256x256 where they come in
+            # whole rounds, K up to RING_GROUP_K and 4,096 rows (us against the library's product and the gating pass, in a graph:
+            # width 1088, inner size 8192, 1,024 / 2,048 / 4,096 rows 36.9 / 46.4, 70.4 / 86.6, 137 / 158; width 1600 49.4 / 58.2, 98.7 /
+            # 110, 187 / 201; width 1984 59.1 / 67.3, 120 / 122, 242 / 229; inner size 4096, 2,048 rows 35.9 / 44.5, 48.3 / 54.3, 58.4 / 63.9).
             if K <= RING_GROUP_K and 256 <= M <= 4096 and (-(-M // 256) * -(-inner // 128)) % self.compute_units == 0:
                 return ops.gemm_mfma(x, plain, torch.empty(M, inner, dtype=self.dtype, device=x.device),
                                      gated=True, tile=(256, 256), activation=activation)

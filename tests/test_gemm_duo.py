@@ -110,6 +110,8 @@ def test_refuses_what_it_cannot_do():
     for bad in (dict(whole=99), dict(whole=-1)):
         with pytest.raises(KernelError, match="whole tiles"):
             ops.gemm_duo(a, w, out, **bad)
+    with pytest.raises(KernelError, match="256x256"):
+        ops.gemm_mfma(a, w, out, tile=(256, 128), whole=0)
     with pytest.raises(KernelError, match="not supported"):
         ops.gemm_duo(a[:, :192], w[:, :192], out)
     with pytest.raises(KernelError, match="do not fit"):
@@ -142,6 +144,19 @@ def test_products_of_long_prompts_take_it(monkeypatch, M, N, K, plain, planes, g
     got = rt.gated_linear(a, rt.weight(w, gated=True))
     assert calls == ([] if gated is None else [gated])
     assert float(((got.double() - want).abs() / (want.abs() + want.abs().mean())).max()) <= 2.0 ** -7 and got.shape == (M, inner)
+
+
+@pytest.mark.gpu
+def test_tiles_of_256_without_halves_are_the_other_kernels(monkeypatch):
+    """gemm_mfma runs its own tiles of 256x256 unless it is told how many of them are whole."""
+    from burn_lm_amd.csrc import ops
+    a, w = operands(300, 264, 256, False, 1)
+    want, calls, real = a.double() @ w.double().T, [], ops.gemm_duo
+    monkeypatch.setattr(ops, "gemm_duo", lambda *x, **k: (calls.append(k["whole"]), real(*x, **k))[1])
+    for whole in (None, 0):
+        got = ops.gemm_mfma(a, w, torch.empty(300, 264, dtype=torch.bfloat16, device="cuda"), tile=(256, 256), whole=whole)
+        assert calls == ([] if whole is None else [0])
+        assert float(((got.double() - want).abs() / (want.abs() + want.abs().mean())).max()) <= 2.0 ** -8
 
 
 @pytest.mark.gpu
