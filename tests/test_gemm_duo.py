@@ -5,9 +5,11 @@ import torch
 
 
 def test_plan_covers_every_tile():
-    """Whole tiles and halves together are all tiles; a plan is never longer than whole tiles alone; its fill is a share."""
+    """Whole tiles and halves together are all tiles: the whole ones are all of them or full rounds; a plan is never longer than whole
+    tiles alone; its fill is a share of what its rounds can hold (two halves take 1.14 of a whole tile's time)."""
     from burn_lm_amd.csrc import ops
     from burn_lm_amd.engine.runtime import DUO_HALF, duo_plan
+    mixed = 0
     for gated in (False, True):
         for M in (1, 128, 129, 256, 257, 511, 512, 1000, 2048, 2166, 4097, 9681):
             for N in (8, 256, 264, 2048, 3072, 8192, 14336):
@@ -15,8 +17,14 @@ def test_plan_covers_every_tile():
                 columns = -(-N // (128 if gated else 256))
                 assert tiles * 2 + tail >= -(-M // 128) * columns and tail in (0, columns)
                 whole, rounds, fill = duo_plan(M, N, 256, gated)
-                assert whole in (tiles, tiles - tiles % 256) and 0 < fill <= 1 / (2 * DUO_HALF) + 1e-9 or rounds > DUO_HALF and fill <= 1
+                assert whole in (tiles, tiles - tiles % 256)
+                mixed += 0 < whole < tiles
+                if rounds <= DUO_HALF:
+                    assert whole == 0 and 0 < fill <= 1 / (2 * DUO_HALF) + 1e-9
+                else:
+                    assert 0 < fill <= 1 + 1e-9
                 assert rounds <= -(-(tiles + tail) // 256) + 1e-9
+    assert mixed >= 5
 
 
 def runtime():

@@ -152,12 +152,17 @@ def test_no_more_memory_than_the_stacked_form():
 
 
 @pytest.mark.parametrize("kind", ["all", "one", "missing"])
-@pytest.mark.parametrize("units", [8, 40, 256])
-@pytest.mark.parametrize("T,E,top,f,D", [(257, 3, 2, 256, 256), (700, 5, 2, 384, 640), (1030, 2, 1, 256, 264 * 128 // 88), (300, 64, 4, 256, 256)])
+@pytest.mark.parametrize("T,E,top,f,D,units",
+                         [(257, 3, 2, 256, 256, 4), (257, 3, 2, 256, 256, 5), (700, 5, 2, 384, 640, 8), (700, 5, 2, 384, 640, 32),
+                          (1030, 2, 1, 256, 384, 8), (1030, 2, 1, 256, 384, 18), (300, 64, 4, 256, 256, 8), (300, 64, 4, 256, 256, 40),
+                          (4000, 4, 3, 384, 768, 256), (2100, 16, 4, 256, 1024, 256)])
 def test_tiles_of_256(monkeypatch, T, E, top, f, D, units, kind):
     """The tiles of 256x256: experts with whole tiles, a half behind them, or halves only (the fewer units, the more rounds there are to
-    choose by), with no rows at all, and columns that end within a tile.  The bound as above."""
+    choose by), with no rows at all, and columns that end within a tile.  Each of these takes them for gate and up and for
+    down: as many halves, an expert's last one half full, as the launch asks for.  The bound as above."""
     from burn_lm_amd.csrc import ops
+    about = (T * top + 64 * E) // 128
+    assert about * -(-f // 128) * 5 >= 2 * units and about * -(-D // 256) >= units
     monkeypatch.setattr(ops, "compute_units", lambda index: units)
     test_kernels(T, E, top, f, D, kind)
 
