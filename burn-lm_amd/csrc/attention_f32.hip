@@ -8,7 +8,8 @@
 // instruction takes is free as long as queries and keys agree: a lane takes four neighbours, one 16-byte read for four
 // instructions.
 //   attn_prefill_f32 : a wavefront has sixteen queries of one head, the four of a block share the pages through shared memory
-//   attn_decode_f32  : the sixteen columns are the heads of one group at one token; wavefronts take pages in turn
+//   attn_decode_f32  : the sixteen columns are the heads of one group at one token; wavefronts take pages in turn, the last ones in
+//                      halves or quarters
 #include <type_traits>
 
 #include "common.h"
@@ -223,11 +224,12 @@ __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
 
 // ---------------------------------------------------------------------------------------------------------------------
 // decoding.  A block has one token, one key-value head and up to sixteen heads of its group; its wavefronts take the pages of
-// the block's piece of the key range in turn, fragments straight from the pages (a page is read by one wavefront only, whole
+// the block's piece of the key range in turn, fragments straight from the pages (a whole page is read by one wavefront only, its
 // lines by neighbouring instructions).  The wavefronts' results meet in shared memory; with several pieces per token the blocks
 // leave theirs in device-coherent memory, count themselves in, and the last one adds them up (as attn_paged does).
-// A page takes a wavefront 128 products, 1.7 us at the matrix cores' rate, behind the fetch of 32 KB; where a round of whole pages would
-// leave wavefronts idle it goes in halves or quarters, one to a wavefront.
+// A page takes a wavefront 128 products, 1.7 us at the matrix cores' rate, behind the fetch of 32 KB; where a last round of whole pages
+// would leave half of the wavefronts idle it goes in halves, 32 keys and 128 bytes of each row of values to a wavefront, and where
+// three quarters, in quarters: 16 keys, 64 bytes, so that two wavefronts read a line of values each in part.
 // Measured (us a layer, 32 heads of 64 in 8 groups, 8 sequences of 400 to 640 keys; before: a wavefront per head, the heads of
 // a group each reading the group's keys and values): 43.8 -> 13.3 in three pieces of whole pages; in a graph of its own 11.4, with
 // halves 10.5; 8 sequences of 8 pages in four pieces 10.6 -> 9.3 in halves, 8.7 in quarters; 24 heads of 128 15.9 -> 12.4.

@@ -14,7 +14,8 @@
 // w + 4 share a SIMD and run half a phase apart: a phase is the reads of six fragments of the next ones, a barrier, 16 instructions
 // with the region's loads in the middle, a barrier.  Bytes go straight from global into shared memory; the waits are the kernel's own.
 // Before (gemm_mfma's 256x256 tile: one barrier a stage, all wavefronts in step): 2,048 rows, 8,192 gated, K = 2,048 118 us, now 100;
-// with K = 3,072 and 9,681 rows 824 us, now 665 (1.46 PFLOP/s).  Walking 4 or 16 row tiles together instead of 8: equal; 16: 6 % behind.
+// with K = 3,072 and 9,681 rows 824 us, now 665 (1.46 PFLOP/s).  Walking 4 row tiles together instead of 8: equal;
+// 16: gated 2,048 rows equal, 9,681 rows 663 against 652, 8,192 cubed 780 against 720.
 #include "gemm_duo.h"
 
 __device__ __forceinline__ float gd_silu(float x) {

@@ -10,7 +10,7 @@
 // The 256 x 128 tiles by eight wavefronts share the compute unit's LDS between the direct loads (48 KB a stage), the wavefronts' reads
 // (128 KB) and 1,024 cycles of matrix instructions; a stage takes 0.75 us, and the last round of blocks is a quarter of the time.
 // Measured within a whole prompt, under the profiler (us, 2,048 tokens, 16 experts of 512 at width 2048, 4 chosen; the stacked products
-// and the gating pass / 256 x 128 / 256 x 256): gate/up with gating 122 / 65 / 49, down 77 / 46.5 / 38.4; lists 6.3.
+// and the gating pass / 256 x 128 / 256 x 256): gate/up with gating 122 / 66 / 53, down 77 / 46.5 / 38.2; lists 6.2.
 // Tried for 256 x 128: 128 x 128 tiles, two blocks a unit (stages of 32: 70 and 43), the compiler's own order of reads, loads and
 // products (72 and 44), four wavefronts of 128 x 64 (83 and 54).
 #include "gemm_duo.h"
@@ -409,7 +409,7 @@ extern "C" int blm_moe_grouped(const void* x, int ldx, const void* w_gate_up, co
   // them: gate/up from halves (an expert's last one half full) on two fifths of the units on, down from as many halves as units.
   // Gate/up and down together, 16 experts of 512 at width 2048, 4 chosen, both by the smaller tiles / both by these / as the rule
   // has it, us: 400 tokens 52 / 58 / 52, 512: 55 / 60 / 55, 600: 58 / 58 / 57, 800: 63 / 59 / 59, 1,000: 76 / 69 / 69, 1,500: 72 / 72 / 72,
-  // 2,048: 113 / 90 / 90, 8,000: 330 / 261 / 261.
+  // 2,048: 113 / 90 / 90, 8,000: 330 / 261 / 261 (all with the hardware's exp2 in the gating; expf takes either size of tiles 4 more at 2,048).
   const long long about = ((long long)T * top + (GD_TILE / 4) * E) / (GD_TILE / 2);
   const int duo_gates = (f + GD_TILE / 2 - 1) / (GD_TILE / 2), duo_columns = (D + GD_TILE - 1) / GD_TILE;
   if (D % 128 == 0 && D >= 256 && ((long long)E * f + f) * D * 2 < (1LL << 32) && about * duo_gates * 5 >= units * 2LL) {
