@@ -18,6 +18,10 @@
 // 16: gated 2,048 rows equal, 9,681 rows 663 against 652, 8,192 cubed 780 against 720.
 #include "gemm_duo.h"
 
+// x * sigmoid(x) with the hardware's exponential and reciprocal, as gemm_mfma has it: off by at most 2^-23 (|x| + 2) of itself, an ulp of
+// each and the rounding of x * log2(e) in front of the first, far below the rounding to bfloat16 behind it.  Gate and up are float here;
+// the library's product and the pass behind it round them to bfloat16 first (2,048 rows, K = 3,072, against 64 bits: 1.66e-3, so 3.09e-3;
+// of gates below -4 alone 1.5e-3 and 6.1e-3).
 __device__ __forceinline__ float gd_silu(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
 }
