@@ -5,6 +5,7 @@
 //   gemv_f32 : up to 16 rows (decode).  Streams a packed copy of the weights once, whole lines at a time.
 // Both want K, lda and the rows' addresses in units of 16 bytes; other operands take gemm_tiled.
 #include "common.h"
+#include "row_scale.h"
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
@@ -224,11 +225,14 @@ struct GvRope {
   int table_width, page_size, nh, nkv, hd, store;
 };
 
-template <int KSTEPS, bool WHOLE, bool ROPE>
+// SCALED: the rows come unscaled (row_scale.h), that many of them to a wavefront.
+template <int KSTEPS, bool WHOLE, bool ROPE, int SCALED>
 __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
     gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wp, float* __restrict__ C, int M, int N, int K,
-                    int lda, int ldc, int n_tiles, int k_steps, int gated, int steps_per_group, int tiles_per_block, GvRope rope) {
+                    int lda, int ldc, int n_tiles, int k_steps, int gated, int steps_per_group, int tiles_per_block, GvRope rope, RowScale scale) {
   __shared__ float red[GV_MAX_WAVES * 256];
+  __shared__ float inv[RS_ROWS];
+  RowScaleLoad<SCALED ? SCALED : 1> scale_load;
   __shared__ int pos_of[16], page_of[16];
   int my_pos = 0, my_seq = -1;
   if (ROPE && threadIdx.x < 16) {
@@ -248,6 +252,7 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
   // activations first, then the first tile's weights behind them, all asked for before any is looked at; weights behind the end
   // of the group are some other step's (a step past the matrix is its last), and they and their activations count as zeros
   f32x4 a[KSTEPS];
+  if (SCALED) scale_load.ask(scale, M, wave, n_waves, lane);
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) a[s] = *reinterpret_cast<const f32x4*>(ap + min(kbase + s * 16, K - 4));
   const int tile_begin = blockIdx.x * tiles_per_block, tile_end = min(n_tiles, tile_begin + tiles_per_block);
@@ -262,6 +267,7 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
   weights(tile_begin, 0, w[0]);
   weights(tile_begin, 1, w[1]);
   __builtin_amdgcn_sched_barrier(0);
+  if (SCALED) scale_load.finish(scale, M, wave, n_waves, lane, inv);
   if (ROPE && threadIdx.x < 16) {            // the barrier of the first tile's sum lies between these writes and their readers
     pos_of[threadIdx.x] = my_pos;
     page_of[threadIdx.x] = my_seq < 0 || !rope.store ? -1 : rope.block_table[(size_t)my_seq * rope.table_width + my_pos / rope.page_size];
@@ -311,6 +317,7 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
       if (!gated) {
         for (int x = 0; x + 1 < n_waves; x += 2) s += red[x * 256 + idx] + red[x * 256 + 256 + idx];
         if (n_waves & 1) s += red[(n_waves - 1) * 256 + idx];
+        if (SCALED) s *= inv[min(m, M - 1)];
         const int n = tile * 16 + col;
         if (ROPE) {
           const float other = blm_dpp<BLM_DPP_XOR1>(s);
@@ -334,6 +341,10 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
         if (n_waves & 1) {
           s += red[(n_waves - 1) * 256 + idx];
           u += red[(n_waves - 1) * 256 + idx + 8];
+        }
+        if (SCALED) {
+          s *= inv[min(m, M - 1)];
+          u *= inv[min(m, M - 1)];
         }
         const int n = tile * 8 + col;
         if (m < M && n < N / 2) C[(size_t)m * ldc + n] = silu_times(s, u);
@@ -371,7 +382,7 @@ extern "C" int blm_gemv_f32_geometry(int M, int N, int K, int groups, int* block
 // their 8 up rows, and C is [M, N / 2].  groups > 1: K in that many groups, a plane of M * N for each (ldc = N), which the
 // reader adds up.
 static int gv_run(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int ldc, int gated, int groups, const GvRope* rope,
-                  hipStream_t stream) {
+                  const RowScale* scale, hipStream_t stream) {
   BLM_REQUIRE(M >= 1 && M <= 16 && N > 0 && K > 0 && lda >= K && ldc >= (rope ? rope->nh * rope->hd : gated ? N / 2 : N), "gemv_f32: bad sizes M=%d N=%d K=%d lda=%d ldc=%d", M, N, K, lda, ldc);
   BLM_REQUIRE(K % 4 == 0 && lda % 4 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)Wp % 16) == 0,
               "gemv_f32: rows must start at multiples of 16 bytes and hold a multiple of four elements (K=%d lda=%d)", K, lda);
@@ -383,14 +394,19 @@ static int gv_run(const void* A, const void* Wp, void* C, int M, int N, int K, i
   gemv_f32_geometry(N, K, groups, &ksteps, &waves, &blocks);
   const int per_block = (n_tiles + blocks - 1) / blocks;
   dim3 grid((unsigned)blocks, (unsigned)groups), block(waves * BLM_WAVE);
+#define BLM_GVS(KS, WHOLE, ROPE, SCALED, SCALE)                                                                         \
+  hipLaunchKernelGGL((gemv_f32_kernel<KS, WHOLE, ROPE, SCALED>), grid, block, 0, stream, (const float*)A, (const float*)Wp, (float*)C, M, \
+                     N, K, lda, ldc, n_tiles, k_steps, gated, steps, per_block, rope ? *rope : GvRope{}, SCALE)
+#define BLM_GVR(KS, WHOLE, ROPE)                                                                                        \
+  do {                                                                                                                  \
+    if (scale == nullptr) BLM_GVS(KS, WHOLE, ROPE, 0, RowScale{});                                                      \
+    else if (M <= waves) BLM_GVS(KS, WHOLE, ROPE, 1, *scale);                                                           \
+    else BLM_GVS(KS, WHOLE, ROPE, RS_SLOTS, *scale);                                                                    \
+  } while (0)
 #define BLM_GVF(KS, WHOLE)                                                                                              \
   do {                                                                                                                  \
-    if (rope)                                                                                                           \
-      hipLaunchKernelGGL((gemv_f32_kernel<KS, WHOLE, true>), grid, block, 0, stream, (const float*)A, (const float*)Wp, (float*)C, M, N, K, \
-                         lda, ldc, n_tiles, k_steps, gated, steps, per_block, *rope);                                   \
-    else                                                                                                                \
-      hipLaunchKernelGGL((gemv_f32_kernel<KS, WHOLE, false>), grid, block, 0, stream, (const float*)A, (const float*)Wp, (float*)C, M, N, K, \
-                         lda, ldc, n_tiles, k_steps, gated, steps, per_block, GvRope{});                                \
+    if (rope) BLM_GVR(KS, WHOLE, true);                                                                                 \
+    else BLM_GVR(KS, WHOLE, false);                                                                                     \
   } while (0)
   const bool whole = K % 16 == 0 && k_steps == groups * steps && steps == waves * ksteps;
   if (ksteps == 4 && whole) BLM_GVF(4, true);
@@ -398,22 +414,49 @@ static int gv_run(const void* A, const void* Wp, void* C, int M, int N, int K, i
   else if (whole) BLM_GVF(16, true);
   else BLM_GVF(16, false);
 #undef BLM_GVF
+#undef BLM_GVR
+#undef BLM_GVS
   BLM_LAUNCH_CHECK("gemv_f32");
   return 0;
 }
 
 extern "C" int blm_gemv_f32(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int ldc, int gated, int groups,
                             hipStream_t stream) {
-  return gv_run(A, Wp, C, M, N, K, lda, ldc, gated, groups, nullptr, stream);
+  return gv_run(A, Wp, C, M, N, K, lda, ldc, gated, groups, nullptr, nullptr, stream);
+}
+
+// The same of up to eight rows that come unscaled: sums [M, n_sums] holds parts of the rows' sums of squares (row_scale.h).
+extern "C" int blm_gemv_f32_scaled(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int ldc, int gated,
+                                   const float* sums, int n_sums, float eps, hipStream_t stream) {
+  BLM_REQUIRE(row_scale_fits(M, sums, n_sums), "gemv_f32_scaled: M=%d with %d sums a row", M, n_sums);
+  const RowScale scale{sums, n_sums, 1.0f / (float)K, eps};
+  return gv_run(A, Wp, C, M, N, K, lda, ldc, gated, 1, nullptr, &scale, stream);
 }
 
 // The q/k/v projection of up to 16 rows with the rotation (rotary partners are neighbouring columns) and the write of keys and
 // values into their pages.  qkv_out [M][ldq]: the queries.
-extern "C" int blm_gemv_f32_qkv_rope(const void* A, const void* Wp, void* qkv_out, const int* positions, const int* token_seq,
-                                     const int* block_table, int table_width, const void* cos_sin, void* kcache, void* vcache, int page_size,
-                                     int M, int K, int lda, int ldq, int nh, int nkv, int hd, int store, hipStream_t stream) {
+static int gv_rope(const void* A, const void* Wp, void* qkv_out, const int* positions, const int* token_seq,
+                   const int* block_table, int table_width, const void* cos_sin, void* kcache, void* vcache, int page_size,
+                   int M, int K, int lda, int ldq, int nh, int nkv, int hd, int store, const RowScale* scale, hipStream_t stream) {
   BLM_REQUIRE(nh > 0 && nkv > 0 && hd > 0 && hd % 2 == 0 && page_size > 0 && table_width > 0, "gemv_f32_qkv_rope: bad geometry (head size %d)", hd);
   BLM_REQUIRE(((uintptr_t)cos_sin % 8) == 0, "gemv_f32_qkv_rope: the table of angles must be 8-byte aligned");
   const GvRope rope{positions, token_seq, block_table, (const float2*)cos_sin, (float*)kcache, (float*)vcache, table_width, page_size, nh, nkv, hd, store};
-  return gv_run(A, Wp, qkv_out, M, (nh + 2 * nkv) * hd, K, lda, ldq, 0, 1, &rope, stream);
+  return gv_run(A, Wp, qkv_out, M, (nh + 2 * nkv) * hd, K, lda, ldq, 0, 1, &rope, scale, stream);
+}
+
+extern "C" int blm_gemv_f32_qkv_rope(const void* A, const void* Wp, void* qkv_out, const int* positions, const int* token_seq,
+                                     const int* block_table, int table_width, const void* cos_sin, void* kcache, void* vcache, int page_size,
+                                     int M, int K, int lda, int ldq, int nh, int nkv, int hd, int store, hipStream_t stream) {
+  return gv_rope(A, Wp, qkv_out, positions, token_seq, block_table, table_width, cos_sin, kcache, vcache, page_size, M, K, lda, ldq, nh, nkv, hd,
+                 store, nullptr, stream);
+}
+
+extern "C" int blm_gemv_f32_qkv_rope_scaled(const void* A, const void* Wp, void* qkv_out, const int* positions, const int* token_seq,
+                                            const int* block_table, int table_width, const void* cos_sin, void* kcache, void* vcache, int page_size,
+                                            int M, int K, int lda, int ldq, int nh, int nkv, int hd, int store, const float* sums,
+                                            int n_sums, float eps, hipStream_t stream) {
+  BLM_REQUIRE(row_scale_fits(M, sums, n_sums), "gemv_f32_qkv_rope_scaled: M=%d with %d sums a row", M, n_sums);
+  const RowScale scale{sums, n_sums, 1.0f / (float)K, eps};
+  return gv_rope(A, Wp, qkv_out, positions, token_seq, block_table, table_width, cos_sin, kcache, vcache, page_size, M, K, lda, ldq, nh, nkv, hd,
+                 store, &scale, stream);
 }

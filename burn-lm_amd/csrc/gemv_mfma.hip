@@ -18,6 +18,7 @@
 // wavefronts are summed through shared memory in a fixed order.  The SwiGLU gating of a
 // feed-forward can be fused into the product that computes gate and up (c_mode 1).
 #include "common.h"
+#include "row_scale.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
@@ -36,11 +37,14 @@ __device__ __forceinline__ float gv_gate(float g, int c_mode) {
   return g / (1.0f + expf(-g));
 }
 
-template <int KSTEPS, int MAXT, bool KEEP_A, typename TC>
+// SCALED: the rows come unscaled (row_scale.h), that many of them to a wavefront.
+template <int KSTEPS, int MAXT, bool KEEP_A, int SCALED, typename TC>
 __global__ void __launch_bounds__(MAXT)
     gemv_mfma_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, TC* __restrict__ C, int M, int N,
-                     int K, int lda, int ldc, int n_tiles, int k_steps, int c_mode, int steps_per_group) {
+                     int K, int lda, int ldc, int n_tiles, int k_steps, int c_mode, int steps_per_group, RowScale scale) {
   extern __shared__ float red[];  // [waves][256]
+  __shared__ float inv[RS_ROWS];
+  RowScaleLoad<SCALED ? SCALED : 1> scale_load;
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
   const int n_waves = blockDim.x / BLM_WAVE;
   const int row = lane & 15, kg = lane >> 4;
@@ -73,6 +77,7 @@ __global__ void __launch_bounds__(MAXT)
     const bool keep = row < M && k < K && step0 + s < group_end;                      \
     a[s] = make_uint4(keep ? a[s].x : 0u, keep ? a[s].y : 0u, keep ? a[s].z : 0u, keep ? a[s].w : 0u); \
   }
+  if (SCALED) scale_load.ask(scale, M, wave, n_waves, lane);
   if (KEEP_A) GV_LOAD_ACTIVATIONS()
 
   // a block takes a run of neighbouring column tiles, so that it streams one contiguous piece of the
@@ -101,6 +106,7 @@ __global__ void __launch_bounds__(MAXT)
     for (int s = 0; s < HALF; ++s) wb[s] = ld16_stream(wt + woff[HALF + s]);
   }
   __builtin_amdgcn_sched_barrier(0);
+  if (SCALED) scale_load.finish(scale, M, wave, n_waves, lane, inv);
   if (KEEP_A) GV_ZERO_ACTIVATIONS()
 #undef GV_LOAD_ACTIVATIONS
 #undef GV_ZERO_ACTIVATIONS
@@ -158,7 +164,7 @@ __global__ void __launch_bounds__(MAXT)
                                                       __builtin_bit_cast(bf16x8_t, w[s]), acc, 0, 0, 0);
     }
     // acc[r] is the product for row m = kg*4 + r and column n = tile*16 + row
-    if (n_waves == 1 && c_mode == 0) {
+    if (!SCALED && n_waves == 1 && c_mode == 0) {
       const int n = tile * 16 + row;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -175,6 +181,7 @@ __global__ void __launch_bounds__(MAXT)
         if (c_mode == 0) {
           float s = 0.f;
           for (int w2 = 0; w2 < n_waves; ++w2) s += red[w2 * 256 + idx];
+          if (SCALED) s *= inv[m];
           const int nn = tile * 16 + col;
           if (m < M && nn < N) C[(size_t)m * ldc + nn] = from_float<TC>(s);
         } else if (col < 8) {
@@ -183,6 +190,10 @@ __global__ void __launch_bounds__(MAXT)
           for (int w2 = 0; w2 < n_waves; ++w2) {
             g += red[w2 * 256 + idx];
             u += red[w2 * 256 + idx + 8];
+          }
+          if (SCALED) {
+            g *= inv[m];
+            u *= inv[m];
           }
           const int nn = tile * 8 + col;
           if (m < M && nn < N / 2) C[(size_t)m * ldc + nn] = from_float<TC>(gv_gate(g, c_mode) * u);
@@ -359,7 +370,7 @@ extern "C" int blm_gemv_mfma_geometry(int M, int N, int K, int k_groups, int* bl
 
 template <typename TC>
 static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int ldc, int c_mode,
-                       int k_groups, hipStream_t stream) {
+                       int k_groups, const RowScale* scale, hipStream_t stream) {
   const int n_tiles = (N + 15) / 16;
   const int k_steps = (K + 31) / 32;
   const int steps_per_group = (k_steps + k_groups - 1) / k_groups;
@@ -383,15 +394,23 @@ static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int
   const int ksteps = geo.ksteps, waves = geo.waves, blocks = geo.blocks;
   dim3 grid(blocks, k_groups), block(waves * BLM_WAVE);
   const size_t smem = (size_t)waves * 256 * sizeof(float);
+#define BLM_GS(KS, MAXT, KEEP, SCALED, SCALE)                                                                   \
+  hipLaunchKernelGGL((gemv_mfma_kernel<KS, MAXT, KEEP, SCALED, TC>), grid, block, smem, stream, (const bf16*)A, \
+                     (const bf16*)Wp, (TC*)C, M, N, K, lda, ldc, n_tiles, k_steps, c_mode, steps_per_group, SCALE)
 #define BLM_GM(KS, MAXT, KEEP)                                                                                  \
-  hipLaunchKernelGGL((gemv_mfma_kernel<KS, MAXT, KEEP, TC>), grid, block, smem, stream, (const bf16*)A,         \
-                     (const bf16*)Wp, (TC*)C, M, N, K, lda, ldc, n_tiles, k_steps, c_mode, steps_per_group)
+  do {                                                                                                          \
+    if (scale == nullptr) BLM_GS(KS, MAXT, KEEP, 0, RowScale{});                                                \
+    else if (M <= waves) BLM_GS(KS, MAXT, KEEP, 1, *scale);                                                     \
+    else if (M <= 2 * waves) BLM_GS(KS, MAXT, KEEP, 2, *scale);                                                 \
+    else BLM_GS(KS, MAXT, KEEP, RS_SLOTS, *scale);                                                              \
+  } while (0)
   if (ksteps == 4) BLM_GM(4, 256, true);
   else if (ksteps == 16 && waves <= 4) BLM_GM(16, 256, true);
   else if (ksteps == 16) BLM_GM(16, 512, true);
   else if (waves <= 8) BLM_GM(32, 512, true);
   else BLM_GM(32, 1024, false);
 #undef BLM_GM
+#undef BLM_GS
   BLM_LAUNCH_CHECK("gemv_mfma");
   return 0;
 }
@@ -404,8 +423,8 @@ static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int
 // k_groups > 1: K is cut into that many groups handled by different blocks; C is then float
 // [k_groups, M, ldc] and holds one partial product per group, to be summed by the reader (the
 // residual add in front of the next norm does it), so narrow outputs still occupy the whole chip.
-extern "C" int blm_gemv_mfma(const void* A, const void* Wp, void* C, int c_dtype, int M, int N, int K, int lda,
-                             int ldc, int c_mode, int k_groups, hipStream_t stream) {
+static int gemv_mfma_entry(const void* A, const void* Wp, void* C, int c_dtype, int M, int N, int K, int lda,
+                             int ldc, int c_mode, int k_groups, const RowScale* scale, hipStream_t stream) {
   BLM_REQUIRE(M >= 1 && M <= 64, "gemv_mfma: M=%d out of range 1..64", M);
   BLM_REQUIRE(N >= 1 && K >= 8 && K % 8 == 0, "gemv_mfma: sizes N=%d K=%d not supported (K a multiple of 8)", N, K);
   BLM_REQUIRE(c_mode == 0 || ((c_mode == 1 || c_mode == 2) && N % 16 == 0 && k_groups == 1),
@@ -420,7 +439,21 @@ extern "C" int blm_gemv_mfma(const void* A, const void* Wp, void* C, int c_dtype
   }
   BLM_REQUIRE(lda % 8 == 0 && lda >= K && ldc >= (c_mode ? N / 2 : N), "gemv_mfma: bad strides lda=%d ldc=%d", lda, ldc);
   BLM_REQUIRE(((uintptr_t)A % 16) == 0 && ((uintptr_t)Wp % 16) == 0, "gemv_mfma: operands must be 16-byte aligned");
-  if (c_dtype == BLM_BF16) return launch_mfma<bf16>(A, Wp, C, M, N, K, lda, ldc, c_mode, k_groups, stream);
-  if (c_dtype == BLM_F32) return launch_mfma<float>(A, Wp, C, M, N, K, lda, ldc, c_mode, k_groups, stream);
+  if (c_dtype == BLM_BF16) return launch_mfma<bf16>(A, Wp, C, M, N, K, lda, ldc, c_mode, k_groups, scale, stream);
+  if (c_dtype == BLM_F32) return launch_mfma<float>(A, Wp, C, M, N, K, lda, ldc, c_mode, k_groups, scale, stream);
   return blm_fail("gemv_mfma: unsupported output dtype %d", c_dtype);
+}
+
+extern "C" int blm_gemv_mfma(const void* A, const void* Wp, void* C, int c_dtype, int M, int N, int K, int lda,
+                             int ldc, int c_mode, int k_groups, hipStream_t stream) {
+  return gemv_mfma_entry(A, Wp, C, c_dtype, M, N, K, lda, ldc, c_mode, k_groups, nullptr, stream);
+}
+
+// The same of up to eight rows that come unscaled: sums [M, n_sums] holds parts of the rows' sums of squares, and the product's row m is
+// multiplied by 1 / sqrt(sum / K + eps) (row_scale.h).
+extern "C" int blm_gemv_mfma_scaled(const void* A, const void* Wp, void* C, int c_dtype, int M, int N, int K, int lda, int ldc,
+                                    int c_mode, const float* sums, int n_sums, float eps, hipStream_t stream) {
+  BLM_REQUIRE(row_scale_fits(M, sums, n_sums), "gemv_mfma_scaled: M=%d with %d sums a row", M, n_sums);
+  const RowScale scale{sums, n_sums, 1.0f / (float)K, eps};
+  return gemv_mfma_entry(A, Wp, C, c_dtype, M, N, K, lda, ldc, c_mode, 1, &scale, stream);
 }

@@ -12,20 +12,25 @@
 // tile, KW..2KW-1 on the second, each on 512 of K; the partial tiles are summed through LDS and
 // the epilogue rotates and scatters them.
 #include "common.h"
+#include "row_scale.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 // QR_KSTEPS: k-steps of 32 per wavefront.  MAXT: most threads of a block (8 or 16 wavefronts).  All
 // loads of a block are in flight at once: its time is one memory latency.
-template <int QR_KSTEPS, int MAXT>
+// SCALED: the rows come unscaled (row_scale.h), that many of them to a wavefront.
+template <int QR_KSTEPS, int MAXT, int SCALED>
 __global__ void __launch_bounds__(MAXT)
     gemv_qkv_rope_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, bf16* __restrict__ qkv_out,
                          const int* __restrict__ positions, const int* __restrict__ token_seq,
                          const int* __restrict__ block_table, int table_width, const float2* __restrict__ cos_sin,
                          bf16* __restrict__ kcache, bf16* __restrict__ vcache, int page_size, int M, int K, int lda,
-                         int ldq, int k_steps, int kw_count, int nh, int nkv, int hd, int pairing, int store) {
+                         int ldq, int k_steps, int kw_count, int nh, int nkv, int hd, int pairing, int store,
+                         RowScale scale) {
   extern __shared__ float red[];   // [2 * kw_count wavefronts][256]
+  __shared__ float inv[RS_ROWS];
+  RowScaleLoad<SCALED ? SCALED : 1> scale_load;
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
   const int row = lane & 15, kg = lane >> 4;
   const int units_per_head = hd / 32;
@@ -40,6 +45,7 @@ __global__ void __launch_bounds__(MAXT)
   const int step0 = kw * QR_KSTEPS;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
 
+  if (SCALED) scale_load.ask(scale, M, wave, 2 * kw_count, lane);
   const bf16* wt = Wp + ((size_t)tile * k_steps * 64 + lane) * 8;
   uint4 w[QR_KSTEPS];
 #pragma unroll
@@ -56,6 +62,7 @@ __global__ void __launch_bounds__(MAXT)
     a[s] = (row < M && k < K) ? v : zero;
   }
   __builtin_amdgcn_sched_barrier(0);
+  if (SCALED) scale_load.finish(scale, M, wave, 2 * kw_count, lane, inv);
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < QR_KSTEPS; ++s)
@@ -75,6 +82,10 @@ __global__ void __launch_bounds__(MAXT)
       x0 += red[k2 * 256 + idx];
       x1 += red[(kw_count + k2) * 256 + idx];
     }
+    if (SCALED) {
+      x0 *= inv[m];
+      x1 *= inv[m];
+    }
     const int b = token_seq[m];
     const int pos = positions[m];
     const int d0 = col0 + c, d1 = col1 + c;      // lanes within the head held by x0 and x1
@@ -91,6 +102,10 @@ __global__ void __launch_bounds__(MAXT)
       for (int k2 = 0; k2 < kw_count; ++k2) {
         p0 += red[k2 * 256 + (idx ^ 1)];
         p1 += red[(kw_count + k2) * 256 + (idx ^ 1)];
+      }
+      if (SCALED) {
+        p0 *= inv[m];
+        p1 *= inv[m];
       }
       const float2 c0 = cos_sin[(size_t)pos * (hd / 2) + (d0 >> 1)];
       const float2 c1 = cos_sin[(size_t)pos * (hd / 2) + (d1 >> 1)];
@@ -123,15 +138,17 @@ __global__ void __launch_bounds__(MAXT)
 // block owns ONE tile and its wavefronts split K.  That is twice as many blocks as with two-tile
 // units, which matters because the whole product is a few blocks per compute unit at most (3072
 // columns are 192 tiles).  Value heads are not rotated.  red: [wavefronts][256].
-template <int QR_KSTEPS>
+template <int QR_KSTEPS, int SCALED>
 __global__ void __launch_bounds__(512)
     gemv_qkv_rope_tile_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, bf16* __restrict__ qkv_out,
                               const int* __restrict__ positions, const int* __restrict__ token_seq,
                               const int* __restrict__ block_table, int table_width,
                               const float2* __restrict__ cos_sin, bf16* __restrict__ kcache,
                               bf16* __restrict__ vcache, int page_size, int M, int K, int lda, int ldq, int k_steps,
-                              int nh, int nkv, int hd, int store) {
+                              int nh, int nkv, int hd, int store, RowScale scale) {
   extern __shared__ float red[];
+  __shared__ float inv[RS_ROWS];
+  RowScaleLoad<SCALED ? SCALED : 1> scale_load;
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
   const int n_waves = blockDim.x / BLM_WAVE;
   const int row = lane & 15, kg = lane >> 4;
@@ -142,6 +159,7 @@ __global__ void __launch_bounds__(512)
   const int step0 = wave * QR_KSTEPS;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
 
+  if (SCALED) scale_load.ask(scale, M, wave, n_waves, lane);
   const bf16* wt = Wp + ((size_t)tile * k_steps * 64 + lane) * 8;
   uint4 w[QR_KSTEPS];
 #pragma unroll
@@ -158,6 +176,7 @@ __global__ void __launch_bounds__(512)
     a[s] = (row < M && k < K) ? v : zero;
   }
   __builtin_amdgcn_sched_barrier(0);
+  if (SCALED) scale_load.finish(scale, M, wave, n_waves, lane, inv);
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < QR_KSTEPS; ++s)
@@ -176,6 +195,10 @@ __global__ void __launch_bounds__(512)
     for (int k2 = 0; k2 < n_waves; ++k2) {
       x += red[k2 * 256 + idx];
       partner += red[k2 * 256 + (idx ^ 1)];
+    }
+    if (SCALED) {
+      x *= inv[m];
+      partner *= inv[m];
     }
     const int b = token_seq[m];
     const int pos = positions[m];
@@ -302,11 +325,11 @@ extern "C" int blm_gemv_qkv_rope_supported(int M, int K, int hd, int pairing) {
 // Wp: pack_weight of W_qkv [(nh + 2 nkv) * hd, K].  qkv_out: [M, ldq] bf16; only its first nh*hd
 // columns (the rotated queries) are written.  Key plane [pages, nkv, page, hd], value plane
 // [pages, nkv, hd, page].  store = 0: keys and values are neither computed nor written.
-extern "C" int blm_gemv_qkv_rope(const void* A, const void* Wp, void* qkv_out, const int* positions,
-                                 const int* token_seq, const int* block_table, int table_width,
+static int qkv_rope_entry(const void* A, const void* Wp, void* qkv_out, const int* positions,
+                          const int* token_seq, const int* block_table, int table_width,
                                  const float* cos_sin, void* kcache, void* vcache, int page_size, int M, int K,
                                  int lda, int ldq, int nh, int nkv, int hd, int pairing, int store,
-                                 hipStream_t stream) {
+                                 const RowScale* scale, hipStream_t stream) {
   BLM_REQUIRE(blm_gemv_qkv_rope_supported(M, K, hd, pairing), "gemv_qkv_rope: M=%d K=%d head_dim=%d pairing=%d not "
               "supported (K a multiple of 8 and at most 4096, head_dim a multiple of 16 for adjacent pairs and of "
               "32 for pairs half a head apart; 17 to 64 rows: adjacent pairs, K at most 2048 above 32 rows)",
@@ -341,10 +364,16 @@ extern "C" int blm_gemv_qkv_rope(const void* A, const void* Wp, void* qkv_out, c
   if (pairing == 0 && (tiles <= 256 || hd % 32 != 0 || k_steps > 96)) {
     // 16 k-steps per wavefront: up to 8 wavefronts
     const int waves = (k_steps + 15) / 16;
-    hipLaunchKernelGGL(gemv_qkv_rope_tile_kernel<16>, dim3(tiles), dim3(waves * BLM_WAVE), (size_t)waves * 256 * sizeof(float),
-                       stream, (const bf16*)A, (const bf16*)Wp, (bf16*)qkv_out, positions, token_seq, block_table,
-                       table_width, (const float2*)cos_sin, (bf16*)kcache, (bf16*)vcache, page_size, M, K, lda, ldq,
-                       k_steps, nh, nkv, hd, store);
+#define BLM_QT(SCALED, SCALE)                                                                                           \
+  hipLaunchKernelGGL((gemv_qkv_rope_tile_kernel<16, SCALED>), dim3(tiles), dim3(waves * BLM_WAVE),                       \
+                     (size_t)waves * 256 * sizeof(float), stream, (const bf16*)A, (const bf16*)Wp, (bf16*)qkv_out,       \
+                     positions, token_seq, block_table, table_width, (const float2*)cos_sin, (bf16*)kcache, (bf16*)vcache, \
+                     page_size, M, K, lda, ldq, k_steps, nh, nkv, hd, store, SCALE)
+    if (scale == nullptr) BLM_QT(0, RowScale{});
+    else if (M <= waves) BLM_QT(1, *scale);
+    else if (M <= 2 * waves) BLM_QT(2, *scale);
+    else BLM_QT(RS_SLOTS, *scale);
+#undef BLM_QT
     BLM_LAUNCH_CHECK("gemv_qkv_rope_tile");
     return 0;
   }
@@ -355,14 +384,42 @@ extern "C" int blm_gemv_qkv_rope(const void* A, const void* Wp, void* qkv_out, c
   const int units = (nh + 2 * nkv) * (hd / 32);
   const size_t smem = (size_t)2 * kw * 256 * sizeof(float);
 #define BLM_QR(KS, MAXT)                                                                                              \
-  hipLaunchKernelGGL((gemv_qkv_rope_kernel<KS, MAXT>), dim3(units), dim3(2 * kw * BLM_WAVE), smem, stream, (const bf16*)A, \
+  do {                                                                                                                \
+    if (scale == nullptr) BLM_QS(KS, MAXT, 0, RowScale{});                                                            \
+    else if (M <= 2 * kw) BLM_QS(KS, MAXT, 1, *scale);                                                                \
+    else BLM_QS(KS, MAXT, RS_SLOTS / 2, *scale);                                                                      \
+  } while (0)
+#define BLM_QS(KS, MAXT, SCALED, SCALE)                                                                               \
+  hipLaunchKernelGGL((gemv_qkv_rope_kernel<KS, MAXT, SCALED>), dim3(units), dim3(2 * kw * BLM_WAVE), smem, stream, (const bf16*)A, \
                      (const bf16*)Wp, (bf16*)qkv_out, positions, token_seq, block_table, table_width,                 \
                      (const float2*)cos_sin, (bf16*)kcache, (bf16*)vcache, page_size, M, K, lda, ldq, k_steps, kw, nh, \
-                     nkv, hd, pairing, store)
+                     nkv, hd, pairing, store, SCALE)
   if (ksteps == 24) BLM_QR(24, 512);
   else if (kw <= 4) BLM_QR(16, 512);
   else BLM_QR(16, 1024);
+#undef BLM_QS
 #undef BLM_QR
   BLM_LAUNCH_CHECK("gemv_qkv_rope");
   return 0;
+}
+
+extern "C" int blm_gemv_qkv_rope(const void* A, const void* Wp, void* qkv_out, const int* positions,
+                                 const int* token_seq, const int* block_table, int table_width,
+                                 const float* cos_sin, void* kcache, void* vcache, int page_size, int M, int K,
+                                 int lda, int ldq, int nh, int nkv, int hd, int pairing, int store,
+                                 hipStream_t stream) {
+  return qkv_rope_entry(A, Wp, qkv_out, positions, token_seq, block_table, table_width, cos_sin, kcache, vcache, page_size, M, K, lda,
+                        ldq, nh, nkv, hd, pairing, store, nullptr, stream);
+}
+
+// The same of up to eight rows that come unscaled, with parts of their sums of squares beside them (row_scale.h).
+extern "C" int blm_gemv_qkv_rope_scaled(const void* A, const void* Wp, void* qkv_out, const int* positions,
+                                        const int* token_seq, const int* block_table, int table_width,
+                                        const float* cos_sin, void* kcache, void* vcache, int page_size, int M, int K,
+                                        int lda, int ldq, int nh, int nkv, int hd, int pairing, int store, const float* sums,
+                                        int n_sums, float eps, hipStream_t stream) {
+  BLM_REQUIRE(row_scale_fits(M, sums, n_sums), "gemv_qkv_rope_scaled: M=%d with %d sums a row", M, n_sums);
+  const RowScale scale{sums, n_sums, 1.0f / (float)K, eps};
+  return qkv_rope_entry(A, Wp, qkv_out, positions, token_seq, block_table, table_width, cos_sin, kcache, vcache, page_size, M, K, lda,
+                        ldq, nh, nkv, hd, pairing, store, &scale, stream);
 }

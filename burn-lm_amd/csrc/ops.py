@@ -11,7 +11,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 45
+ABI_VERSION = 46
 _lib = None
 _lock = threading.Lock()
 
@@ -139,6 +139,13 @@ _SIGNATURES = {
     "blm_gemm_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_gemv_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_gemv_f32_qkv_rope": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 9 + [_c_void_p],
+    "blm_gemv_f32_scaled": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_int, _c_float,
+                            _c_void_p],
+    "blm_gemv_f32_qkv_rope_scaled": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 9 + [_c_void_p, _c_int, _c_float, _c_void_p],
+    "blm_gemv_join_columns": [_c_int, _c_int, _c_int, _c_int],
+    "blm_gemv_join": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "blm_gemv_mfma_scaled": [_c_void_p, _c_void_p, _c_void_p] + [_c_int] * 7 + [_c_void_p, _c_int, _c_float, _c_void_p],
+    "blm_gemv_qkv_rope_scaled": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 10 + [_c_void_p, _c_int, _c_float, _c_void_p],
     "blm_gemv_f32_geometry": [_c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p],
     "blm_gemm_tiled": [_c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                        _c_int, _c_int, _c_void_p],
@@ -630,10 +637,51 @@ def gemv_f32_geometry(M, N, K, groups=1):
     return (blocks.value, waves.value) if ok else None
 
 
-def gemv_f32(a, packed, out, K, gated=False):
+ROW_SUMS = 256       # most partial sums of a row that comes unscaled, and most such rows
+SCALED_ROWS = 8
+
+
+def _scale(who, scale, M):
+    """The arguments of an entry point for rows that come unscaled, scale = (sums, eps): float32 sums [M, n], parts of the rows' sums of
+    squares; the product's rows are multiplied by 1 / sqrt(sum / K + eps)."""
+    sums, eps = scale
+    _gpu(sums)
+    if sums.dtype != torch.float32 or sums.dim() != 2 or sums.shape[0] != M or sums.shape[1] % 4 or not 4 <= sums.shape[1] <= ROW_SUMS \
+            or M > SCALED_ROWS or sums.data_ptr() % 16:
+        raise KernelError(f"{who}: up to {SCALED_ROWS} unscaled rows with float32 sums [rows, n] wanted, n a multiple of four up to {ROW_SUMS}")
+    _contig("sums", sums)
+    return sums.data_ptr(), sums.shape[1], float(eps)
+
+
+def gemv_join_columns(dtype, M, N, K):
+    """Columns of a block of gemv_join for M rows and a matrix [N, K], 0 where it does not take them."""
+    return library().blm_gemv_join_columns(DTYPE_CODE[dtype], int(M), int(N), int(K))
+
+
+def gemv_join(a, packed, h, gamma, y, sums, K):
+    """A product of up to eight rows with the add and the row sums of the norm behind it: h [M, N] (float32) += a [M, K] w^T, y = h * gamma
+    (gamma float32 [N]; y of a's type) and sums [M, N / gemv_join_columns] the parts of the rows' sums of squares, from packed =
+    pack_weight(w) of w [N, K].  What reads y scales its own sums (scale=(sums, eps))."""
+    _gpu(a, packed, h, gamma, y, sums)
+    M, N = h.shape
+    if a.shape != (M, K) or a.stride(1) != 1 or a.dtype not in DTYPE_CODE or packed.dtype != a.dtype or y.dtype != a.dtype or y.shape != h.shape:
+        raise KernelError(f"gemv_join: operands and rows of one type wanted, shapes a={tuple(a.shape)} h={tuple(h.shape)} y={tuple(y.shape)} K={K}")
+    columns = gemv_join_columns(a.dtype, M, N, K)
+    step = 64 // a.element_size()
+    if not columns or packed.numel() != N // 16 * (-(-K // step)) * 16 * step or not packed.is_contiguous():
+        raise KernelError(f"gemv_join: {M} rows of a [{N}, {K}] matrix with {packed.numel()} packed elements")
+    if any(t.dtype != torch.float32 for t in (h, gamma, sums)) or gamma.numel() != N or sums.shape != (M, N // columns):
+        raise KernelError(f"gemv_join: float32 h, gamma [{N}] and sums [{M}, {N // columns}] wanted")
+    _contig("h", h); _contig("gamma", gamma); _contig("y", y); _contig("sums", sums)
+    _call("blm_gemv_join", a.data_ptr(), DTYPE_CODE[a.dtype], packed.data_ptr(), h.data_ptr(), gamma.data_ptr(), y.data_ptr(), sums.data_ptr(), M,
+          N, K, a.stride(0), _stream())
+    return y
+
+
+def gemv_f32(a, packed, out, K, gated=False, scale=None):
     """The float32 product for up to 16 rows, streaming packed = pack_weight(w, gated) of w [N, K] once.  out: float32 [M, N],
     or [groups, M, N] partial products over that many groups of K; gated=True: [M, I] = silu(a gate^T) * (a up^T) for a
-    matrix of 2 I rows."""
+    matrix of 2 I rows.  scale=(sums, eps): up to eight rows that come unscaled (gemv_join), out [M, N] or [M, I]."""
     _gpu(a, packed, out)
     groups = out.shape[0] if out.dim() == 3 else 1
     M, N = out.shape[-2], out.shape[-1] * (2 if gated else 1)
@@ -645,15 +693,22 @@ def gemv_f32(a, packed, out, K, gated=False):
         raise KernelError("gemv_f32: a and out need unit stride along their rows")
     if out.dim() == 3:
         _contig("out", out)
+    if scale is not None:
+        if out.dim() == 3:
+            raise KernelError("gemv_f32: unscaled rows give no partial products")
+        _call("blm_gemv_f32_scaled", a.data_ptr(), packed.data_ptr(), out.data_ptr(), M, N, K, a.stride(0), out.stride(0), 1 if gated else 0,
+              *_scale("gemv_f32", scale, M), _stream())
+        return out
     _call("blm_gemv_f32", a.data_ptr(), packed.data_ptr(), out.data_ptr(), M, N, K, a.stride(0), out.stride(-2), 1 if gated else 0,
           groups, _stream())
     return out
 
 
-def gemv_f32_qkv_rope(x, packed, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache, page_size, nh, nkv, hd, write_kv=True):
+def gemv_f32_qkv_rope(x, packed, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache, page_size, nh, nkv, hd, write_kv=True,
+                      scale=None):
     """Up to 16 float32 rows: x [M, K] @ W_qkv^T from packed = pack_weight(w) of w [(nh + 2 nkv) * hd, K] with rotary partners in
     adjacent rows (K in one group), rotary encoding of q and k, q into qkv_out[:, :nh*hd], k and v into their cache pages, in one
-    kernel."""
+    kernel.  scale=(sums, eps): up to eight rows that come unscaled (gemv_join)."""
     _gpu(x, packed, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache)
     M, K = x.shape
     N = (nh + 2 * nkv) * hd
@@ -668,9 +723,13 @@ def gemv_f32_qkv_rope(x, packed, qkv_out, positions, token_seq, block_table, cos
         raise KernelError("gemv_f32_qkv_rope: cos_sin must be contiguous [positions, head_dim/2, 2]")
     _contig("kcache", kcache); _contig("vcache", vcache)
     _check_planes("gemv_f32_qkv_rope", kcache, vcache, nkv, page_size, hd)
-    _call("blm_gemv_f32_qkv_rope", x.data_ptr(), packed.data_ptr(), qkv_out.data_ptr(), positions.data_ptr(), token_seq.data_ptr(),
-          block_table.data_ptr(), block_table.shape[1], cos_sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), page_size, M, K,
-          x.stride(0), qkv_out.stride(0), nh, nkv, hd, 1 if write_kv else 0, _stream())
+    args = (x.data_ptr(), packed.data_ptr(), qkv_out.data_ptr(), positions.data_ptr(), token_seq.data_ptr(), block_table.data_ptr(),
+            block_table.shape[1], cos_sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), page_size, M, K, x.stride(0), qkv_out.stride(0),
+            nh, nkv, hd, 1 if write_kv else 0)
+    if scale is None:
+        _call("blm_gemv_f32_qkv_rope", *args, _stream())
+    else:
+        _call("blm_gemv_f32_qkv_rope_scaled", *args, *_scale("gemv_f32_qkv_rope", scale, M), _stream())
     return qkv_out
 
 
@@ -724,13 +783,14 @@ def pack_weight(w, gated=False):
     return w.view(Np // 16, 16, Kp // (4 * E), 4, E).permute(0, 2, 3, 1, 4).contiguous().view(-1)
 
 
-def gemv_mfma(a, packed, out, K, gated=False, activation="silu"):
+def gemv_mfma(a, packed, out, K, gated=False, activation="silu", scale=None):
     """bfloat16 product for M <= 64 rows on the matrix cores; streams the packed weights once (17 to 64
     rows: K at most 2048 per group, see gemv_mfma_group_limit).
     packed: pack_weight(w) of w [N, K].  out: bfloat16 or float32 [M, N], or float32
     [groups, M, N]: K is then cut into that many groups whose partial products fill the planes of
     out (the reader sums them).  gated=True: packed = pack_weight(w, gated=True) of a [2I, K] matrix
-    and out is [M, I] = act(a gate^T) * (a up^T) with act = silu, or (activation="gelu_tanh") the tanh form of GELU."""
+    and out is [M, I] = act(a gate^T) * (a up^T) with act = silu, or (activation="gelu_tanh") the tanh form of GELU.
+    scale=(sums, eps): up to eight rows that come unscaled (gemv_join), all of K in one group."""
     _gpu(a, packed, out)
     if activation not in ("silu", "gelu_tanh"):
         raise KernelError(f"gemv_mfma: activation {activation!r} unknown (silu, gelu_tanh)")
@@ -750,8 +810,15 @@ def gemv_mfma(a, packed, out, K, gated=False, activation="silu"):
         raise KernelError("gemv_mfma: a and out need unit stride along their rows")
     if a.dtype != torch.bfloat16 or packed.dtype != torch.bfloat16:
         raise KernelError("gemv_mfma: operands must be bfloat16")
+    mode = (2 if activation == "gelu_tanh" else 1) if gated else 0
+    if scale is not None:
+        if out.dim() == 3:
+            raise KernelError("gemv_mfma: unscaled rows give no partial products")
+        _call("blm_gemv_mfma_scaled", a.data_ptr(), packed.data_ptr(), out.data_ptr(), _code(out), M, N, K, a.stride(0), out.stride(0), mode,
+              *_scale("gemv_mfma", scale, M), _stream())
+        return out
     _call("blm_gemv_mfma", a.data_ptr(), packed.data_ptr(), out.data_ptr(), _code(out), M, N, K, a.stride(0),
-          out.stride(-2), (2 if activation == "gelu_tanh" else 1) if gated else 0, groups, _stream())
+          out.stride(-2), mode, groups, _stream())
     return out
 
 
@@ -964,10 +1031,10 @@ def gemv_qkv_rope_supported(M, K, hd, pairing):
 
 
 def gemv_qkv_rope(x, packed, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache, page_size,
-                  nh, nkv, hd, pairing, write_kv=True):
+                  nh, nkv, hd, pairing, write_kv=True, scale=None):
     """Decode: x [M<=64, K] @ W_qkv^T on the matrix cores, rotary encoding of q and k on the float
     results, q into qkv_out[:, :nh*hd], k and v into their cache pages, all in one kernel.
-    packed: pack_weight of W_qkv [(nh + 2 nkv) * hd, K]."""
+    packed: pack_weight of W_qkv [(nh + 2 nkv) * hd, K].  scale=(sums, eps): up to eight rows that come unscaled (gemv_join)."""
     _gpu(x, packed, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache)
     M, K = x.shape
     N = (nh + 2 * nkv) * hd
@@ -984,10 +1051,13 @@ def gemv_qkv_rope(x, packed, qkv_out, positions, token_seq, block_table, cos_sin
         raise KernelError("gemv_qkv_rope: the cache must be bfloat16")
     _contig("kcache", kcache); _contig("vcache", vcache)
     _check_planes("gemv_qkv_rope", kcache, vcache, nkv, page_size, hd)
-    _call("blm_gemv_qkv_rope", x.data_ptr(), packed.data_ptr(), qkv_out.data_ptr(), positions.data_ptr(),
-          token_seq.data_ptr(), block_table.data_ptr(), block_table.shape[1], cos_sin.data_ptr(), kcache.data_ptr(),
-          vcache.data_ptr(), page_size, M, K, x.stride(0), qkv_out.stride(0), nh, nkv, hd, pairing,
-          1 if write_kv else 0, _stream())
+    args = (x.data_ptr(), packed.data_ptr(), qkv_out.data_ptr(), positions.data_ptr(), token_seq.data_ptr(), block_table.data_ptr(),
+            block_table.shape[1], cos_sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), page_size, M, K, x.stride(0), qkv_out.stride(0),
+            nh, nkv, hd, pairing, 1 if write_kv else 0)
+    if scale is None:
+        _call("blm_gemv_qkv_rope", *args, _stream())
+    else:
+        _call("blm_gemv_qkv_rope_scaled", *args, *_scale("gemv_qkv_rope", scale, M), _stream())
     return qkv_out
 
 

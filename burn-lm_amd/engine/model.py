@@ -70,6 +70,10 @@ class Model:
             p.bind(tensors, rt)
         for b in self.blocks:
             b.bound()
+        self.seams = [None] * (len(self.plan.order) + 1)      # in front of every place, and behind the last
+        for i, (a, b) in enumerate(zip(self.plan.order, self.plan.order[1:])):
+            if b.turn is None and hasattr(self.blocks[a.layer], "seam_to"):
+                self.seams[i + 1] = self.blocks[a.layer].seam_to(self.blocks[b.layer])
 
     def cache_needs(self) -> List:
         return [self.blocks[pl.layer].cache_need() for pl in self.plan.order]
@@ -122,7 +126,11 @@ class Model:
         for i, place in enumerate(self.plan.order):
             if place.turn is not None:
                 delta = self.entry.enter(h, delta, both, place.turn)
-            delta = self.blocks[place.layer].forward(h, delta, step, cache.views[i])
+            block = self.blocks[place.layer]
+            if self.seams[i] is None and self.seams[i + 1] is None:
+                delta = block.forward(h, delta, step, cache.views[i])
+            else:
+                delta = block.forward_to(h, delta, step, cache.views[i], self.seams[i], self.seams[i + 1])
         if step.n_wanted == 0:
             return None
         x = self.final_norm.add_norm(h, delta, rows=step.want_rows, write_h=False)

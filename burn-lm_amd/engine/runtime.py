@@ -34,6 +34,7 @@ import os
 import torch
 
 from ..csrc import ops
+from ..parts.base import Unscaled
 
 SKINNY_MAX_ROWS = 8
 MFMA_SKINNY_MAX_ROWS = 64
@@ -88,6 +89,7 @@ def rows_plan(N, K, compute_units):
 # 2,048 rows at [3072, 2048], [2048, 2048], [16384, 2048], [2048, 8192], [5000, 1416].
 F32_STEP_US = {(128, 128): (2.33, 2.0), (128, 64): (1.25, 1.0), (64, 128): (1.2, 1.0), (64, 64): (0.7, 0.5)}
 F32_SHARE_US = 0.1
+JOIN_BF16_WIDTH = 1024     # see Runtime.join_takes
 F32_SKINNY_MAX_ROWS = 16
 F32_SKINNY_GROUP_K = 2048
 
@@ -602,6 +604,43 @@ class Runtime:
         tiles = ops.gemm_duo_tiles(M, N)[0]
         return whole < tiles and tiles >= self.compute_units
 
+    # ---- products of few rows that do a neighbouring norm's work (ops.gemv_join, parts/block.py) ----
+    def join_takes(self, M, w):
+        """Whether the product of M rows with w can add its result to the residual and leave the next norm's rows (join).  Up to eight
+        rows: beyond, every block's activations, all of K for few columns, cost more than the norm's kernel (a layer of the 1B shape
+        without its attention, us, norms as kernels / joined: 1 row 34.9 / 29.9, 4 rows 36.2 / 31.5, 8 rows 37.6 / 34.1, 16 rows 40.9 /
+        40.2; of the 3B shape 50.3 / 44.3, 52.6 / 45.9, 54.3 / 48.3, 59.2 / 68.7).  bfloat16 from JOIN_BF16_WIDTH columns on: the rows are
+        rounded in front of the norm's factor instead of behind it, as far from 64 bits but elsewhere, and a narrow model, whose
+        steps are the host's time anyway, keeps the roundings that it is compared with value by value."""
+        return (M <= ops.SCALED_ROWS and isinstance(w, LinearWeight) and not w.gated and w.dtype == self.dtype and w.packable
+                and (w.dtype == torch.float32 or w.shape[0] >= JOIN_BF16_WIDTH) and ops.gemv_join_columns(w.dtype, M, *w.shape) > 0 and w.packed is not None)
+
+    def join(self, product, h, gamma, eps):
+        """h += the product; the rows of an RMS norm with gamma (float32) and eps behind it, Unscaled."""
+        x, w = product.x, product.w
+        M, (N, K) = x.shape[0], w.shape
+        y = torch.empty(M, N, dtype=self.dtype, device=x.device)
+        sums = torch.empty(M, N // ops.gemv_join_columns(w.dtype, M, N, K), dtype=torch.float32, device=x.device)
+        return Unscaled(ops.gemv_join(x, w.packed, h, gamma, y, sums, K), sums, eps)
+
+    def gated_takes_unscaled(self, M, w):
+        """Whether gated_linear takes M Unscaled rows: where its packed kernels have them."""
+        if not (isinstance(w, LinearWeight) and w.gated and w.packable and M <= ops.SCALED_ROWS and w.dtype == self.dtype):
+            return False
+        if self.dtype == torch.float32:
+            return w.packed is not None
+        return M <= self.skinny_gated_rows and bool(ops.gemv_mfma_supported(M, *w.shape))
+
+    def qkv_takes_unscaled(self, M, w, head_dim):
+        """The same of a q/k/v projection with rotation in adjacent pairs."""
+        if not (isinstance(w, LinearWeight) and not w.gated and w.packable and M <= ops.SCALED_ROWS and w.dtype == self.dtype):
+            return False
+        N, K = w.shape
+        if self.dtype == torch.float32:
+            return head_dim % 2 == 0 and self.f32_skinny_groups(M, N, K, False) == 1 and w.packed is not None
+        plan = self.qkv_plan(M, N, K)
+        return plan is not None and plan.kernel == "packed" and ops.gemv_qkv_rope_supported(M, K, head_dim, 0)
+
     def _gated_by_library(self, M, K, inner):
         """17 to 64 rows of a gated product that are better left to the library's product and the gating kernel:
         from 33 rows on where K is beyond 4096 (measured at widths 5120 and 8192 with inner sizes of 6144 to 28672:
@@ -642,7 +681,14 @@ class Runtime:
         """act(x gate^T) * (x up^T) for w = [gate rows; up rows] ([2I, K]) -> [M, I]; act is silu or
         (activation="gelu_tanh") the tanh form of GELU.  With few rows in bfloat16 the gating is fused
         into the product (weight(w, gated=True) pairs the rows for it); otherwise the product is followed
-        by the gating kernel."""
+        by the gating kernel.  x may be Unscaled where gated_takes_unscaled says so."""
+        if isinstance(x, Unscaled):
+            out = torch.empty(x.y.shape[0], w.shape[0] // 2, dtype=self.dtype, device=x.y.device)
+            if self.dtype == torch.float32:
+                if activation != "silu":
+                    raise ValueError("gated_linear: float32 rows that come unscaled are gated with silu")
+                return ops.gemv_f32(x.y, w.packed, out, w.shape[1], gated=True, scale=x.scale)
+            return ops.gemv_mfma(x.y, w.packed, out, w.shape[1], gated=True, activation=activation, scale=x.scale)
         M, K = x.shape
         inner = w.shape[0] // 2
         plain = w.w if isinstance(w, LinearWeight) else w

@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 
 
-from .base import KVNeed, Mixer, TensorSpec
+from .base import KVNeed, Mixer, Product, TensorSpec, speaks_for
 
 # Blocks the decode attention aims for when it cuts the key ranges into pieces: one round of at most one
 # block per compute unit, at least half of them busy, and no cutting from one block per unit on.
@@ -123,6 +123,18 @@ class Attention(Mixer):
         if view.v.shape[1:3] != (self.kv_heads, self.head_dim):
             raise ValueError("the attention mixer needs values of the keys' head count and head size")
         return self.output(self.attend(self.project(x, step, view), step, view))
+
+    def last_weight(self):
+        return self.w_o
+
+    def takes_unscaled(self, tokens):
+        return (speaks_for(self.position, "takes_unscaled", "project_encode_store")
+                and self.position.takes_unscaled(tokens, self.w_qkv, self.heads, self.kv_heads, self.head_dim))
+
+    def forward_product(self, x, step, view):
+        if view.v.shape[1:3] != (self.kv_heads, self.head_dim):
+            raise ValueError("the attention mixer needs values of the keys' head count and head size")
+        return Product(self.attend(self.project(x, step, view), step, view), self.w_o)
 
     def project(self, x, step, view):
         """q, k, v of the step's tokens, q and k encoded by position, k and v stored in the cache."""

@@ -133,6 +133,27 @@ class Joining:
     vec: torch.Tensor = None
 
 
+@dataclass
+class Product:
+    """A sublayer's result whose last matrix product has not run yet: x [tokens, K] @ w^T (w a LinearWeight).  Blocks hand it to one
+    another where the product runs together with the norm in front of the next sublayer (parts/block.py)."""
+    x: torch.Tensor
+    w: object
+
+
+@dataclass
+class Unscaled:
+    """A norm's rows without its factor per row: y = (h + delta) * gamma in the activation dtype, and sums (float32 [tokens, n]), parts of
+    the sums of (h + delta)^2.  The product that reads y multiplies its float sums by 1 / sqrt(mean + eps)."""
+    y: torch.Tensor
+    sums: torch.Tensor
+    eps: float
+
+    @property
+    def scale(self):
+        return self.sums, self.eps
+
+
 class Part:
     # True if forward() only launches work on the current stream from device-side data, so that a
     # decode step through this part can be captured into a HIP graph and replayed.  A part that
@@ -169,15 +190,21 @@ class Norm(Part):
         return None
 
 
-def forward_goes_beside(part):
-    """Whether a part's forward_beside is its class's own word on what forward does: a subclass that brings another forward, and
-    nothing beside it, is called by that."""
+def speaks_for(part, word, *about):
+    """Whether a part's method `word` is its class's own word on what the methods `about` do: a subclass (or an object) that brings
+    another of those, and no `word` beside it, is called by them."""
+    if any(a in vars(part) for a in about):
+        return False
     for c in type(part).__mro__:
-        if "forward_beside" in vars(c):
+        if word in vars(c):
             return True
-        if "forward" in vars(c):
+        if any(a in vars(c) for a in about):
             return False
     return False
+
+
+def forward_goes_beside(part):
+    return speaks_for(part, "forward_beside", "forward")
 
 
 class Mixer(Part):
@@ -209,6 +236,16 @@ class Mixer(Part):
         self.w_in = self.rt.weight(torch.cat([own.w, weight.w], dim=0))
         return self.rt.weight(self.w_in.w[self.beside_at:])
 
+    # A mixer or a feed-forward may do without the kernel of a norm beside it, in steps of few tokens (parts/block.py):
+    # * last_weight() is the LinearWeight of its last product (None: it has none to hand on), and forward_product(...) in place of
+    #   forward(...) is a Product of it;
+    # * where takes_unscaled(tokens) says so, the x of forward and forward_product may be Unscaled.
+    def last_weight(self):
+        return None
+
+    def takes_unscaled(self, tokens):
+        return False
+
     def forward_terms(self, x, step, view):
         """The result as a list of Term whose sum it is; a mixer made of several may hand them on one by one."""
         return [Term(self.forward(x, step, view))]
@@ -217,6 +254,12 @@ class Mixer(Part):
 class FeedForward(Part):
     def forward(self, x, step):
         raise NotImplementedError
+
+    def last_weight(self):       # as a mixer's
+        return None
+
+    def takes_unscaled(self, tokens):
+        return False
 
     def forward_terms(self, x, step):
         """The result as a list of Term whose sum it is."""
@@ -238,6 +281,10 @@ class PositionEncoding(Part):
         rows): returns (w_q, w_k, encoding) to use from then on.  An encoding may hand back
         re-ordered rows and a variant of itself that computes the same function on them."""
         return w_q, w_k, self
+
+    def takes_unscaled(self, tokens, w_qkv, heads, kv_heads, head_dim):
+        """Whether project_encode_store takes an Unscaled x of that many tokens."""
+        return False
 
     def project_encode_store(self, x, w_qkv, step, view, heads, kv_heads, head_dim):
         """x @ w_qkv^T, then encode q and k by position and store k, v (unless view.store is

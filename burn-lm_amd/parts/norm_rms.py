@@ -38,6 +38,10 @@ class RMSNorm(Norm):
     def rms_constants(self):
         return self.gamma, self.eps
 
+    def joining(self):
+        """(gamma in float32, eps) for a product that adds its result to the residual and leaves the norm's rows unscaled."""
+        return self.gamma32, self.eps
+
     def post(self, terms):
         """A sublayer's results with this norm behind their sum, for the next norm's add."""
         return Joining(terms, self.gamma32, self.eps)

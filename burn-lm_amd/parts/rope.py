@@ -26,7 +26,7 @@ import math
 import numpy as np
 import torch
 
-from .base import PositionEncoding
+from .base import PositionEncoding, Unscaled
 
 PAIRING = {"interleaved": 0, "half": 1}
 
@@ -129,6 +129,13 @@ class RotaryEncoding(PositionEncoding):
                                   view.k, view.v, view.page_size, heads, kv_heads, head_dim, self.pairing,
                                   write_kv=store)
 
+    def takes_unscaled(self, tokens, w_qkv, heads, kv_heads, head_dim):
+        """The packed kernels of few rows do, bfloat16 and float32."""
+        rt = self.rt
+        if not hasattr(rt, "qkv_takes_unscaled") or self.pairing != PAIRING["interleaved"]:
+            return False
+        return rt.qkv_takes_unscaled(tokens, w_qkv, head_dim)
+
     def project_encode_store(self, x, w_qkv, step, view, heads, kv_heads, head_dim):
         """Projection, rotation and cache write in one kernel (the rotation applied to the float
         accumulators) where the runtime has a fused geometry for these sizes and this encoding's kernel
@@ -136,6 +143,7 @@ class RotaryEncoding(PositionEncoding):
         runtime's answer (Runtime.qkv_plan); what is checked here is only what the rotation itself needs."""
         rt = self.rt
         self._check_pairs()
+        x, scale = (x.y, x.scale) if isinstance(x, Unscaled) else (x, None)
         M, K = x.shape
         n_qkv = (heads + 2 * kv_heads) * head_dim
         plan = rt.qkv_plan(M, n_qkv, K) if hasattr(rt, "qkv_plan") else None
@@ -156,6 +164,8 @@ class RotaryEncoding(PositionEncoding):
                 and hasattr(rt, "f32_qkv_packed")):
             packed = rt.f32_qkv_packed(x, w_qkv, M, n_qkv, K)
             fused = "float32" if packed is not None else None
+        if scale is not None and fused not in ("packed", "float32"):
+            raise ValueError(f"rotary encoding: unscaled rows for a projection that does not take them ({M} rows, {fused})")
         if fused is None:
             return super().project_encode_store(x, w_qkv, step, view, heads, kv_heads, head_dim)
         if step.max_position >= self.n_positions:
@@ -163,7 +173,7 @@ class RotaryEncoding(PositionEncoding):
         if fused == "float32":
             return rt.ops.gemv_f32_qkv_rope(x, packed, torch.empty(M, n_qkv, dtype=torch.float32, device=x.device), step.positions,
                                             step.token_seq, view.block_table(step), self.table, view.k, view.v, view.page_size, heads,
-                                            kv_heads, head_dim, write_kv=view.store)
+                                            kv_heads, head_dim, write_kv=view.store, scale=scale)
         qkv = torch.empty(M, n_qkv, dtype=torch.bfloat16, device=x.device)
         if fused == "tiles":
             if not rt.ops.gemm_duo_takes(x, raw, qkv):
@@ -176,4 +186,4 @@ class RotaryEncoding(PositionEncoding):
                                              columns=plan.columns, rows=plan.rows)
         return rt.ops.gemv_qkv_rope(x, w_qkv.packed, qkv, step.positions, step.token_seq, view.block_table(step),
                                     self.table, view.k, view.v, view.page_size, heads, kv_heads, head_dim,
-                                    self.pairing, write_kv=view.store)
+                                    self.pairing, write_kv=view.store, scale=scale)

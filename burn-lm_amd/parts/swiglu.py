@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import torch
 
-from .base import FeedForward, TensorSpec
+from .base import FeedForward, Product, TensorSpec
 
 
 class SwiGLU(FeedForward):
@@ -38,3 +38,12 @@ class SwiGLU(FeedForward):
     def forward(self, x, step):
         rt = self.rt
         return rt.linear(rt.gated_linear(x, self.w_gate_up), self.w_down, partials=True)
+
+    def last_weight(self):
+        return self.w_down
+
+    def takes_unscaled(self, tokens):
+        return self.rt.gated_takes_unscaled(tokens, self.w_gate_up)
+
+    def forward_product(self, x, step):
+        return Product(self.rt.gated_linear(x, self.w_gate_up), self.w_down)
