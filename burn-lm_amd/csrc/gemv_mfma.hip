@@ -37,12 +37,63 @@ __device__ __forceinline__ float gv_gate(float g, int c_mode) {
   return g / (1.0f + expf(-g));
 }
 
-// SCALED: the rows come unscaled (row_scale.h), that many of them to a wavefront.
-template <int KSTEPS, int MAXT, bool KEEP_A, int SCALED, typename TC>
+// Experts stacked along the columns of a gated product, expert e at pairs e * ffe (a shared expert behind them has the weight at E): a
+// row's weight for the pair's expert multiplies what the gating gives, and is zero for the experts that the row did not choose.  The
+// weights lie in an array, or a table of the row's token names the experts (each with the weight 1 / top): token ids[m], or
+// (*source)[source_rows[m]] where that row number is not negative; a token outside the table chooses none.
+#define GE_ROWS 16
+#define GE_TOP 16
+struct GvExperts {
+  const float* weights;      // [M, E + 1]; null: by the table
+  const int *table, *ids, *source_rows;
+  const int* const* source;
+  int V, top, E, ffe;
+};
+
+// The table's entries for four rows from row0 on, to chosen [GE_ROWS][GE_TOP] (-1: none).  By scalar loads, which do not queue up behind the
+// weights' as vector loads would: their four trips to memory, one behind the other, end before the weights have come.
+__device__ __forceinline__ void ge_look_up(const GvExperts& ex, int M, int row0, int lane, int* chosen) {
+  typedef const __attribute__((address_space(4))) int* scalar_ints;
+  typedef const __attribute__((address_space(4))) uint64_t* scalar_pointer;
+  const scalar_ints ids = (scalar_ints)(uint64_t)ex.ids, table = (scalar_ints)(uint64_t)ex.table;
+  const uint64_t source = ex.source != nullptr ? *(scalar_pointer)(uint64_t)ex.source : 0;
+  int id[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) id[r] = ids[min(row0 + r, M - 1)];
+  if (source != 0) {
+    int from[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) from[r] = ((scalar_ints)(uint64_t)ex.source_rows)[min(row0 + r, M - 1)];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (from[r] >= 0) id[r] = ((scalar_ints)source)[from[r]];       // (without such a row the cell may hold an array that is gone)
+  }
+  for (int k0 = 0; k0 < ex.top; k0 += 4) {
+    int entry[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const bool good = (unsigned)id[i >> 2] < (unsigned)ex.V;
+      entry[i] = table[(size_t)(good ? id[i >> 2] : 0) * ex.top + min(k0 + (i & 3), ex.top - 1)];
+      if (!good) entry[i] = -1;
+    }
+    int mine = entry[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mine = lane == i ? entry[i] : mine;
+    if (lane < 16) chosen[(row0 + (lane >> 2)) * GE_TOP + k0 + (lane & 3)] = mine;
+  }
+}
+
+// SCALED: the rows come unscaled (row_scale.h), that many of them to a wavefront.  EXPERTS (c_mode 1): see GvExperts; 1:
+// weights from the array, 2: by the table.  In place of two
+// kernels around the product, a table's look-up and the gating: a decode step of eight rows through six layers of 16 experts of 512 at
+// width 2048 548 -> 521 us, 5 to 6 us a layer for kernels of 2.5 to 3 each.  (The look-up by vector loads, which wait for the weights in front
+// of them, and both forms' epilogues in one kernel, where every tile waits for the next one's weights: 533.)
+template <int KSTEPS, int MAXT, bool KEEP_A, int SCALED, int EXPERTS, typename TC>
 __global__ void __launch_bounds__(MAXT)
     gemv_mfma_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, TC* __restrict__ C, int M, int N,
-                     int K, int lda, int ldc, int n_tiles, int k_steps, int c_mode, int steps_per_group, RowScale scale) {
+                     int K, int lda, int ldc, int n_tiles, int k_steps, int c_mode, int steps_per_group, RowScale scale, GvExperts ex) {
   extern __shared__ float red[];  // [waves][256]
+  __shared__ int chosen[EXPERTS == 2 ? GE_ROWS * GE_TOP : 1];
   __shared__ float inv[RS_ROWS];
   RowScaleLoad<SCALED ? SCALED : 1> scale_load;
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
@@ -107,6 +158,8 @@ __global__ void __launch_bounds__(MAXT)
   }
   __builtin_amdgcn_sched_barrier(0);
   if (SCALED) scale_load.finish(scale, M, wave, n_waves, lane, inv);
+  if (EXPERTS == 2)      // (rows past the last are the last once more)
+    for (int r = __builtin_amdgcn_readfirstlane(wave) * 4; r < min(M, GE_ROWS); r += n_waves * 4) ge_look_up(ex, M, r, lane, chosen);
   if (KEEP_A) GV_ZERO_ACTIVATIONS()
 #undef GV_LOAD_ACTIVATIONS
 #undef GV_ZERO_ACTIVATIONS
@@ -196,7 +249,18 @@ __global__ void __launch_bounds__(MAXT)
             u *= inv[m];
           }
           const int nn = tile * 8 + col;
-          if (m < M && nn < N / 2) C[(size_t)m * ldc + nn] = from_float<TC>(gv_gate(g, c_mode) * u);
+          if (EXPERTS) {
+            const int e = min(nn / ex.ffe, ex.E);
+            float share = 0.f;
+            if (EXPERTS == 2) {
+              for (int k = 0; k < ex.top; ++k) share = chosen[m * GE_TOP + k] == e ? 1.0f / (float)ex.top : share;
+            } else {
+              share = ex.weights[(size_t)min(m, M - 1) * (ex.E + 1) + e];
+            }
+            if (m < M && nn < N / 2) C[(size_t)m * ldc + nn] = from_float<TC>(share != 0.f ? gv_gate(g, c_mode) * u * share : 0.f);
+          } else if (m < M && nn < N / 2) {
+            C[(size_t)m * ldc + nn] = from_float<TC>(gv_gate(g, c_mode) * u);
+          }
         }
       }
       __syncthreads();
@@ -212,10 +276,10 @@ __global__ void __launch_bounds__(MAXT)
 // current tile is multiplied and reduced (and the first tile's before the activations), so the
 // memory pipeline never idles while the block synchronises; with 16 k-steps the registers do not
 // allow it.
-template <int MT, int KSTEPS, bool PREFETCH, typename TC>
+template <int MT, int KSTEPS, bool PREFETCH, bool EXPERTS, typename TC>
 __global__ void __launch_bounds__(512)
     gemv_mfma_rows_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, TC* __restrict__ C, int M, int N,
-                          int K, int lda, int ldc, int n_tiles, int k_steps, int c_mode, int steps_per_group) {
+                          int K, int lda, int ldc, int n_tiles, int k_steps, int c_mode, int steps_per_group, GvExperts ex) {
   extern __shared__ float red[];  // [waves][MT][256]
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
   const int n_waves = blockDim.x / BLM_WAVE;
@@ -291,13 +355,16 @@ __global__ void __launch_bounds__(512)
         const int nn = tile * 16 + col;
         if (m < M && nn < N) C[(size_t)m * ldc + nn] = from_float<TC>(s);
       } else if (col < 8) {
-        float g = 0.f, u = 0.f;
+        float g = 0.f, u = 0.f, share = 1.0f;
+        const int nn = tile * 8 + col;
+        if (EXPERTS) share = ex.weights[(size_t)min(m, M - 1) * (ex.E + 1) + min(nn / ex.ffe, ex.E)];
         for (int w2 = 0; w2 < n_waves; ++w2) {
           g += red[(w2 * MT + mt) * 256 + i];
           u += red[(w2 * MT + mt) * 256 + i + 8];
         }
-        const int nn = tile * 8 + col;
-        if (m < M && nn < N / 2) C[(size_t)m * ldc + nn] = from_float<TC>(gv_gate(g, c_mode) * u);
+        if (EXPERTS) {
+          if (m < M && nn < N / 2) C[(size_t)m * ldc + nn] = from_float<TC>(share != 0.f ? gv_gate(g, c_mode) * u * share : 0.f);
+        } else if (m < M && nn < N / 2) C[(size_t)m * ldc + nn] = from_float<TC>(gv_gate(g, c_mode) * u);
       }
     }
     __syncthreads();
@@ -370,7 +437,7 @@ extern "C" int blm_gemv_mfma_geometry(int M, int N, int K, int k_groups, int* bl
 
 template <typename TC>
 static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int ldc, int c_mode,
-                       int k_groups, const RowScale* scale, hipStream_t stream) {
+                       int k_groups, const RowScale* scale, const GvExperts* experts, hipStream_t stream) {
   const int n_tiles = (N + 15) / 16;
   const int k_steps = (K + 31) / 32;
   const int steps_per_group = (k_steps + k_groups - 1) / k_groups;
@@ -381,28 +448,37 @@ static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int
     dim3 grid(blocks, k_groups), block(waves * BLM_WAVE);
     const size_t smem = (size_t)waves * mt * 256 * sizeof(float);
 #define BLM_GR(MT, KS, PF)                                                                                      \
-  hipLaunchKernelGGL((gemv_mfma_rows_kernel<MT, KS, PF, TC>), grid, block, smem, stream, (const bf16*)A,        \
-                     (const bf16*)Wp, (TC*)C, M, N, K, lda, ldc, n_tiles, k_steps, c_mode, steps_per_group)
+  do {                                                                                                          \
+    if (experts) BLM_GRE(MT, KS, PF, true, *experts);                                                           \
+    else BLM_GRE(MT, KS, PF, false, GvExperts{});                                                               \
+  } while (0)
+#define BLM_GRE(MT, KS, PF, EXPERTS, EX)                                                                        \
+  hipLaunchKernelGGL((gemv_mfma_rows_kernel<MT, KS, PF, EXPERTS, TC>), grid, block, smem, stream, (const bf16*)A, \
+                     (const bf16*)Wp, (TC*)C, M, N, K, lda, ldc, n_tiles, k_steps, c_mode, steps_per_group, EX)
     if (ks == 16) BLM_GR(2, 16, false);
     else if (mt == 2) BLM_GR(2, 8, true);
     else if (mt == 3) BLM_GR(3, 8, true);
     else BLM_GR(4, 8, true);
 #undef BLM_GR
+#undef BLM_GRE
     BLM_LAUNCH_CHECK("gemv_mfma_rows");
     return 0;
   }
   const int ksteps = geo.ksteps, waves = geo.waves, blocks = geo.blocks;
   dim3 grid(blocks, k_groups), block(waves * BLM_WAVE);
   const size_t smem = (size_t)waves * 256 * sizeof(float);
-#define BLM_GS(KS, MAXT, KEEP, SCALED, SCALE)                                                                   \
-  hipLaunchKernelGGL((gemv_mfma_kernel<KS, MAXT, KEEP, SCALED, TC>), grid, block, smem, stream, (const bf16*)A, \
-                     (const bf16*)Wp, (TC*)C, M, N, K, lda, ldc, n_tiles, k_steps, c_mode, steps_per_group, SCALE)
+#define BLM_GS(KS, MAXT, KEEP, SCALED, SCALE, EXPERTS, EX)                                                      \
+  hipLaunchKernelGGL((gemv_mfma_kernel<KS, MAXT, KEEP, SCALED, EXPERTS, TC>), grid, block, smem, stream,        \
+                     (const bf16*)A, (const bf16*)Wp, (TC*)C, M, N, K, lda, ldc, n_tiles, k_steps, c_mode,      \
+                     steps_per_group, SCALE, EX)
 #define BLM_GM(KS, MAXT, KEEP)                                                                                  \
   do {                                                                                                          \
-    if (scale == nullptr) BLM_GS(KS, MAXT, KEEP, 0, RowScale{});                                                \
-    else if (M <= waves) BLM_GS(KS, MAXT, KEEP, 1, *scale);                                                     \
-    else if (M <= 2 * waves) BLM_GS(KS, MAXT, KEEP, 2, *scale);                                                 \
-    else BLM_GS(KS, MAXT, KEEP, RS_SLOTS, *scale);                                                              \
+    if (experts && experts->weights) BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 1, *experts);                        \
+    else if (experts) BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 2, *experts);                                       \
+    else if (scale == nullptr) BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 0, GvExperts{});                       \
+    else if (M <= waves) BLM_GS(KS, MAXT, KEEP, 1, *scale, 0, GvExperts{});                                 \
+    else if (M <= 2 * waves) BLM_GS(KS, MAXT, KEEP, 2, *scale, 0, GvExperts{});                             \
+    else BLM_GS(KS, MAXT, KEEP, RS_SLOTS, *scale, 0, GvExperts{});                                          \
   } while (0)
   if (ksteps == 4) BLM_GM(4, 256, true);
   else if (ksteps == 16 && waves <= 4) BLM_GM(16, 256, true);
@@ -424,7 +500,7 @@ static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int
 // [k_groups, M, ldc] and holds one partial product per group, to be summed by the reader (the
 // residual add in front of the next norm does it), so narrow outputs still occupy the whole chip.
 static int gemv_mfma_entry(const void* A, const void* Wp, void* C, int c_dtype, int M, int N, int K, int lda,
-                             int ldc, int c_mode, int k_groups, const RowScale* scale, hipStream_t stream) {
+                             int ldc, int c_mode, int k_groups, const RowScale* scale, const GvExperts* experts, hipStream_t stream) {
   BLM_REQUIRE(M >= 1 && M <= 64, "gemv_mfma: M=%d out of range 1..64", M);
   BLM_REQUIRE(N >= 1 && K >= 8 && K % 8 == 0, "gemv_mfma: sizes N=%d K=%d not supported (K a multiple of 8)", N, K);
   BLM_REQUIRE(c_mode == 0 || ((c_mode == 1 || c_mode == 2) && N % 16 == 0 && k_groups == 1),
@@ -439,14 +515,14 @@ static int gemv_mfma_entry(const void* A, const void* Wp, void* C, int c_dtype, 
   }
   BLM_REQUIRE(lda % 8 == 0 && lda >= K && ldc >= (c_mode ? N / 2 : N), "gemv_mfma: bad strides lda=%d ldc=%d", lda, ldc);
   BLM_REQUIRE(((uintptr_t)A % 16) == 0 && ((uintptr_t)Wp % 16) == 0, "gemv_mfma: operands must be 16-byte aligned");
-  if (c_dtype == BLM_BF16) return launch_mfma<bf16>(A, Wp, C, M, N, K, lda, ldc, c_mode, k_groups, scale, stream);
-  if (c_dtype == BLM_F32) return launch_mfma<float>(A, Wp, C, M, N, K, lda, ldc, c_mode, k_groups, scale, stream);
+  if (c_dtype == BLM_BF16) return launch_mfma<bf16>(A, Wp, C, M, N, K, lda, ldc, c_mode, k_groups, scale, experts, stream);
+  if (c_dtype == BLM_F32) return launch_mfma<float>(A, Wp, C, M, N, K, lda, ldc, c_mode, k_groups, scale, experts, stream);
   return blm_fail("gemv_mfma: unsupported output dtype %d", c_dtype);
 }
 
 extern "C" int blm_gemv_mfma(const void* A, const void* Wp, void* C, int c_dtype, int M, int N, int K, int lda,
                              int ldc, int c_mode, int k_groups, hipStream_t stream) {
-  return gemv_mfma_entry(A, Wp, C, c_dtype, M, N, K, lda, ldc, c_mode, k_groups, nullptr, stream);
+  return gemv_mfma_entry(A, Wp, C, c_dtype, M, N, K, lda, ldc, c_mode, k_groups, nullptr, nullptr, stream);
 }
 
 // The same of up to eight rows that come unscaled: sums [M, n_sums] holds parts of the rows' sums of squares, and the product's row m is
@@ -455,5 +531,20 @@ extern "C" int blm_gemv_mfma_scaled(const void* A, const void* Wp, void* C, int 
                                     int c_mode, const float* sums, int n_sums, float eps, hipStream_t stream) {
   BLM_REQUIRE(row_scale_fits(M, sums, n_sums), "gemv_mfma_scaled: M=%d with %d sums a row", M, n_sums);
   const RowScale scale{sums, n_sums, 1.0f / (float)K, eps};
-  return gemv_mfma_entry(A, Wp, C, c_dtype, M, N, K, lda, ldc, c_mode, 1, &scale, stream);
+  return gemv_mfma_entry(A, Wp, C, c_dtype, M, N, K, lda, ldc, c_mode, 1, &scale, nullptr, stream);
+}
+
+// The gated product (silu) of experts stacked along the columns, weighted (GvExperts): W packed as for c_mode 1, E experts of ffe pairs
+// and a shared one behind them if N / 2 is more.  weights [M, E + 1], or null and a table [V, top] of up to 16 rows.
+extern "C" int blm_gemv_experts(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int ldc, int E, int ffe,
+                                const float* weights, const int* table, const int* ids, const int* source_rows, const void* source_cell,
+                                int V, int top, hipStream_t stream) {
+  BLM_REQUIRE(E > 0 && ffe > 0 && (long long)E * ffe <= N / 2, "gemv_experts: %d experts of %d in %d pairs", E, ffe, N / 2);
+  if (weights == nullptr) {
+    BLM_REQUIRE(table != nullptr && ids != nullptr && V > 0 && top > 0 && top <= GE_TOP && M <= GE_ROWS && E * ffe == N / 2,
+                "gemv_experts: a table of up to %d experts a token, for up to %d rows", GE_TOP, GE_ROWS);
+    BLM_REQUIRE((source_rows == nullptr) == (source_cell == nullptr), "gemv_experts: rows and cell of a token source come together");
+  }
+  const GvExperts experts{weights, weights ? nullptr : table, ids, source_rows, (const int* const*)source_cell, V, top, E, ffe};
+  return gemv_mfma_entry(A, Wp, C, BLM_BF16, M, N, K, lda, ldc, 1, 1, nullptr, &experts, stream);
 }

@@ -11,7 +11,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 46
+ABI_VERSION = 47
 _lib = None
 _lock = threading.Lock()
 
@@ -153,6 +153,7 @@ _SIGNATURES = {
                         _c_int, _c_int, _c_void_p],
     "blm_gemv_mfma": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                       _c_int, _c_void_p],
+    "blm_gemv_experts": [_c_void_p] * 3 + [_c_int] * 7 + [_c_void_p] * 5 + [_c_int, _c_int, _c_void_p],
     "blm_gemv_mfma_supported": [_c_int, _c_int, _c_int],
     "blm_gemv_mfma_geometry": [_c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p],
     "blm_gemm_mfma_init": [],
@@ -819,6 +820,41 @@ def gemv_mfma(a, packed, out, K, gated=False, activation="silu", scale=None):
         return out
     _call("blm_gemv_mfma", a.data_ptr(), packed.data_ptr(), out.data_ptr(), _code(out), M, N, K, a.stride(0),
           out.stride(-2), mode, groups, _stream())
+    return out
+
+
+EXPERT_TABLE_ROWS, EXPERT_TABLE_TOP = 16, 16
+
+
+def gemv_experts(x, packed, out, n_experts, expert_inner, weights=None, table=None, ids=None, token_source=None):
+    """out [M, I] = silu(x gate^T) * (x up^T) * (the row's weight for the pair's expert), from packed = pack_weight(w, gated=True) of a
+    [2 I, K] matrix whose pairs are experts of expert_inner each, one behind the other (a shared one behind them has the weight at E);
+    zero where the weight is.  weights: float32 [M, E + 1]; or a table (int32 [vocabulary, top]) that names the experts of the tokens ids
+    [M] (token_source: see moe_table), each with the weight 1 / top, for up to 16 rows and experts a row.  bfloat16, M <= 64."""
+    _gpu(x, packed, out, weights, table, ids)
+    M, K = x.shape
+    I = out.shape[1]
+    if x.dtype != torch.bfloat16 or packed.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or out.shape[0] != M:
+        raise KernelError("gemv_experts: bfloat16 operands wanted, out [M, I]")
+    if packed.numel() != -(-2 * I // 16) * -(-K // 32) * 512 or not packed.is_contiguous() or x.stride(1) != 1 or out.stride(1) != 1:
+        raise KernelError(f"gemv_experts: the packed weights are not those of a [{2 * I}, {K}] matrix, or rows without unit stride")
+    if (weights is None) == (table is None):
+        raise KernelError("gemv_experts: weights or a table")
+    rows = cell = None
+    if weights is not None:
+        _f32("weights", weights, M * (n_experts + 1))
+    else:
+        _i32("table", table); _i32("ids", ids, M)
+        if table.dim() != 2:
+            raise KernelError("gemv_experts: table [vocabulary, top]")
+        if token_source is not None:
+            rows, cell = token_source
+            _i32("source_rows", rows, M)
+            if cell.dtype != torch.int64 or cell.numel() != 1:
+                raise KernelError("gemv_experts: the cell is one int64 on the device")
+    V, top = (0, 0) if table is None else table.shape
+    _call("blm_gemv_experts", x.data_ptr(), packed.data_ptr(), out.data_ptr(), M, 2 * I, K, x.stride(0), out.stride(0), n_experts,
+          expert_inner, _ptr(weights), _ptr(table), _ptr(ids), _ptr(rows), _ptr(cell), V, top, _stream())
     return out
 
 

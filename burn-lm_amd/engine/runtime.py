@@ -623,6 +623,13 @@ class Runtime:
         sums = torch.empty(M, N // ops.gemv_join_columns(w.dtype, M, N, K), dtype=torch.float32, device=x.device)
         return Unscaled(ops.gemv_join(x, w.packed, h, gamma, y, sums, K), sums, eps)
 
+    def experts_take(self, x, w):
+        """Whether the gated product of stacked experts runs with their weights in its epilogue (ops.gemv_experts): where the packed kernel
+        takes the rows.  Elsewhere it is a product and a pass."""
+        return (isinstance(w, LinearWeight) and w.gated and w.packable and x.dtype == w.dtype == torch.bfloat16
+                and x.shape[0] <= MFMA_SKINNY_MAX_ROWS and bool(ops.gemv_mfma_supported(x.shape[0], *w.shape))
+                and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0)
+
     def gated_takes_unscaled(self, M, w):
         """Whether gated_linear takes M Unscaled rows: where its packed kernels have them."""
         if not (isinstance(w, LinearWeight) and w.gated and w.packable and M <= ops.SCALED_ROWS and w.dtype == self.dtype):

@@ -5,7 +5,8 @@ expert of the same form may run for every token, times ``sigmoid(W_sg x)`` (one 
 The router's logits, the choice and the weights are float32.  In steps of few rows all experts run as ONE stacked product:
 their gate and up projections are the rows of one matrix, their down projections the columns of another, and every expert's
 gated activations are multiplied by the token's weight for that expert (zero for experts it did not choose)
-before the one down projection, which so adds the chosen experts' outputs up.  That computes every expert for
+before the one down projection, which so adds the chosen experts' outputs up (up to 64 rows in the gate/up product's own
+epilogue, ``ops.gemv_experts``).  That computes every expert for
 every token, and reads the same weights as a batch that uses every expert.
 
 In steps of many rows of experts without clamps and without a shared one, every token goes through its own experts only
@@ -65,7 +66,7 @@ class RoutedExperts(FeedForward):
         if len({w.dtype for w in ws}) != 1:
             gates, ups, downs = ([w.float() for w in group] for group in (gates, ups, downs))
         self.inner = self.E * self.f + self.s
-        self.w_gate_up = rt.weight(torch.cat(gates + ups, dim=0))
+        self.w_gate_up = self._stacked(gates, ups)
         self.w_down = rt.weight(torch.cat(downs, dim=1).contiguous())
         router = [t("router")] + ([t("shared.sg")] if self.s else [])
         if len({w.dtype for w in router}) != 1:
@@ -76,6 +77,13 @@ class RoutedExperts(FeedForward):
             router.append(torch.zeros(pad, router[0].shape[1], dtype=router[0].dtype, device=router[0].device))
         self.w_router = rt.weight(torch.cat(router, dim=0))
         self.router_bias = t("router_bias").float().contiguous()
+
+    def _stacked(self, gates, ups):
+        """All experts' gates and ups as one matrix.  In pairs where the product of few rows takes the gating and the experts' weights into
+        its epilogue (eight neighbouring pairs belong to one expert there)."""
+        w = torch.cat(gates + ups, dim=0)
+        pairs = self.rt.dtype == w.dtype == torch.bfloat16 and not self.clamped and self.f % 8 == 0 and self.s % 8 == 0
+        return self.rt.weight(w, gated=pairs)
 
     def step_bytes(self, rows):
         return sum(w.w.numel() * w.w.element_size() for w in (self.w_gate_up, self.w_down, self.w_router))
@@ -101,6 +109,9 @@ class RoutedExperts(FeedForward):
         bucket = getattr(step, "bucket", None)
         if self._grouped(bucket[0] if bucket else x.shape[0]) and x.is_contiguous() and x.data_ptr() % 16 == 0:
             return ops.moe_grouped(x, self.w_gate_up.w, self.w_down.w, weights, self.E, self.top)
+        if rt.experts_take(x, self.w_gate_up):
+            act = torch.empty(x.shape[0], self.inner, dtype=x.dtype, device=x.device)
+            return rt.linear(ops.gemv_experts(x, self.w_gate_up.packed, act, self.E, self.f, weights=weights), self.w_down, partials=True)
         gu = rt.linear(x, self.w_gate_up)
         act = torch.empty(x.shape[0], self.inner, dtype=gu.dtype, device=x.device)
         return rt.linear(ops.moe_gate(gu, weights, act, self.E, self.f), self.w_down, partials=True)
@@ -186,7 +197,7 @@ class GroupedRoutedExperts(RoutedExperts):
         if len({w.dtype for w in gates + ups + downs}) != 1:
             gates, ups, downs = ([w.float() for w in group] for group in (gates, ups, downs))
         self.inner = self.E * self.f + self.s
-        self.w_gate_up = rt.weight(torch.cat(gates + ups, dim=0))
+        self.w_gate_up = self._stacked(gates, ups)
         self.w_down = rt.weight(torch.cat(downs, dim=1).contiguous())
         router = t("router")
         pad = (-router.shape[0]) % 16
@@ -257,7 +268,7 @@ class TableExperts(RoutedExperts):
         if len({w.dtype for w in gates + ups + downs}) != 1:
             gates, ups, downs = ([w.float() for w in group] for group in (gates, ups, downs))
         self.inner = self.E * self.f
-        self.w_gate_up = rt.weight(torch.cat(gates + ups, dim=0))
+        self.w_gate_up = self._stacked(gates, ups)
         self.w_down = rt.weight(torch.cat(downs, dim=1).contiguous())
 
     def step_bytes(self, rows):
@@ -266,8 +277,17 @@ class TableExperts(RoutedExperts):
     def step_flops(self, rows):
         return self._expert_flops(rows)
 
+    def _by_table(self, x):
+        """Whether the product of the gates and ups looks the experts up itself."""
+        ops = self.rt.ops
+        return x.shape[0] <= ops.EXPERT_TABLE_ROWS and self.top <= ops.EXPERT_TABLE_TOP and self.rt.experts_take(x, self.w_gate_up)
+
     def forward(self, x, step):
         rt = self.rt
+        if self._by_table(x):
+            act = torch.empty(x.shape[0], self.inner, dtype=x.dtype, device=x.device)
+            rt.ops.gemv_experts(x, self.w_gate_up.packed, act, self.E, self.f, table=self.table, ids=step.token_ids, token_source=step.token_source)
+            return rt.linear(act, self.w_down, partials=True)
         weights = torch.empty(x.shape[0], self.E + 1, dtype=torch.float32, device=x.device)
         rt.ops.moe_table(self.table, step.token_ids, weights, self.E, step.token_source)
         return self._mix(x, weights, step)
