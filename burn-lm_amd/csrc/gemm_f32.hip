@@ -225,11 +225,17 @@ struct GvRope {
   int table_width, page_size, nh, nkv, hd, store;
 };
 
-// SCALED: the rows come unscaled (row_scale.h), that many of them to a wavefront.
-template <int KSTEPS, bool WHOLE, bool ROPE, int SCALED>
+// SCALED: the rows come unscaled (row_scale.h), that many of them to a wavefront.  ONE: every block has one tile.
+// The weights come by buffer loads of their tile's bytes: of none behind a block's last tile, where they bring zeros without a trip to memory.
+// With a branch around them the compiler counts on the way without them, and every part waits for the next part's loads too.
+// Us, eight rows, with the branch, selects of every activation and look-ups of the block's size / so: [3072, 2048] 9.2 / 8.1, [2048, 2048] in two groups
+// 6.8 / 6.1, [16384, 2048] gated 27.0 / 26.0, [2048, 8192] in four 16.3 / 15.1; the head [128256, 2048], 31 tiles a block, 163 / 166.
+// shape: 2 * wavefronts + gated, and the sums of a row that comes unscaled (the arguments' first fourteen dwords come in registers; a block's size would be a load).
+template <int KSTEPS, bool WHOLE, bool ROPE, bool ONE, int SCALED>
 __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
-    gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wp, float* __restrict__ C, int M, int N, int K,
-                    int lda, int ldc, int n_tiles, int k_steps, int gated, int steps_per_group, int tiles_per_block, GvRope rope, RowScale scale) {
+    gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wp, int M, int K, int lda, int n_tiles, int k_steps, int shape,
+                    int steps_per_group, int tiles_per_block, const float* __restrict__ sums, int N, int ldc, float* __restrict__ C, GvRope rope,
+                    float inv_width, float eps) {
   __shared__ float red[GV_MAX_WAVES * 256];
   __shared__ float inv[RS_ROWS];
   RowScaleLoad<SCALED ? SCALED : 1> scale_load;
@@ -241,41 +247,49 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
     my_seq = rope.token_seq[m];
   }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / BLM_WAVE), lane = threadIdx.x & (BLM_WAVE - 1);
-  const int n_waves = blockDim.x / BLM_WAVE;
+  const int n_waves = (shape >> 1) & 31, gated = shape & 1, n_sums = shape >> RS_SHIFT;
   const int row = lane & 15, kg = lane >> 4;
   const int group_begin = blockIdx.y * steps_per_group, group_end = min(k_steps, group_begin + steps_per_group);
   const int step0 = group_begin + wave * KSTEPS;
   const int kbase = step0 * 16 + kg * 4;
   C += (size_t)blockIdx.y * M * ldc;
-  const float* ap = A + (size_t)min(row, M - 1) * lda;   // rows past the last read it again and are zeroed
+  const float* ap = A + (size_t)min(row, M - 1) * lda;   // rows past the last are it once more; their sums go nowhere
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   // activations first, then the first tile's weights behind them, all asked for before any is looked at; weights behind the end
   // of the group are some other step's (a step past the matrix is its last), and they and their activations count as zeros
   f32x4 a[KSTEPS];
-  if (SCALED) scale_load.ask(scale, M, wave, n_waves, lane);
+  if (SCALED) scale_load.ask(sums, n_sums, M, wave, n_waves, lane);
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) a[s] = *reinterpret_cast<const f32x4*>(ap + min(kbase + s * 16, K - 4));
   const int tile_begin = blockIdx.x * tiles_per_block, tile_end = min(n_tiles, tile_begin + tiles_per_block);
   constexpr int PART = KSTEPS >= 16 ? 8 : 2, PARTS = KSTEPS / PART;      // steps whose weights wait in one set of registers
-  auto weights = [&](int tile, int part, f32x4* w) {
-    const float* wt = Wp + ((size_t)tile * k_steps * 64 + lane) * 4;
+  const int wfirst = step0 * 1024 + lane * 16;
+  auto tile_bytes = [&](int tile, bool there) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(Wp + (size_t)tile * k_steps * 256), 0, there ? k_steps * 1024 : 0, 0x00027000);
+  };
+  auto weights = [&](auto bytes, int part, f32x4* w) {
 #pragma unroll
-    for (int s = 0; s < PART; ++s)
-      w[s] = __builtin_bit_cast(f32x4, load16_stream(wt + (size_t)(WHOLE ? step0 + part * PART + s : min(step0 + part * PART + s, k_steps - 1)) * 256));
+    for (int s = 0; s < PART; ++s) w[s] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(bytes, wfirst + (part * PART + s) * 1024, 0, 2));
   };
   f32x4 w[2][PART];
-  weights(tile_begin, 0, w[0]);
-  weights(tile_begin, 1, w[1]);
+  const auto first = tile_bytes(min(tile_begin, n_tiles - 1), true);
+  weights(first, 0, w[0]);
+  weights(first, 1, w[1]);
   __builtin_amdgcn_sched_barrier(0);
-  if (SCALED) scale_load.finish(scale, M, wave, n_waves, lane, inv);
+  if (SCALED) scale_load.finish(n_sums, inv_width, eps, M, wave, n_waves, lane, inv);
   if (ROPE && threadIdx.x < 16) {            // the barrier of the first tile's sum lies between these writes and their readers
     pos_of[threadIdx.x] = my_pos;
     page_of[threadIdx.x] = my_seq < 0 || !rope.store ? -1 : rope.block_table[(size_t)my_seq * rope.table_width + my_pos / rope.page_size];
   }
+  if (!WHOLE)
 #pragma unroll
-  for (int s = 0; s < KSTEPS; ++s) a[s] = row < M && kbase + s * 16 < K && step0 + s < group_end ? a[s] : zero;
-  for (int tile = tile_begin; tile < tile_end; ++tile) {
-    const bool more = tile + 1 < tile_end;
+    for (int s = 0; s < KSTEPS; ++s) {
+      const bool keep = (kbase + s * 16 < K) & (step0 + s < group_end);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[s][e] = keep ? a[s][e] : 0.f;
+    }
+  for (int tile = tile_begin; tile < (ONE ? min(tile_begin + 1, tile_end) : tile_end); ++tile) {
+    const auto here = tile_bytes(tile, true), next = tile_bytes(tile + 1, !ONE && tile + 1 < tile_end);
     f32x4 sum[PARTS];
 #pragma unroll
     for (int p = 0; p < PARTS; ++p) {
@@ -294,9 +308,11 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           acc[(s & 1) * 4 + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[p * PART + s][e], w[p & 1][s][e], acc[(s & 1) * 4 + e], 0, 0, 0);
+#pragma unroll
+      for (int x = 0; x < 8; ++x) asm volatile("" : "+v"(acc[x]) : : "memory");      // the new loads stay behind the products whose registers they take
       __builtin_amdgcn_sched_barrier(0);
-      if (p + 2 < PARTS) weights(tile, p + 2, w[p & 1]);
-      else if (more) weights(tile + 1, p + 2 - PARTS, w[p & 1]);
+      if (p + 2 < PARTS) weights(here, p + 2, w[p & 1]);
+      else if (!ONE) weights(next, p + 2 - PARTS, w[p & 1]);
 #pragma unroll
       for (int x = 4; x; x >>= 1)
 #pragma unroll
@@ -311,7 +327,7 @@ __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)
 #pragma unroll
     for (int r = 0; r < 4; ++r) red[wave * 256 + r * 64 + lane] = sum[0][r];
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    for (int idx = threadIdx.x; idx < 256; idx += blockDim.x) {
+    for (int idx = threadIdx.x; idx < 256; idx += n_waves * BLM_WAVE) {
       const int r = idx >> 6, l2 = idx & 63, col = l2 & 15, m = (l2 >> 4) * 4 + r;
       float s = 0.f, u = 0.f;
       if (!gated) {
@@ -394,9 +410,15 @@ static int gv_run(const void* A, const void* Wp, void* C, int M, int N, int K, i
   gemv_f32_geometry(N, K, groups, &ksteps, &waves, &blocks);
   const int per_block = (n_tiles + blocks - 1) / blocks;
   dim3 grid((unsigned)blocks, (unsigned)groups), block(waves * BLM_WAVE);
+#define BLM_GVO(KS, WHOLE, ROPE, ONE, SCALED, SCALE)                                                                    \
+  hipLaunchKernelGGL((gemv_f32_kernel<KS, WHOLE, ROPE, ONE, SCALED>), grid, block, 0, stream, (const float*)A, (const float*)Wp, M, K, \
+                     lda, n_tiles, k_steps, 2 * waves + (gated ? 1 : 0) + ((SCALE).n << RS_SHIFT), steps, per_block, (SCALE).sums, N, ldc, (float*)C,    \
+                     rope ? *rope : GvRope{}, (SCALE).inv_width, (SCALE).eps)
 #define BLM_GVS(KS, WHOLE, ROPE, SCALED, SCALE)                                                                         \
-  hipLaunchKernelGGL((gemv_f32_kernel<KS, WHOLE, ROPE, SCALED>), grid, block, 0, stream, (const float*)A, (const float*)Wp, (float*)C, M, \
-                     N, K, lda, ldc, n_tiles, k_steps, gated, steps, per_block, rope ? *rope : GvRope{}, SCALE)
+  do {                                                                                                                  \
+    if (per_block == 1) BLM_GVO(KS, WHOLE, ROPE, true, SCALED, SCALE);                                                  \
+    else BLM_GVO(KS, WHOLE, ROPE, false, SCALED, SCALE);                                                                \
+  } while (0)
 #define BLM_GVR(KS, WHOLE, ROPE)                                                                                        \
   do {                                                                                                                  \
     if (scale == nullptr) BLM_GVS(KS, WHOLE, ROPE, 0, RowScale{});                                                      \
@@ -416,6 +438,7 @@ static int gv_run(const void* A, const void* Wp, void* C, int M, int N, int K, i
 #undef BLM_GVF
 #undef BLM_GVR
 #undef BLM_GVS
+#undef BLM_GVO
   BLM_LAUNCH_CHECK("gemv_f32");
   return 0;
 }

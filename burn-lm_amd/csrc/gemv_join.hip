@@ -55,20 +55,21 @@ __device__ __forceinline__ f32x4_t gj_multiply(const gj_piece (&a)[CH], const gj
   return sum + acc[0];
 }
 
+// (What the first loads need stands in the arguments' first fourteen dwords, which come in registers.)
 // STEPS: steps along K per wavefront, of four fragments' 16 bytes (32 bfloat16, 16 float32), two at once with PAIR; CH: loaded at once; WHOLE: the
 // wavefronts' steps are all there
 template <typename T, bool PAIR, int STEPS, int CH, bool WHOLE>
 __global__ void __launch_bounds__(GJ_WAVES* BLM_WAVE)
-    gemv_join_kernel(const T* __restrict__ A, const T* __restrict__ Wp, float* __restrict__ h, const float* __restrict__ gamma,
-                     T* __restrict__ y, float* __restrict__ sums, int M, int N, int K, int lda, int k_steps, int columns) {
+    gemv_join_kernel(const T* __restrict__ A, const T* __restrict__ Wp, int M, int K, int lda, int k_steps, int columns, int blocks,
+                     int n_waves, int N, float* __restrict__ h, const float* __restrict__ gamma, T* __restrict__ y, float* __restrict__ sums) {
   constexpr int EACH = PAIR ? 2 : 1, NC = STEPS / CH, E = 16 / sizeof(T), STEP = 4 * E;
   __shared__ float red[GJ_WAVES][EACH][GJ_ROWS][16 / EACH];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / BLM_WAVE), lane = threadIdx.x & (BLM_WAVE - 1), n_waves = blockDim.x / BLM_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / BLM_WAVE), lane = threadIdx.x & (BLM_WAVE - 1);
   const int i16 = lane & 15, kg = lane >> 4;
   const int sub = PAIR ? i16 >> 3 : 0;                         // the step of a pair that this lane brings
   const int row = PAIR ? i16 & 7 : i16;                        // (rows past the last are the last once more; their sums go nowhere)
   // neighbouring blocks, which may share lines of the weights, on one die
-  const int block = gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
+  const int block = blocks % 8 == 0 ? (blockIdx.x % 8) * (blocks / 8) + blockIdx.x / 8 : blockIdx.x;
   const int n0 = block * columns, n = n0 + (PAIR ? i16 & 7 : min(i16, columns - 1));
   const T* wt = Wp + ((size_t)(n >> 4) * k_steps * 64 + kg * 16 + (n & 15)) * E;
   const T* ap = A + (size_t)min(row, M - 1) * lda;
@@ -129,7 +130,7 @@ __global__ void __launch_bounds__(GJ_WAVES* BLM_WAVE)
     if (own) {
       h[(size_t)om * N + n0 + oc] = t;
       y[(size_t)om * N + n0 + oc] = from_float<T>(t * g);
-      if (oc == 0) sums[(size_t)om * gridDim.x + block] = ss;
+      if (oc == 0) sums[(size_t)om * blocks + block] = ss;
     }
   }
 }
@@ -151,13 +152,13 @@ static void gj_launch(const void* A, const void* Wp, float* h, const float* gamm
 #define BLM_GJ(PAIR, STEPS, CH)                                                                                              \
   do {                                                                                                                       \
     const int per = STEPS * (PAIR ? 2 : 1), waves = (k_steps + per - 1) / per;                                               \
-    const dim3 grid(N / columns), block((waves < 2 ? 2 : waves) * BLM_WAVE);                                                 \
+    const int blocks = N / columns, at_work = waves < 2 ? 2 : waves;                                                         \
     if (waves > 1 && waves * per * step == K)                                                                                \
-      hipLaunchKernelGGL((gemv_join_kernel<T, PAIR, STEPS, CH, true>), grid, block, 0, stream, (const T*)A, (const T*)Wp, h, \
-                         gamma, (T*)y, sums, M, N, K, lda, k_steps, columns);                                                \
+      hipLaunchKernelGGL((gemv_join_kernel<T, PAIR, STEPS, CH, true>), dim3(blocks), dim3(at_work * BLM_WAVE), 0, stream,    \
+                         (const T*)A, (const T*)Wp, M, K, lda, k_steps, columns, blocks, at_work, N, h, gamma, (T*)y, sums); \
     else                                                                                                                     \
-      hipLaunchKernelGGL((gemv_join_kernel<T, PAIR, STEPS, CH, false>), grid, block, 0, stream, (const T*)A, (const T*)Wp, h, \
-                         gamma, (T*)y, sums, M, N, K, lda, k_steps, columns);                                                \
+      hipLaunchKernelGGL((gemv_join_kernel<T, PAIR, STEPS, CH, false>), dim3(blocks), dim3(at_work * BLM_WAVE), 0, stream,   \
+                         (const T*)A, (const T*)Wp, M, K, lda, k_steps, columns, blocks, at_work, N, h, gamma, (T*)y, sums); \
   } while (0)
   if (columns == 8) {
     if (k_steps <= 128) BLM_GJ(true, 8, 8);

@@ -22,6 +22,7 @@
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(4))) uint32_t gv_piece;      // 16 bytes
 
 __device__ __forceinline__ uint4 ld16(const bf16* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ uint4 ld16_stream(const bf16* p) { return load16_stream(p); }   // the weights: read once
@@ -88,16 +89,20 @@ __device__ __forceinline__ void ge_look_up(const GvExperts& ex, int M, int row0,
 // kernels around the product, a table's look-up and the gating: a decode step of eight rows through six layers of 16 experts of 512 at
 // width 2048 548 -> 521 us, 5 to 6 us a layer for kernels of 2.5 to 3 each.  (The look-up by vector loads, which wait for the weights in front
 // of them, and both forms' epilogues in one kernel, where every tile waits for the next one's weights: 533.)
-template <int KSTEPS, int MAXT, bool KEEP_A, int SCALED, int EXPERTS, typename TC>
+// shape: 4 * wavefronts + c_mode, and the sums of a row that comes unscaled.  What the first loads need stands in the arguments' first fourteen dwords, which come in registers;
+// what a kernel asks of its block's and grid's sizes would be a load in front of everything, and the tiles of a block a division.
+// ONE: every block has one tile (a last tile's loads of nothing are 0.5 us of such a short kernel).
+template <int KSTEPS, int MAXT, bool KEEP_A, bool ONE, int SCALED, int EXPERTS, typename TC>
 __global__ void __launch_bounds__(MAXT)
-    gemv_mfma_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, TC* __restrict__ C, int M, int N,
-                     int K, int lda, int ldc, int n_tiles, int k_steps, int c_mode, int steps_per_group, RowScale scale, GvExperts ex) {
+    gemv_mfma_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, int M, int K, int lda, int n_tiles, int k_steps, int shape,
+                     int steps_per_group, int tiles_per_block, const float* __restrict__ sums, int N, int ldc, TC* __restrict__ C,
+                     float inv_width, float eps, GvExperts ex) {
   extern __shared__ float red[];  // [waves][256]
   __shared__ int chosen[EXPERTS == 2 ? GE_ROWS * GE_TOP : 1];
   __shared__ float inv[RS_ROWS];
   RowScaleLoad<SCALED ? SCALED : 1> scale_load;
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
-  const int n_waves = blockDim.x / BLM_WAVE;
+  const int n_waves = (shape >> 2) & 31, c_mode = shape & 3, n_sums = shape >> RS_SHIFT;
   const int row = lane & 15, kg = lane >> 4;
   // blockIdx.y is the K-group: it covers k-steps [group_begin, group_end) and writes plane blockIdx.y of C
   const int group_begin = blockIdx.y * steps_per_group;
@@ -128,13 +133,12 @@ __global__ void __launch_bounds__(MAXT)
     const bool keep = row < M && k < K && step0 + s < group_end;                      \
     a[s] = make_uint4(keep ? a[s].x : 0u, keep ? a[s].y : 0u, keep ? a[s].z : 0u, keep ? a[s].w : 0u); \
   }
-  if (SCALED) scale_load.ask(scale, M, wave, n_waves, lane);
+  if (SCALED) scale_load.ask(sums, n_sums, M, wave, n_waves, lane);
   if (KEEP_A) GV_LOAD_ACTIVATIONS()
 
   // a block takes a run of neighbouring column tiles, so that it streams one contiguous piece of the
   // packed weights (blocks that each read their own region reach a higher memory rate than blocks
   // that all advance through the matrix side by side)
-  const int tiles_per_block = (n_tiles + gridDim.x - 1) / gridDim.x;
   const int tile_begin = blockIdx.x * tiles_per_block, tile_end = min(n_tiles, tile_begin + tiles_per_block);
   // 16 k-steps per wavefront: the weights come in two halves of eight fragments, and each half's
   // registers are asked for the next tile's weights as soon as the matrix instructions that read them
@@ -145,51 +149,62 @@ __global__ void __launch_bounds__(MAXT)
   // sixteen fragments of one tile.)
   constexpr bool PIPE = KSTEPS == 16 && KEEP_A;
   constexpr int HALF = KSTEPS / 2;
-  uint4 wa[PIPE ? HALF : 1], wb[PIPE ? HALF : 1];
-  int woff[PIPE ? KSTEPS : 1];
-  if (PIPE) {
-#pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) woff[s] = (step0 + s < k_steps ? step0 + s : k_steps - 1) * 512;
+  // They are buffer loads of the tile's bytes: of none behind the last tile, where they bring zeros without a trip to memory.  With a
+  // branch around them instead the compiler counts on the way without them: the second half's first product then waits for the first
+  // half's new loads too.  (Steps past the matrix' last are out of the tile's bytes likewise.)
+  // Us, one row, with the branch / so: the head [128256, 2048] 85.5 / 82.5 (6.4 TB/s), [2048, 8192] in two groups 8.47 / 8.36, [3072, 8192] 11.5 /
+  // 11.0, gate/up [16384, 2048] 12.8 / 12.5, [22016, 2560] 20.4 / 19.3; eight rows 87.6 / 85.2, 8.94 / 8.86, 12.1 / 11.6, 13.4 / 13.25, 20.8 / 20.3.
+  gv_piece wa[PIPE ? HALF : 1], wb[PIPE ? HALF : 1];
+  const int wfirst = step0 * 1024 + lane * 16;
+  auto tile_bytes = [&](int tile, bool there) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(Wp + (size_t)tile * k_steps * 512), 0, there ? k_steps * 1024 : 0, 0x00027000);
+  };
+  if (PIPE && ONE) {
     const bf16* wt = Wp + ((size_t)min(tile_begin, n_tiles - 1) * k_steps * 64 + lane) * 8;
 #pragma unroll
-    for (int s = 0; s < HALF; ++s) wa[s] = ld16_stream(wt + woff[s]);
+    for (int s = 0; s < KSTEPS; ++s)
+      (s < HALF ? wa[s % HALF] : wb[s % HALF]) =
+          __builtin_nontemporal_load(reinterpret_cast<const gv_piece*>(wt + (step0 + s < k_steps ? step0 + s : k_steps - 1) * 512));
+  } else if (PIPE) {
+    const auto bytes = tile_bytes(min(tile_begin, n_tiles - 1), true);
 #pragma unroll
-    for (int s = 0; s < HALF; ++s) wb[s] = ld16_stream(wt + woff[HALF + s]);
+    for (int s = 0; s < HALF; ++s) wa[s] = __builtin_amdgcn_raw_buffer_load_b128(bytes, wfirst + s * 1024, 0, 2);
+#pragma unroll
+    for (int s = 0; s < HALF; ++s) wb[s] = __builtin_amdgcn_raw_buffer_load_b128(bytes, wfirst + (HALF + s) * 1024, 0, 2);
   }
   __builtin_amdgcn_sched_barrier(0);
-  if (SCALED) scale_load.finish(scale, M, wave, n_waves, lane, inv);
+  if (SCALED) scale_load.finish(n_sums, inv_width, eps, M, wave, n_waves, lane, inv);
   if (EXPERTS == 2)      // (rows past the last are the last once more)
     for (int r = __builtin_amdgcn_readfirstlane(wave) * 4; r < min(M, GE_ROWS); r += n_waves * 4) ge_look_up(ex, M, r, lane, chosen);
   if (KEEP_A) GV_ZERO_ACTIVATIONS()
 #undef GV_LOAD_ACTIVATIONS
 #undef GV_ZERO_ACTIVATIONS
-  for (int tile = tile_begin; tile < tile_end; ++tile) {
+  for (int tile = tile_begin; tile < (ONE ? min(tile_begin + 1, tile_end) : tile_end); ++tile) {
     const bf16* wt = Wp + ((size_t)tile * k_steps * 64 + lane) * 8;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
     constexpr int CH = KSTEPS < 16 ? KSTEPS : 16;   // weight loads in flight per wavefront
     if (PIPE) {
-      const bool more = tile + 1 < tile_end;
-      const bf16* wnext = Wp + ((size_t)(tile + 1) * k_steps * 64 + lane) * 8;
+      const auto next = tile_bytes(tile + 1, !ONE && tile + 1 < tile_end);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int s = 0; s < HALF; ++s)
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[s]),
                                                       __builtin_bit_cast(bf16x8_t, wa[s]), acc, 0, 0, 0);
+      asm volatile("" : "+v"(acc) : : "memory");     // the new loads stay behind the products whose registers they take
       __builtin_amdgcn_sched_barrier(0);
-      if (more) {
+      if (!ONE)
 #pragma unroll
-        for (int s = 0; s < HALF; ++s) wa[s] = ld16_stream(wnext + woff[s]);
-      }
+        for (int s = 0; s < HALF; ++s) wa[s] = __builtin_amdgcn_raw_buffer_load_b128(next, wfirst + s * 1024, 0, 2);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int s = 0; s < HALF; ++s)
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[HALF + s]),
                                                       __builtin_bit_cast(bf16x8_t, wb[s]), acc, 0, 0, 0);
+      asm volatile("" : "+v"(acc) : : "memory");
       __builtin_amdgcn_sched_barrier(0);
-      if (more) {
+      if (!ONE)
 #pragma unroll
-        for (int s = 0; s < HALF; ++s) wb[s] = ld16_stream(wnext + woff[HALF + s]);
-      }
+        for (int s = 0; s < HALF; ++s) wb[s] = __builtin_amdgcn_raw_buffer_load_b128(next, wfirst + (HALF + s) * 1024, 0, 2);
       __builtin_amdgcn_sched_barrier(0);
     } else
 #pragma unroll
@@ -228,7 +243,7 @@ __global__ void __launch_bounds__(MAXT)
 #pragma unroll
       for (int r = 0; r < 4; ++r) red[wave * 256 + r * 64 + lane] = acc[r];
       __syncthreads();
-      for (int idx = threadIdx.x; idx < 256; idx += blockDim.x) {  // a block may have fewer than 256 threads
+      for (int idx = threadIdx.x; idx < 256; idx += n_waves * BLM_WAVE) {  // a block may have fewer than 256 threads
         const int r = idx >> 6, l2 = idx & 63, col = l2 & 15;
         const int m = (l2 >> 4) * 4 + r;
         if (c_mode == 0) {
@@ -467,10 +482,16 @@ static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int
   const int ksteps = geo.ksteps, waves = geo.waves, blocks = geo.blocks;
   dim3 grid(blocks, k_groups), block(waves * BLM_WAVE);
   const size_t smem = (size_t)waves * 256 * sizeof(float);
+#define BLM_GO(KS, MAXT, KEEP, ONE, SCALED, SCALE, EXPERTS, EX)                                                 \
+  hipLaunchKernelGGL((gemv_mfma_kernel<KS, MAXT, KEEP, ONE, SCALED, EXPERTS, TC>), grid, block, smem, stream,   \
+                     (const bf16*)A, (const bf16*)Wp, M, K, lda, n_tiles, k_steps,                              \
+                     4 * waves + c_mode + ((SCALE).n << RS_SHIFT), steps_per_group, (n_tiles + blocks - 1) / blocks, (SCALE).sums, N, \
+                     ldc, (TC*)C, (SCALE).inv_width, (SCALE).eps, EX)
 #define BLM_GS(KS, MAXT, KEEP, SCALED, SCALE, EXPERTS, EX)                                                      \
-  hipLaunchKernelGGL((gemv_mfma_kernel<KS, MAXT, KEEP, SCALED, EXPERTS, TC>), grid, block, smem, stream,        \
-                     (const bf16*)A, (const bf16*)Wp, (TC*)C, M, N, K, lda, ldc, n_tiles, k_steps, c_mode,      \
-                     steps_per_group, SCALE, EX)
+  do {                                                                                                          \
+    if (KS == 16 && blocks >= n_tiles) BLM_GO(KS, MAXT, KEEP, KS == 16, SCALED, SCALE, EXPERTS, EX);            \
+    else BLM_GO(KS, MAXT, KEEP, false, SCALED, SCALE, EXPERTS, EX);                                             \
+  } while (0)
 #define BLM_GM(KS, MAXT, KEEP)                                                                                  \
   do {                                                                                                          \
     if (experts && experts->weights) BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 1, *experts);                        \
@@ -487,6 +508,7 @@ static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int
   else BLM_GM(32, 1024, false);
 #undef BLM_GM
 #undef BLM_GS
+#undef BLM_GO
   BLM_LAUNCH_CHECK("gemv_mfma");
   return 0;
 }

@@ -17,18 +17,19 @@
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
+// (What the first loads need stands in the arguments' first fourteen dwords, which come in registers.)
 // QR_KSTEPS: k-steps of 32 per wavefront.  MAXT: most threads of a block (8 or 16 wavefronts).  All
 // loads of a block are in flight at once: its time is one memory latency.
 // SCALED: the rows come unscaled (row_scale.h), that many of them to a wavefront.
 template <int QR_KSTEPS, int MAXT, int SCALED>
 __global__ void __launch_bounds__(MAXT)
-    gemv_qkv_rope_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, bf16* __restrict__ qkv_out,
+    gemv_qkv_rope_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, int M, int K, int lda, int k_steps, int shape,
+                         int hd, int nh, int flags, const float* __restrict__ sums, int nkv, bf16* __restrict__ qkv_out,
                          const int* __restrict__ positions, const int* __restrict__ token_seq,
                          const int* __restrict__ block_table, int table_width, const float2* __restrict__ cos_sin,
-                         bf16* __restrict__ kcache, bf16* __restrict__ vcache, int page_size, int M, int K, int lda,
-                         int ldq, int k_steps, int kw_count, int nh, int nkv, int hd, int pairing, int store,
-                         RowScale scale) {
+                         bf16* __restrict__ kcache, bf16* __restrict__ vcache, int page_size, int ldq, float inv_width, float eps) {
   extern __shared__ float red[];   // [2 * kw_count wavefronts][256]
+  const int kw_count = shape & 31, n_sums = shape >> RS_SHIFT, pairing = flags & 1, store = flags >> 1;
   __shared__ float inv[RS_ROWS];
   RowScaleLoad<SCALED ? SCALED : 1> scale_load;
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
@@ -45,7 +46,7 @@ __global__ void __launch_bounds__(MAXT)
   const int step0 = kw * QR_KSTEPS;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
 
-  if (SCALED) scale_load.ask(scale, M, wave, 2 * kw_count, lane);
+  if (SCALED) scale_load.ask(sums, n_sums, M, wave, 2 * kw_count, lane);
   const bf16* wt = Wp + ((size_t)tile * k_steps * 64 + lane) * 8;
   uint4 w[QR_KSTEPS];
 #pragma unroll
@@ -62,7 +63,7 @@ __global__ void __launch_bounds__(MAXT)
     a[s] = (row < M && k < K) ? v : zero;
   }
   __builtin_amdgcn_sched_barrier(0);
-  if (SCALED) scale_load.finish(scale, M, wave, 2 * kw_count, lane, inv);
+  if (SCALED) scale_load.finish(n_sums, inv_width, eps, M, wave, 2 * kw_count, lane, inv);
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < QR_KSTEPS; ++s)
@@ -73,7 +74,7 @@ __global__ void __launch_bounds__(MAXT)
   __syncthreads();
 
   // epilogue: one thread per (token row m, column c of the tiles)
-  for (int idx = threadIdx.x; idx < 256; idx += blockDim.x) {
+  for (int idx = threadIdx.x; idx < 256; idx += 2 * kw_count * BLM_WAVE) {
     const int r = idx >> 6, l2 = idx & 63, c = l2 & 15;
     const int m = (l2 >> 4) * 4 + r;
     if (m >= M) continue;
@@ -140,26 +141,24 @@ __global__ void __launch_bounds__(MAXT)
 // columns are 192 tiles).  Value heads are not rotated.  red: [wavefronts][256].
 template <int QR_KSTEPS, int SCALED>
 __global__ void __launch_bounds__(512)
-    gemv_qkv_rope_tile_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, bf16* __restrict__ qkv_out,
+    gemv_qkv_rope_tile_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, int M, int K, int lda, int k_steps, int shape,
+                              int hd, int nh, int store, const float* __restrict__ sums, int nkv, bf16* __restrict__ qkv_out,
                               const int* __restrict__ positions, const int* __restrict__ token_seq,
                               const int* __restrict__ block_table, int table_width,
                               const float2* __restrict__ cos_sin, bf16* __restrict__ kcache,
-                              bf16* __restrict__ vcache, int page_size, int M, int K, int lda, int ldq, int k_steps,
-                              int nh, int nkv, int hd, int store, RowScale scale) {
+                              bf16* __restrict__ vcache, int page_size, int ldq, float inv_width, float eps) {
   extern __shared__ float red[];
   __shared__ float inv[RS_ROWS];
   RowScaleLoad<SCALED ? SCALED : 1> scale_load;
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
-  const int n_waves = blockDim.x / BLM_WAVE;
   const int row = lane & 15, kg = lane >> 4;
-  const int tiles_per_head = hd / 16;
+  const int tiles_per_head = hd / 16, n_waves = shape & 31, n_sums = shape >> RS_SHIFT;
   const int tile = blockIdx.x;
-  const int head = tile / tiles_per_head, col0 = (tile - head * tiles_per_head) * 16;
-  if (!store && head >= nh) return;   // keys and values belong to another layer's cache: only q is needed
+  if (!store && tile >= nh * tiles_per_head) return;   // keys and values belong to another layer's cache: only q is needed
   const int step0 = wave * QR_KSTEPS;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
 
-  if (SCALED) scale_load.ask(scale, M, wave, n_waves, lane);
+  if (SCALED) scale_load.ask(sums, n_sums, M, wave, n_waves, lane);
   const bf16* wt = Wp + ((size_t)tile * k_steps * 64 + lane) * 8;
   uint4 w[QR_KSTEPS];
 #pragma unroll
@@ -176,7 +175,7 @@ __global__ void __launch_bounds__(512)
     a[s] = (row < M && k < K) ? v : zero;
   }
   __builtin_amdgcn_sched_barrier(0);
-  if (SCALED) scale_load.finish(scale, M, wave, n_waves, lane, inv);
+  if (SCALED) scale_load.finish(n_sums, inv_width, eps, M, wave, n_waves, lane, inv);
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < QR_KSTEPS; ++s)
@@ -187,7 +186,8 @@ __global__ void __launch_bounds__(512)
   __syncthreads();
 
   // epilogue: one thread per (token row m, column c of the tile)
-  for (int idx = threadIdx.x; idx < 256; idx += blockDim.x) {
+  const int head = tile / tiles_per_head, col0 = (tile - head * tiles_per_head) * 16;
+  for (int idx = threadIdx.x; idx < 256; idx += n_waves * BLM_WAVE) {
     const int r = idx >> 6, l2 = idx & 63, c = l2 & 15;
     const int m = (l2 >> 4) * 4 + r;
     if (m >= M) continue;
@@ -366,9 +366,10 @@ static int qkv_rope_entry(const void* A, const void* Wp, void* qkv_out, const in
     const int waves = (k_steps + 15) / 16;
 #define BLM_QT(SCALED, SCALE)                                                                                           \
   hipLaunchKernelGGL((gemv_qkv_rope_tile_kernel<16, SCALED>), dim3(tiles), dim3(waves * BLM_WAVE),                       \
-                     (size_t)waves * 256 * sizeof(float), stream, (const bf16*)A, (const bf16*)Wp, (bf16*)qkv_out,       \
-                     positions, token_seq, block_table, table_width, (const float2*)cos_sin, (bf16*)kcache, (bf16*)vcache, \
-                     page_size, M, K, lda, ldq, k_steps, nh, nkv, hd, store, SCALE)
+                     (size_t)waves * 256 * sizeof(float), stream, (const bf16*)A, (const bf16*)Wp, M, K, lda, k_steps,   \
+                     waves + ((SCALE).n << RS_SHIFT), hd, nh, store ? 1 : 0, (SCALE).sums, nkv, (bf16*)qkv_out, positions, token_seq, \
+                     block_table, table_width, (const float2*)cos_sin, (bf16*)kcache, (bf16*)vcache, page_size, ldq,     \
+                     (SCALE).inv_width, (SCALE).eps)
     if (scale == nullptr) BLM_QT(0, RowScale{});
     else if (M <= waves) BLM_QT(1, *scale);
     else if (M <= 2 * waves) BLM_QT(2, *scale);
@@ -391,9 +392,9 @@ static int qkv_rope_entry(const void* A, const void* Wp, void* qkv_out, const in
   } while (0)
 #define BLM_QS(KS, MAXT, SCALED, SCALE)                                                                               \
   hipLaunchKernelGGL((gemv_qkv_rope_kernel<KS, MAXT, SCALED>), dim3(units), dim3(2 * kw * BLM_WAVE), smem, stream, (const bf16*)A, \
-                     (const bf16*)Wp, (bf16*)qkv_out, positions, token_seq, block_table, table_width,                 \
-                     (const float2*)cos_sin, (bf16*)kcache, (bf16*)vcache, page_size, M, K, lda, ldq, k_steps, kw, nh, \
-                     nkv, hd, pairing, store, SCALE)
+                     (const bf16*)Wp, M, K, lda, k_steps, kw + ((SCALE).n << RS_SHIFT), hd, nh, pairing + (store ? 2 : 0),          \
+                     (SCALE).sums, nkv, (bf16*)qkv_out, positions, token_seq, block_table, table_width, (const float2*)cos_sin,     \
+                     (bf16*)kcache, (bf16*)vcache, page_size, ldq, (SCALE).inv_width, (SCALE).eps)
   if (ksteps == 24) BLM_QR(24, 512);
   else if (kw <= 4) BLM_QR(16, 512);
   else BLM_QR(16, 1024);

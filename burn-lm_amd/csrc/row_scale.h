@@ -9,6 +9,9 @@ struct RowScale {
   int n;               // a multiple of 4, at most RS_SUMS
   float inv_width, eps;
 };
+// (A kernel takes sums and, in its shape's bits from RS_SHIFT on, n among the first of its arguments, which come in registers: the sums
+// are what it asks for first.)
+#define RS_SHIFT 8
 #define RS_SUMS 256    // what a wavefront reads at once
 #define RS_ROWS 8      // most rows
 #define RS_SLOTS 8     // and most that a wavefront takes on (blocks of one wavefront)
@@ -22,18 +25,18 @@ static inline bool row_scale_fits(int M, const float* sums, int n) {
 template <int SLOTS>
 struct RowScaleLoad {
   float4 v[SLOTS];
-  __device__ __forceinline__ void ask(const RowScale& rs, int M, int wave, int n_waves, int lane) {
-    const float* p = rs.sums + min(lane * 4, rs.n - 4);
+  __device__ __forceinline__ void ask(const float* sums, int n, int M, int wave, int n_waves, int lane) {
+    const float* p = sums + min(lane * 4, n - 4);
 #pragma unroll
-    for (int i = 0; i < SLOTS; ++i) v[i] = *reinterpret_cast<const float4*>(p + min(wave + i * n_waves, M - 1) * rs.n);
+    for (int i = 0; i < SLOTS; ++i) v[i] = *reinterpret_cast<const float4*>(p + min(wave + i * n_waves, M - 1) * n);
   }
   // inv [M]: the rows' factors; the caller's next barrier makes them visible
-  __device__ __forceinline__ void finish(const RowScale& rs, int M, int wave, int n_waves, int lane, float* inv) {
+  __device__ __forceinline__ void finish(int n, float inv_width, float eps, int M, int wave, int n_waves, int lane, float* inv) {
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) {
-      const float s = wave_sum(lane * 4 < rs.n ? (v[i].x + v[i].y) + (v[i].z + v[i].w) : 0.f);
+      const float s = wave_sum(lane * 4 < n ? (v[i].x + v[i].y) + (v[i].z + v[i].w) : 0.f);
       const int row = wave + i * n_waves;
-      if (lane == 0 && row < M) inv[row] = 1.0f / sqrtf(s * rs.inv_width + rs.eps);
+      if (lane == 0 && row < M) inv[row] = 1.0f / sqrtf(s * inv_width + eps);
     }
   }
 };
