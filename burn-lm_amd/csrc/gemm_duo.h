@@ -29,6 +29,7 @@ typedef __attribute__((ext_vector_type(4))) unsigned int gd_u32x4;
 template <int V>
 using GdInt = std::integral_constant<int, V>;
 
+#define GD_FIVE_PERCENT 71
 #define GD_REGION (128 * GD_BK * 2)        // bytes: 128 rows of one operand's stage
 
 // A tile's operands: `a` and `b` the same in all lanes, at the first k; row(m) and column(r, h) the bytes from there to row m of the
@@ -173,80 +174,124 @@ __device__ __forceinline__ void gd_whole(gd_f32x4 (&acc)[8][4], const Tile& t, i
   if (wave < 4) GD_BARRIER();
 }
 
-// Half a tile, 128 rows of it: a wavefront has 64 rows and 64 columns.  A stage's fragments are read a stage ahead into a second
-// set of registers, and the ring has three stages.  0.57 of a whole tile's time (its reads of shared memory per product are 4 / 3).
-template <typename Tile>
-__device__ __forceinline__ void gd_half(gd_f32x4 (&acc)[4][4], const Tile& t, int stages, unsigned char* lds, int wave, int lane) {
+// Part of a tile, 32 TILES rows of it: 128 (a half) or 160 (five eighths).  A wavefront has half of them and 64 columns.  A stage's
+// fragments are read a stage ahead into a second set of registers, and the ring has three stages (156 KB for 160 rows, as many as a
+// unit's memory and a wavefront's registers hold).  A half takes 0.57 of a whole tile's time (its reads of shared memory per product are
+// 4 / 3), five eighths GD_FIVE_PERCENT.
+template <int TILES>
+struct GdPart {
+  static constexpr int ROWS = 32 * TILES, LOADS = (ROWS / 8 + 7) / 8;                 // of the rows, per wavefront and stage
+  static constexpr uint32_t A_BYTES = ROWS * GD_BK * 2, STAGE = A_BYTES + 2 * GD_REGION;
+};
+
+template <int TILES, typename Tile>
+__device__ __forceinline__ void gd_part(gd_f32x4 (&acc)[TILES][4], const Tile& t, int stages, unsigned char* lds, int wave, int lane) {
+  using Part = GdPart<TILES>;
+  constexpr int NA = Part::LOADS, ALL = NA + 4;
   const int l16 = lane & 15, quad = lane >> 4, wm = wave >> 2, wn = wave & 3;
-  uint32_t off[3][2];                                      // rows, first columns, second columns
+  // eight rows to a load; beyond 128 rows four loads are left, and wavefronts w and w + 4 bring the same one (each waits for as many)
+  auto group = [&](int i) { return i < 2 ? wave * 2 + i : 16 + (wave & 3); };
+  uint32_t a_off[NA], b_off[2][2];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    const int r = group(i) * 8 + lane / 8;
+    a_off[i] = t.row(r) + gd_piece(r, lane);
+  }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int r = (wave * 2 + i) * 8 + lane / 8;
-    off[0][i] = t.row(r) + gd_piece(r, lane);
-    off[1][i] = t.column(r, 0) + gd_piece(r, lane);
-    off[2][i] = t.column(r, 1) + gd_piece(r, lane);
+    const int r = group(i) * 8 + lane / 8;
+    b_off[0][i] = t.column(r, 0) + gd_piece(r, lane);
+    b_off[1][i] = t.column(r, 1) + gd_piece(r, lane);
   }
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(blm_lds_ptr)lds + (uint32_t)wave * 2048u;
-  auto fetch = [&](int s, int slot, int region, int i) {
-    blm_dma16_to((region == 0 ? t.a : t.b) + (size_t)s * (GD_BK * 2), off[region][i], lds0 + (uint32_t)((slot * 3 + region) * GD_REGION + i * 1024));
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(blm_lds_ptr)lds;
+  auto fetch_a = [&](int s, int slot, int i) {
+    blm_dma16_to(t.a + (size_t)s * (GD_BK * 2), a_off[i], lds0 + (uint32_t)slot * Part::STAGE + (uint32_t)group(i) * 1024u);
+  };
+  auto fetch_b = [&](int s, int slot, int h, int i) {
+    blm_dma16_to(t.b + (size_t)s * (GD_BK * 2), b_off[h][i], lds0 + (uint32_t)slot * Part::STAGE + Part::A_BYTES + (uint32_t)h * GD_REGION + (uint32_t)group(i) * 1024u);
   };
   int a_at[2], b_at[2];
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     const int slot = (4 * q + quad) ^ ((l16 >> 1) & 7);
-    a_at[q] = (wm * 64 + l16) * 128 + slot * 16;
-    b_at[q] = GD_REGION + (wn * 32 + l16) * 128 + slot * 16;
+    a_at[q] = (wm * (16 * TILES) + l16) * 128 + slot * 16;
+    b_at[q] = Part::A_BYTES + (wn * 32 + l16) * 128 + slot * 16;
   }
-  gd_u32x4 a[2][2][4], b0[2][2][2], b1[2][2][2];           // [stage's parity][32 of k][16 rows]
+  gd_u32x4 a[2][2][TILES], b0[2][2][2], b1[2][2][2];       // [stage's parity][32 of k][16 rows]
   auto read_a = [&](int set, int slot) {
-    const unsigned char* at = lds + slot * (3 * GD_REGION);
+    const unsigned char* at = lds + slot * Part::STAGE;
 #pragma unroll
-    for (int x = 0; x < 8; ++x) a[set][x >> 2][x & 3] = *reinterpret_cast<const gd_u32x4*>(at + a_at[x >> 2] + (x & 3) * 2048);
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int x = 0; x < TILES; ++x) a[set][q][x] = *reinterpret_cast<const gd_u32x4*>(at + a_at[q] + x * 2048);
   };
   auto read_b = [&](int set, int slot) {
-    const unsigned char* at = lds + slot * (3 * GD_REGION);
+    const unsigned char* at = lds + slot * Part::STAGE;
 #pragma unroll
     for (int x = 0; x < 4; ++x) b0[set][x >> 1][x & 1] = *reinterpret_cast<const gd_u32x4*>(at + b_at[x >> 1] + (x & 1) * 2048);
 #pragma unroll
     for (int x = 0; x < 4; ++x) b1[set][x >> 1][x & 1] = *reinterpret_cast<const gd_u32x4*>(at + b_at[x >> 1] + GD_REGION + (x & 1) * 2048);
   };
+  auto multiply = [&](auto set_type, auto side_type, auto loads) {
+    constexpr int set = decltype(set_type)::value, side = decltype(side_type)::value;
+    GD_BARRIER();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+#pragma unroll
+      for (int i = 0; i < TILES; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][side * 2 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(gd_bf16x8, side ? b1[set][q][j] : b0[set][q][j]), __builtin_bit_cast(gd_bf16x8, a[set][q][i]), acc[i][side * 2 + j], 0, 0, 0);
+      if (q == 0) {
+        GD_FENCE();
+        loads();
+        GD_FENCE();
+      }
+    }
+    GD_WAIT_LDS();
+    GD_BARRIER();
+  };
   gd_zero(acc);
 
 #pragma unroll
-  for (int s = 0; s < 3; ++s)
+  for (int s = 0; s < 3; ++s) {
 #pragma unroll
-    for (int x = 0; x < 6; ++x) fetch(s, s, x >> 1, x & 1);
-  GD_WAIT_VM(12);
+    for (int i = 0; i < NA; ++i) fetch_a(s, s, i);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) fetch_b(s, s, x >> 1, x & 1);
+  }
+  GD_WAIT_VM(2 * ALL);
   GD_BARRIER();
   read_a(0, 0);
   read_b(0, 0);
   GD_WAIT_LDS();
-  GD_WAIT_VM(10);
+  GD_WAIT_VM(2 * ALL - NA);
   GD_BARRIER();
   if (wave >= 4) GD_BARRIER();
 
-  // slot: of stage s; `left`: stages behind this one that exist (3: three and more)
+  // slot: of stage s; `left`: stages behind this one that exist (3: three and more).  On entry the next stage's rows are there.
   auto stage = [&](int s, int slot, auto set_type, auto left_type) {
     constexpr int set = decltype(set_type)::value, left = decltype(left_type)::value;
     const int next = slot == 2 ? 0 : slot + 1;
     if (left > 0) read_a(set ^ 1, next);
-    if (left > 1) GD_WAIT_VM(6);
+    if (left > 1) GD_WAIT_VM(ALL);                         // all of the next stage
     else if (left == 1) GD_WAIT_VM(0);
-    gd_multiply(acc, a[set], b0[set], 0, 0, [&] {
+    multiply(set_type, GdInt<0>{}, [&] {
       if (left > 2) {
-        fetch(s + 3, slot, 0, 0);
-        fetch(s + 3, slot, 0, 1);
-        fetch(s + 3, slot, 1, 0);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) fetch_a(s + 3, slot, i);
+        fetch_b(s + 3, slot, 0, 0);
       }
     });
     if (left > 0) read_b(set ^ 1, next);
-    if (left > 2) GD_WAIT_VM(7);
+    if (left > 2) GD_WAIT_VM(ALL + 1);                     // the rows of the stage behind the next
     else if (left == 2) GD_WAIT_VM(4);
-    gd_multiply(acc, a[set], b1[set], 0, 1, [&] {
+    multiply(set_type, GdInt<1>{}, [&] {
       if (left > 2) {
-        fetch(s + 3, slot, 1, 1);
-        fetch(s + 3, slot, 2, 0);
-        fetch(s + 3, slot, 2, 1);
+        fetch_b(s + 3, slot, 0, 1);
+        fetch_b(s + 3, slot, 1, 0);
+        fetch_b(s + 3, slot, 1, 1);
       }
     });
     return next;

@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(512, 2)
       gd_store_rope(acc, C, ldc, pos_of, page_of, wm * 128, m0, M, n, N, rope, l16, quad);
     } else {
       gd_f32x4 acc[4][4];
-      gd_half(acc, t, stages, lds, wave, lane);
+      gd_part<4>(acc, t, stages, lds, wave, lane);
       gd_store_rope(acc, C, ldc, pos_of, page_of, wm * 64, m0, M, n, N, rope, l16, quad);
     }
   } else if (!half) {
@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(512, 2)
     else gd_store<MODE, 8, TC>(acc, C, ldc, m0 + wm * 128, M, n, N, l16, quad);
   } else {
     gd_f32x4 acc[4][4];
-    gd_half(acc, t, stages, lds, wave, lane);
+    gd_part<4>(acc, t, stages, lds, wave, lane);
     if (GATED && plain) gd_store<0, 4, bf16>(acc, beside.C, beside.ldc, m0 + wm * 64, M, n, beside.N, l16, quad);
     else gd_store<MODE, 4, TC>(acc, C, ldc, m0 + wm * 64, M, n, N, l16, quad);
   }

@@ -30,9 +30,29 @@ typedef __attribute__((ext_vector_type(4))) unsigned int mg_u32x4;
 __device__ __forceinline__ float mg_gated(float g, float up, float weight) { return g / (1.0f + expf(-g)) * up * weight; }
 
 // weights [T][ld]: an expert's weight for a token, zero where it is not chosen.  lists [E][T]: plane rows place * T + token of
-// the tokens that chose expert e; counts [E].  Blocks behind the first E zero the plane rows of places that no expert takes.
+// the tokens that chose expert e, with the weight's bits beside them (one trip to memory at the start of a tile); counts [E].  Blocks behind the first E zero the plane rows of places that no expert takes.
+// TABLE: a table [V][top] of the token ids names a token's experts instead, each with the weight 1 / top (an id outside it chooses none; the id
+// is (*source)[source_rows[t]] where that row number is there and not negative, else ids[t]): a kernel less than with the weights made
+// first, 3 us, and a row of the table to read for a row of weights.
+struct MgTable {
+  const int *table, *ids, *source_rows;
+  const int* const* source;
+  int V;
+};
+__device__ __forceinline__ const int* mg_table_row(const MgTable& by, int t, int top) {      // null: no expert
+  const int r = by.source_rows ? by.source_rows[t] : -1;
+  const int id = r >= 0 ? (*by.source)[r] : by.ids[t];
+  return (unsigned)id < (unsigned)by.V ? by.table + (size_t)id * top : nullptr;
+}
+// whether entry k of a row names its expert for the first time
+__device__ __forceinline__ bool mg_first(const int* row, int k) {
+  bool first = true;
+  for (int j = 0; j < k; ++j) first &= row[j] != row[k];
+  return first;
+}
+template <bool TABLE>
 __global__ void __launch_bounds__(1024)
-    moe_lists_kernel(const float* __restrict__ weights, int ld, int T, int E, int top, int* __restrict__ lists, int* __restrict__ counts,
+    moe_lists_kernel(const float* __restrict__ weights, int ld, MgTable by, int T, int E, int top, int2* __restrict__ lists, int* __restrict__ counts,
                      float* __restrict__ planes, int D) {
   __shared__ int wave_sum[16];
   __shared__ int taken[64];
@@ -41,7 +61,13 @@ __global__ void __launch_bounds__(1024)
     const int t0 = ((int)blockIdx.x - E) * 64;
     if (tid < 64) {
       int n = top;
-      if (t0 + tid < T) {
+      if (TABLE) {
+        if (t0 + tid < T) {
+          const int* row = mg_table_row(by, t0 + tid, top);
+          n = 0;
+          for (int k = 0; k < top && row != nullptr; ++k) n += mg_first(row, k);
+        }
+      } else if (t0 + tid < T) {
         n = 0;
         for (int e = 0; e < E; ++e) n += weights[(size_t)(t0 + tid) * ld + e] != 0.f;
       }
@@ -57,11 +83,25 @@ __global__ void __launch_bounds__(1024)
   int base = 0;
   for (int t0 = 0; t0 < T; t0 += 1024) {
     const int t = t0 + tid;
-    const float* row = weights + (size_t)t * ld;
-    bool in = t < T && row[e] != 0.f;
+    bool in = false;
     int place = 0;
-    if (in)
-      for (int x = 0; x < e; ++x) place += row[x] != 0.f;
+    float weight = 1.0f / (float)top;
+    if (TABLE) {
+      const int* row = t < T ? mg_table_row(by, t, top) : nullptr;
+      if (row != nullptr)
+        for (int k = 0; k < top; ++k) {
+          const int x = row[k];
+          in |= x == e;
+          if (x < e) place += mg_first(row, k);
+        }
+    } else {
+      const float* row = weights + (size_t)t * ld;
+      in = t < T && row[e] != 0.f;
+      if (in) {
+        weight = row[e];
+        for (int x = 0; x < e; ++x) place += row[x] != 0.f;
+      }
+    }
     in = in && place < top;                 // (weights that are no numbers may be more than top)
     const unsigned long long votes = __builtin_amdgcn_ballot_w64(in);
     if (lane == 0) wave_sum[wave] = __popcll(votes);
@@ -72,7 +112,7 @@ __global__ void __launch_bounds__(1024)
       all += wave_sum[w];
     }
     at += __popcll(votes & ((1ull << lane) - 1));
-    if (in) lists[(size_t)e * T + at] = place * T + t;
+    if (in) lists[(size_t)e * T + at] = make_int2(place * T + t, __float_as_int(weight));
     base += all;
     __syncthreads();
   }
@@ -86,8 +126,7 @@ __global__ void __launch_bounds__(1024)
 // share their rows, the next ones their expert's weights.
 template <int MODE>
 __global__ void __launch_bounds__(64 * MG_WAVES, 2)
-    moe_gemm_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw, const float* __restrict__ weights, int ld_weights,
-                    const int* __restrict__ lists, const int* __restrict__ counts, bf16* __restrict__ act, float* __restrict__ planes,
+    moe_gemm_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw, const int2* __restrict__ lists, const int* __restrict__ counts, bf16* __restrict__ act, float* __restrict__ planes,
                     int T, int E, int N, int K, int inner, int n_tiles) {
   constexpr int STAGE = (MG_BM + MG_BN) * MG_BK, LOADS = (MG_BM + MG_BN) / 8 / MG_WAVES;
   __shared__ __attribute__((aligned(1024))) bf16 lds[3 * STAGE];
@@ -123,8 +162,9 @@ __global__ void __launch_bounds__(64 * MG_WAVES, 2)
   __shared__ int list[MG_BM];
   __shared__ float row_weight[MG_BM];
   if (tid < rows) {
-    list[tid] = lists[(size_t)e * T + m0 + tid];
-    if (MODE == 0) row_weight[tid] = weights[(size_t)(list[tid] % T) * ld_weights + e];
+    const int2 to = lists[(size_t)e * T + m0 + tid];
+    list[tid] = to.x;
+    row_weight[tid] = __int_as_float(to.y);
   }
   __syncthreads();
 
@@ -253,7 +293,7 @@ __global__ void __launch_bounds__(64 * MG_WAVES, 2)
 }
 
 // The same products in the tiles of gemm_duo.h, 256 rows and 256 columns (MODE 0: 128 gates and their ups).  An expert's rows are
-// whole tiles and, where at most 128 are left, a half; or halves all of them where those come in fewer rounds on the `units`.
+// whole tiles and, where at most 128 are left, a half; or halves all of them, or five eighths, where those come in less time on the `units`.
 template <int MODE>
 struct MgTile {
   const char *a, *b;
@@ -300,70 +340,75 @@ __device__ __forceinline__ void mg_store(const gd_f32x4 (&acc)[TILES][4], bf16* 
 
 template <int MODE>
 __global__ void __launch_bounds__(512, 2)
-    moe_duo_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw, const float* __restrict__ weights, int ld_weights,
-                   const int* __restrict__ lists, const int* __restrict__ counts, bf16* __restrict__ act, float* __restrict__ planes,
+    moe_duo_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw, const int2* __restrict__ lists, const int* __restrict__ counts, bf16* __restrict__ act, float* __restrict__ planes,
                    int T, int E, int N, int K, int inner, int n_tiles, int units) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[9 * GD_REGION];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[3 * GdPart<5>::STAGE];
   __shared__ int list[GD_TILE];
   __shared__ float row_weight[GD_TILE];
-  __shared__ int sums[4][8], found[4];
+  __shared__ int sums[5][8], found[4];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / BLM_WAVE), lane = tid & (BLM_WAVE - 1);
-  // a thread for each expert: its whole tiles, its half behind them, its halves if it has nothing else, its rows; and by a scan
-  // those of the experts before it
+  // a thread for each expert: its whole tiles, its half behind them, its halves or five eighths if it has nothing else, its rows; and by
+  // a scan those of the experts before it
   const int mine = tid < E ? counts[tid] : 0, over = mine % GD_TILE;
-  const int own[4] = {mine / GD_TILE + (over > GD_TILE / 2), over > 0 && over <= GD_TILE / 2, (mine + GD_TILE / 2 - 1) / (GD_TILE / 2), mine};
-  int upto[4], all[4];
+  const int own[5] = {mine / GD_TILE + (over > GD_TILE / 2), over > 0 && over <= GD_TILE / 2, (mine + GD_TILE / 2 - 1) / (GD_TILE / 2),
+                      (mine + GdPart<5>::ROWS - 1) / GdPart<5>::ROWS, mine};
+  int upto[5], all[5];
 #pragma unroll
-  for (int x = 0; x < 4; ++x) upto[x] = own[x];
+  for (int x = 0; x < 5; ++x) upto[x] = own[x];
 #pragma unroll
   for (int d = 1; d < BLM_WAVE; d *= 2) {
-    int before[4];
+    int before[5];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) before[x] = __shfl_up(upto[x], d);
+    for (int x = 0; x < 5; ++x) before[x] = __shfl_up(upto[x], d);
 #pragma unroll
-    for (int x = 0; x < 4; ++x) upto[x] += lane >= d ? before[x] : 0;
+    for (int x = 0; x < 5; ++x) upto[x] += lane >= d ? before[x] : 0;
   }
   if (lane == BLM_WAVE - 1)
 #pragma unroll
-    for (int x = 0; x < 4; ++x) sums[x][wave] = upto[x];
+    for (int x = 0; x < 5; ++x) sums[x][wave] = upto[x];
   __syncthreads();
 #pragma unroll
-  for (int x = 0; x < 4; ++x) {
+  for (int x = 0; x < 5; ++x) {
     all[x] = 0;
     for (int w = 0; w < 8; ++w) {
       if (w < wave) upto[x] += sums[x][w];
       all[x] += sums[x][w];
     }
   }
-  // rounds in hundredths of a whole tile's time, a half 57 of them (see gemm_duo.hip)
+  // rounds in hundredths of a whole tile's time, a half 57 of them, five eighths GD_FIVE_PERCENT (see gemm_duo.hip)
   const int wholes = all[0] * n_tiles, rest = wholes % units, beside = rest ? units - rest : 0;
   const int mixed = wholes / units * 100 + (rest ? 100 : 0) + (max(0, all[1] * n_tiles - beside) + units - 1) / units * 57;
-  const bool halved = (all[2] * n_tiles + units - 1) / units * 57 < mixed;
-  const int share1 = halved ? 0 : (wholes + 7) / 8, count2 = all[halved ? 2 : 1] * n_tiles, share2 = (count2 + 7) / 8;
+  const int halves = (all[2] * n_tiles + units - 1) / units * 57, fives = (all[3] * n_tiles + units - 1) / units * GD_FIVE_PERCENT;
+  // the parts behind the whole tiles: 1: an expert's last rows; 2, 3: all of them, in halves or five eighths
+  // (five eighths from K = 1,024 on: what a block does besides its products is the same for a larger and a smaller one, and at K = 512 three
+  // rounds' worth of it cost more than the products saved: 2,048 tokens, 16 experts, down projection 38.6 us against 35.0; gate/up, K = 2,048, 42.6 against 51.4)
+  const int parts = K >= 1024 && fives < min(halves, mixed) ? 3 : halves < mixed ? 2 : 1;
+  const int share1 = parts > 1 ? 0 : (wholes + 7) / 8, count2 = all[parts] * n_tiles, share2 = (count2 + 7) / 8;
   int b = blockIdx.x;
-  const bool half = b >= share1 * 8;
-  if (half) b -= share1 * 8;
-  const int share = half ? share2 : share1, id = (b & 7) * share + (b >> 3);       // a die has a stretch of the tiles
-  if ((b >> 3) >= share || id >= (half ? count2 : wholes)) return;
+  const bool part = b >= share1 * 8;
+  if (part) b -= share1 * 8;
+  const int share = part ? share2 : share1, id = (b & 7) * share + (b >> 3);       // a die has a stretch of the tiles
+  if ((b >> 3) >= share || id >= (part ? count2 : wholes)) return;
   const int nt = id % n_tiles, tile = id / n_tiles;
-  const int kind = half ? (halved ? 2 : 1) : 0;
-  const int last = kind == 0 ? upto[0] : kind == 1 ? upto[1] : upto[2], has = kind == 0 ? own[0] : kind == 1 ? own[1] : own[2];
+  const int kind = part ? parts : 0, most = kind == 0 ? GD_TILE : kind == 3 ? GdPart<5>::ROWS : GD_TILE / 2;      // its rows at most
+  const int last = kind == 0 ? upto[0] : kind == 1 ? upto[1] : kind == 2 ? upto[2] : upto[3];
+  const int has = kind == 0 ? own[0] : kind == 1 ? own[1] : kind == 2 ? own[2] : own[3];
   if (tile < last && tile >= last - has) {
     const int nth = tile - (last - has);
     found[0] = tid;
-    found[1] = kind == 0 ? nth * GD_TILE : kind == 1 ? mine / GD_TILE * GD_TILE : nth * (GD_TILE / 2);
-    found[2] = upto[3] - mine;
+    found[1] = kind == 1 ? mine / GD_TILE * GD_TILE : nth * most;
+    found[2] = upto[4] - mine;
     found[3] = mine;
   }
   __syncthreads();
   const int e = __builtin_amdgcn_readfirstlane(found[0]), m0 = __builtin_amdgcn_readfirstlane(found[1]);
   const int first = __builtin_amdgcn_readfirstlane(found[2]) + m0;
-  const int rows = min(half ? GD_TILE / 2 : GD_TILE, __builtin_amdgcn_readfirstlane(found[3]) - m0);
+  const int rows = min(most, __builtin_amdgcn_readfirstlane(found[3]) - m0);
   const int n0 = nt * (MODE == 0 ? GD_TILE / 2 : GD_TILE), wm = wave >> 2, wn = wave & 3;
   if (tid < GD_TILE) {
-    const int to = lists[(size_t)e * T + m0 + min(tid, rows - 1)];
-    list[tid] = MODE == 0 ? to % T : to;
-    if (MODE == 0) row_weight[tid] = weights[(size_t)(to % T) * ld_weights + e];
+    const int2 to = lists[(size_t)e * T + m0 + min(tid, rows - 1)];
+    list[tid] = MODE == 0 ? to.x % T : to.x;
+    row_weight[tid] = __int_as_float(to.y);
   }
   __syncthreads();
   MgTile<MODE> t;
@@ -377,30 +422,43 @@ __global__ void __launch_bounds__(512, 2)
   t.ldw = ldw;
   t.up = (uint32_t)inner * (uint32_t)ldw * 2u;
   const int n = n0 + wn * (MODE == 0 ? 32 : 64);
-  if (!half) {
+  if (kind == 0) {
     gd_f32x4 acc[8][4];
     gd_whole(acc, t, K / GD_BK, lds, wave, lane);
     mg_store<MODE, 8>(acc, act + (size_t)first * N, planes, list, row_weight, wm * 128, rows, n, N, lane);
+  } else if (kind == 3) {
+    gd_f32x4 acc[5][4];
+    gd_part<5>(acc, t, K / GD_BK, lds, wave, lane);
+    mg_store<MODE, 5>(acc, act + (size_t)first * N, planes, list, row_weight, wm * 80, rows, n, N, lane);
   } else {
     gd_f32x4 acc[4][4];
-    gd_half(acc, t, K / GD_BK, lds, wave, lane);
+    gd_part<4>(acc, t, K / GD_BK, lds, wave, lane);
     mg_store<MODE, 4>(acc, act + (size_t)first * N, planes, list, row_weight, wm * 64, rows, n, N, lane);
   }
 }
 
 // x [T][ldx], w_gate_up [2 E f][D] (the experts' gates, then their ups), w_down [D][E f], weights [T][ld_weights] float;
-// planes [top][T][D] float; lists [E * T], counts [E] ints and act [T * top][f] are workspaces of the call.  No token has more
+// planes [top][T][D] float; lists [E * T] pairs of ints, counts [E] ints and act [T * top][f] are workspaces of the call.  No token has more
 // than top weights that are not zero.
+// weights null: a table of the token ids chooses (moe_lists; its rows' entries differ and lie in [0, E)).
 extern "C" int blm_moe_grouped(const void* x, int ldx, const void* w_gate_up, const void* w_down, const float* weights, int ld_weights,
+                               const int* table, const int* ids, const int* source_rows, const void* source_cell, int V,
                                float* planes, int* lists, int* counts, void* act, int T, int D, int E, int f, int top,
                                int units, hipStream_t stream) {
+  BLM_REQUIRE(weights != nullptr || (table != nullptr && ids != nullptr && V > 0 && (source_rows == nullptr) == (source_cell == nullptr)),
+              "moe_grouped: weights, or a table with its token ids");
   BLM_REQUIRE(T > 0 && E > 0 && E <= MG_MAX_EXPERTS && top > 0 && top <= 64 && top <= E && D % MG_BK == 0 && f % MG_BK == 0 && D > 0 && f > 0,
               "moe_grouped: sizes T=%d D=%d experts=%d of %d, top=%d not supported", T, D, E, f, top);
-  BLM_REQUIRE(ldx >= D && ldx % 8 == 0 && ld_weights >= E && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w_gate_up % 16) == 0 &&
-                  ((uintptr_t)w_down % 16) == 0 && ((uintptr_t)act % 16) == 0, "moe_grouped: rows must start at multiples of 16 bytes");
+  BLM_REQUIRE(ldx >= D && ldx % 8 == 0 && (weights == nullptr || ld_weights >= E) && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w_gate_up % 16) == 0 &&
+                  ((uintptr_t)w_down % 16) == 0 && ((uintptr_t)act % 16) == 0 && ((uintptr_t)lists % 8) == 0, "moe_grouped: rows must start at multiples of 16 bytes");
   BLM_REQUIRE((long long)T * ldx < (1LL << 31) && (long long)D * E * f < (1LL << 31) && (long long)T * top < (1LL << 31) / 2,
               "moe_grouped: operands of 4 GiB and more");
-  hipLaunchKernelGGL(moe_lists_kernel, dim3((unsigned)(E + (T + 63) / 64)), dim3(1024), 0, stream, weights, ld_weights, T, E, top, lists, counts, planes, D);
+  const MgTable by{table, ids, source_rows, (const int* const*)source_cell, V};
+  const dim3 list_blocks((unsigned)(E + (T + 63) / 64));
+  if (weights)
+    hipLaunchKernelGGL(moe_lists_kernel<false>, list_blocks, dim3(1024), 0, stream, weights, ld_weights, by, T, E, top, (int2*)lists, counts, planes, D);
+  else
+    hipLaunchKernelGGL(moe_lists_kernel<true>, list_blocks, dim3(1024), 0, stream, weights, ld_weights, by, T, E, top, (int2*)lists, counts, planes, D);
   BLM_LAUNCH_CHECK("moe_lists");
   const long long row_tiles = ((long long)T * top + MG_BM - 1) / MG_BM + E;       // every expert's last tile may be part empty
   const long long halves = ((long long)T * top + GD_TILE / 2 - 1) / (GD_TILE / 2) + E;
@@ -414,22 +472,22 @@ extern "C" int blm_moe_grouped(const void* x, int ldx, const void* w_gate_up, co
   const int duo_gates = (f + GD_TILE / 2 - 1) / (GD_TILE / 2), duo_columns = (D + GD_TILE - 1) / GD_TILE;
   if (D % 128 == 0 && D >= 256 && ((long long)E * f + f) * D * 2 < (1LL << 32) && about * duo_gates * 5 >= units * 2LL) {
     const int tiles = duo_gates;
-    hipLaunchKernelGGL((moe_duo_kernel<0>), dim3((unsigned)(halves * tiles + 16)), dim3(512), 0, stream, (const bf16*)x, ldx, (const bf16*)w_gate_up, D, weights,
-                       ld_weights, lists, counts, (bf16*)act, planes, T, E, f, D, E * f, tiles, units);
+    hipLaunchKernelGGL((moe_duo_kernel<0>), dim3((unsigned)(halves * tiles + 16)), dim3(512), 0, stream, (const bf16*)x, ldx, (const bf16*)w_gate_up, D,
+                       (const int2*)lists, counts, (bf16*)act, planes, T, E, f, D, E * f, tiles, units);
   } else {
     const int tiles = (f + MG_BN / 2 - 1) / (MG_BN / 2);
     hipLaunchKernelGGL((moe_gemm_kernel<0>), dim3((unsigned)((row_tiles * tiles + 7) / 8 * 8)), dim3(64 * MG_WAVES), 0, stream, (const bf16*)x, ldx,
-                       (const bf16*)w_gate_up, D, weights, ld_weights, lists, counts, (bf16*)act, planes, T, E, f, D, E * f, tiles);
+                       (const bf16*)w_gate_up, D, (const int2*)lists, counts, (bf16*)act, planes, T, E, f, D, E * f, tiles);
   }
   BLM_LAUNCH_CHECK("moe_grouped gate/up");
   if (f % 128 == 0 && f >= 256 && about * duo_columns >= units) {
     const int tiles = duo_columns;
-    hipLaunchKernelGGL((moe_duo_kernel<1>), dim3((unsigned)(halves * tiles + 16)), dim3(512), 0, stream, (const bf16*)act, f, (const bf16*)w_down, E * f, weights,
-                       ld_weights, lists, counts, (bf16*)act, planes, T, E, D, f, E * f, tiles, units);
+    hipLaunchKernelGGL((moe_duo_kernel<1>), dim3((unsigned)(halves * tiles + 16)), dim3(512), 0, stream, (const bf16*)act, f, (const bf16*)w_down, E * f,
+                       (const int2*)lists, counts, (bf16*)act, planes, T, E, D, f, E * f, tiles, units);
   } else {
     const int tiles = (D + MG_BN - 1) / MG_BN;
     hipLaunchKernelGGL((moe_gemm_kernel<1>), dim3((unsigned)((row_tiles * tiles + 7) / 8 * 8)), dim3(64 * MG_WAVES), 0, stream, (const bf16*)act, f,
-                       (const bf16*)w_down, E * f, weights, ld_weights, lists, counts, (bf16*)act, planes, T, E, D, f, E * f, tiles);
+                       (const bf16*)w_down, E * f, (const int2*)lists, counts, (bf16*)act, planes, T, E, D, f, E * f, tiles);
   }
   BLM_LAUNCH_CHECK("moe_grouped down");
   return 0;

@@ -11,7 +11,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 47
+ABI_VERSION = 48
 _lib = None
 _lock = threading.Lock()
 
@@ -52,7 +52,7 @@ _SIGNATURES = {
                      _c_void_p, _c_int, _c_int, _c_void_p],
     "blm_head_gate": [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_map_difference": [_c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_void_p],
-    "blm_moe_grouped": [_c_void_p, _c_int] + [_c_void_p] * 3 + [_c_int] + [_c_void_p] * 4 + [_c_int] * 6 + [_c_void_p],
+    "blm_moe_grouped": [_c_void_p, _c_int] + [_c_void_p] * 3 + [_c_int] + [_c_void_p] * 4 + [_c_int] + [_c_void_p] * 4 + [_c_int] * 6 + [_c_void_p],
     "blm_moe_table": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_int, _c_int, _c_void_p],
     "blm_sigmoid_gate": [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_gelu_glu": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
@@ -1808,25 +1808,37 @@ def compute_units(index):
     return torch.cuda.get_device_properties(index).multi_processor_count
 
 
-def moe_grouped(x, w_gate_up, w_down, weights, n_experts, top):
+def moe_grouped(x, w_gate_up, w_down, weights, n_experts, top, table=None, ids=None, token_source=None):
     """float32 planes [top, T, D] whose sum is ``sum_e weights[t, e] * W_down_e (silu(W_gate_e x) * (W_up_e x))``: every token
     by its own experts only (those with a weight that is not zero, at most `top` of a token).  bfloat16 x [T, D], w_gate_up
-    [2 E f, D] (the experts' gates, then their ups), w_down [D, E f]; weights float32 [T, E + 1] (the last column is not read)."""
-    _gpu(x, w_gate_up, w_down, weights)
+    [2 E f, D] (the experts' gates, then their ups), w_down [D, E f]; weights float32 [T, E + 1] (the last column is not read), or
+    None and a table (int32 [vocabulary, top], entries in [0, E)) of the token ids [T] (token_source: see moe_table)."""
+    _gpu(x, w_gate_up, w_down, weights, table, ids)
     T, D = x.shape
     f = w_down.shape[1] // n_experts
     for name, t in (("x", x), ("w_gate_up", w_gate_up), ("w_down", w_down)):
         _contig(name, t)
         if t.dtype != torch.bfloat16:
             raise KernelError(f"moe_grouped: {name} must be bfloat16")
-    _f32("weights", weights, T * (n_experts + 1))
+    rows = cell = None
+    if weights is not None:
+        _f32("weights", weights, T * (n_experts + 1))
+    else:
+        _i32("table", table); _i32("ids", ids, T)
+        if table.dim() != 2 or table.shape[1] != top:
+            raise KernelError("moe_grouped: table [vocabulary, top]")
+        if token_source is not None:
+            rows, cell = token_source
+            _i32("source_rows", rows, T)
+            if cell.dtype != torch.int64 or cell.numel() != 1:
+                raise KernelError("moe_grouped: the cell is one int64 on the device")
     if tuple(w_gate_up.shape) != (2 * n_experts * f, D) or tuple(w_down.shape) != (D, n_experts * f):
         raise KernelError("moe_grouped: w_gate_up [2 E f, D], w_down [D, E f]")
     planes = torch.empty(top, T, D, dtype=torch.float32, device=x.device)
-    lists = torch.empty(n_experts * T + n_experts, dtype=torch.int32, device=x.device)
+    lists = torch.empty(2 * n_experts * T + n_experts, dtype=torch.int32, device=x.device)
     act = torch.empty(T * top, f, dtype=x.dtype, device=x.device)
-    _call("blm_moe_grouped", x.data_ptr(), D, w_gate_up.data_ptr(), w_down.data_ptr(), weights.data_ptr(), n_experts + 1,
-          planes.data_ptr(), lists.data_ptr(), lists.data_ptr() + 4 * n_experts * T, act.data_ptr(), T, D, n_experts, f, top,
+    _call("blm_moe_grouped", x.data_ptr(), D, w_gate_up.data_ptr(), w_down.data_ptr(), _ptr(weights), n_experts + 1,
+          _ptr(table), _ptr(ids), _ptr(rows), _ptr(cell), 0 if table is None else table.shape[0], planes.data_ptr(), lists.data_ptr(), lists.data_ptr() + 8 * n_experts * T, act.data_ptr(), T, D, n_experts, f, top,
           compute_units(x.device.index), _stream())
     return planes
 

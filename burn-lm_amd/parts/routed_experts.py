@@ -106,8 +106,7 @@ class RoutedExperts(FeedForward):
     def _mix(self, x, weights, step):
         """The experts' results for [tokens, width] by the weights of `route`, without clamps."""
         rt, ops = self.rt, self.rt.ops
-        bucket = getattr(step, "bucket", None)
-        if self._grouped(bucket[0] if bucket else x.shape[0]) and x.is_contiguous() and x.data_ptr() % 16 == 0:
+        if self._runs_grouped(x, step):
             return ops.moe_grouped(x, self.w_gate_up.w, self.w_down.w, weights, self.E, self.top)
         if rt.experts_take(x, self.w_gate_up):
             act = torch.empty(x.shape[0], self.inner, dtype=x.dtype, device=x.device)
@@ -115,6 +114,10 @@ class RoutedExperts(FeedForward):
         gu = rt.linear(x, self.w_gate_up)
         act = torch.empty(x.shape[0], self.inner, dtype=gu.dtype, device=x.device)
         return rt.linear(ops.moe_gate(gu, weights, act, self.E, self.f), self.w_down, partials=True)
+
+    def _runs_grouped(self, x, step):
+        bucket = getattr(step, "bucket", None)
+        return self._grouped(bucket[0] if bucket else x.shape[0]) and x.is_contiguous() and x.data_ptr() % 16 == 0
 
     def _grouped(self, T):
         """Whether in a step of T rows (of a recorded shape: the bucket's) every token goes through its own experts only (rather than all through all)."""
@@ -288,6 +291,9 @@ class TableExperts(RoutedExperts):
             act = torch.empty(x.shape[0], self.inner, dtype=x.dtype, device=x.device)
             rt.ops.gemv_experts(x, self.w_gate_up.packed, act, self.E, self.f, table=self.table, ids=step.token_ids, token_source=step.token_source)
             return rt.linear(act, self.w_down, partials=True)
+        if self._runs_grouped(x, step):
+            return rt.ops.moe_grouped(x, self.w_gate_up.w, self.w_down.w, None, self.E, self.top, table=self.table, ids=step.token_ids,
+                                      token_source=step.token_source)
         weights = torch.empty(x.shape[0], self.E + 1, dtype=torch.float32, device=x.device)
         rt.ops.moe_table(self.table, step.token_ids, weights, self.E, step.token_source)
         return self._mix(x, weights, step)

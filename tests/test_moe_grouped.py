@@ -44,6 +44,49 @@ def test_kernels(T, E, top, f, D, kind):
     assert torch.equal(again, y[:, rows.cuda()])
 
 
+@pytest.mark.parametrize("T,E,top,f,D", [(130, 3, 2, 64, 192), (900, 16, 4, 128, 256), (70, 128, 8, 64, 64)])
+def test_a_table_of_the_tokens(T, E, top, f, D):
+    """The same bits as with the table's weights made first; ids outside the table, ids that wait on the device, entries that repeat."""
+    from burn_lm_amd.csrc import ops
+    g = torch.Generator().manual_seed(T)
+    V = 40
+    x, gu, down = (torch.randn(*s, generator=g).bfloat16().cuda() for s in ((T, D), (2 * E * f, D), (D, E * f)))
+    table = torch.rand(V, E, generator=g).argsort(1)[:, :top].int()
+    table[3, 1] = table[3, 0]
+    table, ids = table.cuda(), torch.randint(0, V, (T,), generator=g).int()
+    ids[5], ids[9], ids[7] = V, -1, 3
+    ids = ids.cuda()
+    picked, rows = torch.randint(0, V, (64,), generator=g).int().cuda(), torch.full((T,), -1, dtype=torch.int32)
+    rows[::3] = 7
+    source = rows.cuda(), torch.tensor([picked.data_ptr()], dtype=torch.int64, device="cuda")
+    for source in (None, source):
+        weights = torch.empty(T, E + 1, device="cuda")
+        ops.moe_table(table, ids, weights, E, source)
+        want = ops.moe_grouped(x, gu, down, weights, E, top)
+        assert torch.equal(ops.moe_grouped(x, gu, down, None, E, top, table=table, ids=ids, token_source=source), want)
+
+
+@pytest.mark.parametrize("rows", [[500, 530, 640, 641], [160, 161, 0, 1], [1000, 20, 300, 700]])
+def test_tiles_of_five_eighths(rows):
+    """Experts whose rows end at, behind and in front of tiles of 160 rows, alone on a few units: halves, wholes and five eighths (which
+    the number of units decides) give the same bits, and those of the small tiles."""
+    from burn_lm_amd.csrc import ops
+    E, f, D = 4, 1024, 1024
+    T = sum(rows)
+    g = torch.Generator().manual_seed(T)
+    x, gu, down = (torch.randn(*s, generator=g).mul_(s[1] ** -0.5).bfloat16().cuda() for s in ((T, D), (2 * E * f, D), (D, E * f)))
+    w = torch.zeros(T, E + 1)
+    w[torch.arange(T), torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(T, generator=g)]] = 0.5
+    w, lists, act = w.cuda(), torch.empty(2 * E * T + E, dtype=torch.int32, device="cuda"), torch.empty(T, f, dtype=torch.bfloat16, device="cuda")
+    results = []
+    for units in (8, 40, 64, 80, 96, 112, 128, 256, 2000):
+        planes = torch.full((1, T, D), float("nan"), device="cuda")
+        ops._call("blm_moe_grouped", x.data_ptr(), D, gu.data_ptr(), down.data_ptr(), w.data_ptr(), E + 1, None, None, None, None, 0,
+                  planes.data_ptr(), lists.data_ptr(), lists.data_ptr() + 8 * E * T, act.data_ptr(), T, D, E, f, 1, units, ops._stream())
+        results.append(planes)
+    assert not results[0].isnan().any() and all(torch.equal(r, results[0]) for r in results[1:])
+
+
 def test_weights_that_are_no_numbers():
     from burn_lm_amd.csrc import ops
     T, E, top, f, D = 150, 4, 2, 64, 64
