@@ -30,10 +30,12 @@ typedef __attribute__((ext_vector_type(4))) unsigned int mg_u32x4;
 __device__ __forceinline__ float mg_gated(float g, float up, float weight) { return g / (1.0f + expf(-g)) * up * weight; }
 
 // weights [T][ld]: an expert's weight for a token, zero where it is not chosen.  lists [E][T]: plane rows place * T + token of
-// the tokens that chose expert e, with the weight's bits beside them (one trip to memory at the start of a tile); counts [E].  Blocks behind the first E zero the plane rows of places that no expert takes.
+// the tokens that chose expert e, with the weight's bits beside them (one trip to memory at the start of a tile); counts [E].  Blocks
+// behind the first E zero the plane rows of places that no expert takes.
 // TABLE: a table [V][top] of the token ids names a token's experts instead, each with the weight 1 / top (an id outside it chooses none; the id
 // is (*source)[source_rows[t]] where that row number is there and not negative, else ids[t]): a kernel less than with the weights made
-// first, 3 us, and a row of the table to read for a row of weights.
+// first.  What bounds it are trips to memory in a row, so the tokens of four rounds of threads are asked for at once (2,048 tokens, 16 experts, 4 of
+// them a token, under the profiler: weights and lists 5.1 + 6.3 us, a round after the other 13.3, so 10.9 and a launch less).
 struct MgTable {
   const int *table, *ids, *source_rows;
   const int* const* source;
@@ -44,11 +46,44 @@ __device__ __forceinline__ const int* mg_table_row(const MgTable& by, int t, int
   const int id = r >= 0 ? (*by.source)[r] : by.ids[t];
   return (unsigned)id < (unsigned)by.V ? by.table + (size_t)id * top : nullptr;
 }
+#define MG_AHEAD 4
+#define MG_ENTRIES 8      // of a row that are held in registers
 // whether entry k of a row names its expert for the first time
 __device__ __forceinline__ bool mg_first(const int* row, int k) {
   bool first = true;
   for (int j = 0; j < k; ++j) first &= row[j] != row[k];
   return first;
+}
+// the first entries of a row, in one or two loads where they allow (places past the row's end repeat its last)
+__device__ __forceinline__ void mg_entries(const int* row, int top, bool fours, int (&v)[MG_ENTRIES]) {
+  if (fours) {
+    const int4 a = *reinterpret_cast<const int4*>(row), b = *reinterpret_cast<const int4*>(row + (top > 4 ? 4 : 0));
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  } else {
+#pragma unroll
+    for (int k = 0; k < MG_ENTRIES; ++k) v[k] = row[min(k, top - 1)];
+  }
+}
+// whether a row names expert e, and how many experts in front of it
+__device__ __forceinline__ bool mg_named(const int* row, const int (&v)[MG_ENTRIES], int top, int e, int& place) {
+  bool in = false;
+  place = 0;
+  if (top <= MG_ENTRIES) {
+#pragma unroll
+    for (int k = 0; k < MG_ENTRIES; ++k) {
+      bool first = k < top;
+#pragma unroll
+      for (int j = 0; j < k; ++j) first &= v[j] != v[k];
+      in |= first && v[k] == e;
+      place += first && v[k] < e;
+    }
+  } else {
+    for (int k = 0; k < top; ++k) {
+      in |= row[k] == e;
+      if (row[k] < e) place += mg_first(row, k);
+    }
+  }
+  return in;
 }
 template <bool TABLE>
 __global__ void __launch_bounds__(1024)
@@ -56,7 +91,9 @@ __global__ void __launch_bounds__(1024)
                      float* __restrict__ planes, int D) {
   __shared__ int wave_sum[16];
   __shared__ int taken[64];
+  __shared__ unsigned long long short_of;      // of 64 tokens those with fewer experts than places
   const int tid = threadIdx.x, wave = tid / BLM_WAVE, lane = tid & (BLM_WAVE - 1);
+  const bool fours = top % 4 == 0 && top <= MG_ENTRIES && ((uintptr_t)by.table & 15) == 0;
   if ((int)blockIdx.x >= E) {
     const int t0 = ((int)blockIdx.x - E) * 64;
     if (tid < 64) {
@@ -64,36 +101,49 @@ __global__ void __launch_bounds__(1024)
       if (TABLE) {
         if (t0 + tid < T) {
           const int* row = mg_table_row(by, t0 + tid, top);
-          n = 0;
-          for (int k = 0; k < top && row != nullptr; ++k) n += mg_first(row, k);
+          int entries[MG_ENTRIES];
+          mg_entries(row != nullptr ? row : by.table, top, fours, entries);
+          mg_named(row, entries, row != nullptr ? top : 0, 0x7fffffff, n);
         }
       } else if (t0 + tid < T) {
         n = 0;
         for (int e = 0; e < E; ++e) n += weights[(size_t)(t0 + tid) * ld + e] != 0.f;
       }
       taken[tid] = n;
+      const unsigned long long few = __builtin_amdgcn_ballot_w64(n < top);
+      if (tid == 0) short_of = few;
     }
     __syncthreads();
-    for (int i = 0; i < 64; ++i)
+    for (unsigned long long few = short_of; few != 0; few &= few - 1) {
+      const int i = __builtin_ctzll(few);
       for (int p = taken[i]; p < top; ++p)
         for (int d = tid; d < D; d += 1024) planes[((size_t)p * T + t0 + i) * D + d] = 0.f;
+    }
     return;
   }
   const int e = blockIdx.x;
   int base = 0;
-  for (int t0 = 0; t0 < T; t0 += 1024) {
+  const int* rows[MG_AHEAD];
+  int entries[MG_AHEAD][MG_ENTRIES];
+  for (int t0 = 0, ahead = 0; t0 < T; t0 += 1024, ++ahead) {
     const int t = t0 + tid;
     bool in = false;
     int place = 0;
     float weight = 1.0f / (float)top;
     if (TABLE) {
-      const int* row = t < T ? mg_table_row(by, t, top) : nullptr;
-      if (row != nullptr)
-        for (int k = 0; k < top; ++k) {
-          const int x = row[k];
-          in |= x == e;
-          if (x < e) place += mg_first(row, k);
-        }
+      if (ahead % MG_AHEAD == 0) {
+#pragma unroll
+        for (int i = 0; i < MG_AHEAD; ++i) rows[i] = mg_table_row(by, min(t + i * 1024, T - 1), top);
+#pragma unroll
+        for (int i = 0; i < MG_AHEAD; ++i) mg_entries(rows[i] != nullptr ? rows[i] : by.table, top, fours, entries[i]);
+      }
+      in = mg_named(rows[0], entries[0], rows[0] != nullptr && t < T ? top : 0, e, place);
+#pragma unroll
+      for (int i = 0; i + 1 < MG_AHEAD; ++i) {
+        rows[i] = rows[i + 1];
+#pragma unroll
+        for (int k = 0; k < MG_ENTRIES; ++k) entries[i][k] = entries[i + 1][k];
+      }
     } else {
       const float* row = weights + (size_t)t * ld;
       in = t < T && row[e] != 0.f;
