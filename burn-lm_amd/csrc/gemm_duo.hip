@@ -213,11 +213,31 @@ __global__ void __launch_bounds__(512, 2)
   }
 }
 
+// A plain product in tiles of 160 rows and 256 columns: 0.71 of a whole tile's time, for rounds that neither whole tiles nor halves fill
+// (2,166 rows of 2,048 columns in two groups of K are 272 halves for 256 units, or 224 of these).  Products of planes, us: [2048, 8192], 2,166
+// rows, two groups 64.9 (1.12 PFLOP/s; halves 97.8, the library's product without planes 74.7), 1,200 rows, four groups 42.3 (55.3; 53.9).
+template <typename TC>
+__global__ void __launch_bounds__(512, 2)
+    gemm_five_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, TC* __restrict__ C, int M, int N, int K, int lda, int ldw,
+                     int ldc, int m_tiles, int n_tiles, int k_per_group) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[3 * GdPart<5>::STAGE];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / BLM_WAVE), lane = tid & (BLM_WAVE - 1);
+  const int total = gridDim.x, die = blockIdx.x & 7, q = total >> 3, r = total & 7, at = die * q + min(die, r) + (blockIdx.x >> 3);
+  const int in_group = GD_GROUP * n_tiles, group = at / in_group, first = group * GD_GROUP, height = min(GD_GROUP, m_tiles - first);
+  const int m0 = (first + (at - group * in_group) % height) * GdPart<5>::ROWS, n0 = (at - group * in_group) / height * GD_TILE;
+  const int k0 = blockIdx.y * k_per_group, stages = min(k_per_group, K - k0) / GD_BK;
+  C += (size_t)blockIdx.y * M * ldc;
+  const GdTile<0> t = {reinterpret_cast<const char*>(A + (size_t)m0 * lda + k0), reinterpret_cast<const char*>(W + (size_t)n0 * ldw + k0), M - m0, N - n0, 0, lda, ldw, false};
+  gd_f32x4 acc[5][4];
+  gd_part<5>(acc, t, stages, lds, wave, lane);
+  gd_store<0, 5, TC>(acc, C, ldc, m0 + (wave >> 2) * 80, M, n0 + (wave & 3) * 64, N, lane & 15, lane >> 4);
+}
+
 // mode 0: C[M, N] = A W^T, W [N, K].  mode 1: W [2N, K] = [gate rows; up rows], C[M, N] = silu(gate) * up; mode 2: the tanh form of
 // GELU in place of silu.  k_groups > 1: C is float [k_groups, M, ldc], a partial product over each group's stretch of K (a multiple
-// of 128).  whole: how many of the tiles are run as whole ones, the others as halves.
+// of 128).  whole: how many of the tiles are run as whole ones, the others as halves.  fives (mode 0): tiles of 160 rows, whole is 0.
 static int gd_run(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, int mode,
-                  int k_groups, int whole, const GdRope* rope, GdBeside beside, hipStream_t stream) {
+                  int k_groups, int whole, bool fives, const GdRope* rope, GdBeside beside, hipStream_t stream) {
   BLM_REQUIRE(M >= 1 && N >= 8 && N % 8 == 0 && K >= 256 && K % 128 == 0, "gemm_duo: sizes M=%d N=%d K=%d not supported", M, N, K);
   BLM_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && ldc % 8 == 0 && lda >= K && ldw >= K && ldc >= (rope ? rope->nh * rope->hd : N), "gemm_duo: bad strides lda=%d ldw=%d ldc=%d",
               lda, ldw, ldc);
@@ -231,6 +251,20 @@ static int gd_run(const void* A, const void* W, void* C, int c_dtype, int M, int
   const int columns = mode != 0 ? GD_TILE / 2 : GD_TILE;
   beside.gate_tiles = (N + columns - 1) / columns;
   const int n_tiles = beside.gate_tiles + (beside.N + GD_TILE - 1) / GD_TILE;
+  if (fives) {
+    BLM_REQUIRE(whole == 0 && mode == 0, "gemm_duo: %d whole tiles of 0, mode %d", whole, mode);
+    const int rows = GdPart<5>::ROWS, five_tiles = (M + rows - 1) / rows;
+    BLM_REQUIRE((long long)five_tiles * n_tiles < (1LL << 30), "gemm_duo: too many tiles");
+    const dim3 grid((unsigned)(five_tiles * n_tiles), (unsigned)k_groups);
+    if (c_dtype == BLM_F32)
+      hipLaunchKernelGGL(gemm_five_kernel<float>, grid, dim3(512), 0, stream, (const bf16*)A, (const bf16*)W, (float*)C, M, N, K, lda, ldw, ldc,
+                         five_tiles, n_tiles, k_per_group);
+    else
+      hipLaunchKernelGGL(gemm_five_kernel<bf16>, grid, dim3(512), 0, stream, (const bf16*)A, (const bf16*)W, (bf16*)C, M, N, K, lda, ldw, ldc,
+                         five_tiles, n_tiles, k_per_group);
+    BLM_LAUNCH_CHECK("gemm_five");
+    return 0;
+  }
   const bool tail = M % GD_TILE != 0 && M % GD_TILE <= GD_TILE / 2;
   const int m_tiles = tail ? M / GD_TILE : (M + GD_TILE - 1) / GD_TILE;
   BLM_REQUIRE((long long)(m_tiles + 1) * n_tiles < (1LL << 29), "gemm_duo: too many tiles");
@@ -251,8 +285,8 @@ static int gd_run(const void* A, const void* W, void* C, int c_dtype, int M, int
 }
 
 extern "C" int blm_gemm_duo(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, int mode,
-                            int k_groups, int whole, hipStream_t stream) {
-  return gd_run(A, W, C, c_dtype, M, N, K, lda, ldw, ldc, mode, k_groups, whole, nullptr, GdBeside{}, stream);
+                            int k_groups, int whole, int fives, hipStream_t stream) {
+  return gd_run(A, W, C, c_dtype, M, N, K, lda, ldw, ldc, mode, k_groups, whole, fives != 0, nullptr, GdBeside{}, stream);
 }
 
 // A gated product (mode 1 or 2) with a plain one of the same rows beside it: W [2N + N2, K], C2[M, N2] the product with the last N2
@@ -262,7 +296,7 @@ extern "C" int blm_gemm_duo_beside(const void* A, const void* W, void* C, void* 
                                    int mode, int whole, hipStream_t stream) {
   BLM_REQUIRE((mode == 1 || mode == 2) && N2 > 0 && N2 % 8 == 0 && ldc2 >= N2 && ldc2 % 8 == 0 && ((uintptr_t)C2 % 16) == 0,
               "gemm_duo_beside: mode %d, %d columns in rows of %d not supported", mode, N2, ldc2);
-  return gd_run(A, W, C, BLM_BF16, M, N, K, lda, ldw, ldc, mode, 1, whole, nullptr, GdBeside{(bf16*)C2, N2, ldc2, 0}, stream);
+  return gd_run(A, W, C, BLM_BF16, M, N, K, lda, ldw, ldc, mode, 1, whole, false, nullptr, GdBeside{(bf16*)C2, N2, ldc2, 0}, stream);
 }
 
 // The q/k/v projection with the rotation of queries and keys (on the float results) and the write of keys and values into their
@@ -273,5 +307,5 @@ extern "C" int blm_gemm_duo_qkv_rope(const void* A, const void* W, void* qkv_out
   BLM_REQUIRE(nh > 0 && nkv > 0 && hd > 0 && hd % 16 == 0 && page_size > 0 && table_width > 0, "gemm_duo_qkv_rope: head size %d not supported (a multiple of 16)", hd);
   BLM_REQUIRE(((uintptr_t)kcache % 16) == 0 && ((uintptr_t)cos_sin % 16) == 0, "gemm_duo_qkv_rope: pages and angles must be 16-byte aligned");
   const GdRope rope{positions, token_seq, block_table, cos_sin, (bf16*)kcache, (bf16*)vcache, table_width, page_size, nh, nkv, hd, store};
-  return gd_run(A, W, qkv_out, BLM_BF16, M, (nh + 2 * nkv) * hd, K, lda, ldw, ldq, 0, 1, whole, &rope, GdBeside{}, stream);
+  return gd_run(A, W, qkv_out, BLM_BF16, M, (nh + 2 * nkv) * hd, K, lda, ldw, ldq, 0, 1, whole, false, &rope, GdBeside{}, stream);
 }

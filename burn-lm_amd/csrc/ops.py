@@ -11,7 +11,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 48
+ABI_VERSION = 49
 _lib = None
 _lock = threading.Lock()
 
@@ -164,8 +164,7 @@ _SIGNATURES = {
     "blm_sink_attn_mfma_init": [],
     "blm_gemm_mfma": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                       _c_int, _c_int, _c_int, _c_void_p],
-    "blm_gemm_duo": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
-                     _c_void_p],
+    "blm_gemm_duo": [_c_void_p] * 3 + [_c_int] * 11 + [_c_void_p],
     "blm_gemm_duo_beside": [_c_void_p] * 4 + [_c_int] * 10 + [_c_void_p],
     "blm_gemm_duo_qkv_rope": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 11 + [_c_void_p],
     "blm_gemv_mfma_group_limit": [_c_int],
@@ -948,11 +947,12 @@ def gemm_duo_takes(a, w, out, gated=False):
             and (2 if gated else 1) * N * w.stride(0) * 2 < 1 << 32 and 256 * a.stride(0) * 2 < 1 << 32)
 
 
-def gemm_duo(a, w, out, gated=False, activation="silu", whole=None):
+def gemm_duo(a, w, out, gated=False, activation="silu", whole=None, fives=False):
     """bfloat16 product of long prompts: out[M, N] = a[M, K] @ w[N, K]^T in tiles of 256x256, of which `whole` (all unless told
     otherwise) are one block's and the others two blocks' with half the rows each.  K in multiples of 128, N of 8.  out: bfloat16, or
     float32 [M, N], or float32 [groups, M, N] partial products over that many groups of K.  gated=True: w is [gate rows; up rows]
-    ([2N, K]) and out (bfloat16) is act(a gate^T) * (a up^T), act as in gemm_mfma."""
+    ([2N, K]) and out (bfloat16) is act(a gate^T) * (a up^T), act as in gemm_mfma.  fives=True: a plain product in
+    tiles of 160 rows, none of them whole ones."""
     _gpu(a, w, out)
     groups = 1
     if out.dim() == 3:
@@ -967,8 +967,12 @@ def gemm_duo(a, w, out, gated=False, activation="silu", whole=None):
         raise KernelError("gemm_duo: a, w and out need unit stride along their rows")
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise KernelError("gemm_duo: operands must be bfloat16")
+    if fives and gated:
+        raise KernelError("gemm_duo: no tiles of 160 rows for gated products")
+    if whole is None:
+        whole = 0 if fives else gemm_duo_tiles(M, N, gated)[0]
     _call("blm_gemm_duo", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out), M, N, K, a.stride(0), w.stride(0), out.stride(-2),
-          (2 if activation == "gelu_tanh" else 1) if gated else 0, groups, gemm_duo_tiles(M, N, gated)[0] if whole is None else whole, _stream())
+          (2 if activation == "gelu_tanh" else 1) if gated else 0, groups, whole, int(fives), _stream())
     return out
 
 

@@ -126,6 +126,8 @@ DUO_QKV_FILL = 0.62
 DUO_HALVES_K = 8192
 DUO_PLANES_FILL = 0.78
 DUO_PLANES_K = 6144
+DUO_FOURS_FILL = 0.6        # see Runtime.duo_part_planes
+DUO_FIVES_FILL = 0.75
 
 
 @functools.lru_cache(maxsize=4096)
@@ -484,6 +486,11 @@ class Runtime:
             planes_out = torch.empty(2, M, N, dtype=torch.float32, device=x.device)
             if ops.gemm_duo_takes(x, w, planes_out):
                 return ops.gemm_duo(x, w, planes_out, whole=0)
+        parts = self.duo_part_planes(M, N, K) if planes and plain_bf16 else None
+        if parts is not None:
+            planes_out = torch.empty(parts[0], M, N, dtype=torch.float32, device=x.device)
+            if ops.gemm_duo_takes(x, w, planes_out):
+                return ops.gemm_duo(x, w, planes_out, whole=0, fives=parts[1])
         if (planes and self.rows_ring and 16 < M <= MFMA_SKINNY_MAX_ROWS and plain_bf16
                 and (M > 32 or K <= 4096 or -(-N // 32) * 8 <= 3 * self.compute_units)):
             # 17 to 64 rows as partial planes (measured against the packed skinny kernel at the 1B, 3B and 8B
@@ -583,6 +590,30 @@ class Runtime:
             return False
         tiles, tail = ops.gemm_duo_tiles(M, N)
         return DUO_PLANES_FILL * self.compute_units <= 2 * (2 * tiles + tail) <= self.compute_units
+
+    def duo_part_planes(self, M, N, K):
+        """(groups of K, fives) with which such a product runs as planes of parts of ops.gemm_duo's tiles, all in one round, or None: halves
+        over four groups, or tiles of 160 rows (fives) over four or two; of the first that fits, with a group of at
+        least RING_GROUP_K, K from DUO_PLANES_K on, and four groups' blocks on DUO_FOURS_FILL of the units, two groups' on DUO_FIVES_FILL.
+        With the norm that adds the planes, us, this / as before (the library where nothing else is said):
+        * halves, four groups: width 2048, K = 8192, 675 / 770 / 883 rows 40.4 / 46.7, 42.4 / 48.0, 44.4 / 50.8; K = 16384 657 / 855 / 962 rows
+          59 / 78, 69 / 90, 70 / 96; width 3072, K = 8192, 537 / 620 rows 43.9 / 51.2, 44.7 / 52.9; width 1024, K = 8192, 1,240 / 1,389 rows
+          35.4 / 42.0, 37.7 / 43.2; width 1536, K = 12288, 845 / 1,132 rows 47.9 / 58.4, 56.0 / 69.6;
+        * 160 rows, four groups: width 2048, K = 8192, 1,035 / 1,147 / 1,274 rows 51.2 / 61.7, 52.1 / 60.3, 53.0 / 63.0; K = 16384 74.9 / 104.6,
+          74.9 / 103.0, 80.7 / 111.6; width 3072, K = 8192, 646 / 778 rows 49.0 / 57.5, 52.1 / 60.7; width 4096, K = 14336, 524 / 599 rows
+          71.4 / 93.8, 72.8 / 98.7;
+        * 160 rows, two groups: width 2048, K = 8192, 2,075 / 2,166 / 2,500 rows 77.6 / 84.5, 79.3 / 86.0, 83.4 / 88.1; width 3072, K = 8192, 1,282 /
+          1,405 / 1,534 rows 74.6 / 77.9, 74.9 / 81.4, 80.5 / 86.8; width 4096, K = 14336, 1,085 / 1,268 rows 115 / 131, 124 / 139; width 2560,
+          K = 11008, 1,554 / 1,915 rows 94.6 / 103.7, 102.2 / 112.7; less full 0.71 of the units, where halves over two groups fit: 74.1 / 68.5;
+        * three groups gain nothing: width 1536, K = 6144, 1,749 to 1,985 rows 1.03 of the library's time."""
+        if not self.fused_gate_up_measured or M <= MID_PLANES_MAX_ROWS or K < DUO_PLANES_K or self.duo_planes(M, N, K):
+            return None
+        for rows, groups, fill in ((128, 4, DUO_FOURS_FILL), (160, 4, DUO_FOURS_FILL), (160, 2, DUO_FIVES_FILL)):
+            blocks = -(-M // rows) * -(-N // 256) * groups
+            if K % (128 * groups) == 0 and K // groups >= RING_GROUP_K and blocks <= self.compute_units \
+                    and M * N * groups >= fill * self.compute_units * rows * 256:
+                return groups, rows == 160
+        return None
 
     def duo_product(self, M, N, K):
         """Whether a plain bfloat16 product of many rows goes to ops.gemm_duo and not to the library (us, duo / library, in turn):
