@@ -2,7 +2,7 @@
 //   argmax : first index of the maximum (lowest index wins ties); a row is searched by 32 blocks.
 //   sample : softmax(logits / temperature) in float, nucleus (top-p) cut, inverse-CDF pick at a
 //            uniform number u given by the caller, walking the kept tokens in index order; a row
-//            is worked on by 16 blocks, each pass over it a kernel of its own.
+//            is worked on by up to 32 blocks, each pass over it a kernel of its own.
 // Nucleus rule: a token is kept while the probability mass of the tokens strictly more likely
 // than it is below p; so the token that crosses p is kept, and tokens tied with it are too.
 //
@@ -14,12 +14,20 @@
 // a token lighter than 2^-32 of the heaviest one counts as no mass.  The pick then walks the kept
 // tokens in index order: every block owns a contiguous slice of the row, cut into chunks of 1024.
 //
-// One compute unit reads a row of 128K logits in about 10 us, and the five passes (maximum, three
-// histograms, pick) each depend on the one before, so a row is cut into up to 16 slices for as
-// many blocks and every pass is one kernel: the blocks of a row leave their part (slice maximum,
-// histogram bins added to the row's with device-wide atomics, chunk masses) in device-coherent
-// memory, count themselves in, and the block that arrives last finishes the pass for the row (the
-// row's maximum, the bin of this level, the pick).  No block ever waits for another.
+// One compute unit reads a row of 128K logits in about 10 us, and the five passes (maximum, three histograms, pick)
+// each depend on the one before, so a row is cut into up to 32 slices for as many blocks and every pass is one
+// kernel, bound by its trips to memory and its barriers.  What a pass finds for the whole row (the maximum of the
+// slices' maxima, the bin of a level) every block of the next one works out for itself from what the blocks left,
+// behind its first loads of logits: 1 to 2 us less than blocks that count themselves in, the last of which works it
+// out.  Only the pick has such an end: the last of the row's blocks to get there draws the token.  No block ever
+// waits for another.  What is asked of all threads (which one has the bin, which are behind the pick) is settled by
+// one thread or one ballot: an atomic on one LDS address is done lane by lane.  And loads stand in no branch of a
+// lane (SmpRow).
+// Blocks of 1,024 threads(see sample_wide_slices) do without two of the passes: the second one lists the weights of
+// the first level's bin, a few in a hundred of the row's, and the pick's blocks each take the other two levels from
+// the list.  All of it, us, before and now: 64 rows of 128,256 tokens 56.3 and 39.2 (6.3 the maximum, 8.4, 8.5 and
+// 15.2 the pick), 64 rows of 32,000 39.5 and 27.9, a row of 128,256 33.3 and 21.9; without the cut 64 rows 25.2 and
+// 13.9, a row 18.0 and 9.3.
 #include <mutex>
 
 #include "common.h"
@@ -142,19 +150,14 @@ extern "C" int blm_argmax_static(const float* logits, int* out, int R, int V, in
 #define SMP_WAVES (SMP_THREADS / BLM_WAVE)
 #define SMP_ROUND 8         // chunks of a slice whose masses are summed behind one barrier
 
-// per row: the maximum, then for the selection the digits found so far, the mass above them and the mass to reach
-struct SampleRow {
-  float mx;
+// behind a level of the selection: the digits found so far, the mass above them and the mass to reach
+struct SampleState {
   uint32_t prefix;
   unsigned long long carry, target;
 };
 
 __device__ __forceinline__ void smp_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float smp_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ unsigned long long smp_load(const unsigned long long* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Whether this block is the last of its row to get here.  What the block wrote before (coherent
 // stores, device-wide atomics) has been acknowledged when it counts itself in; the last one sets
 // the counter back to zero.  All threads get the answer.
@@ -189,130 +192,325 @@ __device__ __forceinline__ unsigned long long shfl_down_u64(unsigned long long v
   return ((unsigned long long)hi << 32) | lo;
 }
 
-// pass 1: the row's maximum; the last block also clears the row's histograms for the passes to come
+// e * 2^32, truncated, of an e <= 1
+__device__ __forceinline__ unsigned long long smp_mass(float e) {
+  return e >= 1.0f ? 1ull << 32 : (unsigned long long)(uint32_t)(e * 4294967296.0f);
+}
+
+// A row's elements below `end`, to be read in pieces of four.  The loads of several pieces stand in no branch of a lane: with smp_load4,
+// whose other side writes the same registers, the compiler has each wait for the one before it, a trip to memory each.
+template <bool VEC>
+struct SmpRow {
+  const float* x;
+  int end;
+  float rest[3];   // VEC: the elements behind the last whole piece (end % 4 of them)
+
+  __device__ __forceinline__ SmpRow(const float* x, int end) : x(x), end(end) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) rest[k] = -INFINITY;
+    if (VEC && end & 3)
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (k < (end & 3)) rest[k] = x[(end & ~3) + k];
+  }
+
+  // N pieces, `step` elements apart, this thread's first at i0; `inside`: every thread's pieces end below `end`
+  template <int N>
+  __device__ __forceinline__ void read(int i0, int step, bool inside, float xs[N][4]) const {
+    if (VEC && inside) {
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const float4 v = *reinterpret_cast<const float4*>(x + i0 + u * step);
+        xs[u][0] = v.x; xs[u][1] = v.y; xs[u][2] = v.z; xs[u][3] = v.w;
+      }
+    } else if (VEC) {
+      float4 v[N];
+#pragma unroll
+      for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const float4*>(x + max(0, min(i0 + u * step, (end & ~3) - 4)));
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const int i = i0 + u * step;
+        const bool whole = i + 3 < end, part = i == (end & ~3);
+        xs[u][0] = whole ? v[u].x : part ? rest[0] : -INFINITY;
+        xs[u][1] = whole ? v[u].y : part ? rest[1] : -INFINITY;
+        xs[u][2] = whole ? v[u].z : part ? rest[2] : -INFINITY;
+        xs[u][3] = whole ? v[u].w : -INFINITY;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xs[u][k] = x[min(i0 + u * step + k, end - 1)];
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (i0 + u * step + k >= end) xs[u][k] = -INFINITY;
+    }
+  }
+};
+
+// the four times four elements of thread `tid` from element c0 on
+template <bool VEC, int THREADS>
+__device__ __forceinline__ void smp_load16(const SmpRow<VEC>& x, int c0, int tid, float xs[4][4]) {
+  x.template read<4>(c0 + tid * 4, THREADS * 4, c0 + 16 * THREADS <= x.end, xs);
+}
+
+// the row's maximum from its slices' (at most SMP_SLICES), to every lane
+__device__ __forceinline__ float smp_row_max(const float* part_max, int n_slices) {
+  const int lane = threadIdx.x & (BLM_WAVE - 1);
+  float m = part_max[min(lane, n_slices - 1)];
+#pragma unroll
+  for (int o = SMP_SLICES / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, BLM_WAVE));
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(m)));
+}
+
+// pass 1: the slices' maxima; clears the row's first n_levels histograms for the passes to come
 template <bool VEC, int THREADS>
 __global__ void __launch_bounds__(THREADS)
-    sample_max_kernel(const float* __restrict__ logits, int V, int ld, int slice_len, float* part_max,
-                      SampleRow* rows, unsigned long long* hist, int n_rows, int* counters, int counter_step, int with_hist) {
+    sample_max_kernel(const float* __restrict__ logits, int V, int ld, int slice_len, float* __restrict__ part_max,
+                      unsigned long long* __restrict__ hist, int n_rows, int n_levels, const float* __restrict__ uniforms,
+                      float* __restrict__ row_uniforms) {
   __shared__ float red[17];
-  __shared__ int flag;
   const int row = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x;
-  const float* x = logits + (size_t)row * ld;
+  const float u = slice == 0 ? uniforms[row] : 0.f;   // it may lie in host memory, a longer way than the logits'
   const int begin = slice * slice_len, end = min(V, begin + slice_len);
+  const SmpRow<VEC> x(logits + (size_t)row * ld, end);
   float mx = -INFINITY;
   for (int c0 = begin; c0 < end; c0 += 16 * THREADS) {
     float xs[4][4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) smp_load4<VEC>(x, c0 + (u * THREADS + tid) * 4, end, xs[u]);
+    smp_load16<VEC, THREADS>(x, c0, tid, xs);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int k = 0; k < 4; ++k) mx = fmaxf(mx, xs[u][k]);
   }
+  for (int b = slice * THREADS + tid; b < n_levels * SMP_BINS; b += gridDim.x * THREADS)
+    hist[((size_t)(b / SMP_BINS) * n_rows + row) * SMP_BINS + b % SMP_BINS] = 0ull;
   mx = block_max(mx, red);
-  if (tid == 0) smp_store(part_max + row * SMP_SLICES + slice, mx);
-  if (!smp_arrive_last(counters + (size_t)row * counter_step, &flag, gridDim.x)) return;
-  float m = tid < (int)gridDim.x ? smp_load(part_max + row * SMP_SLICES + tid) : -INFINITY;
-  m = block_max(m, red);
-  if (tid == 0) {
-    rows[row].mx = m;
-    rows[row].prefix = 0u;
-    rows[row].carry = 0ull;
-    rows[row].target = 0ull;
-  }
-  if (with_hist)
-    for (int level = 0; level < 3; ++level)
-      for (int b = tid; b < SMP_BINS; b += THREADS) hist[((size_t)level * n_rows + row) * SMP_BINS + b] = 0ull;
+  if (tid == 0) part_max[row * SMP_SLICES + slice] = mx;
+  if (slice == 0 && tid == 0) row_uniforms[row] = u;
 }
 
-// passes 2 to 4: level 0 takes bits 29..19 of the weights' bit patterns, level 1 bits 18..8, level 2
-// bits 7..0 (e <= 1, so bits 31 and 30 are clear); the last block finds the lowest bin above which
-// less than the target mass lies
-template <bool VEC, int LEVEL, int THREADS>
-__global__ void __launch_bounds__(THREADS)
-    sample_level_kernel(const float* __restrict__ logits, int V, int ld, int slice_len, float k2, float top_p,
-                        SampleRow* rows, unsigned long long* hist, int n_rows, int* counters, int counter_step) {
-  __shared__ unsigned long long bins[SMP_BINS];
-  constexpr int WAVES = THREADS / BLM_WAVE;
-  __shared__ unsigned long long wave_tot[WAVES];
-  __shared__ unsigned long long chosen_above;
-  __shared__ int flag, found;
-  const int row = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x, lane = tid & (BLM_WAVE - 1), w = tid / BLM_WAVE;
-  const float* x = logits + (size_t)row * ld;
-  const int begin = slice * slice_len, end = min(V, begin + slice_len);
-  const float mx = rows[row].mx;
-  const uint32_t prefix = rows[row].prefix;
-  constexpr int shift = LEVEL == 0 ? 19 : (LEVEL == 1 ? 8 : 0);
-  constexpr uint32_t mask = LEVEL == 2 ? 0xffu : 0x7ffu;
-  constexpr int above_bits = LEVEL == 0 ? 0 : (LEVEL == 1 ? 19 : 8);   // the digits above this level start here
-  for (int b = tid; b < SMP_BINS; b += THREADS) bins[b] = 0ull;
-  __syncthreads();
-  for (int c0 = begin; c0 < end; c0 += 16 * THREADS) {
-    float xs[4][4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) smp_load4<VEC>(x, c0 + (u * THREADS + tid) * 4, end, xs[u]);
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float e = __builtin_amdgcn_exp2f((xs[u][k] - mx) * k2);
-        const uint32_t key = __float_as_uint(e);
-        // the digits above this level must be the ones already chosen (none at the first level)
-        if (LEVEL == 0 || (key >> above_bits) == prefix) {
-          const unsigned long long q = (unsigned long long)(e * 4294967296.0f);
-          if (q) atomicAdd(&bins[(key >> shift) & mask], q);
-        }
-      }
-  }
-  __syncthreads();
-  unsigned long long* row_hist = hist + ((size_t)LEVEL * n_rows + row) * SMP_BINS;
-  for (int b = tid; b < SMP_BINS; b += THREADS)
-    if (bins[b]) __hip_atomic_fetch_add(row_hist + b, bins[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (!smp_arrive_last(counters + (size_t)row * counter_step, &flag, gridDim.x)) return;
+template <int THREADS>
+struct SmpChoose {
+  unsigned long long wave_tot[THREADS / BLM_WAVE], above;
+  int found;
+};
 
-  // a thread looks after eight bins in a row, or two
-  constexpr int PER = SMP_BINS / THREADS;
-  unsigned long long m[PER], tot = 0ull;
+// The lowest bin above which less than `target` lies, where `carry` lies above all bins; thread t holds the masses m of bins
+// [t PER, (t + 1) PER).  `first`: the target is top_p of all mass.  carry becomes what lies above the bin.  All threads get the answer.
+template <int THREADS, int PER>
+__device__ __forceinline__ uint32_t smp_choose(const unsigned long long (&m)[PER], bool first, float top_p, unsigned long long& carry,
+                                               unsigned long long& target, SmpChoose<THREADS>& s) {
+  constexpr int WAVES = THREADS / BLM_WAVE;
+  const int tid = threadIdx.x, lane = tid & (BLM_WAVE - 1), w = tid / BLM_WAVE;
+  unsigned long long tot = 0ull;
 #pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    m[j] = smp_load(row_hist + tid * PER + j);
-    tot += m[j];
-  }
+  for (int j = 0; j < PER; ++j) tot += m[j];
   unsigned long long suf = tot;   // becomes the mass of this thread's bins and of all higher threads' bins
 #pragma unroll
   for (int d = 1; d < BLM_WAVE; d <<= 1) {
     const unsigned long long o = shfl_down_u64(suf, d);
     if (lane + d < BLM_WAVE) suf += o;
   }
-  if (tid == 0) found = 0x7fffffff;
-  if (lane == 0) wave_tot[w] = suf;
+  if (lane == 0) s.wave_tot[w] = suf;
   __syncthreads();
-  for (int k = w + 1; k < WAVES; ++k) suf += wave_tot[k];
-  unsigned long long carry = rows[row].carry, target = rows[row].target;
-  if (LEVEL == 0) {
-    // the whole mass: what every bin holds
-    unsigned long long total = wave_tot[0];
-    for (int k = 1; k < WAVES; ++k) total += wave_tot[k];
+  unsigned long long total = 0ull;   // the whole mass: what every bin holds
+#pragma unroll
+  for (int k = 0; k < WAVES; ++k) {
+    const unsigned long long t = s.wave_tot[k];
+    total += t;
+    suf += k > w ? t : 0ull;
+  }
+  if (first) {
     target = (unsigned long long)((double)top_p * (double)total);
     if (target < 1ull) target = 1ull;
   }
   unsigned long long above = carry + suf - tot;   // above this thread's highest bin
-  int mine = -1;
-  unsigned long long mine_above = 0ull;
+  // the bin is the one that reaches the target; exactly one thread has it (an atomic minimum over all threads that lie above is done
+  // lane by lane, 2 us of a pass)
 #pragma unroll
   for (int j = PER - 1; j >= 0; --j) {
-    if (above < target) { mine = tid * PER + j; mine_above = above; }
+    if (above < target && (above + m[j] >= target || tid * PER + j == 0)) { s.found = tid * PER + j; s.above = above; }
     above += m[j];
   }
-  if (mine >= 0) atomicMin(&found, mine);
   __syncthreads();
-  if (found == mine) chosen_above = mine_above;
-  __syncthreads();
-  if (tid == 0) {
-    rows[row].prefix = (prefix << (LEVEL == 2 ? 8 : 11)) | (uint32_t)found;
-    rows[row].carry = chosen_above;
-    rows[row].target = target;
+  const int found = s.found;
+  carry = s.above;
+  __syncthreads();   // the next call may write again
+  return (uint32_t)found;
+}
+
+// passes 2 to 4: level 0 takes bits 29..19 of the weights' bit patterns, level 1 bits 18..8, level 2 bits 7..0 (e <= 1, so bits 31 and
+// 30 are clear).  LIST (level 1): no histogram; the weights with the digits chosen, in any order, and how many; those beyond `capacity`
+// are only counted.
+template <bool VEC, int LEVEL, bool LIST, int THREADS>
+__global__ void __launch_bounds__(THREADS)
+    sample_level_kernel(const float* __restrict__ logits, int V, int ld, int slice_len, float k2, float top_p,
+                        const float* __restrict__ part_max, SampleState* states, unsigned long long* hist, int n_rows,
+                        uint32_t* __restrict__ list, int* __restrict__ counts, int capacity) {
+  __shared__ unsigned long long bins[LIST ? 1 : SMP_BINS];
+  __shared__ SmpChoose<THREADS> choose;
+  __shared__ int listed;
+  const int row = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x;
+  const int begin = slice * slice_len, end = min(V, begin + slice_len);
+  const SmpRow<VEC> x(logits + (size_t)row * ld, end);
+  constexpr int shift = LEVEL == 0 ? 19 : (LEVEL == 1 ? 8 : 0);
+  constexpr uint32_t mask = LEVEL == 2 ? 0xffu : 0x7ffu;
+  constexpr int above_bits = LEVEL == 0 ? 0 : (LEVEL == 1 ? 19 : 8);   // the digits above this level start here
+  float xs[4][4];
+  smp_load16<VEC, THREADS>(x, begin, tid, xs);
+  const float mx = smp_row_max(part_max + row * SMP_SLICES, gridDim.x);
+  uint32_t prefix = 0u;
+  if (LEVEL > 0) {
+    constexpr int PER = SMP_BINS / THREADS;   // a thread looks after eight bins in a row, or two
+    unsigned long long m[PER], carry = 0ull, target = 0ull;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) m[j] = hist[((size_t)(LEVEL - 1) * n_rows + row) * SMP_BINS + tid * PER + j];
+    if (LEVEL == 2) {
+      prefix = states[row].prefix << 11;
+      carry = states[row].carry;
+      target = states[row].target;
+    }
+    prefix |= smp_choose<THREADS, PER>(m, LEVEL == 1, top_p, carry, target, choose);
+    if (slice == 0 && tid == 0) states[(size_t)(LEVEL - 1) * n_rows + row] = SampleState{prefix, carry, target};
   }
+  if (LIST) {
+    if (tid == 0) listed = 0;
+  } else {
+    for (int b = tid; b < SMP_BINS; b += THREADS) bins[b] = 0ull;
+  }
+  __syncthreads();
+  // Level 0: V tokens of weights up to an eighth above `light` have less mass than the 1 - top_p of it that lies below the cut (the heaviest
+  // alone has 2^32), so no bin that holds one of them can be the cut's: those below `light` count for the whole mass only, in the lowest
+  // bin.  Most of a row, as a rule, and a register's add in place of an atomic one each.
+  const float light = LEVEL == 0 ? 0.5f * (1.0f - top_p) / (float)V : 0.f;
+  uint32_t light_mass = 0u;
+  uint32_t* to = LIST ? list + ((size_t)row * gridDim.x + slice) * capacity : nullptr;
+  for (int c0 = begin; c0 < end; c0 += 16 * THREADS) {
+    if (c0 != begin) smp_load16<VEC, THREADS>(x, c0, tid, xs);
+    if (LIST) {
+      uint32_t keys[4][4];
+      unsigned long long who[4][4];   // the lanes whose element is one, by element
+      int n = 0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float e = __builtin_amdgcn_exp2f((xs[u][k] - mx) * k2);
+          keys[u][k] = __float_as_uint(e);
+          who[u][k] = __ballot((keys[u][k] >> above_bits) == prefix && e >= 0x1p-32f);
+          n += __popcll(who[u][k]);
+        }
+      if (n == 0) continue;
+      int at = 0;   // one place for the wavefront's from all of its elements
+      if ((tid & (BLM_WAVE - 1)) == 0) at = atomicAdd(&listed, n);
+      at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int place = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(who[u][k] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)who[u][k], 0u));
+          if (((who[u][k] >> (tid & (BLM_WAVE - 1))) & 1) && place < capacity) to[place] = keys[u][k];
+          at += __popcll(who[u][k]);
+        }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float e = __builtin_amdgcn_exp2f((xs[u][k] - mx) * k2);
+          const uint32_t key = __float_as_uint(e);
+          if (LEVEL == 0) {
+            const bool is_light = e < light;
+            light_mass += is_light ? (uint32_t)(e * 4294967296.0f) : 0u;
+            if (is_light) continue;
+          }
+          // the digits above this level must be the ones already chosen (none at the first level)
+          if (LEVEL == 0 || (key >> above_bits) == prefix) {
+            const unsigned long long q = smp_mass(e);
+            if (q) atomicAdd(&bins[(key >> shift) & mask], q);
+          }
+        }
+    }
+  }
+  if (LEVEL == 0) {
+#pragma unroll
+    for (int o = BLM_WAVE / 2; o > 0; o >>= 1) light_mass += __shfl_xor(light_mass, o, BLM_WAVE);
+    if ((tid & (BLM_WAVE - 1)) == 0 && light_mass) atomicAdd(&bins[0], (unsigned long long)light_mass);
+  }
+  __syncthreads();
+  if (LIST) {
+    if (tid == 0) counts[row * SMP_SLICES + slice] = listed;
+  } else {
+    unsigned long long* row_hist = hist + ((size_t)LEVEL * n_rows + row) * SMP_BINS;
+    for (int b = tid; b < SMP_BINS; b += THREADS)
+      if (bins[b]) __hip_atomic_fetch_add(row_hist + b, bins[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// Levels 1 and 2 from the row's list of weights in level 0's bin; from the row itself where a slice had more than its list holds (flat
+// logits: a bin is an eighth of a power of two wide).  Returns the smallest kept weight.
+template <bool VEC, int THREADS>
+__device__ __forceinline__ uint32_t smp_choose_listed(const float* x, int V, float mx, float k2, SampleState state, const uint32_t* list,
+                                                      const int* counts, int n_slices, int capacity, unsigned long long* bins,
+                                                      SmpChoose<THREADS>& choose) {
+  constexpr int KEPT = 8;
+  const int tid = threadIdx.x, group = THREADS / n_slices, slice = tid / group, first = tid % group;
+  const uint32_t* mine = list + (size_t)slice * capacity;
+  uint32_t keys[KEPT];   // asked for with their number
+#pragma unroll
+  for (int i = 0; i < KEPT; ++i) keys[i] = mine[min(first + i * group, capacity - 1)];
+  const int lane = tid & (BLM_WAVE - 1), any = counts[min(lane, n_slices - 1)], own = counts[slice];
+  const bool over = __ballot(any > capacity) != 0;
+  const int n = over ? 0 : own;
+#pragma unroll
+  for (int i = 0; i < KEPT; ++i) keys[i] = first + i * group < n ? keys[i] : 0u;
+  uint32_t prefix = state.prefix;
+#pragma unroll
+  for (int level = 1; level < 3; ++level) {
+    const int shift = level == 1 ? 8 : 0, above_bits = level == 1 ? 19 : 8;
+    const uint32_t mask = level == 1 ? 0x7ffu : 0xffu;
+    auto add = [&](uint32_t key, int times = 1) {
+      if ((key >> above_bits) != prefix) return;
+      const unsigned long long q = smp_mass(__uint_as_float(key)) * times;
+      if (q) atomicAdd(&bins[(key >> shift) & mask], q);
+    };
+    for (int b = tid; b <= (int)mask; b += THREADS) bins[b] = 0ull;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < KEPT; ++i) add(keys[i]);
+    for (int i = first + KEPT * group; i < n; i += group) add(mine[i]);
+    if (over) {
+      const SmpRow<VEC> whole(x, V);
+      for (int c0 = 0; c0 < V; c0 += 16 * THREADS) {
+        float xs[4][4];
+        smp_load16<VEC, THREADS>(whole, c0, tid, xs);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            // the first lane's weight once for all lanes that hold the same: equal weights would queue up at one bin
+            const uint32_t key = __float_as_uint(__builtin_amdgcn_exp2f((xs[u][k] - mx) * k2)), lead = __builtin_amdgcn_readfirstlane(key);
+            const int same = __popcll(__ballot(key == lead));
+            if (key != lead || (tid & (BLM_WAVE - 1)) == 0) add(key, key == lead ? same : 1);
+          }
+      }
+    }
+    __syncthreads();
+    if (level == 1) {
+      constexpr int PER = SMP_BINS / THREADS;
+      unsigned long long m[PER];
+#pragma unroll
+      for (int j = 0; j < PER; ++j) m[j] = bins[tid * PER + j];
+      prefix = (prefix << 11) | smp_choose<THREADS, PER>(m, false, 0.f, state.carry, state.target, choose);
+    } else {
+      unsigned long long m[1] = {tid < 256 ? bins[tid] : 0ull};
+      prefix = (prefix << 8) | smp_choose<THREADS, 1>(m, false, 0.f, state.carry, state.target, choose);
+    }
+  }
+  return prefix;
 }
 
 // inclusive prefix over the block's first SMP_THREADS threads in thread order, and their total
@@ -336,39 +534,61 @@ __device__ __forceinline__ float smp_block_scan(float v, float* wave_sums, float
   return before + incl;
 }
 
+// *to becomes the lowest (the highest) thread for which `is` holds, if there is one: one atomic for a wavefront
+__device__ __forceinline__ void smp_lowest(int* to, bool is) {
+  const unsigned long long who = __ballot(is);
+  if ((threadIdx.x & (BLM_WAVE - 1)) == 0 && who) atomicMin(to, (int)threadIdx.x + __builtin_ctzll(who));
+}
+__device__ __forceinline__ void smp_highest(int* to, bool is) {
+  const unsigned long long who = __ballot(is);
+  if ((threadIdx.x & (BLM_WAVE - 1)) == 0 && who) atomicMax(to, (int)threadIdx.x + 63 - __builtin_clzll(who));
+}
+
 // last pass: the kept mass of every chunk; the last block finds the chunk that holds the pick and
-// the token in it.  use_tau 0: no cut, every token with a weight is kept.
-template <bool VEC, int THREADS>
+// the token in it.  CUT 0: none, every token with a weight is kept; 1: from the histograms; 2: from the lists.
+template <bool VEC, int CUT, int THREADS>
 __global__ void __launch_bounds__(THREADS)
-    sample_pick_kernel(const float* __restrict__ logits, const float* __restrict__ uniforms, int* __restrict__ out, int V,
-                       int ld, int slice_len, float k2, int use_tau, const SampleRow* rows, float* chunk_mass,
-                       int* counters, int counter_step) {
+    sample_pick_kernel(const float* __restrict__ logits, const float* __restrict__ row_uniforms, int* __restrict__ out, int V,
+                       int ld, int slice_len, float k2, const float* __restrict__ part_max, const SampleState* __restrict__ states,
+                       const unsigned long long* __restrict__ hist, const uint32_t* __restrict__ list, const int* __restrict__ counts,
+                       int capacity, float* chunk_mass, int* counters, int counter_step) {
   __shared__ float red[17];
   constexpr int GROUPS = THREADS / SMP_THREADS, EACH = GROUPS == 1 ? SMP_ROUND : SMP_ROUND / 2, ROUND = EACH * GROUPS;
   __shared__ float wave_sums[THREADS / BLM_WAVE];
   __shared__ float round_sums[ROUND][SMP_WAVES];
   __shared__ int flag, hit, last_with_mass;
+  __shared__ SmpChoose<THREADS> choose;
+  __shared__ unsigned long long bins[CUT == 2 ? SMP_BINS : 1];
   const int row = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x;
   const float* x = logits + (size_t)row * ld;
   const int begin = slice * slice_len, end = min(V, begin + slice_len);
   const int chunks = slice_len / SMP_CHUNK;            // per slice
-  const float mx = rows[row].mx;
-  const uint32_t tau = use_tau ? rows[row].prefix : 0u;   // smallest kept weight, as a bit pattern
+  // the chunks of the slice, ROUND at a time, a chunk to SMP_THREADS of the threads: all loads first, one barrier per round
+  const int group = tid / SMP_THREADS, part = tid % SMP_THREADS;
+  float xs[EACH][4];
+  const SmpRow<VEC> slice_row(x, end);
+  auto load_round = [&](int c0) {
+    slice_row.template read<EACH>(begin + (c0 + group) * SMP_CHUNK + part * 4, GROUPS * SMP_CHUNK, begin + (c0 + ROUND) * SMP_CHUNK <= end, xs);
+  };
+  load_round(0);
+  const float u = row_uniforms[row];
+  const float mx = smp_row_max(part_max + row * SMP_SLICES, gridDim.x);
+  uint32_t tau = 0u;   // smallest kept weight, as a bit pattern
+  if (CUT == 1) {
+    SampleState state = states[gridDim.y + row];
+    const unsigned long long m[1] = {tid < 256 ? hist[((size_t)2 * gridDim.y + row) * SMP_BINS + tid] : 0ull};
+    tau = (state.prefix << 8) | smp_choose<THREADS, 1>(m, false, 0.f, state.carry, state.target, choose);
+  }
+  if (CUT == 2)
+    tau = smp_choose_listed<VEC, THREADS>(x, V, mx, k2, states[row], list + (size_t)row * gridDim.x * capacity, counts + row * SMP_SLICES,
+                                          gridDim.x, capacity, bins, choose);
   auto kept = [&](float v) {
     const float e = __builtin_amdgcn_exp2f((v - mx) * k2);
     return (__float_as_uint(e) >= tau && e > 0.f) ? e : 0.f;
   };
   float* row_mass = chunk_mass + (size_t)row * gridDim.x * chunks;
-  const float u = uniforms[row];   // asked for early: it may lie in host memory
-  // the chunks of the slice, ROUND at a time, a chunk to SMP_THREADS of the threads: all loads first, one barrier per round
-  const int group = tid / SMP_THREADS, part = tid % SMP_THREADS;
   for (int c0 = 0; c0 < chunks; c0 += ROUND) {
-    float xs[EACH][4];
-#pragma unroll
-    for (int r = 0; r < EACH; ++r) {
-      const int c = c0 + r * GROUPS + group;
-      smp_load4<VEC>(x, begin + c * SMP_CHUNK + part * 4, c < chunks ? end : 0, xs[r]);
-    }
+    if (c0) load_round(c0);
     __syncthreads();   // round_sums may still be read from the round before
 #pragma unroll
     for (int r = 0; r < EACH; ++r) {
@@ -424,8 +644,13 @@ __global__ void __launch_bounds__(THREADS)
       run += t;
     }
   }
-  if (first_idx != 0x7fffffff) atomicMin(&hit, first_idx);
-  if (last_idx >= 0) atomicMax(&last_with_mass, last_idx);
+  if (n <= SMP_THREADS) {   // a wavefront's lowest and highest are its first and last lane's that have one
+    smp_lowest(&hit, first_idx != 0x7fffffff);
+    smp_highest(&last_with_mass, last_idx >= 0);
+  } else {
+    if (first_idx != 0x7fffffff) atomicMin(&hit, first_idx);
+    if (last_idx >= 0) atomicMax(&last_with_mass, last_idx);
+  }
   __syncthreads();
   const int chunk = hit != 0x7fffffff ? hit : last_with_mass;   // rounding may leave u * total at the upper edge
   if (chunk < 0) {   // no token has a weight: cannot happen (the maximum has weight 1); answer something valid
@@ -439,19 +664,17 @@ __global__ void __launch_bounds__(THREADS)
   __syncthreads();
   const int cs = chunk / chunks, cc = chunk % chunks;
   const int i0 = cs * slice_len + cc * SMP_CHUNK + tid * 4;
-  float xs[4], es[4];
-  smp_load4<VEC>(x, i0, in ? min(V, cs * slice_len + slice_len) : 0, xs);
+  float es[4];
+  smp_load4<VEC>(x, i0, in ? min(V, cs * slice_len + slice_len) : 0, xs[0]);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) es[k] = kept(xs[k]);
+  for (int k = 0; k < 4; ++k) es[k] = kept(xs[0][k]);
   const float s4 = ((es[0] + es[1]) + es[2]) + es[3];
   float t;
   const float incl = front + smp_block_scan(s4, wave_sums, t);
   if (tid == 0) { hit = 0x7fffffff; last_with_mass = -1; }
   __syncthreads();
-  if (s4 > 0.f) {
-    if (want < incl) atomicMin(&hit, tid);
-    atomicMax(&last_with_mass, tid);
-  }
+  smp_lowest(&hit, s4 > 0.f && want < incl);
+  smp_highest(&last_with_mass, s4 > 0.f);
   __syncthreads();
   const int owner = hit != 0x7fffffff ? hit : last_with_mass;   // at least one thread has a kept token
   if (tid == owner) {
@@ -469,22 +692,21 @@ __global__ void __launch_bounds__(THREADS)
   }
 }
 
-// Blocks per row: a slice's own time falls with their number, the device-wide atomics of all rows' blocks (histograms, arrivals)
-// grow with it and with the rows, so the best number goes with sqrt(V / R): the power of two next to sqrt(V / (16 R)).  Us, with
-// the nucleus cut, for 4 / 8 / 16 / 32 blocks (before: 32 for one or two rows, else 16): 128,256 logits: 1 row 77.1 / 59.4 /
-// 49.7 / 48.0, 8 rows 79.8 / 59.8 / 52.7 / 49.4, 32 rows 82.9 / 63.7 / 59.1 / 66.4, 64 rows 99.9 / 79.6 / 79.6 / 98.8, 128 rows
-// 118.2 / 110.3 / 127.1 / 148.5, 512 rows 292 / 330 / 402 / 590; 32,000 logits: 8 rows 47.1 / 43.9 / 44.0 / 46.1, 64 rows 50.5 /
-// 53.3 / 62.1 / 80.4, 512 rows 131 / 168 / 244 / 429.  (64 blocks win nowhere.)  All with a cache line for each row's arrival
-// counter: side by side, 1,024 blocks queue up at two lines in every pass (64 rows of 128K in 16 blocks 90.5 us).
-// 16 to 64 rows of a large vocabulary: blocks of 1,024 threads, one to a compute unit, which ask for 16,384 tokens at once; 256
-// threads take 2 us for every 4,096, a trip to memory.  (The pick's sums stay those of 256 threads a chunk.)  Us, 256 threads as
-// above / 1,024 threads in 8 blocks a row up to 32 rows, in 4 beyond: 128,256 logits: 8 rows 35.5 / 37.5, 16 rows 38.6 / 38.3, 24 rows
-// 42.8 / 39.7, 32 rows 44.6 / 40.3, 48 rows 52.3 / 48.4, 64 rows 62.4 / 52.4, 128 rows 90 / 88, 256 rows 136 / 151; 50,021 logits: 32
-// rows 41.7 / 43.9, 48 rows 48.5 / 48.0, 64 rows 51.2 / 49.5, 96 rows 62 / 69.  Without the cut's three passes 33 rows 20.6 / 21.8,
-// 48 rows 22.7 / 23.2, 64 rows 28.9 / 24.5 (128,256) and 22.2 / 22.4 (50,021): there only many rows of the largest.
+// Blocks per row: a slice's own time falls with their number, the device-wide atomics of all rows' blocks (histograms, the pick's
+// arrivals) grow with it and with the rows, so the best number goes with sqrt(V / R): the power of two next to sqrt(V / (16 R)).  Us, for
+// 4 / 8 / 16 / 32 blocks, with the nucleus cut: 128,256 logits: 1 row 45.9 / 31.2 / 24.1 / 22.0, 8 rows 46.0 / 31.9 / 25.5 / 23.6, 128 rows
+// 72 / 69 / 72 / 80, 512 rows 221 / 231 / 225 / 251; 32,000 logits: 8 rows 25.1 / 22.6 / 23.6 / 24.6, 512 rows 78 / 96 / 115 / 194; without
+// it: 128,256 logits: 8 rows 13.8 / 10.6 / 9.3 / 9.6, 64 rows 16.7 / 13.9 / 14.1 / 17.9.  All with a cache line for each row's arrival
+// counter: side by side, 1,024 blocks queue up at two lines (64 rows of 128K in 16 blocks, an arrival in every pass, 90.5 us for 79.6).
+// With the cut, 16 to 128 rows: blocks of 1,024 threads, one to a compute unit, that ask for 16,384 tokens at once and take two of the
+// levels from lists, where a slice has at least three quarters of so many.  Us, 256 threads as above / 1,024 threads in 8 blocks a row up
+// to 32 rows, in 4 up to 64, in 2 up to 128: 128,256 logits: 8 rows 23.6 / 25.9, 16 rows 25.7 / 26.0, 24 rows 28.5 / 27.1, 32 rows 29.3 /
+// 27.9, 64 rows 43.7 / 39.6, 96 rows 57.1 / 55.1, 128 rows 68.8 / 64.9, 192 rows (2 blocks) 95.2 / 96.1; 50,021 logits: 32 rows 31.5 / 31.3,
+// 48 rows 37.1 / 34.9, 64 rows 40.6 / 36.0, 128 rows 59.2 / 47.5; 32,000 logits: 64 rows (4 blocks) 28.1 / 28.8, 128 rows 32.2 / 28.6.
+// Without the cut 64 rows of 128,256 logits 13.9 / 15.7.
 static int sample_wide_slices(int R, int V, int cut) {      // 0: 256 threads
-  const int n = R <= 32 ? 8 : 4;
-  return R >= (cut ? 16 : 56) && R <= 64 && V >= n * (cut ? 12288 : 24576) ? n : 0;
+  const int n = R <= 32 ? 8 : R <= 64 ? 4 : 2;
+  return cut && R >= 16 && R <= 128 && V >= n * 12288 ? n : 0;
 }
 static int sample_slices(int R, int V, int cut) {
   if (const int wide = sample_wide_slices(R, V, cut)) return wide;
@@ -497,6 +719,9 @@ static int sample_slice_len(int R, int V, int cut) {
   return ((V + n - 1) / n + SMP_CHUNK - 1) / SMP_CHUNK * SMP_CHUNK;
 }
 
+// How many of a slice's weights a list holds.
+static int sample_list_capacity(int slice_len) { return slice_len / 4; }
+
 // Bytes of scratch that blm_sample needs for R rows of V logits (see there for the layout).
 extern "C" long long blm_sample_scratch_bytes(int R, int V) {
   long long chunks = 0;
@@ -504,12 +729,12 @@ extern "C" long long blm_sample_scratch_bytes(int R, int V) {
     const long long n = (long long)sample_slices(R, V, cut) * (sample_slice_len(R, V, cut) / SMP_CHUNK);
     chunks = n > chunks ? n : chunks;
   }
-  return (long long)R * (3 * SMP_BINS * 8 + sizeof(SampleRow) + SMP_SLICES * 4 + chunks * 4);
+  const long long wide = sample_wide_slices(R, V, 1), lists = wide * sample_list_capacity(sample_slice_len(R, V, 1));
+  return (long long)R * ((wide ? 1 : 3) * SMP_BINS * 8 + 2 * sizeof(SampleState) + SMP_SLICES * 8 + (1 + chunks + lists) * 4);
 }
 
-// scratch: blm_sample_scratch_bytes(R, V) bytes, 8-byte aligned: three histograms per row, the rows'
-// states, the slices' maxima, the chunks' masses.  counters: R zeroed ints, counter_step apart, left
-// zeroed.
+// scratch: blm_sample_scratch_bytes(R, V) bytes, 8-byte aligned: the rows' histograms, their states behind two levels, the slices'
+// maxima and the lengths of their lists, the rows' uniforms, the chunks' masses, the lists.  counters: R zeroed ints, counter_step apart, left zeroed.
 extern "C" int blm_sample(const float* logits, const float* uniforms, int* out, int R, int V, int ld,
                           float temperature, float top_p, void* scratch, int* counters, int counter_step, hipStream_t stream) {
   BLM_REQUIRE(R > 0 && R <= 65535 && V > 0 && ld >= V, "sample: bad sizes R=%d V=%d ld=%d", R, V, ld);
@@ -518,35 +743,52 @@ extern "C" int blm_sample(const float* logits, const float* uniforms, int* out, 
   BLM_REQUIRE(counter_step >= 1, "sample: counters %d apart", counter_step);
   BLM_REQUIRE(scratch != nullptr && ((uintptr_t)scratch % 8) == 0 && counters != nullptr, "sample: scratch and counters needed");
   const int cut = top_p < 1.0f ? 1 : 0;
-  const int slice_len = sample_slice_len(R, V, cut);
-  unsigned long long* hist = reinterpret_cast<unsigned long long*>(scratch);
-  SampleRow* rows = reinterpret_cast<SampleRow*>(hist + (size_t)3 * R * SMP_BINS);
-  float* part_max = reinterpret_cast<float*>(rows + R);
-  float* chunk_mass = part_max + (size_t)R * SMP_SLICES;
-  const float k2 = 1.4426950408889634f / temperature;
-  const bool vec = ld % 4 == 0 && ((uintptr_t)logits % 16) == 0;
+  const int slices = sample_slices(R, V, cut), slice_len = sample_slice_len(R, V, cut), capacity = sample_list_capacity(slice_len);
   const bool wide = sample_wide_slices(R, V, cut) != 0;
-  dim3 grid(sample_slices(R, V, cut), R), block(wide ? 1024 : SMP_THREADS);
-#define SMP_LAUNCH(VEC, THREADS)                                                                                     \
-  do {                                                                                                               \
-    hipLaunchKernelGGL((sample_max_kernel<VEC, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, part_max, rows, \
-                       hist, R, counters, counter_step, cut);                                                        \
-    if (cut) {                                                                                                       \
-      hipLaunchKernelGGL((sample_level_kernel<VEC, 0, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
-                         rows, hist, R, counters, counter_step);                                                     \
-      hipLaunchKernelGGL((sample_level_kernel<VEC, 1, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
-                         rows, hist, R, counters, counter_step);                                                     \
-      hipLaunchKernelGGL((sample_level_kernel<VEC, 2, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
-                         rows, hist, R, counters, counter_step);                                                     \
-    }                                                                                                                \
-    hipLaunchKernelGGL((sample_pick_kernel<VEC, THREADS>), grid, block, 0, stream, logits, uniforms, out, V, ld, slice_len, k2, \
-                       cut, rows, chunk_mass, counters, counter_step);                                               \
+  const int levels = !cut ? 0 : wide ? 1 : 3;
+  unsigned long long* hist = reinterpret_cast<unsigned long long*>(scratch);
+  SampleState* states = reinterpret_cast<SampleState*>(hist + (size_t)levels * R * SMP_BINS);
+  float* part_max = reinterpret_cast<float*>(states + 2 * (size_t)R);
+  int* counts = reinterpret_cast<int*>(part_max + (size_t)R * SMP_SLICES);
+  float* row_uniforms = reinterpret_cast<float*>(counts + (size_t)R * SMP_SLICES);
+  float* chunk_mass = row_uniforms + R;
+  uint32_t* list = reinterpret_cast<uint32_t*>(chunk_mass + (size_t)R * slices * (slice_len / SMP_CHUNK));
+  const float k2 = 1.4426950408889634f / temperature;
+  const bool vec = V >= 4 && ld % 4 == 0 && ((uintptr_t)logits % 16) == 0;
+  dim3 grid(slices, R), block(wide ? 1024 : SMP_THREADS);
+#define SMP_LEVEL(VEC, LEVEL, LIST, THREADS)                                                                              \
+  hipLaunchKernelGGL((sample_level_kernel<VEC, LEVEL, LIST, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, k2, top_p, \
+                     part_max, states, hist, R, list, counts, capacity)
+#define SMP_PICK(VEC, CUT, THREADS)                                                                                       \
+  hipLaunchKernelGGL((sample_pick_kernel<VEC, CUT, THREADS>), grid, block, 0, stream, logits, row_uniforms, out, V, ld, slice_len, k2, \
+                     part_max, states, hist, list, counts, capacity, chunk_mass, counters, counter_step)
+#define SMP_MAX(VEC, THREADS)                                                                                             \
+  hipLaunchKernelGGL((sample_max_kernel<VEC, THREADS>), grid, block, 0, stream, logits, V, ld, slice_len, part_max, hist, R, levels, \
+                     uniforms, row_uniforms)
+#define SMP_LAUNCH(VEC)                                                                                                   \
+  do {                                                                                                                    \
+    if (wide) {                                                                                                           \
+      SMP_MAX(VEC, 1024);                                                                                                 \
+      SMP_LEVEL(VEC, 0, false, 1024);                                                                                     \
+      SMP_LEVEL(VEC, 1, true, 1024);                                                                                      \
+      SMP_PICK(VEC, 2, 1024);                                                                                             \
+    } else if (cut) {                                                                                                     \
+      SMP_MAX(VEC, SMP_THREADS);                                                                                          \
+      SMP_LEVEL(VEC, 0, false, SMP_THREADS);                                                                              \
+      SMP_LEVEL(VEC, 1, false, SMP_THREADS);                                                                              \
+      SMP_LEVEL(VEC, 2, false, SMP_THREADS);                                                                              \
+      SMP_PICK(VEC, 1, SMP_THREADS);                                                                                      \
+    } else {                                                                                                              \
+      SMP_MAX(VEC, SMP_THREADS);                                                                                          \
+      SMP_PICK(VEC, 0, SMP_THREADS);                                                                                      \
+    }                                                                                                                     \
   } while (0)
-  if (vec && wide) SMP_LAUNCH(true, 1024);
-  else if (vec) SMP_LAUNCH(true, SMP_THREADS);
-  else if (wide) SMP_LAUNCH(false, 1024);
-  else SMP_LAUNCH(false, SMP_THREADS);
+  if (vec) SMP_LAUNCH(true);
+  else SMP_LAUNCH(false);
 #undef SMP_LAUNCH
+#undef SMP_MAX
+#undef SMP_PICK
+#undef SMP_LEVEL
   BLM_LAUNCH_CHECK("sample");
   return 0;
 }
