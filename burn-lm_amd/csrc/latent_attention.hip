@@ -690,8 +690,8 @@ extern "C" int blm_latent_attn(const float* qabs, float* olat, int cache_dtype, 
 //                    four score tiles so that the eight rows a lane supplies are neighbours in the
 //                    transposed page (lat_key_of), as in this library's other matrix-core attention.
 // Fragments come straight from global memory (the pages of a sequence are shared by all its wavefronts and
-// stay in the caches); no shared memory, no barriers.  With n_splits > 1 the half pages of a wavefront's columns
-// are cut into pieces whose partial results a second kernel adds up.
+// stay in the caches); no shared memory, no barriers.  With n_splits > 1 the half pages of 16 columns are cut into
+// pieces (latent_attn_pieces_kernel), whose partial results a second kernel adds up.
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ constexpr int lat_key_of(int t, int i) { return (t >> 1) * 32 + (i >> 2) * 8 + (t & 1) * 4 + (i & 3); }
 
@@ -706,15 +706,13 @@ __device__ __forceinline__ uint4 lat_keep_first(uint4 v, int n) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// HALVES: how many 32-row halves of a page a step of the walk takes (2: whole pages, for unsplit runs; 1: a split run is cut
-// into pieces of half pages, and its blocks are single wavefronts so that they spread over the chip)
 #define LATM_WAVES 4
-template <int R, int DR, int HALVES, int WAVES>
-__global__ void __launch_bounds__(WAVES* BLM_WAVE)
+template <int R, int DR>
+__global__ void __launch_bounds__(LATM_WAVES* BLM_WAVE)
     latent_attn_mfma_kernel(const bf16* __restrict__ q, float* __restrict__ olat, const int* __restrict__ cu_seqlens,
                             const int* __restrict__ lens_after, const int* __restrict__ block_table, int table_width,
                             const bf16* __restrict__ kcache, const bf16* __restrict__ vcache, int B, int H,
-                            int tiles_per_seq, float scale2, int n_splits, float* part_o, float* part_ml, int window,
+                            int tiles_per_seq, float scale2, int window,
                             const float* __restrict__ sinks) {
   constexpr int W = R + DR;
   constexpr int KS = (W + 31) / 32;
@@ -722,10 +720,9 @@ __global__ void __launch_bounds__(WAVES* BLM_WAVE)
   static_assert(R % 16 == 0 && W % 8 == 0, "latent lanes in tiles of 16, rows in pieces of 16 bytes");
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
   const int c = lane & 15, kg = lane >> 4;
-  const int tile_id = blockIdx.x * WAVES + wave;          // over sequences x tiles of 16 columns
+  const int tile_id = blockIdx.x * LATM_WAVES + wave;          // over sequences x tiles of 16 columns
   const int b = tile_id / tiles_per_seq, tile = tile_id - b * tiles_per_seq;
   if (b >= B) return;                                            // the last block's surplus wavefronts
-  const int split = blockIdx.y;
   const int t_first = cu_seqlens[b], n_new = cu_seqlens[b + 1] - t_first;
   const int n_cols = n_new * H;
   if (tile * 16 >= n_cols) return;                               // also a padding sequence
@@ -742,11 +739,9 @@ __global__ void __launch_bounds__(WAVES* BLM_WAVE)
   const int max_qpos = past + last_idx / H;
   const int max_key = after - 1;
   const int min_qpos = past + (tile * 16) / H;                   // and the first one reaches furthest back
-  constexpr int ROWS = 32 * HALVES, TILES = 2 * HALVES;
+  constexpr int ROWS = 64, TILES = 4;
   const int u_lo = (window > 0 && min_qpos - window + 1 > 0) ? (min_qpos - window + 1) / ROWS : 0;
-  const int n_units = max_qpos / ROWS + 1 - u_lo;
-  const int per = (n_units + n_splits - 1) / n_splits;
-  const int u_begin = u_lo + split * per, u_end = min(u_lo + n_units, u_begin + per);
+  const int u_end = max_qpos / ROWS + 1;
   const int lo = window > 0 ? qpos - window + 1 : 0;
   const int* bt = block_table + (size_t)b * table_width;
 
@@ -759,18 +754,18 @@ __global__ void __launch_bounds__(WAVES* BLM_WAVE)
       qf[ks] = (valid && (W % 32 == 0 || d < W)) ? *reinterpret_cast<const uint4*>(qrow + d) : make_uint4(0u, 0u, 0u, 0u);
     }
   }
-  const bool sunk = valid && sinks != nullptr && split == 0;      // a sink counts once
+  const bool sunk = valid && sinks != nullptr;
   float m = sunk ? sinks[head] * 1.4426950408889634f : -INFINITY;
   lat_f32x4 l = sunk ? lat_f32x4{1.f, 1.f, 1.f, 1.f} : lat_f32x4{0.f, 0.f, 0.f, 0.f};
   lat_f32x4 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
 
-  for (int u = u_begin; u < u_end; ++u) {
-    const int page = bt[u * ROWS / 64];
-    const int key0 = u * ROWS, row0 = key0 & 63;
-    const bf16* kp = kcache + ((size_t)page * 64 + row0) * W;
-    const bf16* vp = vcache + (size_t)page * R * 64 + row0;
+  for (int u = u_lo; u < u_end; ++u) {
+    const int page = bt[u];
+    const int key0 = u * ROWS;
+    const bf16* kp = kcache + (size_t)page * 64 * W;
+    const bf16* vp = vcache + (size_t)page * R * 64;
     float s[TILES][4];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
@@ -816,7 +811,7 @@ __global__ void __launch_bounds__(WAVES* BLM_WAVE)
     m = m_new;
     const bool tail = key0 + ROWS - 1 > max_key;       // these rows include places past the data: 0 * garbage must stay 0
 #pragma unroll
-    for (int h = 0; h < HALVES; ++h) {
+    for (int h = 0; h < 2; ++h) {
       uint4 pf;
       pf.x = f32x2_to_bf16x2_bits(s[2 * h][0], s[2 * h][1]);
       pf.y = f32x2_to_bf16x2_bits(s[2 * h][2], s[2 * h][3]);
@@ -837,24 +832,151 @@ __global__ void __launch_bounds__(WAVES* BLM_WAVE)
     }
   }
   float* orow = olat + item * R;
-  if (n_splits == 1) {
-    if (valid) {
-      const float inv = 1.0f / l[0];
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-        *reinterpret_cast<float4*>(orow + dt * 16 + kg * 4) = make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
-    }
-    return;
-  }
-  // leave this piece: per column its maximum, sum and unnormalised result; latent_merge_kernel adds the pieces up
-  const size_t gcol = (size_t)tile_id * 16 + c;
-  float* po = part_o + (gcol * n_splits + split) * R;
+  if (!valid) return;
+  const float inv = 1.0f / l[0];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
-    *reinterpret_cast<float4*>(po + dt * 16 + kg * 4) = make_float4(o[dt][0], o[dt][1], o[dt][2], o[dt][3]);
-  if (kg == 0) {
-    part_ml[(gcol * n_splits + split) * 2] = m;
-    part_ml[(gcol * n_splits + split) * 2 + 1] = l[0];
+    *reinterpret_cast<float4*>(orow + dt * 16 + kg * 4) = make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
+}
+
+// The same for a run whose half pages (32 rows) are cut into pieces: a block of four wavefronts to 16 columns and a piece, per column the
+// maximum, the sum and the unnormalised result; latent_merge_kernel adds the pieces up.  Bound by the trip to memory of a half page
+// (68 KB at 512 + 64 lanes): the wavefronts share its lanes, each multiplies a quarter of the rows' lanes (the scores' parts meet in
+// shared memory) and takes a quarter of the latent's, so a lane has a quarter of the loads, all of them asked for at once.
+// A half page to a single wavefront, its values asked for behind the softmax, before; us with the merge, 16 heads of 512 + 64 lanes, before
+// / now: 1 sequence of 1,125 tokens 18.0 / 10.6, 8 of them 27.7 / 16.5, 8 of 4,000 tokens 44.1 / 28.6, 64 of 600 tokens 53.8 / 33.2; of 256 +
+// 64 lanes, 8 of 2,000 tokens 19.9 / 13.2; of 128 + 32, 8 of 300 tokens 8.1 / 7.6.
+template <int R, int DR>
+__global__ void __launch_bounds__(LATM_WAVES* BLM_WAVE, 2)
+    latent_attn_pieces_kernel(const bf16* __restrict__ q, const int* __restrict__ cu_seqlens, const int* __restrict__ lens_after,
+                              const int* __restrict__ block_table, int table_width, const bf16* __restrict__ kcache,
+                              const bf16* __restrict__ vcache, int H, int tiles_per_seq, float scale2, int n_splits,
+                              float* __restrict__ part_o, float* __restrict__ part_ml, int window, const float* __restrict__ sinks) {
+  constexpr int W = R + DR;
+  constexpr int KS = (W + 31) / 32, MY_KS = (KS + LATM_WAVES - 1) / LATM_WAVES;      // pieces of 32 lanes of a row; a wavefront's
+  constexpr int DT = R / 16, MY_DT = (DT + LATM_WAVES - 1) / LATM_WAVES;             // tiles of 16 lanes of the latent; a wavefront's
+  static_assert(R % 16 == 0 && W % 8 == 0, "latent lanes in tiles of 16, rows in pieces of 16 bytes");
+  __shared__ lat_f32x4 scores[2][LATM_WAVES][2][BLM_WAVE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / BLM_WAVE), lane = threadIdx.x & (BLM_WAVE - 1);
+  const int c = lane & 15, kg = lane >> 4;
+  const int b = blockIdx.x / tiles_per_seq, tile = blockIdx.x - b * tiles_per_seq, split = blockIdx.y;
+  const int t_first = cu_seqlens[b], n_new = cu_seqlens[b + 1] - t_first, after = lens_after[b];
+  const int n_cols = n_new * H;
+  if (tile * 16 >= n_cols) return;                               // the whole block; also a padding sequence
+  const int past = after - n_new;
+  const int idx = tile * 16 + c;                                 // this lane's column
+  const bool valid = idx < n_cols;
+  const int tok = valid ? idx / H : 0, head = valid ? idx - tok * H : 0;
+  const int qpos = valid ? past + tok : -1;
+  const size_t item = (size_t)(t_first + tok) * H + head;
+  const int max_qpos = past + min(tile * 16 + 15, n_cols - 1) / H, max_key = after - 1;       // the last column sees the most
+  const int min_qpos = past + (tile * 16) / H;                                               // and the first reaches furthest back
+  const int u_lo = (window > 0 && min_qpos - window + 1 > 0) ? (min_qpos - window + 1) / 32 : 0;
+  const int n_units = max_qpos / 32 + 1 - u_lo, per = (n_units + n_splits - 1) / n_splits;
+  const int u_begin = u_lo + split * per, u_end = min(u_lo + n_units, u_begin + per);
+  const int lo = window > 0 ? qpos - window + 1 : 0;
+  const int* bt = block_table + (size_t)b * table_width;
+
+  const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+  uint4 qf[MY_KS];
+#pragma unroll
+  for (int i = 0; i < MY_KS; ++i) {
+    const int d = (i * LATM_WAVES + wave) * 32 + kg * 8;
+    qf[i] = *reinterpret_cast<const uint4*>(q + item * W + min(d, W - 8));
+    if (!valid || d >= W) qf[i] = zero;
+  }
+  const bool sunk = valid && sinks != nullptr && split == 0;      // a sink counts once
+  float m = sunk ? sinks[head] * 1.4426950408889634f : -INFINITY;
+  lat_f32x4 l = sunk ? lat_f32x4{1.f, 1.f, 1.f, 1.f} : lat_f32x4{0.f, 0.f, 0.f, 0.f};
+  lat_f32x4 o[MY_DT];
+#pragma unroll
+  for (int i = 0; i < MY_DT; ++i) o[i] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
+
+  for (int u = u_begin; u < u_end; ++u) {
+    const int page = bt[u / 2], key0 = u * 32, row0 = key0 & 63;
+    const bf16* kp = kcache + ((size_t)page * 64 + row0) * W;
+    const bf16* vp = vcache + (size_t)page * R * 64 + row0 + kg * 8;
+    uint4 kf[2][MY_KS], va[MY_DT];
+#pragma unroll
+    for (int i = 0; i < MY_KS; ++i)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        kf[t][i] = *reinterpret_cast<const uint4*>(kp + (size_t)lat_key_of(t, c) * W + min((i * LATM_WAVES + wave) * 32 + kg * 8, W - 8));
+#pragma unroll
+    for (int i = 0; i < MY_DT; ++i) va[i] = *reinterpret_cast<const uint4*>(vp + (size_t)(min(i * LATM_WAVES + wave, DT - 1) * 16 + c) * 64);
+    __builtin_amdgcn_sched_barrier(0);      // all of them in front of the first product
+    lat_f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int i = 0; i < MY_KS; ++i)
+      if (i * LATM_WAVES + wave < KS)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          if (W % 32 != 0 && (i * LATM_WAVES + wave) * 32 + kg * 8 >= W) kf[t][i] = zero;
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lat_bf16x8, kf[t][i]), __builtin_bit_cast(lat_bf16x8, qf[i]), acc[t], 0, 0, 0);
+        }
+    const int buf = u & 1;                  // the other one may still be read
+    scores[buf][wave][0][lane] = acc[0];
+    scores[buf][wave][1][lane] = acc[1];
+    __syncthreads();
+    float s[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      lat_f32x4 sum = scores[buf][0][t][lane];
+#pragma unroll
+      for (int w = 1; w < LATM_WAVES; ++w) sum += scores[buf][w][t][lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int kj = key0 + lat_key_of(t, kg * 4 + r);
+        s[t][r] = (kj <= qpos && kj >= lo) ? sum[r] : -INFINITY;      // whatever the rows past the data hold, it is replaced here
+      }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = blm_max(mx, s[t][r]);
+    mx = rows_max(mx);
+    const float m_new = blm_max(m, mx * scale2);
+    const float corr = (m == m_new) ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        s[t][r] = (s[t][r] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], scale2, -m_new));
+    if (__any(m != m_new)) {
+#pragma unroll
+      for (int i = 0; i < MY_DT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[i][r] *= corr;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) l[r] *= corr;
+    }
+    m = m_new;
+    uint4 pf;
+    pf.x = f32x2_to_bf16x2_bits(s[0][0], s[0][1]);
+    pf.y = f32x2_to_bf16x2_bits(s[0][2], s[0][3]);
+    pf.z = f32x2_to_bf16x2_bits(s[1][0], s[1][1]);
+    pf.w = f32x2_to_bf16x2_bits(s[1][2], s[1][3]);
+    // the softmax's denominator: a row of ones in place of V^T sums the rounded probabilities of every column
+    l = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+        __builtin_bit_cast(lat_bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u)), __builtin_bit_cast(lat_bf16x8, pf), l, 0, 0, 0);
+    const bool tail = key0 + 31 > max_key;       // these rows include places past the data: 0 * garbage must stay 0
+    const int keep = max_key - (key0 + kg * 8) + 1;
+#pragma unroll
+    for (int i = 0; i < MY_DT; ++i)
+      if (i * LATM_WAVES + wave < DT) {
+        if (tail) va[i] = lat_keep_first(va[i], keep);
+        o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lat_bf16x8, va[i]), __builtin_bit_cast(lat_bf16x8, pf), o[i], 0, 0, 0);
+      }
+  }
+  const size_t at = ((size_t)blockIdx.x * 16 + c) * n_splits + split;
+#pragma unroll
+  for (int i = 0; i < MY_DT; ++i)
+    if (i * LATM_WAVES + wave < DT)
+      *reinterpret_cast<float4*>(part_o + at * R + (i * LATM_WAVES + wave) * 16 + kg * 4) = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
+  if (wave == 0 && kg == 0) {
+    part_ml[at * 2] = m;
+    part_ml[at * 2 + 1] = l[0];
   }
 }
 
@@ -942,15 +1064,16 @@ extern "C" int blm_latent_attn_mfma(const void* q, float* olat, const int* cu_se
   const long long waves = (long long)B * tiles;
   BLM_REQUIRE(waves < 2147483647LL, "latent_attn_mfma: too many tiles");
   const float scale2 = scale * 1.4426950408889634f;
-#define BLM_LATM_LAUNCH(r, d, halves, per_block)                                                                        \
-  hipLaunchKernelGGL((latent_attn_mfma_kernel<r, d, halves, per_block>),                                               \
-                     dim3((unsigned)((waves + (per_block)-1) / (per_block)), (unsigned)n_splits), dim3((per_block)*BLM_WAVE), 0, stream, \
-                     (const bf16*)q, olat, cu_seqlens, lens_after, block_table, table_width, (const bf16*)kcache,       \
-                     (const bf16*)vcache, B, H, (int)tiles, scale2, n_splits, part_o, part_ml, window, sinks)
 #define BLM_LATM_CASE(r, d)                                                                                            \
   if (R == r && Dr == d) {                                                                                             \
-    if (n_splits == 1) BLM_LATM_LAUNCH(r, d, 2, LATM_WAVES);                                                            \
-    else BLM_LATM_LAUNCH(r, d, 1, 1);                                                                                  \
+    if (n_splits == 1)                                                                                                 \
+      hipLaunchKernelGGL((latent_attn_mfma_kernel<r, d>), dim3((unsigned)((waves + LATM_WAVES - 1) / LATM_WAVES)),      \
+                         dim3(LATM_WAVES * BLM_WAVE), 0, stream, (const bf16*)q, olat, cu_seqlens, lens_after, block_table, table_width, \
+                         (const bf16*)kcache, (const bf16*)vcache, B, H, (int)tiles, scale2, window, sinks);            \
+    else                                                                                                               \
+      hipLaunchKernelGGL((latent_attn_pieces_kernel<r, d>), dim3((unsigned)waves, (unsigned)n_splits), dim3(LATM_WAVES * BLM_WAVE), 0, \
+                         stream, (const bf16*)q, cu_seqlens, lens_after, block_table, table_width, (const bf16*)kcache, \
+                         (const bf16*)vcache, H, (int)tiles, scale2, n_splits, part_o, part_ml, window, sinks);         \
     BLM_LAUNCH_CHECK("latent_attn_mfma");                                                                              \
     if (n_splits > 1) {                                                                                                \
       hipLaunchKernelGGL(latent_merge_kernel,                                                                          \
@@ -962,6 +1085,5 @@ extern "C" int blm_latent_attn_mfma(const void* q, float* olat, const int* cu_se
   }
   BLM_LATM_SIZES(BLM_LATM_CASE)
 #undef BLM_LATM_CASE
-#undef BLM_LATM_LAUNCH
   return blm_fail("latent_attn_mfma: a latent of %d + %d lanes is not among the sizes it is built for", R, Dr);
 }

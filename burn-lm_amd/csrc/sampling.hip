@@ -23,7 +23,7 @@
 // waits for another.  What is asked of all threads (which one has the bin, which are behind the pick) is settled by
 // one thread or one ballot: an atomic on one LDS address is done lane by lane.  And loads stand in no branch of a
 // lane (SmpRow).
-// Blocks of 1,024 threads(see sample_wide_slices) do without two of the passes: the second one lists the weights of
+// Blocks of 1,024 threads (see sample_wide_slices) do without two of the passes: the second one lists the weights of
 // the first level's bin, a few in a hundred of the row's, and the pick's blocks each take the other two levels from
 // the list.  All of it, us, before and now: 64 rows of 128,256 tokens 56.3 and 39.2 (6.3 the maximum, 8.4, 8.5 and
 // 15.2 the pick), 64 rows of 32,000 39.5 and 27.9, a row of 128,256 33.3 and 21.9; without the cut 64 rows 25.2 and

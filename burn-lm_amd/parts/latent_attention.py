@@ -250,9 +250,12 @@ class LatentAttention(Mixer):
             if step.max_new == 1:
                 waves = step.n_seqs * ((H + 15) // 16)
                 halves = (seen + 31) // 32 + (1 if seen < step.max_len_after else 0)     # a window may begin inside a half page
-                # up to a wavefront for every vector unit of the chip: a wavefront waits out a half page's trip from memory
-                # with nothing else to do, so short pieces are what shortens the step
-                n_splits = max(1, min(halves, (4 * rt.compute_units) // waves, MFMA_MAX_PIECES,
+                # up to a block of four wavefronts for every unit of the chip, which waits out a half page's trip from memory with
+                # nothing else to do, so short pieces are what shortens the step; from a block for every fourth unit on up to four
+                # pieces (16 heads, 512 + 64 lanes, us: 8 sequences of 1,125 tokens 32 pieces 16.5, all 36 half pages 19.0; 16 of 600
+                # tokens, 16 / 19 pieces 17.3 / 19.3; 64 of 600, 4 / 8 / 15 pieces 33.2 / 37.2 / 42.3; 128 of 600, 2 / 4 / 7 pieces
+                # 58.7 / 53.6 / 59.6)
+                n_splits = max(1, min(halves, max(rt.compute_units // waves, min(4, 4 * rt.compute_units // waves)), MFMA_MAX_PIECES,
                                       ops.latent_attn_mfma_max_splits(step.n_seqs, 1, H, R)))
             return ops.latent_attn_mfma(qabs, olat, view.k, view.v, step, view.block_table(step), view.page_size, H, R,
                                         dr, self.scale, n_splits, window=self.window, sinks=self.sinks)
