@@ -241,6 +241,10 @@ __global__ void __launch_bounds__(AF_DECODE_WAVES* BLM_WAVE)
                            const float* __restrict__ kcache, const float* __restrict__ vcache, int nh, int nkv, int hd, float scale,
                            int window, int n_splits, float* part_o, float* part_ml, int* arrivals) {
   constexpr int DS = HD / 16;
+  // Lanes past the head are zeroed behind the loads, which then stand in no branch: behind one the values' loads wait for the keys'.
+  // Heads of 64 in groups of four, 8 sequences of 1 / 4 / 9 / 18 pages, us, 5.2 / 9.0 / 12.1 / 16.9 before, 4.7 / 8.1 / 11.6 / 16.7.  Not for heads of 32 (5.9 / 6.0
+  // at 4 pages) nor for wide ones, whose values take the keys' registers (heads of 128, 9 pages 17.3 / 20.5).
+  constexpr bool FREE = HD == 64;
   __shared__ __attribute__((aligned(16))) float all_o[AF_DECODE_WAVES][16][HD + 4];
   __shared__ float all_m[AF_DECODE_WAVES][16], all_l[AF_DECODE_WAVES][16];
   __shared__ int is_last;
@@ -264,7 +268,11 @@ __global__ void __launch_bounds__(AF_DECODE_WAVES* BLM_WAVE)
   const float* qrow = q + (size_t)token * q_row_stride + (size_t)(head0 + min(c, heads - 1)) * hd;
   f32x4 qf[DS];
 #pragma unroll
-  for (int i = 0; i < DS; ++i) qf[i] = i * 16 + g * 4 < hd ? af_load(qrow + i * 16 + g * 4) : zero;
+  for (int i = 0; i < DS; ++i) qf[i] = FREE ? af_load(qrow + min(i * 16 + g * 4, hd - 4)) : i * 16 + g * 4 < hd ? af_load(qrow + i * 16 + g * 4) : zero;
+  if (FREE && hd < HD)
+#pragma unroll
+    for (int i = 0; i < DS; ++i)
+      if (i * 16 + g * 4 >= hd) qf[i] = zero;
   float m = -INFINITY, l = 0.f;
   f32x4 o[DS];
 #pragma unroll
@@ -277,13 +285,22 @@ __global__ void __launch_bounds__(AF_DECODE_WAVES* BLM_WAVE)
 #pragma unroll
     for (int i = 0; i < DS; ++i)
 #pragma unroll
-      for (int t = 0; t < TILES; ++t) kf[i][t] = i * 16 + g * 4 < hd ? af_load(kcache + base + (size_t)((t0 + t) * 16 + c) * hd + i * 16 + g * 4) : zero;
+      for (int t = 0; t < TILES; ++t) {
+        const float* row = kcache + base + (size_t)((t0 + t) * 16 + c) * hd;
+        kf[i][t] = FREE ? af_load(row + min(i * 16 + g * 4, hd - 4)) : i * 16 + g * 4 < hd ? af_load(row + i * 16 + g * 4) : zero;
+      }
     // wide heads: the values' registers are the keys' once these are multiplied
     if (HD > 64) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int d = 0; HD <= 64 && d < DS; ++d)
 #pragma unroll
       for (int t = 0; t < TILES; ++t) vf[d][t] = af_load(vcache + base + (size_t)min(d * 16 + c, hd - 1) * AF_PAGE + (t0 + t) * 16 + g * 4);
+    if (FREE && hd < HD)
+#pragma unroll
+      for (int i = 0; i < DS; ++i)
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+          if (i * 16 + g * 4 >= hd) kf[i][t] = zero;
     f32x4 s[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) s[t] = zero;
