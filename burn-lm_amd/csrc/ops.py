@@ -253,6 +253,21 @@ def _stream():
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda i: torch.cuda.current_stream(i).cuda_stream)
 
 
+_stream_ids = getattr(torch._C, "_cuda_getCurrentStream", None)
+
+
+def mark():
+    """An event recorded on the current stream.  Event.record() without a stream asks torch.cuda.current_stream(), 3 us of Python;
+    torch's own accessor and the Stream made from its answer take 1."""
+    event = torch.cuda.Event()
+    if _stream_ids is None:
+        event.record()
+    else:
+        stream, device, kind = _stream_ids(torch.cuda.current_device())
+        event.record(torch.cuda.Stream(stream_id=stream, device_index=device, device_type=kind))
+    return event
+
+
 def _call(name, *args):
     lib = library()
     if len(args) != len(_SIGNATURES[name]):

@@ -32,6 +32,7 @@ from typing import Dict, Tuple
 import torch
 
 from ..cache import core as _core
+from ..csrc.ops import mark
 from .batch import Step
 
 BATCH_BUCKETS = (1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128)
@@ -161,8 +162,7 @@ class _Captured:
             self.host_np[self.src_at: self.src_at + self.ahead_rows] = -1
             self.ahead_rows = 0
         self.dev.copy_(self.host, non_blocking=True)
-        self.copied = torch.cuda.Event()
-        self.copied.record()
+        self.copied = mark()
         self.graph.replay()
         return self.logits[: entries.n].clone()   # the graph's own output buffer is overwritten by the next replay
 
@@ -179,8 +179,7 @@ class _Captured:
         self.ahead_rows = n
         self.host_cell[0] = tokens_dev.data_ptr()
         self.dev.copy_(self.host, non_blocking=True)
-        self.copied = torch.cuda.Event()
-        self.copied.record()
+        self.copied = mark()
         if not self.folded:
             torch.index_select(tokens_dev, 0, self.src_rows[:n], out=self.step.token_ids[:n])
         self.graph.replay()

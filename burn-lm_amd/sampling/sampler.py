@@ -13,6 +13,8 @@ from typing import List, Sequence
 
 import torch
 
+from ..csrc.ops import mark
+
 _MASK = (1 << 64) - 1
 UNIFORM_RING = 8
 
@@ -41,8 +43,7 @@ class Picked:
         self.device = device_tokens
         self._host = torch.empty(device_tokens.shape, dtype=device_tokens.dtype, pin_memory=True)
         self._host.copy_(device_tokens, non_blocking=True)
-        self._done = torch.cuda.Event()
-        self._done.record()
+        self._done = mark()
 
     def tokens(self) -> List[int]:
         self._done.synchronize()
@@ -104,9 +105,10 @@ class Sampler:
         else:
             slot = self._pinned_uniforms(requests, indices)
             out = ops.sample(logits, slot[0][:logits.shape[0]], self.temperature, self.top_p)
-            slot[1] = torch.cuda.Event()
-            slot[1].record()
-        return Picked(out)
+        picked = Picked(out)
+        if not self.greedy:
+            slot[1] = picked._done        # the copy of the tokens waits for the kernel that reads the buffer
+        return picked
 
     def pick(self, logits: torch.Tensor, requests: Sequence[int], indices: Sequence[int]) -> List[int]:
         """logits float32 [rows, vocab] on the GPU -> one token per row, as host integers."""
