@@ -242,8 +242,8 @@ __global__ void __launch_bounds__(AF_DECODE_WAVES* BLM_WAVE)
                            int window, int n_splits, float* part_o, float* part_ml, int* arrivals) {
   constexpr int DS = HD / 16;
   // Lanes past the head are zeroed behind the loads, which then stand in no branch: behind one the values' loads wait for the keys'.
-  // Heads of 64 in groups of four, 8 sequences of 1 / 4 / 9 / 18 pages, us, 5.2 / 9.0 / 12.1 / 16.9 before, 4.7 / 8.1 / 11.6 / 16.7.  Not for heads of 32 (5.9 / 6.0
-  // at 4 pages) nor for wide ones, whose values take the keys' registers (heads of 128, 9 pages 17.3 / 20.5).
+  // Heads of 64 in groups of four, 8 sequences of 1 / 4 / 9 / 18 pages, us, 5.2 / 9.0 / 12.1 / 16.9 before, 4.7 / 8.1 / 11.6 / 16.7.
+  // Not for heads of 32 (5.9 / 6.0 at 4 pages) nor for wide ones, whose values take the keys' registers (128, 9 pages: 17.3 / 20.5).
   constexpr bool FREE = HD == 64;
   __shared__ __attribute__((aligned(16))) float all_o[AF_DECODE_WAVES][16][HD + 4];
   __shared__ float all_m[AF_DECODE_WAVES][16], all_l[AF_DECODE_WAVES][16];
