@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(MAXT)
         if (c_mode == 0) {
           float s = 0.f;
           for (int w2 = 0; w2 < n_waves; ++w2) s += red[w2 * 256 + idx];
-          if (SCALED) s *= inv[m];
+          if (SCALED) s *= inv[min(m, M - 1)];
           const int nn = tile * 16 + col;
           if (m < M && nn < N) C[(size_t)m * ldc + nn] = from_float<TC>(s);
         } else if (col < 8) {
@@ -260,8 +260,8 @@ __global__ void __launch_bounds__(MAXT)
             u += red[w2 * 256 + idx + 8];
           }
           if (SCALED) {
-            g *= inv[m];
-            u *= inv[m];
+            g *= inv[min(m, M - 1)];
+            u *= inv[min(m, M - 1)];
           }
           const int nn = tile * 8 + col;
           if (EXPERTS) {

@@ -163,3 +163,24 @@ def test_parts_from_outside_run_as_they_are_written():
     assert plain.inside is not None and plain.seam_to(plain) is not None
     assert plain.seam_to(own) is None and own.seam_to(plain) is None and plain.seam_to(object()) is None
     assert block(PreNormBlock, mixer=made(sub(Attention, "forward"))).inside is None
+
+
+@gpu
+@pytest.mark.parametrize("M", [2, 5, 7])
+def test_rows_behind_the_last(M):
+    """A tile has sixteen rows, a product of unscaled rows eight factors at most: rows behind the last, which have none, leave no trace in
+    what lies behind the result, and more rows than there are factors are refused."""
+    from burn_lm_amd.csrc import ops
+    N, K = 96, 128
+    y, sums, inv = unscaled(M, K, torch.bfloat16, 16, seed=M)
+    w = torch.randn(N, K, device="cuda").bfloat16()
+    for gated, columns in ((False, N), (True, N // 2)):
+        packed = ops.pack_weight(w, gated=gated)
+        out = torch.full((16, columns), -7.0, device="cuda")
+        ops.gemv_mfma(y, packed, out[:M], K, gated=gated, scale=(sums, 1e-5))
+        assert bool((out[M:] == -7.0).all()) and bool(out[:M].isfinite().all())
+        more, longer, room = y.repeat(5, 1)[:9], sums.repeat(5, 1)[:9], torch.empty(9, columns, device="cuda")
+        with pytest.raises(ops.KernelError):
+            ops.gemv_mfma(more, packed, room, K, gated=gated, scale=(longer, 1e-5))
+        with pytest.raises(ops.KernelError):
+            ops.gemv_mfma(y, packed, out[:M], K, gated=gated, scale=(sums[:, :6].contiguous(), 1e-5))
