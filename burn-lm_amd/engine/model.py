@@ -9,7 +9,7 @@ import torch
 
 from .. import registry
 from ..models.plan import ModelPlan
-from ..parts.base import TensorSpec
+from ..parts.base import Product, TensorSpec
 
 
 class Model:
@@ -115,6 +115,15 @@ class Model:
             return self.embedding.forward(step.token_ids)
         return self.embedding.forward_from(step.token_ids, *step.token_source)
 
+    def _seam_behind(self, i, step):
+        """The seam behind a place, if the step goes through it: None where its sizes do not, or a block or a part is another by now."""
+        seam = self.seams[i + 1]
+        if seam is None or not seam.takes(step):
+            return None
+        block, after = (self.blocks[p.layer] for p in self.plan.order[i:i + 2])
+        parts = block.parts_to(after) if hasattr(block, "parts_to") else None
+        return seam if parts is not None and seam.stands(*parts) else None
+
     def forward(self, step, cache):
         """Logits (float32, [wanted rows, vocab]) of one step, or None when no row is wanted."""
         both = None      # a loop's rows [x; x0]: the embedding leaves its half there
@@ -126,11 +135,11 @@ class Model:
         for i, place in enumerate(self.plan.order):
             if place.turn is not None:
                 delta = self.entry.enter(h, delta, both, place.turn)
-            block = self.blocks[place.layer]
-            if self.seams[i] is None and self.seams[i + 1] is None:
+            block, after = self.blocks[place.layer], self._seam_behind(i, step)
+            if after is None and not isinstance(delta, Product):
                 delta = block.forward(h, delta, step, cache.views[i])
             else:
-                delta = block.forward_to(h, delta, step, cache.views[i], self.seams[i], self.seams[i + 1])
+                delta = block.forward_to(h, delta, step, cache.views[i], self.seams[i], after)
         if step.n_wanted == 0:
             return None
         x = self.final_norm.add_norm(h, delta, rows=step.want_rows, write_h=False)

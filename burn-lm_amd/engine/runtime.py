@@ -646,6 +646,10 @@ class Runtime:
         return (M <= ops.SCALED_ROWS and isinstance(w, LinearWeight) and not w.gated and w.dtype == self.dtype and w.packable
                 and (w.dtype == torch.float32 or w.shape[0] >= JOIN_BF16_WIDTH) and ops.gemv_join_columns(w.dtype, M, *w.shape) > 0 and w.packed is not None)
 
+    def join_reads(self, x, w):
+        """Whether join takes these rows: of the weights' type, in whole pieces of 16 bytes (an attention's or a gating's own always are)."""
+        return x.dtype == w.dtype and x.dim() == 2 and x.stride(1) == 1 and x.stride(0) * x.element_size() % 16 == 0 and x.data_ptr() % 16 == 0
+
     def join(self, product, h, gamma, eps):
         """h += the product; the rows of an RMS norm with gamma (float32) and eps behind it, Unscaled."""
         x, w = product.x, product.w

@@ -15,25 +15,35 @@ from .base import Block, Product, speaks_for
 
 class Seam:
     """A sublayer, the norm behind it and the sublayer behind that, where the norm's work can be done by the products of the two: the
-    parts speak for what they would do apart (a part from outside that brings its own forward or norm is called by that)."""
+    parts speak for what they would do apart (a part from outside that brings its own forward or norm is called by that, also one that
+    came or was patched after the model was bound)."""
 
     def __init__(self, front, norm, back):
         self.front, self.norm, self.back = front, norm, back
 
     @classmethod
     def between(cls, front, norm, back):
-        fits = (speaks_for(front, "forward_product", "forward", "output", "forward_after_norm") and speaks_for(norm, "joining", "add_norm")
-                and speaks_for(back, "takes_unscaled", "forward", "forward_after_norm", "project", "forward_product")
-                and hasattr(front, "rt") and hasattr(front.rt, "join_takes"))
-        return cls(front, norm, back) if fits else None
+        seam = cls(front, norm, back)
+        return seam if seam.stands(front, norm, back) else None
 
-    def holds(self, step):
+    def stands(self, front, norm, back):
+        """Whether these parts are the seam's, and still speak for themselves."""
+        return (front is self.front and norm is self.norm and back is self.back
+                and speaks_for(front, "forward_product", "forward", "output", "forward_after_norm") and speaks_for(norm, "joining", "add_norm")
+                and speaks_for(back, "takes_unscaled", "forward", "forward_after_norm", "project", "forward_product")
+                and hasattr(front, "rt") and hasattr(front.rt, "join_takes")
+                and (not hasattr(type(front.rt), "linear") or speaks_for(front.rt, "join", "linear", "gated_linear")))
+
+    def takes(self, step):
         # a step that will be recorded chooses by its recording's size, like every form of a result
         tokens = max(step.n_tokens, (getattr(step, "bucket", None) or (0,))[0])
         return self.front.rt.join_takes(tokens, self.front.last_weight()) and self.back.takes_unscaled(tokens)
 
     def run(self, h, product):
-        return self.front.rt.join(product, h, *self.norm.joining())
+        rt = self.front.rt
+        if not rt.join_reads(product.x, product.w):       # rows from outside, in a form that only the plain products take
+            return self.norm.add_norm(h, rt.linear(product.x, product.w, partials=True))
+        return rt.join(product, h, *self.norm.joining())
 
 
 class PreNormBlock(Block):
@@ -43,22 +53,25 @@ class PreNormBlock(Block):
     def bound(self):
         self.inside = Seam.between(self.mixer, self.ffn_norm, self.feed_forward)
 
+    def parts_to(self, after):
+        """The last part of this block, and the norm and the part that the block behind it begins with; None where one of the two
+        blocks is written otherwise."""
+        blocks = all(isinstance(b, PreNormBlock) and speaks_for(b, "forward_to", "forward") for b in (self, after))
+        return (self.feed_forward, after.mixer_norm, after.mixer) if blocks else None
+
     def seam_to(self, after):
         """The Seam between this block and the one behind it, or None."""
-        if not all(isinstance(b, PreNormBlock) and speaks_for(b, "forward_to", "forward") for b in (self, after)):
-            return None
-        return Seam.between(self.feed_forward, after.mixer_norm, after.mixer)
+        parts = self.parts_to(after)
+        return None if parts is None else Seam.between(*parts)
 
     def forward(self, h, delta, step, view):
         return self.forward_to(h, delta, step, view, None, None)
 
     def forward_to(self, h, delta, step, view, before, after):
-        """forward between two seams (or None): a delta that is a Product is run with the seam before, and the result comes as a Product
-        where the seam after holds."""
+        """forward between two seams: a delta that is a Product is run with the seam before, and the result comes as a Product
+        for the seam after, which holds in this step (or is None)."""
         x = before.run(h, delta) if isinstance(delta, Product) else self.mixer_norm.add_norm(h, delta)
-        if after is not None and not after.holds(step):
-            after = None
-        if self.inside is not None and self.inside.holds(step):
+        if self.inside is not None and self.inside.takes(step) and self.inside.stands(self.mixer, self.ffn_norm, self.feed_forward):
             x = self.inside.run(h, self.mixer.forward_product(x, step, view))
         else:
             a = self.mixer.forward(x, step, view)

@@ -184,3 +184,113 @@ def test_rows_behind_the_last(M):
             ops.gemv_mfma(more, packed, room, K, gated=gated, scale=(longer, 1e-5))
         with pytest.raises(ops.KernelError):
             ops.gemv_mfma(y, packed, out[:M], K, gated=gated, scale=(sums[:, :6].contiguous(), 1e-5))
+
+
+class Log(list):
+    def word(self, what, answer):
+        return lambda *a, **k: (self.append(what), answer)[1]
+
+
+def two_blocks(log):
+    """Two blocks of recording parts on the CPU whose seams all hold, as a bound model has them."""
+    from types import SimpleNamespace
+
+    from burn_lm_amd.engine.model import Model
+    from burn_lm_amd.parts.attention import Attention
+    from burn_lm_amd.parts.base import Product
+    from burn_lm_amd.parts.block import PreNormBlock
+    from burn_lm_amd.parts.norm_rms import RMSNorm
+    from burn_lm_amd.parts.swiglu import SwiGLU
+
+    class Runtime:
+        join_takes = lambda self, tokens, w: tokens <= 8
+        join_reads = lambda self, x, w: True
+        join = lambda self, *a: log.word("join", "rows")()
+        linear = lambda self, *a, **k: log.word("linear", "delta")()
+        gated_linear = linear
+
+    rt = Runtime()
+
+    def recording(cls, name, **words):
+        own = dict(takes_unscaled=lambda self, tokens: True, last_weight=lambda self: None, **words)
+        part = type(name, (cls,), own).__new__(type(name, (cls,), own))
+        part.rt = rt
+        return part
+
+    def sublayer(cls, name):
+        return recording(cls, name, forward=lambda self, *a: log.word(name + ".forward", "delta")(),
+                         forward_after_norm=lambda self, *a: log.word(name + ".forward_after_norm", "delta")(),
+                         forward_product=lambda self, *a: Product(log.word(name + ".forward_product", "x")(), "w"))
+
+    def norm(name):
+        return recording(RMSNorm, name, add_norm=lambda self, *a, **k: log.word(name + ".add_norm", "rows")(), joining=lambda self: ("gamma", 1e-5))
+
+    model = Model.__new__(Model)
+    model.blocks = [PreNormBlock(dict(mixer_norm=norm(f"n{i}"), mixer=sublayer(Attention, f"mixer{i}"), ffn_norm=norm(f"m{i}"),
+                                      feed_forward=sublayer(SwiGLU, f"ffn{i}"))) for i in range(2)]
+    for b in model.blocks:
+        b.bound()
+    model.seams = [None, model.blocks[0].seam_to(model.blocks[1]), None]
+    model.plan = SimpleNamespace(order=[SimpleNamespace(layer=i, turn=None) for i in range(2)])
+    model.entry = None
+    model._embed = lambda step, copy: ("h", None)
+    model.embedding = object()
+
+    def run(tokens=3):
+        del log[:]
+        model.forward(SimpleNamespace(n_tokens=tokens, n_wanted=0), SimpleNamespace(views=[None, None]))
+        return list(log)
+
+    return model, rt, run
+
+
+def test_parts_that_change_behind_the_binding_run_as_they_are():
+    """A part, a norm, a block or a runtime that is patched or exchanged after a model was bound is called by its own words, as in steps
+    of many tokens."""
+    log = Log()
+    joined = ["n0.add_norm", "mixer0.forward_product", "join", "ffn0.forward_product", "join", "mixer1.forward_product", "join", "ffn1.forward"]
+    plain = ["n0.add_norm", "mixer0.forward", "ffn0.forward_after_norm", "n1.add_norm", "mixer1.forward", "ffn1.forward_after_norm"]
+    model, rt, run = two_blocks(log)
+    assert run() == joined and run(9) == plain
+
+    model.blocks[1].mixer.forward = log.word("patched", "delta")
+    assert run() == joined[:3] + ["ffn0.forward", "n1.add_norm", "patched", "ffn1.forward_after_norm"]
+    model, rt, run = two_blocks(log)
+    model.blocks[0].ffn_norm.add_norm = log.word("patched", "rows")
+    assert run() == ["n0.add_norm", "mixer0.forward", "patched", "ffn0.forward_product"] + joined[4:]
+    model, rt, run = two_blocks(log)
+    model.blocks[0].feed_forward = two_blocks(log)[0].blocks[1].feed_forward
+    assert run() == ["n0.add_norm", "mixer0.forward", "ffn1.forward_after_norm", "n1.add_norm"] + joined[5:]
+    model, rt, run = two_blocks(log)
+    model.blocks[1].forward = log.word("patched", "delta")
+    assert run() == joined[:3] + ["ffn0.forward", "patched"]
+    model, rt, run = two_blocks(log)
+    model.blocks[0].forward = log.word("patched", "delta")
+    assert run() == ["patched", "n1.add_norm"] + joined[5:]
+    model, rt, run = two_blocks(log)
+    model.blocks[1] = type("Own", (), dict(forward=lambda self, *a: log.word("own", "delta")()))()
+    assert run() == joined[:3] + ["ffn0.forward", "own"]
+    for word in ("linear", "gated_linear"):
+        model, rt, run = two_blocks(log)
+        setattr(rt, word, log.word("patched", "delta"))
+        assert run() == plain
+
+
+def test_rows_from_outside_go_through_the_plain_products():
+    """Rows that a part from outside hands on in another form than the joined product reads (a stride, an address, a type) take the product
+    and the norm's kernel that they took without the seam."""
+    from types import SimpleNamespace
+
+    from burn_lm_amd.engine.runtime import LinearWeight, Runtime
+    rt = Runtime.__new__(Runtime)
+    w = LinearWeight(torch.zeros(32, 16, dtype=torch.bfloat16))
+    x = torch.zeros(4, 40, dtype=torch.bfloat16)
+    assert rt.join_reads(x[:, :16], w) and rt.join_reads(x[1:, 8:24], w)
+    for rows in (x[:, 1:17], x[:, ::2][:, :16], x[:, :16].float(), x.view(-1)[:144].view(4, 36)[:, :16], x[:, :16].t().contiguous().t()):
+        assert not rt.join_reads(rows, w)
+
+    log = Log()
+    model, rt, run = two_blocks(log)
+    type(rt).join_reads = lambda self, x, w: False
+    assert run() == ["n0.add_norm", "mixer0.forward_product", "linear", "m0.add_norm", "ffn0.forward_product", "linear", "n1.add_norm",
+                     "mixer1.forward_product", "linear", "m1.add_norm", "ffn1.forward"]
