@@ -32,10 +32,14 @@ __device__ __forceinline__ float mg_gated(float g, float up, float weight) { ret
 // weights [T][ld]: an expert's weight for a token, zero where it is not chosen.  lists [E][T]: plane rows place * T + token of
 // the tokens that chose expert e, with the weight's bits beside them (one trip to memory at the start of a tile); counts [E].  Blocks
 // behind the first E zero the plane rows of places that no expert takes.
-// TABLE: a table [V][top] of the token ids names a token's experts instead, each with the weight 1 / top (an id outside it chooses none; the id
-// is (*source)[source_rows[t]] where that row number is there and not negative, else ids[t]): a kernel less than with the weights made
-// first.  What bounds it are trips to memory in a row, so the tokens of four rounds of threads are asked for at once (2,048 tokens, 16 experts, 4 of
-// them a token, under the profiler: weights and lists 5.1 + 6.3 us, a round after the other 13.3, so 10.9 and a launch less).
+// N: a table [V][top] of the token ids, top up to N = 4 or 8, names a token's experts instead, each with the weight 1 / top (an id outside it
+// chooses none; the id is (*source)[source_rows[t]] where that row number is there and not negative, else ids[t]): a kernel less than with
+// the weights made first (N = 0).  What bounds it are trips to memory in a row, so the tokens of four rounds of threads are asked for at once
+// (2,048 tokens, 16 experts, 4 of them a token, under the profiler: weights and lists 5.1 + 6.3 us, a round after the other 13.3, so 10.9
+// and a launch less), and with many tokens the comparing of a row's entries.  A call with products of width 64, in a graph, us, weights / table: 16 experts,
+// 4 a token, 512 / 2,048 / 8,192 tokens 31.4 / 28.1, 36.2 / 32.0, 52.4 / 44.6; 64 experts, 8 a token, 35.8 / 30.0, 46.9 / 36.6, 111.5 / 77.4;
+// 16 experts, 8 a token, 8,192 and 16,384 tokens 76.2 / 76.8 and 124.2 / 127.5.  Longer rows, which every expert would read and compare for
+// every token, are made weights first (64 experts, 16 a token, 2,048 tokens 50.6 / 115; 128 experts, 64 a token 150 / 1,830).
 struct MgTable {
   const int *table, *ids, *source_rows;
   const int* const* source;
@@ -47,45 +51,37 @@ __device__ __forceinline__ const int* mg_table_row(const MgTable& by, int t, int
   return (unsigned)id < (unsigned)by.V ? by.table + (size_t)id * top : nullptr;
 }
 #define MG_AHEAD 4
-#define MG_ENTRIES 8      // of a row that are held in registers
-// whether entry k of a row names its expert for the first time
-__device__ __forceinline__ bool mg_first(const int* row, int k) {
-  bool first = true;
-  for (int j = 0; j < k; ++j) first &= row[j] != row[k];
-  return first;
-}
-// the first entries of a row, in one or two loads where they allow (places past the row's end repeat its last)
-__device__ __forceinline__ void mg_entries(const int* row, int top, bool fours, int (&v)[MG_ENTRIES]) {
+#define MG_ENTRIES 8      // most of a row: they are held in registers
+// the entries of a row, in one or two loads where they allow (places past the row's end repeat its last)
+template <int N>
+__device__ __forceinline__ void mg_entries(const int* row, int top, bool fours, int (&v)[N]) {
   if (fours) {
-    const int4 a = *reinterpret_cast<const int4*>(row), b = *reinterpret_cast<const int4*>(row + (top > 4 ? 4 : 0));
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+#pragma unroll
+    for (int k = 0; k < N; k += 4) {
+      const int4 a = *reinterpret_cast<const int4*>(row + (k < top ? k : 0));
+      v[k] = a.x; v[k + 1] = a.y; v[k + 2] = a.z; v[k + 3] = a.w;
+    }
   } else {
 #pragma unroll
-    for (int k = 0; k < MG_ENTRIES; ++k) v[k] = row[min(k, top - 1)];
+    for (int k = 0; k < N; ++k) v[k] = row[min(k, top - 1)];
   }
 }
-// whether a row names expert e, and how many experts in front of it
-__device__ __forceinline__ bool mg_named(const int* row, const int (&v)[MG_ENTRIES], int top, int e, int& place) {
+// whether a row of `top` entries names expert e, and how many experts in front of it (an entry that repeats counts once)
+template <int N>
+__device__ __forceinline__ bool mg_named(const int (&v)[N], int top, int e, int& place) {
   bool in = false;
   place = 0;
-  if (top <= MG_ENTRIES) {
 #pragma unroll
-    for (int k = 0; k < MG_ENTRIES; ++k) {
-      bool first = k < top;
+  for (int k = 0; k < N; ++k) {
+    bool first = k < top;
 #pragma unroll
-      for (int j = 0; j < k; ++j) first &= v[j] != v[k];
-      in |= first && v[k] == e;
-      place += first && v[k] < e;
-    }
-  } else {
-    for (int k = 0; k < top; ++k) {
-      in |= row[k] == e;
-      if (row[k] < e) place += mg_first(row, k);
-    }
+    for (int j = 0; j < k; ++j) first &= v[j] != v[k];
+    in |= first && v[k] == e;
+    place += first && (unsigned)v[k] < (unsigned)e;
   }
   return in;
 }
-template <bool TABLE>
+template <int N>
 __global__ void __launch_bounds__(1024)
     moe_lists_kernel(const float* __restrict__ weights, int ld, MgTable by, int T, int E, int top, int2* __restrict__ lists, int* __restrict__ counts,
                      float* __restrict__ planes, int D) {
@@ -93,17 +89,19 @@ __global__ void __launch_bounds__(1024)
   __shared__ int taken[64];
   __shared__ unsigned long long short_of;      // of 64 tokens those with fewer experts than places
   const int tid = threadIdx.x, wave = tid / BLM_WAVE, lane = tid & (BLM_WAVE - 1);
-  const bool fours = top % 4 == 0 && top <= MG_ENTRIES && ((uintptr_t)by.table & 15) == 0;
+  constexpr bool TABLE = N > 0;
+  constexpr int HELD = TABLE ? N : 1;
+  const bool fours = top % 4 == 0 && ((uintptr_t)by.table & 15) == 0;
   if ((int)blockIdx.x >= E) {
     const int t0 = ((int)blockIdx.x - E) * 64;
     if (tid < 64) {
       int n = top;
-      if (TABLE) {
+      if constexpr (TABLE) {
         if (t0 + tid < T) {
           const int* row = mg_table_row(by, t0 + tid, top);
-          int entries[MG_ENTRIES];
-          mg_entries(row != nullptr ? row : by.table, top, fours, entries);
-          mg_named(row, entries, row != nullptr ? top : 0, 0x7fffffff, n);
+          int entries[HELD];
+          mg_entries<HELD>(row != nullptr ? row : by.table, top, fours, entries);
+          mg_named<HELD>(entries, row != nullptr ? top : 0, E, n);
         }
       } else if (t0 + tid < T) {
         n = 0;
@@ -124,25 +122,25 @@ __global__ void __launch_bounds__(1024)
   const int e = blockIdx.x;
   int base = 0;
   const int* rows[MG_AHEAD];
-  int entries[MG_AHEAD][MG_ENTRIES];
+  int entries[MG_AHEAD][HELD];
   for (int t0 = 0, ahead = 0; t0 < T; t0 += 1024, ++ahead) {
     const int t = t0 + tid;
     bool in = false;
     int place = 0;
     float weight = 1.0f / (float)top;
-    if (TABLE) {
+    if constexpr (TABLE) {
       if (ahead % MG_AHEAD == 0) {
 #pragma unroll
         for (int i = 0; i < MG_AHEAD; ++i) rows[i] = mg_table_row(by, min(t + i * 1024, T - 1), top);
 #pragma unroll
-        for (int i = 0; i < MG_AHEAD; ++i) mg_entries(rows[i] != nullptr ? rows[i] : by.table, top, fours, entries[i]);
+        for (int i = 0; i < MG_AHEAD; ++i) mg_entries<HELD>(rows[i] != nullptr ? rows[i] : by.table, top, fours, entries[i]);
       }
-      in = mg_named(rows[0], entries[0], rows[0] != nullptr && t < T ? top : 0, e, place);
+      in = mg_named<HELD>(entries[0], rows[0] != nullptr && t < T ? top : 0, e, place);
 #pragma unroll
       for (int i = 0; i + 1 < MG_AHEAD; ++i) {
         rows[i] = rows[i + 1];
 #pragma unroll
-        for (int k = 0; k < MG_ENTRIES; ++k) entries[i][k] = entries[i + 1][k];
+        for (int k = 0; k < HELD; ++k) entries[i][k] = entries[i + 1][k];
       }
     } else {
       const float* row = weights + (size_t)t * ld;
@@ -490,13 +488,13 @@ __global__ void __launch_bounds__(512, 2)
 // x [T][ldx], w_gate_up [2 E f][D] (the experts' gates, then their ups), w_down [D][E f], weights [T][ld_weights] float;
 // planes [top][T][D] float; lists [E * T] pairs of ints, counts [E] ints and act [T * top][f] are workspaces of the call.  No token has more
 // than top weights that are not zero.
-// weights null: a table of the token ids chooses (moe_lists; its rows' entries differ and lie in [0, E)).
+// weights null: a table of the token ids chooses (moe_lists; up to MG_ENTRIES experts a token, entries in [0, E)).
 extern "C" int blm_moe_grouped(const void* x, int ldx, const void* w_gate_up, const void* w_down, const float* weights, int ld_weights,
                                const int* table, const int* ids, const int* source_rows, const void* source_cell, int V,
                                float* planes, int* lists, int* counts, void* act, int T, int D, int E, int f, int top,
                                int units, hipStream_t stream) {
-  BLM_REQUIRE(weights != nullptr || (table != nullptr && ids != nullptr && V > 0 && (source_rows == nullptr) == (source_cell == nullptr)),
-              "moe_grouped: weights, or a table with its token ids");
+  BLM_REQUIRE(weights != nullptr || (table != nullptr && ids != nullptr && V > 0 && top <= MG_ENTRIES && (source_rows == nullptr) == (source_cell == nullptr)),
+              "moe_grouped: weights, or a table of up to %d experts a token with its token ids", MG_ENTRIES);
   BLM_REQUIRE(T > 0 && E > 0 && E <= MG_MAX_EXPERTS && top > 0 && top <= 64 && top <= E && D % MG_BK == 0 && f % MG_BK == 0 && D > 0 && f > 0,
               "moe_grouped: sizes T=%d D=%d experts=%d of %d, top=%d not supported", T, D, E, f, top);
   BLM_REQUIRE(ldx >= D && ldx % 8 == 0 && (weights == nullptr || ld_weights >= E) && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w_gate_up % 16) == 0 &&
@@ -505,10 +503,12 @@ extern "C" int blm_moe_grouped(const void* x, int ldx, const void* w_gate_up, co
               "moe_grouped: operands of 4 GiB and more");
   const MgTable by{table, ids, source_rows, (const int* const*)source_cell, V};
   const dim3 list_blocks((unsigned)(E + (T + 63) / 64));
-  if (weights)
-    hipLaunchKernelGGL(moe_lists_kernel<false>, list_blocks, dim3(1024), 0, stream, weights, ld_weights, by, T, E, top, (int2*)lists, counts, planes, D);
-  else
-    hipLaunchKernelGGL(moe_lists_kernel<true>, list_blocks, dim3(1024), 0, stream, weights, ld_weights, by, T, E, top, (int2*)lists, counts, planes, D);
+#define BLM_ML(N) \
+  hipLaunchKernelGGL(moe_lists_kernel<N>, list_blocks, dim3(1024), 0, stream, weights, ld_weights, by, T, E, top, (int2*)lists, counts, planes, D)
+  if (weights) BLM_ML(0);
+  else if (top <= 4) BLM_ML(4);
+  else BLM_ML(MG_ENTRIES);
+#undef BLM_ML
   BLM_LAUNCH_CHECK("moe_lists");
   const long long row_tiles = ((long long)T * top + MG_BM - 1) / MG_BM + E;       // every expert's last tile may be part empty
   const long long halves = ((long long)T * top + GD_TILE / 2 - 1) / (GD_TILE / 2) + E;

@@ -1827,11 +1827,16 @@ def compute_units(index):
     return torch.cuda.get_device_properties(index).multi_processor_count
 
 
+GROUPED_TABLE_TOP = 8
+
+
 def moe_grouped(x, w_gate_up, w_down, weights, n_experts, top, table=None, ids=None, token_source=None):
     """float32 planes [top, T, D] whose sum is ``sum_e weights[t, e] * W_down_e (silu(W_gate_e x) * (W_up_e x))``: every token
     by its own experts only (those with a weight that is not zero, at most `top` of a token).  bfloat16 x [T, D], w_gate_up
     [2 E f, D] (the experts' gates, then their ups), w_down [D, E f]; weights float32 [T, E + 1] (the last column is not read), or
-    None and a table (int32 [vocabulary, top], entries in [0, E)) of the token ids [T] (token_source: see moe_table)."""
+    None and a table (int32 [vocabulary, top], entries in [0, E)) of the token ids [T] (token_source: see moe_table).  The lists are made
+    from the table itself where it has up to GROUPED_TABLE_TOP experts a token; longer rows, which every expert would read and compare
+    for every token, are made weights first (moe_table)."""
     _gpu(x, w_gate_up, w_down, weights, table, ids)
     T, D = x.shape
     f = w_down.shape[1] // n_experts
@@ -1851,6 +1856,10 @@ def moe_grouped(x, w_gate_up, w_down, weights, n_experts, top, table=None, ids=N
             _i32("source_rows", rows, T)
             if cell.dtype != torch.int64 or cell.numel() != 1:
                 raise KernelError("moe_grouped: the cell is one int64 on the device")
+        if top > GROUPED_TABLE_TOP:
+            weights = torch.empty(T, n_experts + 1, dtype=torch.float32, device=x.device)
+            moe_table(table, ids, weights, n_experts, token_source)
+            table = ids = rows = cell = None
     if tuple(w_gate_up.shape) != (2 * n_experts * f, D) or tuple(w_down.shape) != (D, n_experts * f):
         raise KernelError("moe_grouped: w_gate_up [2 E f, D], w_down [D, E f]")
     planes = torch.empty(top, T, D, dtype=torch.float32, device=x.device)

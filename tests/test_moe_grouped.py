@@ -228,3 +228,22 @@ def test_gating_is_float32(T):
         a, b = ((want * (1 + e * 2.0 ** -21)).bfloat16().float() for e in (-1, 1))
         wrong += int(((y < torch.minimum(a, b)) | (y > torch.maximum(a, b))).sum())
     assert wrong == 0
+
+
+@pytest.mark.parametrize("T,E,top,f,D", [(700, 64, 16, 64, 64), (200, 200, 33, 64, 64), (1300, 9, 9, 64, 64), (1300, 16, 8, 64, 64), (900, 16, 3, 64, 64)])
+def test_a_table_of_many_experts_a_token(T, E, top, f, D, monkeypatch):
+    """Rows of up to eight experts make the lists themselves, longer ones (which every expert would compare entry by entry for every token)
+    are made weights first; the same bits, also with entries that name no expert."""
+    from burn_lm_amd.csrc import ops
+    g = torch.Generator().manual_seed(T + top)
+    x, gu, down = (torch.randn(*s, generator=g).bfloat16().cuda() for s in ((T, D), (2 * E * f, D), (D, E * f)))
+    table = torch.rand(50, E, generator=g).argsort(1)[:, :top].int()
+    table[3, 1] = table[3, 0]
+    table[4, 0], table[4, 2], table[5, 1] = -1, E, -2 ** 31
+    table, ids = table.cuda(), torch.randint(0, 50, (T,), generator=g).int().cuda()
+    weights = torch.empty(T, E + 1, device="cuda")
+    ops.moe_table(table, ids, weights, E)
+    want, calls, real = ops.moe_grouped(x, gu, down, weights, E, top), [], ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    assert torch.equal(ops.moe_grouped(x, gu, down, None, E, top, table=table, ids=ids), want)
+    assert calls == (["blm_moe_table"] if top > 8 else []) + ["blm_moe_grouped"]
