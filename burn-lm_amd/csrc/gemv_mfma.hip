@@ -291,11 +291,19 @@ __global__ void __launch_bounds__(MAXT)
 // current tile is multiplied and reduced (and the first tile's before the activations), so the
 // memory pipeline never idles while the block synchronises; with 16 k-steps the registers do not
 // allow it.
+// EXPERTS: weights from the array, a tile's asked for in front of the next tile's weights (behind them they would wait for them); the gating, some
+// hundred instructions on one or two wavefronts a vector unit, is what bounds it, so every thread has a pair (also without weights), rows without
+// the expert skip it, one barrier a tile does and few wavefronts come in 512 blocks.  Us, product and weighting pass apart / weights
+// asked for in the epilogue, two barriers, half of the threads idle / so: 16 experts of 512, K = 2,048, 17 / 32 / 64 rows 18.6 / 18.8 / 17.5,
+// 20.1 / 19.6 / 18.2, 24.2 / 25.4 / 22.2; 64 of 256, K = 2,048, 17 and 64 rows 29.0 / 30.1 / 27.6 and 35.1 / 38.8 / 32.0; 128 of 128, K = 1,024
+// 19.6 / 22.6 / 17.8 and 23.8 / 31.7 / 23.9 (48 rows 21.3 / 27.2 / 21.8); 128 of 128, K = 512, 64 rows 23.2 / - / 17.9; 8 of 128, K = 1,024 10.9 /
+// 9.5 / 8.6.
 template <int MT, int KSTEPS, bool PREFETCH, bool EXPERTS, typename TC>
 __global__ void __launch_bounds__(512)
     gemv_mfma_rows_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wp, TC* __restrict__ C, int M, int N,
                           int K, int lda, int ldc, int n_tiles, int k_steps, int c_mode, int steps_per_group, GvExperts ex) {
-  extern __shared__ float red[];  // [waves][MT][256]
+  extern __shared__ float both[];  // [waves][MT][256], twice for EXPERTS: the tiles take turns, and one barrier a tile will do
+  __shared__ float share_of[2][EXPERTS ? MT * 16 : 1];      // the rows' weights for the tile's expert
   const int wave = threadIdx.x / BLM_WAVE, lane = threadIdx.x & (BLM_WAVE - 1);
   const int n_waves = blockDim.x / BLM_WAVE;
   const int row = lane & 15, kg = lane >> 4;
@@ -335,6 +343,11 @@ __global__ void __launch_bounds__(512)
   }
 
   for (int tile = tile_begin; tile < tile_end; ++tile) {
+    float share_next = 0.f;
+    const int turn = EXPERTS ? (tile - tile_begin) & 1 : 0;
+    float* red = both + turn * n_waves * MT * 256;
+    // asked for in front of the next tile's weights: behind them it would wait for them
+    if (EXPERTS) share_next = ex.weights[(size_t)min((int)threadIdx.x, M - 1) * (ex.E + 1) + min(tile * 8 / ex.ffe, ex.E)];
     if (PREFETCH) {
       const int next = tile + 1 < tile_end ? tile + 1 : tile;   // the last round re-reads its own (from the cache)
       const bf16* wt = wbase + (size_t)next * k_steps * 512;
@@ -359,30 +372,37 @@ __global__ void __launch_bounds__(512)
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int r = 0; r < 4; ++r) red[(wave * MT + mt) * 256 + r * 64 + lane] = acc[mt][r];
+    if (EXPERTS && threadIdx.x < MT * 16) share_of[turn][threadIdx.x] = share_next;
     __syncthreads();
-    for (int idx = threadIdx.x; idx < MT * 256; idx += blockDim.x) {
-      const int mt = idx >> 8, i = idx & 255;
-      const int r = i >> 6, l2 = i & 63, col = l2 & 15;
-      const int m = mt * 16 + (l2 >> 4) * 4 + r;
-      if (c_mode == 0) {
+    if (c_mode == 0) {
+      for (int idx = threadIdx.x; idx < MT * 256; idx += blockDim.x) {
+        const int mt = idx >> 8, i = idx & 255;
+        const int r = i >> 6, l2 = i & 63, col = l2 & 15;
+        const int m = mt * 16 + (l2 >> 4) * 4 + r;
         float s = 0.f;
         for (int w2 = 0; w2 < n_waves; ++w2) s += red[(w2 * MT + mt) * 256 + i];
         const int nn = tile * 16 + col;
         if (m < M && nn < N) C[(size_t)m * ldc + nn] = from_float<TC>(s);
-      } else if (col < 8) {
-        float g = 0.f, u = 0.f, share = 1.0f;
-        const int nn = tile * 8 + col;
-        if (EXPERTS) share = ex.weights[(size_t)min(m, M - 1) * (ex.E + 1) + min(nn / ex.ffe, ex.E)];
-        for (int w2 = 0; w2 < n_waves; ++w2) {
-          g += red[(w2 * MT + mt) * 256 + i];
-          u += red[(w2 * MT + mt) * 256 + i + 8];
+      }
+    } else {
+      for (int idx = threadIdx.x; idx < MT * 128; idx += blockDim.x) {      // a thread for every pair
+        const int mt = idx >> 7, r = (idx >> 5) & 3, q = (idx >> 3) & 3, col = idx & 7, i = r * 64 + q * 16 + col;
+        const int m = mt * 16 + q * 4 + r, nn = tile * 8 + col;
+        if (m >= M || nn >= N / 2) continue;
+        float share = 1.0f, v = 0.f;
+        if (EXPERTS) share = ex.ffe % 8 == 0 ? share_of[turn][m] : ex.weights[(size_t)m * (ex.E + 1) + min(nn / ex.ffe, ex.E)];
+        if (!EXPERTS || share != 0.f) {
+          float g = 0.f, u = 0.f;
+          for (int w2 = 0; w2 < n_waves; ++w2) {
+            g += red[(w2 * MT + mt) * 256 + i];
+            u += red[(w2 * MT + mt) * 256 + i + 8];
+          }
+          v = EXPERTS ? gv_gate(g, c_mode) * u * share : gv_gate(g, c_mode) * u;
         }
-        if (EXPERTS) {
-          if (m < M && nn < N / 2) C[(size_t)m * ldc + nn] = from_float<TC>(share != 0.f ? gv_gate(g, c_mode) * u * share : 0.f);
-        } else if (m < M && nn < N / 2) C[(size_t)m * ldc + nn] = from_float<TC>(gv_gate(g, c_mode) * u);
+        C[(size_t)m * ldc + nn] = from_float<TC>(v);
       }
     }
-    __syncthreads();
+    if (!EXPERTS) __syncthreads();
     if (PREFETCH) {
 #pragma unroll
       for (int s = 0; s < KSTEPS; ++s) w[s] = wn[s];
@@ -419,7 +439,7 @@ extern "C" int blm_gemv_mfma_supported(int M, int N, int K) {
 struct GemvGeometry {
   int ksteps, waves, blocks;
 };
-static GemvGeometry gemv_geometry(int M, int N, int K, int k_groups) {
+static GemvGeometry gemv_geometry(int M, int N, int K, int k_groups, bool experts = false) {
   const int n_tiles = (N + 15) / 16;
   const int k_steps = (K + 31) / 32;
   const int steps_per_group = (k_steps + k_groups - 1) / k_groups;
@@ -428,7 +448,7 @@ static GemvGeometry gemv_geometry(int M, int N, int K, int k_groups) {
   if (M > 16) {
     g.ksteps = steps_per_group > 64 ? 16 : 8;   // more than 2048 of K per group: two row tiles at most
     g.waves = (steps_per_group + g.ksteps - 1) / g.ksteps;   // at most 8 by the group limit
-    cap = 256 / k_groups;
+    cap = (experts && (g.waves <= 2 || (g.waves <= 4 && n_tiles >= 2048)) ? 512 : 256) / k_groups;
   } else {
     g.waves = plan_k(steps_per_group * 32, &g.ksteps);
     cap = (g.waves > 4 ? 256 : 512) / k_groups;
@@ -456,12 +476,12 @@ static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int
   const int n_tiles = (N + 15) / 16;
   const int k_steps = (K + 31) / 32;
   const int steps_per_group = (k_steps + k_groups - 1) / k_groups;
-  const GemvGeometry geo = gemv_geometry(M, N, K, k_groups);
+  const GemvGeometry geo = gemv_geometry(M, N, K, k_groups, experts != nullptr);
   if (M > 16) {
     const int mt = (M + 15) / 16;
     const int ks = geo.ksteps, waves = geo.waves, blocks = geo.blocks;
     dim3 grid(blocks, k_groups), block(waves * BLM_WAVE);
-    const size_t smem = (size_t)waves * mt * 256 * sizeof(float);
+    const size_t smem = (size_t)waves * mt * 256 * sizeof(float) * (experts ? 2 : 1);
 #define BLM_GR(MT, KS, PF)                                                                                      \
   do {                                                                                                          \
     if (experts) BLM_GRE(MT, KS, PF, true, *experts);                                                           \

@@ -76,3 +76,13 @@ def test_what_is_refused():
         ops.gemv_experts(x, packed, out, 16, 16)
     with pytest.raises(ops.KernelError):
         ops.gemv_experts(x, packed, out, 17, 16, weights=torch.zeros(8, 18, device="cuda"))
+
+
+@pytest.mark.parametrize("M", [16, 17, 32, 33, 64])
+@pytest.mark.parametrize("E,f,s,K", [(4, 12, 0, 64), (6, 4, 24, 200), (600, 16, 8, 1024), (300, 32, 0, 512), (3, 104, 8, 1160)])
+def test_experts_inside_tiles_and_many_tiles_a_block(M, E, f, s, K):
+    """Experts that end inside a tile of eight pairs, and blocks of several tiles, whose weights take turns in shared memory."""
+    from burn_lm_amd.csrc import ops
+    x, w, packed, out, g = case(M, E, f, s, K, seed=2)
+    weights = torch.rand(M, E + 1, generator=g, device="cuda") * (torch.rand(M, E + 1, generator=g, device="cuda") < 0.3)
+    check(ops.gemv_experts(x, packed, out, E, f, weights=weights), x, w, weights, E, f)
