@@ -17,6 +17,8 @@
 // life, so a block that walks several column tiles reads them once.  The partial tiles of the
 // wavefronts are summed through shared memory in a fixed order.  The SwiGLU gating of a
 // feed-forward can be fused into the product that computes gate and up (c_mode 1).
+#include <type_traits>
+
 #include "common.h"
 #include "row_scale.h"
 
@@ -484,8 +486,12 @@ static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int
     const size_t smem = (size_t)waves * mt * 256 * sizeof(float) * (experts ? 2 : 1);
 #define BLM_GR(MT, KS, PF)                                                                                      \
   do {                                                                                                          \
-    if (experts) BLM_GRE(MT, KS, PF, true, *experts);                                                           \
-    else BLM_GRE(MT, KS, PF, false, GvExperts{});                                                               \
+    if constexpr (std::is_same<TC, bf16>::value)      /* (weighted results come in bfloat16 only) */            \
+      if (experts) {                                                                                            \
+        BLM_GRE(MT, KS, PF, true, *experts);                                                                    \
+        break;                                                                                                  \
+      }                                                                                                         \
+    BLM_GRE(MT, KS, PF, false, GvExperts{});                                                                    \
   } while (0)
 #define BLM_GRE(MT, KS, PF, EXPERTS, EX)                                                                        \
   hipLaunchKernelGGL((gemv_mfma_rows_kernel<MT, KS, PF, EXPERTS, TC>), grid, block, smem, stream, (const bf16*)A, \
@@ -512,20 +518,25 @@ static int launch_mfma(const void* A, const void* Wp, void* C, int M, int N, int
     if (KS == 16 && blocks >= n_tiles) BLM_GO(KS, MAXT, KEEP, KS == 16, SCALED, SCALE, EXPERTS, EX);            \
     else BLM_GO(KS, MAXT, KEEP, false, SCALED, SCALE, EXPERTS, EX);                                             \
   } while (0)
-#define BLM_GM(KS, MAXT, KEEP)                                                                                  \
+// (SLOTS: most rows of a wavefront, of eight, with as many wavefronts as such a block has)
+#define BLM_GM(KS, MAXT, KEEP, SLOTS)                                                                           \
   do {                                                                                                          \
-    if (experts && experts->weights) BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 1, *experts);                        \
-    else if (experts) BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 2, *experts);                                       \
-    else if (scale == nullptr) BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 0, GvExperts{});                       \
-    else if (M <= waves) BLM_GS(KS, MAXT, KEEP, 1, *scale, 0, GvExperts{});                                 \
-    else if (M <= 2 * waves) BLM_GS(KS, MAXT, KEEP, 2, *scale, 0, GvExperts{});                             \
-    else BLM_GS(KS, MAXT, KEEP, RS_SLOTS, *scale, 0, GvExperts{});                                          \
+    if constexpr (std::is_same<TC, bf16>::value)                                                                \
+      if (experts) {                                                                                            \
+        if (experts->weights) BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 1, *experts);                               \
+        else BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 2, *experts);                                                \
+        break;                                                                                                  \
+      }                                                                                                         \
+    if (scale == nullptr) BLM_GS(KS, MAXT, KEEP, 0, RowScale{}, 0, GvExperts{});                                \
+    else if (M <= waves) BLM_GS(KS, MAXT, KEEP, 1, *scale, 0, GvExperts{});                                     \
+    else if (M <= 2 * waves) BLM_GS(KS, MAXT, KEEP, (SLOTS < 2 ? SLOTS : 2), *scale, 0, GvExperts{});           \
+    else BLM_GS(KS, MAXT, KEEP, SLOTS, *scale, 0, GvExperts{});                                                 \
   } while (0)
-  if (ksteps == 4) BLM_GM(4, 256, true);
-  else if (ksteps == 16 && waves <= 4) BLM_GM(16, 256, true);
-  else if (ksteps == 16) BLM_GM(16, 512, true);
-  else if (waves <= 8) BLM_GM(32, 512, true);
-  else BLM_GM(32, 1024, false);
+  if (ksteps == 4) BLM_GM(4, 256, true, RS_SLOTS);
+  else if (ksteps == 16 && waves <= 4) BLM_GM(16, 256, true, RS_SLOTS);
+  else if (ksteps == 16) BLM_GM(16, 512, true, 2);
+  else if (waves <= 8) BLM_GM(32, 512, true, 2);
+  else BLM_GM(32, 1024, false, 1);
 #undef BLM_GM
 #undef BLM_GS
 #undef BLM_GO
