@@ -342,15 +342,44 @@ __device__ __forceinline__ uint32_t smp_choose(const unsigned long long (&m)[PER
   return (uint32_t)found;
 }
 
+// A weight of every lane, added to the bin of its digit if the digits above are `prefix`; the first such lane's once for all that hold the
+// same: where a row has many weights in one bin of level 0, few are different, as a rule, and equal ones would queue up at one address.
+__device__ __forceinline__ void smp_add(unsigned long long* bins, uint32_t key, uint32_t prefix, int above_bits, int shift, uint32_t mask) {
+  const bool in = (key >> above_bits) == prefix;
+  const unsigned long long who = __ballot(in);
+  if (who == 0) return;
+  const int leader = __builtin_ctzll(who);
+  const bool same = in && key == (uint32_t)__builtin_amdgcn_readlane(key, leader);
+  const int times = __popcll(__ballot(same));
+  if (!in || (same && (int)(threadIdx.x & (BLM_WAVE - 1)) != leader)) return;
+  const unsigned long long q = smp_mass(__uint_as_float(key)) * (same ? times : 1);
+  if (q) atomicAdd(&bins[(key >> shift) & mask], q);
+}
+
+// f of all elements, in a loop of four at a time: what few rows run is kept short
+template <typename F>
+__device__ __forceinline__ void smp_turn(float (&xs)[4][4], F f) {
+#pragma unroll 1
+  for (int u = 0; u < 4; ++u) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      f(xs[0][k]);
+      xs[0][k] = xs[1][k];
+      xs[1][k] = xs[2][k];
+      xs[2][k] = xs[3][k];
+    }
+  }
+}
+
 // passes 2 to 4: level 0 takes bits 29..19 of the weights' bit patterns, level 1 bits 18..8, level 2 bits 7..0 (e <= 1, so bits 31 and
-// 30 are clear).  LIST (level 1): no histogram; the weights with the digits chosen, in any order, and how many; those beyond `capacity`
-// are only counted.
+// 30 are clear).  LIST (level 1): no histogram; the weights with the digits chosen, in any order, and how many.  Where they are more than
+// `capacity` (flat logits, few different ones: a bin is a sixteenth of a power of two wide) the slice's histogram stands in the list's place.
 template <bool VEC, int LEVEL, bool LIST, int THREADS>
 __global__ void __launch_bounds__(THREADS)
     sample_level_kernel(const float* __restrict__ logits, int V, int ld, int slice_len, float k2, float top_p,
                         const float* __restrict__ part_max, SampleState* states, unsigned long long* hist, int n_rows,
                         uint32_t* __restrict__ list, int* __restrict__ counts, int capacity) {
-  __shared__ unsigned long long bins[LIST ? 1 : SMP_BINS];
+  __shared__ unsigned long long bins[SMP_BINS];
   __shared__ SmpChoose<THREADS> choose;
   __shared__ int listed;
   const int row = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x;
@@ -376,13 +405,10 @@ __global__ void __launch_bounds__(THREADS)
     prefix |= smp_choose<THREADS, PER>(m, LEVEL == 1, top_p, carry, target, choose);
     if (slice == 0 && tid == 0) states[(size_t)(LEVEL - 1) * n_rows + row] = SampleState{prefix, carry, target};
   }
-  if (LIST) {
-    if (tid == 0) listed = 0;
-  } else {
-    for (int b = tid; b < SMP_BINS; b += THREADS) bins[b] = 0ull;
-  }
+  if (LIST && tid == 0) listed = 0;
+  for (int b = tid; b < SMP_BINS; b += THREADS) bins[b] = 0ull;
   __syncthreads();
-  // Level 0: V tokens of weights up to an eighth above `light` have less mass than the 1 - top_p of it that lies below the cut (the heaviest
+  // Level 0: V tokens of weights up to a sixteenth above `light` have less mass than the 1 - top_p of it that lies below the cut (the heaviest
   // alone has 2^32), so no bin that holds one of them can be the cut's: those below `light` count for the whole mass only, in the lowest
   // bin.  Most of a row, as a rule, and a register's add in place of an atomic one each.
   const float light = LEVEL == 0 ? 0.5f * (1.0f - top_p) / (float)V : 0.f;
@@ -443,6 +469,13 @@ __global__ void __launch_bounds__(THREADS)
   __syncthreads();
   if (LIST) {
     if (tid == 0) counts[row * SMP_SLICES + slice] = listed;
+    if (listed <= capacity) return;
+    for (int c0 = begin; c0 < end; c0 += 16 * THREADS) {
+      smp_load16<VEC, THREADS>(x, c0, tid, xs);
+      smp_turn(xs, [&](float v) { smp_add(bins, __float_as_uint(__builtin_amdgcn_exp2f((v - mx) * k2)), prefix, above_bits, shift, mask); });
+    }
+    __syncthreads();
+    for (int b = tid; b < SMP_BINS; b += THREADS) reinterpret_cast<unsigned long long*>(to)[b] = bins[b];
   } else {
     unsigned long long* row_hist = hist + ((size_t)LEVEL * n_rows + row) * SMP_BINS;
     for (int b = tid; b < SMP_BINS; b += THREADS)
@@ -450,21 +483,27 @@ __global__ void __launch_bounds__(THREADS)
   }
 }
 
-// Levels 1 and 2 from the row's list of weights in level 0's bin; from the row itself where a slice had more than its list holds (flat
-// logits: a bin is an eighth of a power of two wide).  Returns the smallest kept weight.
+// Levels 1 and 2 from the slices' lists of weights in level 0's bin; where a slice had more than its list holds, level 1 from the
+// histogram in its place and level 2 from the slice itself.  Returns the smallest kept weight.
+// Bound by the instructions of one compute unit on the row's part of a bin, and by what queues up at one bin.  Draws of 128,256 logits, us, 16 and
+// 64 rows, blocks of 256 threads with histograms / here, every listed weight by an atomic of its own and flat rows read twice / here: normal
+// logits 46.8, 61.4 / 28.0, 41.5 / 28.2, 41.6; rounded to whole numbers (few different weights) 48.3, 67.5 / 55.2, 70.2 / 35.1, 50.5;
+// normal by 0.05 49.3, 67.5 / 39.8, 54.3 / 37.1, 51.3, by 0.01 (a bin holds most of the row) 55.0, 78.8 / 69.4, 92.0 / 57.4, 81.1; all the
+// same 83.8, 132.6 / 81.9, 108.1 / 80.3, 107.7.  Of 50,021 (addresses of four bytes) 64 rows: 57.1 / 37.1 / 38.3, 58.2 / 48.5 / 49.3, 59.2 /
+// 40.3 / 41.6, 64.3 / 72.9 / 64.9, 82.2 / 76.1 / 70.6.
 template <bool VEC, int THREADS>
-__device__ __forceinline__ uint32_t smp_choose_listed(const float* x, int V, float mx, float k2, SampleState state, const uint32_t* list,
-                                                      const int* counts, int n_slices, int capacity, unsigned long long* bins,
-                                                      SmpChoose<THREADS>& choose) {
-  constexpr int KEPT = 8;
+__device__ __forceinline__ uint32_t smp_choose_listed(const float* x, int V, int slice_len, float mx, float k2, SampleState state,
+                                                      const uint32_t* list, const int* counts, int n_slices, int capacity,
+                                                      unsigned long long* bins, SmpChoose<THREADS>& choose) {
+  constexpr int KEPT = 8, PER = SMP_BINS / THREADS;
   const int tid = threadIdx.x, group = THREADS / n_slices, slice = tid / group, first = tid % group;
   const uint32_t* mine = list + (size_t)slice * capacity;
   uint32_t keys[KEPT];   // asked for with their number
 #pragma unroll
   for (int i = 0; i < KEPT; ++i) keys[i] = mine[min(first + i * group, capacity - 1)];
   const int lane = tid & (BLM_WAVE - 1), any = counts[min(lane, n_slices - 1)], own = counts[slice];
-  const bool over = __ballot(any > capacity) != 0;
-  const int n = over ? 0 : own;
+  const unsigned long long over = __ballot(lane < n_slices && any > capacity);      // the slices without a list
+  const int n = own > capacity ? 0 : own;
 #pragma unroll
   for (int i = 0; i < KEPT; ++i) keys[i] = first + i * group < n ? keys[i] : 0u;
   uint32_t prefix = state.prefix;
@@ -472,38 +511,62 @@ __device__ __forceinline__ uint32_t smp_choose_listed(const float* x, int V, flo
   for (int level = 1; level < 3; ++level) {
     const int shift = level == 1 ? 8 : 0, above_bits = level == 1 ? 19 : 8;
     const uint32_t mask = level == 1 ? 0x7ffu : 0xffu;
-    auto add = [&](uint32_t key, int times = 1) {
+    for (int b = tid; b <= (int)mask; b += THREADS) bins[b] = 0ull;
+    __syncthreads();
+    auto add = [&](uint32_t key, int times) {
       if ((key >> above_bits) != prefix) return;
       const unsigned long long q = smp_mass(__uint_as_float(key)) * times;
       if (q) atomicAdd(&bins[(key >> shift) & mask], q);
     };
-    for (int b = tid; b <= (int)mask; b += THREADS) bins[b] = 0ull;
-    __syncthreads();
+    // a wavefront's at once where they are one weight, as in rows of few different ones
+    auto add_all = [&](const auto& of, int i0) {
+      constexpr int N = sizeof(of) / sizeof(of[0]);
+      const uint32_t lead = __builtin_amdgcn_readfirstlane(of[0]);
+      bool alike = i0 + (N - 1) * group < n;
 #pragma unroll
-    for (int i = 0; i < KEPT; ++i) add(keys[i]);
-    for (int i = first + KEPT * group; i < n; i += group) add(mine[i]);
-    if (over) {
-      const SmpRow<VEC> whole(x, V);
-      for (int c0 = 0; c0 < V; c0 += 16 * THREADS) {
-        float xs[4][4];
-        smp_load16<VEC, THREADS>(whole, c0, tid, xs);
+      for (int i = 0; i < N; ++i) alike &= of[i] == lead;
+      if (__ballot(!alike) == 0) {
+        if (lane == 0) add(lead, N * BLM_WAVE);
+      } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int i = 0; i < N; ++i)
+          if (i0 + i * group < n) add(of[i], 1);
+      }
+    };
+    add_all(keys, first);
+    for (int i0 = first + KEPT * group; i0 < n; i0 += 4 * group) {
+      uint32_t more[4];
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            // the first lane's weight once for all lanes that hold the same: equal weights would queue up at one bin
-            const uint32_t key = __float_as_uint(__builtin_amdgcn_exp2f((xs[u][k] - mx) * k2)), lead = __builtin_amdgcn_readfirstlane(key);
-            const int same = __popcll(__ballot(key == lead));
-            if (key != lead || (tid & (BLM_WAVE - 1)) == 0) add(key, key == lead ? same : 1);
-          }
+      for (int i = 0; i < 4; ++i) more[i] = mine[min(i0 + i * group, capacity - 1)];
+      add_all(more, i0);
+    }
+    if (level == 2 && over) {
+      // the logits whose weights may have these digits, to 1e-5 of the exponent (the instruction's error is a hundredth of it)
+      const float low = __log2f(__uint_as_float(prefix << 8)), high = __log2f(__uint_as_float((prefix << 8) | 0xffu));
+      const float centre = 0.5f * (low + high), reach = prefix ? 0.5f * (high - low) + 1e-5f : INFINITY;
+      for (unsigned long long left = over; left; left &= left - 1) {
+        const int begin = __builtin_ctzll(left) * slice_len, end = min(V, begin + slice_len);
+        const SmpRow<VEC> part(x, end);
+        for (int c0 = begin; c0 < end; c0 += 16 * THREADS) {
+          float xs[4][4];
+          smp_load16<VEC, THREADS>(part, c0, tid, xs);
+          smp_turn(xs, [&](float v) {
+            const float t = (v - mx) * k2;
+            if (__ballot(!(fabsf(t - centre) > reach))) smp_add(bins, __float_as_uint(__builtin_amdgcn_exp2f(t)), prefix, above_bits, shift, mask);
+          });
+        }
       }
     }
     __syncthreads();
     if (level == 1) {
-      constexpr int PER = SMP_BINS / THREADS;
       unsigned long long m[PER];
 #pragma unroll
       for (int j = 0; j < PER; ++j) m[j] = bins[tid * PER + j];
+      for (unsigned long long left = over; left; left &= left - 1) {
+        const unsigned long long* of = reinterpret_cast<const unsigned long long*>(list + (size_t)__builtin_ctzll(left) * capacity);
+#pragma unroll
+        for (int j = 0; j < PER; ++j) m[j] += of[tid * PER + j];
+      }
       prefix = (prefix << 11) | smp_choose<THREADS, PER>(m, false, 0.f, state.carry, state.target, choose);
     } else {
       unsigned long long m[1] = {tid < 256 ? bins[tid] : 0ull};
@@ -580,7 +643,7 @@ __global__ void __launch_bounds__(THREADS)
     tau = (state.prefix << 8) | smp_choose<THREADS, 1>(m, false, 0.f, state.carry, state.target, choose);
   }
   if (CUT == 2)
-    tau = smp_choose_listed<VEC, THREADS>(x, V, mx, k2, states[row], list + (size_t)row * gridDim.x * capacity, counts + row * SMP_SLICES,
+    tau = smp_choose_listed<VEC, THREADS>(x, V, slice_len, mx, k2, states[row], list + (size_t)row * gridDim.x * capacity, counts + row * SMP_SLICES,
                                           gridDim.x, capacity, bins, choose);
   auto kept = [&](float v) {
     const float e = __builtin_amdgcn_exp2f((v - mx) * k2);
@@ -719,8 +782,9 @@ static int sample_slice_len(int R, int V, int cut) {
   return ((V + n - 1) / n + SMP_CHUNK - 1) / SMP_CHUNK * SMP_CHUNK;
 }
 
-// How many of a slice's weights a list holds.
-static int sample_list_capacity(int slice_len) { return slice_len / 4; }
+// How many of a slice's weights a list holds: no fewer than its place takes a histogram (SMP_BINS of 64 bits).
+static int sample_list_capacity(int slice_len) { return slice_len / 4 > 2 * SMP_BINS ? slice_len / 4 : 2 * SMP_BINS; }
+static size_t sample_even(size_t n) { return n + (n & 1); }
 
 // Bytes of scratch that blm_sample needs for R rows of V logits (see there for the layout).
 extern "C" long long blm_sample_scratch_bytes(int R, int V) {
@@ -730,7 +794,7 @@ extern "C" long long blm_sample_scratch_bytes(int R, int V) {
     chunks = n > chunks ? n : chunks;
   }
   const long long wide = sample_wide_slices(R, V, 1), lists = wide * sample_list_capacity(sample_slice_len(R, V, 1));
-  return (long long)R * ((wide ? 1 : 3) * SMP_BINS * 8 + 2 * sizeof(SampleState) + SMP_SLICES * 8 + (1 + chunks + lists) * 4);
+  return (long long)R * ((wide ? 1 : 3) * SMP_BINS * 8 + 2 * sizeof(SampleState) + SMP_SLICES * 8 + (1 + chunks + lists) * 4) + 4;
 }
 
 // scratch: blm_sample_scratch_bytes(R, V) bytes, 8-byte aligned: the rows' histograms, their states behind two levels, the slices'
@@ -752,7 +816,7 @@ extern "C" int blm_sample(const float* logits, const float* uniforms, int* out, 
   int* counts = reinterpret_cast<int*>(part_max + (size_t)R * SMP_SLICES);
   float* row_uniforms = reinterpret_cast<float*>(counts + (size_t)R * SMP_SLICES);
   float* chunk_mass = row_uniforms + R;
-  uint32_t* list = reinterpret_cast<uint32_t*>(chunk_mass + (size_t)R * slices * (slice_len / SMP_CHUNK));
+  uint32_t* list = reinterpret_cast<uint32_t*>(row_uniforms + sample_even(R + (size_t)R * slices * (slice_len / SMP_CHUNK)));      // 8 bytes aligned
   const float k2 = 1.4426950408889634f / temperature;
   const bool vec = V >= 4 && ld % 4 == 0 && ((uintptr_t)logits % 16) == 0;
   dim3 grid(slices, R), block(wide ? 1024 : SMP_THREADS);

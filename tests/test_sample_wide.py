@@ -13,6 +13,9 @@ def rows_of(kind, R, V, g):
         return torch.zeros_like(z)
     if kind == "narrow":                     # lists of some rows, some slices, are full
         return z * torch.linspace(0.0, 0.4, R, device="cuda")[:, None]
+    if kind == "part":                       # some of a row's slices have more in the bin than a list holds, the others an entry or none
+        z = torch.where(torch.arange(V, device="cuda") < torch.arange(R, device="cuda")[:, None] * V // R, z * 0.002, z - 9.0)
+        return z.roll(V // 3, 1)
     if kind == "ties":                       # few different weights
         return (z * 2.0).round()
     z[:, V // 3:] = -float("inf")            # masked: slices without any mass, one with a single token
@@ -22,7 +25,7 @@ def rows_of(kind, R, V, g):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind", ["normal", "flat", "narrow", "ties", "masked"])
+@pytest.mark.parametrize("kind", ["normal", "flat", "narrow", "part", "ties", "masked"])
 @pytest.mark.parametrize("R,V,ld", [(16, 98304, 98304), (33, 50021, 50021), (64, 49153, 49156), (64, 128256, 128256), (100, 32000, 32000),
                                     (128, 24578, 24578)])
 def test_draws_are_those_of_a_row_alone(kind, R, V, ld):
