@@ -644,7 +644,31 @@ class Runtime:
         rounded in front of the norm's factor instead of behind it, as far from 64 bits but elsewhere, and a narrow model, whose
         steps are the host's time anyway, keeps the roundings that it is compared with value by value."""
         return (M <= ops.SCALED_ROWS and isinstance(w, LinearWeight) and not w.gated and w.dtype == self.dtype and w.packable
-                and (w.dtype == torch.float32 or w.shape[0] >= JOIN_BF16_WIDTH) and ops.gemv_join_columns(w.dtype, M, *w.shape) > 0 and w.packed is not None)
+                and (w.dtype == torch.float32 or w.shape[0] >= JOIN_BF16_WIDTH) and self.join_gains(w.dtype, M, *w.shape) and w.packed is not None)
+
+    def join_gains(self, dtype, M, N, K):
+        """Whether gemv_join is the shorter way.  It is not for a long K where a block's columns are no whole 64 bytes of the packed weights (its
+        neighbours read the rest of their lines once more), nor in float32 where few columns leave units idle while each block reads all rows'
+        K.  A product and the norm's kernel / this, us, rows 1, 4 and 8:
+        * bfloat16, blocks of 8, 12 and 16 columns: [2048, 16384] 18.2 / 14.0, 17.7 / 14.6, 18.5 / 16.6; [3072, 8192] 14.8 / 14.1, 15.3 / 14.0, 15.2 /
+          15.1; [4096, 16384] 28.9 / 24.9, 29.7 / 25.2, 29.9 / 25.7; [1152, 9216] 9.3 / 8.1, 9.3 / 8.6, 9.8 / 9.9;
+        * of 9, 11, 13 and 15: [2304, 6336] 11.3 / 8.9, 11.4 / 9.3, 11.8 / 10.3; [2304, 9216] 12.7 / 13.2, 12.7 / 12.8, 13.0 / 14.0; [2816, 7744] 13.8 /
+          12.5, 13.7 / 12.5, 14.3 / 13.6; [2816, 11264] 17.3 / 17.8, 17.9 / 18.3, 17.5 / 19.8; [3840, 10560] 19.4 / 18.5, 19.4 / 19.4, 19.8 / 21.0;
+        * of 10 and 14: [2560, 10240] 14.6 / 13.8, 15.1 / 13.3, 14.9 / 14.5; [3584, 9856] 18.5 / 18.6, 19.0 / 18.4, 18.9 / 19.1; [2560, 14080] 17.9 /
+          17.0, 18.4 / 18.1, 18.7 / 20.9; [3584, 14336] 23.7 / 23.7, 24.4 / 24.5, 24.5 / 25.8;
+        * float32, blocks of 8: [1024, 4096] 8.0 / 7.2, 8.2 / 7.7, 8.3 / 8.6; [768, 4224] 9.2 / 9.2, 9.5 / 10.0, 9.8 / 11.2; [1152, 6336] 16.0 / 11.2, 16.9
+          / 11.6, 17.5 / 13.4; [1024, 8192] 11.7 / 12.0, 11.9 / 13.0, 12.0 / 14.6; [1536, 8448] 18.6 / 17.5, 18.9 / 19.7, 19.5 / 20.8; [1792, 14336] 25.9 /
+          22.0, 26.3 / 23.9, 26.6 / 28.1; [2048, 11264] 23.6 / 20.8, 23.6 / 22.1, 24.2 / 25.6; [2048, 16384] 32.6 / 26.2, 33.1 / 27.6, 33.4 / 31.8;
+        * float32, of 9 to 14: [2560, 2560] 12.1 / 9.2, 12.8 / 9.7, 13.1 / 10.5; [3584, 3584] 15.7 / 12.1, 16.1 / 12.5, 16.3 / 13.5; [2304, 6336] 18.7 /
+          20.4, 18.9 / 21.0, 19.3 / 21.0; [3072, 8448] 27.5 / 30.4, 27.2 / 30.4, 27.7 / 32.7; of 16: [4096, 16384] 57.4 / 47.9, 59.1 / 48.9, 59.3 / 51.4."""
+        columns = ops.gemv_join_columns(dtype, M, N, K)
+        if columns == 0:
+            return False
+        if dtype == torch.bfloat16:
+            return columns % 4 == 0 or K <= (8192 if columns % 2 else 10240)
+        if columns > 8:
+            return columns == 16 or K <= 4096
+        return N >= 2048 or K <= 4 * N or (M <= 4 and (N >= 1536 or K <= 6 * N))
 
     def join_reads(self, x, w):
         """Whether join takes these rows: of the weights' type, in whole pieces of 16 bytes (an attention's or a gating's own always are)."""

@@ -186,6 +186,19 @@ def test_rows_behind_the_last(M):
             ops.gemv_mfma(y, packed, out[:M], K, gated=gated, scale=(sums[:, :6].contiguous(), 1e-5))
 
 
+@pytest.mark.parametrize("dtype,N,K,rows", [
+    (torch.bfloat16, 2048, 16384, 8), (torch.bfloat16, 3072, 12288, 8), (torch.bfloat16, 4096, 14336, 8), (torch.bfloat16, 2304, 6336, 8),
+    (torch.bfloat16, 2560, 10240, 8), (torch.bfloat16, 2304, 9216, 0), (torch.bfloat16, 2816, 11264, 0), (torch.bfloat16, 3584, 14336, 0),
+    (torch.float32, 64, 176, 8), (torch.float32, 2048, 8192, 8), (torch.float32, 1024, 4096, 8), (torch.float32, 1152, 6336, 4),
+    (torch.float32, 768, 6144, 0), (torch.float32, 1792, 14336, 4), (torch.float32, 3072, 3072, 8), (torch.float32, 3072, 8448, 0),
+    (torch.float32, 2304, 12672, 0), (torch.float32, 4096, 16384, 8)])
+def test_joined_where_it_is_the_shorter_way(dtype, N, K, rows):
+    """The rows up to which a product is joined with the norm behind it (0: none): not where it was measured slower."""
+    from burn_lm_amd.engine.runtime import Runtime
+    rt = Runtime.__new__(Runtime)
+    assert [rt.join_gains(dtype, M, N, K) for M in range(1, 10)] == [M <= rows for M in range(1, 10)]
+
+
 class Log(list):
     def word(self, what, answer):
         return lambda *a, **k: (self.append(what), answer)[1]
