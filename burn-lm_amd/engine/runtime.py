@@ -640,9 +640,11 @@ class Runtime:
         """Whether the product of M rows with w can add its result to the residual and leave the next norm's rows (join).  Up to eight
         rows: beyond, every block's activations, all of K for few columns, cost more than the norm's kernel (a layer of the 1B shape
         without its attention, us, norms as kernels / joined: 1 row 34.9 / 29.9, 4 rows 36.2 / 31.5, 8 rows 37.6 / 34.1, 16 rows 40.9 /
-        40.2; of the 3B shape 50.3 / 44.3, 52.6 / 45.9, 54.3 / 48.3, 59.2 / 68.7).  bfloat16 from JOIN_BF16_WIDTH columns on: the rows are
-        rounded in front of the norm's factor instead of behind it, as far from 64 bits but elsewhere, and a narrow model, whose
-        steps are the host's time anyway, keeps the roundings that it is compared with value by value."""
+        40.2; of the 3B shape 50.3 / 44.3, 52.6 / 45.9, 54.3 / 48.3, 59.2 / 68.7).  bfloat16 from JOIN_BF16_WIDTH columns on.  Neither time
+        nor error draws that line (a product and its norm apart / joined, us, rows 1 and 8: [64, 176] 4.6 / 2.9, 4.9 / 3.0, [256, 704] 5.2 / 2.9, 5.5 /
+        3.1, [512, 1408] 5.6 / 3.1, 6.1 / 3.4, [768, 3072] 5.9 / 3.9, 6.5 / 4.7; three small models joined and apart are equally far from
+        64 bits, to 3 in a hundred): the rows are rounded in front of the norm's factor instead of behind it, and the widths below
+        are those whose steps are compared, value by value, with an implementation that rounds behind it."""
         return (M <= ops.SCALED_ROWS and isinstance(w, LinearWeight) and not w.gated and w.dtype == self.dtype and w.packable
                 and (w.dtype == torch.float32 or w.shape[0] >= JOIN_BF16_WIDTH) and self.join_gains(w.dtype, M, *w.shape) and w.packed is not None)
 

@@ -13,6 +13,7 @@ layout have the rows of their q/k projections permuted into that order first
 """
 from __future__ import annotations
 
+import copy
 import json
 import math
 import os
@@ -45,13 +46,18 @@ class Rounding:
     and are summed, relative to the row's maximum; or, when keys are visited in pages of
     ``probability_pages``, relative to the maximum of the pages up to the key's own
     (``running_maximum``, one page after the other) or of the key's own page alone (every page on
-    its own), the weights then being scaled, exactly, to the row's maximum."""
+    its own), the weights then being scaled, exactly, to the row's maximum;
+    ``mixer_norm_in_front`` and ``ffn_norm_in_front``: the norm in front of the mixers (but the first
+    layer's) and of the feed-forwards is done by the products on its two sides: the product in front is
+    added unrounded, and the rows are rounded in front of the norm's factor and not behind it."""
 
     def __init__(self, projections=True, gate_up=True, attention_delta=True, feed_forward_delta=True,
-                 probabilities=True, probability_pages=None, running_maximum=True):
+                 probabilities=True, probability_pages=None, running_maximum=True,
+                 mixer_norm_in_front=False, ffn_norm_in_front=False):
         self.projections, self.gate_up = projections, gate_up
         self.attention_delta, self.feed_forward_delta = attention_delta, feed_forward_delta
         self.probabilities, self.probability_pages, self.running_maximum = probabilities, probability_pages, running_maximum
+        self.mixer_norm_in_front, self.ffn_norm_in_front = mixer_norm_in_front, ffn_norm_in_front
 
     r = staticmethod(round_bf16)
 
@@ -220,13 +226,34 @@ def swiglu_feed_forward(x, w_gate, w_up, w_down, rounding=None):
     return _r(rounding, rounding.r(silu(g) * u) @ w_down.T, rounding.feed_forward_delta, 1)
 
 
-def block(x, lw, cfg, freqs, start_pos=0, rounding=None):
+def normed(x, gamma, eps, rounding, in_front):
+    """The norm's rows, rounded behind its factor per row, or in front of it where ``in_front`` holds (one flag, or one per token)."""
+    y = _r(rounding, rms_norm(x, gamma, eps))
+    if in_front is False:
+        return y
+    flags = np.broadcast_to(np.asarray(in_front, dtype=bool), (x.shape[1],))[None, :, None]
+    factor = 1.0 / np.sqrt(np.mean(x * x, axis=-1, keepdims=True) + eps)
+    return np.where(flags, rounding.r(x * np.asarray(gamma, dtype=np.float64)) * factor, y)
+
+
+def block(x, lw, cfg, freqs, start_pos=0, rounding=None, first=False, last=False):
     """h = x + attn(norm1(x)); out = h + ffn(norm2(h)) (LL/nn/transformer.rs:241-256)."""
-    h = x + attention_layer(_r(rounding, rms_norm(x, lw["attention_norm"], cfg["eps"])),
+    mixer_front = ffn_front = False
+    if rounding is not None:
+        mixer_front = False if first else rounding.mixer_norm_in_front
+        ffn_front = rounding.ffn_norm_in_front
+        rounding = copy.copy(rounding)
+        rounding.attention_delta = _unless(rounding.attention_delta, ffn_front, x.shape[1])
+        rounding.feed_forward_delta = _unless(rounding.feed_forward_delta, False if last else rounding.mixer_norm_in_front, x.shape[1])
+    h = x + attention_layer(normed(x, lw["attention_norm"], cfg["eps"], rounding, mixer_front),
                             lw["wq"], lw["wk"], lw["wv"], lw["wo"],
                             cfg["n_heads"], cfg["n_kv_heads"], cfg["head_dim"], freqs, start_pos, rounding)
-    return h + swiglu_feed_forward(_r(rounding, rms_norm(h, lw["ffn_norm"], cfg["eps"])),
+    return h + swiglu_feed_forward(normed(h, lw["ffn_norm"], cfg["eps"], rounding, ffn_front),
                                    lw["w1"], lw["w3"], lw["w2"], rounding)
+
+
+def _unless(flag, front, tokens):
+    return flag if front is False else np.broadcast_to(flag, (tokens,)) & ~np.broadcast_to(front, (tokens,))
 
 
 def transformer_forward(ids, model, start_pos=0, rounding=None):
@@ -236,8 +263,8 @@ def transformer_forward(ids, model, start_pos=0, rounding=None):
     cfg = model["cfg"]
     ids = np.asarray(ids)
     h = model["tok_embeddings"][ids]
-    for lw in model["layers"]:
-        h = block(h, lw, cfg, model["freqs"], start_pos, rounding)
+    for i, lw in enumerate(model["layers"]):
+        h = block(h, lw, cfg, model["freqs"], start_pos, rounding, first=i == 0, last=i + 1 == len(model["layers"]))
     h = _r(rounding, rms_norm(h, model["norm"], cfg["eps"]))
     return h @ model["output"].T
 

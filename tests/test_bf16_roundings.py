@@ -114,3 +114,43 @@ def test_tokens_one_by_one_against_the_plain_implementation_with_the_engines_rou
         want = P.transformer_forward([t], plain, rounding=rounding_for(name, np.where(decoded, 1, head), decoded))[0]
         errors += [rel_err(got[p], want[p]) for p in range(n)]
     check(name, errors)
+
+
+# Which norms the products do in steps of up to eight tokens where the models' width allows it (engine.runtime.JOIN_BF16_WIDTH): in
+# front of the mixers and of the feed-forwards.  B's head size of 24 has no q/k/v product of unscaled rows.
+JOINED = {"A": (True, True), "B": (False, True), "C": (True, True)}
+JOINED_LENGTHS = LENGTHS[2:]
+
+
+@pytest.mark.parametrize("graphs", [True, False])
+def test_narrow_models_with_joined_norms(case, graphs, tmp_path, monkeypatch):
+    """Tokens one by one, recorded and eager, with the norms done by the products beside them, which these widths do without: against the
+    plain implementation with the roundings of that form, in the limits above, and no farther from the exact one than without it.
+    Slack: the errors of a sequence's rows go together, so the root mean square of n sequences' errors varies by 1 / sqrt(2 n), 0.25."""
+    from burn_lm_amd.engine import runtime
+    from burn_lm_amd.engine.loading import load_engine
+    name, plain_engine, plain, reqs = case
+    folder = make_folder(tmp_path, TINIES[name][0], TINIES[name][1])
+    monkeypatch.setattr(runtime, "JOIN_BF16_WIDTH", 0)
+    eng = load_engine(folder, dtype="bfloat16", max_tokens=4096, graphs=graphs)
+    errors, off = [], {"joined": 0.0, "apart": 0.0}
+    for t in (r for r, n in zip(reqs, LENGTHS) if n in JOINED_LENGTHS):
+        n, head = len(t), max(0, len(t) - 32)
+        exact = P.transformer_forward([t], plain)[0]
+        for which, e in (("joined", eng), ("apart", plain_engine)):
+            monkeypatch.setattr(runtime, "JOIN_BF16_WIDTH", 0 if which == "joined" else 1 << 30)
+            s = e.open()
+            rows = [e.step([(s, t[:head], list(range(head)))])] if head else []
+            rows += [e.step([(s, [t[p]], [0])]) for p in range(head, n)]
+            e.close(s)
+            got = np.concatenate([r.double().cpu().numpy() for r in rows])
+            off[which] += float((((got - exact) / np.abs(exact).max(-1, keepdims=True)) ** 2).sum())
+            if which == "joined":
+                step_rows, decoded = np.where(np.arange(n) >= head, 1, head), np.arange(n) >= head
+                rounding = rounding_for(name, step_rows, decoded)
+                rounding.mixer_norm_in_front, rounding.ffn_norm_in_front = (f & (step_rows <= 8) for f in JOINED[name])
+                want = P.transformer_forward([t], plain, rounding=rounding)[0]
+                errors += [rel_err(got[p], want[p]) for p in range(n)]
+    print(f"config {name}: off the exact implementation joined {off['joined'] ** 0.5:.3e}, apart {off['apart'] ** 0.5:.3e}")
+    check(name, errors)
+    assert 0 < off["joined"] <= off["apart"] * 1.25 ** 2 and off["joined"] != off["apart"]
