@@ -73,11 +73,14 @@ def test_products_of_unscaled_rows(dtype, M, N, K, n):
 
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("K,nh,nkv,hd", [(64, 2, 1, 16), (2048, 32, 8, 64), (2048, 24, 8, 128)])
+@pytest.mark.parametrize("K,nh,nkv,hd", [(64, 2, 1, 16), (2048, 32, 8, 64), (2048, 24, 8, 128), (3072, 24, 8, 128), (2080, 34, 4, 128),
+                                         (4096, 32, 8, 128), (4096, 8, 2, 64)])
 @pytest.mark.parametrize("M", [1, 8])
 def test_qkv_of_unscaled_rows(dtype, M, K, nh, nkv, hd):
     """The same kernel on rows that were scaled first (and rounded once more where they are bfloat16) leaves the same queries and pages."""
     from burn_lm_amd.csrc import ops
+    if dtype == torch.float32 and K > 2048:
+        pytest.skip("the float32 kernel takes no more of K in one group")
     y, sums, inv = unscaled(M, K, dtype, 64, seed=K)
     y32 = (y.double() * inv).to(dtype)
     w = (torch.randn((nh + 2 * nkv) * hd, K, device="cuda") / K ** 0.5).to(dtype)
