@@ -66,20 +66,35 @@ def test_a_table_of_the_tokens(T, E, top, f, D):
         assert torch.equal(ops.moe_grouped(x, gu, down, None, E, top, table=table, ids=ids, token_source=source), want)
 
 
-@pytest.mark.parametrize("rows", [[500, 530, 640, 641], [160, 161, 0, 1], [1000, 20, 300, 700]])
+def part_tiles(rows, n_tiles, units):
+    """What moe_duo_kernel runs behind its whole tiles for these rows of the experts (K >= 1,024): 1: an expert's last rows as a half, 2:
+    halves only, 3: tiles of 160 rows only."""
+    up = lambda a, b: -(-a // b)
+    wholes, lone = sum(r // 256 + (r % 256 > 128) for r in rows) * n_tiles, sum(0 < r % 256 <= 128 for r in rows) * n_tiles
+    rest = wholes % units
+    mixed = wholes // units * 100 + (100 if rest else 0) + up(max(0, lone - (units - rest if rest else 0)), units) * 57
+    halves, fives = (up(sum(up(r, size) for r in rows) * n_tiles, units) * cost for size, cost in ((128, 57), (160, 71)))
+    return 3 if fives < min(halves, mixed) else 2 if halves < mixed else 1
+
+
+@pytest.mark.parametrize("rows", [[500, 530, 640, 641], [160, 161, 0, 1], [1000, 20, 300, 700], [320, 321, 160, 159]])
 def test_tiles_of_five_eighths(rows):
     """Experts whose rows end at, behind and in front of tiles of 160 rows, alone on a few units: halves, wholes and five eighths (which
     the number of units decides) give the same bits, and those of the small tiles."""
     from burn_lm_amd.csrc import ops
     E, f, D = 4, 1024, 1024
     T = sum(rows)
+    all_units = (8, 11, 16, 17, 36, 40, 64, 70, 80, 96, 112, 128, 150, 256, 2000)
+    about = (T + 64 * E) // 128
+    for n_tiles, most in ((f // 128, about * (f // 128) * 5 // 2), (D // 256, about * (D // 256))):      # both products reach them
+        assert any(part_tiles(rows, n_tiles, u) == 3 for u in all_units if u <= most)
     g = torch.Generator().manual_seed(T)
     x, gu, down = (torch.randn(*s, generator=g).mul_(s[1] ** -0.5).bfloat16().cuda() for s in ((T, D), (2 * E * f, D), (D, E * f)))
     w = torch.zeros(T, E + 1)
     w[torch.arange(T), torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(T, generator=g)]] = 0.5
     w, lists, act = w.cuda(), torch.empty(2 * E * T + E, dtype=torch.int32, device="cuda"), torch.empty(T, f, dtype=torch.bfloat16, device="cuda")
     results = []
-    for units in (8, 40, 64, 80, 96, 112, 128, 256, 2000):
+    for units in all_units:
         planes = torch.full((1, T, D), float("nan"), device="cuda")
         ops._call("blm_moe_grouped", x.data_ptr(), D, gu.data_ptr(), down.data_ptr(), w.data_ptr(), E + 1, None, None, None, None, 0,
                   planes.data_ptr(), lists.data_ptr(), lists.data_ptr() + 8 * E * T, act.data_ptr(), T, D, E, f, 1, units, ops._stream())
