@@ -229,7 +229,8 @@ struct GvRope {
 // The weights come by buffer loads of their tile's bytes: of none behind a block's last tile, where they bring zeros without a trip to memory.
 // With a branch around them the compiler counts on the way without them, and every part waits for the next part's loads too.
 // Us, eight rows, with the branch, selects of every activation and look-ups of the block's size / so: [3072, 2048] 9.2 / 8.1, [2048, 2048] in two groups
-// 6.8 / 6.1, [16384, 2048] gated 27.0 / 26.0, [2048, 8192] in four 16.3 / 15.1; the head [128256, 2048], 31 tiles a block, 163 / 166.
+// 6.8 / 6.1, [16384, 2048] gated 27.0 / 26.0, [2048, 8192] in four 16.3 / 15.1; the head [128256, 2048], 31 tiles a block, 163 / 166
+// (165.6 / 165.9 with the rest as it is: what it lost is not the loads').
 // shape: 2 * wavefronts + gated, and the sums of a row that comes unscaled (the arguments' first fourteen dwords come in registers; a block's size would be a load).
 template <int KSTEPS, bool WHOLE, bool ROPE, bool ONE, int SCALED>
 __global__ void __launch_bounds__(GV_MAX_WAVES* BLM_WAVE)

@@ -429,7 +429,10 @@ __global__ void __launch_bounds__(512, 2)
   const int halves = (all[2] * n_tiles + units - 1) / units * 57, fives = (all[3] * n_tiles + units - 1) / units * GD_FIVE_PERCENT;
   // the parts behind the whole tiles: 1: an expert's last rows; 2, 3: all of them, in halves or five eighths
   // (five eighths from K = 1,024 on: what a block does besides its products is the same for a larger and a smaller one, and at K = 512 three
-  // rounds' worth of it cost more than the products saved: 2,048 tokens, 16 experts, down projection 38.6 us against 35.0; gate/up, K = 2,048, 42.6 against 51.4)
+  // rounds' worth of it cost more than the products saved: 2,048 tokens, 16 experts, down projection 38.6 us against 35.0; gate/up, K = 2,048, 42.6 against 51.4.
+  // Both products, 130 sizes of 700 to 4,200 tokens, 4 of 16, 2 of 8 or 6 of 64 experts, K of 512 to 4,096, one of the two 1,024 or more: 0.984 of the time without
+  // them in the mean, 0.85 (2,152 tokens, 2 of 8 experts of 1,024, width 2,048, 100.2 -> 85.4 us) to 1.04, more than 1.01 at ten sizes.  With them from
+  // K = 256 on, 130 sizes with a K of 512 to 896: 0.992 of this rule's time, 0.90 to 1.03: the line could lie lower)
   const int parts = K >= 1024 && fives < min(halves, mixed) ? 3 : halves < mixed ? 2 : 1;
   const int share1 = parts > 1 ? 0 : (wholes + 7) / 8, count2 = all[parts] * n_tiles, share2 = (count2 + 7) / 8;
   int b = blockIdx.x;
