@@ -20,6 +20,7 @@ from .base import KVNeed, Mixer, Product, TensorSpec, speaks_for
 DECODE_TARGET_PER_UNIT = 2
 DECODE_MIN_PER_UNIT = 0.5
 DECODE_MAX_PIECES = 32
+DECODE_WIDE_PIECES = 8
 
 
 def decode_splits(pages: int, blocks: int, head_dim: int, compute_units: int = 256) -> int:
@@ -50,9 +51,11 @@ def decode_splits(pages: int, blocks: int, head_dim: int, compute_units: int = 2
     16 pages: 4 pieces 7.9, 8 pieces 7.3), and ranges of up to 16 pages stay whole from a block for every
     fourth compute unit on (heads of 128, 11 pages at batch 8: uncut 12.3, in two 14.0; 16 pages at batch
     16: 16.9 / 18.5; heads of 64, 16 pages at batch 8: 9.1 / 10.0).  Longer ranges of wide heads go down to one page per wavefront
-    while the pieces still run in one round (16 heads of 128 in 4 groups, pieces by the rules above / by this one: 8 sequences of 18
-    pages 4 / 5 pieces 13.7 / 12.8, 24 pages 4 / 6 14.6 / 14.0, 32 pages 4 / 8 15.8 / 15.3; 16 sequences of 18 pages 2 / 4 17.1 / 15.7,
-    24 pages 3 / 4 16.9 / 17.0; in 8 groups, 8 sequences of 18 pages 2 / 4 17.2 / 15.6)."""
+    while the pieces still run in one round and are no more than eight, beyond which their merge costs more than they save (16 heads of
+    128 in 4 groups, pieces by the rules above / by this one: 8 sequences of 18 pages 4 / 5 pieces 13.7 / 12.8, 24 pages 4 / 6 14.6 /
+    14.0, 32 pages 4 / 8 15.8 / 15.3; 16 sequences of 18 pages 2 / 4 17.1 / 15.7, 24 pages 3 / 4 16.9 / 17.0; in 8 groups, 8 sequences
+    of 18 pages 2 / 4 17.2 / 15.6; but in 4 groups 4 sequences of 64 pages 8 / 16 16.1 / 16.9, 2 of 100 pages 16 / 25 15.2 / 15.7, and 16
+    heads of 96, one sequence of 64 pages 8 / 16 13.0 / 14.3)."""
     if blocks >= compute_units or pages <= (12 if head_dim <= 64 else 8):
         return 1
     if pages <= 16 and blocks * 4 >= compute_units:
@@ -62,7 +65,7 @@ def decode_splits(pages: int, blocks: int, head_dim: int, compute_units: int = 2
     if blocks * n < least:
         n = max(n, min(max(1, pages // 2), (least + blocks - 1) // blocks, DECODE_MAX_PIECES))
     if head_dim > 64:
-        n = max(n, min(-(-pages // 4), compute_units // blocks, DECODE_MAX_PIECES))
+        n = max(n, min(-(-pages // 4), compute_units // blocks, DECODE_WIDE_PIECES))
     return max(1, n)
 
 
