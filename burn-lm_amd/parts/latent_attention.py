@@ -42,6 +42,20 @@ EXPAND_MAX_BLOCKS = 65535      # sequences, and pages of one: the launch has a b
 MFMA_MAX_PIECES = 64           # most pieces the matrix-core decode cuts a sequence's half pages into
 
 
+
+def most_pieces(tiles, rank, compute_units):
+    """Into how many pieces the half pages of a decode step's tiles of 16 (token, head) pairs are cut at most.  A block of four wavefronts waits
+    out a half page's trip from memory with nothing else to do, so short pieces are what shortens the step: up to a block for every unit of
+    the chip, and from a block for every fourth unit on up to four pieces (16 heads, 512 + 64 lanes, us: 8 sequences of 1,125 tokens 32
+    pieces 16.5, all 36 half pages 19.0; 16 of 600 tokens, 16 / 19 pieces 17.3 / 19.3; 64 of 600, 4 / 8 / 15 pieces 33.2 / 37.2 / 42.3; 128
+    of 600, 2 / 4 / 7 pieces 58.7 / 53.6 / 59.6).  Of narrow latents, whose half pages are few loads, four blocks for every unit (8 heads, 128 +
+    64 lanes, 24 sequences of 2,500 tokens 10 / 42 pieces 22.1 / 17.9, a wavefront to a piece before 18.4; 40 of 6,000 tokens 6 / 25 68.4 /
+    41.0, 45.9; 64 of 1,125 4 / 16 24.9 / 20.8, 23.1; 4 heads, 64 + 32 lanes, 40 of 2,500 tokens 6 / 25 23.3 / 16.3, 17.4).  Wide ones
+    of long sequences would take twice as many as they are given (256 + 64 lanes, 40 of 2,500 tokens 6 / 12 / 25 46.0 / 36.1 / 39.1, before 51.7)."""
+    most = 4 * compute_units // tiles
+    return min(MFMA_MAX_PIECES, most if rank < 256 else max(compute_units // tiles, min(4, most)))
+
+
 class LatentAttention(Mixer):
     """params: width, heads, dim, rot_dim, vdim, kv_rank, scale, rot_dims, eps, position (the rotary table's
     owner, given by the model builder), pairing ("half", the default, or "adjacent"), q_rank (0, the default: queries
@@ -248,14 +262,8 @@ class LatentAttention(Mixer):
         seen = min(step.max_len_after, self.window) if self.window else step.max_len_after
         if qabs.dtype == torch.bfloat16:        # the matrix-core form: one wavefront per 16 (token, head) pairs
             if step.max_new == 1:
-                waves = step.n_seqs * ((H + 15) // 16)
                 halves = (seen + 31) // 32 + (1 if seen < step.max_len_after else 0)     # a window may begin inside a half page
-                # up to a block of four wavefronts for every unit of the chip, which waits out a half page's trip from memory with
-                # nothing else to do, so short pieces are what shortens the step; from a block for every fourth unit on up to four
-                # pieces (16 heads, 512 + 64 lanes, us: 8 sequences of 1,125 tokens 32 pieces 16.5, all 36 half pages 19.0; 16 of 600
-                # tokens, 16 / 19 pieces 17.3 / 19.3; 64 of 600, 4 / 8 / 15 pieces 33.2 / 37.2 / 42.3; 128 of 600, 2 / 4 / 7 pieces
-                # 58.7 / 53.6 / 59.6)
-                n_splits = max(1, min(halves, max(rt.compute_units // waves, min(4, 4 * rt.compute_units // waves)), MFMA_MAX_PIECES,
+                n_splits = max(1, min(halves, most_pieces(step.n_seqs * ((H + 15) // 16), R, rt.compute_units),
                                       ops.latent_attn_mfma_max_splits(step.n_seqs, 1, H, R)))
             return ops.latent_attn_mfma(qabs, olat, view.k, view.v, step, view.block_table(step), view.page_size, H, R,
                                         dr, self.scale, n_splits, window=self.window, sinks=self.sinks)

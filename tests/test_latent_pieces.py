@@ -41,3 +41,11 @@ def test_pieces(R, Dr, H, window):
                 want = torch.softmax(scores, 1)[:, :k.shape[0]] @ k[:, :R]
                 room = 2.0 ** -8 + 2 * (R + Dr) * 2.0 ** -24 * 40
                 assert float((got[b].double() - want).abs().max()) <= room * float(k[:, :R].abs().max()), (b, pieces)
+
+
+def test_most_pieces():
+    """Wide latents: a block for every unit, up to four pieces from a block for every fourth unit on; narrow ones: four blocks for every unit."""
+    from burn_lm_amd.parts.latent_attention import most_pieces
+    tiles = (1, 8, 16, 64, 90, 200, 300, 1024, 1025)
+    assert [most_pieces(n, 512, 256) for n in tiles] == [64, 32, 16, 4, 4, 4, 3, 1, 0]
+    assert [most_pieces(n, 192, 256) for n in tiles] == [64, 64, 64, 16, 11, 5, 3, 1, 0]
