@@ -234,17 +234,17 @@ __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
 // a group each reading the group's keys and values): 43.8 -> 13.3 in three pieces of whole pages; in a graph of its own 11.4, with
 // halves 10.5; 8 sequences of 8 pages in four pieces 10.6 -> 9.3 in halves, 8.7 in quarters; 24 heads of 128 15.9 -> 12.4.
 // ---------------------------------------------------------------------------------------------------------------------
-template <int HD>
+// FREE: lanes past the head are zeroed behind the loads, which then stand in no branch: behind one the values' loads wait for the keys'.
+// Heads of 64 in groups of four, 8 sequences of 1 / 4 / 9 / 18 pages, us, 5.2 / 9.0 / 12.1 / 16.9 without, 4.7 / 8.1 / 11.6 / 16.7 so.  Not
+// for heads of up to 48, whose lanes past them are a quarter of the loads and more (16 heads of 48, 40 sequences of 9 / 20 pages 42.1 / 76.6
+// without, 44.2 / 80.7 so; of 32, 4 pages 5.9 / 6.0), nor for wide ones, whose values take the keys' registers (128, 9 pages: 17.3 / 20.5).
+template <int HD, bool FREE>
 __global__ void __launch_bounds__(AF_DECODE_WAVES* BLM_WAVE)
     attn_decode_f32_kernel(const float* __restrict__ q, int q_row_stride, float* __restrict__ out, const int* __restrict__ positions,
                            const int* __restrict__ token_seq, const int* __restrict__ block_table, int table_width,
                            const float* __restrict__ kcache, const float* __restrict__ vcache, int nh, int nkv, int hd, float scale,
                            int window, int n_splits, float* part_o, float* part_ml, int* arrivals) {
   constexpr int DS = HD / 16;
-  // Lanes past the head are zeroed behind the loads, which then stand in no branch: behind one the values' loads wait for the keys'.
-  // Heads of 64 in groups of four, 8 sequences of 1 / 4 / 9 / 18 pages, us, 5.2 / 9.0 / 12.1 / 16.9 before, 4.7 / 8.1 / 11.6 / 16.7.
-  // Not for heads of 32 (5.9 / 6.0 at 4 pages) nor for wide ones, whose values take the keys' registers (128, 9 pages: 17.3 / 20.5).
-  constexpr bool FREE = HD == 64;
   __shared__ __attribute__((aligned(16))) float all_o[AF_DECODE_WAVES][16][HD + 4];
   __shared__ float all_m[AF_DECODE_WAVES][16], all_l[AF_DECODE_WAVES][16];
   __shared__ int is_last;
@@ -452,14 +452,15 @@ extern "C" int blm_attn_decode_f32(const void* q, int q_row_stride, void* out, c
   const long long y = (long long)nkv * ((nh / nkv + 15) / 16);
   BLM_REQUIRE(T > 0 && T <= 65535 && y <= 65535, "attn_decode_f32: bad sizes T=%d heads=%d", T, nh);
   dim3 grid((unsigned)n_splits, (unsigned)y, (unsigned)T), block(AF_DECODE_WAVES * BLM_WAVE);
-#define BLM_AFD(HD)                                                                                                       \
-  hipLaunchKernelGGL((attn_decode_f32_kernel<HD>), grid, block, 0, stream, (const float*)q, q_row_stride, (float*)out, positions, \
+#define BLM_AFD(HD, FREE)                                                                                                 \
+  hipLaunchKernelGGL((attn_decode_f32_kernel<HD, FREE>), grid, block, 0, stream, (const float*)q, q_row_stride, (float*)out, positions, \
                      token_seq, block_table, table_width, (const float*)kcache, (const float*)vcache, nh, nkv, hd, scale, window,  \
                      n_splits, part_o, part_ml, arrivals)
-  if (hd <= 32) BLM_AFD(32);
-  else if (hd <= 64) BLM_AFD(64);
-  else if (hd <= 96) BLM_AFD(96);
-  else BLM_AFD(128);
+  if (hd <= 32) BLM_AFD(32, false);
+  else if (hd <= 48) BLM_AFD(64, false);
+  else if (hd <= 64) BLM_AFD(64, true);
+  else if (hd <= 96) BLM_AFD(96, false);
+  else BLM_AFD(128, false);
 #undef BLM_AFD
   BLM_LAUNCH_CHECK("attn_decode_f32");
   return 0;

@@ -43,7 +43,7 @@ def check(got, q, k, v, pos, scale, window, group):
     assert bool(((got.double() - want).abs() <= bound[:, None]).all()), float(((got.double() - want).abs() / bound[:, None]).max())
 
 
-SHAPES = [(4, 4, 64), (8, 2, 64), (6, 1, 24), (5, 1, 4), (40, 2, 16), (6, 2, 128), (8, 1, 100), (3, 3, 72), (7, 1, 96)]
+SHAPES = [(4, 4, 64), (8, 2, 64), (6, 1, 24), (5, 1, 4), (40, 2, 16), (6, 2, 128), (8, 1, 100), (3, 3, 72), (7, 1, 96), (6, 2, 36), (4, 2, 48), (5, 1, 60)]
 
 
 @pytest.mark.parametrize("window", [0, 1, 70])
