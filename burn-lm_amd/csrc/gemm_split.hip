@@ -1,0 +1,335 @@
+// The 32-bit product C[M,N] = A[M,K] * W[N,K]^T of many rows on the bfloat16 matrix instructions, with no less precision than on the
+// float ones: a float is the sum of three bfloat16 (hi, mid, lo, rounded to nearest each: 8 + 8 + 8 bits and their signs, the subtractions
+// between them exact), a product of two floats the sum of nine exact products, and the three that are left out (mid lo, lo mid, lo lo)
+// are below 2^-26 of the whole (floats below 2^-110 have no lo of their own: what is lost of them is below 2^-134).  Six instructions of 16 cycles do 16 x 16 x 32, for which the float ones take 256 cycles.
+//   split_rows : the parts of the rows, in the order of the instruction's fragments
+//   gemm_split : the product; the weights, which are not kept a second time, are split on their way from shared memory
+// What bounds it: the matrix instructions at the clock that the card's power leaves (1.25 to 1.35 PFLOP/s of them), beside them reads of
+// shared memory (a fragment of three parts serves six or twelve instructions) and the splitting: 88 vector instructions for 192
+// matrix ones at 128 x 256.  Every wavefront has all rows of the tile and columns of its own, so that no weight is split twice in a block.
+// Sums: the matrix instruction adds to its accumulator with what falls off below cut, towards minus infinity: a result of 2,048 products by
+// one accumulator is 2.7e-7 off and, the same in all of them, 3e-8 too low, which adds up from layer to layer (logits of the 1B shape
+// 3.7e-6 from 64 bits, with the float instructions 2.8e-6).  So a chunk of 128 of K has an accumulator that starts at zero, small products
+// first, and joins the total by a rounded addition; and every other chunk is summed with its columns negated and subtracted, so that what is
+// cut cancels: 1.7e-7 off (2.17e-7 with the float instructions), 7e-11 too low, and the logits 2.6e-6.
+// Measured (us, the float instructions' best tile before, 1,000 rows): [16384, 2048] gated 493 -> 281 (239 TFLOP/s of float products),
+// [2048, 8192] in four groups 272 -> 148, [3072, 2048] 110 -> 75, [2048, 2048] 78 -> 43; the parts' pass 7 and (K = 8,192) 14.  The scoring of
+// 1,000 tokens at the 1B shape 16.95 -> 11.5 ms.
+// Tried: columns from global memory straight into registers (120 -> 133 us on 64 blocks), tiles of 256 x 256 (two stages fill the
+// shared memory: 334 against 312), two accumulators for small and large products without the rounded additions (5 % faster, 2.7e-7 off),
+// the small products' sums added in every step (1.06e-7 off, registers spill).
+#include <type_traits>
+
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 gs_bf16x8;
+typedef __attribute__((ext_vector_type(4))) float gs_f32x4;
+typedef __attribute__((ext_vector_type(4))) unsigned int gs_u32x4;
+
+#define GS_BK 32
+#define GS_FRAGMENT 1024                  // bytes: 16 rows and 32 of K of one part, 16 bytes a lane
+
+__device__ __forceinline__ float gs_low(uint32_t v) { return __uint_as_float(v << 16); }
+__device__ __forceinline__ float gs_high(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
+
+__device__ __forceinline__ void gs_split(float x, float y, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = f32x2_to_bf16x2_bits(x, y);
+  x -= gs_low(hi);
+  y -= gs_high(hi);
+  mid = f32x2_to_bf16x2_bits(x, y);
+  lo = f32x2_to_bf16x2_bits(x - gs_low(mid), y - gs_high(mid));
+}
+
+// A value that has no such parts, or whose first would round to an infinity: hi keeps an infinity or NaN alone, and is cut off otherwise.
+__device__ __forceinline__ void gs_split_odd(float x, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  const uint32_t bits = __float_as_uint(x);
+  hi = bits >> 16;
+  mid = lo = 0u;
+  if ((bits & 0x7fffffffu) > 0x7f800000u) hi |= 0x40u;
+  else if ((bits & 0x7f800000u) != 0x7f800000u) {
+    x -= gs_low(hi);
+    mid = f32_to_bf16_bits(x);
+    lo = f32_to_bf16_bits(x - gs_low(mid));
+  }
+}
+__device__ __forceinline__ bool gs_odd(float x) { return (__float_as_uint(x) & 0x7fffffffu) >= 0x7f7f8000u; }
+
+// ---------------------------------------------------------------------------------------------------------------------
+// parts of the rows: P [ceil(M / 16)][K / 32][3][64 lanes][8]: lane l holds row l % 16, elements 4 (l / 16) + 0..3 and 16 + 4 (l / 16) + 0..3
+// of the 32; rows behind M are zero.
+__global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict__ X, int ldx, uint4* __restrict__ P, int M, int K) {
+  const int lane = threadIdx.x & 63, steps = K / GS_BK, per_tile = (steps + 3) / 4, tile = blockIdx.x / per_tile;
+  const int ks = (blockIdx.x - tile * per_tile) * 4 + threadIdx.x / 64;
+  if (ks >= steps) return;
+  const int m = tile * 16 + (lane & 15);
+  float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
+  if (m < M) {
+    const float* x = X + (size_t)m * ldx + ks * GS_BK + (lane >> 4) * 4;
+    u = *reinterpret_cast<const float4*>(x);
+    v = *reinterpret_cast<const float4*>(x + 16);
+  }
+  const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+  uint32_t hi[4], mid[4], lo[4];
+  bool odd = false;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) odd |= gs_odd(x[e]);
+  if (!odd) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) gs_split(x[2 * e], x[2 * e + 1], hi[e], mid[e], lo[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t h, m, l;
+      gs_split_odd(x[2 * e], hi[e], mid[e], lo[e]);
+      gs_split_odd(x[2 * e + 1], h, m, l);
+      hi[e] |= h << 16;
+      mid[e] |= m << 16;
+      lo[e] |= l << 16;
+    }
+  }
+  uint4* p = P + ((size_t)tile * steps + ks) * 192 + lane;
+  p[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+  p[64] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
+  p[128] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+}
+
+extern "C" int blm_split_rows(const void* X, void* P, int M, int K, int ldx, hipStream_t stream) {
+  BLM_REQUIRE(M > 0 && K > 0 && K % GS_BK == 0 && ldx >= K && ldx % 4 == 0, "split_rows: sizes M=%d K=%d ldx=%d not supported", M, K, ldx);
+  BLM_REQUIRE(((uintptr_t)X % 16) == 0 && ((uintptr_t)P % 16) == 0, "split_rows: rows and parts must be 16-byte aligned");
+  const long long blocks = (long long)((M + 15) / 16) * ((K / GS_BK + 3) / 4);
+  BLM_REQUIRE(blocks < 2147483647LL, "split_rows: too many rows");
+  hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, (const float*)X, ldx, (uint4*)P, M, K);
+  BLM_LAUNCH_CHECK("split_rows");
+  return 0;
+}
+
+__device__ __forceinline__ float gs_silu_times(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+
+// One element in float, from the floats themselves: where an operand is not finite (or rounds to an infinity as a bfloat16) its parts give NaN
+// (an infinity less itself, or times a part that is zero), which this replaces by what the sum is.
+__device__ __forceinline__ float gs_repair(const unsigned char* P, const float* w, int m, int steps_all, int s_begin, int stages) {
+  float sum = 0.f;
+  const unsigned char* tile = P + (size_t)(m / 16) * steps_all * (3 * GS_FRAGMENT) + (m % 16) * 16;
+  for (int s = s_begin; s < s_begin + stages; ++s)
+    for (int k = 0; k < GS_BK; ++k) {
+      const unsigned char* at = tile + (size_t)s * (3 * GS_FRAGMENT) + (k % 16 / 4) * 256 + (k / 16 * 4 + k % 4) * 2;
+      const float a = to_float(*reinterpret_cast<const bf16*>(at)) +
+                      (to_float(*reinterpret_cast<const bf16*>(at + GS_FRAGMENT)) + to_float(*reinterpret_cast<const bf16*>(at + 2 * GS_FRAGMENT)));
+      sum += a * w[(size_t)s * GS_BK + k];
+    }
+  return sum;
+}
+
+template <int V>
+using GsInt = std::integral_constant<int, V>;
+
+// MT x 16 rows by 8 x NT x 16 columns, eight wavefronts beside each other: each has all rows and 16 NT columns.  Stages of 32 of K: a ring of
+// three of the rows' parts and one of two of each wavefront's own columns.  One barrier a stage, in its middle: behind it the next
+// stage's operands are there, the one after that is asked for, and the next columns are split beside the second half's products.
+// lane l of a product: row l % 16, columns 4 (l / 16) + 0..3.  W rows past the end are the last one again; nothing stores what comes of them.
+template <int MT, int NT, bool GATED>
+__global__ void __launch_bounds__(512, MT * NT <= 4 ? 4 : 2)
+    gemm_split_kernel(const unsigned char* __restrict__ P, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K, int ldc,
+                      int steps_per_group, long long plane, int m_tiles, int n_tiles) {
+  static_assert(!GATED || NT == 2, "a gated wavefront has a tile of gate columns and their up columns");
+  constexpr int A_LOADS = (3 * MT + 7) / 8, B_LOADS = 2 * NT;
+  constexpr int A_STAGE = MT * 3 * GS_FRAGMENT, B_STAGE = 8 * NT * 2048;
+  constexpr int COLUMNS = GATED ? 128 : 128 * NT;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[3 * A_STAGE + 2 * B_STAGE];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / BLM_WAVE), lane = tid & (BLM_WAVE - 1);
+  const int l16 = lane & 15, quad = lane >> 4;
+  const int die = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const int nt = (at / m_tiles) * 8 + die, mt = at % m_tiles;
+  if (nt >= n_tiles) return;
+  const int m0 = mt * MT * 16, n0 = nt * COLUMNS, steps_all = K / GS_BK;
+  const int s_begin = blockIdx.y * steps_per_group, stages = min(steps_per_group, steps_all - s_begin), last = stages - 1;
+
+  const char* a_base = reinterpret_cast<const char*>(P) + ((size_t)(m0 / 16) * steps_all + s_begin) * (3 * GS_FRAGMENT);
+  const char* b_base = reinterpret_cast<const char*>(W + (size_t)n0 * K + (size_t)s_begin * GS_BK);
+  const int row_tiles = (M + 15) / 16 - m0 / 16;
+  uint32_t a_off[A_LOADS], b_off[B_LOADS], a_to[A_LOADS];
+#pragma unroll
+  for (int x = 0; x < A_LOADS; ++x) {
+    int f = x * 8 + wave;
+    if (f >= 3 * MT) f -= 8;              // brings the one before again
+    a_off[x] = (uint32_t)min(f / 3, row_tiles - 1) * (uint32_t)steps_all * (3u * GS_FRAGMENT) + (uint32_t)(f % 3) * GS_FRAGMENT + lane * 16u;
+    a_to[x] = (uint32_t)f * GS_FRAGMENT;
+  }
+#pragma unroll
+  for (int x = 0; x < B_LOADS; ++x) {
+    const int j = x >> 1, r = (x & 1) * 8 + lane / 8, piece = (lane & 7) ^ ((r >> 1) & 7);
+    const int n = min(GATED ? wave * 16 + r : wave * 16 * NT + j * 16 + r, N - 1 - n0);
+    b_off[x] = ((uint32_t)n + (GATED && j ? (uint32_t)N : 0u)) * (uint32_t)K * 4u + piece * 16u;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(blm_lds_ptr)lds;
+  const uint32_t b_to = lds0 + 3 * A_STAGE + (uint32_t)wave * (NT * 2048);
+  auto fetch = [&](int s, int a_slot, int b_slot) {
+    const char *a = a_base + (size_t)s * (3 * GS_FRAGMENT), *b = b_base + (size_t)s * (GS_BK * 4);
+#pragma unroll
+    for (int x = 0; x < B_LOADS; ++x) blm_dma16_to(b, b_off[x], b_to + (uint32_t)(b_slot * B_STAGE + x * 1024));
+#pragma unroll
+    for (int x = 0; x < A_LOADS; ++x) blm_dma16_to(a, a_off[x], lds0 + (uint32_t)(a_slot * A_STAGE) + a_to[x]);
+  };
+
+  const int b_at = 3 * A_STAGE + wave * (NT * 2048) + l16 * 128;
+  const int slot0 = (quad ^ ((l16 >> 1) & 7)) * 16, slot1 = ((4 + quad) ^ ((l16 >> 1) & 7)) * 16;
+  gs_f32x4 raw[NT][2];
+  gs_u32x4 b[2][NT][3];
+  auto read_raw = [&](int slot, int j) {
+    raw[j][0] = *reinterpret_cast<const gs_f32x4*>(lds + slot * B_STAGE + b_at + j * 2048 + slot0);
+    raw[j][1] = *reinterpret_cast<const gs_f32x4*>(lds + slot * B_STAGE + b_at + j * 2048 + slot1);
+  };
+  auto split_half = [&](gs_u32x4 (&to)[NT][3], int j, int x, auto negative) {
+    constexpr bool minus = decltype(negative)::value;
+    uint32_t h[2], m[2], l[2];
+    const gs_f32x4 v = raw[j][x];
+    gs_split(minus ? -v[0] : v[0], minus ? -v[1] : v[1], h[0], m[0], l[0]);
+    gs_split(minus ? -v[2] : v[2], minus ? -v[3] : v[3], h[1], m[1], l[1]);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      to[j][0][2 * x + e] = h[e];
+      to[j][1][2 * x + e] = m[e];
+      to[j][2][2 * x + e] = l[e];
+    }
+  };
+  constexpr int TOGETHER = NT == 1 ? 2 : 1, GROUPS = MT / TOGETHER, HALF = GROUPS > 2 ? GROUPS / 2 : 0;
+  constexpr int first[6] = {2, 0, 1, 1, 0, 0}, second[6] = {0, 2, 1, 0, 1, 0};      // small ones first
+  gs_u32x4 a[2][TOGETHER][3];
+  gs_f32x4 total[MT][NT], t[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) total[i][j] = t[i][j] = gs_f32x4{0.f, 0.f, 0.f, 0.f};
+  auto read_a = [&](int set, int slot, int g) {
+#pragma unroll
+    for (int x = 0; x < TOGETHER; ++x)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        a[set][x][p] = *reinterpret_cast<const gs_u32x4*>(lds + slot * A_STAGE + ((g * TOGETHER + x) * 3 + p) * GS_FRAGMENT + lane * 16);
+  };
+  auto add = [&](int g, auto negative) {
+#pragma unroll
+    for (int x = 0; x < TOGETHER; ++x)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        if (decltype(negative)::value) total[g * TOGETHER + x][j] -= t[g * TOGETHER + x][j];
+        else total[g * TOGETHER + x][j] += t[g * TOGETHER + x][j];
+        t[g * TOGETHER + x][j] = gs_f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  // a stage; on entry its first rows' fragments and its columns' parts are in registers
+  auto stage = [&](int s, int slot, auto place_type, auto negative) {
+    constexpr int place = decltype(place_type)::value, now = place & 1, next = now ^ 1;
+    using NextNegative = std::integral_constant<bool, decltype(negative)::value != (place == 3)>;
+    const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot == 0 ? 2 : slot - 1;
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+      const int set = g & 1;
+      read_a(set ^ 1, g + 1 < GROUPS ? slot : slot1, g + 1 < GROUPS ? g + 1 : 0);
+      if (g == HALF) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + 2 <= last) fetch(s + 2, slot2, now);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) read_raw(next, j);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int p = 0; p < 6; ++p)
+#pragma unroll
+        for (int x = 0; x < TOGETHER; ++x)
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            t[g * TOGETHER + x][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gs_bf16x8, b[now][j][first[p]]),
+                                                                             __builtin_bit_cast(gs_bf16x8, a[set][x][second[p]]), t[g * TOGETHER + x][j], 0, 0, 0);
+      if (place == 3 && g > 0) add(g - 1, negative);
+      // the next columns' parts beside the last products
+#pragma unroll
+      for (int y = 0; y < 2 * NT; ++y)
+        if (g - HALF == y * (GROUPS - HALF) / (2 * NT)) split_half(b[next], y >> 1, y & 1, NextNegative{});
+    }
+    if (place == 3) add(GROUPS - 1, negative);
+    return slot1;
+  };
+  static_assert(GROUPS % 2 == 0, "the first rows' fragments of every stage lie in the same set");
+  fetch(0, 0, 0);
+  fetch(1, 1, 1);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(A_LOADS + B_LOADS) : "memory");
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    read_raw(0, j);
+    split_half(b[0], j, 0, std::false_type{});
+    split_half(b[0], j, 1, std::false_type{});
+  }
+  read_a(0, 0, 0);
+  int slot = 0;
+  auto chunk = [&](int s, auto negative) {
+    slot = stage(s, slot, GsInt<0>{}, negative);
+    slot = stage(s + 1, slot, GsInt<1>{}, negative);
+    slot = stage(s + 2, slot, GsInt<2>{}, negative);
+    slot = stage(s + 3, slot, GsInt<3>{}, negative);
+  };
+  for (int s = 0; s < stages; s += 8) {
+    chunk(s, std::false_type{});
+    if (s + 4 < stages) chunk(s + 4, std::true_type{});
+  }
+
+  float* out = C + (size_t)blockIdx.y * plane;
+  unsigned long long odd = 0;              // elements that are not a number: bit (i * NT + j) * 4 + e, gated i * 4 + e
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = m0 + i * 16 + l16;
+#pragma unroll
+    for (int j = 0; j < (GATED ? 1 : NT); ++j) {
+      const int n = n0 + wave * 16 * (GATED ? 1 : NT) + j * 16 + quad * 4;
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = GATED ? gs_silu_times(total[i][0][e], total[i][NT - 1][e]) : total[i][j][e];
+        odd |= (unsigned long long)(v[e] != v[e]) << ((i * (GATED ? 1 : NT) + j) * 4 + e);
+      }
+      if (m < M && n < N) *reinterpret_cast<float4*>(out + (size_t)m * ldc + n) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  }
+  for (; odd != 0; odd &= odd - 1) {
+    const int at = __builtin_ctzll(odd), tile = at >> 2, i = GATED ? tile : tile / NT, j = GATED ? 0 : tile % NT;
+    const int m = m0 + i * 16 + l16, n = n0 + wave * 16 * (GATED ? 1 : NT) + j * 16 + quad * 4 + (at & 3);
+    if (m >= M || n >= N) continue;
+    float v = gs_repair(P, W + (size_t)n * K, m, steps_all, s_begin, stages);
+    if (GATED) v = gs_silu_times(v, gs_repair(P, W + (size_t)(N + n) * K, m, steps_all, s_begin, stages));
+    out[(size_t)m * ldc + n] = v;
+  }
+}
+
+// P: the parts of A [M, K] (split_rows).  rows x columns: a block's tile, 128 or 64 by 256 or 128 (gated: gate and up columns
+// together, 256).  groups > 1: K in that many groups, C holds a plane of M * N for each (contiguous, ldc = N), which the reader adds up.
+extern "C" int blm_gemm_split(const void* P, const void* W, void* C, int M, int N, int K, int ldc, int gated, int groups, int rows,
+                              int columns, hipStream_t stream) {
+  BLM_REQUIRE(M > 0 && N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0 && ldc >= N && ldc % 4 == 0, "gemm_split: sizes M=%d N=%d K=%d ldc=%d not supported",
+              M, N, K, ldc);
+  BLM_REQUIRE(((uintptr_t)P % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)C % 16) == 0, "gemm_split: operands must be 16-byte aligned");
+  const int steps = groups >= 1 ? (K / 128 + groups - 1) / groups * 4 : 0;
+  BLM_REQUIRE(groups >= 1 && groups <= 64 && (groups == 1 || (!gated && ldc == N)) && (groups - 1) * steps * GS_BK < K, "gemm_split: %d groups of K=%d", groups, K);
+  BLM_REQUIRE(((gated ? N : 0) + 256LL) * K * 4 < (1LL << 32), "gemm_split: gated matrices of 4 GiB and more are not supported (N=%d K=%d)", N, K);
+  BLM_REQUIRE((rows == 128 || rows == 64) && (columns == 256 || (columns == 128 && !gated)), "gemm_split: tile %d x %d", rows, columns);
+  const int per = gated ? columns / 2 : columns;
+  const int m_tiles = (M + rows - 1) / rows, n_tiles = (N + per - 1) / per;
+  const long long blocks = (long long)m_tiles * ((n_tiles + 7) / 8 * 8);
+  BLM_REQUIRE(blocks < 2147483647LL, "gemm_split: too many tiles");
+  dim3 grid((unsigned)blocks, (unsigned)groups), block(512);
+#define GS_RUN(MT, NT, G)                                                                                                             \
+  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, G>), grid, block, 0, stream, (const unsigned char*)P, (const float*)W, (float*)C, M, N, \
+                     K, ldc, steps, (long long)M * N, m_tiles, n_tiles)
+  if (gated) {
+    if (rows == 128) GS_RUN(8, 2, true);
+    else GS_RUN(4, 2, true);
+  } else if (columns == 256) {
+    if (rows == 128) GS_RUN(8, 2, false);
+    else GS_RUN(4, 2, false);
+  } else {
+    if (rows == 128) GS_RUN(8, 1, false);
+    else GS_RUN(4, 1, false);
+  }
+#undef GS_RUN
+  BLM_LAUNCH_CHECK("gemm_split");
+  return 0;
+}

@@ -137,6 +137,8 @@ _SIGNATURES = {
                               _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
                               _c_int, _c_int, _c_void_p, _c_int, _c_float, _c_int, _c_void_p],
     "blm_gemm_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "blm_split_rows": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
+    "blm_gemm_split": [_c_void_p, _c_void_p, _c_void_p] + [_c_int] * 8 + [_c_void_p],
     "blm_gemv_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_gemv_f32_qkv_rope": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 9 + [_c_void_p],
     "blm_gemv_f32_scaled": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_int, _c_float,
@@ -641,6 +643,47 @@ def gemm_f32(a, w, out, gated=False, tile=(128, 128)):
         raise KernelError(f"gemm_f32: tile {tile} is not one of {sorted(F32_TILES)}")
     _call("blm_gemm_f32", a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, a.shape[1], a.stride(0), out.stride(-2), 1 if gated else 0,
           groups, F32_TILES[tile], _stream())
+    return out
+
+
+# rows x columns of a block's tile of gemm_split
+SPLIT_TILES = ((128, 256), (128, 128), (64, 256), (64, 128))
+
+
+def split_takes(M, N, K, gated=False):
+    """Whether gemm_split has these sizes (its rows and weights as f32_rows wants them)."""
+    return M > 0 and K % 128 == 0 and N % 16 == 0 and (not gated or (N + 256) * K * 4 < 1 << 32)
+
+
+def split_rows(a):
+    """The three bfloat16 parts of float32 rows [M, K], in the order gemm_split reads them: [ceil(M / 16), K / 32, 3, 64, 8]."""
+    _gpu(a)
+    M, K = a.shape
+    if a.dtype != torch.float32 or a.stride(1) != 1 or K % 32 != 0 or a.stride(0) % 4 != 0 or a.data_ptr() % 16 != 0:
+        raise KernelError("split_rows: float32 rows in units of 16 bytes and widths in multiples of 32 wanted")
+    parts = torch.empty(-(-M // 16), K // 32, 3, 64, 8, dtype=torch.bfloat16, device=a.device)
+    _call("blm_split_rows", a.data_ptr(), parts.data_ptr(), M, K, a.stride(0), _stream())
+    return parts
+
+
+def gemm_split(parts, w, out, gated=False, tile=(128, 256)):
+    """gemm_f32 by the parts of its rows (split_rows): out [M, N], or [groups, M, N] partial products over that many groups of K;
+    gated=True as there."""
+    _gpu(parts, w, out)
+    groups = out.shape[0] if out.dim() == 3 else 1
+    M, N = out.shape[-2:]
+    K = w.shape[1]
+    if w.dtype != torch.float32 or out.dtype != torch.float32 or out.stride(-1) != 1 or not w.is_contiguous():
+        raise KernelError("gemm_split: float32 weights and results with contiguous rows wanted")
+    if parts.dtype != torch.bfloat16 or not parts.is_contiguous() or tuple(parts.shape) != (-(-M // 16), K // 32, 3, 64, 8):
+        raise KernelError(f"gemm_split: the parts {tuple(parts.shape)} are not those of {M} rows of {K}")
+    if w.shape[0] != N * (2 if gated else 1) or not split_takes(M, N, K, gated):
+        raise KernelError(f"gemm_split: shapes w={tuple(w.shape)} out={tuple(out.shape)} do not fit")
+    if out.dim() == 3:
+        _contig("out", out)
+    if tile not in SPLIT_TILES:
+        raise KernelError(f"gemm_split: tile {tile} is not one of {SPLIT_TILES}")
+    _call("blm_gemm_split", parts.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, out.stride(-2), 1 if gated else 0, groups, *tile, _stream())
     return out
 
 

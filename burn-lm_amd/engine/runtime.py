@@ -5,7 +5,8 @@ Matrix products ``x[M,K] @ w[N,K]^T``:
   reduced-precision matrix mode), whatever the activation dtype.  This is the whole float32 path
   and also what keeps a tensor that a checkpoint stores in 32 bits exact in a bfloat16 run.  With float32
   activations whose rows lie in units of 16 bytes: up to 16 rows ops.gemv_f32 on a packed copy, more rows (from 9
-  on where there is no such copy) ops.gemm_f32 (f32_plan chooses its tile and groups of K); everything else
+  on where there is no such copy) ops.gemm_f32 (f32_plan chooses its tile and groups of K) or, from 100 to 400 rows on,
+  ops.gemm_split (the same products by three exact bfloat16 parts of each float; split_plan); everything else
   ops.gemv_skinny up to 8 rows and ops.gemm_tiled.
 * bfloat16 weights, up to 64 rows (decode): the hand-written skinny kernel on the matrix cores that
   streams the weight once (where the width fits its registers: see ops.gemv_mfma_group_limit).  From
@@ -113,6 +114,39 @@ def f32_plan(M, N, K, compute_units, planes=False, gated=False):
             if best is None or us < best[2] * 0.999:
                 best = ((bm, bn), groups, us)
     return best
+
+
+# Tiles of ops.gemm_split: microseconds for a step of 32 along K of a block while few units are busy, and while all are (the card's
+# power).  Two blocks of the smallest share a unit.  Measured with 17 to 4,000 rows at [16384, 2048] gated, [2048, 8192] in 1 to 8
+# groups, [3072, 2048], [2048, 2048].
+SPLIT_STEP_US = {(128, 256): (1.78, 2.22), (128, 128): (1.0, 1.3), (64, 256): (1.04, 1.32), (64, 128): (0.66, 0.74)}
+SPLIT_PAIR_US = 0.66
+
+
+@functools.lru_cache(maxsize=4096)
+def split_plan(M, N, K, compute_units, planes=False, gated=False):
+    """(tile, groups of K, microseconds with the pass that makes the rows' parts) of ops.gemm_split, as f32_plan has them of
+    ops.gemm_f32; None where it does not have the sizes."""
+    if not ops.split_takes(M, N, K, gated):
+        return None
+    best = None
+    for (bm, bn), (few, all_) in SPLIT_STEP_US.items():
+        if gated and bn != 256:
+            continue
+        tiles = -(-M // bm) * -(-N // (bn // 2 if gated else bn))
+        for groups in (1, 2, 4, 8) if planes and not gated else (1,):
+            steps = -(-K // 128 // groups) * 4
+            if groups > 1 and (K // groups < 256 or (groups - 1) * steps * 32 >= K):
+                continue
+            per_unit = -(-tiles * groups // compute_units)
+            fill = tiles * groups / (per_unit * compute_units)
+            step = few + (all_ - few) * fill
+            if (bm, bn) == (64, 128) and per_unit > 1:
+                step = SPLIT_PAIR_US
+            us = 3.0 + steps * per_unit * step + (M * N * groups * 4 / 5e6 if groups > 1 else 0.0)
+            if best is None or us < best[2] * 0.999:
+                best = ((bm, bn), groups, us)
+    return best[0], best[1], best[2] + max(7.0, M * K * 10 / 6e6)
 
 
 # ops.gemm_duo: what half a tile takes of a whole one's time (K = 2048 / 8192, all blocks at once: 22 of 38 us, 73 of 128), and how
@@ -351,7 +385,15 @@ class Runtime:
                     return ops.sum_planes(parts, out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device))
         if M <= SKINNY_MAX_ROWS:
             return None
-        tile, groups, _ = f32_plan(M, N, K, self.compute_units, planes)
+        tile, groups, us = f32_plan(M, N, K, self.compute_units, planes)
+        split = split_plan(M, N, K, self.compute_units, planes)
+        if split is not None and split[2] < us and (out is None or (out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0)):
+            tile, groups, _ = split
+            if groups > 1:
+                out = torch.empty(groups, M, N, dtype=torch.float32, device=x.device)
+            elif out is None:
+                out = torch.empty(M, N, dtype=torch.float32, device=x.device)
+            return ops.gemm_split(ops.split_rows(x), w, out, tile=tile)
         if groups > 1:
             return ops.gemm_f32(x, w, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), tile=tile)
         return ops.gemm_f32(x, w, out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device), tile=tile)
@@ -769,6 +811,9 @@ class Runtime:
                     return ops.gemv_f32(x, packed, torch.empty(M, inner, dtype=torch.float32, device=x.device), K, gated=True)
             else:
                 tile, _, fused = f32_plan(M, inner, K, self.compute_units, gated=True)
+                split = split_plan(M, inner, K, self.compute_units, gated=True)
+                if split is not None and split[2] < fused:
+                    return ops.gemm_split(ops.split_rows(x), plain, torch.empty(M, inner, dtype=torch.float32, device=x.device), gated=True, tile=split[0])
                 # few rows: the plain product's smaller tiles and the pass behind it (12 bytes an element)
                 if fused <= f32_plan(M, 2 * inner, K, self.compute_units)[2] + 3.0 + M * inner * 12 / 5e6:
                     return ops.gemm_f32(x, plain, torch.empty(M, inner, dtype=torch.float32, device=x.device), gated=True, tile=tile)

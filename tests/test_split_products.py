@@ -1,0 +1,155 @@
+"""The float32 products by three bfloat16 parts of every float (gemm_split): the parts, every tile, edges of tiles, groups of K, gating,
+values that have no parts, the error beside the float instructions', and the runtime's choice.
+
+The bound on an element's error is that of a sum of K products in any order with one rounding per product and addition, as for the float
+instructions (test_f32_products): the products of parts that are left out are below 2^-26 of a product."""
+import pytest
+import torch
+
+from test_f32_products import check, operands
+
+TILES = [(128, 256), (128, 128), (64, 256), (64, 128)]
+INF, NAN = float("inf"), float("nan")
+
+
+def whole_again(parts, M, K):
+    """The floats that the parts add up to (in 64 bits)."""
+    p = parts.double().sum(2).reshape(-1, K // 32, 4, 16, 2, 4)              # [row tile, step, quarter, row, half, element]
+    return p.permute(0, 3, 1, 4, 2, 5).reshape(-1, K)[:M]                    # element 16 half + 4 quarter + e of a step
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,pad", [(1, 32, 0), (16, 64, 4), (17, 160, 0), (45, 416, 8)])
+def test_parts_are_the_float(M, K, pad):
+    from burn_lm_amd.csrc import ops
+    x, _ = operands(M, 1, K, pad)
+    x.mul_(torch.exp2(torch.randint(-60, 60, (M, K), generator=torch.Generator().manual_seed(1)).float().cuda()))
+    x[0, 0], x[-1, -1], x[M // 2, 3] = 0.0, torch.finfo(torch.float32).max, -torch.finfo(torch.float32).max
+    parts = ops.split_rows(x)
+    assert torch.equal(whole_again(parts, M, K), x.double())
+    rest = parts.reshape(-1, K // 32, 3, 4, 16, 8)[-1, :, :, :, M % 16 or 16:]
+    assert bool((rest == 0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K", [(1, 16, 128), (17, 48, 256), (64, 128, 384), (65, 144, 128), (128, 272, 640), (129, 256, 256), (300, 528, 512)])
+def test_tiles(tile, M, N, K):
+    from burn_lm_amd.csrc import ops
+    x, w = operands(M, N, K, pad=4 * (M % 3))
+    parts = ops.split_rows(x)
+    wide = torch.full((M, N + 4), NAN, device="cuda")
+    check(ops.gemm_split(parts, w, wide[:, :N], tile=tile), x, w)
+    assert bool(wide[:, N:].isnan().all())
+    for groups in (2, 5):
+        if (groups - 1) * -(-(K // 128) // groups) < K // 128:
+            check(ops.gemm_split(parts, w, torch.full((groups, M, N), NAN, device="cuda"), tile=tile).sum(0), x, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [(128, 256), (64, 256)])
+@pytest.mark.parametrize("M,I,K", [(17, 16, 128), (64, 128, 384), (130, 144, 256), (129, 400, 512)])
+def test_gated(tile, M, I, K):
+    from burn_lm_amd.csrc import ops
+    x, w = operands(M, 2 * I, K, pad=4)
+    check(ops.gemm_split(ops.split_rows(x), w, torch.full((M, I), NAN, device="cuda"), gated=True, tile=tile), x, w, gated=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,groups", [(2048, 1), (2048, 4), (8192, 1), (8192, 4)])
+@pytest.mark.parametrize("spread", [0.0, 2.0])
+def test_no_further_from_64_bits(K, groups, spread):
+    """2-norm of the error, normal values and ones that spread over some powers of ten: no larger than the float instructions'."""
+    from burn_lm_amd.csrc import ops
+    x, w = operands(300, 512, K, seed=K)
+    g = torch.Generator().manual_seed(2)
+    x, w = (t * torch.exp(spread * torch.randn(t.shape, generator=g)).cuda() for t in (x, w))
+    want = x.double() @ w.double().t()
+    err = lambda y: float((y.double() - want).norm() / want.norm())
+    out = lambda: torch.empty(groups, 300, 512, device="cuda")
+    theirs = err(ops.gemm_f32(x, w, out()).sum(0))
+    for tile in TILES:
+        assert err(ops.gemm_split(ops.split_rows(x), w, out(), tile=tile).sum(0)) <= theirs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+def test_values_without_parts(tile):
+    """Infinities, NaN and floats that round to an infinity as a bfloat16, in rows and in weights: what a sum of float products gives."""
+    from burn_lm_amd.csrc import ops
+    huge = torch.finfo(torch.float32).max
+    x, w = operands(70, 160, 256)
+    w[5, 7] = 0.0
+    w.mul_(2.0 ** -12)
+    for m, k, v in ((1, 7, INF), (2, 9, -INF), (3, 200, NAN), (4, 0, huge), (66, 255, -huge), (68, 30, INF)):
+        x[m, k] = v
+    x[68, 31] = -INF
+    w[20, 40], w[30, 41], w[159, 42], w[40, 50] = INF, -INF, NAN, huge
+    x[:, 50] = x[:, 50].sign() * 2.0 ** -20
+    want = (x.double() @ w.double().t())
+    for groups in (1, 2):
+        got = ops.gemm_split(ops.split_rows(x), w, torch.empty(groups, 70, 160, device="cuda"), tile=tile).sum(0)
+        assert torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isneginf(), want.isneginf())
+        size = x.double().abs() @ w.double().abs().t()
+        fine = want.isfinite() & size.isfinite()
+        assert bool(((got.double() - want).abs()[fine] <= 258 * 2.0 ** -24 * size[fine]).all())
+    if tile[1] == 256:
+        gate = ops.gemm_split(ops.split_rows(x), w, torch.empty(70, 80, device="cuda"), gated=True, tile=tile)
+        with_inf = torch.nn.functional.silu(want[:, :80]) * want[:, 80:]
+        assert torch.equal(gate.isnan(), with_inf.isnan()) and torch.equal(gate.isposinf(), with_inf.float().isposinf())
+        assert torch.equal(gate.isneginf(), with_inf.float().isneginf())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [200, 700])
+@pytest.mark.parametrize("K", [256, 2048, 2052, 4096])
+def test_runtime_takes_every_form(M, K, monkeypatch):
+    """linear and gated_linear where the parts are the faster way: bound weights and plain ones, planes, given tensors (also ones whose
+    rows start where the parts' kernel does not store), rows with a stride, widths that have no parts."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.runtime import Runtime
+    seen = []
+    split = ops.gemm_split
+    monkeypatch.setattr(ops, "gemm_split", lambda *a, **k: seen.append(a[1].shape) or split(*a, **k))
+    rt = Runtime(torch.float32, "cuda:0")
+    x, w = operands(M, 2048, K, pad=8)
+    for weight in (rt.weight(w), w):
+        check(rt.linear(x, weight), x, w)
+        got = rt.linear(x, weight, partials=True)
+        check(got.sum(0) if got.dim() == 3 else got, x, w)
+        for room in (4, 3):
+            given = torch.full((M, 2048 + room), NAN, device="cuda")
+            check(rt.linear(x, weight, out=given[:, :2048]), x, w)
+            assert bool(given[:, 2048:].isnan().all())
+    check(rt.gated_linear(x, rt.weight(w, gated=True)), x, w, gated=True)
+    check(rt.gated_linear(x, w), x, w, gated=True)
+    if K == 2052 or (M, K) == (700, 2048):
+        assert bool(seen) == (K == 2048)
+
+
+@pytest.mark.gpu
+def test_refused():
+    from burn_lm_amd.csrc import ops
+    x, w = operands(40, 64, 256)
+    parts, out = ops.split_rows(x), torch.empty(40, 64, device="cuda")
+    for bad in (lambda: ops.split_rows(x[:, :250]), lambda: ops.split_rows(x[:, 1:]), lambda: ops.split_rows(x.bfloat16()),
+                lambda: ops.gemm_split(parts, w[:63], out[:, :63]), lambda: ops.gemm_split(parts[:2], w, out), lambda: ops.gemm_split(parts, w, out, tile=(64, 64)),
+                lambda: ops.gemm_split(parts, w, torch.empty(3, 40, 64, device="cuda")), lambda: ops.gemm_split(parts, w[:, :200].contiguous(), out),
+                lambda: ops.gemm_split(parts, w, out[:, :32], gated=True, tile=(128, 128)), lambda: ops.gemm_split(parts, w.half(), out)):
+        with pytest.raises(ops.KernelError):
+            bad()
+
+
+def test_plan_keeps_its_bounds():
+    """Sizes that the kernel does not have get no plan; groups of K are whole, and none is empty."""
+    from burn_lm_amd.engine.runtime import split_plan
+    for K in (4, 130, 2052):
+        assert split_plan(100, 64, K, 256) is None
+    assert split_plan(100, 60, 256, 256) is None
+    for M in (17, 65, 1000):
+        for N in (16, 2048, 5008):
+            for K in (128, 1152, 2176, 4224, 8192):
+                tile, groups, us = split_plan(M, N, K, 256, planes=True)
+                assert tile in TILES and (groups - 1) * -(-K // 128 // groups) * 128 < K
+                assert split_plan(M, N, K, 256)[1] == 1 and split_plan(M, N, K, 256, gated=True)[0][1] == 256 and us > 0
