@@ -90,9 +90,12 @@ __device__ void af_plain_query(const float* __restrict__ qrow, float* __restrict
 // prompts.  A unit is sixteen queries of one head; a block's four wavefronts take neighbouring units of one key-value head
 // (the heads of its group at the same queries first), and every page that one of them sees is staged once, through registers
 // that hold the next page while this one is worked on.  Rows in shared memory are padded by four floats, so that the sixteen
-// rows of a fragment meet every bank.  The longest units start first.
+// rows of a fragment meet every bank.  The longest units start first, and every second run of 32 places of a key-value head goes from the
+// shortest to the longest: 512 blocks are on the 256 units at once, and a unit's two have 17 pages between them, not 2 to 32.
 // Measured (us a layer, 32 heads of 64 in 8 groups; before: one wavefront per query and head on the vector units):
-// 1,000 tokens 844 -> 96.7, twice what the products take at their rate alone, if the blocks were even.
+// 1,000 tokens 844 -> 96.7; with the places in turns (in calls of their own) 1,000 tokens 104.7 -> 82.8, 2,048 299 -> 209, three sequences of 333 to
+// 1,201 and 24 heads of 128 232 -> 175, 500 tokens (one block a unit) 36.  What is left is a wavefront's pages one behind the other: some
+// 4.5 us each, of which the products are 1.7.
 // ---------------------------------------------------------------------------------------------------------------------
 template <int HD>     // the head's lanes rounded up to 32, 64, 96 or 128
 __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
@@ -105,10 +108,14 @@ __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
   __shared__ __attribute__((aligned(16))) float v_page[HD * VP];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / BLM_WAVE), lane = tid & (BLM_WAVE - 1);
   const int c = lane & 15, g = lane >> 4;
-  const int seq = blockIdx.z, kvh = blockIdx.y, group = nh / nkv;
+  const int seq = blockIdx.z, group = nh / nkv;
   const int row0 = cu_seqlens[seq], n_q = cu_seqlens[seq + 1] - row0;
   const int units = ((n_q + 15) / 16) * group;
-  const int unit0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * AF_WAVES;
+  // consecutive blocks go to different dies: a die sees the pages of few key-value heads
+  const int at = blockIdx.x + gridDim.x * blockIdx.y, kvh = at % nkv;
+  int place = at / nkv;
+  if ((place & 32) && (place | 31) < (int)gridDim.x) place ^= 31;
+  const int unit0 = ((int)gridDim.x - 1 - place) * AF_WAVES;
   if (unit0 >= units) return;
   const int unit = min(unit0 + wave, units - 1);
   const bool active = unit0 + wave < units;

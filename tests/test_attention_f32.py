@@ -69,6 +69,24 @@ def test_prompts(nh, nkv, hd, window):
             check(got[t], qkv[t, : nh * hd].reshape(nh, hd), keys[b], values[b], positions[t], hd ** -0.5, window, nh // nkv)
 
 
+@pytest.mark.parametrize("lens,nh,nkv", [([600], 8, 1), ([520, 30, 1100], 12, 3), ([1040], 4, 4)])
+def test_prompts_of_many_places(lens, nh, nkv):
+    """More than 32 blocks a key-value head: whole runs of 32 that go the other way round, and runs that are cut short."""
+    from burn_lm_amd.csrc import ops
+    hd, group = 16, nh // nkv
+    table, keys, values, kc, vc = case(lens, nkv, hd, 5)
+    cu = [sum(lens[:b]) for b in range(len(lens) + 1)]
+    qkv = torch.randn(cu[-1], (nh + 2 * nkv) * hd, generator=torch.Generator().manual_seed(6))
+    out = torch.full((cu[-1], nh * hd), 7.0, device="cuda")
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    ops.attn_prefill_f32(qkv.cuda(), qkv.shape[1], out, i32([p for n in lens for p in range(n)]), i32(cu), table.cuda(), kc.cuda(), vc.cuda(), PAGE,
+                         len(lens), max(lens), nh, nkv, hd, hd ** -0.5, 0)
+    got = out.cpu().reshape(-1, nh, hd)
+    for b, n in enumerate(lens):
+        for t in list(range(0, n, 61)) + [n - 1]:
+            check(got[cu[b] + t], qkv[cu[b] + t, : nh * hd].reshape(nh, hd), keys[b], values[b], t, hd ** -0.5, 0, group)
+
+
 @pytest.mark.parametrize("splits", [1, 2, 5])
 @pytest.mark.parametrize("window", [0, 1, 70])
 @pytest.mark.parametrize("nh,nkv,hd", SHAPES)
