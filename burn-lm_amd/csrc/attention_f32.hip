@@ -26,6 +26,14 @@ __device__ __forceinline__ bool af_visible(int key, int pos, int window) { retur
 template <int V>
 using AfInt = std::integral_constant<int, V>;
 
+// e^x of x <= 0 (and -infinity; NaN stays NaN): x log2(e) in two floats, the hardware's power of two of the first and the second's share of the
+// result as its derivative.  Within 2 ulps like expf, in 7 instructions instead of 13; what is below 2^-126 is zero.
+__device__ __forceinline__ float af_exp(float x) {
+  x = blm_max(x, -200.f);
+  const float h = x * 1.44269502f, l = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -h)), p = __builtin_amdgcn_exp2f(h);
+  return fmaf(p, l * 0.693147182f, p);
+}
+
 // Running softmax of one page: s[t][v] holds the scaled scores of this lane's query (l % 16) with keys 16 t + 4 (l / 16) + v,
 // -infinity where the query does not see the key; they become probabilities against the new maximum.  l is this lane's part
 // of the sum.  Returns the factor for what was summed before.
@@ -38,13 +46,13 @@ __device__ __forceinline__ float af_softmax(f32x4* s, float& m, float& l) {
     for (int v = 0; v < 4; ++v) top = fmaxf(top, s[t][v]);
   const float m_new = fmaxf(m, rows_max(top));
   const float base = m_new == -INFINITY ? 0.f : m_new;       // nothing seen yet: every probability is exp(-inf)
-  const float keep = expf(m - base);
+  const float keep = af_exp(m - base);
   float sum = 0.f;
 #pragma unroll
   for (int t = 0; t < TILES; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      s[t][v] = expf(s[t][v] - base);
+      s[t][v] = af_exp(s[t][v] - base);
       sum += s[t][v];
     }
   l = l * keep + sum;
@@ -94,10 +102,12 @@ __device__ void af_plain_query(const float* __restrict__ qrow, float* __restrict
 // shortest to the longest: 512 blocks are on the 256 units at once, and a unit's two have 17 pages between them, not 2 to 32.
 // Measured (us a layer, 32 heads of 64 in 8 groups; before: one wavefront per query and head on the vector units):
 // 1,000 tokens 844 -> 96.7; with the places in turns (in calls of their own) 1,000 tokens 104.7 -> 82.8, 2,048 299 -> 209, three sequences of 333 to
-// 1,201 and 24 heads of 128 232 -> 175, 500 tokens (one block a unit) 36.  What is left is a wavefront's pages one behind the other: some
-// 4.5 us each, of which the products are 1.7.
+// 1,201 and 24 heads of 128 232 -> 175, 500 tokens (one block a unit) 36.  A wavefront's pages then took 4.5 us each, of which the products are
+// 1.7; without a branch for every masked score and every staged piece, and with af_exp: 1,000 tokens 67.7, 2,048 165, the three sequences
+// 155, 500 tokens 27.2, 16 of 300 91 (104).  Two wavefronts for a unit, one on every other page: 83 -> 90, 500 tokens 35 -> 37.6, but 24 heads
+// of 128 121 -> 92.
 // ---------------------------------------------------------------------------------------------------------------------
-template <int HD>     // the head's lanes rounded up to 32, 64, 96 or 128
+template <int HD, bool FULL>     // HD: the head's lanes rounded up to 32, 64, 96 or 128; FULL: it has all of them
 __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
     attn_prefill_f32_kernel(const float* __restrict__ q, int q_row_stride, float* __restrict__ out,
                             const int* __restrict__ positions, const int* __restrict__ cu_seqlens,
@@ -135,7 +145,7 @@ __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
   f32x4 qf[DS];
 #pragma unroll
   for (int i = 0; i < DS; ++i) qf[i] = i * 16 + g * 4 < hd ? af_load(qrow + i * 16 + g * 4) : zero;
-  if (hd < HD)   // the lanes that the head does not have count as zeros
+  if (!FULL)     // the lanes that the head does not have count as zeros
     for (int i = tid; i < AF_PAGE * (HD - hd); i += AF_WAVES * BLM_WAVE) k_page[i / (HD - hd) * KP + hd + i % (HD - hd)] = 0.f;
 
   // a thread's pieces of a page: piece x of the page's hd * 16 pieces of four floats, keys and values alike
@@ -145,23 +155,26 @@ __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
     const size_t base = ((size_t)pages[page] * nkv + kvh) * AF_PAGE * hd;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int x = min(tid + i * AF_WAVES * BLM_WAVE, pieces - 1) * 4;
+      const int x = (FULL ? tid + i * AF_WAVES * BLM_WAVE : min(tid + i * AF_WAVES * BLM_WAVE, pieces - 1)) * 4;
       ks[i] = af_load(kcache + base + x);
       vs[i] = af_load(vcache + base + x);
     }
   };
   auto put = [&](int page) {
+    // what lies behind the last key of the block was never written by this sequence: zeros, lest it be no number
+    if (page * AF_PAGE + AF_PAGE - 1 > block_hi) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vs[i][e] = page * AF_PAGE + (tid + i * AF_WAVES * BLM_WAVE) % 16 * 4 + e <= block_hi ? vs[i][e] : 0.f;
+    }
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int x = tid + i * AF_WAVES * BLM_WAVE;
-      if (hd == HD || x < pieces) {
-        const int kr = hd == HD ? x / (HD / 4) : x / per_row, kx = (x - kr * (hd == HD ? HD / 4 : per_row)) * 4, vr = x / 16, vx = x % 16 * 4;
+      if (FULL || x < pieces) {
+        const int kr = FULL ? x / (HD / 4) : x / per_row, kx = (x - kr * (FULL ? HD / 4 : per_row)) * 4, vr = x / 16, vx = x % 16 * 4;
         *reinterpret_cast<f32x4*>(&k_page[kr * KP + kx]) = ks[i];
-        // what lies behind the last key of the block was never written by this sequence: zeros, lest it be no number
-        f32x4 v = vs[i];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = page * AF_PAGE + vx + e <= block_hi ? v[e] : 0.f;
-        *reinterpret_cast<f32x4*>(&v_page[vr * VP + vx]) = v;
+        *reinterpret_cast<f32x4*>(&v_page[vr * VP + vx]) = vs[i];
       }
     }
   };
@@ -191,9 +204,17 @@ __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
     const int key0 = page * AF_PAGE + g * 4;
     const bool whole = page * AF_PAGE + AF_PAGE - 1 <= wave_lo && (window <= 0 || wave_hi - page * AF_PAGE < window);
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < 4; ++t) s[t] *= scale;
+    if (!whole) {        // a branch for all of them: one for each took as long as the softmax
+      const int from = window > 0 ? pos - window : -1;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) s[t][v] = whole || af_visible(key0 + t * 16 + v, pos, window) ? s[t][v] * scale : -INFINITY;
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int key = key0 + t * 16 + v;
+          s[t][v] = (key <= pos) & (key > from) ? s[t][v] : -INFINITY;
+        }
+    }
     const float keep = af_softmax(s, m, l);
 #pragma unroll
     for (int d = 0; d < DS; ++d) o[d] *= keep;
@@ -435,13 +456,17 @@ extern "C" int blm_attn_prefill_f32(const void* q, int q_row_stride, void* out, 
   const long long blocks = ((long long)(max_new + 15) / 16 * (nh / nkv) + AF_WAVES - 1) / AF_WAVES;
   BLM_REQUIRE(n_seqs > 0 && n_seqs <= 65535 && max_new > 0 && nkv <= 65535 && blocks < 2147483647LL, "attn_prefill_f32: bad sizes");
   dim3 grid((unsigned)blocks, (unsigned)nkv, (unsigned)n_seqs), block(AF_WAVES * BLM_WAVE);
-#define BLM_AFP(HD)                                                                                                       \
-  hipLaunchKernelGGL((attn_prefill_f32_kernel<HD>), grid, block, 0, stream, (const float*)q, q_row_stride, (float*)out, positions, \
+#define BLM_AFP(HD, FULL)                                                                                                             \
+  hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, FULL>), grid, block, 0, stream, (const float*)q, q_row_stride, (float*)out, positions, \
                      cu_seqlens, block_table, table_width, (const float*)kcache, (const float*)vcache, nh, nkv, hd, scale, window)
-  if (hd <= 32) BLM_AFP(32);
-  else if (hd <= 64) BLM_AFP(64);
-  else if (hd <= 96) BLM_AFP(96);
-  else BLM_AFP(128);
+  if (hd == 32) BLM_AFP(32, true);
+  else if (hd < 32) BLM_AFP(32, false);
+  else if (hd == 64) BLM_AFP(64, true);
+  else if (hd < 64) BLM_AFP(64, false);
+  else if (hd == 96) BLM_AFP(96, true);
+  else if (hd < 96) BLM_AFP(96, false);
+  else if (hd == 128) BLM_AFP(128, true);
+  else BLM_AFP(128, false);
 #undef BLM_AFP
   BLM_LAUNCH_CHECK("attn_prefill_f32");
   return 0;
