@@ -12,9 +12,11 @@
 // 3.7e-6 from 64 bits, with the float instructions 2.8e-6).  So a chunk of 128 of K has an accumulator that starts at zero, small products
 // first, and joins the total by a rounded addition; and every other chunk is summed with its columns negated and subtracted, so that what is
 // cut cancels: 1.7e-7 off (2.17e-7 with the float instructions), 7e-11 too low, and the logits 2.6e-6.
-// Measured (us, the float instructions' best tile before, 1,000 rows): [16384, 2048] gated 493 -> 281 (239 TFLOP/s of float products),
-// [2048, 8192] in four groups 272 -> 148, [3072, 2048] 110 -> 75, [2048, 2048] 78 -> 43; the parts' pass 7 and (K = 8,192) 14.  The scoring of
-// 1,000 tokens at the 1B shape 16.95 -> 11.5 ms.
+// Measured (us, the float instructions' best tile and groups / this, without the parts' pass of 3.5 to 5 us, with K = 8,192 14; weights from memory),
+// 1,000 rows: [16384, 2048] gated 502 / 284 (236 TFLOP/s of float products), [2048, 8192] 259 / 157, [3072, 2048] 105 / 75, [2048, 2048] 72 / 47;
+// 256 rows 137 / 90, 74 / 50, 33 / 26, 24 / 18.  Scoring 1,000 tokens at the 1B shape 16.93 -> 10.65 ms.
+// The ring is as deep as the weights' way from memory asks: with the next two stages under way tiles of 64 rows, whose stages are short, took 1.34 us
+// a stage for the 64 x 128, with three 0.70 (1.2 and 1.13 for 64 x 256; four and five: as three).
 // Tried: columns from global memory straight into registers (120 -> 133 us on 64 blocks), tiles of 256 x 256 (two stages fill the
 // shared memory: 334 against 312), two accumulators for small and large products without the rounded additions (5 % faster, 2.7e-7 off),
 // the small products' sums added in every step (1.06e-7 off, registers spill).
@@ -124,23 +126,23 @@ template <int V>
 using GsInt = std::integral_constant<int, V>;
 
 // MT x 16 rows by 8 x NT x 16 columns, eight wavefronts beside each other: each has all rows and 16 NT columns.  Stages of 32 of K: a ring of
-// three of the rows' parts and one of two of each wavefront's own columns.  One barrier a stage, in its middle: behind it the next
-// stage's operands are there, the one after that is asked for, and the next columns are split beside the second half's products.
+// RING of the rows' parts and one of RING - 1 of each wavefront's own columns.  One barrier a stage, in its middle: behind it the next
+// stage's operands are there, the last one of the ring is asked for, and the next columns are split beside the second half's products.
 // lane l of a product: row l % 16, columns 4 (l / 16) + 0..3.  W rows past the end are the last one again; nothing stores what comes of them.
-template <int MT, int NT, bool GATED>
-__global__ void __launch_bounds__(512, MT * NT <= 4 ? 4 : 2)
+template <int MT, int NT, int RING, bool GATED>
+__global__ void __launch_bounds__(512, 2)
     gemm_split_kernel(const unsigned char* __restrict__ P, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K, int ldc,
-                      int steps_per_group, long long plane, int m_tiles, int n_tiles) {
+                      int steps_per_group, long long plane, int m_tiles) {
   static_assert(!GATED || NT == 2, "a gated wavefront has a tile of gate columns and their up columns");
-  constexpr int A_LOADS = (3 * MT + 7) / 8, B_LOADS = 2 * NT;
+  constexpr int A_LOADS = (3 * MT + 7) / 8, B_LOADS = 2 * NT, LOADS = A_LOADS + B_LOADS;
   constexpr int A_STAGE = MT * 3 * GS_FRAGMENT, B_STAGE = 8 * NT * 2048;
   constexpr int COLUMNS = GATED ? 128 : 128 * NT;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[3 * A_STAGE + 2 * B_STAGE];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[RING * A_STAGE + (RING - 1) * B_STAGE];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / BLM_WAVE), lane = tid & (BLM_WAVE - 1);
   const int l16 = lane & 15, quad = lane >> 4;
-  const int die = blockIdx.x & 7, at = blockIdx.x >> 3;
-  const int nt = (at / m_tiles) * 8 + die, mt = at % m_tiles;
-  if (nt >= n_tiles) return;
+  // neighbouring blocks go to different dies: each die gets a run of the tiles, all rows of a column tile before the next one's
+  const int tiles = gridDim.x, die = blockIdx.x & 7, at = die * (tiles >> 3) + min(die, tiles & 7) + (blockIdx.x >> 3);
+  const int nt = at / m_tiles, mt = at - nt * m_tiles;
   const int m0 = mt * MT * 16, n0 = nt * COLUMNS, steps_all = K / GS_BK;
   const int s_begin = blockIdx.y * steps_per_group, stages = min(steps_per_group, steps_all - s_begin), last = stages - 1;
 
@@ -162,7 +164,7 @@ __global__ void __launch_bounds__(512, MT * NT <= 4 ? 4 : 2)
     b_off[x] = ((uint32_t)n + (GATED && j ? (uint32_t)N : 0u)) * (uint32_t)K * 4u + piece * 16u;
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(blm_lds_ptr)lds;
-  const uint32_t b_to = lds0 + 3 * A_STAGE + (uint32_t)wave * (NT * 2048);
+  const uint32_t b_to = lds0 + RING * A_STAGE + (uint32_t)wave * (NT * 2048);
   auto fetch = [&](int s, int a_slot, int b_slot) {
     const char *a = a_base + (size_t)s * (3 * GS_FRAGMENT), *b = b_base + (size_t)s * (GS_BK * 4);
 #pragma unroll
@@ -171,7 +173,7 @@ __global__ void __launch_bounds__(512, MT * NT <= 4 ? 4 : 2)
     for (int x = 0; x < A_LOADS; ++x) blm_dma16_to(a, a_off[x], lds0 + (uint32_t)(a_slot * A_STAGE) + a_to[x]);
   };
 
-  const int b_at = 3 * A_STAGE + wave * (NT * 2048) + l16 * 128;
+  const int b_at = RING * A_STAGE + wave * (NT * 2048) + l16 * 128;
   const int slot0 = (quad ^ ((l16 >> 1) & 7)) * 16, slot1 = ((4 + quad) ^ ((l16 >> 1) & 7)) * 16;
   gs_f32x4 raw[NT][2];
   gs_u32x4 b[2][NT][3];
@@ -217,20 +219,22 @@ __global__ void __launch_bounds__(512, MT * NT <= 4 ? 4 : 2)
         t[g * TOGETHER + x][j] = gs_f32x4{0.f, 0.f, 0.f, 0.f};
       }
   };
+  int a_slot = 0, b_slot = 1;                   // of this stage's rows and of the next one's columns
   // a stage; on entry its first rows' fragments and its columns' parts are in registers
-  auto stage = [&](int s, int slot, auto place_type, auto negative) {
+  auto stage = [&](int s, auto place_type, auto negative) {
     constexpr int place = decltype(place_type)::value, now = place & 1, next = now ^ 1;
     using NextNegative = std::integral_constant<bool, decltype(negative)::value != (place == 3)>;
-    const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot == 0 ? 2 : slot - 1;
+    const int slot = a_slot, slot1 = slot == RING - 1 ? 0 : slot + 1;
 #pragma unroll
     for (int g = 0; g < GROUPS; ++g) {
       const int set = g & 1;
       read_a(set ^ 1, g + 1 < GROUPS ? slot : slot1, g + 1 < GROUPS ? g + 1 : 0);
       if (g == HALF) {
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (s + 2 <= last) fetch(s + 2, slot2, now);
+        if (RING > 3 && s + RING - 2 <= last) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RING - 3) * LOADS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + RING - 1 <= last) fetch(s + RING - 1, slot == 0 ? RING - 1 : slot - 1, b_slot == 0 ? RING - 2 : b_slot - 1);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) read_raw(next, j);
+        for (int j = 0; j < NT; ++j) read_raw(b_slot, j);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -248,12 +252,15 @@ __global__ void __launch_bounds__(512, MT * NT <= 4 ? 4 : 2)
         if (g - HALF == y * (GROUPS - HALF) / (2 * NT)) split_half(b[next], y >> 1, y & 1, NextNegative{});
     }
     if (place == 3) add(GROUPS - 1, negative);
-    return slot1;
+    a_slot = slot1;
+    b_slot = b_slot == RING - 2 ? 0 : b_slot + 1;
   };
   static_assert(GROUPS % 2 == 0, "the first rows' fragments of every stage lie in the same set");
-  fetch(0, 0, 0);
-  fetch(1, 1, 1);
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(A_LOADS + B_LOADS) : "memory");
+#pragma unroll
+  for (int s = 0; s < RING - 1; ++s)
+    if (s <= last) fetch(s, s, s);
+  if (RING - 2 <= last) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RING - 2) * LOADS) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     read_raw(0, j);
@@ -261,12 +268,11 @@ __global__ void __launch_bounds__(512, MT * NT <= 4 ? 4 : 2)
     split_half(b[0], j, 1, std::false_type{});
   }
   read_a(0, 0, 0);
-  int slot = 0;
   auto chunk = [&](int s, auto negative) {
-    slot = stage(s, slot, GsInt<0>{}, negative);
-    slot = stage(s + 1, slot, GsInt<1>{}, negative);
-    slot = stage(s + 2, slot, GsInt<2>{}, negative);
-    slot = stage(s + 3, slot, GsInt<3>{}, negative);
+    stage(s, GsInt<0>{}, negative);
+    stage(s + 1, GsInt<1>{}, negative);
+    stage(s + 2, GsInt<2>{}, negative);
+    stage(s + 3, GsInt<3>{}, negative);
   };
   for (int s = 0; s < stages; s += 8) {
     chunk(s, std::false_type{});
@@ -313,21 +319,21 @@ extern "C" int blm_gemm_split(const void* P, const void* W, void* C, int M, int 
   BLM_REQUIRE((rows == 128 || rows == 64) && (columns == 256 || (columns == 128 && !gated)), "gemm_split: tile %d x %d", rows, columns);
   const int per = gated ? columns / 2 : columns;
   const int m_tiles = (M + rows - 1) / rows, n_tiles = (N + per - 1) / per;
-  const long long blocks = (long long)m_tiles * ((n_tiles + 7) / 8 * 8);
+  const long long blocks = (long long)m_tiles * n_tiles;
   BLM_REQUIRE(blocks < 2147483647LL, "gemm_split: too many tiles");
   dim3 grid((unsigned)blocks, (unsigned)groups), block(512);
-#define GS_RUN(MT, NT, G)                                                                                                             \
-  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, G>), grid, block, 0, stream, (const unsigned char*)P, (const float*)W, (float*)C, M, N, \
-                     K, ldc, steps, (long long)M * N, m_tiles, n_tiles)
+#define GS_RUN(MT, NT, RING, G)                                                                                                             \
+  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, RING, G>), grid, block, 0, stream, (const unsigned char*)P, (const float*)W, (float*)C, M, N, \
+                     K, ldc, steps, (long long)M * N, m_tiles)
   if (gated) {
-    if (rows == 128) GS_RUN(8, 2, true);
-    else GS_RUN(4, 2, true);
+    if (rows == 128) GS_RUN(8, 2, 3, true);
+    else GS_RUN(4, 2, 4, true);
   } else if (columns == 256) {
-    if (rows == 128) GS_RUN(8, 2, false);
-    else GS_RUN(4, 2, false);
+    if (rows == 128) GS_RUN(8, 2, 3, false);
+    else GS_RUN(4, 2, 4, false);
   } else {
-    if (rows == 128) GS_RUN(8, 1, false);
-    else GS_RUN(4, 1, false);
+    if (rows == 128) GS_RUN(8, 1, 3, false);
+    else GS_RUN(4, 1, 4, false);
   }
 #undef GS_RUN
   BLM_LAUNCH_CHECK("gemm_split");

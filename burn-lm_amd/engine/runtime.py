@@ -5,7 +5,8 @@ Matrix products ``x[M,K] @ w[N,K]^T``:
   reduced-precision matrix mode), whatever the activation dtype.  This is the whole float32 path
   and also what keeps a tensor that a checkpoint stores in 32 bits exact in a bfloat16 run.  With float32
   activations whose rows lie in units of 16 bytes: up to 16 rows ops.gemv_f32 on a packed copy, more rows (from 9
-  on where there is no such copy) ops.gemm_f32 (f32_plan chooses its tile and groups of K) or, from 100 to 400 rows on,
+  on where there is no such copy) ops.gemm_f32 (f32_plan chooses its tile and groups of K) or, from
+  some 20 to 200 rows on,
   ops.gemm_split (the same products by three exact bfloat16 parts of each float; split_plan); everything else
   ops.gemv_skinny up to 8 rows and ops.gemm_tiled.
 * bfloat16 weights, up to 64 rows (decode): the hand-written skinny kernel on the matrix cores that
@@ -95,36 +96,43 @@ F32_SKINNY_MAX_ROWS = 16
 F32_SKINNY_GROUP_K = 2048
 
 
+def _planes_us(M, N, groups, planes):
+    """What partial planes cost their reader: their bytes, and where that is a pass of its own its launch and its result's bytes."""
+    return M * N * groups * 4 / 5e6 if planes else 3.0 + M * N * (groups + 1) * 4 / 5e6
+
+
 @functools.lru_cache(maxsize=4096)      # a length asks for some ten; made anew at every product, each took 2 to 12 us of the host
-def f32_plan(M, N, K, compute_units, planes=False, gated=False):
+def f32_plan(M, N, K, compute_units, planes=False, gated=False, added=False):
     """(tile, groups of K, microseconds) of ops.gemm_f32 that a sum of its parts' costs finds fastest: every unit works through
-    its share of the blocks, and every plane of partial products is read once by the norm that adds it.
+    its share of the blocks, and every plane of partial products is read once by the norm that adds it (planes) or by a pass that does
+    (added: for results that have to be whole; few rows of few columns are a handful of blocks that each walk all of K otherwise).
     Against the best tile and groups of the sweep the choice is within 6 % from 250 rows on and within 20 % below."""
     best = None
     for (bm, bn), (alone, shared) in F32_STEP_US.items():
         if gated and bn != 128:
             continue
         tiles = -(-M // bm) * -(-N // (bn // 2 if gated else bn))
-        for groups in (1, 2, 4, 8) if planes and not gated else (1,):
+        for groups in (1, 2, 4, 8) if (planes or added) and not gated else (1,):
             if groups > 1 and K // groups < 128:
                 continue
             steps = -(-K // groups // 32)
             per_unit = -(-tiles * groups // compute_units)
-            us = 3.0 + steps * max(alone, per_unit * shared + F32_SHARE_US) + (M * N * groups * 4 / 5e6 if groups > 1 else 0.0)
+            us = 3.0 + steps * max(alone, per_unit * shared + F32_SHARE_US) + (_planes_us(M, N, groups, planes) if groups > 1 else 0.0)
             if best is None or us < best[2] * 0.999:
                 best = ((bm, bn), groups, us)
     return best
 
 
 # Tiles of ops.gemm_split: microseconds for a step of 32 along K of a block while few units are busy, and while all are (the card's
-# power).  Two blocks of the smallest share a unit.  Measured with 17 to 4,000 rows at [16384, 2048] gated, [2048, 8192] in 1 to 8
-# groups, [3072, 2048], [2048, 2048].
-SPLIT_STEP_US = {(128, 256): (1.78, 2.22), (128, 128): (1.0, 1.3), (64, 256): (1.04, 1.32), (64, 128): (0.66, 0.74)}
-SPLIT_PAIR_US = 0.66
+# power), and a block's first loads and last stores.  Measured on weights that come from memory (ten matrices in turn), 24 to 1,500 rows, [16384, 2048] gated and not, [2048,
+# 8192], [3072, 2048], [2048, 2048], [5120, 3072], [3072, 8192] in 1 to 8 groups.  The choice between both kernels' tiles and groups is within
+# 2 % of the fastest in the mean and never more than 5 % behind what gemm_f32 alone would take.
+SPLIT_STEP_US = {(128, 256): (1.71, 2.3), (128, 128): (0.95, 1.29), (64, 256): (1.07, 1.44), (64, 128): (0.63, 0.82)}
+SPLIT_BLOCK_US = 2.5
 
 
 @functools.lru_cache(maxsize=4096)
-def split_plan(M, N, K, compute_units, planes=False, gated=False):
+def split_plan(M, N, K, compute_units, planes=False, gated=False, added=False):
     """(tile, groups of K, microseconds with the pass that makes the rows' parts) of ops.gemm_split, as f32_plan has them of
     ops.gemm_f32; None where it does not have the sizes."""
     if not ops.split_takes(M, N, K, gated):
@@ -134,19 +142,16 @@ def split_plan(M, N, K, compute_units, planes=False, gated=False):
         if gated and bn != 256:
             continue
         tiles = -(-M // bm) * -(-N // (bn // 2 if gated else bn))
-        for groups in (1, 2, 4, 8) if planes and not gated else (1,):
+        for groups in (1, 2, 4, 8) if (planes or added) and not gated else (1,):
             steps = -(-K // 128 // groups) * 4
             if groups > 1 and (K // groups < 256 or (groups - 1) * steps * 32 >= K):
                 continue
             per_unit = -(-tiles * groups // compute_units)
             fill = tiles * groups / (per_unit * compute_units)
-            step = few + (all_ - few) * fill
-            if (bm, bn) == (64, 128) and per_unit > 1:
-                step = SPLIT_PAIR_US
-            us = 3.0 + steps * per_unit * step + (M * N * groups * 4 / 5e6 if groups > 1 else 0.0)
+            us = 2.0 + per_unit * (SPLIT_BLOCK_US + steps * (few + (all_ - few) * fill)) + (_planes_us(M, N, groups, planes) if groups > 1 else 0.0)
             if best is None or us < best[2] * 0.999:
                 best = ((bm, bn), groups, us)
-    return best[0], best[1], best[2] + max(7.0, M * K * 10 / 6e6)
+    return best[0], best[1], best[2] + max(3.4, 2.3 + M * K * 10 / 7e6)
 
 
 # ops.gemm_duo: what half a tile takes of a whole one's time (K = 2048 / 8192, all blocks at once: 22 of 38 us, 73 of 128), and how
@@ -385,18 +390,20 @@ class Runtime:
                     return ops.sum_planes(parts, out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device))
         if M <= SKINNY_MAX_ROWS:
             return None
-        tile, groups, us = f32_plan(M, N, K, self.compute_units, planes)
-        split = split_plan(M, N, K, self.compute_units, planes)
-        if split is not None and split[2] < us and (out is None or (out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0)):
+        added = not planes and (out is None or (out.is_contiguous() and out.data_ptr() % 16 == 0))
+        tile, groups, us = f32_plan(M, N, K, self.compute_units, planes, added=added)
+        split = split_plan(M, N, K, self.compute_units, planes, added=added)
+        by_parts = split is not None and split[2] < us and (out is None or (out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0))
+        if by_parts:
             tile, groups, _ = split
-            if groups > 1:
-                out = torch.empty(groups, M, N, dtype=torch.float32, device=x.device)
-            elif out is None:
-                out = torch.empty(M, N, dtype=torch.float32, device=x.device)
-            return ops.gemm_split(ops.split_rows(x), w, out, tile=tile)
-        if groups > 1:
-            return ops.gemm_f32(x, w, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), tile=tile)
-        return ops.gemm_f32(x, w, out if out is not None else torch.empty(M, N, dtype=torch.float32, device=x.device), tile=tile)
+        if out is None:
+            out = torch.empty(M, N, dtype=torch.float32, device=x.device) if groups == 1 or added else None
+        into = out if groups == 1 else torch.empty(groups, M, N, dtype=torch.float32, device=x.device)
+        if by_parts:
+            ops.gemm_split(ops.split_rows(x), w, into, tile=tile)
+        else:
+            ops.gemm_f32(x, w, into, tile=tile)
+        return ops.sum_planes(into, out) if groups > 1 and added else into
 
     def rows_plan(self, N, K):
         """(groups of K, columns per block) for a product of 17 to 64 rows that may come as partial planes."""
@@ -812,11 +819,14 @@ class Runtime:
             else:
                 tile, _, fused = f32_plan(M, inner, K, self.compute_units, gated=True)
                 split = split_plan(M, inner, K, self.compute_units, gated=True)
-                if split is not None and split[2] < fused:
-                    return ops.gemm_split(ops.split_rows(x), plain, torch.empty(M, inner, dtype=torch.float32, device=x.device), gated=True, tile=split[0])
+                by_parts = split is not None and split[2] < fused
                 # few rows: the plain product's smaller tiles and the pass behind it (12 bytes an element)
-                if fused <= f32_plan(M, 2 * inner, K, self.compute_units)[2] + 3.0 + M * inner * 12 / 5e6:
-                    return ops.gemm_f32(x, plain, torch.empty(M, inner, dtype=torch.float32, device=x.device), gated=True, tile=tile)
+                apart = [plan(M, 2 * inner, K, self.compute_units, added=True) for plan in (f32_plan, split_plan)]
+                if min(fused, split[2] if by_parts else fused) <= min(p[2] for p in apart if p is not None) + 3.0 + M * inner * 12 / 5e6:
+                    out = torch.empty(M, inner, dtype=torch.float32, device=x.device)
+                    if by_parts:
+                        return ops.gemm_split(ops.split_rows(x), plain, out, gated=True, tile=split[0])
+                    return ops.gemm_f32(x, plain, out, gated=True, tile=tile)
         silu = activation == "silu"      # the row-ring kernel gates with silu only; the others take the activation
         fusable = (x.dtype == plain.dtype == self.dtype == torch.bfloat16 and K % 8 == 0 and x.stride(1) == 1
                    and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and plain.is_contiguous())
