@@ -6,9 +6,8 @@ Matrix products ``x[M,K] @ w[N,K]^T``:
   and also what keeps a tensor that a checkpoint stores in 32 bits exact in a bfloat16 run.  With float32
   activations whose rows lie in units of 16 bytes: up to 16 rows ops.gemv_f32 on a packed copy, more rows (from 9
   on where there is no such copy) ops.gemm_f32 (f32_plan chooses its tile and groups of K) or, from
-  some 20 to 200 rows on,
-  ops.gemm_split (the same products by three exact bfloat16 parts of each float; split_plan); everything else
-  ops.gemv_skinny up to 8 rows and ops.gemm_tiled.
+  some 20 to 200 rows on, ops.gemm_split (the same products by three exact bfloat16 parts of each float; split_plan);
+  everything else ops.gemv_skinny up to 8 rows and ops.gemm_tiled.
 * bfloat16 weights, up to 64 rows (decode): the hand-written skinny kernel on the matrix cores that
   streams the weight once (where the width fits its registers: see ops.gemv_mfma_group_limit).  From
   17 rows on, the products that come as partial planes (output and down projection) and, from 33 rows
@@ -124,9 +123,10 @@ def f32_plan(M, N, K, compute_units, planes=False, gated=False, added=False):
 
 
 # Tiles of ops.gemm_split: microseconds for a step of 32 along K of a block while few units are busy, and while all are (the card's
-# power), and a block's first loads and last stores.  Measured on weights that come from memory (ten matrices in turn), 24 to 1,500 rows, [16384, 2048] gated and not, [2048,
-# 8192], [3072, 2048], [2048, 2048], [5120, 3072], [3072, 8192] in 1 to 8 groups.  The choice between both kernels' tiles and groups is within
-# 2 % of the fastest in the mean and never more than 5 % behind what gemm_f32 alone would take.
+# power), and a block's first loads and last stores.  Measured on weights that come from memory (ten matrices in turn), 24 to 1,500
+# rows, [16384, 2048] gated and not, [2048, 8192], [3072, 2048], [2048, 2048], [5120, 3072], [3072, 8192] in 1 to 8 groups.  The
+# choice between both kernels' tiles and groups is within 2 % of the fastest in the mean and never more than 7 % behind what gemm_f32
+# alone would take.
 SPLIT_STEP_US = {(128, 256): (1.71, 2.3), (128, 128): (0.95, 1.29), (64, 256): (1.07, 1.44), (64, 128): (0.63, 0.82)}
 SPLIT_BLOCK_US = 2.5
 

@@ -129,6 +129,30 @@ def test_runtime_takes_every_form(M, K, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [17, 40, 100])
+@pytest.mark.parametrize("N,K", [(3072, 2048), (330, 2052), (528, 1152)])
+def test_whole_results_of_planes(M, N, K, monkeypatch):
+    """Few rows of few columns that have to come whole run in groups of K whose planes a pass adds: new tensors and given ones; where
+    rows do not lie one behind the other the product writes them itself."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.runtime import Runtime
+    added = []
+    planes = ops.sum_planes
+    monkeypatch.setattr(ops, "sum_planes", lambda y, out: added.append(y.shape[0]) or planes(y, out))
+    rt = Runtime(torch.float32, "cuda:0")
+    x, w = operands(M, N, K, pad=4)
+    whole = rt.linear(x, w)
+    assert whole.shape == (M, N) and added
+    check(whole, x, w)
+    given = torch.full((M, N), NAN, device="cuda")
+    assert rt.linear(x, w, out=given) is given and torch.equal(given, whole)
+    added.clear()
+    wide = torch.full((M, N + 4), NAN, device="cuda")
+    check(rt.linear(x, w, out=wide[:, :N]), x, w)
+    assert not added and bool(wide[:, N:].isnan().all())
+
+
+@pytest.mark.gpu
 def test_refused():
     from burn_lm_amd.csrc import ops
     x, w = operands(40, 64, 256)
@@ -151,5 +175,7 @@ def test_plan_keeps_its_bounds():
         for N in (16, 2048, 5008):
             for K in (128, 1152, 2176, 4224, 8192):
                 tile, groups, us = split_plan(M, N, K, 256, planes=True)
+                assert tile in TILES and (groups - 1) * -(-K // 128 // groups) * 128 < K
+                tile, groups, _ = split_plan(M, N, K, 256, added=True)
                 assert tile in TILES and (groups - 1) * -(-K // 128 // groups) * 128 < K
                 assert split_plan(M, N, K, 256)[1] == 1 and split_plan(M, N, K, 256, gated=True)[0][1] == 256 and us > 0
