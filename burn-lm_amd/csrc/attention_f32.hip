@@ -12,6 +12,7 @@
 //                      halves or quarters
 #include <type_traits>
 
+#include "attn_merge.h"
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -386,31 +387,23 @@ __global__ void __launch_bounds__(AF_DECODE_WAVES* BLM_WAVE)
   }
   __syncthreads();
   const size_t item0 = (size_t)token * nh + head0;
-  // a thread's elements of the block's result: the wavefronts' parts against their common maximum
-  for (int i = tid; i < heads * hd; i += AF_DECODE_WAVES * BLM_WAVE) {
-    const int h = i / hd, d = i - h * hd;
-    float top = all_m[0][h];
-#pragma unroll
-    for (int w = 1; w < AF_DECODE_WAVES; ++w) top = fmaxf(top, all_m[w][h]);
-    const float base = top == -INFINITY ? 0.f : top;
-    float sum = 0.f, weight = 0.f;
-#pragma unroll
-    for (int w = 0; w < AF_DECODE_WAVES; ++w) {
-      const float f = expf(all_m[w][h] - base);
-      sum += f * all_o[w][h][d];
-      weight += f * all_l[w][h];
-    }
+  const auto ex = [](float v) { return expf(v); };
+  const auto put = [&](int h, int d, float4 v) {
+    float* p = orow + h * hd + d;
+    p[0] = v.x;
+    p[1] = v.y;
+    p[2] = v.z;
+    p[3] = v.w;
+  };
+  ag_block<AF_DECODE_WAVES * BLM_WAVE, AF_DECODE_WAVES>(&all_m[0][0], &all_l[0][0], &all_o[0][0][0], 16 * (HD + 4), HD + 4, heads, hd, ex,
+                                                        [&](int h, int d, const AgSum& a) {
     if (n_splits == 1) {
-      orow[i] = sum * (1.0f / weight);
+      put(h, d, a.result());
     } else {
       const size_t at = (item0 + h) * n_splits + split;
-      __hip_atomic_store(part_o + at * hd + d, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (d == 0) {
-        __hip_atomic_store(part_ml + at * 2, top, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(part_ml + at * 2 + 1, weight, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+      ag_leave(a, part_o + at * hd + d, part_ml + at * 2, d == 0);
     }
-  }
+  });
   if (n_splits == 1) return;
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wavefront's stores have been acknowledged
   __syncthreads();
@@ -421,22 +414,8 @@ __global__ void __launch_bounds__(AF_DECODE_WAVES* BLM_WAVE)
   }
   __syncthreads();
   if (!is_last) return;
-  for (int i = tid; i < heads * hd; i += AF_DECODE_WAVES * BLM_WAVE) {
-    const int h = i / hd, d = i - h * hd;
-    float M = -INFINITY, L = 0.f, O = 0.f;
-    for (int sp = 0; sp < n_splits; ++sp) {
-      const size_t at = (item0 + h) * n_splits + sp;
-      const float ms = __hip_atomic_load(part_ml + at * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float ls = __hip_atomic_load(part_ml + at * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float os = __hip_atomic_load(part_o + at * hd + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (ls == 0.f) continue;          // an empty piece
-      const float Mn = fmaxf(M, ms), keep = expf(M - Mn), take = expf(ms - Mn);
-      L = L * keep + ls * take;
-      O = O * keep + os * take;
-      M = Mn;
-    }
-    orow[i] = O * (1.0f / L);
-  }
+  ag_merge<AF_DECODE_WAVES * BLM_WAVE>(part_o + item0 * n_splits * hd, part_ml + item0 * n_splits * 2, heads, n_splits, hd, ex,
+                                       [&](int h, int d, const AgSum& a) { put(h, d, a.result()); });
 }
 
 extern "C" int blm_attn_f32_supported(int hd, int page_size) { return hd >= 4 && hd % 4 == 0 && hd <= 128 && page_size == AF_PAGE ? 1 : 0; }
@@ -482,6 +461,7 @@ extern "C" int blm_attn_decode_f32(const void* q, int q_row_stride, void* out, c
   if (attn_f32_check("attn_decode_f32", q, q_row_stride, kcache, vcache, nh, nkv, hd, table_width, window)) return 1;
   BLM_REQUIRE(n_splits >= 1 && n_splits <= 65535 && (n_splits == 1 || (part_o && part_ml && arrivals)), "attn_decode_f32: %d splits need their workspace", n_splits);
   const long long y = (long long)nkv * ((nh / nkv + 15) / 16);
+  BLM_REQUIRE(((uintptr_t)part_o % 8) == 0 && ((uintptr_t)part_ml % 8) == 0, "attn_decode_f32: the workspace must be 8-byte aligned");
   BLM_REQUIRE(T > 0 && T <= 65535 && y <= 65535, "attn_decode_f32: bad sizes T=%d heads=%d", T, nh);
   dim3 grid((unsigned)n_splits, (unsigned)y, (unsigned)T), block(AF_DECODE_WAVES * BLM_WAVE);
 #define BLM_AFD(HD, FREE)                                                                                                 \

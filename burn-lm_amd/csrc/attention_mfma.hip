@@ -24,6 +24,7 @@
 
 #include <type_traits>
 
+#include "attn_merge.h"
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -815,7 +816,7 @@ __global__ void __launch_bounds__(AM_WAVES* BLM_WAVE) __attribute__((amdgpu_wave
 //   part_o [T, nh, splits, HD] float, part_ml [T, nh, splits, 2] float,
 // merged by whichever split of a (token, head tile) finishes last
 // ---------------------------------------------------------------------------------------
-template <int HD, bool EXT>
+template <int HD, bool EXT, bool WIDE>
 __global__ void __launch_bounds__(AM_WAVES* BLM_WAVE)
     attn_decode_mfma_kernel(const bf16* __restrict__ q, int q_row_stride, const int* __restrict__ positions,
                             const int* __restrict__ token_seq, const int* __restrict__ block_table,
@@ -919,25 +920,48 @@ __global__ void __launch_bounds__(AM_WAVES* BLM_WAVE)
       if (HD % 16 == 0 || d < HD) sm_o[c][d] = o[dt][r];
     }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < 16 * HD; idx += blockDim.x) {
-    const int cc = idx / HD, d = idx - cc * HD;
-    if (g0 + cc >= G) continue;
-    float M = sm_m[0][cc];
+  // WIDE: four dims to a thread, where a dim to each of them would be several rounds
+  const int heads = min(16, G - g0);
+  const size_t first_head = (size_t)t * nh + kvh * G + g0;
+  const auto ex2 = [](float v) { return __builtin_amdgcn_exp2f(v); };   // maxima are in base 2
+  const auto put = [&](int cc, int d, float4 v) {
+    const size_t at = (first_head + cc) * HD + d;
+    am_store(out, at, v.x, out_f32);
+    am_store(out, at + 1, v.y, out_f32);
+    am_store(out, at + 2, v.z, out_f32);
+    am_store(out, at + 3, v.w, out_f32);
+  };
+  if constexpr (WIDE) {
+    ag_block<AM_WAVES * BLM_WAVE, AM_WAVES>(&sm_m[0][0], &sm_l[0][0], reinterpret_cast<const float*>(&sm_area[0][0]), AREA_BYTES / 4, HD, heads, HD, ex2,
+                                            [&](int cc, int d, const AgSum& a) {
+      if (n_splits == 1 || b < 0) {   // nothing to merge (a padding token gives zeros)
+        put(cc, d, b < 0 ? make_float4(0.f, 0.f, 0.f, 0.f) : a.result());
+      } else {
+        const size_t at = (first_head + cc) * n_splits + split;
+        ag_leave(a, part_o + at * HD + d, part_ml + at * 2, d == 0);
+      }
+    });
+  } else {
+    for (int idx = threadIdx.x; idx < 16 * HD; idx += blockDim.x) {
+      const int cc = idx / HD, d = idx - cc * HD;
+      if (g0 + cc >= G) continue;
+      float M = sm_m[0][cc];
 #pragma unroll
-    for (int k = 1; k < AM_WAVES; ++k) M = fmaxf(M, sm_m[k][cc]);
-    float L = 0.f, O = 0.f;
+      for (int k = 1; k < AM_WAVES; ++k) M = fmaxf(M, sm_m[k][cc]);
+      float L = 0.f, O = 0.f;
 #pragma unroll
-    for (int k = 0; k < AM_WAVES; ++k) {
-      const float f = (sm_m[k][cc] == M) ? 1.f : __builtin_amdgcn_exp2f(sm_m[k][cc] - M);   // maxima are in base 2
-      L += sm_l[k][cc] * f;
-      O += reinterpret_cast<const float*>(sm_area[k])[cc * HD + d] * f;
-    }
-    if (n_splits == 1 || b < 0) {   // nothing to merge (a padding token gives zeros)
-      am_store(out, ((size_t)t * nh + kvh * G + g0 + cc) * HD + d, b < 0 ? 0.f : O / L, out_f32);
-    } else {
-      const size_t at = ((size_t)t * nh + kvh * G + g0 + cc) * n_splits + split;
-      coherent_store(part_o + at * HD + d, O);
-      if (d == 0) { coherent_store(part_ml + at * 2, M); coherent_store(part_ml + at * 2 + 1, L); }
+      for (int k = 0; k < AM_WAVES; ++k) {
+        const float f = (sm_m[k][cc] == M) ? 1.f : __builtin_amdgcn_exp2f(sm_m[k][cc] - M);   // maxima are in base 2
+        L += sm_l[k][cc] * f;
+        O += reinterpret_cast<const float*>(sm_area[k])[cc * HD + d] * f;
+      }
+      if (n_splits == 1 || b < 0) {   // nothing to merge (a padding token gives zeros)
+        am_store(out, ((size_t)t * nh + kvh * G + g0 + cc) * HD + d, b < 0 ? 0.f : O / L, out_f32);
+      } else {
+        const size_t at = ((size_t)t * nh + kvh * G + g0 + cc) * n_splits + split;
+        coherent_store(part_o + at * HD + d, O);
+        if (d == 0) { coherent_store(part_ml + at * 2, M); coherent_store(part_ml + at * 2 + 1, L); }
+      }
     }
   }
   if (n_splits == 1 || b < 0) return;
@@ -960,41 +984,46 @@ __global__ void __launch_bounds__(AM_WAVES* BLM_WAVE)
   }
   __syncthreads();
   if (!last) return;
-  for (int idx = threadIdx.x; idx < 16 * HD; idx += blockDim.x) {
-    const int cc = idx / HD, d = idx - cc * HD;
-    if (g0 + cc >= G) continue;
-    const size_t head_at = (size_t)t * nh + kvh * G + g0 + cc;
-    const size_t base = head_at * n_splits;
-    const float* ml = part_ml + base * 2;
-    // AD_MERGE splits per memory round trip, merged online (with eight per trip, 64 splits cost 12 us
-    // of round trips in a row)
-    float M = -INFINITY, L = 0.f, O = 0.f;
-    for (int s0 = 0; s0 < n_splits; s0 += AD_MERGE) {
-      float vm[AD_MERGE], vl[AD_MERGE], po[AD_MERGE];
+  if constexpr (WIDE) {
+    ag_merge<AM_WAVES * BLM_WAVE>(part_o + first_head * n_splits * HD, part_ml + first_head * n_splits * 2, heads, n_splits, HD, ex2,
+                                  [&](int cc, int d, const AgSum& a) { put(cc, d, a.result()); });
+  } else {
+    for (int idx = threadIdx.x; idx < 16 * HD; idx += blockDim.x) {
+      const int cc = idx / HD, d = idx - cc * HD;
+      if (g0 + cc >= G) continue;
+      const size_t head_at = (size_t)t * nh + kvh * G + g0 + cc;
+      const size_t base = head_at * n_splits;
+      const float* ml = part_ml + base * 2;
+      // AD_MERGE splits per memory round trip, merged online (with eight per trip, 64 splits cost 12 us
+      // of round trips in a row)
+      float M = -INFINITY, L = 0.f, O = 0.f;
+      for (int s0 = 0; s0 < n_splits; s0 += AD_MERGE) {
+        float vm[AD_MERGE], vl[AD_MERGE], po[AD_MERGE];
 #pragma unroll
-      for (int i = 0; i < AD_MERGE; ++i) {
-        const int sp = min(s0 + i, n_splits - 1);
-        vm[i] = coherent_load(ml + 2 * sp);
-        vl[i] = coherent_load(ml + 2 * sp + 1);
-        po[i] = coherent_load(part_o + (base + sp) * HD + d);
-      }
-      float Mc = M;
-#pragma unroll
-      for (int i = 0; i < AD_MERGE; ++i) Mc = fmaxf(Mc, vm[i]);
-      const float keep = (M == Mc) ? 1.f : __builtin_amdgcn_exp2f(M - Mc);   // maxima are in base 2
-      L *= keep;
-      O *= keep;
-#pragma unroll
-      for (int i = 0; i < AD_MERGE; ++i) {
-        if (s0 + i < n_splits) {
-          const float f = (vm[i] == Mc) ? 1.f : __builtin_amdgcn_exp2f(vm[i] - Mc);
-          L += vl[i] * f;
-          O += po[i] * f;
+        for (int i = 0; i < AD_MERGE; ++i) {
+          const int sp = min(s0 + i, n_splits - 1);
+          vm[i] = coherent_load(ml + 2 * sp);
+          vl[i] = coherent_load(ml + 2 * sp + 1);
+          po[i] = coherent_load(part_o + (base + sp) * HD + d);
         }
+        float Mc = M;
+#pragma unroll
+        for (int i = 0; i < AD_MERGE; ++i) Mc = fmaxf(Mc, vm[i]);
+        const float keep = (M == Mc) ? 1.f : __builtin_amdgcn_exp2f(M - Mc);   // maxima are in base 2
+        L *= keep;
+        O *= keep;
+#pragma unroll
+        for (int i = 0; i < AD_MERGE; ++i) {
+          if (s0 + i < n_splits) {
+            const float f = (vm[i] == Mc) ? 1.f : __builtin_amdgcn_exp2f(vm[i] - Mc);
+            L += vl[i] * f;
+            O += po[i] * f;
+          }
+        }
+        M = Mc;
       }
-      M = Mc;
+      am_store(out, head_at * HD + d, O / L, out_f32);
     }
-    am_store(out, head_at * HD + d, O / L, out_f32);
   }
 }
 
@@ -1108,19 +1137,23 @@ extern "C" int blm_attn_decode(const void* q, int q_row_stride, void* out, int a
   const int G = nh / nkv;
   const int gtiles = (G + 15) / 16;
   BLM_REQUIRE((long long)nkv * gtiles <= 65535, "attn_decode: too many heads");
+  BLM_REQUIRE(((uintptr_t)part_o % 8) == 0 && ((uintptr_t)part_ml % 8) == 0, "attn_decode: the workspaces must be 8-byte aligned");
   dim3 grid(n_splits, nkv * gtiles, T), block(AM_WAVES * BLM_WAVE);
-#define BLM_AD(HD)                                                                                                 \
-  case HD:                                                                                                         \
-    if (keep_first > 0 || cap > 0.f)                                                                               \
-      hipLaunchKernelGGL((attn_decode_mfma_kernel<HD, true>), grid, block, 0, stream, (const bf16*)q, q_row_stride, \
-                         positions, token_seq, block_table, table_width, (const bf16*)kcache, (const bf16*)vcache,  \
-                         nh, nkv, scale, window, n_splits, part_o, part_ml, arrivals, out, sinks, keep_first, cap, out_f32); \
-    else                                                                                                           \
-      hipLaunchKernelGGL((attn_decode_mfma_kernel<HD, false>), grid, block, 0, stream, (const bf16*)q, q_row_stride, \
-                         positions, token_seq, block_table, table_width, (const bf16*)kcache, (const bf16*)vcache,  \
-                         nh, nkv, scale, window, n_splits, part_o, part_ml, arrivals, out, sinks, 0, 0.f, out_f32);   \
+#define BLM_AD1(HD, EXT, WIDE)                                                                                              \
+  hipLaunchKernelGGL((attn_decode_mfma_kernel<HD, EXT, WIDE>), grid, block, 0, stream, (const bf16*)q, q_row_stride, positions, \
+                     token_seq, block_table, table_width, (const bf16*)kcache, (const bf16*)vcache, nh, nkv, scale, window, \
+                     n_splits, part_o, part_ml, arrivals, out, sinks, EXT ? keep_first : 0, EXT ? cap : 0.f, out_f32)
+  // more dims than threads: four to a thread where results are added up (attn_merge.h)
+  const bool extended = keep_first > 0 || cap > 0.f, wide = (G < 16 ? G : 16) * hd > AM_WAVES * BLM_WAVE;
+#define BLM_AD(HD)                               \
+  case HD:                                       \
+    if (extended && wide) BLM_AD1(HD, true, true); \
+    else if (extended) BLM_AD1(HD, true, false); \
+    else if (wide) BLM_AD1(HD, false, true);     \
+    else BLM_AD1(HD, false, false);              \
     break
   switch (hd) { BLM_AD(16); BLM_AD(32); BLM_AD(48); BLM_AD(64); BLM_AD(80); BLM_AD(96); BLM_AD(112); BLM_AD(128); }
+#undef BLM_AD1
 #undef BLM_AD
   BLM_LAUNCH_CHECK("attn_decode_mfma");
   return 0;

@@ -52,10 +52,9 @@ def decode_splits(pages: int, blocks: int, head_dim: int, compute_units: int = 2
     fourth compute unit on (heads of 128, 11 pages at batch 8: uncut 12.3, in two 14.0; 16 pages at batch
     16: 16.9 / 18.5; heads of 64, 16 pages at batch 8: 9.1 / 10.0).  Longer ranges of wide heads go down to one page per wavefront
     while the pieces still run in one round and are no more than eight, beyond which their merge costs more than they save (16 heads of
-    128 in 4 groups, pieces by the rules above / by this one: 8 sequences of 18 pages 4 / 5 pieces 13.7 / 12.8, 24 pages 4 / 6 14.6 /
-    14.0, 32 pages 4 / 8 15.8 / 15.3; 16 sequences of 18 pages 2 / 4 17.1 / 15.7, 24 pages 3 / 4 16.9 / 17.0; in 8 groups, 8 sequences
-    of 18 pages 2 / 4 17.2 / 15.6; but in 4 groups 4 sequences of 64 pages 8 / 16 16.1 / 16.9, 2 of 100 pages 16 / 25 15.2 / 15.7, and 16
-    heads of 96, one sequence of 64 pages 8 / 16 13.0 / 14.3)."""
+    128 in 4 groups, pieces by the rules above / by this one: 8 sequences of 18 pages 4 / 5 pieces 12.0 / 11.1, 24 pages 4 / 6 12.2 /
+    11.9, 32 pages 4 / 8 13.2 / 13.3; 16 sequences of 18 pages 2 / 4 15.6 / 14.0, 24 pages 3 / 4 15.2 / 15.4; in 8 groups, 8 sequences
+    of 18 pages 2 / 4 17.2 / 15.6; but in 4 groups 4 sequences of 64 pages 8 / 16 13.8 / 14.7, 2 of 100 pages 16 / 25 13.2 / 14.3)."""
     if blocks >= compute_units or pages <= (12 if head_dim <= 64 else 8):
         return 1
     if pages <= 16 and blocks * 4 >= compute_units:
@@ -72,10 +71,10 @@ def decode_splits(pages: int, blocks: int, head_dim: int, compute_units: int = 2
 def decode_splits_f32(pages: int, blocks: int, head_dim: int, compute_units: int = 256) -> int:
     """The same for float32 (ops.attn_decode_f32): a block's eight wavefronts take a quarter, a half or a whole page each, and a
     whole one takes a wavefront about 5 us (8 for wide heads), most of it the fetch's latency and the products of sixteen columns of
-    which a group fills few; the merge takes 1 to 2.  So pieces of two pages, which go in quarters, as long as every block has a
+    which a group fills few; the merge takes some 2.  So pieces of two pages, which go in quarters, as long as every block has a
     compute unit to itself; never more than 16 (us a call, whole / in 2 / 3 / 4 pieces, 32 heads of 64 in 8 groups: 4 pages at batch 8
-    7.9 / 7.8 / - / 7.9; 8 pages at batch 1 11.8 / 10.0 / - / 8.4, at batch 8 11.9 / 10.2 / 10.0 / 8.7; 12 pages at batch 8 16.3 /
-    13.4 / 10.9 / 10.9, at batch 16 17.6 / 15.3 / 19.9; 50 pages at batch 16 55 / 38 / - / 46; 24 heads of 128: 8 pages at batch 8
+    7.9 / 7.8 / - / 7.9; 8 pages at batch 1 11.8 / 10.0 / - / 8.4, at batch 8 11.9 / 10.2 / 10.0 / 8.7; 9 pages at batch 8 14.0 / 13.5 / 10.2 / 10.7; 11 pages
+    at batch 8 17.8 / 14.0 / 11.1 / 10.9, at batch 16 17.6 / 15.3 / 19.9; 50 pages at batch 16 55 / 38 / - / 46; 24 heads of 128: 8 pages at batch 8
     23.8 / 16.0 / - / 12.4).  Few key-value heads behind very many keys would take more
     pieces (one head of 64 at batch 1, 16 / 32 / 64 pieces: 16,000 keys 27 / 25 / 32, 65,000 keys 73 / 49 / 44, 130,000 keys
     135 / 82 / 61; the generic kernel 77, 202 and 248)."""
