@@ -73,8 +73,8 @@ def decode_splits_f32(pages: int, blocks: int, head_dim: int, compute_units: int
     whole one takes a wavefront about 5 us (8 for wide heads), most of it the fetch's latency and the products of sixteen columns of
     which a group fills few; the merge takes some 2.  So pieces of two pages, which go in quarters, as long as every block has a
     compute unit to itself; never more than 16 (us a call, whole / in 2 / 3 / 4 pieces, 32 heads of 64 in 8 groups: 4 pages at batch 8
-    7.9 / 7.8 / - / 7.9; 8 pages at batch 1 11.8 / 10.0 / - / 8.4, at batch 8 11.9 / 10.2 / 10.0 / 8.7; 9 pages at batch 8 14.0 / 13.5 / 10.2 / 10.7; 11 pages
-    at batch 8 17.8 / 14.0 / 11.1 / 10.9, at batch 16 17.6 / 15.3 / 19.9; 50 pages at batch 16 55 / 38 / - / 46; 24 heads of 128: 8 pages at batch 8
+    7.9 / 7.8 / - / 7.9; 8 pages at batch 1 11.8 / 10.0 / - / 8.4, at batch 8 11.9 / 10.2 / 10.0 / 8.7; 9 pages at batch 8 14.0 / 13.5 / 10.2 / 10.7;
+    11 pages 17.8 / 14.0 / 11.1 / 10.9; 12 pages at batch 16 17.6 / 15.3 / 19.9; 50 pages at batch 16 55 / 38 / - / 46; 24 heads of 128: 8 pages at batch 8
     23.8 / 16.0 / - / 12.4).  Few key-value heads behind very many keys would take more
     pieces (one head of 64 at batch 1, 16 / 32 / 64 pieces: 16,000 keys 27 / 25 / 32, 65,000 keys 73 / 49 / 44, 130,000 keys
     135 / 82 / 61; the generic kernel 77, 202 and 248)."""
