@@ -14,7 +14,7 @@
 // cut cancels: 1.7e-7 off (2.17e-7 with the float instructions), 7e-11 too low, and the logits 2.6e-6.
 // Measured (us, the float instructions' best tile and groups / this, without the parts' pass of 3.5 to 5 us, with K = 8,192 14; weights from memory),
 // 1,000 rows: [16384, 2048] gated 502 / 284 (236 TFLOP/s of float products), [2048, 8192] 259 / 157, [3072, 2048] 105 / 75, [2048, 2048] 72 / 47;
-// 256 rows 137 / 90, 74 / 50, 33 / 26, 24 / 18.  Scoring 1,000 tokens at the 1B shape 16.93 -> 10.65 ms.
+// 256 rows 137 / 90, 74 / 50, 33 / 26, 24 / 18.  Scoring 1,000 tokens at the 1B shape 16.93 -> 10.45 ms.
 // The ring is as deep as the weights' way from memory asks: with the next two stages under way tiles of 64 rows, whose stages are short, took 1.34 us
 // a stage for the 64 x 128, with three 0.70 (1.2 and 1.13 for 64 x 256; four and five: as three).
 // Tried: columns from global memory straight into registers (120 -> 133 us on 64 blocks), tiles of 256 x 256 (two stages fill the
@@ -56,6 +56,19 @@ __device__ __forceinline__ void gs_split_odd(float x, uint32_t& hi, uint32_t& mi
 }
 __device__ __forceinline__ bool gs_odd(float x) { return (__float_as_uint(x) & 0x7fffffffu) >= 0x7f7f8000u; }
 
+__device__ __forceinline__ void gs_split_any(float x, float y, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  if (!(gs_odd(x) || gs_odd(y))) {
+    gs_split(x, y, hi, mid, lo);
+  } else {
+    uint32_t h, m, l;
+    gs_split_odd(x, hi, mid, lo);
+    gs_split_odd(y, h, m, l);
+    hi |= h << 16;
+    mid |= m << 16;
+    lo |= l << 16;
+  }
+}
+
 // ---------------------------------------------------------------------------------------------------------------------
 // parts of the rows: P [ceil(M / 16)][K / 32][3][64 lanes][8]: lane l holds row l % 16, elements 4 (l / 16) + 0..3 and 16 + 4 (l / 16) + 0..3
 // of the 32; rows behind M are zero.
@@ -72,23 +85,8 @@ __global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict
   }
   const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
   uint32_t hi[4], mid[4], lo[4];
-  bool odd = false;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) odd |= gs_odd(x[e]);
-  if (!odd) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) gs_split(x[2 * e], x[2 * e + 1], hi[e], mid[e], lo[e]);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      uint32_t h, m, l;
-      gs_split_odd(x[2 * e], hi[e], mid[e], lo[e]);
-      gs_split_odd(x[2 * e + 1], h, m, l);
-      hi[e] |= h << 16;
-      mid[e] |= m << 16;
-      lo[e] |= l << 16;
-    }
-  }
+  for (int e = 0; e < 4; ++e) gs_split_any(x[2 * e], x[2 * e + 1], hi[e], mid[e], lo[e]);
   uint4* p = P + ((size_t)tile * steps + ks) * 192 + lane;
   p[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
   p[64] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
@@ -106,6 +104,12 @@ extern "C" int blm_split_rows(const void* X, void* P, int M, int K, int ldx, hip
 }
 
 __device__ __forceinline__ float gs_silu_times(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+
+// where the first part of row m's column n lies, in the parts of rows of N columns
+__device__ __forceinline__ unsigned char* gs_part_of(float* parts, int m, int n, int N) {
+  return reinterpret_cast<unsigned char*>(parts) + ((size_t)(m / 16) * (N / GS_BK) + n / GS_BK) * (3 * GS_FRAGMENT) + (m % 16 + n % 16 / 4 * 16) * 16 +
+         n % GS_BK / 16 * 8 + n % 4 * 2;
+}
 
 // One element in float, from the floats themselves: where an operand is not finite (or rounds to an infinity as a bfloat16) its parts give NaN
 // (an infinity less itself, or times a part that is zero), which this replaces by what the sum is.
@@ -129,7 +133,10 @@ using GsInt = std::integral_constant<int, V>;
 // RING of the rows' parts and one of RING - 1 of each wavefront's own columns.  One barrier a stage, in its middle: behind it the next
 // stage's operands are there, the last one of the ring is asked for, and the next columns are split beside the second half's products.
 // lane l of a product: row l % 16, columns 4 (l / 16) + 0..3.  W rows past the end are the last one again; nothing stores what comes of them.
-template <int MT, int NT, int RING, bool GATED>
+// PARTS: a gated product whose results go out as the parts of the rows that the next product reads: a lane's four columns are half of its
+// 16 bytes of a fragment.  (Scoring 1,000 tokens at the 1B shape with
+// results and a pass over them / parts: 11.34 / 11.13 ms on one card.)
+template <int MT, int NT, int RING, bool GATED, bool PARTS>
 __global__ void __launch_bounds__(512, 2)
     gemm_split_kernel(const unsigned char* __restrict__ P, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K, int ldc,
                       int steps_per_group, long long plane, int m_tiles) {
@@ -293,7 +300,17 @@ __global__ void __launch_bounds__(512, 2)
         v[e] = GATED ? gs_silu_times(total[i][0][e], total[i][NT - 1][e]) : total[i][j][e];
         odd |= (unsigned long long)(v[e] != v[e]) << ((i * (GATED ? 1 : NT) + j) * 4 + e);
       }
-      if (m < M && n < N) *reinterpret_cast<float4*>(out + (size_t)m * ldc + n) = make_float4(v[0], v[1], v[2], v[3]);
+      if constexpr (PARTS) {
+        if (m0 + i * 16 >= M || n >= N) continue;
+        uint32_t part[2][3];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) gs_split_any(m < M ? v[2 * e] : 0.f, m < M ? v[2 * e + 1] : 0.f, part[e][0], part[e][1], part[e][2]);
+        unsigned char* to = gs_part_of(C, m, n, N);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(to + q * GS_FRAGMENT) = make_uint2(part[0][q], part[1][q]);
+      } else {
+        if (m < M && n < N) *reinterpret_cast<float4*>(out + (size_t)m * ldc + n) = make_float4(v[0], v[1], v[2], v[3]);
+      }
     }
   }
   for (; odd != 0; odd &= odd - 1) {
@@ -302,12 +319,18 @@ __global__ void __launch_bounds__(512, 2)
     if (m >= M || n >= N) continue;
     float v = gs_repair(P, W + (size_t)n * K, m, steps_all, s_begin, stages);
     if (GATED) v = gs_silu_times(v, gs_repair(P, W + (size_t)(N + n) * K, m, steps_all, s_begin, stages));
-    out[(size_t)m * ldc + n] = v;
+    if constexpr (PARTS) {
+      uint32_t part[3];
+      gs_split_odd(v, part[0], part[1], part[2]);
+      for (int q = 0; q < 3; ++q) *reinterpret_cast<uint16_t*>(gs_part_of(C, m, n, N) + q * GS_FRAGMENT) = (uint16_t)part[q];
+    } else {
+      out[(size_t)m * ldc + n] = v;
+    }
   }
 }
 
 // P: the parts of A [M, K] (split_rows).  rows x columns: a block's tile, 128 or 64 by 256 or 128 (gated: gate and up columns
-// together, 256).  groups > 1: K in that many groups, C holds a plane of M * N for each (contiguous, ldc = N), which the reader adds up.
+// together, 256).  gated: 0, 1, or 2 for results that come as parts of rows of N columns, as split_rows makes them.  groups > 1: K in that many groups, C holds a plane of M * N for each (contiguous, ldc = N), which the reader adds up.
 extern "C" int blm_gemm_split(const void* P, const void* W, void* C, int M, int N, int K, int ldc, int gated, int groups, int rows,
                               int columns, hipStream_t stream) {
   BLM_REQUIRE(M > 0 && N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0 && ldc >= N && ldc % 4 == 0, "gemm_split: sizes M=%d N=%d K=%d ldc=%d not supported",
@@ -315,6 +338,7 @@ extern "C" int blm_gemm_split(const void* P, const void* W, void* C, int M, int 
   BLM_REQUIRE(((uintptr_t)P % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)C % 16) == 0, "gemm_split: operands must be 16-byte aligned");
   const int steps = groups >= 1 ? (K / 128 + groups - 1) / groups * 4 : 0;
   BLM_REQUIRE(groups >= 1 && groups <= 64 && (groups == 1 || (!gated && ldc == N)) && (groups - 1) * steps * GS_BK < K, "gemm_split: %d groups of K=%d", groups, K);
+  BLM_REQUIRE(gated >= 0 && gated <= 2 && (gated != 2 || (N % GS_BK == 0 && ldc == N)), "gemm_split: gating %d of %d columns", gated, N);
   BLM_REQUIRE(((gated ? N : 0) + 256LL) * K * 4 < (1LL << 32), "gemm_split: gated matrices of 4 GiB and more are not supported (N=%d K=%d)", N, K);
   BLM_REQUIRE((rows == 128 || rows == 64) && (columns == 256 || (columns == 128 && !gated)), "gemm_split: tile %d x %d", rows, columns);
   const int per = gated ? columns / 2 : columns;
@@ -322,18 +346,21 @@ extern "C" int blm_gemm_split(const void* P, const void* W, void* C, int M, int 
   const long long blocks = (long long)m_tiles * n_tiles;
   BLM_REQUIRE(blocks < 2147483647LL, "gemm_split: too many tiles");
   dim3 grid((unsigned)blocks, (unsigned)groups), block(512);
-#define GS_RUN(MT, NT, RING, G)                                                                                                             \
-  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, RING, G>), grid, block, 0, stream, (const unsigned char*)P, (const float*)W, (float*)C, M, N, \
+#define GS_RUN(MT, NT, RING, G, PARTS)                                                                                                          \
+  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, RING, G, PARTS>), grid, block, 0, stream, (const unsigned char*)P, (const float*)W, (float*)C, M, N, \
                      K, ldc, steps, (long long)M * N, m_tiles)
-  if (gated) {
-    if (rows == 128) GS_RUN(8, 2, 3, true);
-    else GS_RUN(4, 2, 4, true);
+  if (gated == 2) {
+    if (rows == 128) GS_RUN(8, 2, 3, true, true);
+    else GS_RUN(4, 2, 4, true, true);
+  } else if (gated) {
+    if (rows == 128) GS_RUN(8, 2, 3, true, false);
+    else GS_RUN(4, 2, 4, true, false);
   } else if (columns == 256) {
-    if (rows == 128) GS_RUN(8, 2, 3, false);
-    else GS_RUN(4, 2, 4, false);
+    if (rows == 128) GS_RUN(8, 2, 3, false, false);
+    else GS_RUN(4, 2, 4, false, false);
   } else {
-    if (rows == 128) GS_RUN(8, 1, 3, false);
-    else GS_RUN(4, 1, 4, false);
+    if (rows == 128) GS_RUN(8, 1, 3, false, false);
+    else GS_RUN(4, 1, 4, false, false);
   }
 #undef GS_RUN
   BLM_LAUNCH_CHECK("gemm_split");

@@ -655,13 +655,17 @@ def split_takes(M, N, K, gated=False):
     return M > 0 and K % 128 == 0 and N % 16 == 0 and (not gated or (N + 256) * K * 4 < 1 << 32)
 
 
+def _parts(M, K, device):
+    return torch.empty(-(-M // 16), K // 32, 3, 64, 8, dtype=torch.bfloat16, device=device)
+
+
 def split_rows(a):
     """The three bfloat16 parts of float32 rows [M, K], in the order gemm_split reads them: [ceil(M / 16), K / 32, 3, 64, 8]."""
     _gpu(a)
     M, K = a.shape
     if a.dtype != torch.float32 or a.stride(1) != 1 or K % 32 != 0 or a.stride(0) % 4 != 0 or a.data_ptr() % 16 != 0:
         raise KernelError("split_rows: float32 rows in units of 16 bytes and widths in multiples of 32 wanted")
-    parts = torch.empty(-(-M // 16), K // 32, 3, 64, 8, dtype=torch.bfloat16, device=a.device)
+    parts = _parts(M, K, a.device)
     _call("blm_split_rows", a.data_ptr(), parts.data_ptr(), M, K, a.stride(0), _stream())
     return parts
 
@@ -672,19 +676,37 @@ def gemm_split(parts, w, out, gated=False, tile=(128, 256)):
     _gpu(parts, w, out)
     groups = out.shape[0] if out.dim() == 3 else 1
     M, N = out.shape[-2:]
+    if out.dtype != torch.float32 or out.stride(-1) != 1:
+        raise KernelError("gemm_split: float32 results with contiguous rows wanted")
+    if out.dim() == 3:
+        _contig("out", out)
+    _split_check(parts, w, M, N, gated, tile)
+    _call("blm_gemm_split", parts.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, w.shape[1], out.stride(-2), 1 if gated else 0, groups, *tile, _stream())
+    return out
+
+
+def gemm_split_parts(parts, w, M, tile=(128, 256)):
+    """The gated product of gemm_split for M rows, its results as the parts of rows (split_rows) for the product behind it."""
+    _gpu(parts, w)
+    N = w.shape[0] // 2
+    if N % 32:
+        raise KernelError(f"gemm_split_parts: parts of rows of {N}: a multiple of 32 wanted")
+    _split_check(parts, w, M, N, True, tile)
+    out = _parts(M, N, parts.device)
+    _call("blm_gemm_split", parts.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, w.shape[1], N, 2, 1, *tile, _stream())
+    return out
+
+
+def _split_check(parts, w, M, N, gated, tile):
     K = w.shape[1]
-    if w.dtype != torch.float32 or out.dtype != torch.float32 or out.stride(-1) != 1 or not w.is_contiguous():
-        raise KernelError("gemm_split: float32 weights and results with contiguous rows wanted")
+    if w.dtype != torch.float32 or not w.is_contiguous():
+        raise KernelError("gemm_split: float32 weights with contiguous rows wanted")
     if parts.dtype != torch.bfloat16 or not parts.is_contiguous() or tuple(parts.shape) != (-(-M // 16), K // 32, 3, 64, 8):
         raise KernelError(f"gemm_split: the parts {tuple(parts.shape)} are not those of {M} rows of {K}")
     if w.shape[0] != N * (2 if gated else 1) or not split_takes(M, N, K, gated):
-        raise KernelError(f"gemm_split: shapes w={tuple(w.shape)} out={tuple(out.shape)} do not fit")
-    if out.dim() == 3:
-        _contig("out", out)
+        raise KernelError(f"gemm_split: w={tuple(w.shape)} does not fit results of {M} x {N}")
     if tile not in SPLIT_TILES:
         raise KernelError(f"gemm_split: tile {tile} is not one of {SPLIT_TILES}")
-    _call("blm_gemm_split", parts.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, out.stride(-2), 1 if gated else 0, groups, *tile, _stream())
-    return out
 
 
 def gemv_f32_geometry(M, N, K, groups=1):

@@ -151,7 +151,12 @@ def split_plan(M, N, K, compute_units, planes=False, gated=False, added=False):
             us = 2.0 + per_unit * (SPLIT_BLOCK_US + steps * (few + (all_ - few) * fill)) + (_planes_us(M, N, groups, planes) if groups > 1 else 0.0)
             if best is None or us < best[2] * 0.999:
                 best = ((bm, bn), groups, us)
-    return best[0], best[1], best[2] + max(3.4, 2.3 + M * K * 10 / 7e6)
+    return best[0], best[1], best[2] + split_rows_us(M, K)
+
+
+def split_rows_us(M, K):
+    """The pass that makes the rows' parts."""
+    return max(3.4, 2.3 + M * K * 10 / 7e6)
 
 
 # ops.gemm_duo: what half a tile takes of a whole one's time (K = 2048 / 8192, all blocks at once: 22 of 38 us, 73 of 128), and how
@@ -794,6 +799,33 @@ class Runtime:
                     return ops.gemm_duo_beside(x, stacked, out, z, activation=activation, whole=whole)
         return self.gated_linear(x, w, activation=activation), self.linear(x, beside)
 
+    def f32_gated_plan(self, M, inner, K):
+        """(whether by parts, tile) of the float32 gated product, or None for few rows, where the plain product's smaller tiles and the
+        pass behind it (12 bytes an element) are faster."""
+        tile, _, us = f32_plan(M, inner, K, self.compute_units, gated=True)
+        split = split_plan(M, inner, K, self.compute_units, gated=True)
+        by_parts = split is not None and split[2] < us
+        if by_parts:
+            tile, _, us = split
+        apart = [plan(M, 2 * inner, K, self.compute_units, added=True) for plan in (f32_plan, split_plan)]
+        return (by_parts, tile) if us <= min(p[2] for p in apart if p is not None) + 3.0 + M * inner * 12 / 5e6 else None
+
+    def gated_pair(self, x, w, down):
+        """linear(gated_linear(x, w), down, partials=True): in float32 the first product leaves its rows as the parts that the second
+        reads, where both run by parts."""
+        if not isinstance(x, Unscaled) and self.dtype == torch.float32 and x.shape[0] > F32_SKINNY_MAX_ROWS:
+            plain, narrow = (v.w if isinstance(v, LinearWeight) else v for v in (w, down))
+            M, K = x.shape
+            N, inner = narrow.shape
+            if plain.shape[0] == 2 * inner and ops.f32_rows(x, plain) and narrow.dtype == torch.float32 and narrow.is_contiguous() and narrow.data_ptr() % 16 == 0:
+                gated, split = self.f32_gated_plan(M, inner, K), split_plan(M, N, inner, self.compute_units, planes=True)
+                if gated is not None and gated[0] and split is not None and \
+                        split[2] - split_rows_us(M, inner) < f32_plan(M, N, inner, self.compute_units, True)[2]:
+                    parts = ops.gemm_split_parts(ops.split_rows(x), plain, M, tile=gated[1])
+                    shape = (M, N) if split[1] == 1 else (split[1], M, N)
+                    return ops.gemm_split(parts, narrow, torch.empty(shape, dtype=torch.float32, device=x.device), tile=split[0])
+        return self.linear(self.gated_linear(x, w), down, partials=True)
+
     def gated_linear(self, x, w, activation="silu"):
         """act(x gate^T) * (x up^T) for w = [gate rows; up rows] ([2I, K]) -> [M, I]; act is silu or
         (activation="gelu_tanh") the tanh form of GELU.  With few rows in bfloat16 the gating is fused
@@ -817,16 +849,12 @@ class Runtime:
                 if packed is not None:
                     return ops.gemv_f32(x, packed, torch.empty(M, inner, dtype=torch.float32, device=x.device), K, gated=True)
             else:
-                tile, _, fused = f32_plan(M, inner, K, self.compute_units, gated=True)
-                split = split_plan(M, inner, K, self.compute_units, gated=True)
-                by_parts = split is not None and split[2] < fused
-                # few rows: the plain product's smaller tiles and the pass behind it (12 bytes an element)
-                apart = [plan(M, 2 * inner, K, self.compute_units, added=True) for plan in (f32_plan, split_plan)]
-                if min(fused, split[2] if by_parts else fused) <= min(p[2] for p in apart if p is not None) + 3.0 + M * inner * 12 / 5e6:
+                plan = self.f32_gated_plan(M, inner, K)
+                if plan is not None:
                     out = torch.empty(M, inner, dtype=torch.float32, device=x.device)
-                    if by_parts:
-                        return ops.gemm_split(ops.split_rows(x), plain, out, gated=True, tile=split[0])
-                    return ops.gemm_f32(x, plain, out, gated=True, tile=tile)
+                    if plan[0]:
+                        return ops.gemm_split(ops.split_rows(x), plain, out, gated=True, tile=plan[1])
+                    return ops.gemm_f32(x, plain, out, gated=True, tile=plan[1])
         silu = activation == "silu"      # the row-ring kernel gates with silu only; the others take the activation
         fusable = (x.dtype == plain.dtype == self.dtype == torch.bfloat16 and K % 8 == 0 and x.stride(1) == 1
                    and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and plain.is_contiguous())

@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import torch
 
-from .base import FeedForward, Product, TensorSpec
+from .base import FeedForward, Product, TensorSpec, speaks_for
 
 
 class SwiGLU(FeedForward):
@@ -37,6 +37,8 @@ class SwiGLU(FeedForward):
 
     def forward(self, x, step):
         rt = self.rt
+        if speaks_for(rt, "gated_pair", "linear", "gated_linear"):
+            return rt.gated_pair(x, self.w_gate_up, self.w_down)
         return rt.linear(rt.gated_linear(x, self.w_gate_up), self.w_down, partials=True)
 
     def last_weight(self):

@@ -56,6 +56,35 @@ def test_gated(tile, M, I, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile", [(128, 256), (64, 256)])
+@pytest.mark.parametrize("M,I,K", [(17, 32, 128), (64, 128, 384), (130, 160, 256), (129, 416, 512)])
+def test_gated_results_as_parts(tile, M, I, K):
+    """The parts add up to those of the results that the same product stores, also of what is no finite number; rows behind the last are zero."""
+    from burn_lm_amd.csrc import ops
+    x, w = operands(M, 2 * I, K)
+    x[M // 2, 5], x[M - 1, 9], w[3, 7], w[I + 5, 8] = INF, NAN, -INF, torch.finfo(torch.float32).max
+    rows = ops.split_rows(x)
+    want = ops.split_rows(ops.gemm_split(rows, w, torch.empty(M, I, device="cuda"), gated=True, tile=tile))
+    parts = ops.gemm_split_parts(rows, w, M, tile=tile)
+    assert torch.equal(*(torch.nan_to_num(whole_again(p, M, I), 7.0, 1e300, -1e300) for p in (parts, want)))
+    assert bool((parts.reshape(-1, I // 32, 3, 4, 16, 8)[-1, :, :, :, M % 16 or 16:] == 0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [17, 100, 500])
+@pytest.mark.parametrize("I,K,N", [(1024, 512, 512), (4096, 1024, 1024), (416, 512, 256), (1000, 256, 128)])
+def test_pair(M, I, K, N):
+    """Both products of a feed-forward in one call: what they are apart, within the second one's own bound on either order of its sums."""
+    from burn_lm_amd.engine.runtime import Runtime
+    rt = Runtime(torch.float32, "cuda:0")
+    x, w = operands(M, 2 * I, K, pad=4)
+    _, down = operands(1, N, I)
+    got = rt.gated_pair(x, rt.weight(w, gated=True), rt.weight(down))
+    mid = rt.gated_linear(x, w)
+    check(got.sum(0) if got.dim() == 3 else got, mid, down)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("K,groups", [(2048, 1), (2048, 4), (8192, 1), (8192, 4)])
 @pytest.mark.parametrize("spread", [0.0, 2.0])
 def test_no_further_from_64_bits(K, groups, spread):
