@@ -14,7 +14,7 @@
 // cut cancels: 1.7e-7 off (2.17e-7 with the float instructions), 7e-11 too low, and the logits 2.6e-6.
 // Measured (us, the float instructions' best tile and groups / this, without the parts' pass of 3.5 to 5 us, with K = 8,192 14; weights from memory),
 // 1,000 rows: [16384, 2048] gated 502 / 284 (236 TFLOP/s of float products), [2048, 8192] 259 / 157, [3072, 2048] 105 / 75, [2048, 2048] 72 / 47;
-// 256 rows 137 / 90, 74 / 50, 33 / 26, 24 / 18.  Scoring 1,000 tokens at the 1B shape 16.93 -> 10.45 ms.
+// 256 rows 137 / 90, 74 / 50, 33 / 26, 24 / 18.  Scoring 1,000 tokens at the 1B shape 16.92 -> 10.6 ms.
 // The ring is as deep as the weights' way from memory asks: with the next two stages under way tiles of 64 rows, whose stages are short, took 1.34 us
 // a stage for the 64 x 128, with three 0.70 (1.2 and 1.13 for 64 x 256; four and five: as three).
 // Tried: columns from global memory straight into registers (120 -> 133 us on 64 blocks), tiles of 256 x 256 (two stages fill the
@@ -133,13 +133,24 @@ using GsInt = std::integral_constant<int, V>;
 // RING of the rows' parts and one of RING - 1 of each wavefront's own columns.  One barrier a stage, in its middle: behind it the next
 // stage's operands are there, the last one of the ring is asked for, and the next columns are split beside the second half's products.
 // lane l of a product: row l % 16, columns 4 (l / 16) + 0..3.  W rows past the end are the last one again; nothing stores what comes of them.
-// PARTS: a gated product whose results go out as the parts of the rows that the next product reads: a lane's four columns are half of its
-// 16 bytes of a fragment.  (Scoring 1,000 tokens at the 1B shape with
-// results and a pass over them / parts: 11.34 / 11.13 ms on one card.)
-template <int MT, int NT, int RING, bool GATED, bool PARTS>
+// MODE 1, 2: gated (GATED).  2 (PARTS): the results go out as the parts of the rows that the next product reads: a lane's four columns are
+// half of its 16 bytes of a fragment.  (Scoring 1,000 tokens at the 1B shape with results and a pass over them / parts: 11.34 / 11.13 ms
+// on one card.)
+// MODE 3 (ROPE): W is a q/k/v projection with rotary partners in adjacent rows: a lane's four columns are two pairs, which it turns; queries go
+// to C, keys and values to their pages.  (us with the parts' pass, product and rotation kernel / this: [3072, 2048] 500 rows 57.9 / 54.7, 1,000 91.2 /
+// 84.5, 2,048 158 / 148; [5120, 3072] 500 rows 129 / 111, 1,000 214 / 194.  With a row's look-ups between the stores the gain was half of that.)
+struct GsRope {
+  const int *positions, *token_seq, *block_table;
+  const float2* cos_sin;
+  float *kcache, *vcache;      // [pages, nkv, page, hd], [pages, nkv, hd, page]
+  int table_width, page_size, nh, nkv, hd, store;
+};
+
+template <int MT, int NT, int RING, int MODE>
 __global__ void __launch_bounds__(512, 2)
     gemm_split_kernel(const unsigned char* __restrict__ P, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K, int ldc,
-                      int steps_per_group, long long plane, int m_tiles) {
+                      int steps_per_group, long long plane, int m_tiles, GsRope rope) {
+  constexpr bool GATED = MODE == 1 || MODE == 2, PARTS = MODE == 2, ROPE = MODE == 3;
   static_assert(!GATED || NT == 2, "a gated wavefront has a tile of gate columns and their up columns");
   constexpr int A_LOADS = (3 * MT + 7) / 8, B_LOADS = 2 * NT, LOADS = A_LOADS + B_LOADS;
   constexpr int A_STAGE = MT * 3 * GS_FRAGMENT, B_STAGE = 8 * NT * 2048;
@@ -287,10 +298,50 @@ __global__ void __launch_bounds__(512, 2)
   }
 
   float* out = C + (size_t)blockIdx.y * plane;
+  // ROPE: where row m goes (columns of key and value heads of a row without a page go nowhere), and the angles of a lane's two pairs: asked for
+  // for all rows at once, since behind the first store every look-up is a trip of its own
+  auto page_of = [&](int b, int pos) { return rope.store && b >= 0 ? rope.block_table[(size_t)b * rope.table_width + pos / rope.page_size] : -1; };
+  auto angle = [&](int pos, int d) { return rope.cos_sin[(size_t)pos * (rope.hd / 2) + d / 2]; };
+  auto turn = [&](float2 cs, float& x, float& y) {
+    const float t = x;
+    x = t * cs.x - y * cs.y;
+    y = t * cs.y + y * cs.x;
+  };
+  int slots[ROPE ? MT : 1], pages[ROPE ? MT : 1];
+  float2 angles[ROPE ? MT : 1][NT][2];
+  if constexpr (ROPE) {
+    int seqs[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = min(m0 + i * 16 + l16, M - 1);
+      slots[i] = rope.positions[m];
+      seqs[i] = rope.token_seq[m];
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      pages[i] = page_of(seqs[i], slots[i]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int d = min(n0 + wave * 16 * NT + j * 16 + quad * 4, N - 4) % rope.hd;
+        angles[i][j][0] = angle(slots[i], d);
+        angles[i][j][1] = angle(slots[i], d + 2);
+      }
+      slots[i] %= rope.page_size;
+    }
+  }
+  int slot = 0, page = -1;
+  auto value_at = [&](int head, int d) {
+    return rope.vcache + (((size_t)page * rope.nkv + (head - rope.nh - rope.nkv)) * rope.hd + d) * rope.page_size + slot;
+  };
+  auto key_at = [&](int head, int d) { return rope.kcache + (((size_t)page * rope.nkv + (head - rope.nh)) * rope.page_size + slot) * rope.hd + d; };
   unsigned long long odd = 0;              // elements that are not a number: bit (i * NT + j) * 4 + e, gated i * 4 + e
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int m = m0 + i * 16 + l16;
+    if constexpr (ROPE) {
+      slot = slots[i];
+      page = pages[i];
+    }
 #pragma unroll
     for (int j = 0; j < (GATED ? 1 : NT); ++j) {
       const int n = n0 + wave * 16 * (GATED ? 1 : NT) + j * 16 + quad * 4;
@@ -300,7 +351,20 @@ __global__ void __launch_bounds__(512, 2)
         v[e] = GATED ? gs_silu_times(total[i][0][e], total[i][NT - 1][e]) : total[i][j][e];
         odd |= (unsigned long long)(v[e] != v[e]) << ((i * (GATED ? 1 : NT) + j) * 4 + e);
       }
-      if constexpr (PARTS) {
+      if constexpr (ROPE) {
+        if (m >= M || n >= N) continue;
+        const int head = n / rope.hd, d = n - head * rope.hd;
+        if (head < rope.nh + rope.nkv) {
+          turn(angles[i][j][0], v[0], v[1]);
+          turn(angles[i][j][1], v[2], v[3]);
+          if (head < rope.nh) *reinterpret_cast<float4*>(out + (size_t)m * ldc + n) = make_float4(v[0], v[1], v[2], v[3]);
+          else if (page >= 0) *reinterpret_cast<float4*>(key_at(head, d)) = make_float4(v[0], v[1], v[2], v[3]);
+        } else if (page >= 0) {
+          float* to = value_at(head, d);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) to[e * rope.page_size] = v[e];
+        }
+      } else if constexpr (PARTS) {
         if (m0 + i * 16 >= M || n >= N) continue;
         uint32_t part[2][3];
 #pragma unroll
@@ -317,6 +381,19 @@ __global__ void __launch_bounds__(512, 2)
     const int at = __builtin_ctzll(odd), tile = at >> 2, i = GATED ? tile : tile / NT, j = GATED ? 0 : tile % NT;
     const int m = m0 + i * 16 + l16, n = n0 + wave * 16 * (GATED ? 1 : NT) + j * 16 + quad * 4 + (at & 3);
     if (m >= M || n >= N) continue;
+    if constexpr (ROPE) {      // with its partner, of which the turned one is made as well
+      const int pos = rope.positions[m];
+      slot = pos % rope.page_size;
+      page = page_of(rope.token_seq[m], pos);
+      const int head = n / rope.hd, d = (n - head * rope.hd) & ~1, first = n & ~1;
+      float x = gs_repair(P, W + (size_t)first * K, m, steps_all, s_begin, stages), y = gs_repair(P, W + (size_t)(first + 1) * K, m, steps_all, s_begin, stages);
+      if (head < rope.nh + rope.nkv) turn(angle(pos, d), x, y);
+      if (head >= rope.nh && page < 0) continue;
+      float* to = head < rope.nh ? out + (size_t)m * ldc + first : head < rope.nh + rope.nkv ? key_at(head, d) : value_at(head, d);
+      to[0] = x;
+      to[head < rope.nh + rope.nkv ? 1 : rope.page_size] = y;
+      continue;
+    }
     float v = gs_repair(P, W + (size_t)n * K, m, steps_all, s_begin, stages);
     if (GATED) v = gs_silu_times(v, gs_repair(P, W + (size_t)(N + n) * K, m, steps_all, s_begin, stages));
     if constexpr (PARTS) {
@@ -328,6 +405,10 @@ __global__ void __launch_bounds__(512, 2)
     }
   }
 }
+
+#define GS_RUN(MT, NT, RING, MODE, rope)                                                                                                          \
+  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, RING, MODE>), grid, block, 0, stream, (const unsigned char*)P, (const float*)W, (float*)C, M, N, K, \
+                     ldc, steps, (long long)M * N, m_tiles, rope)
 
 // P: the parts of A [M, K] (split_rows).  rows x columns: a block's tile, 128 or 64 by 256 or 128 (gated: gate and up columns
 // together, 256).  gated: 0, 1, or 2 for results that come as parts of rows of N columns, as split_rows makes them.  groups > 1: K in that many groups, C holds a plane of M * N for each (contiguous, ldc = N), which the reader adds up.
@@ -346,23 +427,49 @@ extern "C" int blm_gemm_split(const void* P, const void* W, void* C, int M, int 
   const long long blocks = (long long)m_tiles * n_tiles;
   BLM_REQUIRE(blocks < 2147483647LL, "gemm_split: too many tiles");
   dim3 grid((unsigned)blocks, (unsigned)groups), block(512);
-#define GS_RUN(MT, NT, RING, G, PARTS)                                                                                                          \
-  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, RING, G, PARTS>), grid, block, 0, stream, (const unsigned char*)P, (const float*)W, (float*)C, M, N, \
-                     K, ldc, steps, (long long)M * N, m_tiles)
   if (gated == 2) {
-    if (rows == 128) GS_RUN(8, 2, 3, true, true);
-    else GS_RUN(4, 2, 4, true, true);
+    if (rows == 128) GS_RUN(8, 2, 3, 2, GsRope{});
+    else GS_RUN(4, 2, 4, 2, GsRope{});
   } else if (gated) {
-    if (rows == 128) GS_RUN(8, 2, 3, true, false);
-    else GS_RUN(4, 2, 4, true, false);
+    if (rows == 128) GS_RUN(8, 2, 3, 1, GsRope{});
+    else GS_RUN(4, 2, 4, 1, GsRope{});
   } else if (columns == 256) {
-    if (rows == 128) GS_RUN(8, 2, 3, false, false);
-    else GS_RUN(4, 2, 4, false, false);
+    if (rows == 128) GS_RUN(8, 2, 3, 0, GsRope{});
+    else GS_RUN(4, 2, 4, 0, GsRope{});
   } else {
-    if (rows == 128) GS_RUN(8, 1, 3, false, false);
-    else GS_RUN(4, 1, 4, false, false);
+    if (rows == 128) GS_RUN(8, 1, 3, 0, GsRope{});
+    else GS_RUN(4, 1, 4, 0, GsRope{});
+  }
+  BLM_LAUNCH_CHECK("gemm_split");
+  return 0;
+}
+
+// The q/k/v projection of many rows with the rotation and the page writes behind it.  Wq: W_qkv [(nh + 2 nkv) * hd, K], rotary partners in adjacent
+// rows; qkv_out [M, ldc], of which the first nh * hd columns (the turned queries) are written; store = 0: no keys and values.
+extern "C" int blm_gemm_split_qkv_rope(const void* P, const void* Wq, void* qkv_out, const int* positions, const int* token_seq, const int* block_table,
+                                       int table_width, const float* cos_sin, void* kcache, void* vcache, int page_size, int M, int K, int ldc, int nh,
+                                       int nkv, int hd, int store, int rows, int columns, hipStream_t stream) {
+  BLM_REQUIRE(nh > 0 && nkv > 0 && hd > 0 && hd % 4 == 0 && page_size > 0 && table_width > 0, "gemm_split_qkv_rope: bad geometry (head size %d)", hd);
+  const int N = (nh + 2 * nkv) * hd;
+  BLM_REQUIRE(M > 0 && N % 16 == 0 && K > 0 && K % 128 == 0 && ldc >= nh * hd && ldc % 4 == 0, "gemm_split_qkv_rope: sizes M=%d N=%d K=%d ldc=%d not supported", M, N, K, ldc);
+  BLM_REQUIRE(((uintptr_t)P % 16) == 0 && ((uintptr_t)Wq % 16) == 0 && ((uintptr_t)qkv_out % 16) == 0 && ((uintptr_t)kcache % 16) == 0 && ((uintptr_t)vcache % 4) == 0 &&
+                  ((uintptr_t)cos_sin % 8) == 0, "gemm_split_qkv_rope: operands must be 16-byte aligned (angles 8-byte)");
+  BLM_REQUIRE((rows == 128 || rows == 64) && (columns == 256 || columns == 128), "gemm_split_qkv_rope: tile %d x %d", rows, columns);
+  const int m_tiles = (M + rows - 1) / rows, used = store ? N : nh * hd;
+  const long long blocks = (long long)m_tiles * ((used + columns - 1) / columns);
+  BLM_REQUIRE(blocks < 2147483647LL, "gemm_split_qkv_rope: too many tiles");
+  const GsRope rope{positions, token_seq, block_table, (const float2*)cos_sin, (float*)kcache, (float*)vcache, table_width, page_size, nh, nkv, hd, store};
+  const void *W = Wq, *C = qkv_out;
+  const int steps = K / GS_BK;
+  dim3 grid((unsigned)blocks, 1), block(512);
+  if (columns == 256) {
+    if (rows == 128) GS_RUN(8, 2, 3, 3, rope);
+    else GS_RUN(4, 2, 4, 3, rope);
+  } else {
+    if (rows == 128) GS_RUN(8, 1, 3, 3, rope);
+    else GS_RUN(4, 1, 4, 3, rope);
   }
 #undef GS_RUN
-  BLM_LAUNCH_CHECK("gemm_split");
+  BLM_LAUNCH_CHECK("gemm_split_qkv_rope");
   return 0;
 }

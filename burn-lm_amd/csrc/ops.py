@@ -140,6 +140,7 @@ _SIGNATURES = {
     "blm_split_rows": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
     "blm_gemm_split": [_c_void_p, _c_void_p, _c_void_p] + [_c_int] * 8 + [_c_void_p],
     "blm_gemv_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "blm_gemm_split_qkv_rope": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 10 + [_c_void_p],
     "blm_gemv_f32_qkv_rope": [_c_void_p] * 6 + [_c_int] + [_c_void_p] * 3 + [_c_int] * 9 + [_c_void_p],
     "blm_gemv_f32_scaled": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_int, _c_float,
                             _c_void_p],
@@ -695,6 +696,27 @@ def gemm_split_parts(parts, w, M, tile=(128, 256)):
     out = _parts(M, N, parts.device)
     _call("blm_gemm_split", parts.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, w.shape[1], N, 2, 1, *tile, _stream())
     return out
+
+
+def gemm_split_qkv_rope(x, w, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache, page_size, nh, nkv, hd, write_kv=True, tile=(128, 256)):
+    """gemv_f32_qkv_rope for many float32 rows, by the parts of x and w [(nh + 2 nkv) * hd, K] as bound (head sizes of a multiple of four)."""
+    _gpu(x, w, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache)
+    M, N = x.shape[0], (nh + 2 * nkv) * hd
+    if any(t.dtype != torch.float32 for t in (qkv_out, kcache, vcache, cos_sin)):
+        raise KernelError("gemm_split_qkv_rope: float32 operands, pages and angles wanted")
+    if qkv_out.shape[0] != M or qkv_out.stride(1) != 1 or qkv_out.shape[1] < nh * hd:
+        raise KernelError("gemm_split_qkv_rope: qkv_out must be [M, >= heads*head_dim] with unit stride along rows")
+    _i32("positions", positions, M); _i32("token_seq", token_seq, M); _i32("block_table", block_table)
+    if cos_sin.shape[1:] != (hd // 2, 2) or not cos_sin.is_contiguous():
+        raise KernelError("gemm_split_qkv_rope: cos_sin must be contiguous [positions, head_dim/2, 2]")
+    _contig("kcache", kcache); _contig("vcache", vcache)
+    _check_planes("gemm_split_qkv_rope", kcache, vcache, nkv, page_size, hd)
+    parts = split_rows(x)
+    _split_check(parts, w, M, N, False, tile)
+    _call("blm_gemm_split_qkv_rope", parts.data_ptr(), w.data_ptr(), qkv_out.data_ptr(), positions.data_ptr(), token_seq.data_ptr(), block_table.data_ptr(),
+          block_table.shape[1], cos_sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), page_size, M, w.shape[1], qkv_out.stride(0), nh, nkv, hd,
+          1 if write_kv else 0, *tile, _stream())
+    return qkv_out
 
 
 def _split_check(parts, w, M, N, gated, tile):

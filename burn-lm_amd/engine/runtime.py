@@ -615,6 +615,17 @@ class Runtime:
             return None
         return w.packed
 
+    def f32_qkv_split(self, x, w, M, N, K):
+        """The tile of ops.gemm_split_qkv_rope for a float32 q/k/v projection of many rows, or None where a product and the kernel that turns
+        its results and fills the pages (4 us and 8 bytes an element) are faster: where groups of K are, whose planes have to be added first."""
+        if not (M > F32_SKINNY_MAX_ROWS and x.dtype == torch.float32 and ops.f32_rows(x, w)):
+            return None
+        split = split_plan(M, N, K, self.compute_units)
+        if split is None:
+            return None
+        apart = min(plan(M, N, K, self.compute_units, added=True)[2] for plan in (f32_plan, split_plan))
+        return split[0] if split[2] < apart + 4.0 + M * N * 8 / 3.5e6 else None
+
     def duo_tiles(self, M, N):
         """How many of a product's tiles ops.gemm_duo runs as whole ones."""
         return duo_plan(M, N, self.compute_units)[0]

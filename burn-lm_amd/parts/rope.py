@@ -164,6 +164,10 @@ class RotaryEncoding(PositionEncoding):
                 and hasattr(rt, "f32_qkv_packed")):
             packed = rt.f32_qkv_packed(x, w_qkv, M, n_qkv, K)
             fused = "float32" if packed is not None else None
+        elif (self.pairing == PAIRING["interleaved"] and x.dtype == view.k.dtype == torch.float32 and head_dim % 4 == 0 and raw is not None
+                and view.k.data_ptr() % 16 == 0 and hasattr(rt, "f32_qkv_split")):
+            tile = rt.f32_qkv_split(x, raw, M, n_qkv, K)
+            fused = "parts" if tile is not None else None
         if scale is not None and fused not in ("packed", "float32"):
             raise ValueError(f"rotary encoding: unscaled rows for a projection that does not take them ({M} rows, {fused})")
         if fused is None:
@@ -174,6 +178,10 @@ class RotaryEncoding(PositionEncoding):
             return rt.ops.gemv_f32_qkv_rope(x, packed, torch.empty(M, n_qkv, dtype=torch.float32, device=x.device), step.positions,
                                             step.token_seq, view.block_table(step), self.table, view.k, view.v, view.page_size, heads,
                                             kv_heads, head_dim, write_kv=view.store, scale=scale)
+        if fused == "parts":
+            return rt.ops.gemm_split_qkv_rope(x, raw, torch.empty(M, n_qkv, dtype=torch.float32, device=x.device), step.positions, step.token_seq,
+                                              view.block_table(step), self.table, view.k, view.v, view.page_size, heads, kv_heads, head_dim,
+                                              write_kv=view.store, tile=tile)
         qkv = torch.empty(M, n_qkv, dtype=torch.bfloat16, device=x.device)
         if fused == "tiles":
             if not rt.ops.gemm_duo_takes(x, raw, qkv):

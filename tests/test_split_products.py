@@ -182,6 +182,40 @@ def test_whole_results_of_planes(M, N, K, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,K,nh,nkv,hd", [(17, 128, 2, 1, 64), (130, 256, 3, 1, 48), (64, 384, 5, 1, 36 * 4), (100, 128, 2, 2, 20 * 4), (300, 256, 8, 4, 4)])
+def test_projection_with_rotation_and_pages(tile, M, K, nh, nkv, hd):
+    """Queries and pages are those of the same product followed by the rotation kernel (a rotation is two products and a sum: an ulp of the larger
+    one apart at most), also of what is no finite number; rows of no sequence write no page, heads may end inside a tile of columns."""
+    from burn_lm_amd.csrc import ops
+    g = torch.Generator().manual_seed(M + K)
+    N, page = (nh + 2 * nkv) * hd, 64
+    x, w = operands(M, N, K)
+    w.mul_(K ** -0.5)
+    x[M - 1, 3], w[nh * hd + 1, 9], x[5, 9] = INF, NAN, 0.0
+    pos = ((torch.arange(M) * 37 + 5) % 250).int().cuda()
+    seq = torch.arange(M, dtype=torch.int32)
+    seq[1] = -1
+    seq, table = seq.cuda(), torch.randperm(4 * M, generator=g).view(M, 4).int().cuda()
+    cs = torch.randn(256, hd // 2, 2, generator=g).cuda()
+    got = []
+    for fused in (True, False):
+        k, v = (torch.full((4 * M, nkv, *s), 9.0, device="cuda") for s in ((page, hd), (hd, page)))
+        for store in (False, True):
+            out = torch.full((M, N), 7.0, device="cuda")
+            if fused:
+                ops.gemm_split_qkv_rope(x, w, out, pos, seq, table, cs, k, v, page, nh, nkv, hd, write_kv=store, tile=tile)
+                assert bool((out[:, nh * hd:] == 7).all())
+            else:
+                ops.gemm_split(ops.split_rows(x), w, out, tile=tile)
+                ops.rope_kv_write(out, pos, seq, table, cs, k, v, page, nh, nkv, hd, 0, write_kv=store)
+            assert store or bool((k == 9).all() and (v == 9).all())
+        got.append((out[:, :nh * hd][seq >= 0], k, v))
+    for a, b in zip(*got):
+        assert torch.allclose(a, b, rtol=2.0 ** -21, atol=2.0 ** -20, equal_nan=True)
+
+
+@pytest.mark.gpu
 def test_refused():
     from burn_lm_amd.csrc import ops
     x, w = operands(40, 64, 256)
