@@ -1,7 +1,8 @@
 // The 32-bit product C[M,N] = A[M,K] * W[N,K]^T of many rows on the bfloat16 matrix instructions, with no less precision than on the
 // float ones: a float is the sum of three bfloat16 (hi, mid, lo, rounded to nearest each: 8 + 8 + 8 bits and their signs, the subtractions
 // between them exact), a product of two floats the sum of nine exact products, and the three that are left out (mid lo, lo mid, lo lo)
-// are below 2^-26 of the whole (floats below 2^-110 have no lo of their own: what is lost of them is below 2^-134).  Six instructions of 16 cycles do 16 x 16 x 32, for which the float ones take 256 cycles.
+// are below 2^-26 of the whole (floats below 2^-110 have no lo of their own: what is lost of them is below 2^-134).  Six instructions
+// of 16 cycles do 16 x 16 x 32, for which the float ones take 256 cycles.
 //   split_rows : the parts of the rows, in the order of the instruction's fragments
 //   gemm_split : the product; the weights, which are not kept a second time, are split on their way from shared memory
 // What bounds it: the matrix instructions at the clock that the card's power leaves (1.25 to 1.35 PFLOP/s of them), beside them reads of
@@ -14,7 +15,7 @@
 // cut cancels: 1.7e-7 off (2.17e-7 with the float instructions), 7e-11 too low, and the logits 2.6e-6.
 // Measured (us, the float instructions' best tile and groups / this, without the parts' pass of 3.5 to 5 us, with K = 8,192 14; weights from memory),
 // 1,000 rows: [16384, 2048] gated 502 / 284 (236 TFLOP/s of float products), [2048, 8192] 259 / 157, [3072, 2048] 105 / 75, [2048, 2048] 72 / 47;
-// 256 rows 137 / 90, 74 / 50, 33 / 26, 24 / 18.  Scoring 1,000 tokens at the 1B shape 16.92 -> 10.6 ms.
+// 256 rows 137 / 90, 74 / 50, 33 / 26, 24 / 18.  Scoring 1,000 tokens at the 1B shape 16.9 -> 10.8 ms.
 // The ring is as deep as the weights' way from memory asks: with the next two stages under way tiles of 64 rows, whose stages are short, took 1.34 us
 // a stage for the 64 x 128, with three 0.70 (1.2 and 1.13 for 64 x 256; four and five: as three).
 // Tried: columns from global memory straight into registers (120 -> 133 us on 64 blocks), tiles of 256 x 256 (two stages fill the
@@ -458,7 +459,8 @@ extern "C" int blm_gemm_split_qkv_rope(const void* P, const void* Wq, void* qkv_
   const int m_tiles = (M + rows - 1) / rows, used = store ? N : nh * hd;
   const long long blocks = (long long)m_tiles * ((used + columns - 1) / columns);
   BLM_REQUIRE(blocks < 2147483647LL, "gemm_split_qkv_rope: too many tiles");
-  const GsRope rope{positions, token_seq, block_table, (const float2*)cos_sin, (float*)kcache, (float*)vcache, table_width, page_size, nh, nkv, hd, store};
+  const GsRope rope{positions, token_seq, block_table, (const float2*)cos_sin, (float*)kcache, (float*)vcache,
+                    table_width, page_size, nh, nkv, hd, store};
   const void *W = Wq, *C = qkv_out;
   const int steps = K / GS_BK;
   dim3 grid((unsigned)blocks, 1), block(512);
