@@ -17,6 +17,13 @@
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
+// Column c of a pair of neighbours, turned: the partner's product rounded, the sum of both rounded once.  Left to the compiler, which of
+// the two products is the rounded one changes with the code around them, and with it single results.
+__device__ __forceinline__ float turned(float x, float partner, float2 cs, int c) {
+  const float other = partner * cs.y;
+  return fmaf(x, cs.x, (c & 1) == 0 ? -other : other);
+}
+
 // (What the first loads need stands in the arguments' first fourteen dwords, which come in registers.)
 // QR_KSTEPS: k-steps of 32 per wavefront.  MAXT: most threads of a block (8 or 16 wavefronts).  All
 // loads of a block are in flight at once: its time is one memory latency.
@@ -157,22 +164,7 @@ __global__ void __launch_bounds__(512)
   if (!store && tile >= nh * tiles_per_head) return;   // keys and values belong to another layer's cache: only q is needed
   const int step0 = wave * QR_KSTEPS;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-  const int head = tile / tiles_per_head, col0 = (tile - head * tiles_per_head) * 16;
-  // a thread's output of the tile: row m, column c
-  auto row_of = [&](int idx) { return ((idx & 63) >> 4) * 4 + ((idx >> 6) & 3); };
-  int pos, b, page = -1;
-  float2 cs = make_float2(1.f, 0.f);     // value heads are stored as they are
-  auto ask = [&](int idx) {
-    const int m = min(row_of(idx), M - 1);
-    pos = positions[m];
-    b = token_seq[m];
-  };
-  auto ask_more = [&](int idx) {
-    if (head < nh + nkv) cs = cos_sin[(size_t)pos * (hd / 2) + ((col0 + (idx & 15)) >> 1)];
-    if (head >= nh && b >= 0) page = block_table[(size_t)b * table_width + pos / page_size];
-  };
 
-  ask(threadIdx.x);
   if (SCALED) scale_load.ask(sums, n_sums, M, wave, n_waves, lane);
   const bf16* wt = Wp + ((size_t)tile * k_steps * 64 + lane) * 8;
   uint4 w[QR_KSTEPS];
@@ -181,9 +173,6 @@ __global__ void __launch_bounds__(512)
     const int st = step0 + s;
     w[s] = load16_stream(wt + (size_t)(st < k_steps ? st : k_steps - 1) * 512);   // the weights: read once
   }
-  __builtin_amdgcn_sched_barrier(0);
-  ask_more(threadIdx.x);
-  __builtin_amdgcn_sched_barrier(0);
   const bf16* ap = A + (size_t)(row < M ? row : M - 1) * lda;
   uint4 a[QR_KSTEPS];
 #pragma unroll
@@ -204,13 +193,10 @@ __global__ void __launch_bounds__(512)
   __syncthreads();
 
   // epilogue: one thread per (token row m, column c of the tile)
+  const int head = tile / tiles_per_head, col0 = (tile - head * tiles_per_head) * 16;
   for (int idx = threadIdx.x; idx < 256; idx += n_waves * BLM_WAVE) {
-    const int c = idx & 15, m = row_of(idx);
-    if (idx != threadIdx.x) {      // fewer than four wavefronts
-      page = -1;
-      ask(idx);
-      ask_more(idx);
-    }
+    const int r = idx >> 6, l2 = idx & 63, c = l2 & 15;
+    const int m = (l2 >> 4) * 4 + r;
     if (m >= M) continue;
     float x = 0.f, partner = 0.f;   // column c and its neighbour c ^ 1
     for (int k2 = 0; k2 < n_waves; ++k2) {
@@ -221,14 +207,21 @@ __global__ void __launch_bounds__(512)
       x *= inv[m];
       partner *= inv[m];
     }
+    const int b = token_seq[m];
+    const int pos = positions[m];
     const int d = col0 + c;
-    float y = x;
-    if (head < nh + nkv) y = (c & 1) == 0 ? x * cs.x - partner * cs.y : partner * cs.y + x * cs.x;
+    float y = x;     // value heads are stored as they are
+    if (head < nh + nkv) {
+      const float2 cs = cos_sin[(size_t)pos * (hd / 2) + (d >> 1)];
+      y = turned(x, partner, cs, c);
+    }
     const bf16 o = from_float<bf16>(y);
     if (head < nh) {
       qkv_out[(size_t)m * ldq + (size_t)head * hd + d] = o;
-    } else if (page >= 0) {
+    } else if (b >= 0) {
+      const int page = block_table[(size_t)b * table_width + pos / page_size];
       const int slot = pos % page_size;
+      if (page < 0) continue;
       if (head < nh + nkv) kcache[(((size_t)page * nkv + (head - nh)) * page_size + slot) * hd + d] = o;
       else vcache[((size_t)page * nkv + (head - nh - nkv)) * hd * page_size + (size_t)d * page_size + slot] = o;
     }
@@ -309,7 +302,7 @@ __global__ void __launch_bounds__(512)
     float y = x;     // value heads are stored as they are
     if (head < nh + nkv) {
       const float2 cs = cos_sin[(size_t)pos * (hd / 2) + (d >> 1)];
-      y = (c & 1) == 0 ? x * cs.x - partner * cs.y : partner * cs.y + x * cs.x;
+      y = turned(x, partner, cs, c);
     }
     const bf16 o = from_float<bf16>(y);
     if (head < nh) {
