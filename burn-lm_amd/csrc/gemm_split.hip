@@ -12,7 +12,9 @@
 // one accumulator is 2.7e-7 off and, the same in all of them, 3e-8 too low, which adds up from layer to layer (logits of the 1B shape
 // 3.7e-6 from 64 bits, with the float instructions 2.8e-6).  So a chunk of 128 of K has an accumulator that starts at zero, small products
 // first, and joins the total by a rounded addition; and every other chunk is summed with its columns negated and subtracted, so that what is
-// cut cancels: 1.7e-7 off (2.17e-7 with the float instructions), 7e-11 too low, and the logits 2.6e-6.
+// cut cancels: 1.7e-7 off (2.17e-7 with the float instructions), 7e-11 too low, and the logits 2.6e-6.  It cancels in pairs, so a group of K with
+// an odd number of chunks has its last one in two halves of opposite sign (mean error of normal operands, without / with: K = 128 -8e-9 / 1e-10,
+// 640 -4e-9 / -3e-10, 3,072 in 8 groups of three -1.4e-8 / 0; 2-norms 1.52 / 0.97, 1.59 / 1.52, 1.64 / 1.50e-7, the float instructions' 2.0 to 2.1).
 // Measured (us, the float instructions' best tile and groups / this, without the parts' pass of 3.5 to 5 us, with K = 8,192 14; weights from memory),
 // 1,000 rows: [16384, 2048] gated 502 / 284 (236 TFLOP/s of float products), [2048, 8192] 259 / 157, [3072, 2048] 105 / 75, [2048, 2048] 72 / 47;
 // 256 rows 137 / 90, 74 / 50, 33 / 26, 24 / 18.  Scoring 1,000 tokens at the 1B shape 16.9 -> 10.8 ms.
@@ -129,6 +131,11 @@ __device__ __forceinline__ float gs_repair(const unsigned char* P, const float* 
 
 template <int V>
 using GsInt = std::integral_constant<int, V>;
+using GsPlus = std::false_type;
+using GsMinus = std::true_type;
+__device__ __forceinline__ gs_f32x4 gs_signed(gs_f32x4 v, GsPlus) { return v; }
+__device__ __forceinline__ gs_f32x4 gs_signed(gs_f32x4 v, GsMinus) { return -v; }
+__device__ __forceinline__ gs_f32x4 gs_signed(gs_f32x4 v, uint32_t mask) { return __builtin_bit_cast(gs_f32x4, __builtin_bit_cast(gs_u32x4, v) ^ mask); }
 
 // MT x 16 rows by 8 x NT x 16 columns, eight wavefronts beside each other: each has all rows and 16 NT columns.  Stages of 32 of K: a ring of
 // RING of the rows' parts and one of RING - 1 of each wavefront's own columns.  One barrier a stage, in its middle: behind it the next
@@ -147,7 +154,9 @@ struct GsRope {
   int table_width, page_size, nh, nkv, hd, store;
 };
 
-template <int MT, int NT, int RING, int MODE>
+// PAIRS: every group of K is an even number of chunks of 128, and a stage's sign is known to the compiler.  Else it is a mask (for all groups:
+// 128 x 256 0.5 to 2 % slower; 200 rows of [3072, 3072] in 8 groups of three 32.3 -> 33.2 us).
+template <int MT, int NT, int RING, int MODE, bool PAIRS>
 __global__ void __launch_bounds__(512, 2)
     gemm_split_kernel(const unsigned char* __restrict__ P, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K, int ldc,
                       int steps_per_group, long long plane, int m_tiles, GsRope rope) {
@@ -200,12 +209,12 @@ __global__ void __launch_bounds__(512, 2)
     raw[j][0] = *reinterpret_cast<const gs_f32x4*>(lds + slot * B_STAGE + b_at + j * 2048 + slot0);
     raw[j][1] = *reinterpret_cast<const gs_f32x4*>(lds + slot * B_STAGE + b_at + j * 2048 + slot1);
   };
-  auto split_half = [&](gs_u32x4 (&to)[NT][3], int j, int x, auto negative) {
-    constexpr bool minus = decltype(negative)::value;
+  // sign: GsPlus, GsMinus or a mask of the sign's bit
+  auto split_half = [&](gs_u32x4 (&to)[NT][3], int j, int x, auto sign) {
     uint32_t h[2], m[2], l[2];
-    const gs_f32x4 v = raw[j][x];
-    gs_split(minus ? -v[0] : v[0], minus ? -v[1] : v[1], h[0], m[0], l[0]);
-    gs_split(minus ? -v[2] : v[2], minus ? -v[3] : v[3], h[1], m[1], l[1]);
+    const gs_f32x4 v = gs_signed(raw[j][x], sign);
+    gs_split(v[0], v[1], h[0], m[0], l[0]);
+    gs_split(v[2], v[3], h[1], m[1], l[1]);
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       to[j][0][2 * x + e] = h[e];
@@ -228,21 +237,22 @@ __global__ void __launch_bounds__(512, 2)
       for (int p = 0; p < 3; ++p)
         a[set][x][p] = *reinterpret_cast<const gs_u32x4*>(lds + slot * A_STAGE + ((g * TOGETHER + x) * 3 + p) * GS_FRAGMENT + lane * 16);
   };
-  auto add = [&](int g, auto negative) {
+  auto add = [&](int g, auto sign) {
 #pragma unroll
     for (int x = 0; x < TOGETHER; ++x)
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        if (decltype(negative)::value) total[g * TOGETHER + x][j] -= t[g * TOGETHER + x][j];
-        else total[g * TOGETHER + x][j] += t[g * TOGETHER + x][j];
+        total[g * TOGETHER + x][j] += gs_signed(t[g * TOGETHER + x][j], sign);
         t[g * TOGETHER + x][j] = gs_f32x4{0.f, 0.f, 0.f, 0.f};
       }
   };
+  const GsPlus plus;
+  const GsMinus minus;
   int a_slot = 0, b_slot = 1;                   // of this stage's rows and of the next one's columns
   // a stage; on entry its first rows' fragments and its columns' parts are in registers
-  auto stage = [&](int s, auto place_type, auto negative) {
+  // (next_sign: that of the next stage's columns, negated where their chunk is subtracted)
+  auto stage = [&](int s, auto place_type, auto sign, auto next_sign) __attribute__((always_inline)) {
     constexpr int place = decltype(place_type)::value, now = place & 1, next = now ^ 1;
-    using NextNegative = std::integral_constant<bool, decltype(negative)::value != (place == 3)>;
     const int slot = a_slot, slot1 = slot == RING - 1 ? 0 : slot + 1;
 #pragma unroll
     for (int g = 0; g < GROUPS; ++g) {
@@ -264,13 +274,13 @@ __global__ void __launch_bounds__(512, 2)
           for (int j = 0; j < NT; ++j)
             t[g * TOGETHER + x][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gs_bf16x8, b[now][j][first[p]]),
                                                                              __builtin_bit_cast(gs_bf16x8, a[set][x][second[p]]), t[g * TOGETHER + x][j], 0, 0, 0);
-      if (place == 3 && g > 0) add(g - 1, negative);
+      if (place == 3 && g > 0) add(g - 1, sign);
       // the next columns' parts beside the last products
 #pragma unroll
       for (int y = 0; y < 2 * NT; ++y)
-        if (g - HALF == y * (GROUPS - HALF) / (2 * NT)) split_half(b[next], y >> 1, y & 1, NextNegative{});
+        if (g - HALF == y * (GROUPS - HALF) / (2 * NT)) split_half(b[next], y >> 1, y & 1, next_sign);
     }
-    if (place == 3) add(GROUPS - 1, negative);
+    if (place == 3) add(GROUPS - 1, sign);
     a_slot = slot1;
     b_slot = b_slot == RING - 2 ? 0 : b_slot + 1;
   };
@@ -283,19 +293,39 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     read_raw(0, j);
-    split_half(b[0], j, 0, std::false_type{});
-    split_half(b[0], j, 1, std::false_type{});
+    split_half(b[0], j, 0, plus);
+    split_half(b[0], j, 1, plus);
   }
   read_a(0, 0, 0);
-  auto chunk = [&](int s, auto negative) {
-    stage(s, GsInt<0>{}, negative);
-    stage(s + 1, GsInt<1>{}, negative);
-    stage(s + 2, GsInt<2>{}, negative);
-    stage(s + 3, GsInt<3>{}, negative);
-  };
-  for (int s = 0; s < stages; s += 8) {
-    chunk(s, std::false_type{});
-    if (s + 4 < stages) chunk(s + 4, std::true_type{});
+  if constexpr (PAIRS) {
+    for (int s = 0; s < stages; s += 8) {
+      stage(s, GsInt<0>{}, plus, plus);
+      stage(s + 1, GsInt<1>{}, plus, plus);
+      stage(s + 2, GsInt<2>{}, plus, plus);
+      stage(s + 3, GsInt<3>{}, plus, minus);
+      if (s + 4 < stages) {      // (always: without a branch here the compiler mixes both chunks and 128 x 256 spills, 284 -> 387 us)
+        stage(s + 4, GsInt<0>{}, minus, minus);
+        stage(s + 5, GsInt<1>{}, minus, minus);
+        stage(s + 6, GsInt<2>{}, minus, minus);
+        stage(s + 7, GsInt<3>{}, minus, plus);
+      }
+    }
+  } else {
+    uint32_t sign = 0u;
+    const uint32_t flip = 0x80000000u;
+    for (int s = 0; s < stages; s += 4) {
+      const bool halves = s + 4 == stages && sign == 0u;      // the last one without a second
+      stage(s, GsInt<0>{}, sign, sign);
+      stage(s + 1, GsInt<1>{}, sign, halves ? flip : sign);
+      if (halves) {
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) add(g, plus);
+        sign = flip;
+      }
+      stage(s + 2, GsInt<2>{}, sign, sign);
+      stage(s + 3, GsInt<3>{}, sign, sign ^ flip);
+      sign ^= flip;
+    }
   }
 
   float* out = C + (size_t)blockIdx.y * plane;
@@ -407,9 +437,14 @@ __global__ void __launch_bounds__(512, 2)
   }
 }
 
-#define GS_RUN(MT, NT, RING, MODE, rope)                                                                                                          \
-  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, RING, MODE>), grid, block, 0, stream, (const unsigned char*)P, (const float*)W, (float*)C, M, N, K, \
-                     ldc, steps, (long long)M * N, m_tiles, rope)
+#define GS_LAUNCH(MT, NT, RING, MODE, PAIRS, rope)                                                                                          \
+  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, RING, MODE, PAIRS>), grid, block, 0, stream, (const unsigned char*)P, (const float*)W, (float*)C, \
+                     M, N, K, ldc, steps, (long long)M * N, m_tiles, rope)
+#define GS_RUN(MT, NT, RING, MODE, rope)                       \
+  do {                                                         \
+    if (K % 256 == 0 && steps % 8 == 0) GS_LAUNCH(MT, NT, RING, MODE, true, rope); \
+    else GS_LAUNCH(MT, NT, RING, MODE, false, rope);           \
+  } while (0)
 
 // P: the parts of A [M, K] (split_rows).  rows x columns: a block's tile, 128 or 64 by 256 or 128 (gated: gate and up columns
 // together, 256).  gated: 0, 1, or 2 for results that come as parts of rows of N columns, as split_rows makes them.  groups > 1: K in that many groups, C holds a plane of M * N for each (contiguous, ldc = N), which the reader adds up.
@@ -472,6 +507,7 @@ extern "C" int blm_gemm_split_qkv_rope(const void* P, const void* Wq, void* qkv_
     else GS_RUN(4, 1, 4, 3, rope);
   }
 #undef GS_RUN
+#undef GS_LAUNCH
   BLM_LAUNCH_CHECK("gemm_split_qkv_rope");
   return 0;
 }

@@ -102,6 +102,28 @@ def test_no_further_from_64_bits(K, groups, spread):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K,groups", [(128, 1), (256, 1), (384, 1), (640, 1), (1152, 1), (2560, 4), (3072, 8), (4224, 7), (11008, 8)])
+@pytest.mark.parametrize("positive", [False, True])
+def test_no_offset(K, groups, positive):
+    """What the matrix instruction cuts cancels in every group of K, odd numbers of chunks among them (4,224: of five, and of three in the last):
+    the mean of the errors is what so many independent ones leave, within five standard deviations, and their 2-norm no larger than the float
+    instructions'."""
+    from burn_lm_amd.csrc import ops
+    M, N = 300, 512
+    x, w = operands(M, N, K, seed=K + 1)
+    if positive:
+        x, w = x.abs(), w.abs()
+    want = x.double() @ w.double().t()
+    out = lambda: torch.empty(groups, M, N, device="cuda")
+    theirs = (ops.gemm_f32(x, w, out()).sum(0).double() - want).norm()
+    for tile in TILES:
+        planes = ops.gemm_split(ops.split_rows(x), w, out(), tile=tile)
+        err = planes.double().sum(0) - want                                  # (without the roundings of the planes' sum)
+        assert abs(float(err.mean())) <= 5 * float(err.std()) / (M * N) ** 0.5
+        assert (planes.sum(0).double() - want).norm() <= theirs
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("tile", TILES)
 def test_values_without_parts(tile):
     """Infinities, NaN and floats that round to an infinity as a bfloat16, in rows and in weights: what a sum of float products gives."""
