@@ -114,19 +114,12 @@ __device__ __forceinline__ unsigned char* gs_part_of(float* parts, int m, int n,
          n % GS_BK / 16 * 8 + n % 4 * 2;
 }
 
-// One element in float, from the floats themselves: where an operand is not finite (or rounds to an infinity as a bfloat16) its parts give NaN
-// (an infinity less itself, or times a part that is zero), which this replaces by what the sum is.
-__device__ __forceinline__ float gs_repair(const unsigned char* P, const float* w, int m, int steps_all, int s_begin, int stages) {
-  float sum = 0.f;
-  const unsigned char* tile = P + (size_t)(m / 16) * steps_all * (3 * GS_FRAGMENT) + (m % 16) * 16;
-  for (int s = s_begin; s < s_begin + stages; ++s)
-    for (int k = 0; k < GS_BK; ++k) {
-      const unsigned char* at = tile + (size_t)s * (3 * GS_FRAGMENT) + (k % 16 / 4) * 256 + (k / 16 * 4 + k % 4) * 2;
-      const float a = to_float(*reinterpret_cast<const bf16*>(at)) +
-                      (to_float(*reinterpret_cast<const bf16*>(at + GS_FRAGMENT)) + to_float(*reinterpret_cast<const bf16*>(at + 2 * GS_FRAGMENT)));
-      sum += a * w[(size_t)s * GS_BK + k];
-    }
-  return sum;
+// What a weight does to a sum's being a number: zeros, infinities and NaN as they are, all others 2^-100 with their sign (sums of so many rows'
+// first parts times these stay finite).
+__device__ __forceinline__ uint32_t gs_kind(float x) {
+  const uint32_t bits = __float_as_uint(x), top = bits & 0x7fffffffu;
+  if (top >= 0x7f800000u) return bits >> 16 | (top > 0x7f800000u ? 0x40u : 0u);
+  return top == 0u ? 0u : (bits >> 16 & 0x8000u) | 0x0d80u;
 }
 
 template <int V>
@@ -328,6 +321,107 @@ __global__ void __launch_bounds__(512, 2)
     }
   }
 
+  // Sums that are not numbers.  An operand that is not finite, or rounds to an infinity as a bfloat16, has made NaN of all its products (an infinity
+  // less itself, or times a part that is zero); also chunks may have overflowed in opposite directions.  The wavefront asks its rows' first parts and its
+  // columns' kinds, by the same instructions, which sums are infinities or NaN whatever the numbers among their operands, and leaves off as soon
+  // as all of them are NaN; what is left are sums of finite operands, which the float instructions add up, a tile of rows at a time.
+  // (us, 512 rows of [2048, 2048]: clean 127, all rows NaN 134, one NaN or infinity a row or a column 335, a weight a column that rounds to an infinity
+  // 900; with every such sum walked by the lane that has it 7,900 in all these cases.  Marked unlikely: in line the code cost a clean prompt 0.9 %.)
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) any |= total[i][j][e] != total[i][j][e];
+  if (__builtin_expect(__any(any), 0)) {
+    const float* w[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int n = GATED ? wave * 16 + l16 : wave * 16 * NT + j * 16 + l16;
+      w[j] = W + ((size_t)min(n0 + n, N - 1) + (GATED && j ? (size_t)N : 0)) * K + (size_t)s_begin * GS_BK + quad * 4;
+    }
+    const char* rows = a_base + lane * 16;
+    const size_t row_tile = (size_t)steps_all * (3 * GS_FRAGMENT);
+    auto number = [](float x) { return (__float_as_uint(x) & 0x7f800000u) != 0x7f800000u; };
+    for (int s = 0; s < stages; ++s) {
+      gs_u32x4 kind[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          const gs_f32x4 v = *reinterpret_cast<const gs_f32x4*>(w[j] + s * GS_BK + x * 16);
+          kind[j][2 * x] = gs_kind(v[0]) | gs_kind(v[1]) << 16;
+          kind[j][2 * x + 1] = gs_kind(v[2]) | gs_kind(v[3]) << 16;
+        }
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const gs_u32x4 first_part = *reinterpret_cast<const gs_u32x4*>(rows + min(i, row_tiles - 1) * row_tile + (size_t)s * (3 * GS_FRAGMENT));
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          t[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gs_bf16x8, kind[j]), __builtin_bit_cast(gs_bf16x8, first_part), t[i][j], 0, 0, 0);
+      }
+      if (s % 8 == 0) {
+        bool open = false;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) open |= total[i][j][e] != total[i][j][e] && t[i][j][e] == t[i][j][e];
+        if (!__any(open)) break;
+      }
+    }
+    uint32_t left = 0;           // tiles of rows
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      bool open = false;
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (total[i][j][e] != total[i][j][e]) {
+            if (number(t[i][j][e])) open = true;
+            else total[i][j][e] = t[i][j][e];
+          }
+      if (__any(open)) left |= 1u << i;
+    }
+    for (; left != 0; left &= left - 1) {
+      const int tile = __builtin_ctz(left);
+      const char* row = rows + min(tile, row_tiles - 1) * row_tile;
+      gs_f32x4 sum[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) sum[j] = gs_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+      for (int s = 0; s < stages; ++s) {
+        gs_u32x4 part[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) part[p] = *reinterpret_cast<const gs_u32x4*>(row + (size_t)s * (3 * GS_FRAGMENT) + p * GS_FRAGMENT);
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const gs_f32x4 v = *reinterpret_cast<const gs_f32x4*>(w[j] + s * GS_BK + x * 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int at = 2 * x + e / 2;
+              const float a = e % 2 ? gs_high(part[0][at]) + (gs_high(part[1][at]) + gs_high(part[2][at]))
+                                    : gs_low(part[0][at]) + (gs_low(part[1][at]) + gs_low(part[2][at]));
+              sum[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], a, sum[j], 0, 0, 0);
+            }
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        if (i == tile)
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (total[i][j][e] != total[i][j][e] && number(t[i][j][e])) total[i][j][e] = sum[j][e];
+    }
+  }
+
   float* out = C + (size_t)blockIdx.y * plane;
   // ROPE: where row m goes (columns of key and value heads of a row without a page go nowhere), and the angles of a lane's two pairs: asked for
   // for all rows at once, since behind the first store every look-up is a trip of its own
@@ -365,7 +459,6 @@ __global__ void __launch_bounds__(512, 2)
     return rope.vcache + (((size_t)page * rope.nkv + (head - rope.nh - rope.nkv)) * rope.hd + d) * rope.page_size + slot;
   };
   auto key_at = [&](int head, int d) { return rope.kcache + (((size_t)page * rope.nkv + (head - rope.nh)) * rope.page_size + slot) * rope.hd + d; };
-  unsigned long long odd = 0;              // elements that are not a number: bit (i * NT + j) * 4 + e, gated i * 4 + e
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int m = m0 + i * 16 + l16;
@@ -378,10 +471,7 @@ __global__ void __launch_bounds__(512, 2)
       const int n = n0 + wave * 16 * (GATED ? 1 : NT) + j * 16 + quad * 4;
       float v[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[e] = GATED ? gs_silu_times(total[i][0][e], total[i][NT - 1][e]) : total[i][j][e];
-        odd |= (unsigned long long)(v[e] != v[e]) << ((i * (GATED ? 1 : NT) + j) * 4 + e);
-      }
+      for (int e = 0; e < 4; ++e) v[e] = GATED ? gs_silu_times(total[i][0][e], total[i][NT - 1][e]) : total[i][j][e];
       if constexpr (ROPE) {
         if (m >= M || n >= N) continue;
         const int head = n / rope.hd, d = n - head * rope.hd;
@@ -406,33 +496,6 @@ __global__ void __launch_bounds__(512, 2)
       } else {
         if (m < M && n < N) *reinterpret_cast<float4*>(out + (size_t)m * ldc + n) = make_float4(v[0], v[1], v[2], v[3]);
       }
-    }
-  }
-  for (; odd != 0; odd &= odd - 1) {
-    const int at = __builtin_ctzll(odd), tile = at >> 2, i = GATED ? tile : tile / NT, j = GATED ? 0 : tile % NT;
-    const int m = m0 + i * 16 + l16, n = n0 + wave * 16 * (GATED ? 1 : NT) + j * 16 + quad * 4 + (at & 3);
-    if (m >= M || n >= N) continue;
-    if constexpr (ROPE) {      // with its partner, of which the turned one is made as well
-      const int pos = rope.positions[m];
-      slot = pos % rope.page_size;
-      page = page_of(rope.token_seq[m], pos);
-      const int head = n / rope.hd, d = (n - head * rope.hd) & ~1, first = n & ~1;
-      float x = gs_repair(P, W + (size_t)first * K, m, steps_all, s_begin, stages), y = gs_repair(P, W + (size_t)(first + 1) * K, m, steps_all, s_begin, stages);
-      if (head < rope.nh + rope.nkv) turn(angle(pos, d), x, y);
-      if (head >= rope.nh && page < 0) continue;
-      float* to = head < rope.nh ? out + (size_t)m * ldc + first : head < rope.nh + rope.nkv ? key_at(head, d) : value_at(head, d);
-      to[0] = x;
-      to[head < rope.nh + rope.nkv ? 1 : rope.page_size] = y;
-      continue;
-    }
-    float v = gs_repair(P, W + (size_t)n * K, m, steps_all, s_begin, stages);
-    if (GATED) v = gs_silu_times(v, gs_repair(P, W + (size_t)(N + n) * K, m, steps_all, s_begin, stages));
-    if constexpr (PARTS) {
-      uint32_t part[3];
-      gs_split_odd(v, part[0], part[1], part[2]);
-      for (int q = 0; q < 3; ++q) *reinterpret_cast<uint16_t*>(gs_part_of(C, m, n, N) + q * GS_FRAGMENT) = (uint16_t)part[q];
-    } else {
-      out[(size_t)m * ldc + n] = v;
     }
   }
 }

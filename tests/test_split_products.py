@@ -152,6 +152,76 @@ def test_values_without_parts(tile):
         assert torch.equal(gate.isneginf(), with_inf.float().isneginf())
 
 
+def sprinkled(M, N, K, what):
+    """Operands with values that are no finite number (or round to none as a bfloat16) in the places that `what` names."""
+    x, w = operands(M, N, K, seed=len(what))
+    w.mul_(2.0 ** -12)
+    g = torch.Generator().manual_seed(7)
+    at = lambda n: torch.randint(0, K, (n,), generator=g).cuda()
+    huge, sign = torch.finfo(torch.float32).max, lambda n: (torch.randint(0, 2, (n,), generator=g) * 2 - 1).float().cuda()
+    rows, columns = torch.arange(M, device="cuda"), torch.arange(N, device="cuda")
+    if what == "rows of NaN":
+        x[:] = NAN
+    elif what == "a NaN a row":
+        x[rows, at(M)] = NAN
+    elif what == "an infinity a row":
+        x[rows, at(M)] = INF * sign(M)
+    elif what == "a NaN a column":
+        w[columns, at(N)] = NAN
+    elif what == "an infinity a column":
+        w[columns, at(N)] = INF * sign(N)
+    elif what == "a huge weight a column":
+        x.mul_(2.0 ** -20)
+        w[columns, at(N)] = huge * sign(N)
+    else:      # some of each, and clean rows and columns between them
+        x.mul_(2.0 ** -20)
+        for k, v in enumerate((NAN, INF, -INF, huge, -huge, 0.0)):
+            x[17 * k + 3::101, 5 * k + 2] = v
+            w[29 * k + 1::97, 7 * k + 4] = v
+    return x, w
+
+
+SPRINKLED = ["rows of NaN", "a NaN a row", "an infinity a row", "a NaN a column", "an infinity a column", "a huge weight a column", "some of each"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", SPRINKLED)
+@pytest.mark.parametrize("tile,M,N,K", [((128, 256), 150, 528, 1024), ((64, 128), 300, 400, 384)])
+def test_sums_that_are_no_numbers(what, tile, M, N, K):
+    """NaN and infinities where a sum of float products has them, and numbers within their bound everywhere else."""
+    from burn_lm_amd.csrc import ops
+    x, w = sprinkled(M, N, K, what)
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    got = ops.gemm_split(ops.split_rows(x), w, torch.empty(M, N, device="cuda"), tile=tile)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isposinf(), want.float().isposinf()) and torch.equal(got.isneginf(), want.float().isneginf())
+    fine = want.isfinite() & (size < 1e38)
+    assert bool(((got.double() - want).abs()[fine] <= (K + 2) * 2.0 ** -24 * size[fine]).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", SPRINKLED)
+def test_sums_that_are_no_numbers_in_time(what):
+    """Such a product stays within a few times a clean one's time (where every sum was walked one lane at a time: some hundred times)."""
+    from burn_lm_amd.csrc import ops
+    M, N, K = 512, 2048, 2048
+
+    def us(x, w):
+        parts, out, times = ops.split_rows(x), torch.empty(M, N, device="cuda"), []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            ops.gemm_split(parts, w, out, tile=(128, 256))
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 1e3)
+        return sorted(times)[2]
+
+    clean, these = us(*operands(M, N, K)), us(*sprinkled(M, N, K, what))
+    print(f"{what}: {these:.0f} us, clean {clean:.0f}")
+    assert these < 16 * clean
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [200, 700])
 @pytest.mark.parametrize("K", [256, 2048, 2052, 4096])
