@@ -27,14 +27,6 @@ __device__ __forceinline__ bool af_visible(int key, int pos, int window) { retur
 template <int V>
 using AfInt = std::integral_constant<int, V>;
 
-// e^x of x <= 0 (and -infinity; NaN stays NaN): x log2(e) in two floats, the hardware's power of two of the first and the second's share of the
-// result as its derivative.  Within 2 ulps like expf, in 7 instructions instead of 13; what is below 2^-126 is zero.
-__device__ __forceinline__ float af_exp(float x) {
-  x = blm_max(x, -200.f);
-  const float h = x * 1.44269502f, l = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -h)), p = __builtin_amdgcn_exp2f(h);
-  return fmaf(p, l * 0.693147182f, p);
-}
-
 // Running softmax of one page: s[t][v] holds the scaled scores of this lane's query (l % 16) with keys 16 t + 4 (l / 16) + v,
 // -infinity where the query does not see the key; they become probabilities against the new maximum.  l is this lane's part
 // of the sum.  Returns the factor for what was summed before.
@@ -47,13 +39,13 @@ __device__ __forceinline__ float af_softmax(f32x4* s, float& m, float& l) {
     for (int v = 0; v < 4; ++v) top = fmaxf(top, s[t][v]);
   const float m_new = fmaxf(m, rows_max(top));
   const float base = m_new == -INFINITY ? 0.f : m_new;       // nothing seen yet: every probability is exp(-inf)
-  const float keep = af_exp(m - base);
+  const float keep = expf(m - base);
   float sum = 0.f;
 #pragma unroll
   for (int t = 0; t < TILES; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      s[t][v] = af_exp(s[t][v] - base);
+      s[t][v] = expf(s[t][v] - base);
       sum += s[t][v];
     }
   l = l * keep + sum;
@@ -104,8 +96,9 @@ __device__ void af_plain_query(const float* __restrict__ qrow, float* __restrict
 // Measured (us a layer, 32 heads of 64 in 8 groups; before: one wavefront per query and head on the vector units):
 // 1,000 tokens 844 -> 96.7; with the places in turns (in calls of their own) 1,000 tokens 104.7 -> 82.8, 2,048 299 -> 209, three sequences of 333 to
 // 1,201 and 24 heads of 128 232 -> 175, 500 tokens (one block a unit) 36.  A wavefront's pages then took 4.5 us each, of which the products are
-// 1.7; without a branch for every masked score and every staged piece, and with af_exp: 1,000 tokens 67.7, 2,048 165, the three sequences
-// 155, 500 tokens 27.2, 16 of 300 91 (104).  Two wavefronts for a unit, one on every other page: 83 -> 90, 500 tokens 35 -> 37.6, but 24 heads
+// 1.7; without a branch for every masked score and every staged piece: 1,000 tokens 71, 2,048 186, the three sequences
+// 166, 500 tokens 28.3, 16 of 300 92 (104).  An exponential by the hardware's power of two and a correction took 4 us less of the 1,000 tokens'
+// (66.8) and 20 of 2,048's; it was up to 2 ulps off where the library's is one, and zero below 2^-126.  Two wavefronts for a unit, one on every other page: 83 -> 90, 500 tokens 35 -> 37.6, but 24 heads
 // of 128 121 -> 92.
 // ---------------------------------------------------------------------------------------------------------------------
 template <int HD, bool FULL>     // HD: the head's lanes rounded up to 32, 64, 96 or 128; FULL: it has all of them

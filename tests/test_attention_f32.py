@@ -87,6 +87,27 @@ def test_prompts_of_many_places(lens, nh, nkv):
             check(got[cu[b] + t], qkv[cu[b] + t, : nh * hd].reshape(nh, hd), keys[b], values[b], t, hd ** -0.5, 0, group)
 
 
+@pytest.mark.parametrize("hd", [4, 64])
+def test_prompts_probabilities(hd):
+    """Every query sees one key with score zero, one with a score of its own and others that are out of sight, and the value of the second alone is one:
+    the result is the exponential, and an ulp is what the library promises for it, also where that is below 2^-126."""
+    from burn_lm_amd.csrc import ops
+    nh, n = 64, 64
+    g = torch.Generator().manual_seed(hd)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    q, keys, values = torch.zeros(n, (nh + 2) * hd), torch.zeros(PAGE, hd), torch.zeros(hd, PAGE)
+    score = -17.0 - 86.0 * torch.rand(n, nh, generator=g)
+    rows = q[:, : nh * hd].view(n, nh, hd)
+    rows[..., 0], rows[..., 1] = score, 1.0
+    keys[1, 0], keys[2:, 1], values[:, 1] = 1.0, -1e30, 1.0
+    out = torch.empty(n, nh * hd, device="cuda")
+    ops.attn_prefill_f32(q.cuda(), q.shape[1], out, i32(list(range(n))), i32([0, n]), i32([[0]]), keys[None, None].cuda(), values[None, None].cuda(), PAGE,
+                         1, n, nh, 1, hd, 1.0, 0)
+    got, want = out.cpu().view(n, nh, hd)[2:].double(), score[2:, :, None].double().exp()
+    ulp = torch.exp2(torch.floor(torch.log2(want)).clamp_min(-126.0) - 23)
+    assert bool(((got - want).abs() <= ulp).all()), float(((got - want).abs() / ulp).max())
+
+
 @pytest.mark.parametrize("splits", [1, 2, 5])
 @pytest.mark.parametrize("window", [0, 1, 70])
 @pytest.mark.parametrize("nh,nkv,hd", SHAPES)
