@@ -87,26 +87,37 @@ __device__ void af_plain_query(const float* __restrict__ qrow, float* __restrict
     if (lane + x * BLM_WAVE < hd) out[lane + x * BLM_WAVE] = acc[x] * (1.0f / l);
 }
 
+// The place, from the longest to the shortest, of block `at` of nkv heads' n blocks each; block at + nkv has the next place of its head.  A unit
+// starts with the blocks at and at + units, which is units / nkv places further: the second run of that many, whole or not, is turned round, so that the
+// longest has the shortest beside it.  What comes later starts as units become free, the longest first.
+// (us a layer, every second whole run of 32 turned, which is right for 8 key-value heads alone / this; heads of 64: 2,048 tokens of 16 heads without
+// groups 126 / 101, 1,000 of 32 / 32 67.6 / 55.7, of 32 / 4 66 / 54, of 32 / 8 (a second run of 31, which was not turned) 71 / 59.7, 3,000 of 32 / 16
+// 402 / 349, of 32 / 8 367 / 350, 2,048 of 32 / 8 186 / 186, of 32 / 4 173 / 174.5; every second run turned: 3,000 of 32 / 8 374, 2,048 of 32 / 4 180.
+// Behind another kernel, whose last blocks free the units one by one, 1,000 of 32 / 8 take 56.7 / 55.4.)
+__host__ __device__ __forceinline__ int af_place(int at, int n, int nkv, int units) {
+  const int place = at / nkv, run = units > nkv ? units / nkv : 1;
+  return place >= run && place < 2 * run ? run + min(n, 2 * run) - 1 - place : place;
+}
+
 // ---------------------------------------------------------------------------------------------------------------------
 // prompts.  A unit is sixteen queries of one head; a block's four wavefronts take neighbouring units of one key-value head
 // (the heads of its group at the same queries first), and every page that one of them sees is staged once, through registers
 // that hold the next page while this one is worked on.  Rows in shared memory are padded by four floats, so that the sixteen
-// rows of a fragment meet every bank.  The longest units start first, and every second run of 32 places of a key-value head goes from the
-// shortest to the longest: 512 blocks are on the 256 units at once, and a unit's two have 17 pages between them, not 2 to 32.
+// rows of a fragment meet every bank.  The longest units start first, those that share a compute unit with them from the shortest up (af_place):
+// 32 heads of 64 in 8 groups have 504 blocks for 1,000 tokens, and a unit's two have 17 pages between them, not 2 to 32.
 // Measured (us a layer, 32 heads of 64 in 8 groups; before: one wavefront per query and head on the vector units):
-// 1,000 tokens 844 -> 96.7; with the places in turns (in calls of their own) 1,000 tokens 104.7 -> 82.8, 2,048 299 -> 209, three sequences of 333 to
-// 1,201 and 24 heads of 128 232 -> 175, 500 tokens (one block a unit) 36.  A wavefront's pages then took 4.5 us each, of which the products are
-// 1.7; without a branch for every masked score and every staged piece: 1,000 tokens 71, 2,048 186, the three sequences
-// 166, 500 tokens 28.3, 16 of 300 92 (104).  An exponential by the hardware's power of two and a correction took 4 us less of the 1,000 tokens'
-// (66.8) and 20 of 2,048's; it was up to 2 ulps off where the library's is one, and zero below 2^-126.  Two wavefronts for a unit, one on every other page: 83 -> 90, 500 tokens 35 -> 37.6, but 24 heads
-// of 128 121 -> 92.
+// 1,000 tokens 844 -> 96.7; a key-value head's blocks on few dies, no branch for every masked score and every staged piece: 71, and 59.7 in that order (behind the projection 55.4)
+// (in the same steps 2,048 tokens 290 -> 186, three sequences of 333 to 1,201 and 24 heads of 128 231 -> 166, 500 tokens 35 -> 28.3, 16 of 300 109 -> 97).
+// An exponential by the hardware's power of two and a correction took 4 us less of 1,000 tokens and 20 of 2,048; it was up to 2 ulps off where the
+// library's is one, and zero below 2^-126.  Two wavefronts for a unit, one on every other page: 83 -> 90, 500 tokens 35 -> 37.6, but 24 heads of 128
+// 121 -> 92.
 // ---------------------------------------------------------------------------------------------------------------------
 template <int HD, bool FULL>     // HD: the head's lanes rounded up to 32, 64, 96 or 128; FULL: it has all of them
 __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
     attn_prefill_f32_kernel(const float* __restrict__ q, int q_row_stride, float* __restrict__ out,
                             const int* __restrict__ positions, const int* __restrict__ cu_seqlens,
                             const int* __restrict__ block_table, int table_width, const float* __restrict__ kcache,
-                            const float* __restrict__ vcache, int nh, int nkv, int hd, float scale, int window) {
+                            const float* __restrict__ vcache, int nh, int nkv, int hd, float scale, int window, int compute_units) {
   constexpr int KP = HD + 4, VP = AF_PAGE + 4, DS = HD / 16, PER = HD * AF_PAGE / 4 / (AF_WAVES * BLM_WAVE);
   __shared__ __attribute__((aligned(16))) float k_page[AF_PAGE * KP];
   __shared__ __attribute__((aligned(16))) float v_page[HD * VP];
@@ -117,9 +128,7 @@ __global__ void __launch_bounds__(AF_WAVES* BLM_WAVE, HD <= 64 ? 3 : 2)
   const int units = ((n_q + 15) / 16) * group;
   // consecutive blocks go to different dies: a die sees the pages of few key-value heads
   const int at = blockIdx.x + gridDim.x * blockIdx.y, kvh = at % nkv;
-  int place = at / nkv;
-  if ((place & 32) && (place | 31) < (int)gridDim.x) place ^= 31;
-  const int unit0 = ((int)gridDim.x - 1 - place) * AF_WAVES;
+  const int unit0 = ((int)gridDim.x - 1 - af_place(at, gridDim.x, nkv, compute_units)) * AF_WAVES;
   if (unit0 >= units) return;
   const int unit = min(unit0 + wave, units - 1);
   const bool active = unit0 + wave < units;
@@ -421,16 +430,18 @@ static int attn_f32_check(const char* name, const void* q, int q_row_stride, con
   return 0;
 }
 
+extern "C" int blm_attn_prefill_f32_place(int at, int blocks, int nkv, int compute_units) { return af_place(at, blocks, nkv, compute_units); }
+
 extern "C" int blm_attn_prefill_f32(const void* q, int q_row_stride, void* out, const int* positions, const int* cu_seqlens,
                                     const int* block_table, int table_width, const void* kcache, const void* vcache, int n_seqs,
-                                    int max_new, int nh, int nkv, int hd, float scale, int window, hipStream_t stream) {
+                                    int max_new, int nh, int nkv, int hd, float scale, int window, int compute_units, hipStream_t stream) {
   if (attn_f32_check("attn_prefill_f32", q, q_row_stride, kcache, vcache, nh, nkv, hd, table_width, window)) return 1;
   const long long blocks = ((long long)(max_new + 15) / 16 * (nh / nkv) + AF_WAVES - 1) / AF_WAVES;
-  BLM_REQUIRE(n_seqs > 0 && n_seqs <= 65535 && max_new > 0 && nkv <= 65535 && blocks < 2147483647LL, "attn_prefill_f32: bad sizes");
+  BLM_REQUIRE(n_seqs > 0 && n_seqs <= 65535 && max_new > 0 && nkv <= 65535 && blocks < 2147483647LL && compute_units > 0, "attn_prefill_f32: bad sizes");
   dim3 grid((unsigned)blocks, (unsigned)nkv, (unsigned)n_seqs), block(AF_WAVES * BLM_WAVE);
 #define BLM_AFP(HD, FULL)                                                                                                             \
   hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, FULL>), grid, block, 0, stream, (const float*)q, q_row_stride, (float*)out, positions, \
-                     cu_seqlens, block_table, table_width, (const float*)kcache, (const float*)vcache, nh, nkv, hd, scale, window)
+                     cu_seqlens, block_table, table_width, (const float*)kcache, (const float*)vcache, nh, nkv, hd, scale, window, compute_units)
   if (hd == 32) BLM_AFP(32, true);
   else if (hd < 32) BLM_AFP(32, false);
   else if (hd == 64) BLM_AFP(64, true);

@@ -11,7 +11,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 49
+ABI_VERSION = 50
 _lib = None
 _lock = threading.Lock()
 
@@ -125,7 +125,8 @@ _SIGNATURES = {
                        _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p],
     "blm_attn_f32_supported": [_c_int, _c_int],
     "blm_attn_prefill_f32": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int,
-                             _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_void_p],
+                             _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void_p],
+    "blm_attn_prefill_f32_place": [_c_int] * 4,
     "blm_attn_decode_f32": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int,
                             _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p],
     "blm_attn_decode": [_c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int,
@@ -484,8 +485,13 @@ def attn_prefill_f32(q, q_row_stride, out, positions, cu_seqlens, block_table, k
         raise KernelError("attn_prefill_f32: the page table has fewer rows than there are sequences")
     _call("blm_attn_prefill_f32", q.data_ptr(), q_row_stride, out.data_ptr(), positions.data_ptr(), cu_seqlens.data_ptr(),
           block_table.data_ptr(), block_table.shape[1], kcache.data_ptr(), vcache.data_ptr(), int(n_seqs), int(max_new), nh, nkv, hd,
-          float(scale), int(window), _stream())
+          float(scale), int(window), compute_units(q.device.index), _stream())
     return out
+
+
+def attn_prefill_f32_place(at, blocks, nkv, units):
+    """Which of its head's places, from the longest to the shortest, block `at` of nkv heads' blocks has on that many compute units."""
+    return library().blm_attn_prefill_f32_place(int(at), int(blocks), int(nkv), int(units))
 
 
 def attn_decode_f32(q, q_row_stride, out, positions, token_seq, block_table, kcache, vcache, page_size, nh, nkv, hd, scale, window=0,
