@@ -26,7 +26,7 @@ import math
 import numpy as np
 import torch
 
-from .base import PositionEncoding, Unscaled
+from .base import PositionEncoding, Unscaled, speaks_for
 
 PAIRING = {"interleaved": 0, "half": 1}
 
@@ -129,10 +129,14 @@ class RotaryEncoding(PositionEncoding):
                                   view.k, view.v, view.page_size, heads, kv_heads, head_dim, self.pairing,
                                   write_kv=store)
 
+    def _asks_linear(self):
+        """Whether the runtime brings a linear of its own without a plan for projections beside it: it is called by that for every projection."""
+        return hasattr(type(self.rt), "linear") and not speaks_for(self.rt, "qkv_plan", "linear")
+
     def takes_unscaled(self, tokens, w_qkv, heads, kv_heads, head_dim):
         """The packed kernels of few rows do, bfloat16 and float32."""
         rt = self.rt
-        if not hasattr(rt, "qkv_takes_unscaled") or self.pairing != PAIRING["interleaved"]:
+        if not hasattr(rt, "qkv_takes_unscaled") or self.pairing != PAIRING["interleaved"] or self._asks_linear():
             return False
         return rt.qkv_takes_unscaled(tokens, w_qkv, head_dim)
 
@@ -150,7 +154,9 @@ class RotaryEncoding(PositionEncoding):
         bf16 = x.dtype == view.k.dtype == torch.bfloat16 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
         raw, packable = getattr(w_qkv, "w", None), getattr(w_qkv, "packable", False)
         fused = None
-        if (plan is not None and plan.kernel == "rows" and bf16 and self.pairing == PAIRING["interleaved"]
+        if self._asks_linear():
+            pass
+        elif (plan is not None and plan.kernel == "rows" and bf16 and self.pairing == PAIRING["interleaved"]
                 and raw is not None and raw.dtype == torch.bfloat16 and raw.is_contiguous()
                 and head_dim % 2 == 0 and K % 8 == 0 and x.stride(1) == 1):
             fused = "rows"
