@@ -659,7 +659,7 @@ SPLIT_TILES = ((128, 256), (128, 128), (64, 256), (64, 128))
 
 def split_takes(M, N, K, gated=False):
     """Whether gemm_split has these sizes (its rows and weights as f32_rows wants them)."""
-    return M > 0 and K % 128 == 0 and N % 16 == 0 and (not gated or (N + 256) * K * 4 < 1 << 32)
+    return M > 0 and K % 128 == 0 and N % 16 == 0 and ((N if gated else 0) + 256) * K * 4 < 1 << 32
 
 
 def _parts(M, K, device):

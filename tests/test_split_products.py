@@ -326,6 +326,9 @@ def test_plan_keeps_its_bounds():
     for K in (4, 130, 2052):
         assert split_plan(100, 64, K, 256) is None
     assert split_plan(100, 60, 256, 256) is None
+    # lanes' offsets into the weights are 32 bits: 256 columns of 2^22, and of the gated product all gate columns besides
+    assert split_plan(100, 16, 1 << 22, 256) is None and split_plan(100, 16, (1 << 22) - 128, 256) is not None
+    assert split_plan(100, 1 << 19, 2048, 256, gated=True) is None and split_plan(100, 1 << 19, 2048, 256) is not None
     for M in (17, 65, 1000):
         for N in (16, 2048, 5008):
             for K in (128, 1152, 2176, 4224, 8192):
