@@ -2,12 +2,14 @@
 // float ones: a float is the sum of three bfloat16 (hi, mid, lo, rounded to nearest each: 8 + 8 + 8 bits and their signs, the subtractions
 // between them exact), a product of two floats the sum of nine exact products, and the three that are left out (mid lo, lo mid, lo lo)
 // are below 2^-26 of the whole (floats below 2^-110 have no lo of their own: what is lost of them is below 2^-134).  Six instructions
-// of 16 cycles do 16 x 16 x 32, for which the float ones take 256 cycles.
+// of 16 cycles do 16 x 16 x 32, for which the float ones take 256 cycles.  (Floats as sums of three bfloat16: Henry, Tang and Heinecke, "Leveraging
+// the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", ARITH 2019.)
 //   split_rows : the parts of the rows, in the order of the instruction's fragments
 //   gemm_split : the product; the weights, which are not kept a second time, are split on their way from shared memory
-// What bounds it: the matrix instructions at the clock that the card's power leaves (1.25 to 1.35 PFLOP/s of them), beside them reads of
-// shared memory (a fragment of three parts serves six or twelve instructions) and the splitting: 88 vector instructions for 192
-// matrix ones at 128 x 256.  Every wavefront has all rows of the tile and columns of its own, so that no weight is split twice in a block.
+// What bounds it: the matrix instructions at the clock that the card's power leaves (1.3 to 1.4 PFLOP/s of them), beside them reads of
+// shared memory (a fragment of three parts serves six or twelve instructions), the splitting, 88 vector instructions (104 where a chunk is negated)
+// for a stage's 96 matrix ones at 128 x 256, and a chunk's 64 additions.  Every wavefront has all rows of the tile and columns of its own, so that
+// no weight is split twice in a block.
 // Sums: the matrix instruction adds to its accumulator with what falls off below cut, towards minus infinity: a result of 2,048 products by
 // one accumulator is 2.7e-7 off and, the same in all of them, 3e-8 too low, which adds up from layer to layer (logits of the 1B shape
 // 3.7e-6 from 64 bits, with the float instructions 2.8e-6).  So a chunk of 128 of K has an accumulator that starts at zero, small products
@@ -15,8 +17,8 @@
 // cut cancels: 1.7e-7 off (2.17e-7 with the float instructions), 7e-11 too low, and the logits 2.6e-6.  It cancels in pairs, so a group of K with
 // an odd number of chunks has its last one in two halves of opposite sign (mean error of normal operands, without / with: K = 128 -8e-9 / 1e-10,
 // 640 -4e-9 / -3e-10, 3,072 in 8 groups of three -1.4e-8 / 0; 2-norms 1.52 / 0.97, 1.59 / 1.52, 1.64 / 1.50e-7, the float instructions' 2.0 to 2.1).
-// Measured (us, the float instructions' best tile and groups / this, without the parts' pass of 3.5 to 5 us, with K = 8,192 14; weights from memory),
-// 1,000 rows: [16384, 2048] gated 502 / 284 (236 TFLOP/s of float products), [2048, 8192] 259 / 157, [3072, 2048] 105 / 75, [2048, 2048] 72 / 47;
+// Measured (us, the float instructions' best tile and groups / this, without the parts' pass of 2.7 to 6 us, with K = 8,192 14; weights from memory),
+// 1,000 rows: [16384, 2048] gated 502 / 284 (236 TFLOP/s of float products, 1.42 PFLOP/s; cards differ, up to 300), [2048, 8192] 259 / 157, [3072, 2048] 105 / 75, [2048, 2048] 72 / 47;
 // 256 rows 137 / 90, 74 / 50, 33 / 26, 24 / 18.  Scoring 1,000 tokens at the 1B shape 16.9 -> 10.8 ms.
 // The ring is as deep as the weights' way from memory asks: with the next two stages under way tiles of 64 rows, whose stages are short, took 1.34 us
 // a stage for the 64 x 128, with three 0.70 (1.2 and 1.13 for 64 x 256; four and five: as three).

@@ -85,6 +85,27 @@ def test_pair(M, I, K, N):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,I,K,N", [(331, 4096, 1024, 1024), (200, 4992, 1152, 1152), (497, 4992, 1152, 1152), (1001, 2176, 1024, 512)])
+def test_pair_by_parts(M, I, K, N, monkeypatch):
+    """Sizes at which the first product does leave parts, rows that end inside a tile and inner sizes of an odd number of chunks among them: as above,
+    also with a row of no numbers, which is one in the result and none of the others."""
+    from burn_lm_amd.csrc import ops
+    from burn_lm_amd.engine.runtime import Runtime
+    left, parts = [], ops.gemm_split_parts
+    monkeypatch.setattr(ops, "gemm_split_parts", lambda *a, **k: left.append(1) or parts(*a, **k))
+    rt = Runtime(torch.float32, "cuda:0")
+    x, w = operands(M, 2 * I, K, pad=4)
+    _, down = operands(1, N, I)
+    x[M - 2] = NAN
+    got = rt.gated_pair(x, rt.weight(w, gated=True), rt.weight(down))
+    assert left == [1]
+    got, mid = got.sum(0) if got.dim() == 3 else got, rt.gated_linear(x, w)
+    assert bool(got[M - 2].isnan().all())
+    rest = torch.arange(M, device="cuda") != M - 2
+    check(got[rest], mid[rest], down)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("K,groups", [(2048, 1), (2048, 4), (8192, 1), (8192, 4)])
 @pytest.mark.parametrize("spread", [0.0, 2.0])
 def test_no_further_from_64_bits(K, groups, spread):
