@@ -48,9 +48,14 @@ struct GrRope {
 
 #define GR_MAX_ROWS 256   // four blocks of 64 rows
 
-// Weights from this size on, where one block reads each of them, are loaded past the caches, which keep the rows that every block reads.
-// Measured with weights from memory, 64 / 32 rows, us: [16384, 2048] (67 MB) gated 17.7 / 16.1 -> 16.7 / 15.1, [2048, 8192] (34 MB) in groups
-// 11.2 -> 10.9 (32 rows); [3072, 2048] and [2048, 2048] (8 to 13 MB) are the same either way, and models of such sizes may fit the last-level cache.
+// Weights from this size on, where one block reads each of them, are loaded past the caches, which keep the rows that every block reads.  That is
+// worth little while matrices are small and costs much where a model's weights fit the last-level cache (256 MB), as none with layers of such
+// matrices does: the bound is an eighth of it.
+// us at 64 / 32 rows, through the caches -> past them, weights from memory (and from the last-level cache): 12.6 MB [3072, 2048] 6.55 / 5.44 -> 6.50 /
+// 5.41 (5.4 / 4.4 -> 5.9 / 5.0); 21 MB [5120, 2048] 10.2 / 9.0 -> 10.0 / 8.9 (7.5 / 6.0 -> 9.4 / 7.7); 25 MB [2048, 6144] 9.3 / 7.7 -> 9.2 / 7.5
+// (7.5 / 6.3 -> 8.2 / 6.7); 29 MB [7168, 2048] 11.5 / 9.6 -> 11.3 / 9.5 (8.3 / 6.7 -> 9.8 / 8.7); 34 MB [2048, 8192] 12.0 / 10.1 -> 11.6 / 9.8 (9.1 / 7.8 -> 10.3 /
+// 8.7), [8192, 2048] 12.3 / 10.4 -> 12.0 / 10.1; 50 MB [3072, 8192] 17.5 / 14.3 -> 17.1 / 13.7, gated [12288, 2048] 16.4 / 13.9 -> 16.1 / 13.4; 67 MB gated
+// [16384, 2048] 18.7 / 18.0 -> 18.0 / 16.8 (13.3 / 12.6 -> 16.6 / 15.2); 101 MB gated [16384, 3072] 24.5 / 22.0 -> 23.6 / 20.8.
 #define GR_ONCE_BYTES ((size_t)32 << 20)
 
 template <int BM, int BN, int BK, int R, int MODE, typename TC>

@@ -31,8 +31,8 @@ def decode_splits(pages: int, blocks: int, head_dim: int, compute_units: int = 2
     one per compute unit: a second, partial round costs more than longer pieces do (us per call at a
     context of 4,096, blocks in brackets; heads of 64, batch 6: 4 pieces (192) 13.8, 5 (240) 14.0, 6 (288)
     16.2, 8 (384) 14.9, 10 (480) 14.5; batch 10: 3 (240) 18.5, 4 (320) 21.2, 6 (480) 18.9, 7 (560) 21.5;
-    batch 24: whole (192) 32.3, 3 (576) 41.6; heads of 128, whose blocks fill a compute unit's shared
-    memory alone: batch 10: 3 (240) 32.8, 4 (320) 44.0; batch 20: whole (160) 54.0, 2 (320) 71.9; the
+    batch 24: whole (192) 32.3, 3 (576) 41.6; 24 heads of 128 in 8 groups, whose blocks fill a compute unit's
+    shared memory alone: batch 10: 3 (240) 33.0, 4 (320) 41.6; batch 20: whole (160) 57.9, 2 (320) 72.2; the
     same at contexts of 2,048 and 16,384).
     Measured at context 4096, head_dim 64, ms per step: batch 1: 16 pieces 0.870, 8: 0.880, 64: 1.002;
     batch 2: 8 pieces 0.909, 16: 0.928; batch 4: 8 pieces 0.961, 16: 0.988; batch 8: 4 and 8 pieces equal.
@@ -44,17 +44,19 @@ def decode_splits(pages: int, blocks: int, head_dim: int, compute_units: int = 2
     wavefront and (for heads up to 64) three: a merge costs three trips through device-coherent memory in a
     row, about 3 us, a further page per wavefront about 2 (us per call, cut in two / uncut, 32 heads of 64
     in 8 groups: 8 pages at batch 1 7.1 / 6.6, at batch 8 8.1 / 7.0; 11 pages 7.9 / 8.0 and 9.0 / 8.4;
-    16 pages, cut in four, 7.3 / 10.2; heads of 128: 8 pages 11.1 / 11.1, 11 pages 12.8 / 13.7).  Where a
+    16 pages, cut in four, 7.3 / 10.2; 24 heads of 128 in 8 groups: 8 pages at batch 1 9.7 / 9.3, at batch 8 10.7 / 10.5).  Where a
     range is cut although the blocks are few, it is cut down to two pages per piece, not four (one
-    compute unit brings a page of wide heads, 32 KB, no faster than 60 GB/s: heads of 128 at batch 1,
-    11 pages: 2 pieces 13.0, uncut 11.1, 6 pieces 10.4; 16 pages: 4 pieces 12.1, 8 pieces 10.7; heads of 64,
+    compute unit brings a page of wide heads, 32 KB, no faster than 60 GB/s: these heads of 128 at batch 1,
+    11 pages: 2 pieces 11.0, uncut 11.5, 6 pieces 8.2; 16 pages: 4 pieces 9.9, 8 pieces 8.5; heads of 64,
     16 pages: 4 pieces 7.9, 8 pieces 7.3), and ranges of up to 16 pages stay whole from a block for every
-    fourth compute unit on (heads of 128, 11 pages at batch 8: uncut 12.3, in two 14.0; 16 pages at batch
-    16: 16.9 / 18.5; heads of 64, 16 pages at batch 8: 9.1 / 10.0).  Longer ranges of wide heads go down to one page per wavefront
+    fourth compute unit on (heads of 64, 16 pages at batch 8: uncut 9.1, in two 10.0; for heads of 128 it was so with a merge of a dim a
+    thread, and is not with four: 11 pages at batch 8 12.1 / 12.1, in three 11.4; 16 pages at batch 16 18.0 / 17.1).  Longer ranges of wide heads go down to one page per wavefront
     while the pieces still run in one round and are no more than eight, beyond which their merge costs more than they save (16 heads of
     128 in 4 groups, pieces by the rules above / by this one: 8 sequences of 18 pages 4 / 5 pieces 12.0 / 11.1, 24 pages 4 / 6 12.2 /
-    11.9, 32 pages 4 / 8 13.2 / 13.3; 16 sequences of 18 pages 2 / 4 15.6 / 14.0, 24 pages 3 / 4 15.2 / 15.4; in 8 groups, 8 sequences
-    of 18 pages 2 / 4 17.2 / 15.6; but in 4 groups 4 sequences of 64 pages 8 / 16 13.8 / 14.7, 2 of 100 pages 16 / 25 13.2 / 14.3)."""
+    11.9, 32 pages 4 / 8 13.3 / 13.4, 48 pages 6 / 8 15.2 / 15.5; 16 sequences of 18 pages 2 / 4 14.5 / 13.9, 24 pages 3 / 4 14.8 / 15.0; 4 sequences
+    of 24 pages 4 / 8 11.9 / 10.5; in 8 groups, 8 sequences of 18 pages 2 / 4 14.9 / 14.2, 24 pages 3 / 4 15.5 / 15.5, 4 of 24 pages 3 / 6 13.5 / 12.0; so up
+    to 8 % faster at 18 to 24 pages and 1 to 2 % slower at some longer ranges; in 4 groups 4 sequences of 64 pages 8 / 16 14.2 / 14.7, 2 of 100 pages
+    16 / 25 13.0 / 14.3)."""
     if blocks >= compute_units or pages <= (12 if head_dim <= 64 else 8):
         return 1
     if pages <= 16 and blocks * 4 >= compute_units:
