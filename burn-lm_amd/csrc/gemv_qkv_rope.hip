@@ -164,7 +164,22 @@ __global__ void __launch_bounds__(512)
   if (!store && tile >= nh * tiles_per_head) return;   // keys and values belong to another layer's cache: only q is needed
   const int step0 = wave * QR_KSTEPS;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+  const int head = tile / tiles_per_head, col0 = (tile - head * tiles_per_head) * 16;
+  // a thread's output of the tile: row m, column c
+  auto row_of = [&](int idx) { return ((idx & 63) >> 4) * 4 + ((idx >> 6) & 3); };
+  int pos, b, page = -1;
+  float2 cs = make_float2(1.f, 0.f);     // value heads are stored as they are
+  auto ask = [&](int idx) {
+    const int m = min(row_of(idx), M - 1);
+    pos = positions[m];
+    b = token_seq[m];
+  };
+  auto ask_more = [&](int idx) {
+    if (head < nh + nkv) cs = cos_sin[(size_t)pos * (hd / 2) + ((col0 + (idx & 15)) >> 1)];
+    if (head >= nh && b >= 0) page = block_table[(size_t)b * table_width + pos / page_size];
+  };
 
+  ask(threadIdx.x);
   if (SCALED) scale_load.ask(sums, n_sums, M, wave, n_waves, lane);
   const bf16* wt = Wp + ((size_t)tile * k_steps * 64 + lane) * 8;
   uint4 w[QR_KSTEPS];
@@ -173,6 +188,9 @@ __global__ void __launch_bounds__(512)
     const int st = step0 + s;
     w[s] = load16_stream(wt + (size_t)(st < k_steps ? st : k_steps - 1) * 512);   // the weights: read once
   }
+  __builtin_amdgcn_sched_barrier(0);
+  ask_more(threadIdx.x);
+  __builtin_amdgcn_sched_barrier(0);
   const bf16* ap = A + (size_t)(row < M ? row : M - 1) * lda;
   uint4 a[QR_KSTEPS];
 #pragma unroll
@@ -193,10 +211,13 @@ __global__ void __launch_bounds__(512)
   __syncthreads();
 
   // epilogue: one thread per (token row m, column c of the tile)
-  const int head = tile / tiles_per_head, col0 = (tile - head * tiles_per_head) * 16;
   for (int idx = threadIdx.x; idx < 256; idx += n_waves * BLM_WAVE) {
-    const int r = idx >> 6, l2 = idx & 63, c = l2 & 15;
-    const int m = (l2 >> 4) * 4 + r;
+    const int c = idx & 15, m = row_of(idx);
+    if (idx != threadIdx.x) {      // fewer than four wavefronts
+      page = -1;
+      ask(idx);
+      ask_more(idx);
+    }
     if (m >= M) continue;
     float x = 0.f, partner = 0.f;   // column c and its neighbour c ^ 1
     for (int k2 = 0; k2 < n_waves; ++k2) {
@@ -207,21 +228,14 @@ __global__ void __launch_bounds__(512)
       x *= inv[m];
       partner *= inv[m];
     }
-    const int b = token_seq[m];
-    const int pos = positions[m];
     const int d = col0 + c;
-    float y = x;     // value heads are stored as they are
-    if (head < nh + nkv) {
-      const float2 cs = cos_sin[(size_t)pos * (hd / 2) + (d >> 1)];
-      y = turned(x, partner, cs, c);
-    }
+    float y = x;
+    if (head < nh + nkv) y = turned(x, partner, cs, c);
     const bf16 o = from_float<bf16>(y);
     if (head < nh) {
       qkv_out[(size_t)m * ldq + (size_t)head * hd + d] = o;
-    } else if (b >= 0) {
-      const int page = block_table[(size_t)b * table_width + pos / page_size];
+    } else if (page >= 0) {
       const int slot = pos % page_size;
-      if (page < 0) continue;
       if (head < nh + nkv) kcache[(((size_t)page * nkv + (head - nh)) * page_size + slot) * hd + d] = o;
       else vcache[((size_t)page * nkv + (head - nh - nkv)) * hd * page_size + (size_t)d * page_size + slot] = o;
     }
