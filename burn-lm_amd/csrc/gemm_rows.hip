@@ -48,9 +48,10 @@ struct GrRope {
 
 #define GR_MAX_ROWS 256   // four blocks of 64 rows
 
-// Weights from this size on, where one block reads each of them, are loaded past the caches, which keep the rows that every block reads.  That is
-// worth little while matrices are small and costs much where a model's weights fit the last-level cache (256 MB), as none with layers of such
-// matrices does: the bound is an eighth of it.
+// Weights from this size on, where one block reads each of them and the caller says that they come from memory (once), are loaded past the caches,
+// which keep the rows that every block reads.  That is worth little while matrices are small and costs much where a model's weights stay in the
+// last-level cache (256 MB) from step to step.  (Decode steps of 24 to 64 sequences: layers of the 1B shape, 122 MB each, one 173 -> 177 us, two 222 -> 227,
+// three 289 -> 276; of the 3B shape, 201 MB, one 238 -> 243, two 330 -> 312.)
 // us at 64 / 32 rows, through the caches -> past them, weights from memory (and from the last-level cache): 12.6 MB [3072, 2048] 6.55 / 5.44 -> 6.50 /
 // 5.41 (5.4 / 4.4 -> 5.9 / 5.0); 21 MB [5120, 2048] 10.2 / 9.0 -> 10.0 / 8.9 (7.5 / 6.0 -> 9.4 / 7.7); 25 MB [2048, 6144] 9.3 / 7.7 -> 9.2 / 7.5
 // (7.5 / 6.3 -> 8.2 / 6.7); 29 MB [7168, 2048] 11.5 / 9.6 -> 11.3 / 9.5 (8.3 / 6.7 -> 9.8 / 8.7); 34 MB [2048, 8192] 12.0 / 10.1 -> 11.6 / 9.8 (9.1 / 7.8 -> 10.3 /
@@ -307,14 +308,14 @@ static int gr_prepare() {
 }
 
 template <int BM, int BN, int BK, int R, int MODE, typename TC>
-static int gr_launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int k_groups,
+static int gr_launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int k_groups, int from_memory,
                      hipStream_t stream, GrRope rope = GrRope{}) {
   constexpr size_t smem = (size_t)4 * R * (BM + BN) * BK * sizeof(bf16);
   static_assert(smem >= (size_t)4 * BM * (BN + 4) * sizeof(float), "the partial tiles fit where the ring was");
   const int n_tiles = (N + (MODE == 1 ? BN / 2 : BN) - 1) / (MODE == 1 ? BN / 2 : BN);
   const int k_per_group = ((K + k_groups - 1) / k_groups + BK - 1) / BK * BK;
   dim3 grid((unsigned)n_tiles, (unsigned)k_groups, (unsigned)((M + BM - 1) / BM)), block(256);
-  const int once = grid.z == 1 && (size_t)(MODE == 1 ? 2 : 1) * N * ldw * sizeof(bf16) >= GR_ONCE_BYTES;
+  const int once = from_memory && grid.z == 1 && (size_t)(MODE == 1 ? 2 : 1) * N * ldw * sizeof(bf16) >= GR_ONCE_BYTES;
   hipLaunchKernelGGL((gemm_rows_kernel<BM, BN, BK, R, MODE, TC>), grid, block, smem, stream, (const bf16*)A, (const bf16*)W, (TC*)C, M,
                      N, K, lda, ldw, ldc, k_per_group, once, rope);
   BLM_LAUNCH_CHECK("gemm_rows");
@@ -338,7 +339,7 @@ extern "C" int blm_gemm_rows_init() {
 // for the gated product from 33 rows on and for partial planes (32 columns when that still gives every
 // compute unit a block, else 64) at all of them.
 extern "C" int blm_gemm_rows(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc,
-                             int mode, int k_groups, int columns, hipStream_t stream) {
+                             int mode, int k_groups, int columns, int once, hipStream_t stream) {
   BLM_REQUIRE(M >= 1 && M <= GR_MAX_ROWS && N >= 1 && K >= 8 && K % 8 == 0,
               "gemm_rows: sizes M=%d N=%d K=%d not supported (M <= %d, K a multiple of 8)", M, N, K, GR_MAX_ROWS);
   BLM_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K && ldc >= N, "gemm_rows: bad strides lda=%d ldw=%d ldc=%d", lda, ldw, ldc);
@@ -351,8 +352,8 @@ extern "C" int blm_gemm_rows(const void* A, const void* W, void* C, int c_dtype,
   BLM_REQUIRE((size_t)64 * lda * 2 < ((size_t)1 << 32) && (size_t)(mode == 1 ? 2 : 1) * N * ldw * 2 < ((size_t)1 << 32),
               "gemm_rows: matrices of 4 GiB and more are not supported (lda=%d, N=%d, ldw=%d)", lda, N, ldw);
 #define GR_GO(BM, BN, R, MODE)                                                                                       \
-  return c_dtype == BLM_BF16 ? gr_launch<BM, BN, 64, R, MODE, bf16>(A, W, C, M, N, K, lda, ldw, ldc, k_groups, stream) \
-                             : gr_launch<BM, BN, 64, R, MODE, float>(A, W, C, M, N, K, lda, ldw, ldc, k_groups, stream)
+  return c_dtype == BLM_BF16 ? gr_launch<BM, BN, 64, R, MODE, bf16>(A, W, C, M, N, K, lda, ldw, ldc, k_groups, once, stream) \
+                             : gr_launch<BM, BN, 64, R, MODE, float>(A, W, C, M, N, K, lda, ldw, ldc, k_groups, once, stream)
   // up to 32 rows: half the rows staged, and a deeper ring in the room that leaves
   if (mode == 1) {
     if (M > 32) GR_GO(64, 64, 2, 1);
@@ -377,7 +378,7 @@ extern "C" int blm_gemm_rows(const void* A, const void* W, void* C, int c_dtype,
 extern "C" int blm_gemm_rows_qkv_rope(const void* A, const void* W, void* qkv_out, const int* positions, const int* token_seq,
                                       const int* block_table, int table_width, const float* cos_sin, void* kcache, void* vcache,
                                       int page_size, int M, int K, int lda, int ldw, int ldq, int nh, int nkv, int hd, int store,
-                                      int columns, int rows, hipStream_t stream) {
+                                      int columns, int rows, int once, hipStream_t stream) {
   BLM_REQUIRE(columns == 32 || columns == 64, "gemm_rows_qkv_rope: %d columns per block: 32 or 64", columns);
   BLM_REQUIRE(rows == 64 || (rows == 32 && columns == 32), "gemm_rows_qkv_rope: %d rows per block: 64, or 32 with 32 columns", rows);
   BLM_REQUIRE(M >= 1 && M <= GR_MAX_ROWS && K >= 8 && K % 8 == 0 && hd >= 2 && hd % 2 == 0,
@@ -393,7 +394,7 @@ extern "C" int blm_gemm_rows_qkv_rope(const void* A, const void* W, void* qkv_ou
               "gemm_rows_qkv_rope: matrices of 4 GiB and more are not supported");
   const GrRope rope{positions, token_seq, block_table, (const float2*)cos_sin, (bf16*)kcache, (bf16*)vcache,
                     table_width, page_size, nh, nkv, hd, store};
-  if (columns == 64) return gr_launch<64, 64, 64, 2, 2, bf16>(A, W, qkv_out, M, N, K, lda, ldw, ldq, 1, stream, rope);
-  if (M > 32 && rows != 32) return gr_launch<64, 32, 64, 3, 2, bf16>(A, W, qkv_out, M, N, K, lda, ldw, ldq, 1, stream, rope);
-  return gr_launch<32, 32, 64, 5, 2, bf16>(A, W, qkv_out, M, N, K, lda, ldw, ldq, 1, stream, rope);
+  if (columns == 64) return gr_launch<64, 64, 64, 2, 2, bf16>(A, W, qkv_out, M, N, K, lda, ldw, ldq, 1, once, stream, rope);
+  if (M > 32 && rows != 32) return gr_launch<64, 32, 64, 3, 2, bf16>(A, W, qkv_out, M, N, K, lda, ldw, ldq, 1, once, stream, rope);
+  return gr_launch<32, 32, 64, 5, 2, bf16>(A, W, qkv_out, M, N, K, lda, ldw, ldq, 1, once, stream, rope);
 }

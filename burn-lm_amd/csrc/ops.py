@@ -11,7 +11,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 50
+ABI_VERSION = 51
 _lib = None
 _lock = threading.Lock()
 
@@ -163,7 +163,7 @@ _SIGNATURES = {
     "blm_gemm_mfma_init": [],
     "blm_gemm_rows_init": [],
     "blm_gemm_rows": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
-                      _c_int, _c_void_p],
+                      _c_int, _c_int, _c_void_p],
     "blm_attn_paged_init": [],
     "blm_sink_attn_mfma_init": [],
     "blm_gemm_mfma": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
@@ -178,7 +178,7 @@ _SIGNATURES = {
                           _c_int, _c_void_p],
     "blm_gemm_rows_qkv_rope": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p,
                                _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
-                               _c_int, _c_int, _c_int, _c_void_p],
+                               _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "blm_argmax": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p],
     "blm_probe_read": [_c_void_p, ctypes.c_longlong, _c_void_p, _c_int, _c_void_p],
     "blm_probe_mfma": [_c_int, _c_int, _c_int, _c_void_p, _c_void_p],
@@ -1145,12 +1145,13 @@ def gemm_rows_init(device=None):
         _rows_ready.add(index)
 
 
-def gemm_rows(a, w, out, gated=False, columns=64):
+def gemm_rows(a, w, out, gated=False, columns=64, once=False):
     """bfloat16 product for few rows (made for 17 to 64; up to 256 as one block for every 64 rows) whose loads
     never stop for a barrier: out = a[M, K] @ w[N, K]^T, w as the checkpoint stores it.  out: bfloat16 or float32 [M, N], or float32 [groups, M, N] partial
     products over that many groups of K (the reader sums them).  gated=True: w is [gate rows; up rows]
     ([2I, K]) and out is [M, I] = silu(a gate^T) * (a up^T).  columns: 64 or (without gating) 32 columns
-    of out (of gate and up together when gated) per block."""
+    of out (of gate and up together when gated) per block.  once: the weights come from memory and are not wanted in
+    the caches, which wide ones are then loaded past."""
     _gpu(a, w, out)
     gemm_rows_init(a.device)
     groups = 1
@@ -1167,7 +1168,7 @@ def gemm_rows(a, w, out, gated=False, columns=64):
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise KernelError("gemm_rows: operands must be bfloat16")
     _call("blm_gemm_rows", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out), M, N, K, a.stride(0), w.stride(0),
-          out.stride(-2), 1 if gated else 0, groups, int(columns), _stream())
+          out.stride(-2), 1 if gated else 0, groups, int(columns), 1 if once else 0, _stream())
     return out
 
 
@@ -1210,11 +1211,11 @@ def gemv_qkv_rope(x, packed, qkv_out, positions, token_seq, block_table, cos_sin
 
 
 def gemm_rows_qkv_rope(x, w, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache, page_size,
-                       nh, nkv, hd, write_kv=True, columns=32, rows=64):
+                       nh, nkv, hd, write_kv=True, columns=32, rows=64, once=False):
     """17 to 256 rows: x [M, K] @ W_qkv^T (w [(nh + 2 nkv) * hd, K] as bound, rotary partners in adjacent
     rows), rotary encoding of q and k on the float results, q into qkv_out[:, :nh*hd], k and v into
     their cache pages, in one kernel (the product of gemm_rows).  columns: 32 or 64 per block; rows: 64
-    staged per block, or 32 (with 32 columns), which is what runs up to 32 rows in any case."""
+    staged per block, or 32 (with 32 columns), which is what runs up to 32 rows in any case; once as in gemm_rows."""
     _gpu(x, w, qkv_out, positions, token_seq, block_table, cos_sin, kcache, vcache)
     gemm_rows_init(x.device)
     M, K = x.shape
@@ -1235,7 +1236,7 @@ def gemm_rows_qkv_rope(x, w, qkv_out, positions, token_seq, block_table, cos_sin
     _call("blm_gemm_rows_qkv_rope", x.data_ptr(), w.data_ptr(), qkv_out.data_ptr(), positions.data_ptr(),
           token_seq.data_ptr(), block_table.data_ptr(), block_table.shape[1], cos_sin.data_ptr(), kcache.data_ptr(),
           vcache.data_ptr(), page_size, M, K, x.stride(0), w.stride(0), qkv_out.stride(0), nh, nkv, hd,
-          1 if write_kv else 0, columns, rows, _stream())
+          1 if write_kv else 0, columns, rows, 1 if once else 0, _stream())
     return qkv_out
 
 

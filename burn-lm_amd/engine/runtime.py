@@ -93,6 +93,7 @@ F32_SHARE_US = 0.1
 JOIN_BF16_WIDTH = 1024     # see Runtime.join_takes
 F32_SKINNY_MAX_ROWS = 16
 F32_SKINNY_GROUP_K = 2048
+LAST_LEVEL_BYTES = 256 << 20      # the cache in front of the memory
 
 
 def _planes_us(M, N, groups, planes):
@@ -275,6 +276,8 @@ class LinearWeight:
 
 
 class Runtime:
+    bound_bytes = 0      # of the matrices bound so far that could stay in the last-level cache (one bound twice counts twice)
+
     def __init__(self, dtype=torch.bfloat16, device="cuda:0"):
         if dtype not in (torch.bfloat16, torch.float32):
             raise ValueError(f"activation dtype must be bfloat16 or float32, got {dtype}")
@@ -321,6 +324,8 @@ class Runtime:
         gated_linear(); its packed copy pairs each gate row with its up row."""
         w = w.contiguous()
         N, K = w.shape
+        size = w.numel() * w.element_size()
+        self.bound_bytes += size if size <= LAST_LEVEL_BYTES else 0
         # (a K too long for one group of the skinny product still runs in several, as partial planes; the gated
         # product has no planes)
         packable = w.dtype == torch.bfloat16 and K % 8 == 0 and K >= 8 and (
@@ -331,6 +336,12 @@ class Runtime:
             gated = gated and N % 16 == 0 and K <= F32_SKINNY_GROUP_K
             return LinearWeight(w, packable, gated, room=self.packing_room)
         return LinearWeight(w, packable, gated)
+
+    @property
+    def streams_weights(self):
+        """Whether a step finds its weights in memory, not in the last-level cache, where the step before would have left them (see GR_ONCE_BYTES of
+        gemm_rows.hip)."""
+        return self.bound_bytes > LAST_LEVEL_BYTES
 
     def k_groups(self, N, K, M=1):
         """Into how many groups a skinny product's K is cut: the fewest whose stretch of K is at most
@@ -564,7 +575,7 @@ class Runtime:
                 if g2:
                     return ops.gemm_mfma(x, w, torch.empty(g2, M, N, dtype=torch.float32, device=x.device), tile=tile)
             if groups > 1:
-                return ops.gemm_rows(x, w, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), columns=columns)
+                return ops.gemm_rows(x, w, torch.empty(groups, M, N, dtype=torch.float32, device=x.device), columns=columns, once=self.streams_weights)
         if packable and M <= MFMA_SKINNY_MAX_ROWS and aligned:
             if planes:
                 groups = self.k_groups(N, K, M)
@@ -880,7 +891,7 @@ class Runtime:
             # from 17 rows on where the blocks come in one round, or in two where K is short (us at 17 / 24 / 32
             # rows against the packed kernel: width 2048, inner 8192: 14.0 / 14.3 / 14.3 against 16.4 / 17.7 / 18.2;
             # width 1536: 11.8 / 11.9 / 12.0 against 13.3 / 14.1 / 14.6; 3B: 10-15 %)
-            return ops.gemm_rows(x, plain, torch.empty(M, inner, dtype=self.dtype, device=x.device), gated=True)
+            return ops.gemm_rows(x, plain, torch.empty(M, inner, dtype=self.dtype, device=x.device), gated=True, once=self.streams_weights)
         if (isinstance(w, LinearWeight) and w.packable and w.gated and x.dtype == torch.bfloat16 and not by_library
                 and M <= self.skinny_gated_rows and ops.gemv_mfma_supported(M, w.shape[0], K)
                 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0):

@@ -197,7 +197,7 @@ class RotaryEncoding(PositionEncoding):
         if fused == "rows":
             return rt.ops.gemm_rows_qkv_rope(x, raw, qkv, step.positions, step.token_seq, view.block_table(step), self.table,
                                              view.k, view.v, view.page_size, heads, kv_heads, head_dim, write_kv=view.store,
-                                             columns=plan.columns, rows=plan.rows)
+                                             columns=plan.columns, rows=plan.rows, once=getattr(rt, "streams_weights", False))
         return rt.ops.gemv_qkv_rope(x, w_qkv.packed, qkv, step.positions, step.token_seq, view.block_table(step),
                                     self.table, view.k, view.v, view.page_size, heads, kv_heads, head_dim,
                                     self.pairing, write_kv=view.store, scale=scale)
